@@ -836,23 +836,95 @@ extern "C" int rgx_morton_order(const float *pos, int64_t n, int64_t *codes, int
 // Fused multi-tensor gather for the periodic reordering of the point cloud: every
 // per-Gaussian tensor (parameters, Adam moments, statistics) is permuted with the same index
 // (classes/point_cloud.py:1031-1044, classes/optimizer.py:54-66: one `tensor[index]` launch per
-// tensor there).  blockIdx.y picks the tensor; a thread moves one 32-bit word, so writes are
-// coalesced and the reads of a row are contiguous.
+// tensor there).  A workgroup takes RGX_GATHER_ROWS consecutive output rows, fetches their source rows'
+// numbers once and moves the rows of one tensor after the other, in the widest pieces that the rows'
+// length and the tensors' alignment allow (16, 12, 8 or 4 bytes): writes are coalesced, the reads of a
+// row are contiguous, and every thread has up to four reads in flight.  Bound by memory: one 32-bit word per
+// thread, its row found by a 64-bit division and its number fetched per word, took 0.743 ms for the 15
+// tensors of a 1 M cloud (1.42 GB); this takes 0.438 ms (3.2 TB/s).
 #define RGX_GATHER_MAX 24
+#define RGX_GATHER_ROWS 128
+#define RGX_GATHER_LONG 4096 // a row of at least this many pieces is moved by the workgroup on its own
 struct GatherArgs {
     const uint32_t *src[RGX_GATHER_MAX];
     uint32_t *dst[RGX_GATHER_MAX];
-    int32_t row_words[RGX_GATHER_MAX];
+    int32_t pieces[RGX_GATHER_MAX];  // per row
+    uint32_t magic[RGX_GATHER_MAX];  // floor(2^32 / pieces) + 1: p / pieces = umulhi(p, magic) for p * pieces < 2^32
+    uint8_t words[RGX_GATHER_MAX];   // 32-bit words of a piece
+    int32_t count;
 };
+template <int W>
+struct Piece {
+    uint32_t v[W];
+};
+template <int W>
+__device__ __forceinline__ Piece<W> piece_load(const uint32_t *p)
+{
+    Piece<W> x;
+    if constexpr (W == 4) {
+        const uint4 u = *(const uint4 *)p;
+        x.v[0] = u.x; x.v[1] = u.y; x.v[2] = u.z; x.v[3] = u.w;
+    } else if constexpr (W == 2) {
+        const uint2 u = *(const uint2 *)p;
+        x.v[0] = u.x; x.v[1] = u.y;
+    } else {
+#pragma unroll
+        for (int k = 0; k < W; ++k) x.v[k] = p[k];
+    }
+    return x;
+}
+template <int W>
+__device__ __forceinline__ void piece_store(uint32_t *p, const Piece<W> &x)
+{
+    if constexpr (W == 4) *(uint4 *)p = make_uint4(x.v[0], x.v[1], x.v[2], x.v[3]);
+    else if constexpr (W == 2) *(uint2 *)p = make_uint2(x.v[0], x.v[1]);
+    else {
+#pragma unroll
+        for (int k = 0; k < W; ++k) p[k] = x.v[k];
+    }
+}
+
+template <int W>
+__device__ __forceinline__ void gather_tensor(const uint32_t *src, uint32_t *dst, int pieces, uint32_t magic, const int64_t *s_row,
+                                              int64_t row0, int rows)
+{
+    uint32_t *out = dst + row0 * ((int64_t)pieces * W);
+    if (pieces >= RGX_GATHER_LONG) {
+        for (int r = 0; r < rows; ++r)
+            for (int q = threadIdx.x; q < pieces; q += 256)
+                piece_store<W>(out + ((int64_t)r * pieces + q) * W, piece_load<W>(src + (s_row[r] * pieces + q) * W));
+        return;
+    }
+    const int total = rows * pieces; // < RGX_GATHER_ROWS * RGX_GATHER_LONG
+    auto from = [&](int p) {
+        const int r = pieces == 1 ? p : (int)__umulhi((uint32_t)p, magic);
+        return src + (s_row[r] * pieces + (p - r * pieces)) * W;
+    };
+    int p = threadIdx.x;
+    for (; p + 3 * 256 < total; p += 4 * 256) {
+        Piece<W> x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = piece_load<W>(from(p + k * 256));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) piece_store<W>(out + (int64_t)(p + k * 256) * W, x[k]);
+    }
+    for (; p < total; p += 256) piece_store<W>(out + (int64_t)p * W, piece_load<W>(from(p)));
+}
 
 __global__ __launch_bounds__(256) void k_gather_rows(const GatherArgs A, const int64_t *__restrict__ order, int64_t n)
 {
-    const int t = blockIdx.y;
-    const int64_t rw = A.row_words[t];
-    const int64_t total = n * rw;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t row = e / rw, w = e - row * rw;
-        A.dst[t][e] = A.src[t][order[row] * rw + w];
+    __shared__ int64_t s_row[RGX_GATHER_ROWS];
+    const int64_t row0 = (int64_t)blockIdx.x * RGX_GATHER_ROWS;
+    const int rows = (int)(n - row0 < RGX_GATHER_ROWS ? n - row0 : RGX_GATHER_ROWS);
+    if ((int)threadIdx.x < rows) s_row[threadIdx.x] = order[row0 + threadIdx.x];
+    __syncthreads();
+    for (int t = blockIdx.y; t < A.count; t += gridDim.y) {
+        switch (A.words[t]) {
+        case 4: gather_tensor<4>(A.src[t], A.dst[t], A.pieces[t], A.magic[t], s_row, row0, rows); break;
+        case 3: gather_tensor<3>(A.src[t], A.dst[t], A.pieces[t], A.magic[t], s_row, row0, rows); break;
+        case 2: gather_tensor<2>(A.src[t], A.dst[t], A.pieces[t], A.magic[t], s_row, row0, rows); break;
+        default: gather_tensor<1>(A.src[t], A.dst[t], A.pieces[t], A.magic[t], s_row, row0, rows); break;
+        }
     }
 }
 
@@ -868,16 +940,21 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
     for (int base = 0; base < count; base += RGX_GATHER_MAX) {
         GatherArgs A;
         const int m = count - base < RGX_GATHER_MAX ? count - base : RGX_GATHER_MAX;
-        int64_t most = 0;
+        A.count = m;
         for (int i = 0; i < m; ++i) {
             A.src[i] = (const uint32_t *)src[base + i];
             A.dst[i] = (uint32_t *)dst[base + i];
-            A.row_words[i] = (int32_t)(row_bytes[base + i] / 4);
-            most = most > n * A.row_words[i] ? most : n * A.row_words[i];
+            const int32_t words = (int32_t)(row_bytes[base + i] / 4);
+            const uintptr_t at = (uintptr_t)A.src[i] | (uintptr_t)A.dst[i];
+            const int w = words % 4 == 0 && (at & 15) == 0 ? 4 : words % 3 == 0 ? 3 : words % 2 == 0 && (at & 7) == 0 ? 2 : 1;
+            A.words[i] = (uint8_t)w;
+            A.pieces[i] = words / w;
+            A.magic[i] = (uint32_t)((1ull << 32) / (uint32_t)A.pieces[i] + 1);
         }
-        int64_t blocks = (most + 255) / 256;
-        if (blocks > 65536) blocks = 65536; // grid-stride beyond that
-        hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)blocks, (unsigned)m), dim3(256), 0, (hipStream_t)stream, A, order, n);
+        const int64_t blocks = (n + RGX_GATHER_ROWS - 1) / RGX_GATHER_ROWS;
+        // a workgroup goes through all tensors where there are enough of them to fill the chip several times over
+        const int split = blocks >= 2048 ? 1 : m;
+        hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)blocks, (unsigned)split), dim3(256), 0, (hipStream_t)stream, A, order, n);
         RGX_LAUNCH_CHECK();
     }
     return RGX_OK;
