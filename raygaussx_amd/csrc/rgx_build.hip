@@ -7,6 +7,7 @@
 #include <float.h>
 
 #include <algorithm>
+#include <type_traits>
 
 // ---------------------------------------------------------------------------
 // order-preserving float <-> int encoding for atomicMin/atomicMax
@@ -56,17 +57,6 @@ __global__ void k_refit_begin(WsHeader *h, int64_t n)
 }
 __device__ __forceinline__ bool gate_closed(const int32_t *gate) { return gate != nullptr && *gate == 0; }
 
-__device__ __forceinline__ float wave_min(float v)
-{
-    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-    return v;
-}
-__device__ __forceinline__ float wave_max(float v)
-{
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
-}
-
 // k-sigma AABB of a rotated ellipsoid (optix_utils.py:49-77), canonical arithmetic.
 __global__ __launch_bounds__(256) void k_aabb(const float *__restrict__ pos, const float *__restrict__ scale,
                                               const float *__restrict__ quat, const float *__restrict__ dens,
@@ -103,7 +93,7 @@ __global__ __launch_bounds__(256) void k_aabb(const float *__restrict__ pos, con
     __shared__ float red[4][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
-        const float mn = wave_min(b[a]), mx = wave_max(b[a + 3]);
+        const float mn = wave_min_all(b[a]), mx = wave_max_all(b[a + 3]);
         if (lane == 0) { red[wave][a] = mn; red[wave][a + 3] = mx; }
     }
     __syncthreads();
@@ -574,7 +564,7 @@ __global__ __launch_bounds__(256) void k_take_boxes(const float *__restrict__ in
     __shared__ float red[4][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
-        const float mn = wave_min(b[a]), mx = wave_max(b[a + 3]);
+        const float mn = wave_min_all(b[a]), mx = wave_max_all(b[a + 3]);
         if (lane == 0) { red[wave][a] = mn; red[wave][a + 3] = mx; }
     }
     __syncthreads();
@@ -746,7 +736,7 @@ __global__ __launch_bounds__(256) void k_pos_minmax(const float *__restrict__ po
     __shared__ float red[4][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
-        const float mn = wave_min(b[a]), mx = wave_max(b[a + 3]);
+        const float mn = wave_min_all(b[a]), mx = wave_max_all(b[a + 3]);
         if (lane == 0) { red[wave][a] = mn; red[wave][a + 3] = mx; }
     }
     __syncthreads();
@@ -964,104 +954,192 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
 // Mean squared distance of every point to its three nearest neighbours: distCUDA2 of the
 // simple-knn extension (submodules/simple-knn/simple_knn.cu:186-222; used to initialise the scales,
 // classes/point_cloud.py:252).  As there: points sorted along a Morton curve, boxes of consecutive
-// sorted points, every point scans the boxes that can still hold one of its three nearest (the
-// pruning is exact, so the result is the exact 3-NN mean whatever the order and the box size).
-// Here the boxes have two levels (256 points, 64 boxes) so that a point looks at a few hundred box
-// bounds instead of all n / 256, and the sorted points are gathered once so that the scans read
-// consecutive memory.  Distances are (dx*dx + dy*dy) + dz*dz without contraction.
-#define RGX_KNN_BOX 256
-#define RGX_KNN_SUPER 64
+// sorted points, boxes that cannot hold one of the three nearest are left out (the pruning is exact,
+// so the result is the exact 3-NN mean whatever the order and the box size).
+// Here a wavefront searches for the 64 consecutive points of the curve that it owns, together: three
+// levels of boxes (16 points, 64 leaves, 64 boxes), of which each lane tests one child against the
+// bounds of the wavefront's points and the largest distance any of them still has to beat; the leaves that
+// are left are tested by every lane for its own point, and a leaf that some lane needs is read once, as
+// scalars, and met by all lanes in straight-line code.  What bounds it is the issue of those distance
+// computations (12 instructions per point and leaf point); one lane searching on its own through boxes of
+// 256 points made every lane of a wavefront wait for the scans of all others: 5.26 ms at 1 M points,
+// 2.20 ms at 54 k points of a heavy-tailed cloud, against 0.44 and 0.15 ms now.
+// Distances are (dx*dx + dy*dy) + dz*dz without contraction; rounding is monotone, so the distance to a
+// box that holds a point, computed the same way, is never larger than the distance to the point.
+#define RGX_KNN_LEAF 16
+#define RGX_KNN_FAN 64
+#define RGX_KNN_BOX (RGX_KNN_LEAF * RGX_KNN_FAN)
+#ifndef RGX_KNN_SEGS
+#define RGX_KNN_SEGS 4
+#endif
+#define RGX_KNN_NEAR 4 // leaves before and after a wavefront's own that it looks at first
 
-__global__ __launch_bounds__(256) void k_knn_gather(const float *__restrict__ pos, const uint32_t *__restrict__ order, int64_t n,
-                                                    float4 *__restrict__ pts)
+// Gathers the sorted points and bounds them: one workgroup per box of 1024.  A point with a coordinate that is
+// not a number is at no distance from any other: it becomes a point at infinity, and such points, like the
+// padding behind the last one, are in no box's bounds.
+__global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restrict__ pos, const uint32_t *__restrict__ order,
+                                                            int64_t n, float4 *__restrict__ pts, float4 *__restrict__ leaves,
+                                                            float4 *__restrict__ boxes, int32_t *supers_enc)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int64_t j = order[i];
-    pts[i] = make_float4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], 0.f);
-}
-
-// bounds of `per` consecutive items: points (float4) at level 0, boxes (lo, hi pairs) above
-__global__ __launch_bounds__(256) void k_knn_bounds(const float4 *__restrict__ lo_in, const float4 *__restrict__ hi_in,
-                                                    int stride, int64_t n_in, int per, float4 *__restrict__ out)
-{
-    const int64_t b = blockIdx.x;
-    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int64_t i = b * per + threadIdx.x; i < n_in && i < (b + 1) * per; i += blockDim.x) {
-        const float4 l = lo_in[i * stride], h = hi_in[i * stride];
-        mn[0] = fminf(mn[0], l.x); mn[1] = fminf(mn[1], l.y); mn[2] = fminf(mn[2], l.z);
-        mx[0] = fmaxf(mx[0], h.x); mx[1] = fmaxf(mx[1], h.y); mx[2] = fmaxf(mx[2], h.z);
+    const int64_t i = (int64_t)blockIdx.x * RGX_KNN_BOX + threadIdx.x;
+    float4 p = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+    if (i < n) {
+        const int64_t j = order[i];
+        const float x = pos[3 * j], y = pos[3 * j + 1], z = pos[3 * j + 2];
+        if (x == x && y == y && z == z) p = make_float4(x, y, z, 0.f);
     }
-    __shared__ float red[4][6];
+    pts[i] = p;
+    const bool fin = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
+    float mn[3] = {fin ? p.x : INFINITY, fin ? p.y : INFINITY, fin ? p.z : INFINITY};
+    float mx[3] = {fin ? p.x : -INFINITY, fin ? p.y : -INFINITY, fin ? p.z : -INFINITY};
+    auto spread = [&](int o) {
+        for (int a = 0; a < 3; ++a) {
+            mn[a] = fminf(mn[a], __shfl_xor(mn[a], o));
+            mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], o));
+        }
+    };
+    for (int o = 1; o < RGX_KNN_LEAF; o <<= 1) spread(o);
+    if ((threadIdx.x & (RGX_KNN_LEAF - 1)) == 0) {
+        const int64_t l = i / RGX_KNN_LEAF;
+        leaves[2 * l] = make_float4(mn[0], mn[1], mn[2], 0.f);
+        leaves[2 * l + 1] = make_float4(mx[0], mx[1], mx[2], 0.f);
+    }
+    for (int o = RGX_KNN_LEAF; o < 64; o <<= 1) spread(o);
+    __shared__ float red[RGX_KNN_BOX / 64][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int a = 0; a < 3; ++a) {
-        const float l = wave_min(mn[a]), h = wave_max(mx[a]);
-        if (lane == 0) { red[wave][a] = l; red[wave][a + 3] = h; }
-    }
+    if (lane == 0)
+        for (int a = 0; a < 3; ++a) {
+            red[wave][a] = mn[a];
+            red[wave][a + 3] = mx[a];
+        }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int a = 0; a < 6; ++a)
-            for (int w = 1; w < 4; ++w) red[0][a] = a < 3 ? fminf(red[0][a], red[w][a]) : fmaxf(red[0][a], red[w][a]);
-        out[2 * b] = make_float4(red[0][0], red[0][1], red[0][2], 0.f);
-        out[2 * b + 1] = make_float4(red[0][3], red[0][4], red[0][5], 0.f);
+    if (threadIdx.x < 6) {
+        const int a = threadIdx.x;
+        float v = red[0][a];
+        for (int w = 1; w < RGX_KNN_BOX / 64; ++w) v = a < 3 ? fminf(v, red[w][a]) : fmaxf(v, red[w][a]);
+        ((float *)(boxes + 2 * (int64_t)blockIdx.x))[a < 3 ? a : a + 1] = v;
+        int32_t *super = supers_enc + 6 * (int64_t)(blockIdx.x / RGX_KNN_FAN);
+        if (a < 3) atomicMin(&super[a], enc_f(v));
+        else atomicMax(&super[a], enc_f(v));
     }
 }
 
-// simple_knn.cu:124-135 distBoxPoint
-__device__ __forceinline__ float knn_box_dist(float4 lo, float4 hi, float4 p)
+__global__ __launch_bounds__(256) void k_knn_begin(int32_t *mn, int32_t *mx, int32_t *supers_enc, int64_t ns)
 {
-    float dx = 0.f, dy = 0.f, dz = 0.f;
-    if (p.x < lo.x || p.x > hi.x) dx = fminf(fabsf(p.x - lo.x), fabsf(p.x - hi.x));
-    if (p.y < lo.y || p.y > hi.y) dy = fminf(fabsf(p.y - lo.y), fabsf(p.y - hi.y));
-    if (p.z < lo.z || p.z > hi.z) dz = fminf(fabsf(p.z - lo.z), fabsf(p.z - hi.z));
+    if (threadIdx.x < 3) {
+        mn[threadIdx.x] = enc_f(INFINITY);
+        mx[threadIdx.x] = enc_f(-INFINITY);
+    }
+    for (int64_t k = threadIdx.x; k < 6 * ns; k += blockDim.x) supers_enc[k] = enc_f(k % 6 < 3 ? INFINITY : -INFINITY);
+}
+
+// Squared distance between two boxes (a point is a box of no size): simple_knn.cu:124-135 distBoxPoint.
+__device__ __forceinline__ float knn_box_dist(f3 lo, f3 hi, f3 qlo, f3 qhi)
+{
+    const float dx = fmaxf(fmaxf(lo.x - qhi.x, qlo.x - hi.x), 0.f);
+    const float dy = fmaxf(fmaxf(lo.y - qhi.y, qlo.y - hi.y), 0.f);
+    const float dz = fmaxf(fmaxf(lo.z - qhi.z, qlo.z - hi.z), 0.f);
     return (dx * dx + dy * dy) + dz * dz;
 }
 
-// simple_knn.cu:137-151 updateKBest<3>
-__device__ __forceinline__ void knn_update(float4 ref, float4 q, float *best)
-{
-    const float dx = q.x - ref.x, dy = q.y - ref.y, dz = q.z - ref.z;
-    float dist = (dx * dx + dy * dy) + dz * dz;
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-        if (best[j] > dist) {
-            const float t = best[j];
-            best[j] = dist;
-            dist = t;
-        }
-}
-
-// simple_knn.cu:153-184 boxMeanDist
+// simple_knn.cu:137-184 updateKBest<3>, boxMeanDist
 __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, const uint32_t *__restrict__ order, int64_t n,
-                                              const float4 *__restrict__ boxes, int64_t nb, const float4 *__restrict__ supers,
-                                              int64_t ns, float *__restrict__ out)
+                                              const float4 *__restrict__ leaves, const float4 *__restrict__ boxes, int64_t nb,
+                                              const int32_t *__restrict__ supers_enc, int64_t ns, float *__restrict__ out)
 {
+    const int lane = threadIdx.x & 63;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 p = pts[i];
-    float best[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
-    for (int64_t j = i - 3 < 0 ? 0 : i - 3; j <= (i + 3 > n - 1 ? n - 1 : i + 3); ++j)
-        if (j != i) knn_update(p, pts[j], best);
-    const float reject = best[2];
-    best[0] = best[1] = best[2] = FLT_MAX;
-    for (int64_t s = 0; s < ns; ++s) {
-        const float ds = knn_box_dist(supers[2 * s], supers[2 * s + 1], p);
-        if (ds > reject || ds > best[2]) continue;
-        const int64_t b1 = (s + 1) * RGX_KNN_SUPER < nb ? (s + 1) * RGX_KNN_SUPER : nb;
-        for (int64_t b = s * RGX_KNN_SUPER; b < b1; ++b) {
-            const float d = knn_box_dist(boxes[2 * b], boxes[2 * b + 1], p);
-            if (d > reject || d > best[2]) continue;
-            const int64_t j1 = (b + 1) * RGX_KNN_BOX < n ? (b + 1) * RGX_KNN_BOX : n;
-            for (int64_t j = b * RGX_KNN_BOX; j < j1; ++j)
-                if (j != i) knn_update(p, pts[j], best);
+    if (i - lane >= n) return; // whole wave
+    const float4 p4 = pts[i]; // (the array is padded to whole boxes)
+    const f3 p = mk3(p4.x, p4.y, p4.z);
+    const bool act = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
+    // The wavefront's points as RGX_KNN_SEGS runs of the curve, cut where it jumps farthest: the bounds of a run that
+    // spans such a jump would meet most of the cloud (one such wavefront was the whole launch's time).
+    uint64_t cuts = 0;
+    {
+        const f3 prev = mk3(__shfl_up(p.x, 1), __shfl_up(p.y, 1), __shfl_up(p.z, 1));
+        const f3 step = p - prev;
+        float gap = lane > 0 ? dot3(step, step) : -1.f;
+        if (!(gap < INFINITY)) gap = -1.f;
+        for (int k = 1; k < RGX_KNN_SEGS; ++k) {
+            const float g = wave_max_all(gap);
+            const uint64_t at = __ballot(gap == g && g > 0.f);
+            if (at == 0) break;
+            cuts |= at & -at;
+            if (lane == __builtin_ctzll(at)) gap = -1.f;
         }
     }
-    out[order[i]] = ((best[0] + best[1]) + best[2]) / 3.0f;
+    const int seg = __popcll(cuts & (~0ull >> (63 - lane)));
+    f3 slo[RGX_KNN_SEGS], shi[RGX_KNN_SEGS];
+    float reach[RGX_KNN_SEGS]; // the largest distance a point of the run still has to beat
+    for (int k = 0; k < RGX_KNN_SEGS; ++k) {
+        const bool in = act && seg == k;
+        slo[k] = mk3(wave_min_all(in ? p.x : INFINITY), wave_min_all(in ? p.y : INFINITY), wave_min_all(in ? p.z : INFINITY));
+        shi[k] = mk3(wave_max_all(in ? p.x : -INFINITY), wave_max_all(in ? p.y : -INFINITY), wave_max_all(in ? p.z : -INFINITY));
+    }
+    float b0 = FLT_MAX, b1 = FLT_MAX, b2 = FLT_MAX; // the three smallest so far, ascending
+    auto meet = [&](int l, auto own) { // all points of leaf l (the same in every lane)
+        l = __builtin_amdgcn_readfirstlane(l);
+        const float4 *q = pts + (int64_t)l * RGX_KNN_LEAF;
+#pragma unroll
+        for (int k = 0; k < RGX_KNN_LEAF; ++k) {
+            const float dx = q[k].x - p.x, dy = q[k].y - p.y, dz = q[k].z - p.z;
+            float d = (dx * dx + dy * dy) + dz * dz;
+            if constexpr (decltype(own)::value) d = (int64_t)l * RGX_KNN_LEAF + k == i ? FLT_MAX : d;
+            b2 = __builtin_amdgcn_fmed3f(b1, b2, d);
+            b1 = __builtin_amdgcn_fmed3f(b0, b1, d);
+            b0 = fminf(b0, d);
+        }
+    };
+    // the points nearby on the curve first: they leave little for the boxes
+    const int leaf0 = __builtin_amdgcn_readfirstlane((int)((i - lane) / RGX_KNN_LEAF));
+    for (int l = leaf0; l < leaf0 + 64 / RGX_KNN_LEAF; ++l) meet(l, std::true_type{});
+    const int n_leaves = (int)(nb * RGX_KNN_FAN);
+    const int done0 = std::max(leaf0 - RGX_KNN_NEAR, 0), done1 = std::min(leaf0 + 64 / RGX_KNN_LEAF + RGX_KNN_NEAR, n_leaves);
+    for (int l = done0; l < leaf0; ++l) meet(l, std::false_type{});
+    for (int l = leaf0 + 64 / RGX_KNN_LEAF; l < done1; ++l) meet(l, std::false_type{});
+    auto measure = [&]() {
+        for (int k = 0; k < RGX_KNN_SEGS; ++k) reach[k] = wave_max_all(act && seg == k ? b2 : -1.f);
+    };
+    measure();
+    auto open = [&](f3 lo, f3 hi) { // is the box within some run's reach?
+        bool o = false;
+        for (int k = 0; k < RGX_KNN_SEGS; ++k) o |= knn_box_dist(lo, hi, slo[k], shi[k]) < reach[k];
+        return o;
+    };
+    auto open_at = [&](const float4 *b) {
+        const float4 lo = b[0], hi = b[1];
+        return open(mk3(lo.x, lo.y, lo.z), mk3(hi.x, hi.y, hi.z));
+    };
+    for (int64_t s0 = 0; s0 < ns; s0 += 64) {
+        bool super = false;
+        if (s0 + lane < ns) {
+            const int32_t *e = supers_enc + 6 * (s0 + lane);
+            super = open(mk3(dec_f(e[0]), dec_f(e[1]), dec_f(e[2])), mk3(dec_f(e[3]), dec_f(e[4]), dec_f(e[5])));
+        }
+        for (uint64_t ms = __ballot(super); ms; ms &= ms - 1) {
+            const int64_t box0 = (s0 + __builtin_ctzll(ms)) * RGX_KNN_FAN;
+            for (uint64_t mb = __ballot(box0 + lane < nb && open_at(boxes + 2 * (box0 + lane))); mb; mb &= mb - 1) {
+                const int l0 = (int)(box0 + __builtin_ctzll(mb)) * RGX_KNN_FAN;
+                const float4 lo = leaves[2 * (int64_t)(l0 + lane)], hi = leaves[2 * (int64_t)(l0 + lane) + 1];
+                const bool near = (l0 + lane < done0 || l0 + lane >= done1) && open(mk3(lo.x, lo.y, lo.z), mk3(hi.x, hi.y, hi.z));
+                const uint64_t some = __ballot(near);
+                for (uint64_t ml = some; ml; ml &= ml - 1) {
+                    const int t = __builtin_ctzll(ml);
+                    auto at = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), t)); };
+                    const float d = knn_box_dist(mk3(at(lo.x), at(lo.y), at(lo.z)), mk3(at(hi.x), at(hi.y), at(hi.z)), p, p);
+                    if (__any(act && d < b2)) meet(l0 + t, std::false_type{});
+                }
+                if (some) measure();
+            }
+        }
+    }
+    if (i < n) out[order[i]] = act ? ((b0 + b1) + b2) / 3.0f : INFINITY;
 }
 
 struct KnnLayout {
     MortonLayout m;
-    size_t pts, boxes, supers, total;
+    size_t pts, leaves, boxes, supers, total;
     int64_t nb, ns;
 };
 static inline KnnLayout knn_layout(int64_t n)
@@ -1070,11 +1148,12 @@ static inline KnnLayout knn_layout(int64_t n)
     K.m = morton_layout(n);
     const size_t nn = (size_t)(n > 0 ? n : 1);
     K.nb = (int64_t)((nn + RGX_KNN_BOX - 1) / RGX_KNN_BOX);
-    K.ns = (K.nb + RGX_KNN_SUPER - 1) / RGX_KNN_SUPER;
+    K.ns = (K.nb + RGX_KNN_FAN - 1) / RGX_KNN_FAN;
     size_t off = K.m.total;
-    K.pts = off;    off = rgx_align_up(off + nn * 16, 256);
+    K.pts = off;    off = rgx_align_up(off + (size_t)K.nb * RGX_KNN_BOX * 16, 256);
+    K.leaves = off; off = rgx_align_up(off + (size_t)K.nb * RGX_KNN_FAN * 32, 256);
     K.boxes = off;  off = rgx_align_up(off + (size_t)K.nb * 32, 256);
-    K.supers = off; off = rgx_align_up(off + (size_t)K.ns * 32, 256);
+    K.supers = off; off = rgx_align_up(off + (size_t)K.ns * 24, 256);
     K.total = off;
     return K;
 }
@@ -1098,8 +1177,9 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     int32_t *mn = (int32_t *)(w + K.m.enc), *mx = mn + 4;
     uint32_t *k0 = (uint32_t *)(w + K.m.keys0), *k1 = (uint32_t *)(w + K.m.keys1);
     uint32_t *v0 = (uint32_t *)(w + K.m.vals0), *v1 = (uint32_t *)(w + K.m.vals1);
-    float4 *pts = (float4 *)(w + K.pts), *boxes = (float4 *)(w + K.boxes), *supers = (float4 *)(w + K.supers);
-    hipLaunchKernelGGL(k_init_enc, dim3(1), dim3(64), 0, s, mn, mx);
+    float4 *pts = (float4 *)(w + K.pts), *leaves = (float4 *)(w + K.leaves), *boxes = (float4 *)(w + K.boxes);
+    int32_t *supers = (int32_t *)(w + K.supers);
+    hipLaunchKernelGGL(k_knn_begin, dim3(1), dim3(256), 0, s, mn, mx, supers, K.ns);
     hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 256), dim3(256), 0, s, pos, n, mn, mx);
     hipLaunchKernelGGL(k_decode_enc, dim3(1), dim3(64), 0, s, mn, mx);
     hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, (const float *)mn, (const float *)mx, k0, v0,
@@ -1107,10 +1187,8 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     RGX_LAUNCH_CHECK();
     const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + K.m.hist), s);
     if (r < 0) return r;
-    hipLaunchKernelGGL(k_knn_gather, grid_for(n, 256), dim3(256), 0, s, pos, v0, n, pts);
-    hipLaunchKernelGGL(k_knn_bounds, dim3((unsigned)K.nb), dim3(256), 0, s, pts, pts, 1, n, RGX_KNN_BOX, boxes);
-    hipLaunchKernelGGL(k_knn_bounds, dim3((unsigned)K.ns), dim3(256), 0, s, boxes, boxes + 1, 2, K.nb, RGX_KNN_SUPER, supers);
-    hipLaunchKernelGGL(k_knn3, grid_for(n, 256), dim3(256), 0, s, pts, v0, n, boxes, K.nb, supers, K.ns, mean_dist2);
+    hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)K.nb), dim3(RGX_KNN_BOX), 0, s, pos, v0, n, pts, leaves, boxes, supers);
+    hipLaunchKernelGGL(k_knn3, grid_for(n, 256), dim3(256), 0, s, pts, v0, n, leaves, boxes, K.nb, supers, K.ns, mean_dist2);
     RGX_LAUNCH_CHECK();
     return RGX_OK;
 }

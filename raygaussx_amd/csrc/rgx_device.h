@@ -49,6 +49,24 @@ __device__ __forceinline__ f3 apply_sinv_rt(f3 x, f3 U, f3 V, f3 W, f3 inv_s)
     return mk3(rx * inv_s.x, ry * inv_s.y, rz * inv_s.z);
 }
 
+// wave-wide reductions with DPP (all 64 lanes must be active)
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_f(float identity, float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(identity), __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
+}
+__device__ __forceinline__ float wave_min_all(float v)
+{
+    v = fminf(v, dpp_f<0xB1, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x4E, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x141, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x140, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x142, 0xa>(INFINITY, v));
+    v = fminf(v, dpp_f<0x143, 0xc>(INFINITY, v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+__device__ __forceinline__ float wave_max_all(float v) { return -wave_min_all(-v); }
+
 // 64-byte primitive record (cuda_train/forward/gaussians_aabb.h:7-12).
 struct __align__(16) Prim {
     float4 pos4;       // eye - centre, 0

@@ -174,36 +174,6 @@ template <bool STATS>
 using CountersFor = typename std::conditional<STATS, Counters, NoCounters>::type;
 
 // ---------------------------------------------------------------------------
-// wave-wide reductions with DPP (all 64 lanes must be active)
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_f(float identity, float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(identity), __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
-}
-// total in lane 63
-__device__ __forceinline__ float wave_sum_to63(float v)
-{
-    v += dpp_f<0xB1, 0xf>(0.f, v);  // quad_perm [1,0,3,2]
-    v += dpp_f<0x4E, 0xf>(0.f, v);  // quad_perm [2,3,0,1]
-    v += dpp_f<0x141, 0xf>(0.f, v); // row_half_mirror
-    v += dpp_f<0x140, 0xf>(0.f, v); // row_mirror
-    v += dpp_f<0x142, 0xa>(0.f, v); // row_bcast:15 into rows 1,3
-    v += dpp_f<0x143, 0xc>(0.f, v); // row_bcast:31 into rows 2,3
-    return v;
-}
-__device__ __forceinline__ float wave_min_all(float v)
-{
-    v = fminf(v, dpp_f<0xB1, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x4E, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x141, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x140, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x142, 0xa>(INFINITY, v));
-    v = fminf(v, dpp_f<0x143, 0xc>(INFINITY, v));
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-__device__ __forceinline__ float wave_max_all(float v) { return -wave_min_all(-v); }
-
-// ---------------------------------------------------------------------------
 // Per-lane queries through the skip links.
 //
 // First-hit query: optixTrace with SBT offset 0 (gaussians_aabb.cu:234-247, 300-313),
