@@ -79,6 +79,7 @@ struct MarchParams {
     uint32_t *records;      // hit-list record stream, rec_tile_words per tile, or null
     int32_t rec_tile_words;
     int32_t only_overflow;  // backward: handle only the tiles whose record overflowed
+    int32_t rec_pieces, rec_first, rec_equal, rec_turn; // the pieces of a tile's record (record_pieces)
     uint32_t *tile_order;   // launch order lists (or null: as launched)
     int32_t use_tile_order; // 0: as launched; 1: per XCD, its tiles' list positions from the heaviest to the lightest (k_tile_order);
                             // 2: per XCD, the blocks of tiles it renders, heaviest first (k_block_order)
@@ -596,12 +597,12 @@ __host__ __device__ __forceinline__ TileGrid tile_grid(int tiles_x, int tiles_y)
     g.per_xcd = (g.blocks_x * blocks_y + 7) >> 3;
     return g;
 }
-__device__ __forceinline__ bool tile_origin(const MarchParams &P, int &px0, int &py0, int *tile_out = nullptr)
+__device__ __forceinline__ bool tile_origin(const MarchParams &P, unsigned id, int &px0, int &py0, int *tile_out = nullptr)
 {
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
-    const int xcd = blockIdx.x & 7;
+    const int xcd = id & 7;
     const int per_block = g.bw * g.bh;
-    int j = blockIdx.x >> 3;
+    int j = id >> 3;
     int block;
     if (P.use_tile_order == 2) {
         block = (int)P.tile_order[xcd * g.per_xcd + j / per_block];
@@ -1025,7 +1026,8 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 // instead of sweeping the tree and evaluating the predicate again.  Per tile a region of
 // rec_tile_words 32-bit words:
 //   word 0: status (RGX_REC_COMPLETE, _OVERFLOWED, _COMPLETE_SUMS);  word 1: words used;
-//   from word 4, per iteration: WINDOW when a table was built, one LISTS per table, then TRAIL
+//   words 4 .. 4 + RGX_REC_PIECES_MAX: where a backward can start in the middle of a tile (below);
+//   from word RGX_REC_HEAD, per iteration: WINDOW when a table was built, one LISTS per table, then TRAIL
 //   WINDOW: {tag | C, -, -, -}, pid[pad4(C)]            the table's Gaussians, by slot
 //   LISTS:  {tag | last << 8 | nw, len[4], -, -, -}, slot bytes of row r in pad4(len[r]) / 4 words
 //           for r = 0..3, mask[nw][64], half[2][4][nw]   (the TileLds arrays of the same names;
@@ -1057,6 +1059,40 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 #define RGX_REC_WINDOW 0x57000000u
 #define RGX_REC_LISTS 0x4C000000u
 #define RGX_REC_TRAIL 0x54000000u
+// Pieces of a tile's record.  A tile is a serial march for the forward, but with the rays' state at a few of its
+// iterations (transmittance, colour so far, position, step) the backward can replay the stretches between
+// them side by side, each with a wavefront of its own: a launch no longer lasts as long as its longest tile.
+// A piece ends once it has enough blending iterations, where a new window begins anyway or it has become half as long
+// again (the next one then begins with the resident window's WINDOW item once more).  The states, state[piece][8][64],
+// go to a slot of the sample-sum pool; word 4 of the tile's region: how many | slot << 8, words 5 ..: where in the
+// region the iterations of the pieces after the first begin.
+// How many, and how long, by the number of tiles (3072 wavefronts are resident at a time):
+//   up to half of that: up to 16 short pieces, to fill the chip (4 k Gaussians, 128x128: 0.61 -> 0.17 ms);
+//   beyond: up to 8, the first two 4 iterations long and each later one half as long again, so that short and
+//     long tiles alike have several (300 k Gaussians, 800x800: 3.24 -> 2.94 ms; 1 M: 6.46 -> 6.29);
+//   beyond four rounds of tiles the end of a launch is a small part of it, and what a piece costs (its state, its window
+//     set up and flushed once more) weighs as much: none (3 M, 1237x822: 15.1 ms, 15.5 with pieces from 4 iterations, 14.8
+//     with pieces from 8, but 0.2 more in the forward).
+#define RGX_REC_PIECES_MAX 16
+#define RGX_REC_HEAD (4 + RGX_REC_PIECES_MAX)
+#define RGX_REC_STATE_WORDS (8 * 64)
+static_assert((RGX_REC_PIECES_MAX - 1) * RGX_REC_STATE_WORDS <= RGX_SUM_SLOT_WORDS, "a slot holds the states of a tile");
+struct RecordPieces {
+    int most;  // pieces
+    int first; // blending iterations of the first ones
+    int equal; // as many as this have that length; then they grow
+    bool turn; // the XCDs replay different pieces at a time
+};
+static inline RecordPieces record_pieces(int tiles)
+{
+    if (tiles <= 1536) return {RGX_REC_PIECES_MAX, 2, 8, false};
+    // (up to two rounds of tiles, the deepest pieces of all tiles would run at once, and add to the same few far
+    // Gaussians: 150 k Gaussians, 619x411: 1.82 ms, turned 1.62.  The pieces that one XCD replays at a time stay at
+    // one depth: its L2 holds the Gaussians of one depth, not of all (1 M, 800x800: 6.3 ms, 9.7 with mixed depths).)
+    if (tiles <= 2 * 3072) return {RGX_REC_PIECES_MAX / 2, 4, 2, true};
+    if (tiles <= 4 * 3072) return {RGX_REC_PIECES_MAX / 2, 4, 2, false};
+    return {1, 0, 0, false};
+}
 
 // Words 2 and 3 of a tile's region name the launch the record belongs to (number of Gaussians,
 // image size, step), so that a backward handed a record of another scene or view recomputes the
@@ -1086,6 +1122,10 @@ struct Recorder {
     bool ovf;       // the region is exhausted
     bool sums;      // every blending iteration so far got a sample-sum slot
     int slot;       // the current iteration's sample-sum slot, or -1
+    int length;     // blending iterations of the current piece after which the next one is due
+    int states = 0;      // states kept: pieces before the current one
+    int state_slot = -1; // where
+    int since = 0;       // blending iterations of the current piece
     uint32_t batch_next = 0; // the next slot of the batch this tile last took from the pool
     int batch_left = 0;      // slots left in that batch
     __device__ __forceinline__ bool on() const { return reg != nullptr && !ovf; }
@@ -1094,6 +1134,46 @@ struct Recorder {
     {
         if (off + size + 72 > cap) ovf = true;
         return !ovf;
+    }
+
+    // A slot of the pool, or -1 where it is empty.
+    // (RGX_SUM_SLOT_BATCH slots per request: a request is a round trip to one counter that every tile of the
+    // launch shares, and where iterations are short the tiles spend a good part of their time waiting on it)
+    __device__ __forceinline__ int take_slot(const MarchParams &P)
+    {
+        if (batch_left == 0) {
+            uint32_t s = 0;
+            if (threadIdx.x == 0) s = atomicAdd(P.sum_next, (uint32_t)RGX_SUM_SLOT_BATCH);
+            batch_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
+            batch_left = RGX_SUM_SLOT_BATCH;
+        }
+        const uint32_t s = batch_next++;
+        --batch_left;
+        return s < (uint32_t)P.sum_slots ? (int)s : -1;
+    }
+
+    // Does the next piece begin with this iteration?  reuse: the iteration goes on with the resident window.
+    __device__ __forceinline__ bool piece_due(const MarchParams &P, bool reuse) const
+    {
+        return since >= (reuse ? length + (length >> 1) : length) && states < P.rec_pieces - 1 && on() && sums;
+    }
+    __device__ __forceinline__ void begin_piece(const MarchParams &P, const RayState &R, float Cr, float Cg, float Cb)
+    {
+        if (state_slot < 0) {
+            state_slot = take_slot(P);
+            if (state_slot < 0) {
+                sums = false; // the pool is empty
+                return;
+            }
+        }
+        if (threadIdx.x == 0) reg[5 + states] = (uint32_t)off;
+        float *st = (float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + states * RGX_REC_STATE_WORDS + threadIdx.x;
+        st[0] = R.T; st[64] = R.tbuffer; st[2 * 64] = R.tenter; st[3 * 64] = R.dt;
+        st[4 * 64] = Cr; st[5 * 64] = Cg; st[6 * 64] = Cb;
+        ((uint32_t *)st)[7 * 64] = (R.active ? 1u : 0u) | (R.searching ? 2u : 0u) | (R.first ? 4u : 0u);
+        ++states;
+        since = 0;
+        if (states >= P.rec_equal) length += (length + 1) >> 1;
     }
 
     __device__ __forceinline__ void write_window(const TileLds &L, int C)
@@ -1135,20 +1215,12 @@ struct Recorder {
     {
         slot = -1;
         if (!on()) return;
+        since += blends ? 1 : 0;
         if (blends && P.sum_next) {
             // every blending iteration asks, also those of a tile that has gone without once: the counter then
             // ends at the launch's whole demand, which is what the next record of this view's shape is sized from
-            // (RGX_SUM_SLOT_BATCH slots per request: a request is a round trip to one counter that every tile of the
-            // launch shares, and where iterations are short the tiles spend a good part of their time waiting on it)
-            if (batch_left == 0) {
-                uint32_t s = 0;
-                if (threadIdx.x == 0) s = atomicAdd(P.sum_next, (uint32_t)RGX_SUM_SLOT_BATCH);
-                batch_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
-                batch_left = RGX_SUM_SLOT_BATCH;
-            }
-            const uint32_t s = batch_next++;
-            --batch_left;
-            if (sums && s < (uint32_t)P.sum_slots) slot = (int)s;
+            const int s = take_slot(P);
+            if (sums && s >= 0) slot = s;
             else sums = false;
         }
         uint32_t *it = reg + off;
@@ -1166,6 +1238,7 @@ struct Recorder {
         if (reg && threadIdx.x == 0) {
             reg[0] = ovf ? RGX_REC_OVERFLOWED : (sums ? RGX_REC_COMPLETE_SUMS : RGX_REC_COMPLETE);
             reg[1] = (uint32_t)off;
+            reg[4] = (uint32_t)states | (uint32_t)max(state_slot, 0) << 8;
             reg[2] = record_mark(P, 0);
             reg[3] = record_mark(P, 1);
         }
@@ -1732,9 +1805,9 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
     static_assert(RECORD || !HALF, "the colour sums' format is a property of the record");
     RGX_TILE_LDS();
     int px0, py0, tile;
-    if (!tile_origin(P, px0, py0, &tile)) return; // whole wave
+    if (!tile_origin(P, blockIdx.x, px0, py0, &tile)) return; // whole wave
     typename std::conditional<RECORD, Recorder, NoRecorder>::type rec;
-    if constexpr (RECORD) rec = Recorder{P.records + (int64_t)tile * P.rec_tile_words, 4, P.rec_tile_words, false, P.sum_pool != nullptr, -1};
+    if constexpr (RECORD) rec = Recorder{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
     int px, py;
     lane_pixel(px0, py0, px, py);
     const bool valid = px < P.cam.width && py < P.cam.height;
@@ -1758,6 +1831,15 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
         float found = -1.0f, searched_to = 0.f;
         if (__any(need || (R.active && R.searching))) {
             const float dt = R.dt;
+            if constexpr (RECORD) {
+                if (rec.piece_due(P, false)) {
+                    const bool reuse = Wn.resident && wave_max_all(need || (R.active && R.searching) ? thi : -INFINITY) <= Wn.hi;
+                    if (rec.piece_due(P, reuse)) {
+                        rec.begin_piece(P, R, Cr, Cg, Cb);
+                        if (reuse) rec.write_window(L, Wn.n);
+                    }
+                }
+            }
             float sg[RGX_CHUNK_SIZE], cr[RGX_CHUNK_SIZE], cg[RGX_CHUNK_SIZE], cb[RGX_CHUNK_SIZE];
 #pragma unroll
             for (int i = 0; i < RGX_CHUNK_SIZE; ++i) sg[i] = cr[i] = cg[i] = cb[i] = 0.f;
@@ -1980,12 +2062,17 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     static_assert(REPLAY || !SUMS, "sample sums come with a record");
     static_assert(SUMS || !HALF, "the colour sums' format is a property of the sample sums");
     int px0, py0, tile;
-    if (!tile_origin(P, px0, py0, &tile)) return; // whole wave
+    // A launch that replays sample sums has a grid for every piece of the tiles' records, the last (longest) pieces first.
+    const unsigned grid = SUMS ? gridDim.x / (unsigned)P.rec_pieces : gridDim.x;
+    const int turn = P.rec_turn ? (int)(blockIdx.x & 7) : 0; // (the workgroup's XCD)
+    const int piece = SUMS ? (2 * P.rec_pieces - 1 - (int)(blockIdx.x / grid) - turn) % P.rec_pieces : 0;
+    if (!tile_origin(P, SUMS ? blockIdx.x % grid : blockIdx.x, px0, py0, &tile)) return; // whole wave
     const uint32_t *reg = P.records ? P.records + (int64_t)tile * P.rec_tile_words : nullptr;
     if (REPLAY) {
         // overflowed, not this launch's, or with / without sample sums: another kernel handles the tile
         if (record_status(P, reg) != (SUMS ? RGX_REC_COMPLETE_SUMS : RGX_REC_COMPLETE)) return;
         if (SUMS && HALF != (P.m.record_format == 1)) return; // (the launcher picks the variant of the record's format)
+        if (SUMS && piece > (int)(uni_u32(reg[4]) & 0xffu)) return; // the record has fewer pieces
     } else if (P.only_overflow) {
         if (record_usable(P, reg)) return; // replayed
     }
@@ -2233,9 +2320,30 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
 
     RGX_SEC(cn, RGX_SEC_SETUP);
     if constexpr (REPLAY) {
-        const int used = min((int)uni_u32(reg[1]), P.rec_tile_words);
-        Replayer<SUMS> rp = {RecordView<SUMS>{reg, s_stage, -(1 << 30), used}, 4, -1, false, RL};
-        while (__any(R.active) && !rp.lost) {
+        int used = min((int)uni_u32(reg[1]), P.rec_tile_words), start = RGX_REC_HEAD;
+        if constexpr (SUMS) {
+            const int states = (int)(uni_u32(reg[4]) & 0xffu);
+            if (piece < states && piece + 1 < P.rec_pieces) used = min((int)uni_u32(reg[5 + piece]), used);
+            const uint32_t state_slot = uni_u32(reg[4]) >> 8;
+            if (piece > 0 && state_slot < (uint32_t)P.sum_slots) {
+                // the piece starts with the state the forward had there; what the loss's gradient still sees of the ray's
+                // colour is what the forward had not yet added to it
+                start = min((int)uni_u32(reg[5 + piece - 1]), used);
+                const float *st = (const float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + (piece - 1) * RGX_REC_STATE_WORDS + lane;
+                R.T = st[0];
+                R.tbuffer = st[64];
+                R.tenter = st[2 * 64];
+                R.dt = st[3 * 64];
+                R.slab_spacing = R.dt * RGX_BUFFER_SIZE;
+                D -= dot3(g, mk3(st[4 * 64], st[5 * 64], st[6 * 64]));
+                const uint32_t flags = ((const uint32_t *)st)[7 * 64];
+                R.active = flags & 1u;
+                R.searching = flags & 2u;
+                R.first = flags & 4u;
+            }
+        }
+        Replayer<SUMS> rp = {RecordView<SUMS>{reg, s_stage, -(1 << 30), used}, start, -1, false, RL};
+        while (__any(R.active) && !rp.lost && (!SUMS || rp.at < used)) {
             iteration([&](bool need, float, float, int &p0, bool &, float &found, float &searched_to, auto a, auto mid, auto b) {
                 return rp.template slab<SUMS>(P, R, need, p0, found, searched_to, cn, a, mid, b);
             });
@@ -2451,7 +2559,7 @@ __global__ __launch_bounds__(64) void k_collect_tiles(const MarchParams P, const
 {
     RGX_TILE_LDS();
     int px0, py0;
-    if (!tile_origin(P, px0, py0)) return;
+    if (!tile_origin(P, blockIdx.x, px0, py0)) return;
     const int lane = threadIdx.x;
     int px, py;
     lane_pixel(px0, py0, px, py);
@@ -2606,6 +2714,11 @@ static int fill_params(MarchParams &P, const void *ws, const RgxCamera *cam, con
     P.records = nullptr;
     P.rec_tile_words = 0;
     P.only_overflow = 0;
+    const RecordPieces rp = record_pieces(P.tiles_x * P.tiles_y);
+    P.rec_pieces = march->record_format == 1 ? min(rp.most, RGX_SUM_SLOT_WORDS_HALF / RGX_REC_STATE_WORDS + 1) : rp.most;
+    P.rec_first = rp.first;
+    P.rec_equal = rp.equal;
+    P.rec_turn = rp.turn;
     // room for the tile order?  (a workspace sized for fewer rays, or an image of extreme proportions, goes without)
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const size_t order_words = (size_t)8 * g.per_xcd * g.bw * g.bh;
@@ -2840,7 +2953,8 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
             hipLaunchKernelGGL(k_tile_order, dim3(8), dim3(256), 0, s, P);
             P.use_tile_order = 1;
         }
-        if (P.sum_pool) rgx_launch_march_bwd(RGX_BWD_SUMS, stats != nullptr, P.m.record_format == 1, march_grid(P), s, P);
+        if (P.sum_pool)
+            rgx_launch_march_bwd(RGX_BWD_SUMS, stats != nullptr, P.m.record_format == 1, dim3(march_grid(P).x * (unsigned)P.rec_pieces), s, P);
         rgx_launch_march_bwd(RGX_BWD_LISTS, stats != nullptr, false, march_grid(P), s, P);
         P.only_overflow = 1;
         P.use_tile_order = 0;

@@ -411,6 +411,25 @@ def test_dynamic_sampling_lobes_supersampling_black_background(gx, orc):
                                              "sph_gauss_features", "bandwidth_sharpness", "lobe_axis"))
 
 
+@pytest.mark.parametrize("w,h,half", [(52, 44, True), (321, 307, False), (321, 307, True)])
+def test_backward_in_pieces_equals_recomputation(gx, w, h, half):
+    """The record of a tile cut into pieces that are replayed side by side, each from the rays' state that the
+    forward kept: few tiles (up to 16 pieces; 11 with half-precision sums, whose slots hold fewer states) and
+    between half a round and two rounds of tiles (up to 8, the XCDs at different pieces)."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(2, n=5000, sh_degree=1, seed=21))
+    sc["scales"] = sc["scales"] * 3.0
+    cam = scenes.make_camera(2, 1, width=w, height=h)
+    cfg = dict(dt_step=0.004, dynamic_sampling=True, max_prim_slice=4096)
+    dloss = np.random.default_rng(3).normal(size=(w * h, 3)).astype(np.float32)
+    _step(f"pieces {w}x{h} half={half}")
+    a = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    b = gx.gpu_render(sc, cam, cfg, want_grad=dloss, half_sums=half)
+    assert b["stats_bwd"]["nodes_visited"] == 0 and a["stats_bwd"]["hit_pairs"] == b["stats_bwd"]["hit_pairs"] > 10000
+    for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+        cos, rel = gx.cos_rel(b["grads"][k], a["grads"][k])
+        assert cos >= 1 - 1e-6 and rel <= (1e-3 if half else 1e-4), (k, cos, rel)
+
+
 def test_long_hit_lists_spill_and_truncation(gx, orc):
     """Fat Gaussians: slabs with far more than 32 hits (LDS part + spill area), then a tiny
     max_prim_slice to exercise the silent truncation path and its counter."""
