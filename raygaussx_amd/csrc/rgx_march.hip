@@ -1981,6 +1981,889 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
     RGX_SEC_FLUSH(cn, RECORD ? RGX_SECK_FWD_RECORD : RGX_SECK_FWD_PLAIN);
 }
 
+// ---------------------------------------------------------------------------
+// The forward with four wavefronts per tile.  One wavefront per tile leaves most of the chip idle where an image has
+// few tiles, and ends every launch in a tail as long as one tile's serial march.  Here a workgroup of four marches the
+// tile: wavefront w has the 16 rays of the tile's 4x4 block w, each ray four times over (lane = 16 * sub + ray), and
+// the four copies share the ray's work -- in the filter they test four table entries at a time, in the shading
+// every fourth hit each; the copies' sample sums are then added up across the wavefront's rows (permlane swaps) so that
+// copy `sub` ends up with samples 4 sub .. 4 sub + 3 of the half, and blends those.  The tree is swept by all four wavefronts, 256 nodes or leaves at a time, into one table for the tile.
+// A record is written in the same format, 4x4 block by block.
+// Bound by the latency of the march's chain of slabs: an iteration costs a wavefront some 9 000 clocks, of which the
+// filter 0.27, the lists and the barriers around them 0.21, shading 0.13, the sweep 0.12 and the blend 0.11 (4 k
+// Gaussians, 128x128).  Two wavefronts per SIMD: up to 512 tiles are resident at once, and nothing is spilled.
+#define RGX_TEAM_QCAP 1024
+#define RGX_TEAM_DFS_MARGIN 96 // (see RGX_DFS_MARGIN: a step pops at most as many nodes as leave this margin free)
+template <int CAP>
+struct TeamShared {
+    static constexpr int WORDS = (CAP + 31) / 32;
+    float tab[CAP * RGX_TAB];
+    int32_t queue[RGX_TEAM_QCAP];
+    int32_t leafq[512];
+    uint32_t mask[WORDS][3][4][16]; // hits over the block's list: all, with samples in the first / second half
+    uint32_t cnt[4];                // a sweep step's counts
+    float4 red[2][4];               // team_exchange
+    int32_t msg[8];                 // list lengths; [4]: the batch of sample-sum slots taken
+    uint8_t rowlist[4][(CAP + 3) & ~3];
+    uint8_t rel[4][(CAP + 3) & ~3];
+};
+struct TeamPos {
+    int wave, lane, sub, ray;
+};
+
+// What the four wavefronts have to agree on: minimum, two maxima, OR.  The barrier in here also ends every
+// wavefront's use of what was in the shared memory before it.
+struct TeamWord {
+    float lo, hi, ahead;
+    uint32_t flags;
+};
+template <int CAP>
+__device__ __forceinline__ TeamWord team_exchange(TeamShared<CAP> &S, const TeamPos &tp, int &turn, float lo, float hi, float ahead, uint32_t flags)
+{
+    if (tp.lane == 0) S.red[turn][tp.wave] = make_float4(lo, hi, ahead, __uint_as_float(flags));
+    __syncthreads();
+    const float4 a = S.red[turn][0], b = S.red[turn][1], c = S.red[turn][2], d = S.red[turn][3];
+    turn ^= 1;
+    auto uni = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
+    return {uni(fminf(fminf(a.x, b.x), fminf(c.x, d.x))), uni(fmaxf(fmaxf(a.y, b.y), fmaxf(c.y, d.y))),
+            uni(fmaxf(fmaxf(a.z, b.z), fmaxf(c.z, d.z))),
+            uni_u32(__float_as_uint(a.w) | __float_as_uint(b.w) | __float_as_uint(c.w) | __float_as_uint(d.w))};
+}
+// minimum / maximum over a row of 16 lanes, all rows holding the same values
+__device__ __forceinline__ float row_min_all(float v)
+{
+    v = fminf(v, dpp_f<0xB1, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x4E, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x141, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x140, 0xf>(INFINITY, v));
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ __forceinline__ float row_max_all(float v) { return -row_min_all(-v); }
+
+// a's upper 32 lanes and b's lower 32 lanes change places; the same with the rows of 16 of each half
+__device__ __forceinline__ void swap32(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+// the value of each of the four copies of a ray, in every copy
+__device__ __forceinline__ void copies(float v, float (&out)[4])
+{
+    float a = v, b = v; // -> a: copies 0 and 1 (in the lower and upper rows of both halves), b: copies 2 and 3
+    swap32(a, b);
+    float a1 = a, b1 = b;
+    swap16(a, a1);
+    swap16(b, b1);
+    out[0] = a; out[1] = a1; out[2] = b; out[3] = b1;
+}
+// 16 values per lane -> four: copy `sub` gets the sums over the copies of v[4 sub .. 4 sub + 3]
+__device__ __forceinline__ void sum_copies(float (&v)[RGX_CHUNK_SIZE], float (&out)[4])
+{
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        swap32(v[i], v[i + 8]);
+        v[i] += v[i + 8];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        swap16(v[i], v[i + 4]);
+        out[i] = v[i] + v[i + 4];
+    }
+}
+
+// What a leaf whose box passed turns into: its ellipsoid against the frustum, and its table entry (as in sweep_next,
+// whose kernels have no register for a function that returns one).
+struct LeafEntry {
+    f3 U, V, W, inv, Oe;
+    float dmin, dmax, k, c;
+    bool plain; // passed plain_roots()
+    __device__ __forceinline__ void store(float4 *dst, int32_t left) const
+    {
+        dst[0] = make_float4(U.x, U.y, U.z, dmin);
+        dst[1] = make_float4(V.x, V.y, V.z, dmax);
+        dst[2] = make_float4(W.x, W.y, W.z, k);
+        dst[3] = make_float4(inv.x, inv.y, inv.z, c);
+        dst[4] = make_float4(Oe.x, Oe.y, Oe.z, __int_as_float(~left));
+    }
+};
+__device__ __forceinline__ bool leaf_entry(const MarchParams &P, const Frustum &F, int32_t left, LeafEntry &e)
+{
+    const Prim p = P.prims[~left];
+    quat_to_cols(p.quat4, e.U, e.V, e.W);
+    const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
+    // semi-axes of the k-sigma ellipsoid: k * scale = 1 / inv_inter
+    // (bounds only: hardware reciprocal and square root, their last-bit error is inside the 1.001 factors)
+    const f3 ax = mk3(__builtin_amdgcn_rcpf(p.inv_inter4.x), __builtin_amdgcn_rcpf(p.inv_inter4.y), __builtin_amdgcn_rcpf(p.inv_inter4.z));
+    const float dist = __builtin_amdgcn_sqrtf(dot3(O, O));
+    const float amax = fmaxf(ax.x, fmaxf(ax.y, ax.z));
+    const float rad = amax * 1.001f + 1e-5f * dist + F.pad;
+    // Along a ray of direction d the ellipsoid lies within (centre - eye).d -+ |A R^T d|.  For
+    // d = dc that is depth -+ h; a ray at angle <= delta from dc moves the centre term by at
+    // most |depth| delta^2 / 2 + |offset of the centre from the central ray| delta and the
+    // extent by at most amax delta.  The bounding sphere's shell bounds the same range.
+    const float depth = -dot3(O, F.dc);
+    const f3 off = mk3(-O.x - depth * F.dc.x, -O.y - depth * F.dc.y, -O.z - depth * F.dc.z);
+    const float eu = dot3(e.U, F.dc) * ax.x, ev = dot3(e.V, F.dc) * ax.y, ew = dot3(e.W, F.dc) * ax.z;
+    const float ext = __builtin_amdgcn_sqrtf((eu * eu + ev * ev) + ew * ew) * 1.001f;
+    const float slack = 1.5f * (0.5f * fabsf(depth) * F.delta * F.delta + (__builtin_amdgcn_sqrtf(dot3(off, off)) + amax) * F.delta) +
+                        1e-5f * dist + F.pad;
+    e.dmin = fmaxf(dist - rad, depth - ext - slack);
+    e.dmax = fminf(dist + rad, depth + ext + slack);
+    bool ok = p.inv_inter4.w == p.inv_inter4.w; // k is NaN below the density threshold: never hit
+    ok = ok && e.dmax >= F.t0 && e.dmin <= F.t1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const f3 n = F.n[k];
+        // the ellipsoid reaches h beyond its centre along n; centre - eye = -O
+        const float hu = dot3(e.U, n) * ax.x, hv = dot3(e.V, n) * ax.y, hw = dot3(e.W, n) * ax.z;
+        const float h = __builtin_amdgcn_sqrtf((hu * hu + hv * hv) + hw * hw) * 1.001f;
+        ok = ok && !(-dot3(n, O) - h > F.pad);
+    }
+    if (ok) {
+        e.k = p.inv_inter4.w;
+        e.inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
+        e.Oe = apply_sinv_rt(O, e.U, e.V, e.W, e.inv);
+        e.c = fmaf(e.Oe.x, e.Oe.x, fmaf(e.Oe.y, e.Oe.y, fmaf(e.Oe.z, e.Oe.z, -1.0f)));
+        e.plain = plain_roots(e.inv, e.c);
+    }
+    return ok;
+}
+
+template <int CAP>
+__device__ __forceinline__ void team_sweep_begin(const MarchParams &P, Sweep &S, const Frustum &F, TeamShared<CAP> &T)
+{
+    S.lqn = 0;
+    if (F.cut_n > 0) {
+        S.qn = F.cut_n;
+        if ((int)threadIdx.x < F.cut_n) T.queue[threadIdx.x] = F.cut_node;
+    } else {
+        S.qn = P.n > 0 ? 1 : 0;
+        if (threadIdx.x == 0) T.queue[0] = 0;
+    }
+    __syncthreads();
+}
+
+// exclusive sum over the team's wavefronts of a 16-bit count in each half of a word, and the totals; two barriers have to
+// separate one call's word from the next one's (the caller's own barrier is the second)
+template <int CAP>
+__device__ __forceinline__ void team_counts(TeamShared<CAP> &T, const TeamPos &tp, uint32_t mine, uint32_t &before, uint32_t &total)
+{
+    if (tp.lane == 0) T.cnt[tp.wave] = mine;
+    __syncthreads();
+    const uint32_t c0 = T.cnt[0], c1 = T.cnt[1], c2 = T.cnt[2], c3 = T.cnt[3];
+    before = uni_u32((tp.wave > 0 ? c0 : 0u) + (tp.wave > 1 ? c1 : 0u) + (tp.wave > 2 ? c2 : 0u));
+    total = uni_u32(c0 + c1 + c2 + c3);
+}
+
+// frustum_cut by the team: at most 256 nodes, one per lane
+template <int CAP>
+__device__ __forceinline__ void team_frustum_cut(const MarchParams &P, Frustum &F, float t_far, TeamShared<CAP> &T, const TeamPos &tp)
+{
+    const uint64_t lt = (1ull << tp.lane) - 1ull;
+    const float4 *nodes4 = (const float4 *)P.nodes;
+    const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
+    F.t0 = 0.f;
+    F.t1 = INFINITY;
+    F.pad = 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f);
+    int32_t node = threadIdx.x == 0 && P.n > 0 ? 0 : -1;
+    int count = P.n > 0 ? 1 : 0;
+    for (int level = 0; level < 64 && count > 0; ++level) {
+        bool keep = false, inner = false;
+        int32_t left = 0, right = 0;
+        if ((uint32_t)node < n_nodes) {
+            const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
+            right = P.right[max(0, min(node, (int32_t)P.n - 2))];
+            if (frustum_overlaps(F, a, b)) {
+                left = __float_as_int(a.w);
+                inner = left >= 0;
+                keep = !inner;
+            }
+        }
+        const uint64_t bk = __ballot(keep), bi = __ballot(inner);
+        uint32_t before, total;
+        team_counts(T, tp, (uint32_t)__popcll(bk) | (uint32_t)__popcll(bi) << 16, before, total);
+        const int kept = total & 0xffff, opened = total >> 16, next = kept + 2 * opened;
+        if (opened == 0 || next > 256) break;
+        if (keep) T.queue[(before & 0xffff) + __popcll(bk & lt)] = node;
+        if (inner) {
+            const int at = kept + 2 * ((int)(before >> 16) + __popcll(bi & lt));
+            T.queue[at] = left;
+            T.queue[at + 1] = right;
+        }
+        __syncthreads();
+        node = (int)threadIdx.x < next ? T.queue[threadIdx.x] : -1;
+        count = next;
+    }
+    F.cut_n = count;
+    F.cut_node = node;
+    __syncthreads();
+}
+
+// sweep_next by the team
+template <int CAP, typename Cn>
+__device__ int team_sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, TeamShared<CAP> &T, const TeamPos &tp, bool &done, bool &plain,
+                               Cn &cn)
+{
+    plain = true;
+    const uint64_t lt = (1ull << tp.lane) - 1ull;
+    const float4 *nodes4 = (const float4 *)P.nodes;
+    const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
+    int C = 0;
+    while ((S.qn > 0 || S.lqn > 0) && C < CAP) {
+        if (S.lqn >= 256 || S.qn == 0) {
+            const int m = S.lqn < 256 ? S.lqn : 256;
+            const bool mine = (int)threadIdx.x < m;
+            const int32_t left = mine ? T.leafq[S.lqn - m + threadIdx.x] : 0;
+            S.lqn -= m;
+            LeafEntry e;
+            const bool hit = mine && leaf_entry(P, F, left, e);
+            const uint64_t bl = __ballot(hit), rough = __ballot(hit && !e.plain);
+            uint32_t before, total;
+            team_counts(T, tp, (uint32_t)__popcll(bl) | (rough ? 0x10000u : 0u), before, total);
+            const int hits = total & 0xffff, room = CAP - C, rank = (int)(before & 0xffff) + __popcll(bl & lt);
+            plain = plain && (total >> 16) == 0;
+            if (hit) {
+                if (rank < room) e.store((float4 *)(T.tab + (C + rank) * RGX_TAB), left);
+                else T.leafq[S.lqn + rank - room] = left; // no room: back to the queue, for the next table
+            }
+            C += hits < room ? hits : room;
+            S.lqn += hits < room ? 0 : hits - room;
+            __syncthreads();
+            continue;
+        }
+        const int spare = RGX_TEAM_QCAP - RGX_TEAM_DFS_MARGIN - S.qn;
+        const int m = min(min(S.qn, 256), max(spare, 1));
+        const int base = S.qn - m;
+        int32_t node = -1;
+        if ((int)threadIdx.x < m) node = T.queue[base + threadIdx.x];
+        bool leaf_hit = false, inner_hit = false;
+        int32_t left = 0, right = 0;
+        if ((uint32_t)node < n_nodes) {
+            const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
+            right = P.right[max(0, min(node, (int32_t)P.n - 2))];
+            if (frustum_overlaps(F, a, b)) {
+                left = __float_as_int(a.w);
+                leaf_hit = left < 0;
+                inner_hit = !leaf_hit;
+            }
+        }
+        if (threadIdx.x == 0) cn.nodes += (unsigned)m;
+        const uint64_t bl = __ballot(leaf_hit), bi = __ballot(inner_hit);
+        uint32_t before, total;
+        team_counts(T, tp, (uint32_t)__popcll(bl) | (uint32_t)__popcll(bi) << 16, before, total); // (every node has been read)
+        if (leaf_hit) T.leafq[S.lqn + (before & 0xffff) + __popcll(bl & lt)] = left; // fewer than 256 waiting + at most 256 new
+        S.lqn += (int)(total & 0xffff);
+        if (inner_hit) {
+            const int pos = base + 2 * ((int)(before >> 16) + __popcll(bi & lt));
+            if (pos + 1 < RGX_TEAM_QCAP) {
+                T.queue[pos] = right;
+                T.queue[pos + 1] = left;
+            } else if (P.faults) {
+                atomicAdd(&P.faults[1], 1u);
+            }
+        }
+        S.qn = min(base + 2 * (int)(total >> 16), RGX_TEAM_QCAP);
+        __syncthreads();
+    }
+    done = S.qn == 0 && S.lqn == 0;
+    return C;
+}
+
+// filter_table for a block's 16 rays, four entries at a time.  len: the block's list length (wave-uniform); first, second:
+// this ray's masks over the list's first 32 entries.
+template <bool SEARCH, int PART, bool PLAIN, int CAP, typename Cn>
+__device__ __forceinline__ void team_filter(TeamShared<CAP> &T, const TeamPos &tp, int C, float t0, float t1, const LaneQuery &Q, int &p0, bool &ov,
+                                            float &found, int &len, uint32_t (&own)[2], Cn &cn)
+{
+    len = 0;
+    own[0] = own[1] = 0u;
+    // the entries whose shell meets the block's range
+    int nrel = 0;
+    for (int h = 0; h < CAP; h += 64) {
+        const int c = h + tp.lane;
+        bool rel = false;
+        if (c < C) rel = T.tab[c * RGX_TAB + 7] >= t0 && T.tab[c * RGX_TAB + 3] <= t1;
+        const uint64_t b = __ballot(rel);
+        if (rel) T.rel[tp.wave][nrel + __popcll(b & ((1ull << tp.lane) - 1ull))] = (uint8_t)c;
+        nrel += __popcll(b);
+    }
+    if (tp.lane == 0) cn.cands += (unsigned)nrel;
+    __builtin_amdgcn_wave_barrier();
+    uint32_t bits = 0, first = 0, second = 0;
+    auto flush = [&](int w) {
+        if (tp.sub == 0) {
+            T.mask[w][0][tp.wave][tp.ray] = bits;
+            T.mask[w][1][tp.wave][tp.ray] = first;
+            T.mask[w][2][tp.wave][tp.ray] = second;
+        }
+        if (w == 0) {
+            own[0] = first;
+            own[1] = second;
+        }
+        bits = first = second = 0;
+    };
+    // max_prim_slice cuts a ray's list in the order of the entries: where it could, one entry at a time
+    const int step = __any(p0 + nrel > Q.cap) ? 1 : 4;
+    for (int i = 0; i < nrel; i += step) {
+        const bool there = tp.sub < step && i + tp.sub < nrel;
+        const int c = there ? T.rel[tp.wave][i + tp.sub] : 0;
+        float r1, r2;
+        constexpr bool EXIT = std::is_same<Cn, NoCounters>::value;
+        const bool ok = lane_roots<PLAIN, EXIT>((const float4 *)(T.tab + c * RGX_TAB), Q.dir, r1, r2) && there;
+        if constexpr (EXIT) {
+            if (!__any(ok)) continue;
+        }
+        if constexpr (SEARCH) {
+            const float ts = fmaxf(Q.slo, r1);
+            const bool sfound = Q.search && ok && ts <= fminf(Q.shi, r2);
+            found = sfound ? (found < 0.0f ? ts : fminf(found, ts)) : found;
+        }
+        const bool seg = Q.need && !(SEARCH && Q.search) && !ov && ok && fmaxf(Q.tlo, r1) <= fminf(Q.thi, r2);
+        const bool f = r1 < Q.tmid, g = r2 > Q.tmid;
+        bool hit = seg && (PART == 0 || (PART == 1 ? f : g));
+        const bool counts = PART != 2 || !f;
+        if (step == 1) { // (copy 0 decides for all)
+            const bool over = seg && counts && p0 >= Q.cap;
+            hit = hit && !over;
+            const uint64_t bo = __ballot(over);
+            ov = ov || ((uint32_t)bo >> tp.ray & 1u);
+        }
+        const uint64_t bh = __ballot(hit);
+        if (bh == 0) continue;
+        if (tp.lane == 0) cn.cands_hit++;
+        const uint64_t bf = __ballot(hit && f), bg = __ballot(hit && g), bc = __ballot(hit && counts);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const uint32_t h = (uint32_t)(bh >> (16 * s)) & 0xffffu;
+            if (h == 0) continue;
+            const int at = len & 31;
+            bits |= (h >> tp.ray & 1u) << at;
+            first |= ((uint32_t)(bf >> (16 * s)) >> tp.ray & 1u) << at;
+            second |= ((uint32_t)(bg >> (16 * s)) >> tp.ray & 1u) << at;
+            p0 += (uint32_t)(bc >> (16 * s)) >> tp.ray & 1u;
+            if (tp.lane == 16 * s) T.rowlist[tp.wave][len] = (uint8_t)c;
+            ++len;
+            if ((len & 31) == 0) flush((len >> 5) - 1);
+        }
+    }
+    if (len & 31) flush(len >> 5);
+    if constexpr (SEARCH) {
+        float v[4];
+        copies(found < 0.0f ? INFINITY : found, v);
+        const float best = fminf(fminf(v[0], v[1]), fminf(v[2], v[3]));
+        found = best < INFINITY ? best : -1.0f;
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+// shade_lanes for a block: each copy of a ray takes every fourth of the ray's hits
+template <int CAP, typename Body>
+__device__ __forceinline__ void team_shade(const MarchParams &P, TeamShared<CAP> &T, const TeamPos &tp, int len, bool run, int half,
+                                           const uint32_t (&own)[2], Body body)
+{
+    const int nw = (len + 31) >> 5;
+    auto mine = [&](uint32_t bits) { // without the first `sub` hits
+        bits = tp.sub > 0 ? bits & (bits - 1u) : bits;
+        bits = tp.sub > 1 ? bits & (bits - 1u) : bits;
+        return tp.sub > 2 ? bits & (bits - 1u) : bits;
+    };
+    int w = 0;
+    uint32_t bits = run && nw > 0 ? mine(half ? own[1] : own[0]) : 0u;
+    for (;;) {
+        while (bits == 0u && run && w + 1 < nw) {
+            ++w;
+            bits = mine(T.mask[w][1 + half][tp.wave][tp.ray]);
+        }
+        const bool has = bits != 0u;
+        if (!__any(has)) break;
+        int c = 0;
+        if (has) {
+            c = T.rowlist[tp.wave][w * 32 + __builtin_ctz(bits)];
+            bits &= bits - 1u;
+            bits &= bits - 1u;
+            bits &= bits - 1u;
+            bits &= bits - 1u;
+        }
+        const float4 *tab = (const float4 *)(T.tab + c * RGX_TAB);
+        const int32_t pid = __float_as_int(T.tab[c * RGX_TAB + 19]);
+        body(Entry<true>{tab, P.prims + pid, pid, c}, has);
+    }
+}
+
+// Recorder for a team: all its lanes carry the same offsets and flags.
+struct TeamRecorder : Recorder {
+    template <int CAP>
+    __device__ __forceinline__ void window(const TeamShared<CAP> &T, int C)
+    {
+        if (!on() || !fits(4 + ((C + 3) & ~3))) return;
+        uint32_t *it = reg + off;
+        if (threadIdx.x == 0) it[0] = RGX_REC_WINDOW | (uint32_t)C;
+        for (int i = threadIdx.x; i < C; i += 256) it[4 + i] = __float_as_uint(T.tab[i * RGX_TAB + 19]);
+        off += 4 + ((C + 3) & ~3);
+    }
+    // the blocks' list lengths are in T.msg
+    template <int CAP>
+    __device__ __forceinline__ void lists(const TeamShared<CAP> &T, const TeamPos &tp, bool last)
+    {
+        if (!on()) return;
+        const int l0 = (int)uni_u32((uint32_t)T.msg[0] & 0xffffu), l1 = (int)uni_u32((uint32_t)T.msg[1] & 0xffffu);
+        const int l2 = (int)uni_u32((uint32_t)T.msg[2] & 0xffffu), l3 = (int)uni_u32((uint32_t)T.msg[3] & 0xffffu);
+        const int nw = (max(max(l0, l1), max(l2, l3)) + 31) >> 5;
+        const int q0 = (l0 + 3) >> 2, q1 = (l1 + 3) >> 2, q2 = (l2 + 3) >> 2, q3 = (l3 + 3) >> 2;
+        const int size = 8 + q0 + q1 + q2 + q3 + nw * 72;
+        if (!fits(size)) return;
+        uint32_t *it = reg + off;
+        if (threadIdx.x == 0) {
+            it[0] = RGX_REC_LISTS | (last ? 0x100u : 0u) | (uint32_t)nw;
+            it[1] = (uint32_t)l0; it[2] = (uint32_t)l1; it[3] = (uint32_t)l2; it[4] = (uint32_t)l3;
+        }
+        const int len = tp.wave == 0 ? l0 : tp.wave == 1 ? l1 : tp.wave == 2 ? l2 : l3;
+        const int base = 8 + (tp.wave > 0 ? q0 : 0) + (tp.wave > 1 ? q1 : 0) + (tp.wave > 2 ? q2 : 0);
+        const uint32_t *slots = (const uint32_t *)T.rowlist[tp.wave];
+        if (tp.lane < ((len + 3) >> 2)) it[base + tp.lane] = slots[tp.lane];
+        const int mbase = 8 + q0 + q1 + q2 + q3, words = (len + 31) >> 5;
+        // copy s of a ray writes word s, s + 4, ...; words past the block's own list are zero
+        for (int w = tp.sub; w < nw; w += 4) it[mbase + w * 64 + tp.wave * 16 + tp.ray] = w < words ? T.mask[w][0][tp.wave][tp.ray] : 0u;
+        // which entries reach each half for some ray of the block
+        for (int w = 0; w < nw; ++w)
+            for (int half = 0; half < 2; ++half) {
+                const uint32_t v = row_or(w < words ? T.mask[w][1 + half][tp.wave][tp.ray] : 0u);
+                if (tp.lane == 0) it[mbase + nw * 64 + (half * 4 + tp.wave) * nw + w] = v;
+            }
+        off += size;
+    }
+    // A slot from the pool: thread 0 asks, where the last batch is used up (a barrier in there, for all or for none).
+    template <int CAP>
+    __device__ __forceinline__ int team_slot(const MarchParams &P, TeamShared<CAP> &T)
+    {
+        if (batch_left == 0) {
+            if (threadIdx.x == 0) T.msg[4] = (int32_t)atomicAdd(P.sum_next, (uint32_t)RGX_SUM_SLOT_BATCH);
+            __syncthreads();
+            batch_next = uni_u32((uint32_t)T.msg[4]);
+            batch_left = RGX_SUM_SLOT_BATCH;
+        }
+        const uint32_t s = batch_next++;
+        --batch_left;
+        return s < (uint32_t)P.sum_slots ? (int)s : -1;
+    }
+    template <int CAP>
+    __device__ __forceinline__ void trailer(const MarchParams &P, TeamShared<CAP> &T, const TeamPos &tp, bool any_search, float cover, float found, bool blends)
+    {
+        slot = -1;
+        if (!on()) return;
+        since += blends ? 1 : 0;
+        if (blends && P.sum_next) {
+            const int s = team_slot(P, T);
+            if (sums && s >= 0) slot = s;
+            else sums = false;
+        }
+        uint32_t *it = reg + off;
+        if (threadIdx.x == 0) {
+            it[0] = RGX_REC_TRAIL | (any_search ? 1u : 0u);
+            it[1] = __float_as_uint(cover);
+            it[2] = (uint32_t)(slot + 1);
+        }
+        if (any_search && tp.sub == 0) it[4 + tp.wave * 16 + tp.ray] = __float_as_uint(found);
+        off += 4 + (any_search ? 64 : 0);
+    }
+    // Cr, Cg, Cb: the copies' shares of the ray's colour
+    template <int CAP>
+    __device__ __forceinline__ void piece(const MarchParams &P, TeamShared<CAP> &T, const TeamPos &tp, const RayState &R, float Cr, float Cg, float Cb)
+    {
+        if (state_slot < 0) {
+            state_slot = team_slot(P, T);
+            if (state_slot < 0) {
+                sums = false;
+                return;
+            }
+        }
+        if (threadIdx.x == 0) reg[5 + states] = (uint32_t)off;
+        float r[4], g[4], b[4];
+        copies(Cr, r);
+        copies(Cg, g);
+        copies(Cb, b);
+        if (tp.sub == 0) {
+            float *st = (float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + states * RGX_REC_STATE_WORDS + tp.wave * 16 + tp.ray;
+            st[0] = R.T; st[64] = R.tbuffer; st[2 * 64] = R.tenter; st[3 * 64] = R.dt;
+            st[4 * 64] = (r[0] + r[1]) + (r[2] + r[3]);
+            st[5 * 64] = (g[0] + g[1]) + (g[2] + g[3]);
+            st[6 * 64] = (b[0] + b[1]) + (b[2] + b[3]);
+            ((uint32_t *)st)[7 * 64] = (R.active ? 1u : 0u) | (R.searching ? 2u : 0u) | (R.first ? 4u : 0u);
+        }
+        ++states;
+        since = 0;
+        if (states >= P.rec_equal) length += (length + 1) >> 1;
+    }
+};
+
+#define RGX_TEAM_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool RECORD, bool VIEWER, bool STATS, bool HALF = false>
+__global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const MarchParams P)
+{
+    constexpr int CAP = RGX_CCAP;
+    static_assert(CAP <= 256, "a slot of the table is a byte");
+    __shared__ __align__(16) TeamShared<CAP> T;
+    int px0, py0, tile;
+    if (!tile_origin(P, blockIdx.x, px0, py0, &tile)) return; // whole workgroup
+    const int lane = threadIdx.x & 63;
+    const TeamPos tp = {__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane, lane >> 4, lane & 15};
+    typename std::conditional<RECORD, TeamRecorder, NoRecorder>::type rec;
+    if constexpr (RECORD) rec = TeamRecorder{{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first}};
+    const int px = px0 + (tp.wave & 1) * 4 + (tp.ray & 3), py = py0 + (tp.wave >> 1) * 4 + (tp.ray >> 2);
+    const bool valid = px < P.cam.width && py < P.cam.height;
+    CountersFor<STATS> cn;
+    RGX_SEC_START(cn, 0);
+    int turn = 0;
+    Frustum F;
+    frustum_planes(P.cam, px0, py0, F);
+    RayState R;
+    ray_begin<false>(P, px, py, valid, R);
+    {
+        const TeamWord far = team_exchange(T, tp, turn, 0.f, row_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f), 0.f, 0u);
+        team_frustum_cut(P, F, far.hi, T, tp);
+    }
+    const f3 dir = R.dir;
+    float Cr = 0.f, Cg = 0.f, Cb = 0.f, depth = 0.f; // this copy's shares
+    Window Wn = {0.f, 0, false, 4, false, false};
+    RGX_SEC(cn, RGX_SEC_SETUP);
+    constexpr uint32_t ACTIVE = 1u, WANT = 2u, SEARCH = 4u, NEED = 8u, RUN = 16u;
+
+    for (;;) {
+        float tlo, thi;
+        const bool need = slab_begin<true>(P, R, tlo, thi);
+        const bool srch = R.active && R.searching, want = need || srch;
+        const float w0 = row_min_all(want ? tlo : INFINITY), w1 = row_max_all(want ? thi : -INFINITY);
+        const TeamWord all = team_exchange(T, tp, turn, w0, w1, row_max_all(want ? tlo + (float)Wn.k * R.slab_spacing : -INFINITY),
+                                           (__any(R.active) ? ACTIVE : 0u) | (__any(want) ? WANT : 0u) | (__any(srch) ? SEARCH : 0u) | (__any(need) ? NEED : 0u));
+        if (!(all.flags & ACTIVE)) break;
+        RGX_SEC(cn, RGX_SEC_TOP);
+        int p0 = 0;
+        bool ov = false;
+        float found = -1.0f, searched_to = 0.f;
+        if (all.flags & WANT) {
+            const float t0 = all.lo, t1 = all.hi, dt = R.dt;
+            const bool any_search = all.flags & SEARCH;
+            if constexpr (RECORD) {
+                if (rec.piece_due(P, Wn.resident && t1 <= Wn.hi)) {
+                    rec.piece(P, T, tp, R, Cr, Cg, Cb);
+                    if (Wn.resident && t1 <= Wn.hi) rec.window(T, Wn.n);
+                }
+            }
+            const float tmid = fmaf(dt, (float)RGX_CHUNK_SIZE, R.tbuffer);
+            const bool split = !RECORD && Wn.crowded && (all.flags & NEED);
+            int len = 0, q0 = 0, seen = 0;
+            uint32_t own[2] = {0u, 0u};
+            bool run = need, qov = false;
+            float sg[RGX_CHUNK_SIZE], cr[RGX_CHUNK_SIZE], cg[RGX_CHUNK_SIZE], cb[RGX_CHUNK_SIZE];
+            bool live = false; // the block has hits in this half, and sums
+            f3 rdt = dir * fmaf(dt, 0.5f, R.tbuffer);
+            auto accumulate = [&](const auto &e, bool hit) {
+                if (hit) {
+                    const float4 col = e.prim->rgba4;
+                    f3 U, V, W, inv;
+                    float k;
+                    e.frame(U, V, W, inv, k);
+                    HitSetup hs = hit_setup(U, V, W, inv, k, e.prim->pos4, dir, rdt, dt);
+                    const float rho = col.w;
+#pragma unroll
+                    for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
+                        const float gw = hs.power < hs.cut ? gauss_weight(hs.power) : 0.0f;
+                        sg[i] = fmaf(rho, gw, sg[i]);
+                        cr[i] = fmaf(col.x, gw, cr[i]);
+                        cg[i] = fmaf(col.y, gw, cg[i]);
+                        cb[i] = fmaf(col.z, gw, cb[i]);
+                        hs.power += hs.inc;
+                        hs.inc += hs.inc_st;
+                    }
+                }
+            };
+            // The half's sums over the copies, four samples per copy; they are blended (a ray without hits has none, and
+            // stays as it is) and kept in the iteration's sample-sum slot, if it has one.
+            auto blend = [&](int half) {
+                float d4[4], r4[4], g4[4], b4[4];
+                if (live) {
+                    sum_copies(sg, d4);
+                    sum_copies(cr, r4);
+                    sum_copies(cg, g4);
+                    sum_copies(cb, b4);
+                } else {
+                    if constexpr (!RECORD) return;
+                    else if (rec.slot < 0) return;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) d4[i] = r4[i] = g4[i] = b4[i] = 0.f;
+                }
+                live = false;
+                // The transmittance goes through the 16 samples one after the other, in every copy, as it does where one
+                // lane has them all: a replay of the record rounds it the same way.
+                float w4[4], s4[4], Tb = R.T, T_all = R.T;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x = d4[i] * dt;
+                    w4[i] = __expf(-x);
+                    s4[i] = dt * ((1.0f - w4[i]) * __builtin_amdgcn_rcpf(fmaxf(x, 1e-6f)));
+                }
+                {
+                    float w0[4], w1[4], w2[4], w3[4];
+                    copies(w4[0], w0);
+                    copies(w4[1], w1);
+                    copies(w4[2], w2);
+                    copies(w4[3], w3);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        Tb = tp.sub == c ? T_all : Tb;
+                        T_all = (((T_all * w0[c]) * w1[c]) * w2[c]) * w3[c];
+                    }
+                }
+                float t_sample = fmaf(dt, (float)(half * RGX_CHUNK_SIZE + 4 * tp.sub) + 0.5f, R.tbuffer); // (viewer)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float ts = Tb * s4[i];
+                    Cr = fmaf(ts, r4[i], Cr);
+                    Cg = fmaf(ts, g4[i], Cg);
+                    Cb = fmaf(ts, b4[i], Cb);
+                    if constexpr (VIEWER) {
+                        depth += Tb * (1.0f - w4[i]) * t_sample;
+                        t_sample += dt;
+                    }
+                    Tb *= w4[i];
+                }
+                R.T = T_all;
+                if constexpr (RECORD) {
+                    if (rec.slot >= 0) {
+                        float *slot = (float *)(P.sum_pool + (int64_t)rec.slot * (P.sum_slot_words / 4));
+                        const int first = half * RGX_CHUNK_SIZE + 4 * tp.sub, at = tp.wave * 16 + tp.ray;
+                        float *dens = slot + first * 64 + at;
+                        if constexpr (!HALF) {
+                            float *col = slot + RGX_BUFFER_SIZE * 64 + (first * 64 + at) * 3;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                __builtin_nontemporal_store(d4[i], dens + i * 64);
+                                __builtin_nontemporal_store(r4[i], col + i * 192);
+                                __builtin_nontemporal_store(g4[i], col + i * 192 + 1);
+                                __builtin_nontemporal_store(b4[i], col + i * 192 + 2);
+                            }
+                        } else {
+                            float big = 0.f;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                __builtin_nontemporal_store(d4[i], dens + i * 64);
+                                big = fmaxf(big, fmaxf(fabsf(r4[i]), fmaxf(fabsf(g4[i]), fabsf(b4[i]))));
+                            }
+                            float v[4];
+                            copies(big, v);
+                            big = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+                            const int e = big > 0.f ? __builtin_amdgcn_frexp_expf(big) : 0;
+                            const float down = __builtin_amdgcn_ldexpf(1.0f, -e);
+                            uint32_t *col = (uint32_t *)slot + RGX_BUFFER_SIZE * 64 + half * (24 * 64) + 6 * tp.sub * 64 + at;
+                            auto value = [&](int k) { return (k % 3 == 0 ? r4[k / 3] : k % 3 == 1 ? g4[k / 3] : b4[k / 3]) * down; };
+#pragma unroll
+                            for (int k = 0; k < 6; ++k) {
+                                const __half2 two = __floats2half2_rn(value(2 * k), value(2 * k + 1));
+                                __builtin_nontemporal_store(*(const uint32_t *)&two, col + k * 64);
+                            }
+                            if (tp.sub == 0)
+                                __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(1.0f, e), slot + RGX_BUFFER_SIZE * 64 + 2 * 24 * 64 + half * 64 + at);
+                        }
+                    }
+                }
+            };
+            for (int phase = 0; phase < 2; ++phase) {
+                const bool reuse = !split && Wn.resident && t1 <= Wn.hi;
+                float lo = t0, hi = t1;
+                if (split) {
+                    if (phase == 0) {
+                        hi = team_exchange(T, tp, turn, 0.f, row_max_all(need ? fminf(thi, tmid) : -INFINITY), 0.f, 0u).hi;
+                    } else {
+                        const TeamWord second = team_exchange(T, tp, turn, row_min_all(run && tmid < thi ? fmaxf(tlo, tmid) : INFINITY),
+                                                              row_max_all(run ? thi : -INFINITY), 0.f, 0u);
+                        lo = second.lo;
+                        hi = second.hi;
+                    }
+                    if (!(lo <= hi)) break;
+                }
+                Sweep S = {0, 0};
+                if (!reuse) {
+                    float wend = hi;
+                    if (!split && phase == 0 && Wn.k > 1) wend = fmaxf(t1, all.ahead);
+                    frustum_range(F, lo, wend);
+                    team_sweep_begin(P, S, F, T);
+                }
+                bool first = true, more = true;
+                while (more) {
+                    int C;
+                    bool plain;
+                    if (reuse) {
+                        C = Wn.n;
+                        plain = Wn.plain;
+                        more = false;
+                    } else {
+                        bool done;
+                        C = team_sweep_next(P, S, F, T, tp, done, plain, cn);
+                        if (split) {
+                            seen += C;
+                        } else if (phase == 0 && first) {
+                            if (done) {
+                                Wn.hi = F.t1;
+                                Wn.n = C;
+                                Wn.resident = true;
+                                Wn.plain = plain;
+                                Wn.crowded = false;
+                                if (C > RGX_KHI) Wn.k = Wn.k > 1 ? Wn.k / 2 : 1;
+                                else if (C < RGX_KLO && Wn.k < 32) Wn.k *= 2;
+                            } else if (Wn.k > 1) {
+                                Wn.k = 1;
+                                frustum_range(F, t0, t1);
+                                team_sweep_begin(P, S, F, T);
+                                continue;
+                            } else {
+                                Wn.resident = false;
+                                Wn.crowded = true;
+                            }
+                        }
+                        first = false;
+                        more = !done;
+                    }
+                    RGX_SEC(cn, RGX_SEC_SWEEP);
+                    if constexpr (RECORD) {
+                        if (phase == 0 && !reuse) rec.window(T, C);
+                    }
+                    RGX_SEC(cn, RGX_SEC_LISTS);
+                    if (phase == 0 || !Wn.resident || split) {
+                        const float cover = split ? hi : (Wn.resident ? Wn.hi : t1);
+                        const LaneQuery Q = {R.dir, run, tlo, thi, phase == 0 && srch, R.tbuffer, fminf(R.texit, cover), P.m.max_prim_slice, tmid};
+                        const bool real = phase == 0 || split;
+                        int cnt = real ? p0 : q0;
+                        bool cut = real ? ov : qov;
+                        float best = phase == 0 ? found : -1.0f;
+                        // the block's own range (its searching rays look through the whole table)
+                        const float from = fmaxf(lo, w0);
+                        auto filter = [&](auto search, auto part) {
+                            const float to = decltype(search)::value ? cover : fminf(hi, w1);
+                            if (__builtin_expect(plain, 1)) team_filter<decltype(search)::value, decltype(part)::value, true>(T, tp, C, from, to, Q, cnt, cut, best, len, own, cn);
+                            else team_filter<decltype(search)::value, decltype(part)::value, false>(T, tp, C, from, to, Q, cnt, cut, best, len, own, cn);
+                        };
+                        using std::integral_constant;
+                        if (!split) {
+                            if (phase == 0 && __any(srch)) filter(std::true_type{}, integral_constant<int, 0>{});
+                            else filter(std::false_type{}, integral_constant<int, 0>{});
+                        } else if (phase == 0) {
+                            if (__any(srch)) filter(std::true_type{}, integral_constant<int, 1>{});
+                            else filter(std::false_type{}, integral_constant<int, 1>{});
+                        } else {
+                            filter(std::false_type{}, integral_constant<int, 2>{});
+                        }
+                        if (real) {
+                            p0 = cnt;
+                            ov = cut;
+                        } else {
+                            q0 = cnt;
+                            qov = cut;
+                        }
+                        RGX_SEC(cn, RGX_SEC_FILTER);
+                        if (phase == 0) {
+                            found = best;
+                            searched_to = fmaxf(Q.slo, Q.shi);
+                            if constexpr (RECORD) {
+                                if (tp.lane == 0) T.msg[tp.wave] = len;
+                                const bool blends = __any(need && p0 > 0);
+                                if (tp.lane == 0 && blends) T.msg[tp.wave] = len | 0x10000;
+                                __syncthreads();
+                                rec.lists(T, tp, !more);
+                            }
+                        }
+                    }
+                    RGX_SEC(cn, RGX_SEC_LISTS);
+                    if (len > 0 && __any(run)) {
+                        if (!live) {
+#pragma unroll
+                            for (int i = 0; i < RGX_CHUNK_SIZE; ++i) sg[i] = cr[i] = cg[i] = cb[i] = 0.f;
+                            live = true;
+                        }
+                        team_shade(P, T, tp, len, run, phase, own, accumulate);
+                    }
+                    RGX_SEC(cn, RGX_SEC_SHADE);
+                    if (more) __syncthreads(); // every wavefront is done with the table
+                }
+                if (phase == 0) {
+                    if constexpr (RECORD) {
+                        const bool blends = uni_u32((uint32_t)(T.msg[0] | T.msg[1] | T.msg[2] | T.msg[3]) & 0x10000u) != 0;
+                        rec.trailer(P, T, tp, any_search, Wn.resident ? Wn.hi : t1, found, blends);
+                    }
+                    RGX_SEC(cn, RGX_SEC_LISTS);
+                    const bool has = need && (p0 > 0 || split);
+                    blend(0);
+                    RGX_SEC(cn, RGX_SEC_BLEND);
+                    rdt = dir * fmaf(dt, 16.5f, R.tbuffer);
+                    run = has && R.T > P.m.t_eps;
+                    if (Wn.resident && !split) continue; // the lists are still there
+                    if (!(team_exchange(T, tp, turn, 0.f, 0.f, 0.f, __any(run) ? RUN : 0u).flags & RUN)) break;
+                }
+            }
+            blend(1);
+            RGX_SEC(cn, RGX_SEC_BLEND);
+            if (split && seen < CAP / 2) Wn.crowded = false;
+            if (need && p0 > 0 && tp.sub == 0) {
+                cn.slabs++;
+                cn.hit_pairs += p0;
+            }
+            if (ov && tp.sub == 0) cn.overflow++;
+        }
+        if constexpr (STATS) {
+            Counters mine = {};
+            slab_end(R, need, p0, found, searched_to, mine);
+            if (tp.sub == 0) {
+                cn.rays_hit += mine.rays_hit;
+                cn.empty += mine.empty;
+            }
+        } else {
+            slab_end(R, need, p0, found, searched_to, cn);
+        }
+        RGX_SEC(cn, RGX_SEC_END);
+    }
+    {
+        float r[4], g[4], b[4];
+        copies(Cr, r);
+        copies(Cg, g);
+        copies(Cb, b);
+        Cr = (r[0] + r[1]) + (r[2] + r[3]);
+        Cg = (g[0] + g[1]) + (g[2] + g[3]);
+        Cb = (b[0] + b[1]) + (b[2] + b[3]);
+        if constexpr (VIEWER) {
+            copies(depth, r);
+            depth = (r[0] + r[1]) + (r[2] + r[3]);
+        }
+    }
+    if (valid && tp.sub == 0) {
+        const int64_t ray = (int64_t)py * P.cam.width + px;
+        if constexpr (VIEWER) {
+            *(uchar4 *)(P.frame + 4 * ray) = make_uchar4(quantize8(Cr), quantize8(Cg), quantize8(Cb), 255);
+            P.depth[ray] = depth;
+        } else {
+            const float bg = P.m.white_background ? 1.0f : 0.0f;
+            P.ray_colors[3 * ray] = Cr + R.T * bg;
+            P.ray_colors[3 * ray + 1] = Cg + R.T * bg;
+            P.ray_colors[3 * ray + 2] = Cb + R.T * bg;
+        }
+        if constexpr (STATS) {
+            if (P.ray_counts) {
+                P.ray_counts[2 * ray] = cn.slabs;
+                P.ray_counts[2 * ray + 1] = cn.hit_pairs;
+            }
+        }
+    }
+    rec.finish(P);
+    flush_stats(P.stats, cn);
+    RGX_SEC(cn, RGX_SEC_EPILOGUE);
+    RGX_SEC_FLUSH(cn, RECORD ? RGX_SECK_FWD_RECORD : RGX_SECK_FWD_PLAIN);
+}
+
 // sum over the 16 lanes of each row, left in every lane of the row.  (Every lane of these four
 // patterns reads a lane of its own row, so bound_ctrl changes nothing but the instruction: without
 // it the last stage, whose add the compiler sinks into the one-lane-per-row branch that uses it,
@@ -2791,6 +3674,44 @@ static inline dim3 march_grid(const MarchParams &P)
     return dim3((unsigned)(8 * g.per_xcd * g.bw * g.bh));
 }
 
+// Up to this many tiles four wavefronts march a tile (k_march_team), beyond it one.  The team's wavefronts repeat the
+// per-iteration work that one wavefront does once for 64 rays, so it loses where the chip is full anyway (10 000 tiles: 1.5
+// to 2.5 times as long); with few tiles the launch is one tile's latency.  Measured, ms without / with the team: 4 k
+// Gaussians in a cube, 256 tiles 1.29 / 0.62, 1 024 tiles 0.88 / 0.52; 100 k in a ball, 256 tiles 7.8 / 2.9, 1 600 tiles
+// 2.4 / 1.2; frames of 60 k heavy-tailed with the adaptive step, 256 tiles 1.43 / 0.74, 625 tiles 1.03 / 0.92, 1 024 tiles
+// 0.94 / 0.98.  Not in training with the adaptive step: the team adds up a sample's hits in another order, the next step's
+// length depends on the last bit of the transmittance, and a sample that so crosses a Gaussian's cut-off moves that
+// Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians): equally exact, but no longer the gradients
+// that larger images and earlier builds give.
+#ifndef RGX_TEAM_TILES
+#define RGX_TEAM_TILES 768
+#endif
+// half: the record's colour sums are in half precision
+static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, hipStream_t s)
+{
+    const bool team = P.tiles_x * P.tiles_y <= RGX_TEAM_TILES && !(P.records && P.m.dynamic_sampling);
+    const dim3 grid = march_grid(P), block(team ? 256 : 64);
+#define RGX_FWD(...)                                                                            \
+    do {                                                                                        \
+        if (team) hipLaunchKernelGGL((k_march_team<__VA_ARGS__>), grid, block, 0, s, P);        \
+        else hipLaunchKernelGGL((k_march_fwd<__VA_ARGS__>), grid, block, 0, s, P);              \
+    } while (0)
+    if (viewer) {
+        if (counting) RGX_FWD(false, true, true);
+        else RGX_FWD(false, true, false);
+    } else if (P.records && half) {
+        if (counting) RGX_FWD(true, false, true, true);
+        else RGX_FWD(true, false, false, true);
+    } else if (P.records) {
+        if (counting) RGX_FWD(true, false, true);
+        else RGX_FWD(true, false, false);
+    } else {
+        if (counting) RGX_FWD(false, false, true);
+        else RGX_FWD(false, false, false);
+    }
+#undef RGX_FWD
+}
+
 static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
                                 float *ray_colors, void *march_ws, size_t march_ws_bytes, void *records, size_t records_bytes,
                                 RgxStats *stats, uint32_t *ray_counts, void *stream);
@@ -2829,16 +3750,8 @@ static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxM
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
     if (P.sum_pool || P.faults) hipLaunchKernelGGL(k_clear2, dim3(1), dim3(64), 0, (hipStream_t)stream, (float4 *)P.sum_next, (float4 *)P.faults);
     order_blocks(P, (hipStream_t)stream);
-    if (P.records && P.sum_pool && P.m.record_format == 1) {
-        if (counting) hipLaunchKernelGGL((k_march_fwd<true, false, true, true>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-        else hipLaunchKernelGGL((k_march_fwd<true, false, false, true>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-    } else if (P.records) {
-        if (counting) hipLaunchKernelGGL((k_march_fwd<true, false, true>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-        else hipLaunchKernelGGL((k_march_fwd<true, false, false>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-    } else {
-        if (counting) hipLaunchKernelGGL((k_march_fwd<false, false, true>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-        else hipLaunchKernelGGL((k_march_fwd<false, false, false>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-    }
+    const bool half = P.sum_pool && P.m.record_format == 1;
+    launch_forward(P, false, counting, half, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
     RGX_LAUNCH_CHECK();
     return RGX_OK;
@@ -2857,8 +3770,7 @@ extern "C" int rgx_march_viewer(const void *ws, const RgxCamera *cam, const RgxM
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
     if (P.faults) hipLaunchKernelGGL(k_clear2, dim3(1), dim3(64), 0, (hipStream_t)stream, (float4 *)nullptr, (float4 *)P.faults);
     order_blocks(P, (hipStream_t)stream);
-    if (stats) hipLaunchKernelGGL((k_march_fwd<false, true, true>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
-    else hipLaunchKernelGGL((k_march_fwd<false, true, false>), march_grid(P), dim3(64), 0, (hipStream_t)stream, P);
+    launch_forward(P, true, stats != nullptr, false, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
     RGX_LAUNCH_CHECK();
     return RGX_OK;

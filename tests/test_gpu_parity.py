@@ -430,6 +430,36 @@ def test_backward_in_pieces_equals_recomputation(gx, w, h, half):
         assert cos >= 1 - 1e-6 and rel <= (1e-3 if half else 1e-4), (k, cos, rel)
 
 
+@pytest.mark.parametrize("w,h", [(1, 1), (9, 7), (216, 224), (224, 224)])
+@pytest.mark.parametrize("config,scale,dyn", [(0, 1.0, False), (2, 4.0, True)])
+def test_forward_with_one_and_with_four_wavefronts_per_tile(gx, orc, w, h, config, scale, dyn):
+    """The smallest images and both sides of the number of tiles (756, 784) at which the forward goes over from four
+    wavefronts per tile to one; sparse slabs, and slabs whose candidates fill several tables.  With and without a
+    record, counting and not."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(config, n=6000, sh_degree=1, seed=31))
+    sc["scales"] = sc["scales"] * scale
+    cam = scenes.make_camera(config, 1, width=w, height=h)
+    cfg = dict(dt_step=0.004, dynamic_sampling=dyn, max_prim_slice=4096)
+    ids = np.unique(np.random.default_rng(6).integers(0, w * h, 300))
+    img, st, ctx = orc.render_forward(sc, cam, cfg["dt_step"], dyn, 4096, ray_ids=ids)
+    dloss = np.zeros((w * h, 3), np.float32)
+    dloss[ids] = np.random.default_rng(7).normal(size=(len(ids), 3)).astype(np.float32)
+    _step(f"wavefronts per tile {w}x{h} config {config}")
+    _, counts = gx.gpu_forward_counts(sc, cam, cfg)
+    same, rephased, edge = gx.comparable_rays(orc, ctx, img, counts, ids)
+    assert rephased + edge <= (0.05 * len(ids) if dyn else 0)
+    dloss[ids[~same]] = 0
+    og, _ = orc.render_backward(sc, ctx, img, dloss)
+    plain = gx.gpu_render(sc, cam, cfg)["image"]
+    for stats in (True, False):
+        out = gx.gpu_render(sc, cam, cfg, want_grad=dloss, stats=stats)
+        for image in (out["image"], plain):
+            assert np.abs(image[ids] - img[ids])[same].max() <= IMG_TOL
+        assert np.abs(out["image"] - plain).max() <= (5e-3 if dyn else 1e-5)      # (adaptive: a ray may be re-phased)
+        if w > 1:
+            _check_grads(gx, out["grads"], og)
+
+
 def test_long_hit_lists_spill_and_truncation(gx, orc):
     """Fat Gaussians: slabs with far more than 32 hits (LDS part + spill area), then a tiny
     max_prim_slice to exercise the silent truncation path and its counter."""
