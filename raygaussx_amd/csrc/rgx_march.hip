@@ -39,7 +39,7 @@
 #ifndef RGX_KLO
 #define RGX_KLO (RGX_CCAP / 3)       // one that stayed below this, twice as many
 #endif
-#define RGX_MASK_WORDS ((RGX_CCAP + 31) / 32) // 32-bit words of a hit mask over a row's list
+#define RGX_MASK_WORDS ((RGX_CCAP + 31) / 32) // 32-bit words of a hit mask over the list
 // Above QCAP - margin the sweep pops one node at a time (depth-first).  A breadth-first step pops
 // up to 64 nodes and pushes up to 128, so it leaves at most QCAP - margin + 64 entries; a
 // depth-first step adds at most one entry per level it descends, and a Karras tree over 63-bit
@@ -757,8 +757,8 @@ struct TileLds {
     int32_t *queue;        // [RGX_QCAP]
     int32_t *leafq;        // [128]: leaves waiting for the sweep's ellipsoid test
     float *tab;            // [RGX_CCAP * RGX_TAB]
-    uint8_t *rowlist;      // [4][RGX_CCAP]: per 16-lane row, table slots some lane of the row hits
-    uint32_t (*mask)[64];  // [RGX_MASK_WORDS][64]: per lane, hit bits over its row's list
+    uint8_t *list;         // [RGX_CCAP]: table slots that some ray of the tile hits
+    uint32_t (*mask)[64];  // [RGX_MASK_WORDS][64]: per lane, hit bits over the list
     uint32_t (*half)[4][RGX_MASK_WORDS]; // [2][row][word]: list entries with samples in the slab's first / second 16
 };
 
@@ -850,6 +850,19 @@ __device__ __forceinline__ HitSetup hit_setup(f3 U, f3 V, f3 W, f3 inv, float k,
     return h;
 }
 
+// How close to zero the filter's u (below) may come before it stops deciding.  With N = |Oe| = sqrt(c + 1), e = 2^-24,
+// a ray that meets the ellipsoid or nearly so, and the same computed a, b, De, Oe in both forms: the
+// predicate's r2 = (b + s) / a is within 3 e (N + 1) + 6 e of the exact root of those numbers in whitened
+// units; its r1 = c / q within 16 e N, since c is rounded (3 e N^2) and a, b need not belong to that c exactly
+// (9 e N^2), over q > 0.86 N; u's own point tc is within 3 e N, and its square as far again with half-chord
+// and distance at most one: 38 e N + 40 e, plus 470 (e N)^2, which up to N = 2^15 is below 2 e N + 24 e.
+// A quotient c / q is that well behaved, and a line with b < 0 that surely missed, only with the eye outside the
+// ellipsoid's double (c >= 3): entries nearer than that, or further than N = 2^15, are decided by their roots.
+__device__ __forceinline__ float filter_margin(float c)
+{
+    return c >= 3.0f && c <= 0x1p30f ? fmaf(__builtin_amdgcn_sqrtf(c + 1.0f), 41.0f * 0x1p-24f, 66.0f * 0x1p-24f) : INFINITY;
+}
+
 // What one lane asks of the candidate table in this iteration.
 struct LaneQuery {
     f3 dir;
@@ -862,87 +875,121 @@ struct LaneQuery {
 };
 
 // Filter: every lane tests the table entries whose distance shell meets [t0, t1] (the union of
-// the lanes' intervals).  A wave is four 16-lane rows, each row a 4x4 pixel block; an entry hit
-// by any marching lane of a row is appended to that row's list, and each lane keeps its own hit
-// bits over its row's list.  Per list entry the row also notes whether any of its rays can have
+// the lanes' intervals).  An entry hit by any marching lane is appended to the iteration's list, and each lane
+// keeps its own hit bits over it.  A wave is four 16-lane rows, each row a 4x4 pixel block: per list entry a row
+// also notes whether any of its rays can have
 // samples inside the Gaussian in the slab's first 16 samples and in its second 16 (the chord
 // [r1, r2] against tmid; a sample lies half a step from tmid, rounding moves a root by far less),
-// so that each half is shaded from its own, shorter list.  len (row-uniform) is the list length; p0 / ov count this lane's
+// so that each half is shaded from its own, shorter list.  len (wave-uniform) is the list length; p0 / ov count this lane's
 // hits and note the max_prim_slice cut (__anyhit__ah's optixTerminateRay, 352-356); found is
 // the running minimum of the searching lanes.
-// SEARCH: some lane of the wave is searching (otherwise the first-hit query's part is left out).
-// PART (the same for all lanes): 0: all hits of [tlo, thi]; 1: only those reaching the first 16
+// part (the same for all lanes): 0: all hits of [tlo, thi]; 1: only those reaching the first 16
 // samples; 2: only those reaching the second 16, of which the ones that also reach the first are
-// not counted again.  PLAIN: every entry of the table passed plain_roots().
-template <bool SEARCH, int PART, bool PLAIN, typename Cn>
-__device__ __forceinline__ void filter_table(const TileLds &L, int C, float t0, float t1, const LaneQuery &Q, int &p0, bool &ov,
-                                             float &found, int &len, uint32_t (&own)[2], Cn &cn)
+// not counted again.  plain: every entry of the table passed plain_roots().
+//
+// The filter is bound by the number of its instructions, of whatever kind, and by how long each waits for the one
+// before: three wavefronts per SIMD issue at most one each in some five clocks.  The reference's
+// predicate is two divisions and a square root, correctly rounded, one after the other.  What decides is
+// whether the ray's segment meets the ellipsoid, and for nearly every ray and entry that does not take the roots:
+// with tc the line's closest point to the centre and d2 its squared whitened distance there, the point of
+// the segment closest to tc lies at u = (x - tc)^2 a + d2 - 1 from the surface, and u < 0 says hit.  Where
+// some ray's |u| is within filter_margin() of zero -- u and the predicate's comparisons may then fall on different
+// sides -- the wavefront takes the exact roots for that entry, as it does where a searching ray may have
+// found something, whose t it needs.  What the lanes decide stays in scalar registers, one list serves the
+// whole wavefront, and the entries' slots are collected in a register.
+template <typename Cn>
+__device__ __forceinline__ void filter_table(const TileLds &L, int C, float t0, float t1, const LaneQuery &Q, int part, bool plain,
+                                             int &p0, bool &ov, float &found, int &len_out, uint32_t (&own)[2], Cn &cn)
 {
-    const int lane = threadIdx.x, row = lane >> 4;
-    len = 0;
+    const int lane = threadIdx.x;
+    int len = 0;
+    uint32_t first = 0, second = 0; // this lane's hits with samples in the first / second half
+    int slots = 0;                  // lane i: slot of entry i of the list's current 64
     own[0] = own[1] = 0u;
-    uint32_t bits = 0, first = 0, second = 0; // this lane's hits; those with samples in the first / second half
+    const bool asks = Q.need && !Q.search;
+    const uint64_t searching = __ballot(Q.search);
+    // the segment and where its halves meet (rays that ask nothing: far from everything)
+    const float none = 1e15f;
+    const float lo = Q.search ? Q.slo : asks ? Q.tlo : none, hi = Q.search ? Q.shi : asks ? Q.thi : none;
+    const float mid = Q.search ? hi : asks ? fminf(Q.tmid, hi) : none;
+    // max_prim_slice cuts a ray's list in the order of the entries: where it could, entry by entry
+    const bool slow = !plain || __any(asks && (ov || p0 + C > Q.cap));
+    const uint64_t take_first = part != 2 ? ~0ull : 0ull, take_second = part != 1 ? ~0ull : 0ull;
     auto flush = [&](int w) {
+        const uint32_t bits = (part != 2 ? first : 0u) | (part != 1 ? second : 0u);
         L.mask[w][lane] = bits;
+        if (!slow) p0 += __popc(part == 2 ? second & ~first : bits);
         if (w == 0) { // the ray's own notes on the list's first 32 entries stay with it (see shade_lanes)
             own[0] = first;
             own[1] = second;
         }
         const uint32_t f = row_or(first), g = row_or(second);
         if ((lane & 15) == 0) {
-            L.half[0][row][w] = f;
-            L.half[1][row][w] = g;
+            L.half[0][lane >> 4][w] = f;
+            L.half[1][lane >> 4][w] = g;
         }
-        bits = first = second = 0;
+        first = second = 0;
+        if (lane < len - (w & ~1) * 32) L.list[(w & ~1) * 32 + lane] = (uint8_t)slots;
     };
-    for (int h = 0; h < (RGX_CCAP + 63) / 64; ++h) {
-        const int cl = h * 64 + lane;
+    for (int h = 0; h < RGX_CCAP; h += 64) {
+        const int cl = h + lane;
         bool rel = false;
+        float margins = INFINITY;
         if (cl < C) {
             const float dmin = L.tab[cl * RGX_TAB + 3], dmax = L.tab[cl * RGX_TAB + 7];
             rel = dmax >= t0 && dmin <= t1;
+            margins = slow ? INFINITY : filter_margin(L.tab[cl * RGX_TAB + 15]);
         }
         uint64_t m = __ballot(rel);
         if (lane == 0) cn.cands += (unsigned)__popcll(m);
         while (m) {
-            const int c = h * 64 + __builtin_ctzll(m);
+            const int i = __builtin_ctzll(m), c = h + i;
             m &= m - 1;
-            // straight-line code: every lane evaluates both queries' predicates, its state selects
-            float r1, r2;
-            // (the counting kernels go without the early exit: it costs their recording variant its registers)
-            constexpr bool EXIT = std::is_same<Cn, NoCounters>::value;
-            const bool ok = lane_roots<PLAIN, EXIT>((const float4 *)(L.tab + c * RGX_TAB), Q.dir, r1, r2);
-            if constexpr (EXIT) {
-                if (!__any(ok)) continue;
-            }
-            // first-hit query (searching lanes): smallest max(slo, r1) over the entries hit in [slo, shi]
-            if constexpr (SEARCH) {
+            const float margin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(margins), i));
+            const float4 *e = (const float4 *)((const char *)L.tab + __builtin_amdgcn_readfirstlane(c * (RGX_TAB * 4)));
+            const float4 e0 = e[0], e1 = e[1], e2 = e[2], e3 = e[3], e4 = e[4];
+            const f3 De = apply_sinv_rt(Q.dir, mk3(e0.x, e0.y, e0.z), mk3(e1.x, e1.y, e1.z), mk3(e2.x, e2.y, e2.z), mk3(e3.x, e3.y, e3.z));
+            const float a = fmaf(De.x, De.x, fmaf(De.y, De.y, De.z * De.z));
+            const float b = -fmaf(e4.x, De.x, fmaf(e4.y, De.y, e4.z * De.z));
+            const float tc = b * __builtin_amdgcn_rcpf(a);
+            const f3 Pc = mk3(fmaf(tc, De.x, e4.x), fmaf(tc, De.y, e4.y), fmaf(tc, De.z, e4.z));
+            const float out = fmaf(Pc.x, Pc.x, fmaf(Pc.y, Pc.y, Pc.z * Pc.z)) - 1.0f;
+            const float x1 = __builtin_amdgcn_fmed3f(tc, lo, mid) - tc, x2 = __builtin_amdgcn_fmed3f(tc, mid, hi) - tc;
+            const float u1 = fmaf(x1 * x1, a, out), u2 = fmaf(x2 * x2, a, out);
+            uint64_t f = __ballot(!(u1 > margin)), g = __ballot(!(u2 > margin));
+            const uint64_t sure = __ballot(fminf(fabsf(u1), fabsf(u2)) > margin);
+            if ((f | g) == 0) continue;
+            if (__builtin_expect((~sure | ((f | g) & searching)) != 0, 0)) {
+                float r1, r2;
+                const bool ok = lane_roots<false, false>(e, Q.dir, r1, r2);
+                // first-hit query (searching lanes): smallest max(slo, r1) over the entries hit in [slo, shi]
                 const float ts = fmaxf(Q.slo, r1);
                 const bool sfound = Q.search && ok && ts <= fminf(Q.shi, r2);
                 found = sfound ? (found < 0.0f ? ts : fminf(found, ts)) : found;
+                // collect query (marching lanes); every hit is noted for a half at least
+                bool seg = asks && !ov && ok && fmaxf(Q.tlo, r1) <= fminf(Q.thi, r2);
+                const bool to_second = r2 > Q.tmid, to_first = r1 < Q.tmid || !to_second;
+                if (slow) {
+                    const bool counts = part != 2 || !to_first, over = seg && counts && p0 >= Q.cap;
+                    ov = ov || over;
+                    seg = seg && !over;
+                    p0 += seg && counts && (part != 1 || to_first) ? 1 : 0;
+                }
+                f = __ballot(seg && to_first);
+                g = __ballot(seg && to_second);
             }
-            // collect query (marching lanes)
-            const bool seg = Q.need && !(SEARCH && Q.search) && !ov && ok && fmaxf(Q.tlo, r1) <= fminf(Q.thi, r2);
-            const bool f = r1 < Q.tmid, g = r2 > Q.tmid;
-            const bool counts = PART != 2 || !f;
-            const bool over = seg && counts && p0 >= Q.cap;
-            ov = ov || over;
-            const bool hit = seg && !over && (PART == 0 || (PART == 1 ? f : g));
-            p0 += (hit && counts) ? 1 : 0;
-            const uint32_t in_first = (hit && f) ? 1u : 0u, in_second = (hit && g) ? 1u : 0u;
-            const uint64_t bal = __ballot(hit);
-            if (lane == 0 && bal) cn.cands_hit++;
-            if ((bal >> (row * 16)) & 0xffffull) {
-                bits |= (uint32_t)hit << (len & 31);
-                first |= in_first << (len & 31);
-                second |= in_second << (len & 31);
-                if ((lane & 15) == 0) L.rowlist[row * RGX_CCAP + len] = (uint8_t)c;
-                ++len;
-                if ((len & 31) == 0) flush((len >> 5) - 1);
-            }
+            if (((f & take_first) | (g & take_second)) == 0) continue;
+            if (lane == 0) cn.cands_hit++;
+            const uint32_t bit = 1u << (len & 31);
+            first |= __builtin_amdgcn_inverse_ballot_w64(f) ? bit : 0u;
+            second |= __builtin_amdgcn_inverse_ballot_w64(g) ? bit : 0u;
+            slots = lane == (len & 63) ? c : slots;
+            ++len;
+            if ((len & 31) == 0) flush((len >> 5) - 1);
         }
     }
     if (len & 31) flush(len >> 5);
+    len_out = len;
     __syncthreads();
 }
 
@@ -962,22 +1009,34 @@ struct HalfRows {
     static constexpr int group = RGX_GRAD_GROUP;
 };
 
-// Shade: the four rows walk their own lists in lock step; body(entry, hit, live) runs whenever
-// some lane hits (hit: this lane hits this entry; live: this lane's row still has an entry at i).
+// Shade: the four rows walk the entries that one of their own rays hits in lock step; body(entry, hit, live) runs whenever
+// some lane hits (hit: this lane hits this entry; live: this lane's row still has an entry).
 template <typename Body>
 __device__ __forceinline__ void shade_rows(const MarchParams &P, const TileLds &L, int len, bool run, Body body)
 {
-    const int lane = threadIdx.x, row = lane >> 4;
-    const int l0 = __builtin_amdgcn_readlane(len, 0), l1 = __builtin_amdgcn_readlane(len, 16);
-    const int l2 = __builtin_amdgcn_readlane(len, 32), l3 = __builtin_amdgcn_readlane(len, 48);
-    const int maxlen = max(max(l0, l1), max(l2, l3));
-    uint32_t bits = 0;
-    for (int i = 0; i < maxlen; ++i) {
-        if ((i & 31) == 0) bits = L.mask[i >> 5][lane];
-        const bool live = i < len;
-        const bool hit = run && live && ((bits >> (i & 31)) & 1u);
+    const int lane = threadIdx.x;
+    const int nw = (len + 31) >> 5;
+    int w = 0;
+    uint32_t own = nw > 0 ? L.mask[0][lane] : 0u, bits = row_or(own);
+    for (;;) {
+        // (all lanes of a row hold the same bits and the same w)
+        while (__any(bits == 0u && w + 1 < nw)) {
+            const bool next = bits == 0u && w + 1 < nw;
+            const uint32_t m = next ? L.mask[w + 1][lane] : 0u;
+            const uint32_t o = row_or(m);
+            if (next) {
+                ++w;
+                own = m;
+                bits = o;
+            }
+        }
+        const bool live = bits != 0u;
+        if (!__any(live)) break;
+        const int at = live ? __builtin_ctz(bits) : 0;
+        bits &= bits - 1u;
+        const bool hit = run && live && ((own >> at) & 1u);
         if (__ballot(hit)) {
-            const int c = live ? L.rowlist[row * RGX_CCAP + i] : 0;
+            const int c = live ? L.list[w * 32 + at] : 0;
             const float4 *tab = (const float4 *)(L.tab + c * RGX_TAB);
             const int32_t pid = __float_as_int(L.tab[c * RGX_TAB + 19]);
             body(Entry<true>{tab, P.prims + pid, pid, c}, hit, live, Half<0>{});
@@ -985,8 +1044,8 @@ __device__ __forceinline__ void shade_rows(const MarchParams &P, const TileLds &
     }
 }
 
-// Shade, one ray at a time: every lane walks its own hits (the set bits of its mask over its
-// row's list), so the trip count is the longest hit list of a ray instead of the longest row list.
+// Shade, one ray at a time: every lane walks its own hits (the set bits of its mask over the
+// list), so the trip count is the longest hit list of a ray.
 // For bodies that need no sum over the rays of a row.  The order of a ray's hits is that of
 // shade_rows.  Only the entries that can reach half `half` of the slab's samples are visited; the
 // body gets Half<TAG>.  For the list's first 32 entries the ray goes by its own chords (own[half]: its
@@ -1009,7 +1068,7 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
         if (!__any(has)) break;
         int c = 0;
         if (has) {
-            c = L.rowlist[row * RGX_CCAP + w * 32 + __builtin_ctz(bits)];
+            c = L.list[w * 32 + __builtin_ctz(bits)];
             bits &= bits - 1u;
         }
         const float4 *tab = (const float4 *)(L.tab + c * RGX_TAB);
@@ -1029,9 +1088,9 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 //   words 4 .. 4 + RGX_REC_PIECES_MAX: where a backward can start in the middle of a tile (below);
 //   from word RGX_REC_HEAD, per iteration: WINDOW when a table was built, one LISTS per table, then TRAIL
 //   WINDOW: {tag | C, -, -, -}, pid[pad4(C)]            the table's Gaussians, by slot
-//   LISTS:  {tag | last << 8 | nw, len[4], -, -, -}, slot bytes of row r in pad4(len[r]) / 4 words
+//   LISTS:  {tag | one << 9 | last << 8 | nw, len[4], -, -, -}, slot bytes of row r in pad4(len[r]) / 4 words
 //           for r = 0..3, mask[nw][64], half[2][4][nw]   (the TileLds arrays of the same names;
-//           bytes and words past a row's length are junk)
+//           bytes and words past a row's length are junk).  one: the rows share one list, written once.
 //   TRAIL:  {tag | any_search, cover (float), sample-sum slot + 1, -}, found[64] when any_search
 //
 // Sample sums.  A record with room beyond RGX_REC_LIST_WORDS per tile also has a pool of slots
@@ -1059,6 +1118,7 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 #define RGX_REC_WINDOW 0x57000000u
 #define RGX_REC_LISTS 0x4C000000u
 #define RGX_REC_TRAIL 0x54000000u
+#define RGX_REC_ONE_LIST 0x200u    // LISTS: see above
 // Pieces of a tile's record.  A tile is a serial march for the forward, but with the rays' state at a few of its
 // iterations (transmittance, colour so far, position, step) the backward can replay the stretches between
 // them side by side, each with a wavefront of its own: a launch no longer lasts as long as its longest tile.
@@ -1189,24 +1249,16 @@ struct Recorder {
     {
         if (!on()) return;
         const int lane = threadIdx.x, row = lane >> 4;
-        const int l0 = __builtin_amdgcn_readlane(len, 0), l1 = __builtin_amdgcn_readlane(len, 16);
-        const int l2 = __builtin_amdgcn_readlane(len, 32), l3 = __builtin_amdgcn_readlane(len, 48);
-        const int nw = (max(max(l0, l1), max(l2, l3)) + 31) >> 5;
-        const int q0 = (l0 + 3) >> 2, q1 = (l1 + 3) >> 2, q2 = (l2 + 3) >> 2, q3 = (l3 + 3) >> 2;
-        const int size = 8 + q0 + q1 + q2 + q3 + nw * 72;
+        const int nw = (len + 31) >> 5, q = (len + 3) >> 2;
+        const int size = 8 + q + nw * 72;
         if (!fits(size)) return;
         uint32_t *it = reg + off;
-        if (lane == 0) {
-            it[0] = RGX_REC_LISTS | (last ? 0x100u : 0u) | (uint32_t)nw;
-            it[1] = (uint32_t)l0; it[2] = (uint32_t)l1; it[3] = (uint32_t)l2; it[4] = (uint32_t)l3;
-        }
-        const int base = 8 + (row > 0 ? q0 : 0) + (row > 1 ? q1 : 0) + (row > 2 ? q2 : 0);
-        const uint32_t *slots = (const uint32_t *)(L.rowlist + row * RGX_CCAP);
-        for (int i = lane & 15; i < ((len + 3) >> 2); i += 16) it[base + i] = slots[i];
-        const int mbase = 8 + q0 + q1 + q2 + q3;
-        for (int w = 0; w < nw; ++w) it[mbase + w * 64 + lane] = L.mask[w][lane];
+        if (lane < 5) it[lane] = lane == 0 ? RGX_REC_LISTS | RGX_REC_ONE_LIST | (last ? 0x100u : 0u) | (uint32_t)nw : (uint32_t)len;
+        if (lane < q) it[8 + lane] = ((const uint32_t *)L.list)[lane];
+        static_assert(RGX_CCAP <= 4 * 64, "a word of the list per lane");
+        for (int w = 0; w < nw; ++w) it[8 + q + w * 64 + lane] = L.mask[w][lane];
         if ((lane & 15) < 2) // two lanes per row: one per half
-            for (int w = 0; w < nw; ++w) it[mbase + nw * 64 + ((lane & 15) * 4 + row) * nw + w] = L.half[lane & 15][row][w];
+            for (int w = 0; w < nw; ++w) it[8 + q + nw * 64 + ((lane & 15) * 4 + row) * nw + w] = L.half[lane & 15][row][w];
         off += size;
     }
 
@@ -1408,11 +1460,13 @@ template <bool COUNT, int WALK, typename Body, typename Cn, typename Rv>
 __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLds &RL, const Rv &rv, int it, bool run, int &p0, Body body, Cn &cn)
 {
     const int lane = threadIdx.x, row = lane >> 4;
-    const int nw = (int)(rv.uni(it) & 0xffu);
+    const uint32_t item = rv.uni(it);
+    const int nw = (int)(item & 0xffu);
+    const bool one = item & RGX_REC_ONE_LIST;
     const int l0 = (int)rv.uni(it + 1), l1 = (int)rv.uni(it + 2), l2 = (int)rv.uni(it + 3), l3 = (int)rv.uni(it + 4);
-    const int q0 = (l0 + 3) >> 2, q1 = (l1 + 3) >> 2, q2 = (l2 + 3) >> 2, q3 = (l3 + 3) >> 2;
+    const int q0 = (l0 + 3) >> 2, q1 = one ? 0 : (l1 + 3) >> 2, q2 = one ? 0 : (l2 + 3) >> 2, q3 = one ? 0 : (l3 + 3) >> 2;
     const int len = row == 0 ? l0 : row == 1 ? l1 : row == 2 ? l2 : l3;
-    const int slots_at = it + 8 + (row > 0 ? q0 : 0) + (row > 1 ? q1 : 0) + (row > 2 ? q2 : 0); // the row's slot bytes start at this word
+    const int slots_at = it + 8 + (row > 0 && !one ? q0 : 0) + (row > 1 ? q1 : 0) + (row > 2 ? q2 : 0); // the row's slot bytes start at this word
     const int masks_at = it + 8 + q0 + q1 + q2 + q3 + lane;                                      // word w of this lane: masks_at + w * 64
     (void)RL.rowlist;
     if constexpr (WALK == WALK_NONE) {
@@ -1612,21 +1666,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 int cnt = real ? p0 : q0;
                 bool cut = real ? ov : qov;
                 float best = phase == 0 ? found : -1.0f;
-                auto filter = [&](auto search, auto part) {
-                    const float far = decltype(search)::value ? cover : hi;
-                    if (std::is_same<Rec, NoRecorder>::value ? __builtin_expect(plain, 1) : plain) filter_table<decltype(search)::value, decltype(part)::value, true>(L, C, lo, far, Q, cnt, cut, best, len, own, cn);
-                    else filter_table<decltype(search)::value, decltype(part)::value, false>(L, C, lo, far, Q, cnt, cut, best, len, own, cn);
-                };
-                using std::integral_constant;
-                if (!split) {
-                    if (phase == 0 && any_search) filter(std::true_type{}, integral_constant<int, 0>{});
-                    else filter(std::false_type{}, integral_constant<int, 0>{});
-                } else if (phase == 0) {
-                    if (any_search) filter(std::true_type{}, integral_constant<int, 1>{});
-                    else filter(std::false_type{}, integral_constant<int, 1>{});
-                } else {
-                    filter(std::false_type{}, integral_constant<int, 2>{});
-                }
+                filter_table(L, C, lo, phase == 0 && any_search ? cover : hi, Q, split ? 1 + phase : 0, plain, cnt, cut, best, len, own, cn);
                 if (real) {
                     p0 = cnt;
                     ov = cut;
@@ -1673,8 +1713,11 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
 template <typename Rv>
 __device__ __forceinline__ int lists_size(const Rv &rv, int it)
 {
-    const int nw = (int)(rv.uni(it) & 0xffu);
-    const int l0 = (int)rv.uni(it + 1), l1 = (int)rv.uni(it + 2), l2 = (int)rv.uni(it + 3), l3 = (int)rv.uni(it + 4);
+    const uint32_t item = rv.uni(it);
+    const int nw = (int)(item & 0xffu);
+    const int l0 = (int)rv.uni(it + 1);
+    if (item & RGX_REC_ONE_LIST) return 8 + ((l0 + 3) >> 2) + nw * 72;
+    const int l1 = (int)rv.uni(it + 2), l2 = (int)rv.uni(it + 3), l3 = (int)rv.uni(it + 4);
     return 8 + ((l0 + 3) >> 2) + ((l1 + 3) >> 2) + ((l2 + 3) >> 2) + ((l3 + 3) >> 2) + nw * 72;
 }
 
@@ -1773,10 +1816,10 @@ struct Replayer {
     __shared__ int32_t s_queue[RGX_QCAP];                             \
     __shared__ int32_t s_leafq[128];                                  \
     __shared__ __align__(16) float s_tab[RGX_CCAP * RGX_TAB];         \
-    __shared__ uint8_t s_rowlist[4 * RGX_CCAP];                       \
+    __shared__ __align__(4) uint8_t s_list[RGX_CCAP];                 \
     __shared__ uint32_t s_mask[RGX_MASK_WORDS][64];                   \
     __shared__ uint32_t s_half[2][4][RGX_MASK_WORDS];                 \
-    const TileLds L = {s_queue, s_leafq, s_tab, s_rowlist, s_mask, s_half}
+    const TileLds L = {s_queue, s_leafq, s_tab, s_list, s_mask, s_half}
 
 // lane -> pixel: row r = lane / 16 is the 4x4 block (r & 1, r >> 1) of the 8x8 tile
 __device__ __forceinline__ void lane_pixel(int px0, int py0, int &px, int &py)

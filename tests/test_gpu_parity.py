@@ -270,6 +270,48 @@ def test_tile_cooperative_collect_hit_sets_bit_exact(gx, orc, c0):
         np.testing.assert_array_equal(cnt.cpu().numpy(), c_cpu)
 
 
+@pytest.mark.parametrize("thin,spread", [(0.02, 0.5), (1e-3, 0.5), (2e-5, 0.5), (2e-8, 0.5), (0.3, 1.0)])
+def test_hit_sets_of_segments_that_end_at_a_surface(gx, orc, thin, spread):
+    """Segments that end exactly at a Gaussian's entry, one ulp before it and one after: the filter's shortcut must leave
+    these to the exact roots.  Gaussians as thin as ``thin`` along one axis, some 10 to 10^8 of their radii away (from
+    2e-5 on beyond the range of the shortcut, at 2e-8 of the plain division too), and around the eye."""
+    from raygaussx_amd import optix_utils as u_ox
+    cam = scenes.make_camera(0, 0, width=40, height=24)
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=500, seed=77))
+    rng = np.random.default_rng(5)
+    eye = cam.camera_center.numpy()
+    if spread == 1.0:      # the eye among them
+        sc["positions"] = (eye + rng.normal(size=(500, 3))).astype(np.float32)
+    else:
+        sc["positions"] = (sc["positions"] * spread).astype(np.float32)
+    sc["scales"] = rng.uniform(0.05, 0.2, (500, 3)).astype(np.float32)
+    sc["scales"][:, 1] = thin * rng.uniform(0.5, 1.5, 500).astype(np.float32)
+    rgb = np.ones((500, 3), np.float32)
+    d = gx.to_dev(sc)
+    prims = orc.pack_prims(eye, sc["positions"], sc["scales"], sc["quaternions"], sc["densities"], rgb)
+    gas = u_ox.AccelerationStructure(500, gx.DEV).build_from_gaussians(d["positions"], d["scales"], d["quaternions"], d["densities"])
+    ps = u_ox.pack_prims(gas, eye, d["positions"], d["scales"], d["quaternions"], d["densities"], torch.from_numpy(rgb).to(gx.DEV))
+    dirs = orc.ray_dirs(orc.camera_struct(cam))
+    R = len(dirs)
+    start = rng.uniform(0, 4, R).astype(np.float32) if spread == 1.0 else rng.uniform(0, 2, R).astype(np.float32)
+    t = orc.first_hit(prims, dirs, start, np.full(R, 100.0, np.float32))
+    hit = t > start      # (a ray that starts inside reports its start)
+    assert hit.sum() > (R // 20 if spread == 1.0 else R // 4)
+    t = np.where(hit, t, start + np.float32(1.0)).astype(np.float32)
+    dv = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).to(gx.DEV)
+    for cap in (512, 2):
+        for thi in (t, np.nextafter(t, np.float32(0)), np.nextafter(t, np.float32(1e9))):
+            tlo = np.maximum(start, thi - np.float32(0.3)).astype(np.float32)
+            want_n, want = orc.trace_segments(prims, dirs, tlo, thi, cap)
+            for uncounted in (False, True):
+                _step(f"segments ending at a surface, thin {thin}, cap {cap}, uncounted {uncounted}")
+                n, ids = u_ox.collect_tiles(gas, u_ox.camera_struct(cam), ps, dv(tlo), dv(thi), cap, uncounted=uncounted)
+                n, ids = n.cpu().numpy(), ids.cpu().numpy()
+                np.testing.assert_array_equal(n, want_n)
+                if cap == 512:
+                    np.testing.assert_array_equal(np.sort(np.where(ids < 0, 1 << 30, ids), 1), np.sort(np.where(want < 0, 1 << 30, want), 1))
+
+
 def _check_grads(gx, got, want, keys=("positions", "scales", "quaternions", "densities", "color_features")):
     for k in keys:
         cos, rel = gx.cos_rel(got[k], want[k])
