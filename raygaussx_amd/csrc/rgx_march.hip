@@ -863,6 +863,25 @@ __device__ __forceinline__ float filter_margin(float c)
     return c >= 3.0f && c <= 0x1p30f ? fmaf(__builtin_amdgcn_sqrtf(c + 1.0f), 41.0f * 0x1p-24f, 66.0f * 0x1p-24f) : INFINITY;
 }
 
+// Adds a hit's samples to the half's sums: those within the cut-off, by the execution mask (a comparison that writes it
+// and a scalar move that restores it cost less than a comparison, two wait states and a select).
+__device__ __forceinline__ void accumulate_samples(HitSetup hs, float4 col, float (&sg)[RGX_CHUNK_SIZE], float (&cr)[RGX_CHUNK_SIZE],
+                                                   float (&cg)[RGX_CHUNK_SIZE], float (&cb)[RGX_CHUNK_SIZE])
+{
+    const uint64_t lanes = __builtin_amdgcn_read_exec();
+#pragma unroll
+    for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
+        const float gw = gauss_weight(hs.power);
+        asm("v_cmpx_lt_f32_e32 vcc, %[p], %[cut]\n\tv_fmac_f32_e32 %[a], %[w], %[g]\n\tv_fmac_f32_e32 %[r], %[x], %[g]\n\t"
+            "v_fmac_f32_e32 %[gg], %[y], %[g]\n\tv_fmac_f32_e32 %[b], %[z], %[g]\n\ts_mov_b64 exec, %[l]"
+            : [a] "+v"(sg[i]), [r] "+v"(cr[i]), [gg] "+v"(cg[i]), [b] "+v"(cb[i])
+            : [p] "v"(hs.power), [cut] "v"(hs.cut), [g] "v"(gw), [x] "v"(col.x), [y] "v"(col.y), [z] "v"(col.z), [w] "v"(col.w), [l] "s"(lanes)
+            : "vcc");
+        hs.power += hs.inc;
+        hs.inc += hs.inc_st;
+    }
+}
+
 // What one lane asks of the candidate table in this iteration.
 struct LaneQuery {
     f3 dir;
@@ -1894,17 +1913,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                     float k;
                     e.frame(U, V, W, inv, k);
                     HitSetup hs = hit_setup(U, V, W, inv, k, e.prim->pos4, dir, rdt, dt);
-                    const float rho = col.w;
-#pragma unroll
-                    for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
-                        const float gw = hs.power < hs.cut ? gauss_weight(hs.power) : 0.0f;
-                        sg[i] = fmaf(rho, gw, sg[i]);
-                        cr[i] = fmaf(col.x, gw, cr[i]);
-                        cg[i] = fmaf(col.y, gw, cg[i]);
-                        cb[i] = fmaf(col.z, gw, cb[i]);
-                        hs.power += hs.inc;
-                        hs.inc += hs.inc_st;
-                    }
+                    accumulate_samples(hs, col, sg, cr, cg, cb);
                 }
             };
             auto blend = [&](bool second_chunk) { // gaussians_aabb.cu:195-201
@@ -2614,17 +2623,7 @@ __global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const Ma
                     float k;
                     e.frame(U, V, W, inv, k);
                     HitSetup hs = hit_setup(U, V, W, inv, k, e.prim->pos4, dir, rdt, dt);
-                    const float rho = col.w;
-#pragma unroll
-                    for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
-                        const float gw = hs.power < hs.cut ? gauss_weight(hs.power) : 0.0f;
-                        sg[i] = fmaf(rho, gw, sg[i]);
-                        cr[i] = fmaf(col.x, gw, cr[i]);
-                        cg[i] = fmaf(col.y, gw, cg[i]);
-                        cb[i] = fmaf(col.z, gw, cb[i]);
-                        hs.power += hs.inc;
-                        hs.inc += hs.inc_st;
-                    }
+                    accumulate_samples(hs, col, sg, cr, cg, cb);
                 }
             };
             // The half's sums over the copies, four samples per copy; they are blended (a ray without hits has none, and
@@ -3147,19 +3146,22 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                     // the forward's sample recurrence (the mask is the one the forward blended with)
                     const HitSetup hs = hit_setup(U, V, W, inv, k, e5, dir, rdt0, dt);
                     const f3 Mx0 = hs.Mx0, Md = hs.Md;
-                    const float cut = hs.cut, inc_st = hs.inc_st;
+                    const float cut0 = hs.cut, cut1 = use_second ? cut0 : -1.0f, inc_st = hs.inc_st; // (the second chunk's gate is in its cut-off)
+                    const uint64_t lanes = __builtin_amdgcn_read_exec();
                     float power = hs.power, inc = hs.inc;
                     float s0 = 0.f, s1 = 0.f, s2 = 0.f, gc = 0.f;
 #pragma unroll
                     for (int i = 0; i < RGX_BUFFER_SIZE; ++i) {
-                        const bool on = power < cut && (i < RGX_CHUNK_SIZE || use_second);
-                        const float wd = on ? gauss_weight(power) : 0.0f;
-                        const float y = fmaf(PA[i], dcg, PB[i]) * wd;
+                        const float wd = gauss_weight(power);
+                        float y = fmaf(PA[i], dcg, PB[i]) * wd;
                         const float u = (float)i - 15.5f;
-                        s0 += y;
-                        s1 = fmaf(y, u, s1);
-                        s2 = fmaf(y, u * u, s2);
-                        gc = fmaf(wd, PA[i], gc);
+                        // (within the cut-off, by the execution mask: see accumulate_samples)
+                        asm("v_cmpx_lt_f32_e32 vcc, %[p], %[cut]\n\tv_add_f32_e32 %[s0], %[y], %[s0]\n\tv_fmac_f32_e32 %[s1], %[u], %[y]\n\t"
+                            "v_fmac_f32_e32 %[s2], %[uu], %[y]\n\tv_fmac_f32_e32 %[gc], %[a], %[w]\n\ts_mov_b64 exec, %[l]"
+                            : [s0] "+v"(s0), [s1] "+v"(s1), [s2] "+v"(s2), [gc] "+v"(gc)
+                            : [p] "v"(power), [cut] "v"(i < RGX_CHUNK_SIZE ? cut0 : cut1), [y] "v"(y), [a] "v"(PA[i]), [w] "v"(wd),
+                              [u] "i"(__builtin_bit_cast(uint32_t, u)), [uu] "i"(__builtin_bit_cast(uint32_t, u * u)), [l] "s"(lanes)
+                            : "vcc");
                         power += inc;
                         inc += inc_st;
                     }
