@@ -273,6 +273,16 @@ struct Frustum {
     f3 dc;       // the tile's central direction
     float delta; // no ray of the tile is further than this angle from dc
     float t0, t1, pad;
+    float near2, far2; // frustum_misses: bounds on the squares of twice the distance to a box's furthest and of that to its nearest point
+    __device__ __forceinline__ void range(float from, float to, float padding)
+    {
+        t0 = from;
+        t1 = to;
+        pad = padding;
+        const float near_t = t0 - pad, far_t = t1 + pad;
+        near2 = near_t > 0.f ? near_t * near_t * (4.0f * 0.9999f) : -1.0f;
+        far2 = far_t * far_t * 1.0001f;
+    }
     int32_t cut_node; // per lane: one node of the tile's cut through the tree (frustum_cut), or -1
     int cut_n;        // nodes in the cut (wave-uniform); 0: sweeps start at the root
 };
@@ -313,25 +323,25 @@ __device__ __forceinline__ void frustum_planes(const RgxCamera &cam, int px0, in
     for (int k = 0; k < 4; ++k) F.n[k] = mk3(uni(F.n[k].x), uni(F.n[k].y), uni(F.n[k].z));
 }
 
-__device__ __forceinline__ bool frustum_overlaps(const Frustum &F, float4 a, float4 b)
+// Whether the box [a, b] may meet the frustum: in twice its centre c and extent e from the eye, plane k's distance to the
+// corner furthest inside is n.c - |n|.e, six multiply-adds and no select per axis (a step of the descent costs a
+// third less than with the corner picked by the normal's signs, and 24 scalar registers of those signs are free).  A large
+// box's near corner comes out of large terms: e is widened by more than their rounding (16 ulps).
+__device__ __forceinline__ bool frustum_misses(const Frustum &F, float4 a, float4 b)
 {
     const f3 lo = mk3(a.x - F.o.x, a.y - F.o.y, a.z - F.o.z), hi = mk3(b.x - F.o.x, b.y - F.o.y, b.z - F.o.z);
-    bool out = false;
+    const f3 c = lo + hi, e = (hi - lo) * (1.0f + 0x1p-19f);
+    float d[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const f3 n = F.n[k];
-        // box corner closest to the inside of plane k
-        const float d = (n.x * (n.x > 0.f ? lo.x : hi.x) + n.y * (n.y > 0.f ? lo.y : hi.y)) + n.z * (n.z > 0.f ? lo.z : hi.z);
-        out |= d > F.pad;
+        d[k] = fmaf(n.x, c.x, fmaf(-fabsf(n.x), e.x, fmaf(n.y, c.y, fmaf(-fabsf(n.y), e.y, fmaf(n.z, c.z, -fabsf(n.z) * e.z)))));
     }
-    // distance shell
+    // distance shell (dmax: of twice the furthest corner)
     const float nx = fmaxf(fmaxf(lo.x, -hi.x), 0.f), ny = fmaxf(fmaxf(lo.y, -hi.y), 0.f), nz = fmaxf(fmaxf(lo.z, -hi.z), 0.f);
-    const float fx = fmaxf(fabsf(lo.x), fabsf(hi.x)), fy = fmaxf(fabsf(lo.y), fabsf(hi.y)), fz = fmaxf(fabsf(lo.z), fabsf(hi.z));
-    const float dmin2 = (nx * nx + ny * ny) + nz * nz, dmax2 = (fx * fx + fy * fy) + fz * fz;
-    const float near_t = F.t0 - F.pad, far_t = F.t1 + F.pad;
-    out |= near_t > 0.f && dmax2 < near_t * near_t * 0.9999f;
-    out |= dmin2 > far_t * far_t * 1.0001f;
-    return !out;
+    const float fx = fabsf(c.x) + e.x, fy = fabsf(c.y) + e.y, fz = fabsf(c.z) + e.z;
+    const float dmin2 = fmaf(nx, nx, fmaf(ny, ny, nz * nz)), dmax2 = fmaf(fx, fx, fmaf(fy, fy, fz * fz));
+    return (fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3])) > 2.0f * F.pad) | (dmax2 < F.near2) | (dmin2 > F.far2);
 }
 
 // Candidate table.  A Gaussian that survives the sweep is turned, by the lane that found
@@ -385,6 +395,12 @@ __device__ __forceinline__ bool plain_roots(f3 inv, float c)
     return lo >= 0x1p-23f && hi <= 0x1p22f && fabsf(c) >= 0x1p-46f && fabsf(c) <= 0x1p46f;
 }
 
+// how many of the mask's lanes come before this one
+__device__ __forceinline__ int rank_in(uint64_t mask)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
 struct Sweep {
     int qn;  // stack entries (wave-uniform)
     int lqn; // leaves waiting for their ellipsoid test (wave-uniform)
@@ -403,6 +419,39 @@ __device__ __forceinline__ void sweep_begin(const MarchParams &P, Sweep &S, cons
     __syncthreads();
 }
 
+// A leaf's ellipsoid against the frustum, and the range of distances from the eye that bounds it along the tile's rays.
+// (Bounds only: hardware reciprocal and square root and multiply-adds, their last-bit errors are inside the 1.001 factors.)
+__device__ __forceinline__ bool leaf_meets(const Frustum &F, const Prim &p, f3 U, f3 V, f3 W, float &dmin, float &dmax)
+{
+    auto dot = [](f3 a, f3 b) { return fmaf(a.x, b.x, fmaf(a.y, b.y, a.z * b.z)); };
+    const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
+    // semi-axes of the k-sigma ellipsoid: k * scale = 1 / inv_inter
+    const f3 ax = mk3(__builtin_amdgcn_rcpf(p.inv_inter4.x), __builtin_amdgcn_rcpf(p.inv_inter4.y), __builtin_amdgcn_rcpf(p.inv_inter4.z));
+    // how far the ellipsoid reaches beyond its centre along n
+    auto extent = [&](f3 n) {
+        const float a = dot(U, n) * ax.x, b = dot(V, n) * ax.y, c = dot(W, n) * ax.z;
+        return __builtin_amdgcn_sqrtf(fmaf(a, a, fmaf(b, b, c * c))) * 1.001f;
+    };
+    const float dist = __builtin_amdgcn_sqrtf(dot(O, O));
+    const float amax = fmaxf(ax.x, fmaxf(ax.y, ax.z));
+    const float rad = amax * 1.001f + 1e-5f * dist + F.pad;
+    // Along a ray of direction d the ellipsoid lies within (centre - eye).d -+ |A R^T d|.  For
+    // d = dc that is depth -+ h; a ray at angle <= delta from dc moves the centre term by at
+    // most |depth| delta^2 / 2 + |offset of the centre from the central ray| delta and the
+    // extent by at most amax delta.  The bounding sphere's shell bounds the same range.
+    const float depth = -dot(O, F.dc);
+    const f3 off = mk3(fmaf(depth, F.dc.x, O.x), fmaf(depth, F.dc.y, O.y), fmaf(depth, F.dc.z, O.z));
+    const float ext = extent(F.dc);
+    const float slack = 1.5f * (0.5f * fabsf(depth) * F.delta * F.delta + (__builtin_amdgcn_sqrtf(dot(off, off)) + amax) * F.delta) +
+                        1e-5f * dist + F.pad;
+    dmin = fmaxf(dist - rad, depth - ext - slack);
+    dmax = fminf(dist + rad, depth + ext + slack);
+    bool ok = (p.inv_inter4.w == p.inv_inter4.w) & (dmax >= F.t0) & (dmin <= F.t1); // k is NaN below the density threshold: never hit
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ok = ok & !(-dot(F.n[k], O) - extent(F.n[k]) > F.pad); // centre - eye = -O
+    return ok;
+}
+
 // The tile's cut through the tree.  Every sweep of a tile tests the same top of the tree against the
 // same four planes -- a dozen steps of one to a few dozen nodes, each waiting on memory.  Done once
 // instead: descend from the root, level by level, keeping the nodes that meet the frustum at any
@@ -414,9 +463,7 @@ __device__ __forceinline__ void frustum_cut(const MarchParams &P, Frustum &F, fl
     const uint64_t lt = (1ull << lane) - 1ull;
     const float4 *nodes4 = (const float4 *)P.nodes;
     const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
-    F.t0 = 0.f;
-    F.t1 = INFINITY; // no distance shell
-    F.pad = 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f);
+    F.range(0.f, INFINITY, 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f)); // no distance shell
     int32_t node = lane == 0 && P.n > 0 ? 0 : -1;
     int count = P.n > 0 ? 1 : 0;
     for (int level = 0; level < 64 && count > 0; ++level) {
@@ -425,7 +472,7 @@ __device__ __forceinline__ void frustum_cut(const MarchParams &P, Frustum &F, fl
         if ((uint32_t)node < n_nodes) {
             const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
             right = P.right[max(0, min(node, (int32_t)P.n - 2))]; // with the box, not after the test (n = 1: no internal node, word 0 of the padded array)
-            if (frustum_overlaps(F, a, b)) {
+            if (!frustum_misses(F, a, b)) {
                 left = __float_as_int(a.w);
                 inner = left >= 0;
                 keep = !inner;
@@ -461,116 +508,73 @@ __device__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int3
 {
     plain = true;
     const int lane = threadIdx.x;
-    const uint64_t lt = (1ull << lane) - 1ull;
     const float4 *nodes4 = (const float4 *)P.nodes;
     const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
     int C = 0;
-    while ((S.qn > 0 || S.lqn > 0) && C < RGX_CCAP) {
-        if (S.lqn >= 64 || S.qn == 0) {
-            // Leaves whose boxes passed wait in a queue until there are 64 of them (or no node is
-            // left): the expensive part -- fetch the Gaussian, test its ellipsoid, build its table
-            // entry -- then runs with every lane busy, not with the few leaves one step turns up.
-            const int m = S.lqn < 64 ? S.lqn : 64;
-            bool leaf_hit = lane < m;
-            const int32_t left = leaf_hit ? s_leafq[S.lqn - m + lane] : 0;
-            S.lqn -= m;
-            Prim p;
-            f3 U, V, W;
-            float dmin = 0.f, dmax = 0.f;
-            if (leaf_hit) {
-                p = P.prims[~left];
-                quat_to_cols(p.quat4, U, V, W);
-                const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
-                // semi-axes of the k-sigma ellipsoid: k * scale = 1 / inv_inter
-                // (bounds only: hardware reciprocal and square root, their last-bit error is inside the 1.001 factors)
-                const f3 ax = mk3(__builtin_amdgcn_rcpf(p.inv_inter4.x), __builtin_amdgcn_rcpf(p.inv_inter4.y), __builtin_amdgcn_rcpf(p.inv_inter4.z));
-                const float dist = __builtin_amdgcn_sqrtf(dot3(O, O));
-                const float amax = fmaxf(ax.x, fmaxf(ax.y, ax.z));
-                const float rad = amax * 1.001f + 1e-5f * dist + F.pad;
-                // Along a ray of direction d the ellipsoid lies within (centre - eye).d -+ |A R^T d|.  For
-                // d = dc that is depth -+ h; a ray at angle <= delta from dc moves the centre term by at
-                // most |depth| delta^2 / 2 + |offset of the centre from the central ray| delta and the
-                // extent by at most amax delta.  The bounding sphere's shell bounds the same range.
-                const float depth = -dot3(O, F.dc);
-                const f3 off = mk3(-O.x - depth * F.dc.x, -O.y - depth * F.dc.y, -O.z - depth * F.dc.z);
-                const float eu = dot3(U, F.dc) * ax.x, ev = dot3(V, F.dc) * ax.y, ew = dot3(W, F.dc) * ax.z;
-                const float ext = __builtin_amdgcn_sqrtf((eu * eu + ev * ev) + ew * ew) * 1.001f;
-                const float slack = 1.5f * (0.5f * fabsf(depth) * F.delta * F.delta + (__builtin_amdgcn_sqrtf(dot3(off, off)) + amax) * F.delta) +
-                                    1e-5f * dist + F.pad;
-                dmin = fmaxf(dist - rad, depth - ext - slack);
-                dmax = fminf(dist + rad, depth + ext + slack);
-                bool ok = p.inv_inter4.w == p.inv_inter4.w; // k is NaN below the density threshold: never hit
-                ok = ok && dmax >= F.t0 && dmin <= F.t1;
-    #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const f3 n = F.n[k];
-                    // the ellipsoid reaches h beyond its centre along n; centre - eye = -O
-                    const float hu = dot3(U, n) * ax.x, hv = dot3(V, n) * ax.y, hw = dot3(W, n) * ax.z;
-                    const float h = __builtin_amdgcn_sqrtf((hu * hu + hv * hv) + hw * hw) * 1.001f;
-                    ok = ok && !(-dot3(n, O) - h > F.pad);
-                }
-                leaf_hit = ok;
-            }
-            // the table takes what it has room for; the rest goes back to the queue for the next table
-            const int rank = __popcll(__ballot(leaf_hit) & lt), room = RGX_CCAP - C;
-            const bool back = leaf_hit && rank >= room;
-            leaf_hit = leaf_hit && rank < room;
-            const uint64_t bb = __ballot(back);
-            if (back) s_leafq[S.lqn + __popcll(bb & lt)] = left;
-            S.lqn += __popcll(bb);
-            const uint64_t bl = __ballot(leaf_hit);
-            if (leaf_hit) {
-                float4 *dst = (float4 *)(s_tab + (C + rank) * RGX_TAB);
-                const f3 inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
-                const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
-                dst[0] = make_float4(U.x, U.y, U.z, dmin);
-                dst[1] = make_float4(V.x, V.y, V.z, dmax);
-                dst[2] = make_float4(W.x, W.y, W.z, p.inv_inter4.w);
-                const f3 Oe = apply_sinv_rt(O, U, V, W, inv);
-                const float c = fmaf(Oe.x, Oe.x, fmaf(Oe.y, Oe.y, fmaf(Oe.z, Oe.z, -1.0f)));
-                dst[3] = make_float4(inv.x, inv.y, inv.z, c);
-                dst[4] = make_float4(Oe.x, Oe.y, Oe.z, __int_as_float(~left));
-                leaf_hit = plain_roots(inv, c); // from here on: this lane's entry is a plain one
-            }
-            plain = plain && __ballot(leaf_hit) == bl;
-            C += __popcll(bl);
-            __syncthreads();
-            continue;
-        }
-        // a step of the descent: up to 64 nodes, one per lane
-        const int m = S.qn > RGX_QCAP - RGX_DFS_MARGIN ? 1 : (S.qn < 64 ? S.qn : 64);
-        const int base = S.qn - m;
-        int32_t node = -1;
-        if (lane < m) node = s_queue[base + lane];
-        __syncthreads();
-        S.qn = base;
-        bool leaf_hit = false, inner_hit = false;
-        int32_t left = 0, right = 0;
-        if ((uint32_t)node < n_nodes) {
-            const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
+    while (C < RGX_CCAP) {
+        while (S.qn > 0 && S.lqn < 64) {
+            // A step of the descent: up to 64 nodes, one per lane.  (Lanes beyond them repeat the last one, and their results are
+            // masked: straight-line code.  The wavefront's LDS accesses take place in program order.)
+            const int m = S.qn > RGX_QCAP - RGX_DFS_MARGIN ? 1 : (S.qn < 64 ? S.qn : 64);
+            const int base = S.qn - m;
+            const uint32_t popped = (uint32_t)s_queue[base + min(lane, m - 1)], node = min(popped, n_nodes - 1u);
+            __builtin_amdgcn_wave_barrier();
+            const float4 *box = (const float4 *)((const char *)nodes4 + ((uint64_t)node << 5));
+            const float4 a = box[0], b = box[1];
             // the right child is fetched along with the box, not after the test: one memory round trip per step, not two
-            right = P.right[max(0, min(node, (int32_t)P.n - 2))];
-            if (frustum_overlaps(F, a, b)) {
-                left = __float_as_int(a.w);
-                leaf_hit = left < 0;
-                inner_hit = !leaf_hit;
+            const int32_t right = P.right[min(node, (uint32_t)max((int32_t)P.n - 2, 0))]; // (a leaf has none)
+            const int32_t left = __float_as_int(a.w);
+            const uint64_t pass = (~0ull >> (64 - m)) & ~__ballot(frustum_misses(F, a, b)) & __ballot(popped < n_nodes);
+            const uint64_t leaves = pass & __ballot(left < 0), inner = pass & ~leaves;
+            if (lane == 0) cn.nodes += (unsigned)m;
+            if (__builtin_amdgcn_inverse_ballot_w64(leaves)) s_leafq[S.lqn + rank_in(leaves)] = left; // fewer than 64 waiting + at most 64 new <= 128
+            S.lqn += __popcll(leaves);
+            S.qn = base + 2 * __popcll(inner);
+            if (__builtin_expect(S.qn <= RGX_QCAP, 1)) {
+                if (__builtin_amdgcn_inverse_ballot_w64(inner)) {
+                    const int pos = base + 2 * rank_in(inner);
+                    s_queue[pos] = right;
+                    s_queue[pos + 1] = left;
+                }
+            } else { // cannot happen (see RGX_DFS_MARGIN); if it did, the drop is counted, not silent
+                S.qn = base;
+                if (lane == 0 && P.faults) atomicAdd(&P.faults[1], (uint32_t)__popcll(inner));
             }
+            __builtin_amdgcn_wave_barrier();
         }
-        if (lane == 0) cn.nodes += (unsigned)m;
-        const uint64_t bl = __ballot(leaf_hit), bi = __ballot(inner_hit);
-        if (leaf_hit) s_leafq[S.lqn + __popcll(bl & lt)] = left; // fewer than 64 waiting + at most 64 new <= 128
-        S.lqn += __popcll(bl);
-        if (inner_hit) {
-            const int pos = S.qn + 2 * __popcll(bi & lt);
-            if (pos + 1 < RGX_QCAP) { // cannot fail (see RGX_DFS_MARGIN); if it did, the drop is counted, not silent
-                s_queue[pos] = right;
-                s_queue[pos + 1] = left;
-            } else if (P.faults) {
-                atomicAdd(&P.faults[1], 1u);
-            }
+        if (S.lqn == 0) break;
+        // Leaves whose boxes passed wait in a queue until there are 64 of them (or no node is
+        // left): the expensive part -- fetch the Gaussian, test its ellipsoid, build its table
+        // entry -- then runs with every lane busy, not with the few leaves one step turns up.
+        const int m = S.lqn < 64 ? S.lqn : 64;
+        S.lqn -= m;
+        const int32_t left = s_leafq[S.lqn + min(lane, m - 1)]; // (as in a step of the descent)
+        const Prim p = P.prims[(uint32_t)~left];
+        f3 U, V, W;
+        quat_to_cols(p.quat4, U, V, W);
+        float dmin, dmax;
+        uint64_t hits = (~0ull >> (64 - m)) & __ballot(leaf_meets(F, p, U, V, W, dmin, dmax));
+        const int rank = rank_in(hits), room = RGX_CCAP - C;
+        if (__popcll(hits) > room) {
+            // the table takes what it has room for; the rest goes back to the queue for the next table
+            const uint64_t back = hits & __ballot(rank >= room);
+            if (__builtin_amdgcn_inverse_ballot_w64(back)) s_leafq[S.lqn + rank - room] = left;
+            S.lqn += __popcll(back);
+            hits &= ~back;
         }
-        S.qn += 2 * __popcll(bi);
-        if (S.qn > RGX_QCAP) S.qn = RGX_QCAP;
+        const f3 inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
+        const f3 Oe = apply_sinv_rt(mk3(p.pos4.x, p.pos4.y, p.pos4.z), U, V, W, inv);
+        const float c = fmaf(Oe.x, Oe.x, fmaf(Oe.y, Oe.y, fmaf(Oe.z, Oe.z, -1.0f)));
+        if (__builtin_amdgcn_inverse_ballot_w64(hits)) {
+            float4 *dst = (float4 *)(s_tab + (C + rank) * RGX_TAB);
+            dst[0] = make_float4(U.x, U.y, U.z, dmin);
+            dst[1] = make_float4(V.x, V.y, V.z, dmax);
+            dst[2] = make_float4(W.x, W.y, W.z, p.inv_inter4.w);
+            dst[3] = make_float4(inv.x, inv.y, inv.z, c);
+            dst[4] = make_float4(Oe.x, Oe.y, Oe.z, __int_as_float(~left));
+        }
+        plain = plain && (hits & ~__ballot(plain_roots(inv, c))) == 0;
+        C += __popcll(hits);
         __syncthreads();
     }
     done = S.qn == 0 && S.lqn == 0;
@@ -1587,9 +1591,7 @@ struct Window {
 
 __device__ __forceinline__ void frustum_range(Frustum &F, float t0, float t1)
 {
-    F.t0 = t0;
-    F.t1 = t1;
-    F.pad = 2.0f * RGX_PAD_REL * fmaxf(t1, 1.0f);
+    F.range(t0, t1, 2.0f * RGX_PAD_REL * fmaxf(t1, 1.0f));
 }
 
 // One slab iteration's work on the candidate tables, in two phases that share a single copy of
@@ -2150,34 +2152,7 @@ __device__ __forceinline__ bool leaf_entry(const MarchParams &P, const Frustum &
     const Prim p = P.prims[~left];
     quat_to_cols(p.quat4, e.U, e.V, e.W);
     const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
-    // semi-axes of the k-sigma ellipsoid: k * scale = 1 / inv_inter
-    // (bounds only: hardware reciprocal and square root, their last-bit error is inside the 1.001 factors)
-    const f3 ax = mk3(__builtin_amdgcn_rcpf(p.inv_inter4.x), __builtin_amdgcn_rcpf(p.inv_inter4.y), __builtin_amdgcn_rcpf(p.inv_inter4.z));
-    const float dist = __builtin_amdgcn_sqrtf(dot3(O, O));
-    const float amax = fmaxf(ax.x, fmaxf(ax.y, ax.z));
-    const float rad = amax * 1.001f + 1e-5f * dist + F.pad;
-    // Along a ray of direction d the ellipsoid lies within (centre - eye).d -+ |A R^T d|.  For
-    // d = dc that is depth -+ h; a ray at angle <= delta from dc moves the centre term by at
-    // most |depth| delta^2 / 2 + |offset of the centre from the central ray| delta and the
-    // extent by at most amax delta.  The bounding sphere's shell bounds the same range.
-    const float depth = -dot3(O, F.dc);
-    const f3 off = mk3(-O.x - depth * F.dc.x, -O.y - depth * F.dc.y, -O.z - depth * F.dc.z);
-    const float eu = dot3(e.U, F.dc) * ax.x, ev = dot3(e.V, F.dc) * ax.y, ew = dot3(e.W, F.dc) * ax.z;
-    const float ext = __builtin_amdgcn_sqrtf((eu * eu + ev * ev) + ew * ew) * 1.001f;
-    const float slack = 1.5f * (0.5f * fabsf(depth) * F.delta * F.delta + (__builtin_amdgcn_sqrtf(dot3(off, off)) + amax) * F.delta) +
-                        1e-5f * dist + F.pad;
-    e.dmin = fmaxf(dist - rad, depth - ext - slack);
-    e.dmax = fminf(dist + rad, depth + ext + slack);
-    bool ok = p.inv_inter4.w == p.inv_inter4.w; // k is NaN below the density threshold: never hit
-    ok = ok && e.dmax >= F.t0 && e.dmin <= F.t1;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const f3 n = F.n[k];
-        // the ellipsoid reaches h beyond its centre along n; centre - eye = -O
-        const float hu = dot3(e.U, n) * ax.x, hv = dot3(e.V, n) * ax.y, hw = dot3(e.W, n) * ax.z;
-        const float h = __builtin_amdgcn_sqrtf((hu * hu + hv * hv) + hw * hw) * 1.001f;
-        ok = ok && !(-dot3(n, O) - h > F.pad);
-    }
+    const bool ok = leaf_meets(F, p, e.U, e.V, e.W, e.dmin, e.dmax);
     if (ok) {
         e.k = p.inv_inter4.w;
         e.inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
@@ -2221,9 +2196,7 @@ __device__ __forceinline__ void team_frustum_cut(const MarchParams &P, Frustum &
     const uint64_t lt = (1ull << tp.lane) - 1ull;
     const float4 *nodes4 = (const float4 *)P.nodes;
     const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
-    F.t0 = 0.f;
-    F.t1 = INFINITY;
-    F.pad = 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f);
+    F.range(0.f, INFINITY, 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f));
     int32_t node = threadIdx.x == 0 && P.n > 0 ? 0 : -1;
     int count = P.n > 0 ? 1 : 0;
     for (int level = 0; level < 64 && count > 0; ++level) {
@@ -2232,7 +2205,7 @@ __device__ __forceinline__ void team_frustum_cut(const MarchParams &P, Frustum &
         if ((uint32_t)node < n_nodes) {
             const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
             right = P.right[max(0, min(node, (int32_t)P.n - 2))];
-            if (frustum_overlaps(F, a, b)) {
+            if (!frustum_misses(F, a, b)) {
                 left = __float_as_int(a.w);
                 inner = left >= 0;
                 keep = !inner;
@@ -2300,7 +2273,7 @@ __device__ int team_sweep_next(const MarchParams &P, Sweep &S, const Frustum &F,
         if ((uint32_t)node < n_nodes) {
             const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
             right = P.right[max(0, min(node, (int32_t)P.n - 2))];
-            if (frustum_overlaps(F, a, b)) {
+            if (!frustum_misses(F, a, b)) {
                 left = __float_as_int(a.w);
                 leaf_hit = left < 0;
                 inner_hit = !leaf_hit;
