@@ -809,6 +809,8 @@ struct Entry {
     const Prim *prim;
     int32_t pid;       // index in Morton order
     int slot;          // its slot in the candidate table of the current window
+    __device__ __forceinline__ float4 position() const { return prim->pos4; }
+    __device__ __forceinline__ float4 colour() const { return prim->rgba4; }
     __device__ __forceinline__ void frame(f3 &U, f3 &V, f3 &W, f3 &inv, float &k) const
     {
         if constexpr (FROM_TABLE) {
@@ -825,6 +827,26 @@ struct Entry {
             inv = mk3(i4.x, i4.y, i4.z);
             k = i4.w;
         }
+    }
+};
+
+// An entry of the replay whose record has been asked for beforehand (replay_lists).
+struct EntryAhead {
+    const float4 *tab;
+    const Prim *prim;
+    int32_t pid;
+    int slot;
+    float4 pos4, inv4, rgba4;
+    __device__ __forceinline__ float4 position() const { return pos4; }
+    __device__ __forceinline__ float4 colour() const { return rgba4; }
+    __device__ __forceinline__ void frame(f3 &U, f3 &V, f3 &W, f3 &inv, float &k) const
+    {
+        const float *f = (const float *)tab; // as in Entry<false>
+        U = mk3(f[0], f[RGX_CCAP], f[2 * RGX_CCAP]);
+        V = mk3(f[3 * RGX_CCAP], f[4 * RGX_CCAP], f[5 * RGX_CCAP]);
+        W = mk3(f[6 * RGX_CCAP], f[7 * RGX_CCAP], f[8 * RGX_CCAP]);
+        inv = mk3(inv4.x, inv4.y, inv4.z);
+        k = inv4.w;
     }
 };
 
@@ -1118,19 +1140,22 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 //
 // Sample sums.  A record with room beyond RGX_REC_LIST_WORDS per tile also has a pool of slots
 // shared by all tiles: per slab iteration that blends something, the per-sample density and colour
-// sums the forward blended -- sum rho w as [32 samples][64 rays], then sum rgb rho w as
-// [32 samples][64 rays][3].  The
+// sums the forward blended -- sum rho w, then the red, green and blue of sum rgb rho w, each as [8][64 rays][4 consecutive
+// samples]: 16 bytes per lane and access, and in registers a multiple of the even-aligned tuples that loads land
+// in (three colours of a sample together take four registers while they are on their way).  The
 // backward reads them back instead of walking the hit lists a second time to rebuild them.  The
 // iteration's TRAIL item names its slot (word 2: slot + 1, 0 = none).  Tiles take slots from a
 // bump counter; a tile that found the pool empty is marked lists-only (status 0).
 #define RGX_REC_LIST_WORDS 16384   // hit-list words per tile when the record also holds sample sums
 #define RGX_SUM_SLOT_WORDS 8192    // 32 samples x 64 rays x 4 words
 // With RgxMarch::record_format 1 a slot keeps the colour sums in half precision: the density sums as before
-// ([32 samples][64 rays] floats: the transmittance must replay bit for bit), then per chunk of 16 samples and ray
+// (floats: the transmittance must replay bit for bit), then per chunk of 16 samples and ray
 // the 48 colour sums divided by a power of two that brings the largest to [1/2, 1) and rounded to binary16, two to a
 // word ([2 chunks][24 words][64 rays]), then that power of two per chunk and ray ([2][64] floats).  The scale makes
 // the format safe for any density (plain binary16 overflows at 65504); the sums keep 11 bits relative to each
 // value down to 2^-14 of the chunk's largest.
+typedef float quad __attribute__((ext_vector_type(4)));
+typedef uint32_t quad_bits __attribute__((ext_vector_type(4)));
 #define RGX_SUM_SLOT_WORDS_HALF (2048 + 2 * 24 * 64 + 2 * 64)
 #ifndef RGX_SUM_SLOT_BATCH
 #define RGX_SUM_SLOT_BATCH 2       // slots a tile takes from the pool at a time (the last batch's unused ones stay empty)
@@ -1550,9 +1575,17 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
         asm volatile("" :: "v"(bits)); // the first words have arrived: their wait belongs to the set-up, not to the first trip
 #endif
         RGX_SEC(cn, RGX_SEC_PRETRIP);
-        for (;;) {
+        // A trip's chain -- position in the list, slot, Gaussian, its record in memory -- is walked one trip ahead: the record's
+        // words arrive while the trip before goes through its samples.
+        struct Ahead {
+            bool live, hit;
+            int slot;
+            int32_t pid;
+            float4 pos4, inv4, rgba4;
+        };
+        auto ahead = [&]() {
             // (all lanes of a group hold the same bits and the same w: the DPP moves below run with the whole group active)
-            while (__any(bits == 0u && w + 1 < nwr)) {
+            while (nw > 1 && __any(bits == 0u && w + 1 < nwr)) {
                 const bool next = bits == 0u && w + 1 < nwr;
                 const uint32_t m = next ? lane_word(w + 1) : 0u;
                 const uint32_t o = group_or(m);
@@ -1562,17 +1595,24 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
                     bits = o;
                 }
             }
-            const bool live = bits != 0u;
-            if (!__any(live)) break;
-            int pos = 0;
-            if (live) {
-                pos = __builtin_ctz(bits);
-                bits &= bits - 1u;
-            }
-            const bool hit = live && ((mword >> pos) & 1u);
-            const int slot = live ? min((int)slots[min(w * 32 + pos, RGX_CCAP - 1)], RGX_CCAP - 1) : 0;
-            const int32_t pid = (int32_t)(RL.pid[slot] & ~RGX_SLOT_TOUCHED);
-            body(Entry<false>{(const float4 *)(RL.frame + slot), P.prims + pid, pid, slot}, hit, live, HalfRows{});
+            Ahead a;
+            a.live = bits != 0u;
+            const int pos = __builtin_ctz(bits | 0x80000000u);
+            bits &= bits - 1u;
+            a.hit = a.live && ((mword >> pos) & 1u);
+            a.slot = min((int)slots[min(w * 32 + pos, RGX_CCAP - 1)], RGX_CCAP - 1);
+            a.pid = (int32_t)(RL.pid[a.slot] & ~RGX_SLOT_TOUCHED);
+            const Prim *prim = P.prims + (uint32_t)a.pid;
+            a.pos4 = prim->pos4;
+            a.inv4 = prim->inv_inter4;
+            a.rgba4 = prim->rgba4;
+            return a;
+        };
+        Ahead next = ahead();
+        while (__any(next.live)) {
+            const Ahead a = next;
+            next = ahead();
+            body(EntryAhead{(const float4 *)(RL.frame + a.slot), P.prims + (uint32_t)a.pid, a.pid, a.slot, a.pos4, a.inv4, a.rgba4}, a.hit, a.live, HalfRows{});
         }
     }
     return 8 + q0 + q1 + q2 + q3 + nw * 72;
@@ -1947,25 +1987,24 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                 if constexpr (RECORD) {
                     if (rec.slot >= 0) {
                         float *slot = (float *)(P.sum_pool + (int64_t)rec.slot * (P.sum_slot_words / 4));
-                        float *dens = slot + first_sample * 64 + threadIdx.x;
-                        if constexpr (!HALF) {
-                            float *col = slot + RGX_BUFFER_SIZE * 64 + (first_sample * 64 + threadIdx.x) * 3;
+                        // written once, read once by the backward: keep them out of the caches' way
+                        const auto desc = __builtin_amdgcn_make_buffer_rsrc(slot, 0, P.sum_slot_words * 4, 0x00020000);
+                        auto keep = [&](const float (&v)[RGX_CHUNK_SIZE], int component) {
 #pragma unroll
-                            for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
-                                // written once, read once by the backward: keep them out of the caches' way
-                                __builtin_nontemporal_store(sg[i], dens + i * 64);
-                                __builtin_nontemporal_store(cr[i], col + i * 192);
-                                __builtin_nontemporal_store(cg[i], col + i * 192 + 1);
-                                __builtin_nontemporal_store(cb[i], col + i * 192 + 2);
-                            }
+                            for (int i = 0; i < RGX_CHUNK_SIZE; i += 4)
+                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(quad_bits, (quad){v[i], v[i + 1], v[i + 2], v[i + 3]}), desc, threadIdx.x * 16,
+                                                                       (component * RGX_BUFFER_SIZE + first_sample + i) * 256, 2);
+                        };
+                        keep(sg, 0);
+                        if constexpr (!HALF) {
+                            keep(cr, 1);
+                            keep(cg, 2);
+                            keep(cb, 3);
                         } else {
                             const int chunk = first_sample / RGX_CHUNK_SIZE;
                             float big = 0.f;
 #pragma unroll
-                            for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
-                                __builtin_nontemporal_store(sg[i], dens + i * 64);
-                                big = fmaxf(big, fmaxf(fabsf(cr[i]), fmaxf(fabsf(cg[i]), fabsf(cb[i]))));
-                            }
+                            for (int i = 0; i < RGX_CHUNK_SIZE; ++i) big = fmaxf(big, fmaxf(fabsf(cr[i]), fmaxf(fabsf(cg[i]), fabsf(cb[i]))));
                             // big = f * 2^e with f in [1/2, 1): everything times 2^-e lies in (-1, 1)
                             const int e = big > 0.f ? __builtin_amdgcn_frexp_expf(big) : 0;
                             const float down = __builtin_amdgcn_ldexpf(1.0f, -e);
@@ -2654,23 +2693,16 @@ __global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const Ma
                     if (rec.slot >= 0) {
                         float *slot = (float *)(P.sum_pool + (int64_t)rec.slot * (P.sum_slot_words / 4));
                         const int first = half * RGX_CHUNK_SIZE + 4 * tp.sub, at = tp.wave * 16 + tp.ray;
-                        float *dens = slot + first * 64 + at;
+                        quad *q = (quad *)slot + first / 4 * 64 + at;
+                        __builtin_nontemporal_store((quad){d4[0], d4[1], d4[2], d4[3]}, q);
                         if constexpr (!HALF) {
-                            float *col = slot + RGX_BUFFER_SIZE * 64 + (first * 64 + at) * 3;
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                __builtin_nontemporal_store(d4[i], dens + i * 64);
-                                __builtin_nontemporal_store(r4[i], col + i * 192);
-                                __builtin_nontemporal_store(g4[i], col + i * 192 + 1);
-                                __builtin_nontemporal_store(b4[i], col + i * 192 + 2);
-                            }
+                            __builtin_nontemporal_store((quad){r4[0], r4[1], r4[2], r4[3]}, q + RGX_BUFFER_SIZE / 4 * 64);
+                            __builtin_nontemporal_store((quad){g4[0], g4[1], g4[2], g4[3]}, q + 2 * (RGX_BUFFER_SIZE / 4 * 64));
+                            __builtin_nontemporal_store((quad){b4[0], b4[1], b4[2], b4[3]}, q + 3 * (RGX_BUFFER_SIZE / 4 * 64));
                         } else {
                             float big = 0.f;
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                __builtin_nontemporal_store(d4[i], dens + i * 64);
-                                big = fmaxf(big, fmaxf(fabsf(r4[i]), fmaxf(fabsf(g4[i]), fabsf(b4[i]))));
-                            }
+                            for (int i = 0; i < 4; ++i) big = fmaxf(big, fmaxf(fabsf(r4[i]), fmaxf(fabsf(g4[i]), fabsf(b4[i]))));
                             float v[4];
                             copies(big, v);
                             big = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
@@ -3043,15 +3075,35 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             // (1') the same from the forward's sample sums: PA = sum rho w, PB = g . sum rgb rho w
             auto load_sums = [&](const float4 *slot) {
                 RGX_SEC(cn, RGX_SEC_WALK);
-                const float *dens = (const float *)slot + lane;
+                // Through a buffer descriptor: one register of address for all of them.  Six of the eight groups of four samples' colours are
+                // in flight with the densities; with all of them the kernel has no register left, and the compiler makes
+                // them wait for each other.
+                constexpr int QUADS = RGX_BUFFER_SIZE / 4;
+                const auto desc = __builtin_amdgcn_make_buffer_rsrc((void *)slot, 0, P.sum_slot_words * 4, 0x00020000);
+                auto load = [&](int i) { return __builtin_bit_cast(quad, __builtin_amdgcn_raw_buffer_load_b128(desc, lane * 16, i * 1024, 2)); };
 #pragma unroll
-                for (int i = 0; i < RGX_BUFFER_SIZE; ++i) PA[i] = __builtin_nontemporal_load(dens + i * 64);
+                for (int i = 0; i < QUADS; ++i) {
+                    const quad d = load(i);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) PA[4 * i + k] = d[k];
+                }
                 if constexpr (!HALF) {
-                    const float *col = (const float *)slot + RGX_BUFFER_SIZE * 64 + lane * 3;
+                    quad r[QUADS], gr[QUADS], b[QUADS];
+                    auto ask = [&](int i) {
+                        r[i] = load(QUADS + i);
+                        gr[i] = load(2 * QUADS + i);
+                        b[i] = load(3 * QUADS + i);
+                        __builtin_amdgcn_sched_barrier(0);
+                    };
 #pragma unroll
-                    for (int i = 0; i < RGX_BUFFER_SIZE; ++i)
-                        PB[i] = fmaf(g.x, __builtin_nontemporal_load(col + i * 192),
-                                     fmaf(g.y, __builtin_nontemporal_load(col + i * 192 + 1), g.z * __builtin_nontemporal_load(col + i * 192 + 2)));
+                    for (int i = 0; i < 6; ++i) ask(i);
+#pragma unroll
+                    for (int i = 0; i < QUADS; ++i) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) PB[4 * i + k] = fmaf(g.x, r[i][k], fmaf(g.y, gr[i][k], g.z * b[i][k]));
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (i + 6 < QUADS) ask(i + 6);
+                    }
                 } else {
 #pragma unroll
                     for (int chunk = 0; chunk < 2; ++chunk) {
@@ -3109,8 +3161,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 for (int c = 0; c < RGX_NSUM; ++c) out[c] = 0.f;
                 const int32_t pid = e.pid;
                 if (hit) {
-                    const Prim *pr = e.prim;
-                    const float4 col = pr->rgba4, e5 = pr->pos4;
+                    const float4 col = e.colour(), e5 = e.position();
                     f3 U, V, W, inv;
                     float k;
                     e.frame(U, V, W, inv, k);
