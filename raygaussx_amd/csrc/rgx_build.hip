@@ -147,15 +147,19 @@ __device__ __forceinline__ uint64_t expand21(uint64_t x)
     return x;
 }
 
-// 21 bits per axis of the box centre, relative to the scene bbox
-__global__ __launch_bounds__(256) void k_morton63(const float *__restrict__ boxes, int64_t n, const WsHeader *hdr,
+// 21 bits per axis of the box centre, relative to the scene bbox (whose final form the first thread leaves in the header)
+__global__ __launch_bounds__(256) void k_morton63(const float *__restrict__ boxes, int64_t n, WsHeader *hdr,
                                                   uint64_t *__restrict__ keys, uint32_t *__restrict__ vals)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     uint64_t q[3];
     for (int a = 0; a < 3; ++a) {
-        const float lo = hdr->bb_min[a], ext = hdr->bb_max[a] - lo;
+        const float lo = dec_f(hdr->bb_min_enc[a]), hi = dec_f(hdr->bb_max_enc[a]), ext = hi - lo;
+        if (i == 0) {
+            hdr->bb_min[a] = lo;
+            hdr->bb_max[a] = hi;
+        }
         const float c = 0.5f * boxes[6 * i + a] + 0.5f * boxes[6 * i + 3 + a];
         float u = ext > 0.f ? (c - lo) / ext : 0.f;
         u = fminf(fmaxf(u, 0.f), 1.f);
@@ -311,9 +315,112 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restri
     }
 }
 
+// A sort of few keys: all passes in one workgroup, the keys in registers and their new order in LDS.  What the passes
+// above take for them is the latency of their launches, 24 for 64-bit keys (building the tree over 4 096 boxes
+// 181 us, with this 98; over 8 192 185 and 125; with a bitonic network, which moves every key through LDS 78 and 91 times
+// instead of 8, 117 and 177).  Each wavefront has a run
+// of the keys, and ranks 64 at a time as k_rs_scatter does.  The limit is what fits LDS (12 bytes a key, and 16 KB of counters).
+#define RGX_SORT_SMALL 8192
+template <typename K>
+__global__ __launch_bounds__(1024) void k_sort_small(K *__restrict__ keys, uint32_t *__restrict__ vals, int n, int bits)
+{
+    constexpr int WAVES = 16, ITEMS = RGX_SORT_SMALL / 1024;
+    __shared__ K lkey[RGX_SORT_SMALL];
+    __shared__ uint32_t lval[RGX_SORT_SMALL];
+    __shared__ uint32_t cnt[WAVES][256];
+    __shared__ uint32_t wave_total[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rounds = (n + 1023) / 1024, base = wave * rounds * 64; // wave w has the keys [base, base + 64 rounds)
+    K key[ITEMS];
+    uint32_t val[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int i = base + r * 64 + lane;
+        const bool valid = r < rounds && i < n;
+        key[r] = valid ? keys[i] : (K)0;
+        val[r] = valid ? vals[i] : 0u;
+    }
+    for (int shift = 0; shift < bits; shift += 8) {
+        for (int d = lane; d < 256; d += 64) cnt[wave][d] = 0;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r)
+            if (r < rounds && base + r * 64 + lane < n) atomicAdd(&cnt[wave][(uint32_t)(key[r] >> shift) & 255u], 1u);
+        __syncthreads();
+        // where each (digit, wave) run starts: digits before waves
+        uint32_t total = 0, upto = 0;
+        if (threadIdx.x < 256) {
+            for (int w = 0; w < WAVES; ++w) total += cnt[w][threadIdx.x];
+            upto = total;
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t t = __shfl_up(upto, o);
+                if (lane >= o) upto += t;
+            }
+            if (lane == 63) wave_total[wave] = upto;
+        }
+        __syncthreads();
+        if (threadIdx.x < 256) {
+            uint32_t at = upto - total;
+            for (int w = 0; w < wave; ++w) at += wave_total[w];
+            for (int w = 0; w < WAVES; ++w) {
+                const uint32_t c = cnt[w][threadIdx.x];
+                cnt[w][threadIdx.x] = at;
+                at += c;
+            }
+        }
+        __syncthreads();
+        volatile uint32_t *cur = cnt[wave];
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            if (r >= rounds) break;
+            const bool valid = base + r * 64 + lane < n;
+            const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+            uint64_t same = __ballot(valid);
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t bal = __ballot(bit);
+                same &= bit ? bal : ~bal;
+            }
+            const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
+            if (valid) {
+                const uint32_t at = cur[d] + rank;
+                lkey[at] = key[r];
+                lval[at] = val[r];
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (valid && rank == 0) cur[d] += __popcll(same);
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const int i = base + r * 64 + lane;
+            if (r < rounds && i < n) {
+                key[r] = lkey[i];
+                val[r] = lval[i];
+            }
+        }
+        // (the next pass writes lkey and lval after two more barriers)
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int i = base + r * 64 + lane;
+        if (r < rounds && i < n) {
+            keys[i] = key[r];
+            vals[i] = val[r];
+        }
+    }
+}
+
+// Sorts (k0, v0) by key, stable, with (k1, v1) as the second buffers.
 template <typename K>
 static int radix_sort(K *k0, uint32_t *v0, K *k1, uint32_t *v1, int64_t n, int bits, uint32_t *hist, hipStream_t s)
 {
+    if (n <= RGX_SORT_SMALL) {
+        hipLaunchKernelGGL(k_sort_small<K>, dim3(1), dim3(1024), 0, s, k0, v0, (int)n, bits);
+        RGX_LAUNCH_CHECK();
+        return 0;
+    }
     const int nblocks = (int)((n + RGX_RS_TILE - 1) / RGX_RS_TILE);
     K *ki = k0, *ko = k1;
     uint32_t *vi = v0, *vo = v1;
@@ -503,10 +610,11 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
 }
 
 __global__ __launch_bounds__(256) void k_skip_links(int64_t n, Node *__restrict__ nodes, const int32_t *__restrict__ parent,
-                                                    const int32_t *__restrict__ right, const int32_t *gate = nullptr)
+                                                    const int32_t *__restrict__ right, WsHeader *h, const int32_t *gate = nullptr)
 {
     const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= 2 * n - 1 || gate_closed(gate)) return;
+    if (id == 0) h->built = 1; // (the last kernel of a build)
     int32_t cur = (int32_t)id, skip = -1;
     for (;;) {
         const int32_t p = parent[cur];
@@ -517,7 +625,7 @@ __global__ __launch_bounds__(256) void k_skip_links(int64_t n, Node *__restrict_
     nodes[id].skip = skip;
 }
 
-__global__ void k_mark_built(WsHeader *h, const int32_t *gate = nullptr)
+__global__ void k_mark_built(WsHeader *h, const int32_t *gate = nullptr) // of an empty scene
 {
     if (!gate_closed(gate)) h->built = 1;
 }
@@ -617,7 +725,6 @@ static int build_impl(const float *pos, const float *scale, const float *quat, c
         else
             hipLaunchKernelGGL(k_aabb, grid_reduce(n, 256), dim3(256), 0, s, pos, scale, quat, dens, n, sigma_threshold, boxes,
                                hdr->bb_min_enc, hdr->bb_max_enc);
-        hipLaunchKernelGGL(k_finish_bbox, dim3(1), dim3(64), 0, s, hdr, (float *)nullptr, (float *)nullptr);
         hipLaunchKernelGGL(k_morton63, grid_for(n, 256), dim3(256), 0, s, boxes, n, hdr, k0, v0);
         RGX_LAUNCH_CHECK();
         const int r = radix_sort<uint64_t>(k0, v0, k1, v1, n, 64, hist, s);
@@ -629,9 +736,10 @@ static int build_impl(const float *pos, const float *scale, const float *quat, c
             hipLaunchKernelGGL(k_karras, grid_for(n - 1, 256), dim3(256), 0, s, k0, n, nodes, parent, right, other_end);
             hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, flags);
         }
-        hipLaunchKernelGGL(k_skip_links, grid_for(2 * n - 1, 256), dim3(256), 0, s, n, nodes, parent, right);
+        hipLaunchKernelGGL(k_skip_links, grid_for(2 * n - 1, 256), dim3(256), 0, s, n, nodes, parent, right, hdr);
+    } else {
+        hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr);
     }
-    hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr);
     rgx_span_end(span, s);
     RGX_LAUNCH_CHECK();
     return RGX_OK;
@@ -665,9 +773,10 @@ extern "C" int rgx_refit_aabbs(const float *bboxes, int64_t n, void *ws, size_t 
         hipLaunchKernelGGL(k_finish_bbox, dim3(1), dim3(64), 0, s, hdr, (float *)nullptr, (float *)nullptr, gate);
         hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, order, n, nodes, parent, flags, (uint32_t *)(w + L.vals1), gate);
         if (n > 1) hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, flags, gate);
-        hipLaunchKernelGGL(k_skip_links, grid_for(2 * n - 1, 256), dim3(256), 0, s, n, nodes, parent, right, gate);
+        hipLaunchKernelGGL(k_skip_links, grid_for(2 * n - 1, 256), dim3(256), 0, s, n, nodes, parent, right, hdr, gate);
+    } else {
+        hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr, gate);
     }
-    hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr, gate);
     rgx_span_end(span, s);
     RGX_LAUNCH_CHECK();
     return RGX_OK;

@@ -3372,10 +3372,25 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
 // tiles.  One workgroup per XCD list: counting sort over 1024 size classes (order within a class
 // does not matter); tiles outside the image and tiles without a usable record go last.
 #define RGX_ORDER_BINS 1024
+// the sum of the values of the threads before this one; s_wave: a word per wavefront
+__device__ __forceinline__ uint32_t block_sum_before(uint32_t v, uint32_t *s_wave)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t upto = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(upto, o);
+        if (lane >= o) upto += t;
+    }
+    if (lane == 63) s_wave[wave] = upto;
+    __syncthreads();
+    uint32_t before = upto - v;
+    for (int w = 0; w < wave; ++w) before += s_wave[w];
+    return before;
+}
 __global__ __launch_bounds__(256) void k_tile_order(const MarchParams P)
 {
     __shared__ uint32_t s_bin[RGX_ORDER_BINS];
-    __shared__ uint32_t s_part[256];
+    __shared__ uint32_t s_part[4];
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int per_block = g.bw * g.bh, cnt = g.per_xcd * per_block, xcd = blockIdx.x;
     auto size_class = [&](int j) -> uint32_t {
@@ -3392,21 +3407,10 @@ __global__ __launch_bounds__(256) void k_tile_order(const MarchParams P)
     __syncthreads();
     for (int j = threadIdx.x; j < cnt; j += 256) atomicAdd(&s_bin[size_class(j)], 1u);
     __syncthreads();
-    // first position of each class, classes in descending order: thread t owns classes 4t .. 4t+3
-    const int c0 = 4 * threadIdx.x;
+    // first position of each class, classes in descending order: thread t owns four
+    const int c0 = RGX_ORDER_BINS - 4 - 4 * threadIdx.x;
     const uint32_t n0 = s_bin[c0], n1 = s_bin[c0 + 1], n2 = s_bin[c0 + 2], n3 = s_bin[c0 + 3];
-    s_part[threadIdx.x] = n0 + n1 + n2 + n3;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0; // tiles in heavier classes
-        for (int t = 255; t >= 0; --t) {
-            const uint32_t c = s_part[t];
-            s_part[t] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    const uint32_t base = s_part[threadIdx.x];
+    const uint32_t base = block_sum_before(n0 + n1 + n2 + n3, s_part); // tiles in heavier classes
     s_bin[c0 + 3] = base;
     s_bin[c0 + 2] = base + n3;
     s_bin[c0 + 1] = base + n3 + n2;
@@ -3472,7 +3476,7 @@ __global__ __launch_bounds__(256) void k_block_cost(const MarchParams P, uint32_
 
 __global__ __launch_bounds__(1024) void k_block_order(const MarchParams P, const uint32_t *__restrict__ cost, uint32_t *__restrict__ order)
 {
-    __shared__ uint32_t s_bin[RGX_ORDER_BINS];
+    __shared__ uint32_t s_bin[RGX_ORDER_BINS], s_wave[16];
     __shared__ uint32_t s_max;
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh), slots = 8 * g.per_xcd;
@@ -3482,19 +3486,17 @@ __global__ __launch_bounds__(1024) void k_block_order(const MarchParams P, const
     __syncthreads();
     uint32_t mx = 0;
     for (int b = threadIdx.x; b < nb; b += blockDim.x) mx = max(mx, cost[b]);
-    atomicMax(&s_max, mx);
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(&s_max, mx);
     __syncthreads();
     const uint64_t top = s_max;
     auto bin = [&](int b) { return (uint32_t)(RGX_ORDER_BINS - 1) - (uint32_t)((uint64_t)cost[b] * (RGX_ORDER_BINS - 1) / top); }; // heaviest first
     for (int b = threadIdx.x; b < nb; b += blockDim.x) atomicAdd(&s_bin[bin(b)], 1u);
     __syncthreads();
-    if (threadIdx.x == 0) { // exclusive scan of 1024 bins: a few microseconds, once per launch
-        uint32_t run = 0;
-        for (int i = 0; i < RGX_ORDER_BINS; ++i) {
-            const uint32_t c = s_bin[i];
-            s_bin[i] = run;
-            run += c;
-        }
+    {
+        static_assert(RGX_ORDER_BINS == 1024, "a bin per thread");
+        const uint32_t before = block_sum_before(s_bin[threadIdx.x], s_wave);
+        s_bin[threadIdx.x] = before;
     }
     __syncthreads();
     for (int b = threadIdx.x; b < nb; b += blockDim.x) {

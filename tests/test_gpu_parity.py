@@ -571,6 +571,40 @@ def test_morton_order_bit_exact(gx, orc):
         np.testing.assert_array_equal(order.cpu().numpy(), orc.morton_order(pos))
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 1023, 1025, 4096, 8191, 8192, 8193])
+def test_orders_of_few_keys(gx, orc, n):
+    """Both sorts on either side of the sizes at which one workgroup sorts, with keys that tie: the points' order against the
+    oracle's, the tree's against the codes recomputed from the boxes and scene box it left in its workspace."""
+    import ctypes as C
+    from raygaussx_amd import _lib
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.reordering import morton_order
+    rng = np.random.default_rng(n)
+    pos = rng.normal(size=(n, 3)).astype(np.float32)
+    pos[n // 2:] = pos[:n - n // 2]
+    _step(f"orders of {n} keys")
+    np.testing.assert_array_equal(morton_order(torch.from_numpy(pos).to(gx.DEV)).cpu().numpy(), orc.morton_order(pos))
+    scale, quat = np.full((n, 3), 0.01, np.float32), np.tile(np.float32([1, 0, 0, 0]), (n, 1))
+    dens = np.ones(n, np.float32)
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*(torch.from_numpy(a).to(gx.DEV) for a in (pos, scale, quat, dens)))
+    lay = (C.c_size_t * 6)()
+    _lib.check(_lib.lib().rgx_build_layout(C.c_int64(n), lay))
+    torch.cuda.synchronize()
+    view = lambda k, nbytes, t: gas.ws[lay[k]:lay[k] + nbytes].view(t).cpu().numpy()
+    boxes, order, header = view(0, n * 24, torch.float32).reshape(n, 6), view(1, n * 4, torch.int32), view(5, 24, torch.float32)
+    np.testing.assert_array_equal(header[:3], boxes[:, :3].min(0))
+    np.testing.assert_array_equal(header[3:], boxes[:, 3:].max(0))
+    ext = header[3:] - header[:3]
+    centre = np.float32(0.5) * boxes[:, :3] + np.float32(0.5) * boxes[:, 3:]
+    u = np.clip((centre - header[:3]) / np.where(ext > 0, ext, 1), 0, 1).astype(np.float32) * np.float32(2 ** 21)
+    q = np.minimum(u.astype(np.int64), 2 ** 21 - 1)
+    code = np.zeros(n, np.int64)
+    for b in range(21):
+        for a in range(3):
+            code |= ((q[:, a] >> b) & 1) << (3 * b + 2 - a)
+    np.testing.assert_array_equal(order, np.argsort(code, kind="stable"))
+
+
 def test_reorder_tensors_is_the_per_tensor_gather(gx):
     """PointCloud.reorder_zordercurve's gathers (classes/point_cloud.py:1031-1044) in one launch:
     every tensor equals numpy's `t[index]`, for the parameter shapes of a point cloud with Adam
