@@ -3006,6 +3006,32 @@ __device__ __forceinline__ void group_sums_split(const float (&out)[RGX_NSUM], f
     }
 }
 
+// Adds the groups' sums to those of their slots in LDS, every lane one or two of its group's.  An atomic float add takes the LDS
+// unit, which all of a CU's wavefronts share, some four clocks a lane; so where a row's two groups are at one slot, as
+// often in dense scenes, the first adds for both (3 M Gaussians 1237x822: 8.4 -> 8.1 ms, 1 M 800x800: 5.03 -> 4.94).
+// The same between rows costs as much as it saves, and plain reads and writes, with the groups at one slot taking
+// turns, wait too long (12.3 -> 12.8 and 5.7 -> 6.3 ms when measured).
+// r: as group_sums_split leaves it; todo: the lane's group has something to add.  Returns whether the lane's group added.
+__device__ __forceinline__ bool add_group_sums(float *acc, const float (&r)[7], int slot, bool todo)
+{
+    const int lane = threadIdx.x, q = lane & 3;
+    const bool upper = lane & 4, two = q < (upper ? 2 : 3); // lane q of a quad: its components q and q + 4
+    const float r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3], r4 = r[4], r5 = r[5], r6 = r[6];
+    float v0 = q == 0 ? r0 : q == 1 ? r1 : q == 2 ? r2 : r3, v1 = q == 0 ? r4 : q == 1 ? r5 : r6;
+    const int key = todo ? slot : -1 - lane;
+    const bool both = key == __builtin_amdgcn_update_dpp(0, key, 0x128, 0xf, 0xf, true); // row_ror:8
+    const float other0 = row_take<0x128>(v0), other1 = row_take<0x128>(v1);
+    v0 = both ? v0 + other0 : v0;
+    v1 = both ? v1 + other1 : v1;
+    todo = todo && !(both && (lane & 8));
+    if (todo) {
+        float *dst = acc + ((upper ? 7 : 0) + q) * RGX_CCAP + slot;
+        unsafeAtomicAdd(dst, v0);
+        if (two) unsafeAtomicAdd(dst + 4 * RGX_CCAP, v1);
+    }
+    return todo;
+}
+
 // ---------------------------------------------------------------------------
 // Backward: __raygen__rg of cuda_train/backward/gaussians_aabb.cu:209-497.
 //
@@ -3024,7 +3050,7 @@ __device__ __forceinline__ void group_sums_split(const float (&out)[RGX_NSUM], f
 // nineteen running sums; the `power < k^2` mask follows the forward's 32-step recurrence, i.e. it
 // is the mask the forward blended with.  Per Gaussian the moments turn into 13 sums in its whitened
 // frame (RGX_NSUM); those are summed over the rays of a group of lanes (a row of 16 in the walk by rows, half a
-// row in a replay) with DPP adds and carried on by one lane per group (two in a replay: group_sums_split); the
+// row in a replay) with DPP adds and carried on by one lane per group (all eight in a replay: add_group_sums); the
 // change of variables to the 14 gradient words comes after all sums.
 template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false>
 __device__ __forceinline__ void march_bwd(const MarchParams &P)
@@ -3250,23 +3276,15 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 // summed over the group's rays; one lane per group carries the sums on
                 const uint64_t bal = __ballot(hit);
                 if constexpr (REPLAY && GROUP == 8) {
-                    // the group's sums end up in two of its lanes, seven components in the first, six in the fifth
                     float r[7];
                     group_sums_split(out, r);
-                    const int first = lane & ~7;
-                    if ((lane & 3) == 0 && live && ((bal >> first) & 0xffull)) {
-                        const bool upper = lane & 4;
-                        if (!upper) {
-                            if constexpr (STATS) {
-                                if (!(atomicOr(&s_pid[e.slot], RGX_SLOT_TOUCHED) & RGX_SLOT_TOUCHED)) cn.grad_atomics += 14;
-                            } else {
-                                atomicOr(&s_pid[e.slot], RGX_SLOT_TOUCHED);
-                            }
+                    const bool adds = add_group_sums(s_acc, r, e.slot, live && ((bal >> (lane & ~7)) & 0xffull));
+                    if (adds) {
+                        if constexpr (STATS) {
+                            if ((lane & 7) == 0 && !(atomicOr(&s_pid[e.slot], RGX_SLOT_TOUCHED) & RGX_SLOT_TOUCHED)) cn.grad_atomics += 14;
+                        } else {
+                            s_pid[e.slot] = (uint32_t)e.pid | RGX_SLOT_TOUCHED;
                         }
-                        float *dst = &s_acc[(upper ? 7 * RGX_CCAP : 0) + e.slot];
-#pragma unroll
-                        for (int c = 0; c < 6; ++c) unsafeAtomicAdd(dst + c * RGX_CCAP, r[c]);
-                        if (!upper) unsafeAtomicAdd(dst + 6 * RGX_CCAP, r[6]);
                     }
                     RGX_SEC(cn, RGX_SEC_SHADE);
                     return;
