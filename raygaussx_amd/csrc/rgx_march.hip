@@ -1999,13 +1999,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                 }
             };
             auto blend = [&](bool second_chunk) { // gaussians_aabb.cu:195-201
-                float t_sample = R.tbuffer + 0.5f * dt; // the viewer's running sample position (cuda_gui/gaussians_aabb.cu:189)
-                if constexpr (VIEWER) {
-                    if (second_chunk) {
-#pragma unroll
-                        for (int i = 0; i < RGX_CHUNK_SIZE; ++i) t_sample += dt; // as the first chunk left it
-                    }
-                }
+                const float first_sample = second_chunk ? 16.5f : 0.5f; // (viewer: cuda_gui/gaussians_aabb.cu:189)
 #pragma unroll
                 for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
                     const float x = sg[i] * dt;
@@ -2016,8 +2010,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                     Cg = fmaf(ts, cg[i], Cg);
                     Cb = fmaf(ts, cb[i], Cb);
                     if constexpr (VIEWER) {
-                        depth += R.T * (1.0f - w) * t_sample;
-                        t_sample += dt;
+                        depth += R.T * (1.0f - w) * fmaf(dt, first_sample + (float)i, R.tbuffer);
                     }
                     R.T *= w;
                 }
