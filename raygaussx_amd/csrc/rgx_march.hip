@@ -350,11 +350,29 @@ __device__ __forceinline__ bool frustum_misses(const Frustum &F, float4 a, float
 // (S^-1 R^T (eye - centre) and its squared norm - 1), and the distance shell [dmin, dmax]
 // from the eye that bounds the ellipsoid.  The values are produced by the same operations,
 // in the same order, as in line_roots(), so using them changes no rounding.
-//   float4 0: U.xyz, dmin     1: V.xyz, dmax     2: W.xyz, k      3: inv_inter.xyz, c
-//          4: Oe.xyz, sorted index
+//   U.xyz V.xyz W.xyz inv_inter.xyz | Oe.xyz, sorted index | dmin, dmax, k, c
+// in this order without gaps: the filter reads the first sixteen words, as four LDS reads and without holes in the
+// registers they land in (three words of a quadruple take four).
 // (80 bytes, sized so that 12 wavefronts' tables fit one CU's LDS; what only the shading of an
 // actual hit needs -- eye - centre and the colour -- is read from the primitive record.)
 #define RGX_TAB 20
+enum { RGX_TAB_PID = 15, RGX_TAB_DMIN = 16, RGX_TAB_DMAX = 17, RGX_TAB_K = 18, RGX_TAB_C = 19 };
+__device__ __forceinline__ void table_store(float4 *e, f3 U, f3 V, f3 W, f3 inv, f3 Oe, int32_t pid, float dmin, float dmax, float k, float c)
+{
+    e[0] = make_float4(U.x, U.y, U.z, V.x);
+    e[1] = make_float4(V.y, V.z, W.x, W.y);
+    e[2] = make_float4(W.z, inv.x, inv.y, inv.z);
+    e[3] = make_float4(Oe.x, Oe.y, Oe.z, __int_as_float(pid));
+    e[4] = make_float4(dmin, dmax, k, c);
+}
+__device__ __forceinline__ void table_frame(const float4 *e, f3 &U, f3 &V, f3 &W, f3 &inv)
+{
+    const float4 a = e[0], b = e[1], c = e[2];
+    U = mk3(a.x, a.y, a.z);
+    V = mk3(a.w, b.x, b.y);
+    W = mk3(b.z, b.w, c.x);
+    inv = mk3(c.y, c.z, c.w);
+}
 
 // Cooperative sweep of the BVH: the node stack is shared by the wave, every step pops up to
 // 64 nodes (one per lane) and tests their boxes against the frustum.  Internal nodes that pass
@@ -566,12 +584,7 @@ __device__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int3
         const f3 Oe = apply_sinv_rt(mk3(p.pos4.x, p.pos4.y, p.pos4.z), U, V, W, inv);
         const float c = fmaf(Oe.x, Oe.x, fmaf(Oe.y, Oe.y, fmaf(Oe.z, Oe.z, -1.0f)));
         if (__builtin_amdgcn_inverse_ballot_w64(hits)) {
-            float4 *dst = (float4 *)(s_tab + (C + rank) * RGX_TAB);
-            dst[0] = make_float4(U.x, U.y, U.z, dmin);
-            dst[1] = make_float4(V.x, V.y, V.z, dmax);
-            dst[2] = make_float4(W.x, W.y, W.z, p.inv_inter4.w);
-            dst[3] = make_float4(inv.x, inv.y, inv.z, c);
-            dst[4] = make_float4(Oe.x, Oe.y, Oe.z, __int_as_float(~left));
+            table_store((float4 *)(s_tab + (C + rank) * RGX_TAB), U, V, W, inv, Oe, ~left, dmin, dmax, p.inv_inter4.w, c);
         }
         plain = plain && (hits & ~__ballot(plain_roots(inv, c))) == 0;
         C += __popcll(hits);
@@ -773,12 +786,14 @@ struct TileLds {
 template <bool PLAIN, bool EXIT>
 __device__ __forceinline__ bool lane_roots(const float4 *e, f3 dir, float &r1, float &r2)
 {
-    const float4 e0 = e[0], e1 = e[1], e2 = e[2], e3 = e[3], e4 = e[4];
-    const f3 De = apply_sinv_rt(dir, mk3(e0.x, e0.y, e0.z), mk3(e1.x, e1.y, e1.z), mk3(e2.x, e2.y, e2.z), mk3(e3.x, e3.y, e3.z));
+    f3 U, V, W, inv;
+    table_frame(e, U, V, W, inv);
+    const float4 e4 = e[3];
+    const f3 De = apply_sinv_rt(dir, U, V, W, inv);
     const f3 Oe = mk3(e4.x, e4.y, e4.z);
     const float a = fmaf(De.x, De.x, fmaf(De.y, De.y, De.z * De.z));
     const float b = -fmaf(Oe.x, De.x, fmaf(Oe.y, De.y, Oe.z * De.z));
-    const float c = e3.w;
+    const float c = ((const float *)e)[RGX_TAB_C];
     const float inv_a = PLAIN ? div_rn_plain(1.0f, a) : 1.0f / a;
     const float b_inv_a = b * inv_a;
     const f3 Pc = mk3(fmaf(b_inv_a, De.x, Oe.x), fmaf(b_inv_a, De.y, Oe.y), fmaf(b_inv_a, De.z, Oe.z));
@@ -814,10 +829,8 @@ struct Entry {
     __device__ __forceinline__ void frame(f3 &U, f3 &V, f3 &W, f3 &inv, float &k) const
     {
         if constexpr (FROM_TABLE) {
-            const float4 e0 = tab[0], e1 = tab[1], e2 = tab[2], e3 = tab[3];
-            U = mk3(e0.x, e0.y, e0.z); V = mk3(e1.x, e1.y, e1.z); W = mk3(e2.x, e2.y, e2.z);
-            inv = mk3(e3.x, e3.y, e3.z);
-            k = e2.w;
+            table_frame(tab, U, V, W, inv);
+            k = ((const float *)tab)[RGX_TAB_K];
         } else {
             const float *f = (const float *)tab; // component-major: word c of this slot at f[c * RGX_CCAP]
             U = mk3(f[0], f[RGX_CCAP], f[2 * RGX_CCAP]);
@@ -1005,9 +1018,9 @@ __device__ __forceinline__ void filter_table(const TileLds &L, int C, float t0, 
         bool rel = false;
         float margins = INFINITY;
         if (cl < C) {
-            const float dmin = L.tab[cl * RGX_TAB + 3], dmax = L.tab[cl * RGX_TAB + 7];
+            const float dmin = L.tab[cl * RGX_TAB + RGX_TAB_DMIN], dmax = L.tab[cl * RGX_TAB + RGX_TAB_DMAX];
             rel = dmax >= t0 && dmin <= t1;
-            margins = slow ? INFINITY : filter_margin(L.tab[cl * RGX_TAB + 15]);
+            margins = slow ? INFINITY : filter_margin(L.tab[cl * RGX_TAB + RGX_TAB_C]);
         }
         uint64_t m = __ballot(rel);
         if (lane == 0) cn.cands += (unsigned)__popcll(m);
@@ -1016,8 +1029,10 @@ __device__ __forceinline__ void filter_table(const TileLds &L, int C, float t0, 
             m &= m - 1;
             const float margin = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(margins), i));
             const float4 *e = (const float4 *)((const char *)L.tab + __builtin_amdgcn_readfirstlane(c * (RGX_TAB * 4)));
-            const float4 e0 = e[0], e1 = e[1], e2 = e[2], e3 = e[3], e4 = e[4];
-            const f3 De = apply_sinv_rt(Q.dir, mk3(e0.x, e0.y, e0.z), mk3(e1.x, e1.y, e1.z), mk3(e2.x, e2.y, e2.z), mk3(e3.x, e3.y, e3.z));
+            f3 U, V, W, inv;
+            table_frame(e, U, V, W, inv);
+            const float4 e4 = e[3];
+            const f3 De = apply_sinv_rt(Q.dir, U, V, W, inv);
             const float a = fmaf(De.x, De.x, fmaf(De.y, De.y, De.z * De.z));
             const float b = -fmaf(e4.x, De.x, fmaf(e4.y, De.y, e4.z * De.z));
             const float tc = b * __builtin_amdgcn_rcpf(a);
@@ -1107,7 +1122,7 @@ __device__ __forceinline__ void shade_rows(const MarchParams &P, const TileLds &
         if (__ballot(hit)) {
             const int c = live ? L.list[w * 32 + at] : 0;
             const float4 *tab = (const float4 *)(L.tab + c * RGX_TAB);
-            const int32_t pid = __float_as_int(L.tab[c * RGX_TAB + 19]);
+            const int32_t pid = __float_as_int(L.tab[c * RGX_TAB + RGX_TAB_PID]);
             body(Entry<true>{tab, P.prims + pid, pid, c}, hit, live, Half<0>{});
         }
     }
@@ -1141,7 +1156,7 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
             bits &= bits - 1u;
         }
         const float4 *tab = (const float4 *)(L.tab + c * RGX_TAB);
-        const int32_t pid = __float_as_int(L.tab[c * RGX_TAB + 19]);
+        const int32_t pid = __float_as_int(L.tab[c * RGX_TAB + RGX_TAB_PID]);
         body(Entry<true>{tab, P.prims + pid, pid, c}, has, has, Half<TAG>{});
     }
 }
@@ -1313,7 +1328,7 @@ struct Recorder {
         if (!on() || !fits(4 + ((C + 3) & ~3))) return;
         uint32_t *it = reg + off;
         if (threadIdx.x == 0) it[0] = RGX_REC_WINDOW | (uint32_t)C;
-        for (int i = threadIdx.x; i < C; i += 64) it[4 + i] = __float_as_uint(L.tab[i * RGX_TAB + 19]);
+        for (int i = threadIdx.x; i < C; i += 64) it[4 + i] = __float_as_uint(L.tab[i * RGX_TAB + RGX_TAB_PID]);
         off += 4 + ((C + 3) & ~3);
     }
 
@@ -2212,11 +2227,7 @@ struct LeafEntry {
     bool plain; // passed plain_roots()
     __device__ __forceinline__ void store(float4 *dst, int32_t left) const
     {
-        dst[0] = make_float4(U.x, U.y, U.z, dmin);
-        dst[1] = make_float4(V.x, V.y, V.z, dmax);
-        dst[2] = make_float4(W.x, W.y, W.z, k);
-        dst[3] = make_float4(inv.x, inv.y, inv.z, c);
-        dst[4] = make_float4(Oe.x, Oe.y, Oe.z, __int_as_float(~left));
+        table_store(dst, U, V, W, inv, Oe, ~left, dmin, dmax, k, c);
     }
 };
 __device__ __forceinline__ bool leaf_entry(const MarchParams &P, const Frustum &F, int32_t left, LeafEntry &e)
@@ -2386,7 +2397,7 @@ __device__ __forceinline__ void team_filter(TeamShared<CAP> &T, const TeamPos &t
     for (int h = 0; h < CAP; h += 64) {
         const int c = h + tp.lane;
         bool rel = false;
-        if (c < C) rel = T.tab[c * RGX_TAB + 7] >= t0 && T.tab[c * RGX_TAB + 3] <= t1;
+        if (c < C) rel = T.tab[c * RGX_TAB + RGX_TAB_DMAX] >= t0 && T.tab[c * RGX_TAB + RGX_TAB_DMIN] <= t1;
         const uint64_t b = __ballot(rel);
         if (rel) T.rel[tp.wave][nrel + __popcll(b & ((1ull << tp.lane) - 1ull))] = (uint8_t)c;
         nrel += __popcll(b);
@@ -2489,7 +2500,7 @@ __device__ __forceinline__ void team_shade(const MarchParams &P, TeamShared<CAP>
             bits &= bits - 1u;
         }
         const float4 *tab = (const float4 *)(T.tab + c * RGX_TAB);
-        const int32_t pid = __float_as_int(T.tab[c * RGX_TAB + 19]);
+        const int32_t pid = __float_as_int(T.tab[c * RGX_TAB + RGX_TAB_PID]);
         body(Entry<true>{tab, P.prims + pid, pid, c}, has);
     }
 }
@@ -2502,7 +2513,7 @@ struct TeamRecorder : Recorder {
         if (!on() || !fits(4 + ((C + 3) & ~3))) return;
         uint32_t *it = reg + off;
         if (threadIdx.x == 0) it[0] = RGX_REC_WINDOW | (uint32_t)C;
-        for (int i = threadIdx.x; i < C; i += 256) it[4 + i] = __float_as_uint(T.tab[i * RGX_TAB + 19]);
+        for (int i = threadIdx.x; i < C; i += 256) it[4 + i] = __float_as_uint(T.tab[i * RGX_TAB + RGX_TAB_PID]);
         off += 4 + ((C + 3) & ~3);
     }
     // the blocks' list lengths are in T.msg
