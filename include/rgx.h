@@ -187,8 +187,8 @@ int rgx_march_workspace_bytes(int64_t n, int64_t n_rays, int32_t max_prim_slice,
  * scenes).  Tiles that found the pool empty are replayed from their hit lists alone. */
 int rgx_march_records_bytes(int32_t width, int32_t height, int32_t tile_words, size_t *bytes);
 
-/* Replaces launch_pipeline_forward / launch_pipeline_test (optix_utils.py:222-322,
- * 503-601) and the OptiX programs of cuda_train/forward/gaussians_aabb.cu:
+/* Replaces launch_pipeline_forward (optix_utils.py:222-322) and the OptiX programs of
+ * cuda_train/forward/gaussians_aabb.cu:
  * ray_colors (W*H,3), row-major pixels.  cam, march: host structs.
  * prims: from rgx_pack_prims with the same ws.  records (16-byte aligned, may be NULL):
  * where to write the hit-list record.  stats may be NULL, and should be outside diagnostics:
@@ -196,6 +196,13 @@ int rgx_march_records_bytes(int32_t width, int32_t height, int32_t tile_words, s
 int rgx_march_forward(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims,
                       int64_t n, float *ray_colors, void *march_ws, size_t march_ws_bytes,
                       void *records, size_t records_bytes, RgxStats *stats, void *stream);
+
+/* Replaces launch_pipeline_test (optix_utils.py:503-601): rgx_march_forward without a record, for an image
+ * that no backward follows.  A backward without a record marches the rays once more and has to meet the
+ * forward's samples and hits again; this launch need not be met, so small images may go through a kernel that
+ * adds up a sample's hits, and cuts a list at max_prim_slice, in another order (equally exact). */
+int rgx_march_test(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims,
+                   int64_t n, float *ray_colors, void *march_ws, size_t march_ws_bytes, RgxStats *stats, void *stream);
 
 /* Test hook: rgx_march_forward through the counting kernels, with the counters also kept per ray:
  * ray_counts (W*H, 2) = slabs blended and the sum of their hit-list lengths (the per-ray share of

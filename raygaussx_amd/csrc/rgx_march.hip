@@ -3810,21 +3810,33 @@ static inline dim3 march_grid(const MarchParams &P)
 }
 
 // Up to this many tiles four wavefronts march a tile (k_march_team), beyond it one.  The team's wavefronts repeat the
-// per-iteration work that one wavefront does once for 64 rays, so it loses where the chip is full anyway (10 000 tiles: 1.5
-// to 2.5 times as long); with few tiles the launch is one tile's latency.  Measured, ms without / with the team: 4 k
-// Gaussians in a cube, 256 tiles 1.29 / 0.62, 1 024 tiles 0.88 / 0.52; 100 k in a ball, 256 tiles 7.8 / 2.9, 1 600 tiles
-// 2.4 / 1.2; frames of 60 k heavy-tailed with the adaptive step, 256 tiles 1.43 / 0.74, 625 tiles 1.03 / 0.92, 1 024 tiles
-// 0.94 / 0.98.  Not in training with the adaptive step: the team adds up a sample's hits in another order, the next step's
-// length depends on the last bit of the transmittance, and a sample that so crosses a Gaussian's cut-off moves that
-// Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians): equally exact, but no longer the gradients
-// that larger images and earlier builds give.
+// per-iteration work that one wavefront does once for 64 rays, so it loses where the chip is full anyway; with few tiles
+// the launch is one tile's latency.  Measured, ms of a frame with one wavefront / with four:
+//     tiles                                      256          625          784         1 024        1 600        2 500
+//     fixed step, 4 k Gaussians in a cube    1.04 / 0.55  0.83 / 0.47  0.76 / 0.44  0.71 / 0.43  0.68 / 0.55  0.61 / 0.76
+//     fixed step, 100 k in a ball            4.32 / 2.38  2.54 / 1.58  2.51 / 1.54  2.24 / 1.36  1.68 / 1.20  1.35 / 1.03
+//     adaptive step, 60 k heavy-tailed       1.85 / 1.21  1.14 / 1.02  1.14 / 1.01  1.04 / 1.07  0.97 / 1.58  0.89 / 2.19
+//     adaptive step, 3 M heavy-tailed        9.77 / 4.00  6.73 / 4.53  5.84 / 4.16  5.83 / 4.07  4.57 / 5.59  4.44 / 7.03
+// One line for all launches, below the first loss of any of them (the adaptive frames at 1 024 tiles).  It is not where
+// the fixed step crosses over: that gains up to some 1 600 tiles.
+//
+// Which launches: those whose image is the end of it (rgx_march_test, the viewer), and those that leave a record
+// with the fixed step.  The team adds up a sample's hits in another order, and where max_prim_slice cuts a ray's list it
+// keeps other hits, equally exact both.
+//   No record: the backward searches the tree again, one wavefront per tile, and has to meet the hits and the
+//     transmittance of the forward: that is k_march_fwd then, whatever the step.
+//   A record and the adaptive step: the next step's length depends on the last bit of the transmittance, and a sample that
+//     so crosses a Gaussian's cut-off moves that Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians):
+//     no longer the gradients that larger images give.  k_march_fwd.
+//   A record and the fixed step: what the backward replays is what the team recorded.  (A tile whose region overflowed is
+//     searched again; if max_prim_slice also cut lists in it, they may be cut to other hits there.)
 #ifndef RGX_TEAM_TILES
 #define RGX_TEAM_TILES 768
 #endif
-// half: the record's colour sums are in half precision
-static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, hipStream_t s)
+// half: the record's colour sums are in half precision; image_only: no backward follows this launch
+static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, bool image_only, hipStream_t s)
 {
-    const bool team = P.tiles_x * P.tiles_y <= RGX_TEAM_TILES && !(P.records && P.m.dynamic_sampling);
+    const bool team = P.tiles_x * P.tiles_y <= RGX_TEAM_TILES && (image_only || (P.records && !P.m.dynamic_sampling));
     const dim3 grid = march_grid(P), block(team ? 256 : 64);
 #define RGX_FWD(...)                                                                            \
     do {                                                                                        \
@@ -3849,14 +3861,20 @@ static void launch_forward(const MarchParams &P, bool viewer, bool counting, boo
 
 static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
                                 float *ray_colors, void *march_ws, size_t march_ws_bytes, void *records, size_t records_bytes,
-                                RgxStats *stats, uint32_t *ray_counts, void *stream);
+                                RgxStats *stats, uint32_t *ray_counts, bool image_only, void *stream);
 
 extern "C" int rgx_march_forward(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
                                  float *ray_colors, void *march_ws, size_t march_ws_bytes, void *records, size_t records_bytes,
                                  RgxStats *stats, void *stream)
 {
     return march_forward_launch(ws, cam, march, prims, n, ray_colors, march_ws, march_ws_bytes, records, records_bytes, stats,
-                                nullptr, stream);
+                                nullptr, false, stream);
+}
+
+extern "C" int rgx_march_test(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
+                              float *ray_colors, void *march_ws, size_t march_ws_bytes, RgxStats *stats, void *stream)
+{
+    return march_forward_launch(ws, cam, march, prims, n, ray_colors, march_ws, march_ws_bytes, nullptr, 0, stats, nullptr, true, stream);
 }
 
 extern "C" int rgx_march_forward_counts(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
@@ -3865,12 +3883,12 @@ extern "C" int rgx_march_forward_counts(const void *ws, const RgxCamera *cam, co
 {
     if (!ray_counts) return RGX_EINVAL;
     return march_forward_launch(ws, cam, march, prims, n, ray_colors, march_ws, march_ws_bytes, records, records_bytes, stats,
-                                ray_counts, stream);
+                                ray_counts, false, stream);
 }
 
 static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
                                 float *ray_colors, void *march_ws, size_t march_ws_bytes, void *records, size_t records_bytes,
-                                RgxStats *stats, uint32_t *ray_counts, void *stream)
+                                RgxStats *stats, uint32_t *ray_counts, bool image_only, void *stream)
 {
     const DeviceScope on_device(ws);
     MarchParams P;
@@ -3886,7 +3904,7 @@ static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxM
     if (P.sum_pool || P.faults) hipLaunchKernelGGL(k_clear2, dim3(1), dim3(64), 0, (hipStream_t)stream, (float4 *)P.sum_next, (float4 *)P.faults);
     order_blocks(P, (hipStream_t)stream);
     const bool half = P.sum_pool && P.m.record_format == 1;
-    launch_forward(P, false, counting, half, (hipStream_t)stream);
+    launch_forward(P, false, counting, half, image_only, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
     RGX_LAUNCH_CHECK();
     return RGX_OK;
@@ -3905,7 +3923,7 @@ extern "C" int rgx_march_viewer(const void *ws, const RgxCamera *cam, const RgxM
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
     if (P.faults) hipLaunchKernelGGL(k_clear2, dim3(1), dim3(64), 0, (hipStream_t)stream, (float4 *)nullptr, (float4 *)P.faults);
     order_blocks(P, (hipStream_t)stream);
-    launch_forward(P, true, stats != nullptr, false, (hipStream_t)stream);
+    launch_forward(P, true, stats != nullptr, false, true, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
     RGX_LAUNCH_CHECK();
     return RGX_OK;

@@ -355,9 +355,10 @@ def record_use(cam, device, n=0, record_format=0):
 
 
 def march_forward(gas, cam, prims, dt_step, dynamic_sampling, max_prim_slice, white_background,
-                  t_eps=TRANSMITTANCE_EPSILON, stats=None, records=None, ray_counts=False, record_format=0):
+                  t_eps=TRANSMITTANCE_EPSILON, stats=None, records=None, ray_counts=False, record_format=0, backward_follows=True):
     """``ray_counts=True`` (test hook): also returns an (n_rays, 2) int32 tensor, per ray the slabs blended and
-    the sum of their hit-list lengths."""
+    the sum of their hit-list lengths.  ``backward_follows=False``: the image is the end of it (``rgx_march_test``;
+    a launch that leaves a record or counts per ray is the same either way)."""
     n, dev = prims.shape[0], prims.device
     n_rays = cam.width * cam.height
     m = L.RgxMarch(dt_step, int(bool(dynamic_sampling)), int(max_prim_slice), int(bool(white_background)), t_eps, int(record_format))
@@ -370,6 +371,10 @@ def march_forward(gas, cam, prims, dt_step, dynamic_sampling, max_prim_slice, wh
                                                  C.c_size_t(0 if records is None else records.numel()), L.ptr(stats),
                                                  L.ptr(counts), L.stream(dev)))
         return ray_colors, counts
+    if records is None and not backward_follows:
+        L.check(L.lib().rgx_march_test(L.ptr(gas.ws), C.byref(cam), C.byref(m), L.ptr(prims), C.c_int64(n), L.ptr(ray_colors),
+                                       L.ptr(ws), C.c_size_t(ws.numel()), L.ptr(stats), L.stream(dev)))
+        return ray_colors
     L.check(L.lib().rgx_march_forward(L.ptr(gas.ws), C.byref(cam), C.byref(m), L.ptr(prims), C.c_int64(n),
                                       L.ptr(ray_colors), L.ptr(ws), C.c_size_t(ws.numel()), L.ptr(records),
                                       C.c_size_t(0 if records is None else records.numel()), L.ptr(stats),
@@ -442,12 +447,13 @@ def launch_pipeline_test(pipeline, sbt, gas, bbox_min, bbox_max, dt_step, dynami
                          color_features, positions, scales, quaternions, max_prim_slice, rnd_sample=0,
                          supersampling=(1, 1), white_background=True, hit_prim_idx=None,
                          t_eps=TRANSMITTANCE_EPSILON, stats=None):
-    """optix_utils.py:503-601: the inference launch; same kernel as the training forward."""
-    return launch_pipeline_forward(pipeline, sbt, gas, bbox_min, bbox_max, dt_step, dynamic_sampling, camera,
-                                   densities, color_features, positions, scales, quaternions, max_prim_slice,
-                                   rnd_sample=rnd_sample, supersampling=supersampling,
-                                   white_background=white_background, hit_prim_idx=hit_prim_idx, t_eps=t_eps,
-                                   stats=stats)
+    """optix_utils.py:503-601: the inference launch, as ``launch_pipeline_forward`` but for an image that no
+    backward follows."""
+    cam = camera_struct(camera, supersampling)
+    prims = pack_prims(gas, cam, L.f32(positions), L.f32(scales), L.f32(quaternions), L.f32(densities),
+                       L.f32(color_features))
+    return march_forward(gas, cam, prims, dt_step, dynamic_sampling, max_prim_slice, white_background, t_eps, stats,
+                         backward_follows=False)
 
 
 def launch_pipeline_backward(pipeline, sbt, gas, bbox_min, bbox_max, dt_step, dynamic_sampling, camera,

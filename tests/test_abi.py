@@ -82,6 +82,7 @@ def test_bad_arguments_are_rejected_before_any_launch():
     march = _lib.RgxMarch(0.0025, 0, 2048, 1, 1e-3)
     assert lib.rgx_march_forward(null, C.byref(cam), C.byref(march), null, C.c_int64(0), null, null, C.c_size_t(0), null,
                                  C.c_size_t(0), null, null) == -1                                           # no tree
+    assert lib.rgx_march_test(null, C.byref(cam), C.byref(march), null, C.c_int64(0), null, null, C.c_size_t(0), null, null) == -1
     with pytest.raises(_lib.RgxError):
         _lib.check(-2)
 

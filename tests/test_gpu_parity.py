@@ -502,6 +502,39 @@ def test_forward_with_one_and_with_four_wavefronts_per_tile(gx, orc, w, h, confi
             _check_grads(gx, out["grads"], og)
 
 
+@pytest.mark.parametrize("dyn,cap,scale", [(True, 4096, 1.0), (True, 4096, 4.0), (False, 4096, 1.0), (False, 8, 4.0)])
+def test_forward_without_a_record_is_the_march_that_its_backward_repeats(gx, dyn, cap, scale):
+    """A backward without a record searches the tree again, with one wavefront per tile: its forward has to add up and
+    to cut off the hits of a ray as that does, whatever the number of tiles.  The same rays as the first rows of an
+    image eight times as high (a power of two: the same directions in every bit), whose 1040 tiles always have one
+    wavefront each, come out the same in every bit.  An image that no backward follows only has to be near."""
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.render_optix import compute_rgb
+    w, h = 100, 80          # (whole tiles downwards: the same rays take part in each)
+    sc = gx.to_dev(scenes.scene_to_numpy(scenes.make_scene(2, n=6000, sh_degree=0, seed=31)))
+    cam = scenes.make_camera(2, 1, width=w, height=h)
+    cs, tall = u_ox.camera_struct(cam), u_ox.camera_struct(cam)
+    tall.height, tall.tan_half_fov_y, tall.principal_y = 8 * h, 8 * cs.tan_half_fov_y, cs.principal_y / 8
+    params = sc["positions"], sc["scales"] * scale, sc["quaternions"], sc["densities"]
+    gas = u_ox.AccelerationStructure(6000, gx.DEV).build_from_gaussians(*params)
+    rgb = compute_rgb(cam.camera_center, sc["positions"], sc["color_features"], None, None, None, 0, 0)
+    prims = u_ox.pack_prims(gas, cs, *params, rgb)
+    _step(f"forward without a record, adaptive {dyn}, cut at {cap}")
+    image = u_ox.march_forward(gas, cs, prims, 0.004, dyn, cap, True)
+    assert torch.equal(image, u_ox.march_forward(gas, tall, prims, 0.004, dyn, cap, True)[:w * h])
+    assert (image - 1.0).abs().max() > 0.1                                    # (not the background)
+    only = u_ox.launch_pipeline_test(None, None, gas, None, None, 0.004, dyn, cam, params[3], rgb, *params[:3], cap)
+    if cap > 8:
+        assert (only - image).abs().max() <= (5e-3 if dyn else 1e-5)          # (adaptive: a ray may be re-phased)
+    # the same through the autograd function: with a backward to come, and without
+    np_scene = {k: v.cpu().numpy() for k, v in sc.items()}
+    np_scene["scales"] = np_scene["scales"] * np.float32(scale)
+    cfg = dict(dt_step=0.004, dynamic_sampling=dyn, max_prim_slice=cap)
+    out = gx.gpu_render(np_scene, cam, cfg, want_grad=np.ones((w * h, 3), np.float32), stats=False, record_hits=False)
+    assert np.array_equal(out["image"], image.cpu().numpy())
+    assert np.array_equal(gx.gpu_render(np_scene, cam, cfg, stats=False)["image"], only.cpu().numpy())
+
+
 def test_long_hit_lists_spill_and_truncation(gx, orc):
     """Fat Gaussians: slabs with far more than 32 hits (LDS part + spill area), then a tiny
     max_prim_slice to exercise the silent truncation path and its counter."""
