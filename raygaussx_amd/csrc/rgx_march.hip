@@ -904,6 +904,14 @@ __device__ __forceinline__ float filter_margin(float c)
 
 // Adds a hit's samples to the half's sums: those within the cut-off, by the execution mask (a comparison that writes it
 // and a scalar move that restores it cost less than a comparison, two wait states and a select).
+// What the compiler cannot see inside the assembly is arranged there:
+//   a sum is written before the last inputs are read: early-clobber ("+&v"), no input shares its register;
+//   gw comes from a transcendental, whose result the next instruction may not read yet: the comparison, which reads
+//     only the power, comes first;
+//   a vector write of the mask needs five instructions before a data-parallel or cross-lane instruction, and one of vcc
+//     four before v_div_fmas or v_readlane take it: the four multiply-adds and the scalar move are those five;
+//   a vector write of a register needs two before a data-parallel or permlane read of it: the scalar move is one, and the
+//     sums are next read after the hit's branch has ended, whose scalar instructions are more than the other.
 __device__ __forceinline__ void accumulate_samples(HitSetup hs, float4 col, float (&sg)[RGX_CHUNK_SIZE], float (&cr)[RGX_CHUNK_SIZE],
                                                    float (&cg)[RGX_CHUNK_SIZE], float (&cb)[RGX_CHUNK_SIZE])
 {
@@ -913,7 +921,7 @@ __device__ __forceinline__ void accumulate_samples(HitSetup hs, float4 col, floa
         const float gw = gauss_weight(hs.power);
         asm("v_cmpx_lt_f32_e32 vcc, %[p], %[cut]\n\tv_fmac_f32_e32 %[a], %[w], %[g]\n\tv_fmac_f32_e32 %[r], %[x], %[g]\n\t"
             "v_fmac_f32_e32 %[gg], %[y], %[g]\n\tv_fmac_f32_e32 %[b], %[z], %[g]\n\ts_mov_b64 exec, %[l]"
-            : [a] "+v"(sg[i]), [r] "+v"(cr[i]), [gg] "+v"(cg[i]), [b] "+v"(cb[i])
+            : [a] "+&v"(sg[i]), [r] "+&v"(cr[i]), [gg] "+&v"(cg[i]), [b] "+&v"(cb[i])
             : [p] "v"(hs.power), [cut] "v"(hs.cut), [g] "v"(gw), [x] "v"(col.x), [y] "v"(col.y), [z] "v"(col.z), [w] "v"(col.w), [l] "s"(lanes)
             : "vcc");
         hs.power += hs.inc;
@@ -3253,10 +3261,11 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                             const float wd = gauss_weight(S.power[j]);
                             const float y = fmaf(PA[i], dcg, PB[i]) * wd;
                             const float u = (float)i - 15.5f;
-                            // (see accumulate_samples)
+                            // (see accumulate_samples; here only scalar moves write the mask, and s0 to gc next go through
+                            // the moments' arithmetic)
                             asm("s_mov_b64 exec, %[in]\n\tv_add_f32_e32 %[s0], %[y], %[s0]\n\tv_fmac_f32_e32 %[s1], %[u], %[y]\n\t"
                                 "v_fmac_f32_e32 %[s2], %[uu], %[y]\n\tv_fmac_f32_e32 %[gc], %[a], %[w]\n\ts_mov_b64 exec, %[l]"
-                                : [s0] "+v"(s0), [s1] "+v"(s1), [s2] "+v"(s2), [gc] "+v"(gc)
+                                : [s0] "+&v"(s0), [s1] "+&v"(s1), [s2] "+&v"(s2), [gc] "+&v"(gc)
                                 : [in] "s"(S.in[j]), [y] "v"(y), [a] "v"(PA[i]), [w] "v"(wd), [u] "i"(__builtin_bit_cast(uint32_t, u)),
                                   [uu] "i"(__builtin_bit_cast(uint32_t, u * u)), [l] "s"(lanes));
                         }

@@ -194,3 +194,21 @@ def test_bench_finds_its_stored_profile_figures():
         assert issue and issue["instructions_per_launch"] > 1e9 and 0.0 < issue["frac"] <= 1.0 and issue["peak"] == 600.0
         assert bench.valu_issue(workload, key, 0.01, "cpu")["above_peak"]       # an impossible pairing is flagged, frac capped
     assert bench.stored_traffic("c4_1M_800x800", "no_such_kernel") == (None, None)
+
+
+def test_assembly_of_several_instructions_does_not_share_registers_between_outputs_and_inputs():
+    """An assembly statement that writes an output before it has read its last input must say so ("&"): without it the
+    compiler may give the output's register to an input that holds the same value."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "raygaussx_amd", "csrc")
+    seen = 0
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".h")):
+            continue
+        text = open(os.path.join(csrc, name)).read()
+        for m in re.finditer(r'\basm\s*(?:volatile)?\s*\(((?:\s*"(?:[^"\\]|\\.)*")+)\s*:([^:;]*):', text):
+            code = "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', m.group(1)))
+            outputs = re.findall(r'"([=+][^"]*)"', m.group(2))
+            if outputs and len([i for i in re.split(r"\\n(?:\\t)?", code) if i.strip()]) > 1:
+                seen += 1
+                assert all("&" in o for o in outputs), (name, code[:60], outputs)
+    assert seen >= 3
