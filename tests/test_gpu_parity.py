@@ -535,6 +535,34 @@ def test_forward_without_a_record_is_the_march_that_its_backward_repeats(gx, dyn
     assert np.array_equal(gx.gpu_render(np_scene, cam, cfg, stats=False)["image"], only.cpu().numpy())
 
 
+@pytest.mark.parametrize("w,h", [(52, 44), (216, 224)])
+def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
+    """What the four wavefronts of a tile leave for the backward, in each form: sample sums in floats and in half
+    precision, and hit lists alone.  The image does not depend on the form.  Float sums and lists give the gradients of
+    a backward that searches the tree; half precision rounds a colour sum by at most 2^-12 of the chunk's
+    largest, and a gradient's norm is that of many of them: 2^-12 of it."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=5000, sh_degree=1, seed=21))
+    sc["scales"] = sc["scales"] * 2.0
+    cam = scenes.make_camera(0, 0, width=w, height=h)
+    cfg = dict(dt_step=0.004, dynamic_sampling=False, max_prim_slice=4096)
+    dloss = np.random.default_rng(3).normal(size=(w * h, 3)).astype(np.float32)
+    _step(f"record forms {w}x{h}")
+    tree = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    forms = [("sums", dict(), 1e-4), ("half sums", dict(half_sums=True), 2.0 ** -12), ("lists", dict(rec_tile_words=16384), 1e-4)]
+    images = []
+    for name, kw, tol in forms:
+        for _ in range(2):                     # (the second view's pool is sized from the first)
+            out = gx.gpu_render(sc, cam, cfg, want_grad=dloss, **kw)
+        assert out["stats_bwd"]["nodes_visited"] == 0 and out["stats_bwd"]["hit_pairs"] == tree["stats_bwd"]["hit_pairs"] > 10000
+        images.append(out["image"])
+        for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+            cos, rel = gx.cos_rel(out["grads"][k], tree["grads"][k])
+            print(f"{name}, {k}: rel {rel:.2e}", flush=True)
+            assert cos >= 1 - 1e-6 and rel <= tol, (name, k, cos, rel)
+    assert np.array_equal(images[0], images[1]) and np.array_equal(images[0], images[2])
+    assert np.abs(images[0] - tree["image"]).max() <= 1e-5
+
+
 def test_long_hit_lists_spill_and_truncation(gx, orc):
     """Fat Gaussians: slabs with far more than 32 hits (LDS part + spill area), then a tiny
     max_prim_slice to exercise the silent truncation path and its counter."""
@@ -660,6 +688,26 @@ def test_reorder_tensors_is_the_per_tensor_gather(gx):
             np.testing.assert_array_equal(got.cpu().numpy(), src[idx])
 
 
+@pytest.mark.parametrize("n,words,offset", [
+    (5, 4 * 4096, 0), (3, 4 * 4095, 0), (130, 4 * 4097, 0),        # a row of 16-byte pieces, either side of the long ones
+    (3, 3 * 4099, 0), (3, 2 * 4097, 0), (2, 4099, 0), (2, 8195, 0),   # 12-, 8- and 4-byte pieces (4099, 8195: primes' worth)
+    (257, 4, 1), (257, 8, 2), (257, 6, 1), (257, 2, 1), (257, 9, 1), (4, 4 * 4096, 1), (4, 4 * 4096, 2),   # off a 16- or 8-byte boundary
+    (262_145, 1, 0), (262_145, 12, 0)])                              # one workgroup for all tensors of its rows
+def test_reorder_tensors_of_long_rows_and_off_alignment(gx, n, words, offset):
+    """Rows of every width of piece, so long that a workgroup moves them one by one, and tensors that begin off the
+    boundary that the widest pieces ask for (``offset`` words into their storage)."""
+    from raygaussx_amd.reordering import reorder_tensors
+    gen = torch.Generator(gx.DEV).manual_seed(n + words)
+    store = torch.randint(-2 ** 31, 2 ** 31 - 1, (n * words + offset,), dtype=torch.int32, device=gx.DEV, generator=gen)
+    t = store[offset:].view(n, words)
+    assert t.data_ptr() % 16 == 4 * offset
+    order = torch.randperm(n, device=gx.DEV, generator=gen)
+    _step(f"gather {n} rows of {words} words at {offset}")
+    plain = torch.arange(n, device=gx.DEV, dtype=torch.float32)
+    got, second = reorder_tensors(order, [t, plain])
+    assert torch.equal(got, t[order]) and torch.equal(second, plain[order])
+
+
 def test_reference_style_inference_loop_reuses_the_tree(gx, orc, c0):
     """scripts/test.py:50-126 pattern: boxes -> one acceleration structure -> several cameras."""
     from raygaussx_amd import optix_utils as u_ox
@@ -771,6 +819,48 @@ def test_dist2_knn3_bit_exact(gx, orc):
     ids = rng.choice(1_000_000, 2000, replace=False)
     d, _ = cKDTree(p.astype(np.float64)).query(p[ids].astype(np.float64), k=4)
     np.testing.assert_allclose(got[ids], (d[:, 1:] ** 2).mean(1), rtol=1e-5)
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 63, 64, 65, 1023, 1024, 1025, 65_535, 65_536, 65_537])
+def test_dist2_knn3_at_the_sizes_of_its_boxes(gx, orc, n):
+    """Either side of a leaf, a wavefront, a box and a box of boxes."""
+    from raygaussx_amd.simple_knn import distCUDA2
+    p = np.random.default_rng(n).normal(size=(n, 3)).astype(np.float32)
+    p[n // 2:] *= 30.0
+    _step(f"distCUDA2 n={n}")
+    got = distCUDA2(torch.from_numpy(p).to(gx.DEV)).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), orc.dist2_knn3(p).view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["outliers", "two clumps", "nan", "inf", "nan and inf", "all nan", "huge"])
+def test_dist2_knn3_of_clouds_that_the_curve_does_not_sort(gx, orc, kind):
+    """A few far points leave nearly all the others in one or two cells of the Morton grid, in whose order they say nothing of
+    where they lie.  A point with a coordinate that is no number, or infinite, is no one's neighbour and has none."""
+    from raygaussx_amd.simple_knn import distCUDA2
+    rng = np.random.default_rng(5)
+    n = 6000
+    p = rng.normal(size=(n, 3)).astype(np.float32)
+    if kind == "outliers":
+        p[::900] *= 1e5
+    elif kind == "two clumps":
+        p *= 1e-3
+        p[1::2] += 1e4
+    elif kind == "all nan":
+        p[:] = np.nan
+    elif kind == "huge":
+        p[:10] *= 1e30                                 # squared distances beyond the float range
+    if "nan" in kind and kind != "all nan":
+        p[3::50, 1] = np.nan
+        p[64:128] = np.nan                             # a whole wavefront's worth
+    if "inf" in kind:
+        p[7::40, 2] = np.inf
+        p[9::71, 0] = -np.inf
+        p[200:264, 0] = np.inf
+    _step(f"distCUDA2, {kind}")
+    got = distCUDA2(torch.from_numpy(p).to(gx.DEV)).cpu().numpy()
+    ref = orc.dist2_knn3(p)
+    assert (np.isfinite(ref).all(), np.isfinite(ref).any()) == (kind in ("outliers", "two clumps"), kind != "all nan")
+    np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
 def test_training_loop_as_the_reference_writes_it_reduces_the_loss(gx):
