@@ -13,7 +13,11 @@ metric "Mrays/s fwd+bwd @1M Gaussians 800x800" is quoted on -- one camera of the
 upper-hemisphere orbit per step.  Inputs are resident in HBM before the timed region.
 
 Prints ONE JSON line.  ``roofline`` prices the dominant kernel (the backward march) with its
-algorithmic bytes (64+56 B per ray-slab-hit + 24 B per ray) over its own HIP-event time;
+algorithmic bytes (64+56 B per ray-slab-hit + 24 B per ray) over its own HIP-event time.  Those
+bytes count a Gaussian's record and gradient once per hit; the kernels read and add them from caches and
+LDS for most hits, so ``frac`` is a rate of work in units of the HBM peak, not a share of a bound,
+and passes 1 where hits are dense.  ``counted_frac`` is the share: the HBM bytes that a profiler run counted
+(``traffic``) over the same time and peak.
 ``cpu_baseline`` times the CPU oracle on a bounded ray sample of the same workload.
 ``fwd_fps_c3`` is the other half of the headline metric, measured in the same run: frames per second
 of the forward-only render of the 3 M-Gaussian scene at 1920x1080 along its orbit, tree built once,
@@ -144,6 +148,11 @@ def valu_issue(workload, kernel_key, kernel_ms, dev):
                 above_peak=bool(rate > peak))
 
 
+def counted_frac(traffic, kernel_ms):
+    """Share of the HBM peak that a kernel's counted traffic takes over its time; None without a stored count."""
+    return round(traffic / (kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 5) if traffic and kernel_ms > 0 else None
+
+
 def stored_traffic(workload, kernel_key):
     """HBM bytes per launch of a march kernel as a profiler run measured them: rocprofv3 --pmc FETCH_SIZE /
     WRITE_SIZE of this script, scaled by the same counters' reading for a 1 GiB copy (--calibrate-copy).
@@ -263,7 +272,8 @@ def inference_leg(dev, frames, warmup):
                 workload=name, gaussians=n, width=width, height=height, t_eps=cfg["t_eps"], dynamic_sampling=cfg["dynamic_sampling"],
                 frame="sh + pack + march fwd, 1 view, tree built once and reused",
                 roofline=dict(bound="hbm", kernel="k_march_fwd", achieved=round(gbps, 2), peak=HBM_PEAK_GBPS, unit="GB/s",
-                              frac=round(gbps / HBM_PEAK_GBPS, 5), traffic=traffic, traffic_source=source,
+                              frac=round(gbps / HBM_PEAK_GBPS, 5), counted_frac=counted_frac(traffic, ms_kernel), traffic=traffic,
+                              traffic_source=source,
                               kernel_ms=round(ms_kernel, 4), algorithmic_bytes=int(nbytes), hit_pairs_per_launch=int(hits),
                               valu_issue=valu_issue(name, "march_forward", ms_kernel, dev)),
                 frame_roofline=dict(bytes_per_frame=int(frame_bytes), frac=round(frame_bytes / (ms_frame * 1e-3) / 1e9 / HBM_PEAK_GBPS, 5),
@@ -475,12 +485,13 @@ def training_leg(dev, workload, steps, warmup, opts, in_flight=1):
         gbps = nbytes / (avg * 1e-3) / 1e9 if avg > 0 else 0.0
         per_kernel[key] = dict(kernel=name, kernel_ms=round(avg, 4), algorithmic_bytes=int(nbytes), achieved=round(gbps, 2),
                                frac=round(gbps / HBM_PEAK_GBPS, 5),
+                               counted_frac=counted_frac(stored_traffic(workload, key)[0], avg) if default_record else None,
                                valu_issue=valu_issue(workload, key, avg, dev) if default_record else None)
     kname = max(per_kernel, key=lambda k: per_kernel[k]["kernel_ms"])
     dom = per_kernel[kname]
     traffic, traffic_source = stored_traffic(workload, kname) if default_record else (None, None)
     roofline = dict(bound="hbm", kernel=dom["kernel"], achieved=dom["achieved"], peak=HBM_PEAK_GBPS, unit="GB/s", frac=dom["frac"],
-                    traffic=traffic, traffic_source=traffic_source,
+                    counted_frac=dom["counted_frac"], traffic=traffic, traffic_source=traffic_source,
                     kernel_ms=dom["kernel_ms"], algorithmic_bytes=dom["algorithmic_bytes"],
                     hit_pairs_per_launch=int(hits_per_launch), march_kernels=per_kernel)
     # whole-step roofline-derived rate: all algorithmic bytes of one step at peak bandwidth
@@ -612,20 +623,21 @@ def main():
             others[name] = dict(value=o["value"], unit="Mrays/s", ms_per_step=o["ms_per_step"], steps=o["steps"], warmup=o["warmup"],
                                 step_roofline_frac=o["step_roofline"]["frac"], roofline_mrays=o["step_roofline"]["roofline_mrays"],
                                 dominant_kernel=dom["kernel"], dominant_kernel_ms=dom["kernel_ms"], dominant_kernel_frac=dom["frac"],
-                                march_kernels={k: dict(kernel_ms=v["kernel_ms"], frac=v["frac"],
+                                dominant_kernel_counted_frac=dom["counted_frac"],
+                                march_kernels={k: dict(kernel_ms=v["kernel_ms"], frac=v["frac"], counted_frac=v["counted_frac"],
                                                        lane_slots_per_pair_at_measured_issue_rate=v["lane_slots_per_pair_at_measured_issue_rate"])
                                                for k, v in dom["march_kernels"].items()},
                                 hit_pairs_per_launch=dom["hit_pairs_per_launch"], kernels_ms=o["kernels_ms"], memory=o["memory"],
                                 config=o["config"])
         out["other_workloads"] = others
     if args.cpu_rays > 0:
-        # the box grants a job 16 host threads whatever os.cpu_count() shows: the baseline uses those, and says so
+        # a job may be granted fewer threads than os.cpu_count() shows: the baseline takes 16 at most, and says so
         threads = min(16, os.cpu_count() or 1)
         out["cpu_baseline"] = cpu_baseline(scene, scenes.make_camera(config, 0, width=width, height=height), cfg,
                                            args.cpu_rays if n <= 1_000_000 else min(args.cpu_rays, 16384), threads,
                                            backward=not (args.forward_only or args.workload.endswith("_fwd")))
         out["cpu_baseline"]["host_cpus"] = os.cpu_count()
-        out["cpu_baseline"]["threads_note"] = "min(16, host cpus): 16 is this GPU box's CPU share per job"
+        out["cpu_baseline"]["threads_note"] = "min(16, host cpus)"
     else:
         out["cpu_baseline"] = None
     print(json.dumps(out), flush=True)
