@@ -10,15 +10,18 @@
 //      window, or sweeps the BVH cooperatively (node stack in LDS, one node per lane per step,
 //      starting from the tile's cut through the tree) for the Gaussians whose ellipsoids meet
 //      the tile's frustum in the depth range wanted;
-//   2. filters: a wave-uniform loop over the table in which every lane evaluates the exact hit
-//      predicate for ITS ray and slab (so hit sets are those of a per-ray query); the result is,
-//      per 4x4 pixel row, the list of entries hit, and per lane its hit bits over that list;
-//   3. shades: every lane walks its own hits (forward, the backward's density pass), or the four
-//      rows walk their lists in lock step and sum each entry's 13 whitened-frame sums over the
-//      row's 16 rays with DPP adds (the backward's gradient pass).
+//   2. filters: a wave-uniform loop over the table in which every lane tests ITS ray and slab against the
+//      entry, without the hit predicate's roots unless a decision is close, and then by the exact
+//      predicate (so hit sets are those of a per-ray query); the result is the tile's list of entries hit,
+//      per lane its hit bits over that list, and per 4x4 pixel row which entries reach each half of the samples;
+//   3. shades: every lane walks its own hits (forward, the backward's density pass), or groups of lanes
+//      walk the entries that one of their rays hits, in lock step, and sum each entry's 13 whitened-frame
+//      sums over their rays with DPP adds (the backward's gradient pass: half rows of 8 lanes in a replay, rows
+//      of 16 in the backward that searches the tree).
+// An image of few tiles is marched by four wavefronts per tile (k_march_team, launch_forward).
 // The forward can record what 1 and 2 produced, and the per-sample density and colour sums of 3;
-// the replaying backward then needs no tree, no table, no predicate and no density pass, and
-// sums a window's gradients in LDS before adding them to memory.
+// the replaying backward then needs no tree, no table, no predicate and no density pass, sums a window's
+// gradients in LDS before adding them to memory, and replays a tile in several pieces side by side.
 // The first-hit query (once per ray, and after an empty slab) runs on the same candidate tables.
 // The per-lane skip-link queries below serve the segment test hooks (arbitrary rays).
 #include "rgx_device.h"
@@ -102,7 +105,7 @@ enum { RGX_SEC_SWEEP = 0, RGX_SEC_FILTER = 1, RGX_SEC_SHADE = 2, RGX_SEC_LISTS =
        RGX_SEC_SETUP = 6, RGX_SEC_TOP = 7, RGX_SEC_END = 8, RGX_SEC_EPILOGUE = 9, RGX_SEC_WALK = 10, RGX_SEC_FLUSH = 11 };
 enum { RGX_SEC_PARSE = RGX_SEC_SWEEP, RGX_SEC_COUNT = RGX_SEC_FILTER, RGX_SEC_PRETRIP = RGX_SEC_LISTS }; // the replaying backward's names for sections it has no other use for
 enum { RGX_SECK_FWD_RECORD = 0, RGX_SECK_FWD_PLAIN = 1, RGX_SECK_BWD_SUMS = 2, RGX_SECK_BWD_LISTS = 3, RGX_SECK_BWD_TREE = 4, RGX_NSECK = 5 };
-#define RGX_SEC_ROWS 65536 // workgroups per launch the table has rows for (a 1920x1080 launch has 33 024)
+#define RGX_SEC_ROWS 65536 // rows of the table: a workgroup's own up to that many (a 1920x1080 launch has 33 024), shared beyond
 // [forward / backward][workgroup][section]; word RGX_NSEC of a row counts the waves that used it, the next word names their
 // kernel, words 14 and 15 are the start and end of the last wave that used it on the 100 MHz wall clock.
 // The sums live in memory, not in registers: the march kernels have no registers to spare, and a census that made them
@@ -113,19 +116,19 @@ struct SectionClock {
     unsigned *row = nullptr;
     __device__ __forceinline__ void start(int pass)
     {
-        row = blockIdx.x < RGX_SEC_ROWS ? g_section_cycles[pass][blockIdx.x] : nullptr;
-        if (threadIdx.x == 0 && row) row[14] = (unsigned)wall_clock64(); // when the wave started, 100 MHz ticks (the last launch's)
+        row = g_section_cycles[pass][blockIdx.x % RGX_SEC_ROWS]; // (a replay in pieces has more workgroups than rows)
+        if (threadIdx.x == 0) row[14] = (unsigned)wall_clock64(); // when the wave started, 100 MHz ticks (the last launch's)
         last = (unsigned)__builtin_readcyclecounter();
     }
     __device__ __forceinline__ void to(int k)
     {
         const unsigned now = (unsigned)__builtin_readcyclecounter();
-        if (threadIdx.x == 0 && row) atomicAdd(row + k, now - last);
+        if (threadIdx.x == 0) atomicAdd(row + k, now - last);
         last = now;
     }
     __device__ __forceinline__ void flush(int kernel)
     {
-        if (threadIdx.x != 0 || !row) return;
+        if (threadIdx.x != 0) return;
         atomicAdd(row + RGX_NSEC, 1u);
         row[RGX_NSEC + 1] = (unsigned)kernel;
         row[15] = (unsigned)wall_clock64(); // and when it ended
@@ -1579,7 +1582,6 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
     const int len = row == 0 ? l0 : row == 1 ? l1 : row == 2 ? l2 : l3;
     const int slots_at = it + 8 + (row > 0 && !one ? q0 : 0) + (row > 1 ? q1 : 0) + (row > 2 ? q2 : 0); // the row's slot bytes start at this word
     const int masks_at = it + 8 + q0 + q1 + q2 + q3 + lane;                                      // word w of this lane: masks_at + w * 64
-    (void)RL.rowlist;
     if constexpr (WALK == WALK_NONE) {
         const int nwr = run ? min((len + 31) >> 5, nw) : 0;
         if (COUNT)
@@ -1605,7 +1607,6 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
             body(Entry<false>{(const float4 *)(RL.frame + slot), P.prims + pid, pid, slot}, has, has, Half<(WALK & 1)>{});
         }
     } else {
-        const int maxlen = min(max(max(l0, l1), max(l2, l3)), nw * 32);
         RGX_SEC(cn, RGX_SEC_WALK);
         // the rows' slot lists go to LDS first: every trip starts by looking its slot up, and from memory that
         // look-up is a round trip at the head of the trip's chain of dependent loads
@@ -1616,7 +1617,6 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
             __syncthreads();
         }
         static_assert(!COUNT, "the rows' walk counts nothing");
-        (void)maxlen;
         // Each half of a row (8 lanes, 2 x 4 pixels) walks the entries that one of its own rays hits: the set bits
         // of the OR of its lanes' masks.  Fewer trips than with whole rows in lock step (a trip lasts until the
         // longest list of the wave is done, and half a row's list is shorter than the row's).
@@ -3545,8 +3545,9 @@ enum { RGX_BWD_TREE, RGX_BWD_LISTS, RGX_BWD_SUMS };
 __attribute__((visibility("hidden"))) void rgx_launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s,
                                                                 const MarchParams &P);
 #if RGX_MARCH_TU != 1
-// The backward that searches the tree, and the one that replays the forward's record.  (Three
-// waves per SIMD with some spilling measured faster for the replay than two waves without.)
+// The backward that searches the tree, and those that replay the forward's record: its lists, or its sample sums.
+// (The replay of lists alone keeps the 64 density and colour sums it rebuilds across two walks, and spills 200 bytes a
+// lane; it runs for the first view of a shape, and where memory is short.)
 template <bool STATS>
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd(const MarchParams P) { march_bwd<false, false, STATS>(P); }
 template <bool STATS>
@@ -3592,7 +3593,7 @@ __global__ __launch_bounds__(64) void k_collect_tiles(const MarchParams P, const
     lane_pixel(px0, py0, px, py);
     const bool valid = px < P.cam.width && py < P.cam.height;
     const int64_t ray = (int64_t)py * P.cam.width + px;
-    CountersFor<STATS> cn; // without counters the filter compiles in its early exit, as in the kernels a training loop runs
+    CountersFor<STATS> cn; // with counters or without, as the march kernels
     Frustum F;
     frustum_planes(P.cam, px0, py0, F);
     const f3 dir = compute_ray(P.cam, (unsigned)px, (unsigned)py);

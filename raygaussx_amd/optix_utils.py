@@ -500,7 +500,7 @@ def trace_segments(gas, prims, eye, dirs, tlo, thi, cap):
 
 def collect_tiles(gas, cam, prims, tlo, thi, cap, uncounted=False):
     """Hit lists of per-pixel segments through the tile-cooperative collect (test hook).  ``uncounted``:
-    the filter as the kernels launched without a statistics block compile it (with its early exit)."""
+    without counters, as the kernels launched without a statistics block."""
     n_rays = cam.width * cam.height
     counts = torch.zeros(n_rays, dtype=torch.int32, device=prims.device)
     ids = torch.full((n_rays, cap), -1, dtype=torch.int32, device=prims.device)

@@ -243,7 +243,7 @@ def test_tile_cooperative_collect_hit_sets_bit_exact(gx, orc, c0):
     traces = [orc.march_trace(ctx["cs"], ctx["ms"], ctx["bmin"], ctx["bmax"], ctx["prims"], r)[0] for r in range(R)]
     cams = u_ox.camera_struct(cam)
     checked = 0
-    # uncounted: the filter as the kernels without a statistics block compile it (early exit for entries no ray's line meets)
+    # uncounted: the filter without counters, as in the kernels launched without a statistics block
     for rank, uncounted in ((0, False), (0, True), (1, True), (4, False), (4, True), (9, True)):
         tlo = np.ones(R, np.float32)
         thi = np.zeros(R, np.float32)          # thi < tlo: pixel idle
@@ -330,7 +330,7 @@ def test_backward_config0_gradients(gx, orc, c0):
     assert out["stats_bwd"]["hit_pairs"] == ost["hit_pairs"]
     for k in ("sph_gauss_features", "bandwidth_sharpness", "lobe_axis"):
         assert out["grads"][k] is None
-    # the kernels a training loop runs (no statistics block: no counters, early-exit filter), with each kind of record
+    # the kernels a training loop runs (no statistics block: no counters), with each kind of record
     for label, kw in (("default record", {}), ("hit lists only", dict(rec_tile_words=16384)), ("no record", dict(record_hits=False))):
         _step("forward+backward config0, uncounted kernels, " + label)
         out = gx.gpu_render(sc, cam, cfg, want_grad=dloss, stats=False, **kw)
