@@ -12,8 +12,8 @@ Workload (``config.workload``): the 1 M-Gaussian scene of the training-stress co
 metric "Mrays/s fwd+bwd @1M Gaussians 800x800" is quoted on -- one camera of the
 upper-hemisphere orbit per step.  Inputs are resident in HBM before the timed region.
 
-Prints ONE JSON line.  ``roofline`` prices the dominant kernel (the backward march) with its
-algorithmic bytes (64+56 B per ray-slab-hit + 24 B per ray) over its own HIP-event time.  Those
+Prints ONE JSON line.  ``roofline`` prices the dominant kernel (the march launch that takes longer) with its
+algorithmic bytes (forward 64 B per ray-slab-hit + 12 B per ray, backward 120 and 24) over its own HIP-event time.  Those
 bytes count a Gaussian's record and gradient once per hit; the kernels read and add them from caches and
 LDS for most hits, so ``frac`` is a rate of work in units of the HBM peak, not a share of a bound,
 and passes 1 where hits are dense.  ``counted_frac`` is the share: the HBM bytes that a profiler run counted

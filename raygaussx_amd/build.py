@@ -28,12 +28,14 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
          "-Wno-unused-command-line-argument"]
 # The march kernels have no register to spare, and what the machine-code loop-invariant code motion hoists out
 # of their slab loops (addresses, constants, selects of wave-uniform values) it pays for with spills inside them:
-# without it the recording forward runs 3-4 % faster (36 -> 20 bytes of spills per lane; the plain forward and
-# the replaying backward lose theirs altogether and run as before).
+# without it the recording forward and the replaying backward spill nothing (16 and 24 bytes per lane with it).  It is
+# worth little by now: 3 M Gaussians 1237x822 9.74 -> 9.67 ms forward, 8.60 -> 8.59 backward, 1 M 800x800 equal.
 NO_LICM = ["-mllvm", "-disable-machine-licm=1"]
 # The march source is compiled twice: once for everything but the backward kernels, without the scheduling pass
-# that runs after register allocation (the forward without a record runs 1-3 % faster on what the first
-# scheduler left), and once for the backward kernels alone, which that pass helps by about 1 %.
+# that runs after register allocation, and once for the backward kernels alone, with it.  The backward needs the
+# pass (3 M Gaussians 8.59 ms, 8.71 without; 1 M 5.04 and 5.06).  The forwards ran 1-3 % faster without it when they
+# were divided off; the kernels have changed since, and now they run 1-1.5 % slower without (1 M recording forward
+# 5.32 ms, 5.26 with the pass; 3 M 9.67 and 9.53; 3 M 1920x1080 frame 17.12 and 16.89): the division has outlived its reason.
 # (source, object name, flags of that compilation)
 UNITS = [("rgx_api.hip", "rgx_api", []), ("rgx_build.hip", "rgx_build", []), ("rgx_pergauss.hip", "rgx_pergauss", []),
          ("rgx_image.hip", "rgx_image", []),

@@ -1071,8 +1071,10 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
 // are left are tested by every lane for its own point, and a leaf that some lane needs is read once, as
 // scalars, and met by all lanes in straight-line code.  What bounds it is the issue of those distance
 // computations (12 instructions per point and leaf point); one lane searching on its own through boxes of
-// 256 points made every lane of a wavefront wait for the scans of all others: 5.26 ms at 1 M points,
-// 2.20 ms at 54 k points of a heavy-tailed cloud, against 0.44 and 0.15 ms now.
+// 256 points made every lane of a wavefront wait for the scans of all others.  The whole call, sort and boxes included,
+// took 4.6-5.5 ms for 1 M points of a ball and 2.2-3.1 ms for 54 k of a heavy-tailed cloud (eight draws of each); it takes
+// 0.53-0.57 and 0.20-0.34 ms.  This search is 0.46 ms of the former; of the latter it is what the draws differ in (0.26 of 0.34
+// ms in one): the launch lasts as long as the wavefront whose points lie farthest apart.
 // Distances are (dx*dx + dy*dy) + dz*dz without contraction; rounding is monotone, so the distance to a
 // box that holds a point, computed the same way, is never larger than the distance to the point.
 #define RGX_KNN_LEAF 16

@@ -3799,8 +3799,9 @@ static void order_blocks(MarchParams &P, hipStream_t s)
 {
     // The order only matters for the end of a launch, where ever fewer tiles still run: with many
     // rounds of tiles per wave slot (3072 slots: 12 per CU) that end is a small part of the launch
-    // and the pass over the primitive records costs more than it brings (measured: 1 M Gaussians at
-    // 800x800, 3.3 rounds: forward 7.14 -> 7.02 ms; 3 M Gaussians at 1920x1080, 10.5 rounds: 22.35 -> 22.55 ms).
+    // and the pass over the primitive records takes what it brings (forward without -> with the order: 1 M Gaussians at
+    // 800x800, 3.3 rounds: 5.51 -> 5.32 ms; 300 k there 2.84 -> 2.82; 3 M at 1237x822, 5.2 rounds: 9.71 -> 9.67; 3 M at
+    // 1920x1080, 10.5 rounds: 17.12 -> 17.09).
     if (!P.tile_order || P.n == 0 || (int64_t)P.tiles_x * P.tiles_y > 6 * 3072) return;
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);
