@@ -184,7 +184,7 @@ def _adaptive_gates(gx, orc, sc, cam, cfg, ids, img, st, ctx, dloss, max_aside=0
 
 
 def test_heavy_tailed_scene_ray_sample_against_the_oracle(gx, orc):
-    """The unbounded-scene generator (configs[2]: a dense core plus a shell of large background
+    """The unbounded-scene generator (a dense core plus a shell of large background
     Gaussians) at 1 M Gaussians and its own image size: crowded slabs that need several candidate
     tables, rays that cross hundreds of Gaussians.
 
@@ -204,7 +204,7 @@ def test_heavy_tailed_scene_ray_sample_against_the_oracle(gx, orc):
     for adaptive in (False, True):
         cfg = dict(scenes.CONFIGS[2], dynamic_sampling=adaptive)
         img, st, ctx = orc.render_forward(sc, cam, cfg["dt_step"], cfg["dynamic_sampling"], cfg["max_prim_slice"], ray_ids=ids)
-        _step(f"configs[2] scene, 1 M Gaussians, 1237x822, adaptive step {adaptive}")
+        _step(f"heavy-tailed scene, 1 M Gaussians, 1237x822, adaptive step {adaptive}")
         # measured with the adaptive step: 1 re-phased + 15 on a cut-off edge of 256 rays (6 %), 1 above the gate
         _adaptive_gates(gx, orc, sc, cam, cfg, ids, img, st, ctx, dloss, max_aside=0.12, max_missed=0.01)
 
@@ -334,7 +334,7 @@ def test_inference_orbit_3M_gaussians_1080p(gx, orc):
     sc = scenes.scene_to_numpy(scenes.make_scene(3, n=n))
     sc = {k: sc[k] for k in PARAMS}
     d = gx.to_dev(sc)
-    _step("configs[3]: tree of 3 M Gaussians, built once")
+    _step("tree of 3 M Gaussians, built once")
     tree = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(d["positions"], d["scales"], d["quaternions"], d["densities"])
     rephased = missed = total = 0
     for index in (0, 101, 233):
@@ -342,7 +342,7 @@ def test_inference_orbit_3M_gaussians_1080p(gx, orc):
         ids = np.unique(np.random.default_rng(40 + index).integers(0, w * h, 160))
         img, st, ctx = orc.render_forward(sc, cam, cfg["dt_step"], True, cfg["max_prim_slice"], t_eps=cfg["t_eps"], ray_ids=ids)
         assert st["hit_pairs"] > 50000 and st["overflow_rays"] == 0
-        _step(f"configs[3]: camera {index}")
+        _step(f"1920x1080, camera {index}")
         rgb = compute_rgb(cam.camera_center, d["positions"], d["color_features"], None, None, None, 0, 3)
         frames = [u_ox.launch_pipeline_test(None, None, tree, None, None, cfg["dt_step"], True, cam.to(gx.DEV), d["densities"], rgb,
                                             d["positions"], d["scales"], d["quaternions"], cfg["max_prim_slice"], t_eps=cfg["t_eps"])
@@ -364,7 +364,7 @@ def test_inference_orbit_3M_gaussians_1080p(gx, orc):
 
 
 def test_heavy_tailed_scene_at_3M_gaussians(gx, orc):
-    """configs[2] at its own size: 3 M Gaussians, 1237x822, adaptive step, forward and backward."""
+    """The heavy-tailed scene at its own size: 3 M Gaussians, 1237x822, adaptive step, forward and backward."""
     n, w, h = 3_000_000, 1237, 822
     cfg = scenes.CONFIGS[2]
     sc = scenes.scene_to_numpy(scenes.make_scene(2, n=n))
@@ -374,7 +374,7 @@ def test_heavy_tailed_scene_at_3M_gaussians(gx, orc):
     dloss = np.zeros((w * h, 3), np.float32)
     dloss[ids] = np.random.default_rng(28).normal(size=(len(ids), 3)).astype(np.float32)
     img, st, ctx = orc.render_forward(sc, cam, cfg["dt_step"], True, cfg["max_prim_slice"], ray_ids=ids)
-    _step("configs[2]: 3 M Gaussians, 1237x822, adaptive step, forward + backward")
+    _step("heavy-tailed scene, 3 M Gaussians, 1237x822, adaptive step, forward + backward")
     _adaptive_gates(gx, orc, sc, cam, cfg, ids, img, st, ctx, dloss)
 
 
@@ -473,7 +473,7 @@ def test_object_scene_300k_gaussians_800x800(gx, orc):
             orc.set_backward_mask_form(0)
         og, _ = orc.render_backward(sc, ctx, img, dl)
         assert st["hit_pairs"] > 40000 and st["overflow_rays"] == 0
-        _step(f"configs[1]: 300 k Gaussians, 800x800, camera {index}, {int((~stable).sum())} rays on a cut-off edge")
+        _step(f"300 k Gaussians, 800x800, camera {index}, {int((~stable).sum())} rays on a cut-off edge")
         _, counts = gx.gpu_forward_counts(sc, cam, cfg)
         assert np.array_equal(counts[ids], oc)                  # slabs blended and hit-list lengths, ray by ray
         images = []
@@ -557,7 +557,7 @@ def test_training_stress_1M_1024x1024_windows_with_reorder_and_rebuild(gx, orc):
             print(f"{label} {k}: 1 - cos {1 - cos:.2e}, rel {rel:.2e}", flush=True)
             assert cos >= COS_MIN and rel <= REL_MAX, (label, k, cos, rel)
 
-    _step("configs[4] at 1024x1024: window of 20 views, one tree")
+    _step("1 M Gaussians, 1024x1024: window of 20 views, one tree")
     params = [torch.from_numpy(sc[k]).to(gx.DEV).requires_grad_(True) for k in PARAMS]
     got, want, worst, gas, _ = window(params, sc, list(range(20)), None, 24)
     assert worst <= IMG_TOL
@@ -580,7 +580,7 @@ def test_training_stress_1M_1024x1024_windows_with_reorder_and_rebuild(gx, orc):
     assert np.all(np.diff(codes.astype(np.int64)) >= 0)                     # and leaves the cloud sorted along the curve
     params2 = [t.requires_grad_(True) for t in moved]
 
-    _step("configs[4] at 1024x1024: second window, tree rebuilt in place over the renumbered Gaussians")
+    _step("1 M Gaussians, 1024x1024: second window, tree rebuilt in place over the renumbered Gaussians")
     ws_before = gas.ws.data_ptr()
     got2, want2, worst2, gas2, first2 = window(params2, scene2, list(range(20, 40)), gas, 24)
     assert gas2 is gas and gas.ws.data_ptr() == ws_before and worst2 <= IMG_TOL

@@ -12,7 +12,7 @@ from raygaussx_amd import scenes
 
 pytestmark = pytest.mark.gpu
 
-# north_star's gradient gates; equal inputs through the same kernels differ only in the order of the
+# the gradient gates; equal inputs through the same kernels differ only in the order of the
 # fp32 atomic adds, so the test holds the two entry points much closer than the gates
 COS_MIN, REL_MAX = 0.9999, 1e-3
 REL_SAME_KERNELS = 1e-5
