@@ -934,9 +934,12 @@ __device__ __forceinline__ void accumulate_samples(HitSetup hs, float4 col, floa
 
 // Four samples of the recurrence: their powers, and for each the rays for which it lies inside the cut-off.  The rays of a
 // trip walk lists of one order and so are at similar depths: for many a block of four no ray has a sample, and then its
-// exponentials and sums are left out: 23 % of the backward's blocks at 1 M Gaussians 800x800 (5.25 -> 5.0 ms), 58 % at 3 M
-// 1237x822 (10.0 -> 8.4 ms).  In the forward, whose walks have two chunks and more rays per trip, it is 9 and 30 %, and the
-// branches cost more than that (3 M 1920x1080: 17.4 -> 17.7 ms).
+// exponentials and sums are left out: 23 % of the backward's blocks at 1 M Gaussians 800x800 (5.27 -> 5.07 ms), 58 % at 3 M
+// 1237x822 (10.1 -> 8.4 ms).  Where tiles are light and few a wavefront has its SIMD to itself and waits for the branch:
+// 4 k Gaussians 128x128 0.142 -> 0.161 ms, 100 k 400x400 0.567 -> 0.590, 300 k 440x440 1.47 -> 1.51 (the replay of lists
+// alone the same); up to 3 000 tiles other scenes gain as much as these lose (3 M 256x256 2.32 -> 2.04, 1 M 440x440 2.75 -> 2.55), so
+// one form serves all.  In the forward, whose walks have two chunks and more rays per trip, it is 9 and 30 % of the blocks, and
+// the branches cost more than that (3 M 1920x1080: 17.4 -> 17.7 ms).
 #define RGX_SAMPLE_BLOCK 4
 struct SampleBlock {
     float power[RGX_SAMPLE_BLOCK];
