@@ -5,7 +5,7 @@
 evaluation (fused multiply-adds only where the source says fmaf);
 ``-munsafe-fp-atomics`` selects the hardware fp32 atomic add for the gradient
 scatter; packed-fp32 code generation is disabled; the march kernels' source is compiled without
-machine-code loop-invariant code motion, in two pieces with different scheduling (``UNITS``).
+machine-code loop-invariant code motion (``UNITS``).
 
 ``python -m raygaussx_amd.build --resources`` also prints what every kernel takes: registers,
 bytes of register spills per lane, LDS.  The march kernels are sized for three wavefronts per SIMD
@@ -31,18 +31,13 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # without it the recording forward and the replaying backward spill nothing (16 and 24 bytes per lane with it).  It is
 # worth little by now: 3 M Gaussians 1237x822 9.74 -> 9.67 ms forward, 8.60 -> 8.59 backward, 1 M 800x800 equal.
 NO_LICM = ["-mllvm", "-disable-machine-licm=1"]
-# The march source is compiled twice: once for everything but the backward kernels, without the scheduling pass
-# that runs after register allocation, and once for the backward kernels alone, with it.  The backward needs the
-# pass (3 M Gaussians 8.59 ms, 8.71 without; 1 M 5.04 and 5.06).  The forwards ran 1-3 % faster without it when they
-# were divided off; the kernels have changed since, and now they run 1-1.5 % slower without (1 M recording forward
-# 5.32 ms, 5.26 with the pass; 3 M 9.67 and 9.53; 3 M 1920x1080 frame 17.12 and 16.89): the division has outlived its reason.
+# (The scheduling pass that runs after register allocation stays on for all of them.  The forwards once ran 1-3 % faster
+# without it and were compiled apart for that; with it they now take 5.24 instead of 5.28 ms at 1 M 800x800, 9.47 instead of
+# 9.63 at 3 M 1237x822, 16.9 instead of 17.1 for the 3 M 1920x1080 frame, 0.607 instead of 0.631 for 4 k Gaussians 128x128.)
 # (source, object name, flags of that compilation)
 UNITS = [("rgx_api.hip", "rgx_api", []), ("rgx_build.hip", "rgx_build", []), ("rgx_pergauss.hip", "rgx_pergauss", []),
          ("rgx_image.hip", "rgx_image", []),
-         ("rgx_march.hip", "rgx_march", ["-DRGX_MARCH_TU=1", *NO_LICM, "-mllvm", "-enable-post-misched=0"]),
-         ("rgx_march.hip", "rgx_march_bwd", ["-DRGX_MARCH_TU=2", *NO_LICM])]
-# The diagnostic build keeps the march source in one piece (its cycle table is one device variable).
-UNITS_SECTIONS = UNITS[:4] + [("rgx_march.hip", "rgx_march", NO_LICM)]
+         ("rgx_march.hip", "rgx_march", NO_LICM)]
 
 
 def _resource_table(compiler_output):
@@ -69,14 +64,14 @@ def _resource_table(compiler_output):
     return "\n".join(out)
 
 
-def build(verbose=False, extra=(), lib=LIB, tag="", resources=False, units=None):
+def build(verbose=False, extra=(), lib=LIB, tag="", resources=False):
     """``extra``: more hipcc flags; ``lib`` / ``tag``: write a differently named library and objects;
-    ``resources``: print every kernel's register, spill and LDS use; ``units``: the compilations (``UNITS``)."""
+    ``resources``: print every kernel's register, spill and LDS use."""
     objs = []
     procs = []
     if resources:
         extra = [*extra, "-Rpass-analysis=kernel-resource-usage"]
-    for src, name, flags in (UNITS if units is None else units):
+    for src, name, flags in UNITS:
         obj = os.path.join(CSRC, name + tag + ".o")
         cmd = ["hipcc", *FLAGS, *flags, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
@@ -108,7 +103,7 @@ def build_sections(**kw):
     """The diagnostic build with the per-section cycle census of the march kernels compiled in
     (``-DRGX_SECTION_CLOCKS``): ``librgx_sections.so`` beside the product library, which it never replaces.
     ``RGX_LIB_PATH=raygaussx_amd/librgx_sections.so python bench.py --sections`` reads the census."""
-    return build(extra=["-DRGX_SECTION_CLOCKS"], lib=SECTIONS_LIB, tag="_sections", units=UNITS_SECTIONS, **kw)
+    return build(extra=["-DRGX_SECTION_CLOCKS"], lib=SECTIONS_LIB, tag="_sections", **kw)
 
 
 if __name__ == "__main__":

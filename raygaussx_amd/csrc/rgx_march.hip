@@ -50,12 +50,6 @@
 // stack never holds more than QCAP - 96 + 93 < QCAP entries, whatever the scene.
 #define RGX_DFS_MARGIN 160
 #define RGX_LDS_HITS 32    // per-lane list of the stand-alone collect hook
-// This source can be compiled as one translation unit (RGX_MARCH_TU undefined or 0) or as two, so that the
-// backward kernels can be given other compiler flags than the rest: 1 = everything except the three backward
-// kernels, 2 = only those and the function that launches them.
-#ifndef RGX_MARCH_TU
-#define RGX_MARCH_TU 0
-#endif
 // The march kernels are sized (registers and LDS) for three wavefronts per SIMD.
 #ifndef RGX_WAVES_ATTR
 #define RGX_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(3, 3)))
@@ -3398,7 +3392,6 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     RGX_SEC_FLUSH(cn, REPLAY ? (SUMS ? RGX_SECK_BWD_SUMS : RGX_SECK_BWD_LISTS) : RGX_SECK_BWD_TREE);
 }
 
-#if RGX_MARCH_TU != 2
 // Launch order of the replaying backward.  A tile is one wavefront's work from start to end, so a
 // launch ends with a tail in which ever fewer tiles are still running; the tail is as long as the
 // tiles that start last.  The records say how much work each tile is (words used), so every XCD
@@ -3540,14 +3533,6 @@ __global__ __launch_bounds__(1024) void k_block_order(const MarchParams P, const
     }
 }
 
-#endif // RGX_MARCH_TU != 2
-
-// The three backward kernels are launched through this one function, which lives in the translation unit
-// that holds them.
-enum { RGX_BWD_TREE, RGX_BWD_LISTS, RGX_BWD_SUMS };
-__attribute__((visibility("hidden"))) void rgx_launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s,
-                                                                const MarchParams &P);
-#if RGX_MARCH_TU != 1
 // The backward that searches the tree, and those that replay the forward's record: its lists, or its sample sums.
 // (The replay of lists alone keeps the 64 density and colour sums it rebuilds across two walks, and spills 200 bytes a
 // lane; it runs for the first view of a shape, and where memory is short.)
@@ -3561,7 +3546,8 @@ template <bool STATS, bool HALF = false>
 #endif
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR_SUMS void k_march_bwd_replay_sums(const MarchParams P) { march_bwd<true, true, STATS, HALF>(P); }
 
-void rgx_launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
+enum { RGX_BWD_TREE, RGX_BWD_LISTS, RGX_BWD_SUMS };
+static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
 {
     const dim3 wave(64);
     if (which == RGX_BWD_SUMS) {
@@ -3577,9 +3563,6 @@ void rgx_launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream
         else hipLaunchKernelGGL(k_march_bwd<false>, grid, wave, 0, s, P);
     }
 }
-#endif // RGX_MARCH_TU != 1
-
-#if RGX_MARCH_TU != 2
 
 // Test hook for the cooperative collect: per pixel a segment [tlo, thi] (thi < tlo = pixel idle);
 // writes each ray's hit count (negated when cut at cap) and the INPUT indices of its hits.
@@ -4033,12 +4016,12 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
             P.use_tile_order = 1;
         }
         if (P.sum_pool)
-            rgx_launch_march_bwd(RGX_BWD_SUMS, stats != nullptr, P.m.record_format == 1, dim3(march_grid(P).x * (unsigned)P.rec_pieces), s, P);
-        rgx_launch_march_bwd(RGX_BWD_LISTS, stats != nullptr, false, march_grid(P), s, P);
+            launch_march_bwd(RGX_BWD_SUMS, stats != nullptr, P.m.record_format == 1, dim3(march_grid(P).x * (unsigned)P.rec_pieces), s, P);
+        launch_march_bwd(RGX_BWD_LISTS, stats != nullptr, false, march_grid(P), s, P);
         P.only_overflow = 1;
         P.use_tile_order = 0;
     }
-    rgx_launch_march_bwd(RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
+    launch_march_bwd(RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
     rgx_span_end(span, s);
     span = timed ? rgx_span_begin(RGX_T_UNPERMUTE, s) : nullptr;
     hipLaunchKernelGGL(k_unpermute_grads, grid_for(n, 256), dim3(256), 0, s, (const float4 *)P.gbuf, P.place, n, ddens, drgb,
@@ -4290,4 +4273,3 @@ extern "C" int rgx_probe_valu_rate(int32_t waves, int32_t iters, int32_t kind, f
     RGX_LAUNCH_CHECK();
     return RGX_OK;
 }
-#endif // RGX_MARCH_TU != 2
