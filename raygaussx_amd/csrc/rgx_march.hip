@@ -1093,12 +1093,9 @@ struct Half {
 };
 // Tag of a walk in which the two halves of a row (8 lanes each) walk on their own.  (Groups of 4 make
 // still fewer trips, but four times a row's adds to the window's sums in LDS: measured slower.)
-#ifndef RGX_GRAD_GROUP
-#define RGX_GRAD_GROUP 8
-#endif
 struct HalfRows {
     static constexpr int value = 0;
-    static constexpr int group = RGX_GRAD_GROUP;
+    static constexpr int group = 8;
 };
 
 // Shade: the four rows walk the entries that one of their own rays hits in lock step; body(entry, hit, live) runs whenever
@@ -1448,15 +1445,14 @@ __device__ __forceinline__ void sums_to_gradients(const Prim *pr, const float *s
 }
 
 // The replaying backward keeps, per tile, the sums of the current window's Gaussians in LDS (one
-// column of RGX_NSUM per table slot): a row's share is added there with LDS atomics, and the
+// row of RGX_NSUM per table slot): the groups of lanes add their shares there (GroupAdd), and the
 // gradients go to memory once per window instead of once per row, slab and Gaussian.
-#define RGX_SLOT_TOUCHED 0x80000000u
 // The record as the replay reads it: the tile's region in memory, of which the words
 // [at, at + RGX_STAGE_WORDS) are also held in LDS once stage() has fetched them.  An iteration's items are
 // read word by word, each read depending on the last (a head gives a size gives the next head), and from
 // memory every link of that chain is a round trip; staged, the chain costs one.  Words outside the staged
 // range are read from memory as before.
-#define RGX_STAGE_WORDS 512
+#define RGX_STAGE_WORDS 448 // (as many as fit beside the rest: twelve tiles per CU)
 template <bool STAGED>
 struct RecordView {
     const uint32_t *reg; // the tile's region
@@ -1493,8 +1489,9 @@ struct RecordView {
 };
 
 struct ReplayLds {
-    float *acc;        // [RGX_NSUM][RGX_CCAP], component-major so that different slots fall in different banks
-    uint32_t *pid;     // [RGX_CCAP]: the window's Gaussians by slot; top bit: the slot has something in acc
+    float *acc;        // [RGX_CCAP][RGX_NSUM]: a group's lanes meet a row in different banks
+    uint32_t *pid;     // [RGX_CCAP]: the window's Gaussians by slot
+    uint8_t *mark;     // [RGX_CCAP]: 0, or (the slot has something in acc) 1 + the group that last claimed it (GroupAdd)
     float *frame;      // [9][RGX_CCAP]: rotation columns U, V, W of the window's Gaussians
     uint8_t *rowlist;  // [4][RGX_CCAP]: the slot lists of the LISTS item whose gradient pass is running
 };
@@ -1513,16 +1510,17 @@ __device__ __forceinline__ void replay_flush(const MarchParams &P, const ReplayL
     const int lane = threadIdx.x;
     for (int first = 0; first < RGX_CCAP; first += 64) {
         const int slot = first + lane;
-        const uint32_t word = slot < RGX_CCAP ? RL.pid[slot] : 0u;
-        const uint64_t touched = __ballot((word & RGX_SLOT_TOUCHED) != 0u);
-        if (word & RGX_SLOT_TOUCHED) {
-            const uint32_t pid = word & ~RGX_SLOT_TOUCHED;
-            RL.pid[slot] = pid;
+        const bool mine = slot < RGX_CCAP && RL.mark[slot] != 0;
+        const uint64_t touched = __ballot(mine);
+        if (mine) {
+            const uint32_t pid = RL.pid[slot];
+            RL.mark[slot] = 0;
+            cn.grad_atomics += 14;
             float sums[RGX_NSUM], out[14];
 #pragma unroll
             for (int c = 0; c < RGX_NSUM; ++c) {
-                sums[c] = RL.acc[c * RGX_CCAP + slot];
-                RL.acc[c * RGX_CCAP + slot] = 0.f;
+                sums[c] = RL.acc[slot * RGX_NSUM + c];
+                RL.acc[slot * RGX_NSUM + c] = 0.f;
             }
             sums_to_gradients(P.prims + pid, sums, out);
             float *row = RL.frame + rank_in(touched) * RGX_FLUSH_ROW;
@@ -1600,7 +1598,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
                 slot = min((int)rv.byte(slots_at, w * 32 + __builtin_ctz(bits)), RGX_CCAP - 1);
                 bits &= bits - 1u;
             }
-            const int32_t pid = (int32_t)(RL.pid[slot] & ~RGX_SLOT_TOUCHED);
+            const int32_t pid = (int32_t)RL.pid[slot];
             body(Entry<false>{(const float4 *)(RL.frame + slot), P.prims + pid, pid, slot}, has, has, Half<(WALK & 1)>{});
         }
     } else {
@@ -1625,7 +1623,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
         auto group_or = [](uint32_t m) {
             m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, true);  // quad_perm [1,0,3,2]
             m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);  // quad_perm [2,3,0,1]
-            if (RGX_GRAD_GROUP >= 8) m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true); // row_half_mirror
+            m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true); // row_half_mirror
             return m;
         };
         int w = 0;
@@ -1661,7 +1659,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
             bits &= bits - 1u;
             a.hit = a.live && ((mword >> pos) & 1u);
             a.slot = min((int)slots[min(w * 32 + pos, RGX_CCAP - 1)], RGX_CCAP - 1);
-            a.pid = (int32_t)(RL.pid[a.slot] & ~RGX_SLOT_TOUCHED);
+            a.pid = (int32_t)RL.pid[a.slot];
             const Prim *prim = P.prims + (uint32_t)a.pid;
             a.pos4 = prim->pos4;
             a.inv4 = prim->inv_inter4;
@@ -3008,38 +3006,79 @@ __device__ __forceinline__ void group_sums_split(const float (&out)[RGX_NSUM], f
                  : "v"(out[0]), "v"(out[1]), "v"(out[2]), "v"(out[3]), "v"(out[4]), "v"(out[5]), "v"(out[6]), "v"(out[7]),
                    "v"(out[8]), "v"(out[9]), "v"(out[10]), "v"(out[11]), "v"(out[12]));
 #pragma unroll
+    for (int c = 0; c < 7; ++c) r[c] += row_take<0xB1>(r[c]); // quad_perm [1,0,3,2]
+    __builtin_amdgcn_sched_barrier(0); // (a component's two steps one right after the other would wait for each other)
+#pragma unroll
     for (int c = 0; c < 7; ++c) {
-        r[c] += row_take<0xB1>(r[c]); // quad_perm [1,0,3,2]
         r[c] += row_take<0x4E>(r[c]); // quad_perm [2,3,0,1]
         asm volatile("" : "+v"(r[c])); // (here, for all lanes: otherwise the last add moves under the condition of the adds to LDS and leaves a move behind)
     }
 }
 
-// Adds the groups' sums to those of their slots in LDS, every lane one or two of its group's.  An atomic float add takes the LDS
-// unit, which all of a CU's wavefronts share, some four clocks a lane; so where a row's two groups are at one slot, as
-// often in dense scenes, the first adds for both (3 M Gaussians 1237x822: 8.4 -> 8.1 ms, 1 M 800x800: 5.03 -> 4.94).
-// The same between rows costs as much as it saves, and plain reads and writes, with the groups at one slot taking
-// turns, wait too long (12.3 -> 12.8 and 5.7 -> 6.3 ms when measured).
-// r: as group_sums_split leaves it; todo: the lane's group has something to add.  Returns whether the lane's group added.
-__device__ __forceinline__ bool add_group_sums(float *acc, const float (&r)[7], int slot, bool todo)
+// LDS words that the lanes of one wavefront hand to each other: a wavefront's LDS accesses take place in program order,
+// and these stay in it (plain ones the compiler may forward, or move past each other where lanes differ in address).
+template <typename T>
+__device__ __forceinline__ T lds_get(const T *p)
 {
-    const int lane = threadIdx.x, q = lane & 3;
-    const bool upper = lane & 4, two = q < (upper ? 2 : 3); // lane q of a quad: its components q and q + 4
-    const float r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3], r4 = r[4], r5 = r[5], r6 = r[6];
-    float v0 = q == 0 ? r0 : q == 1 ? r1 : q == 2 ? r2 : r3, v1 = q == 0 ? r4 : q == 1 ? r5 : r6;
-    const int key = todo ? slot : -1 - lane;
-    const bool both = key == __builtin_amdgcn_update_dpp(0, key, 0x128, 0xf, 0xf, true); // row_ror:8
-    const float other0 = row_take<0x128>(v0), other1 = row_take<0x128>(v1);
-    v0 = both ? v0 + other0 : v0;
-    v1 = both ? v1 + other1 : v1;
-    todo = todo && !(both && (lane & 8));
-    if (todo) {
-        float *dst = acc + ((upper ? 7 : 0) + q) * RGX_CCAP + slot;
-        unsafeAtomicAdd(dst, v0);
-        if (two) unsafeAtomicAdd(dst + 4 * RGX_CCAP, v1);
-    }
-    return todo;
+    return __hip_atomic_load((const __attribute__((address_space(3))) T *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
+template <typename T>
+__device__ __forceinline__ void lds_put(T *p, T v)
+{
+    __hip_atomic_store((__attribute__((address_space(3))) T *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// Adds the groups' sums of a trip to those of their slots in LDS, every lane one or two of its group's.  An atomic float
+// add takes the LDS unit, which all of a CU's wavefronts share, some four clocks a lane: at 3 M Gaussians 1237x822, with
+// 5.9 groups adding in a trip, that was a seventh of the kernel's time.  So
+//   where a row's two groups are at one slot, as often in dense scenes, the first adds for both (between rows it costs as much
+//     as it saves);
+//   of the groups that are then left at a slot, one adds by reading and writing it: every group leaves its number in the
+//     slot's mark, and the one that finds its own there reads the slot's sums beforehand -- begin(), long enough before
+//     end() that no wait is left -- and writes them back with its own added;
+//   the others (a third to a quarter of the groups that add) add atomically after those writes.
+// Backward with all groups adding atomically -> now: 3 M 1237x822 8.53 -> 7.58 ms, 300 k 800x800 2.00 -> 1.91, 1 M 800x800
+// 4.98 -> 4.89.  (Without any adds it would take 7.37, 1.89 and 4.85.)
+struct GroupAdd {
+    bool todo, both, first; // this lane's group adds; for the row's other group as well; reading and writing the slot
+    float old0, old1;       // what the slot's sums were before this trip
+    // adds: the lane's group has something for `slot`
+    __device__ __forceinline__ void begin(const float *acc, uint8_t *mark, int slot, bool adds)
+    {
+        const int lane = threadIdx.x, q = lane & 3;
+        const int key = adds ? slot : -1 - lane;
+        both = key == __builtin_amdgcn_update_dpp(0, key, 0x128, 0xf, 0xf, true); // row_ror:8
+        todo = adds && !(both && (lane & 8));
+        const uint8_t group = (uint8_t)((lane >> 3) + 1);
+        if (todo) lds_put(mark + slot, group);
+        first = lds_get(mark + slot) == group;
+        const float *src = acc + slot * RGX_NSUM + ((lane & 4 ? 7 : 0) + q);
+        old0 = lds_get(src);
+        old1 = lds_get(src + (q < (lane & 4 ? 2 : 3) ? 4 : 0));
+    }
+    // r: as group_sums_split leaves it
+    __device__ __forceinline__ void end(float *acc, const float (&r)[7], int slot) const
+    {
+        const int lane = threadIdx.x, q = lane & 3;
+        const bool upper = lane & 4, two = q < (upper ? 2 : 3); // lane q of a quad: its components q and q + 4
+        const float r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3], r4 = r[4], r5 = r[5], r6 = r[6];
+        float v0 = q == 0 ? r0 : q == 1 ? r1 : q == 2 ? r2 : r3, v1 = q == 0 ? r4 : q == 1 ? r5 : r6;
+        const float other0 = row_take<0x128>(v0), other1 = row_take<0x128>(v1);
+        v0 = both ? v0 + other0 : v0;
+        v1 = both ? v1 + other1 : v1;
+        float *dst = acc + slot * RGX_NSUM + ((upper ? 7 : 0) + q);
+        if (todo && first) {
+            lds_put(dst, old0 + v0);
+            if (two) lds_put(dst + 4, old1 + v1);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (todo && !first) {
+            unsafeAtomicAdd(dst, v0);
+            if (two) unsafeAtomicAdd(dst + 4, v1);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Backward: __raygen__rg of cuda_train/backward/gaussians_aabb.cu:209-497.
@@ -3059,7 +3098,7 @@ __device__ __forceinline__ bool add_group_sums(float *acc, const float (&r)[7], 
 // nineteen running sums; the `power < k^2` mask follows the forward's 32-step recurrence, i.e. it
 // is the mask the forward blended with.  Per Gaussian the moments turn into 13 sums in its whitened
 // frame (RGX_NSUM); those are summed over the rays of a group of lanes (a row of 16 in the walk by rows, half a
-// row in a replay) with DPP adds and carried on by one lane per group (all eight in a replay: add_group_sums); the
+// row in a replay) with DPP adds and carried on by one lane per group (all eight in a replay: GroupAdd); the
 // change of variables to the 14 gradient words comes after all sums.
 template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false>
 __device__ __forceinline__ void march_bwd(const MarchParams &P)
@@ -3086,11 +3125,15 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     __shared__ uint32_t s_pid[REPLAY ? RGX_CCAP : 1];
     __shared__ float s_frame[REPLAY ? 9 * RGX_CCAP : 1];
     __shared__ __align__(4) uint8_t s_rowlist[REPLAY ? 4 * RGX_CCAP : 4];
-    __shared__ uint32_t s_stage[REPLAY && SUMS ? RGX_STAGE_WORDS : 1]; // (with it the kernel's LDS comes to the forward's 12 800 bytes)
-    const ReplayLds RL = {s_acc, s_pid, s_frame, s_rowlist};
+    __shared__ uint32_t s_stage[REPLAY && SUMS ? RGX_STAGE_WORDS : 1];
+    __shared__ uint8_t s_mark[REPLAY ? RGX_CCAP : 1];
+    const ReplayLds RL = {s_acc, s_pid, s_mark, s_frame, s_rowlist};
     if constexpr (REPLAY) {
         for (int i = lane; i < RGX_NSUM * RGX_CCAP; i += 64) s_acc[i] = 0.f;
-        for (int i = lane; i < RGX_CCAP; i += 64) s_pid[i] = 0u;
+        for (int i = lane; i < RGX_CCAP; i += 64) {
+            s_pid[i] = 0u;
+            s_mark[i] = 0;
+        }
         __syncthreads();
     }
     int px, py;
@@ -3230,6 +3273,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             // (3) per table entry: moments per lane, row sum, one set of atomics per row
             auto gradients = [&](const auto &e, bool hit, bool live, auto which) {
                 constexpr int GROUP = decltype(which)::group; // lanes that share this trip's entry
+                static_assert(!REPLAY || GROUP == 8, "a replay walks by half rows");
                 RGX_SEC(cn, RGX_SEC_WALK);
                 float out[RGX_NSUM];
 #pragma unroll
@@ -3285,42 +3329,26 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 }
                 // summed over the group's rays; one lane per group carries the sums on
                 const uint64_t bal = __ballot(hit);
-                if constexpr (REPLAY && GROUP == 8) {
+                if constexpr (REPLAY) {
+                    GroupAdd add;
+                    add.begin(s_acc, s_mark, e.slot, live && ((bal >> (lane & ~7)) & 0xffull) != 0);
+                    __builtin_amdgcn_sched_barrier(0); // (what begin() asks LDS for arrives behind the sums)
                     float r[7];
                     group_sums_split(out, r);
-                    const bool adds = add_group_sums(s_acc, r, e.slot, live && ((bal >> (lane & ~7)) & 0xffull));
-                    if (adds) {
-                        if constexpr (STATS) {
-                            if ((lane & 7) == 0 && !(atomicOr(&s_pid[e.slot], RGX_SLOT_TOUCHED) & RGX_SLOT_TOUCHED)) cn.grad_atomics += 14;
-                        } else {
-                            s_pid[e.slot] = (uint32_t)e.pid | RGX_SLOT_TOUCHED;
-                        }
-                    }
+                    add.end(s_acc, r, e.slot);
                     RGX_SEC(cn, RGX_SEC_SHADE);
                     return;
                 }
 #pragma unroll
                 for (int c = 0; c < RGX_NSUM; ++c) out[c] = group_sum<GROUP>(out[c]);
                 if ((lane & (GROUP - 1)) == 0 && live && ((bal >> lane) & ((1ull << GROUP) - 1ull))) {
-                    if constexpr (REPLAY) {
-                        // to the window's sums in LDS; a slot's first touch is what replay_flush()
-                        // later turns into 14 adds to memory
-                        if constexpr (STATS) {
-                            if (!(atomicOr(&s_pid[e.slot], RGX_SLOT_TOUCHED) & RGX_SLOT_TOUCHED)) cn.grad_atomics += 14;
-                        } else {
-                            atomicOr(&s_pid[e.slot], RGX_SLOT_TOUCHED);
-                        }
+                    // to memory
+                    float grad[14];
+                    sums_to_gradients(e.prim, out, grad);
+                    float *dst = P.gbuf + (int64_t)pid * 16;
 #pragma unroll
-                        for (int c = 0; c < RGX_NSUM; ++c) unsafeAtomicAdd(&s_acc[c * RGX_CCAP + e.slot], out[c]);
-                    } else {
-                        // to memory
-                        float grad[14];
-                        sums_to_gradients(e.prim, out, grad);
-                        float *dst = P.gbuf + (int64_t)pid * 16;
-#pragma unroll
-                        for (int c = 0; c < 14; ++c) unsafeAtomicAdd(dst + c, grad[c]);
-                        cn.grad_atomics += 14;
-                    }
+                    for (int c = 0; c < 14; ++c) unsafeAtomicAdd(dst + c, grad[c]);
+                    cn.grad_atomics += 14;
                 }
                 RGX_SEC(cn, RGX_SEC_SHADE);
             };

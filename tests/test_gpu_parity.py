@@ -453,6 +453,29 @@ def test_dynamic_sampling_lobes_supersampling_black_background(gx, orc):
                                              "sph_gauss_features", "bandwidth_sharpness", "lobe_axis"))
 
 
+@pytest.mark.parametrize("n,scale", [(1, 12.0), (2, 12.0), (112, 8.0), (113, 8.0), (600, 2.0), (3000, 0.5)])
+@pytest.mark.parametrize("words", [None, 16384])
+def test_window_sums_of_groups_at_one_slot_and_at_many(gx, n, scale, words):
+    """A replay's groups of lanes add to a window's sums at the same table slot in one trip (one Gaussian that
+    covers the image: all eight of them) or at eight different ones (small Gaussians), with tables around their size
+    of 112: the gradients of the backward that adds every row's share to memory.  Sums of at most some 10^5
+    terms in another order: 2e-5, as for the other replays."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=n, sh_degree=0, seed=31))
+    sc["scales"] = sc["scales"] * scale
+    sc["positions"] = sc["positions"] * 0.4
+    sc["densities"] = sc["densities"] + 0.2
+    cam = scenes.make_camera(0, 1, width=44, height=36)
+    cfg = dict(dt_step=0.004, dynamic_sampling=False, max_prim_slice=4096)
+    dloss = np.random.default_rng(5).normal(size=(44 * 36, 3)).astype(np.float32)
+    _step(f"window sums n={n} scale={scale} words={words}")
+    a = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    b = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=words, stats=False)
+    assert a["stats_bwd"]["hit_pairs"] > 500
+    for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+        cos, rel = gx.cos_rel(b["grads"][k], a["grads"][k])
+        assert cos >= 1 - 1e-9 and rel <= 2e-5, (k, cos, rel)
+
+
 @pytest.mark.parametrize("w,h,half", [(52, 44, True), (321, 307, False), (321, 307, True)])
 def test_backward_in_pieces_equals_recomputation(gx, w, h, half):
     """The record of a tile cut into pieces that are replayed side by side, each from the rays' state that the
