@@ -929,18 +929,21 @@ __device__ __forceinline__ void accumulate_samples(HitSetup hs, float4 col, floa
 // Four samples of the recurrence: their powers, and for each the rays for which it lies inside the cut-off.  The rays of a
 // trip walk lists of one order and so are at similar depths: for many a block of four no ray has a sample, and then its
 // exponentials and sums are left out: 23 % of the backward's blocks at 1 M Gaussians 800x800 (5.27 -> 5.07 ms), 58 % at 3 M
-// 1237x822 (10.1 -> 8.4 ms).  Where tiles are light and few a wavefront has its SIMD to itself and waits for the branch:
+// 1237x822 (10.1 -> 8.4 ms).  The others run for the rays that have a sample in them only (`any`): the same instructions, and
+// less power, which is what the clock of a card under this load depends on (1 M 800x800 5.03 -> 4.86 ms).
+// Where tiles are light and few a wavefront has its SIMD to itself and waits for the branch:
 // 4 k Gaussians 128x128 0.142 -> 0.161 ms, 100 k 400x400 0.567 -> 0.590, 300 k 440x440 1.47 -> 1.51 (the replay of lists
 // alone the same); up to 3 000 tiles other scenes gain as much as these lose (3 M 256x256 2.32 -> 2.04, 1 M 440x440 2.75 -> 2.55), so
 // one form serves all.  In the forward, whose walks have two chunks and more rays per trip, it is 9 and 30 % of the blocks, and
-// the branches cost more than that (3 M 1920x1080: 17.4 -> 17.7 ms).
+// the branches cost more than that (3 M 1920x1080: 17.4 -> 17.7 ms; masks without the branches 16.9 -> 17.3).
 #define RGX_SAMPLE_BLOCK 4
 struct SampleBlock {
     float power[RGX_SAMPLE_BLOCK];
     uint64_t in[RGX_SAMPLE_BLOCK];
-    __device__ __forceinline__ bool step(HitSetup &h, float cut)
+    uint64_t any; // the rays with a sample in the block
+    __device__ __forceinline__ void step(HitSetup &h, float cut)
     {
-        uint64_t any = 0;
+        any = 0;
 #pragma unroll
         for (int k = 0; k < RGX_SAMPLE_BLOCK; ++k) {
             power[k] = h.power;
@@ -949,7 +952,6 @@ struct SampleBlock {
             h.power += h.inc;
             h.inc += h.inc_st;
         }
-        return any != 0;
     }
 };
 
@@ -3153,6 +3155,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
         g = mk3(P.dloss[3 * ray], P.dloss[3 * ray + 1], P.dloss[3 * ray + 2]);
         D = dot3(g, mk3(P.fwd_colors[3 * ray], P.fwd_colors[3 * ray + 1], P.fwd_colors[3 * ray + 2]));
     }
+    const bool any_odd = REPLAY && __any(!(fabsf(g.x) < INFINITY && fabsf(g.y) < INFINITY && fabsf(g.z) < INFINITY));
 
     // one slab iteration; `drive(need, tlo, thi, p0, ov, found, searched_to, body_a, mid, body_b)` supplies the hit lists
     auto iteration = [&](auto drive) {
@@ -3163,7 +3166,8 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
         float found = -1.0f, searched_to = 0.f;
         RGX_SEC(cn, RGX_SEC_TOP);
         if (__any(need || (R.active && R.searching))) {
-            const float dt = R.dt, tbuffer = R.tbuffer;
+            // (a ray that is not marching may be at no finite place)
+            const float dt = R.dt, tbuffer = need ? R.tbuffer : 0.0f;
             // (1) s_k and g.c~_k  -> PA, PB
             float PA[RGX_BUFFER_SIZE], PB[RGX_BUFFER_SIZE];
 #pragma unroll
@@ -3275,27 +3279,36 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 constexpr int GROUP = decltype(which)::group; // lanes that share this trip's entry
                 static_assert(!REPLAY || GROUP == 8, "a replay walks by half rows");
                 RGX_SEC(cn, RGX_SEC_WALK);
+                const uint64_t bal = __ballot(hit);
+                GroupAdd add;
                 float out[RGX_NSUM];
+                // In a replay all lanes go through the trip, those without a hit with a Gaussian of no extent (k = 0: no sample
+                // is inside its cut-off, and its whitened frame is zero): their sums come out as zeros, and neither those
+                // nor a branch have to be made for them (3 M 1237x822 7.56 -> 7.44 ms, 4 k 128x128 0.161 -> 0.157).
+                // (Where dL/dC is no number, zero times that is not zero: any_odd.)
+                if constexpr (!REPLAY) {
 #pragma unroll
-                for (int c = 0; c < RGX_NSUM; ++c) out[c] = 0.f;
+                    for (int c = 0; c < RGX_NSUM; ++c) out[c] = 0.f;
+                }
                 const int32_t pid = e.pid;
-                if (hit) {
+                if (REPLAY || hit) {
                     const float4 col = e.colour(), e5 = e.position();
                     f3 U, V, W, inv;
                     float k;
                     e.frame(U, V, W, inv, k);
+                    if constexpr (REPLAY) k = hit ? k : 0.0f;
                     const float rho = col.w;
                     const float dcg = dot3(mk3(col.x, col.y, col.z), g) * __builtin_amdgcn_rcpf(rho);
                     // the forward's sample recurrence (the mask is the one the forward blended with)
                     HitSetup hs = hit_setup(U, V, W, inv, k, e5, dir, rdt0, dt);
                     const f3 Mx0 = hs.Mx0, Md = hs.Md;
                     const float cut0 = hs.cut, cut1 = use_second ? cut0 : -1.0f; // (the second chunk's gate is in its cut-off)
-                    const uint64_t lanes = __builtin_amdgcn_read_exec();
                     float s0 = 0.f, s1 = 0.f, s2 = 0.f, gc = 0.f;
 #pragma unroll
                     for (int b = 0; b < RGX_BUFFER_SIZE; b += RGX_SAMPLE_BLOCK) {
                         SampleBlock S;
-                        if (!S.step(hs, b < RGX_CHUNK_SIZE ? cut0 : cut1)) continue;
+                        S.step(hs, b < RGX_CHUNK_SIZE ? cut0 : cut1);
+                        if (!__builtin_amdgcn_inverse_ballot_w64(S.any)) continue;
 #pragma unroll
                         for (int j = 0; j < RGX_SAMPLE_BLOCK; ++j) {
                             const int i = b + j;
@@ -3308,9 +3321,10 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                                 "v_fmac_f32_e32 %[s2], %[uu], %[y]\n\tv_fmac_f32_e32 %[gc], %[a], %[w]\n\ts_mov_b64 exec, %[l]"
                                 : [s0] "+&v"(s0), [s1] "+&v"(s1), [s2] "+&v"(s2), [gc] "+&v"(gc)
                                 : [in] "s"(S.in[j]), [y] "v"(y), [a] "v"(PA[i]), [w] "v"(wd), [u] "i"(__builtin_bit_cast(uint32_t, u)),
-                                  [uu] "i"(__builtin_bit_cast(uint32_t, u * u)), [l] "s"(lanes));
+                                  [uu] "i"(__builtin_bit_cast(uint32_t, u * u)), [l] "s"(S.any));
                         }
                     }
+                    if constexpr (REPLAY) add.begin(s_acc, s_mark, e.slot, live && ((bal >> (lane & ~7)) & 0xffull) != 0);
                     // moments -> sums in the whitened frame.  (Mx)_k = Mxc + u_k dt Md, Mxc at the slab centre (u = 0)
                     const f3 Mxc = Mx0 + Md * (15.5f * dt);
                     const float m1 = s1 * dt, m2 = s2 * (dt * dt);
@@ -3319,6 +3333,10 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                     const float gcol = gc * rho;
                     out[0] = s0;
                     out[1] = g.x * gcol; out[2] = g.y * gcol; out[3] = g.z * gcol;
+                    if (REPLAY && __builtin_expect(any_odd, 0)) {
+#pragma unroll
+                        for (int c = 1; c < 4; ++c) out[c] = hit ? out[c] : 0.f;
+                    }
                     out[4] = B.x; out[5] = B.y; out[6] = B.z;
                     out[7] = fmaf(Mxc.x, B.x, Md.x * E.x);
                     out[8] = fmaf(Mxc.y, B.y, Md.y * E.y);
@@ -3328,11 +3346,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                     out[12] = fmaf(Mxc.y, B.z, Md.y * E.z);
                 }
                 // summed over the group's rays; one lane per group carries the sums on
-                const uint64_t bal = __ballot(hit);
                 if constexpr (REPLAY) {
-                    GroupAdd add;
-                    add.begin(s_acc, s_mark, e.slot, live && ((bal >> (lane & ~7)) & 0xffull) != 0);
-                    __builtin_amdgcn_sched_barrier(0); // (what begin() asks LDS for arrives behind the sums)
                     float r[7];
                     group_sums_split(out, r);
                     add.end(s_acc, r, e.slot);

@@ -476,6 +476,47 @@ def test_window_sums_of_groups_at_one_slot_and_at_many(gx, n, scale, words):
         assert cos >= 1 - 1e-9 and rel <= 2e-5, (k, cos, rel)
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("words", [None, 16384])
+def test_a_loss_gradient_that_is_no_number_stays_with_the_gaussians_its_ray_hits(gx, bad, words):
+    """dL/dC of one ray is not a number: the Gaussians that this ray does not hit keep their gradients."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=4096, sh_degree=0, seed=31))
+    cam = scenes.make_camera(0, 1, width=64, height=64)
+    cfg = dict(dt_step=0.004, dynamic_sampling=False, max_prim_slice=4096)
+    dloss = np.random.default_rng(5).normal(size=(64 * 64, 3)).astype(np.float32)
+    ray = 30 * 64 + 33
+    only = np.zeros_like(dloss)
+    only[ray] = 1.0
+    _step(f"odd loss {bad} words={words}")
+    hit = np.abs(gx.gpu_render(sc, cam, cfg, want_grad=only, record_hits=False)["grads"]["color_features"]).sum((1, 2)) > 0
+    dloss[ray] = 0.0
+    a = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    dloss[ray] = bad
+    b = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=words, stats=False)
+    assert 1 <= hit.sum() < 400
+    for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+        assert np.isfinite(b["grads"][k][~hit]).all(), k
+        cos, rel = gx.cos_rel(b["grads"][k][~hit], a["grads"][k][~hit])
+        assert cos >= 1 - 1e-9 and rel <= 2e-5, (k, cos, rel)
+
+
+def test_rays_beside_the_scene_leave_its_gradients_alone(gx):
+    """Rays along an axis that pass the scene's box stand at no finite place; they share lane groups with rays that hit."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=300, sh_degree=0, seed=31))
+    sc["positions"] = sc["positions"] * np.array([0.3, 0.03, 0.3], np.float32) + np.array([0.0, 0.12, 0.0], np.float32)
+    sc["scales"] = sc["scales"] * 0.3
+    cam = scenes.look_at_camera((3.0, 0.0, 0.0), fov_x_deg=30, width=33, height=33)      # the middle column: y = 0 throughout
+    cfg = dict(dt_step=0.004, dynamic_sampling=False, max_prim_slice=4096)
+    dloss = np.random.default_rng(5).normal(size=(33 * 33, 3)).astype(np.float32)
+    _step("rays beside the scene")
+    a = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    b = gx.gpu_render(sc, cam, cfg, want_grad=dloss, stats=False)
+    for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+        assert np.isfinite(b["grads"][k]).all() and np.abs(b["grads"][k]).sum() > 0, k
+        cos, rel = gx.cos_rel(b["grads"][k], a["grads"][k])
+        assert cos >= 1 - 1e-9 and rel <= 2e-5, (k, cos, rel)
+
+
 @pytest.mark.parametrize("w,h,half", [(52, 44, True), (321, 307, False), (321, 307, True)])
 def test_backward_in_pieces_equals_recomputation(gx, w, h, half):
     """The record of a tile cut into pieces that are replayed side by side, each from the rays' state that the
