@@ -1065,16 +1065,18 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
 // classes/point_cloud.py:252).  As there: points sorted along a Morton curve, boxes of consecutive
 // sorted points, boxes that cannot hold one of the three nearest are left out (the pruning is exact,
 // so the result is the exact 3-NN mean whatever the order and the box size).
-// Here a wavefront searches for the 64 consecutive points of the curve that it owns, together: three
+// Here a wavefront searches for the consecutive points of the curve that it owns, together: three
 // levels of boxes (16 points, 64 leaves, 64 boxes), of which each lane tests one child against the
 // bounds of the wavefront's points and the largest distance any of them still has to beat; the leaves that
-// are left are tested by every lane for its own point, and a leaf that some lane needs is read once, as
-// scalars, and met by all lanes in straight-line code.  What bounds it is the issue of those distance
-// computations (12 instructions per point and leaf point); one lane searching on its own through boxes of
-// 256 points made every lane of a wavefront wait for the scans of all others.  The whole call, sort and boxes included,
-// took 4.6-5.5 ms for 1 M points of a ball and 2.2-3.1 ms for 54 k of a heavy-tailed cloud (eight draws of each); it takes
-// 0.53-0.57 and 0.20-0.34 ms.  This search is 0.46 ms of the former; of the latter it is what the draws differ in (0.26 of 0.34
-// ms in one): the launch lasts as long as the wavefront whose points lie farthest apart.
+// are left are tested by every lane for its own point, and a leaf that some lane needs is read once and met by
+// all lanes in straight-line code.  One lane searching on its own through boxes of
+// 256 points made every lane of a wavefront wait for the scans of all others.  A wavefront owns 64 points, or 32, 16 or 8 whose
+// 2, 4 or 8 lanes each meet their share of a leaf (knn_lanes): a large cloud is bound by the issue of the distance
+// computations (12 instructions per point and leaf point, with 64 points and the leaf's points as scalars), a small one by its
+// longest wavefront, which gets shorter with the stretch of the curve whose bounds it has to search.
+// The whole call, sort and boxes included, us, with 64 points a wavefront / with as many as knn_lanes says:
+//     heavy-tailed cloud of 1 000, 5 000, 20 000, 54 k, 150 k, 300 k, 1 M, 3 M  61/39 122/65 221/107 269/138 319/207 377/340 867/719 1 610
+//     ball or cube of 20 000, 54 k, 300 k, 1 M                                154/104 177/134 269/249 559/560
 // Distances are (dx*dx + dy*dy) + dz*dz without contraction; rounding is monotone, so the distance to a
 // box that holds a point, computed the same way, is never larger than the distance to the point.
 #define RGX_KNN_LEAF 16
@@ -1153,24 +1155,32 @@ __device__ __forceinline__ float knn_box_dist(f3 lo, f3 hi, f3 qlo, f3 qhi)
     return (dx * dx + dy * dy) + dz * dz;
 }
 
-// simple_knn.cu:137-184 updateKBest<3>, boxMeanDist
+// Lanes per point.  The lines lie where the larger number stops gaining for either kind of cloud (us with 8 / 4 / 2 / 1 lanes a
+// point: 54 k heavy-tailed 138 / 151 / 168 / 269, ball 134 / 132 / 139 / 177; 150 k heavy-tailed 225 / 207 / 253 / 319; 300 k 341 / 350 /
+// 340 / 377, ball 300 / 249 / 248 / 269; 1 M 925 / 693 / 719 / 867, ball 782 / 602 / 560 / 559; 3 M 2 739 / 1 965 / 1 705 / 1 610).
+static inline int knn_lanes(int64_t n) { return n <= 1 << 16 ? 8 : n <= 1 << 18 ? 4 : n <= 1 << 20 ? 2 : 1; }
+
+// simple_knn.cu:137-184 updateKBest<3>, boxMeanDist.  C: lanes per point.
+template <int C>
 __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, const uint32_t *__restrict__ order, int64_t n,
                                               const float4 *__restrict__ leaves, const float4 *__restrict__ boxes, int64_t nb,
                                               const int32_t *__restrict__ supers_enc, int64_t ns, float *__restrict__ out)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i - lane >= n) return; // whole wave
+    constexpr int P = 64 / C, EACH = RGX_KNN_LEAF / C; // points of a wavefront; points of a leaf that a lane meets
+    const int lane = threadIdx.x & 63, copy = lane / P;
+    const int64_t first = __builtin_amdgcn_readfirstlane((int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6)) * (int64_t)P;
+    if (first >= n) return; // whole wave
+    const int64_t i = first + (lane & (P - 1));
     const float4 p4 = pts[i]; // (the array is padded to whole boxes)
     const f3 p = mk3(p4.x, p4.y, p4.z);
     const bool act = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
     // The wavefront's points as RGX_KNN_SEGS runs of the curve, cut where it jumps farthest: the bounds of a run that
     // spans such a jump would meet most of the cloud (one such wavefront was the whole launch's time).
-    uint64_t cuts = 0;
+    uint64_t cuts = 0; // over the first P lanes
     {
         const f3 prev = mk3(__shfl_up(p.x, 1), __shfl_up(p.y, 1), __shfl_up(p.z, 1));
         const f3 step = p - prev;
-        float gap = lane > 0 ? dot3(step, step) : -1.f;
+        float gap = lane > 0 && lane < P ? dot3(step, step) : -1.f;
         if (!(gap < INFINITY)) gap = -1.f;
         for (int k = 1; k < RGX_KNN_SEGS; ++k) {
             const float g = wave_max_all(gap);
@@ -1180,7 +1190,7 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
             if (lane == __builtin_ctzll(at)) gap = -1.f;
         }
     }
-    const int seg = __popcll(cuts & (~0ull >> (63 - lane)));
+    const int seg = __popcll(cuts & (~0ull >> (63 - (lane & (P - 1)))));
     f3 slo[RGX_KNN_SEGS], shi[RGX_KNN_SEGS];
     float reach[RGX_KNN_SEGS]; // the largest distance a point of the run still has to beat
     for (int k = 0; k < RGX_KNN_SEGS; ++k) {
@@ -1188,30 +1198,42 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
         slo[k] = mk3(wave_min_all(in ? p.x : INFINITY), wave_min_all(in ? p.y : INFINITY), wave_min_all(in ? p.z : INFINITY));
         shi[k] = mk3(wave_max_all(in ? p.x : -INFINITY), wave_max_all(in ? p.y : -INFINITY), wave_max_all(in ? p.z : -INFINITY));
     }
-    float b0 = FLT_MAX, b1 = FLT_MAX, b2 = FLT_MAX; // the three smallest so far, ascending
+    float b0 = FLT_MAX, b1 = FLT_MAX, b2 = FLT_MAX; // the three smallest that this lane has met, ascending
+    auto put = [](float &c0, float &c1, float &c2, float d) {
+        c2 = __builtin_amdgcn_fmed3f(c1, c2, d);
+        c1 = __builtin_amdgcn_fmed3f(c0, c1, d);
+        c0 = fminf(c0, d);
+    };
     auto meet = [&](int l, auto own) { // all points of leaf l (the same in every lane)
         l = __builtin_amdgcn_readfirstlane(l);
-        const float4 *q = pts + (int64_t)l * RGX_KNN_LEAF;
+        const float4 *q = pts + (int64_t)l * RGX_KNN_LEAF + (C > 1 ? copy * EACH : 0);
 #pragma unroll
-        for (int k = 0; k < RGX_KNN_LEAF; ++k) {
+        for (int k = 0; k < EACH; ++k) {
             const float dx = q[k].x - p.x, dy = q[k].y - p.y, dz = q[k].z - p.z;
             float d = (dx * dx + dy * dy) + dz * dz;
-            if constexpr (decltype(own)::value) d = (int64_t)l * RGX_KNN_LEAF + k == i ? FLT_MAX : d;
-            b2 = __builtin_amdgcn_fmed3f(b1, b2, d);
-            b1 = __builtin_amdgcn_fmed3f(b0, b1, d);
-            b0 = fminf(b0, d);
+            if constexpr (decltype(own)::value) d = (int64_t)l * RGX_KNN_LEAF + copy * EACH + k == i ? FLT_MAX : d;
+            put(b0, b1, b2, d);
+        }
+    };
+    float t0, t1, worst; // the three smallest that the point's lanes have met
+    auto measure = [&]() {
+        t0 = b0;
+        t1 = b1;
+        worst = b2;
+        for (int o = P; o < 64; o <<= 1) {
+            const float o0 = __shfl_xor(t0, o), o1 = __shfl_xor(t1, o), o2 = __shfl_xor(worst, o);
+            put(t0, t1, worst, o0);
+            put(t0, t1, worst, o1);
+            put(t0, t1, worst, o2);
         }
     };
     // the points nearby on the curve first: they leave little for the boxes
-    const int leaf0 = __builtin_amdgcn_readfirstlane((int)((i - lane) / RGX_KNN_LEAF));
-    for (int l = leaf0; l < leaf0 + 64 / RGX_KNN_LEAF; ++l) meet(l, std::true_type{});
+    const int leaf0 = (int)(first / RGX_KNN_LEAF), leaf1 = (int)((first + P - 1) / RGX_KNN_LEAF) + 1;
+    for (int l = leaf0; l < leaf1; ++l) meet(l, std::true_type{});
     const int n_leaves = (int)(nb * RGX_KNN_FAN);
-    const int done0 = std::max(leaf0 - RGX_KNN_NEAR, 0), done1 = std::min(leaf0 + 64 / RGX_KNN_LEAF + RGX_KNN_NEAR, n_leaves);
+    const int done0 = std::max(leaf0 - RGX_KNN_NEAR, 0), done1 = std::min(leaf1 + RGX_KNN_NEAR, n_leaves);
     for (int l = done0; l < leaf0; ++l) meet(l, std::false_type{});
-    for (int l = leaf0 + 64 / RGX_KNN_LEAF; l < done1; ++l) meet(l, std::false_type{});
-    auto measure = [&]() {
-        for (int k = 0; k < RGX_KNN_SEGS; ++k) reach[k] = wave_max_all(act && seg == k ? b2 : -1.f);
-    };
+    for (int l = leaf1; l < done1; ++l) meet(l, std::false_type{});
     measure();
     auto open = [&](f3 lo, f3 hi) { // is the box within some run's reach?
         bool o = false;
@@ -1239,13 +1261,13 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
                     const int t = __builtin_ctzll(ml);
                     auto at = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), t)); };
                     const float d = knn_box_dist(mk3(at(lo.x), at(lo.y), at(lo.z)), mk3(at(hi.x), at(hi.y), at(hi.z)), p, p);
-                    if (__any(act && d < b2)) meet(l0 + t, std::false_type{});
+                    if (__any(act && d < worst)) meet(l0 + t, std::false_type{});
                 }
                 if (some) measure();
             }
         }
     }
-    if (i < n) out[order[i]] = act ? ((b0 + b1) + b2) / 3.0f : INFINITY;
+    if (i < n && copy == 0) out[order[i]] = act ? ((t0 + t1) + worst) / 3.0f : INFINITY;
 }
 
 struct KnnLayout {
@@ -1299,7 +1321,17 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + K.m.hist), s);
     if (r < 0) return r;
     hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)K.nb), dim3(RGX_KNN_BOX), 0, s, pos, v0, n, pts, leaves, boxes, supers);
-    hipLaunchKernelGGL(k_knn3, grid_for(n, 256), dim3(256), 0, s, pts, v0, n, leaves, boxes, K.nb, supers, K.ns, mean_dist2);
+    const auto search = [&](auto lanes) {
+        constexpr int C = decltype(lanes)::value;
+        hipLaunchKernelGGL(k_knn3<C>, grid_for(n * C, 256), dim3(256), 0, s, pts, v0, n, leaves, boxes, K.nb, supers, K.ns, mean_dist2);
+    };
+    switch (knn_lanes(n)) {
+    case 8: search(std::integral_constant<int, 8>{}); break;
+    case 4: search(std::integral_constant<int, 4>{}); break;
+    case 2: search(std::integral_constant<int, 2>{}); break;
+    default: search(std::integral_constant<int, 1>{});
+    }
     RGX_LAUNCH_CHECK();
     return RGX_OK;
 }
+        for (int k = 0; k < RGX_KNN_SEGS; ++k) reach[k] = wave_max_all(act && seg == k ? worst : -1.f);

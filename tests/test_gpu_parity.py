@@ -896,6 +896,23 @@ def test_dist2_knn3_at_the_sizes_of_its_boxes(gx, orc, n):
     np.testing.assert_array_equal(got.view(np.uint32), orc.dist2_knn3(p).view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [65_535, 65_536, 65_537, 262_143, 262_144, 262_145, 1_048_576, 1_048_577])
+def test_dist2_knn3_with_any_number_of_lanes_per_point(gx, n):
+    """Either side of the sizes at which the search changes its number of lanes per point: the first 9 001 points, with a nan and an
+    outlier among them, are far from all others, so their distances are those of the small cloud alone, bit for bit."""
+    from raygaussx_amd.simple_knn import distCUDA2
+    rng = np.random.default_rng(n)
+    near = rng.normal(size=(9001, 3)).astype(np.float32)
+    near[5] = np.nan
+    near[17] = (40.0, 0.0, 0.0)
+    far = (rng.normal(size=(n - 9001, 3)) + np.array([1000.0, 0.0, 0.0])).astype(np.float32)
+    _step(f"knn lanes n={n}")
+    small = distCUDA2(torch.from_numpy(near).to(gx.DEV)).cpu().numpy()
+    got = distCUDA2(torch.from_numpy(np.concatenate([near, far])).to(gx.DEV)).cpu().numpy()
+    np.testing.assert_array_equal(got[:9001], small)
+    assert np.isfinite(got[9001:]).all()
+
+
 @pytest.mark.parametrize("kind", ["outliers", "two clumps", "nan", "inf", "nan and inf", "all nan", "huge"])
 def test_dist2_knn3_of_clouds_that_the_curve_does_not_sort(gx, orc, kind):
     """A few far points leave nearly all the others in one or two cells of the Morton grid, in whose order they say nothing of
