@@ -218,33 +218,19 @@ __global__ __launch_bounds__(256) void k_rs_scan_rows(uint32_t *__restrict__ his
     if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
-template <typename K>
-__global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
-                                                               K *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n,
-                                                               int shift, const uint32_t *__restrict__ hist, int nblocks,
-                                                               const uint32_t *__restrict__ totals)
+// One tile's keys to their places.  digit_base: where the keys of digit threadIdx.x begin in the output; before: how many of
+// them other tiles put in front of this one's.  put(place, key, value) writes.
+template <typename K, int ITEMS, typename Put>
+__device__ __forceinline__ void rs_scatter_tile(const K *__restrict__ kin, const uint32_t *__restrict__ vin, int64_t n, int shift,
+                                                uint32_t digit_base, uint32_t before, uint32_t (&cnt)[4][256], uint32_t (&wave_total)[4], Put put)
 {
-    static_assert(RGX_RS_THREADS == 256, "one thread per digit");
-    __shared__ uint32_t cnt[4][256];
-    __shared__ uint32_t wave_total[4];
+    constexpr int TILE = RGX_RS_THREADS * ITEMS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int w = 0; w < 4; ++w) cnt[w][threadIdx.x] = 0;
-    // digit_base: exclusive scan of the digits' totals, thread d for digit d
-    const uint32_t total = totals[threadIdx.x];
-    uint32_t incl = total;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t t = __shfl_up(incl, o);
-        if (lane >= o) incl += t;
-    }
-    if (lane == 63) wave_total[wave] = incl;
-    __syncthreads();
-    uint32_t digit_base = incl - total;
-    for (int w = 0; w < wave; ++w) digit_base += wave_total[w];
-    // wave w owns the contiguous 512 keys [base + 512 w, +512), 64 per round
-    const int64_t base = (int64_t)blockIdx.x * RGX_RS_TILE + (int64_t)wave * (64 * RGX_RS_ITEMS);
-    K key[RGX_RS_ITEMS];
-    uint32_t val[RGX_RS_ITEMS];
-    for (int r = 0; r < RGX_RS_ITEMS; ++r) {
+    // wave w owns the contiguous 64 ITEMS keys from base, 64 per round
+    const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)wave * (64 * ITEMS);
+    K key[ITEMS];
+    uint32_t val[ITEMS];
+    for (int r = 0; r < ITEMS; ++r) {
         const int64_t i = base + r * 64 + lane;
         key[r] = 0;
         val[r] = 0;
@@ -260,8 +246,8 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restri
     // 64 lanes writing to as many streams.  local: where a (wave, digit) run starts in the tile's order;
     // delta[d]: output position minus position in the tile's order, for digit d.
     __shared__ uint32_t delta[256];
-    __shared__ K lkey[RGX_RS_TILE];
-    __shared__ uint32_t lval[RGX_RS_TILE];
+    __shared__ K lkey[TILE];
+    __shared__ uint32_t lval[TILE];
     {
         const int d = threadIdx.x;
         uint32_t c[4], tile_count = 0;
@@ -276,7 +262,7 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restri
         __syncthreads();
         uint32_t local = upto - tile_count;
         for (int w = 0; w < wave; ++w) local += wave_total[w];
-        delta[d] = digit_base + hist[(size_t)d * nblocks + blockIdx.x] - local;
+        delta[d] = digit_base + before - local;
         for (int w = 0; w < 4; ++w) {
             cnt[w][d] = local;
             local += c[w];
@@ -284,7 +270,7 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restri
     }
     __syncthreads();
     volatile uint32_t *cur = cnt[wave];
-    for (int r = 0; r < RGX_RS_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const int64_t i = base + r * 64 + lane;
         const bool valid = i < n;
         const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
@@ -305,14 +291,97 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restri
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    const int64_t tile_base = (int64_t)blockIdx.x * RGX_RS_TILE;
-    const int tile_n = (int)(n - tile_base < RGX_RS_TILE ? n - tile_base : RGX_RS_TILE);
+    const int64_t tile_base = (int64_t)blockIdx.x * TILE;
+    const int tile_n = (int)(n - tile_base < TILE ? n - tile_base : TILE);
     for (int p = threadIdx.x; p < tile_n; p += RGX_RS_THREADS) {
         const K k = lkey[p];
-        const uint32_t out = (uint32_t)p + delta[(uint32_t)(k >> shift) & 255u];
-        kout[out] = k;
-        vout[out] = lval[p];
+        put((uint32_t)p + delta[(uint32_t)(k >> shift) & 255u], k, lval[p]);
     }
+}
+
+// exclusive scan over the 256 threads' values
+__device__ __forceinline__ uint32_t rs_sum_before(uint32_t v, uint32_t (&wave_total)[4])
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t incl = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(incl, o);
+        if (lane >= o) incl += t;
+    }
+    if (lane == 63) wave_total[wave] = incl;
+    __syncthreads();
+    uint32_t sum = incl - v;
+    for (int w = 0; w < wave; ++w) sum += wave_total[w];
+    return sum;
+}
+
+// order: where the last pass leaves the values, or null (then vout as every pass)
+template <typename K>
+__global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                               K *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n,
+                                                               int shift, const uint32_t *__restrict__ hist, int nblocks,
+                                                               const uint32_t *__restrict__ totals, int64_t *__restrict__ order)
+{
+    static_assert(RGX_RS_THREADS == 256, "one thread per digit");
+    __shared__ uint32_t cnt[4][256];
+    __shared__ uint32_t wave_total[4];
+    for (int w = 0; w < 4; ++w) cnt[w][threadIdx.x] = 0;
+    const uint32_t digit_base = rs_sum_before(totals[threadIdx.x], wave_total);
+    rs_scatter_tile<K, RGX_RS_ITEMS>(kin, vin, n, shift, digit_base, hist[(size_t)threadIdx.x * nblocks + blockIdx.x], cnt, wave_total,
+                                     [&](uint32_t at, K k, uint32_t v) {
+                                         if (order) {
+                                             order[at] = (int64_t)v;
+                                         } else {
+                                             kout[at] = k;
+                                             vout[at] = v;
+                                         }
+                                     });
+}
+
+// Fewer keys (rs_short): two launches per pass.  What a pass of three launches takes for them is mostly their latency, some four
+// microseconds each; here the tiles' counts lie row by row, and every block of the scatter sums up the rows before its own
+// and all of them.  Tree over 9 000, 54 k, 100 k, 150 k, 200 k boxes, three launches a pass / two, us: 211/152 228/198 246/213
+// 262/241 271/262 (262 k: 276/274, 500 k: 332/361, the rows are too many then); with 512 keys a tile up to 65 536 and
+// 1 024 beyond (54 k with 1 024 or 2 048 a tile 204 and 225, 150 k with 512 or 2 048 260 and 266).  One launch a pass, the next
+// pass's digits counted by atomic adds as the keys are written: 152, 206, 248, 349, 355, its adds wait for memory one by one.
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_count(const K *__restrict__ keys, int64_t n, int shift, uint32_t *__restrict__ counts)
+{
+    __shared__ uint32_t h[256];
+    h[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int64_t i = ((int64_t)blockIdx.x * ITEMS + r) * RGX_RS_THREADS + threadIdx.x;
+        if (i < n) atomicAdd(&h[(uint32_t)(keys[i] >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    counts[(size_t)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+}
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_pass(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                            K *__restrict__ kout, uint32_t *__restrict__ vout, int64_t n, int shift,
+                                                            const uint32_t *__restrict__ counts, int tiles, int64_t *__restrict__ order)
+{
+    __shared__ uint32_t cnt[4][256];
+    __shared__ uint32_t wave_total[4];
+    for (int w = 0; w < 4; ++w) cnt[w][threadIdx.x] = 0;
+    uint32_t before = 0, total = 0;
+#pragma unroll 16
+    for (int t = 0; t < tiles; ++t) {
+        const uint32_t c = counts[(size_t)t * 256 + threadIdx.x];
+        total += c;
+        before += t < (int)blockIdx.x ? c : 0u;
+    }
+    const uint32_t digit_base = rs_sum_before(total, wave_total);
+    rs_scatter_tile<K, ITEMS>(kin, vin, n, shift, digit_base, before, cnt, wave_total, [&](uint32_t at, K k, uint32_t v) {
+        if (order) {
+            order[at] = (int64_t)v;
+        } else {
+            kout[at] = k;
+            vout[at] = v;
+        }
+    });
 }
 
 // A sort of few keys: all passes in one workgroup, the keys in registers and their new order in LDS.  What the passes
@@ -320,7 +389,6 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_scatter(const K *__restri
 // 181 us, with this 98; over 8 192 185 and 125; with a bitonic network, which moves every key through LDS 78 and 91 times
 // instead of 8, 117 and 177).  Each wavefront has a run
 // of the keys, and ranks 64 at a time as k_rs_scatter does.  The limit is what fits LDS (12 bytes a key, and 16 KB of counters).
-#define RGX_SORT_SMALL 8192
 template <typename K>
 __global__ __launch_bounds__(1024) void k_sort_small(K *__restrict__ keys, uint32_t *__restrict__ vals, int n, int bits)
 {
@@ -412,24 +480,44 @@ __global__ __launch_bounds__(1024) void k_sort_small(K *__restrict__ keys, uint3
     }
 }
 
-// Sorts (k0, v0) by key, stable, with (k1, v1) as the second buffers.
+// the values of a sort in one workgroup, as 64-bit numbers
+__global__ __launch_bounds__(256) void k_order64(const uint32_t *__restrict__ v, int64_t n, int64_t *__restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = (int64_t)v[i];
+}
+
+// Sorts (k0, v0) by key, stable, with (k1, v1) as the second buffers.  hist: rs_hist_words(n).  order: where the values go in the end, or null.
 template <typename K>
-static int radix_sort(K *k0, uint32_t *v0, K *k1, uint32_t *v1, int64_t n, int bits, uint32_t *hist, hipStream_t s)
+static int radix_sort(K *k0, uint32_t *v0, K *k1, uint32_t *v1, int64_t n, int bits, uint32_t *hist, hipStream_t s, int64_t *order = nullptr)
 {
     if (n <= RGX_SORT_SMALL) {
         hipLaunchKernelGGL(k_sort_small<K>, dim3(1), dim3(1024), 0, s, k0, v0, (int)n, bits);
+        if (order) hipLaunchKernelGGL(k_order64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, v0, n, order);
         RGX_LAUNCH_CHECK();
         return 0;
     }
+    const RsShort F = rs_short(n);
     const int nblocks = (int)((n + RGX_RS_TILE - 1) / RGX_RS_TILE);
     K *ki = k0, *ko = k1;
     uint32_t *vi = v0, *vo = v1;
     for (int shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_rs_hist<K>, dim3(nblocks), dim3(RGX_RS_THREADS), 0, s, ki, n, shift, hist, nblocks);
-        uint32_t *totals = hist + (size_t)256 * nblocks;
-        hipLaunchKernelGGL(k_rs_scan_rows, dim3(256), dim3(256), 0, s, hist, nblocks, totals);
-        hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nblocks), dim3(RGX_RS_THREADS), 0, s, ki, vi, ko, vo, n, shift, hist, nblocks,
-                           totals);
+        int64_t *const last = shift + 8 >= bits ? order : nullptr;
+        if (F.tiles) {
+            const auto pass = [&](auto items) {
+                constexpr int ITEMS = decltype(items)::value;
+                hipLaunchKernelGGL((k_rs_count<K, ITEMS>), dim3(F.tiles), dim3(RGX_RS_THREADS), 0, s, ki, n, shift, hist);
+                hipLaunchKernelGGL((k_rs_pass<K, ITEMS>), dim3(F.tiles), dim3(RGX_RS_THREADS), 0, s, ki, vi, ko, vo, n, shift, hist, F.tiles, last);
+            };
+            if (F.tile_bits == 9) pass(std::integral_constant<int, 2>{});
+            else pass(std::integral_constant<int, 4>{});
+        } else {
+            hipLaunchKernelGGL(k_rs_hist<K>, dim3(nblocks), dim3(RGX_RS_THREADS), 0, s, ki, n, shift, hist, nblocks);
+            uint32_t *totals = hist + (size_t)256 * nblocks;
+            hipLaunchKernelGGL(k_rs_scan_rows, dim3(256), dim3(256), 0, s, hist, nblocks, totals);
+            hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nblocks), dim3(RGX_RS_THREADS), 0, s, ki, vi, ko, vo, n, shift, hist, nblocks,
+                               totals, last);
+        }
         K *tk = ki; ki = ko; ko = tk;
         uint32_t *tv = vi; vi = vo; vo = tv;
     }
@@ -836,12 +924,21 @@ extern "C" int rgx_build_order(const void *ws, int64_t n, int32_t *order_out, vo
 __global__ __launch_bounds__(256) void k_pos_minmax(const float *__restrict__ pos, int64_t n, int32_t *mn_enc, int32_t *mx_enc)
 {
     float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        for (int a = 0; a < 3; ++a) {
-            const float v = pos[3 * i + a];
-            b[a] = fminf(b[a], v);
-            b[a + 3] = fmaxf(b[a + 3], v);
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += 4 * step) {
+        float v[4][3];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { // (four points in flight; past the end: the first again)
+            const int64_t j = i + k * step < n ? i + k * step : i;
+            for (int a = 0; a < 3; ++a) v[k][a] = pos[3 * j + a];
         }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            for (int a = 0; a < 3; ++a) {
+                b[a] = fminf(b[a], v[k][a]);
+                b[a + 3] = fmaxf(b[a + 3], v[k][a]);
+            }
+    }
     __shared__ float red[4][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
@@ -856,27 +953,22 @@ __global__ __launch_bounds__(256) void k_pos_minmax(const float *__restrict__ po
     }
 }
 
-__global__ __launch_bounds__(256) void k_morton30(const float *__restrict__ pos, int64_t n, const float *__restrict__ mn,
-                                                  const float *__restrict__ mx, uint32_t *__restrict__ keys,
+__global__ __launch_bounds__(256) void k_morton30(const float *__restrict__ pos, int64_t n, const int32_t *__restrict__ mn_enc,
+                                                  const int32_t *__restrict__ mx_enc, uint32_t *__restrict__ keys,
                                                   uint32_t *__restrict__ vals, int64_t *__restrict__ codes)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     uint32_t code = 0;
     for (int a = 0; a < 3; ++a) {
-        const float scale = 1023.0f / ((mx[a] - mn[a]) + 1e-9f); // reordering_utils.py:73
-        const int32_t q = (int32_t)((pos[3 * i + a] - mn[a]) * scale); // .to(torch.int32): truncation
+        const float mn = dec_f(mn_enc[a]), mx = dec_f(mx_enc[a]);
+        const float scale = 1023.0f / ((mx - mn) + 1e-9f); // reordering_utils.py:73
+        const int32_t q = (int32_t)((pos[3 * i + a] - mn) * scale); // .to(torch.int32): truncation
         for (int b = 0; b < 10; ++b) code |= (uint32_t)((q >> b) & 1) << (3 * b + a); // reordering_utils.py:98-102
     }
     keys[i] = code;
     vals[i] = (uint32_t)i;
     if (codes) codes[i] = (int64_t)code;
-}
-
-__global__ __launch_bounds__(256) void k_order64(const uint32_t *__restrict__ v, int64_t n, int64_t *__restrict__ out)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (int64_t)v[i];
 }
 
 struct MortonLayout {
@@ -885,14 +977,14 @@ struct MortonLayout {
 static inline MortonLayout morton_layout(int64_t n)
 {
     MortonLayout L;
-    const size_t nn = (size_t)(n > 0 ? n : 1), nblocks = (nn + RGX_RS_TILE - 1) / RGX_RS_TILE;
+    const size_t nn = (size_t)(n > 0 ? n : 1);
     size_t off = 0;
     L.enc = off;   off = rgx_align_up(off + 8 * sizeof(int32_t), 256);
     L.keys0 = off; off = rgx_align_up(off + nn * 4, 256);
     L.keys1 = off; off = rgx_align_up(off + nn * 4, 256);
     L.vals0 = off; off = rgx_align_up(off + nn * 4, 256);
     L.vals1 = off; off = rgx_align_up(off + nn * 4, 256);
-    L.hist = off;  off = rgx_align_up(off + 256 * (nblocks + 1) * 4, 256);
+    L.hist = off;  off = rgx_align_up(off + rs_hist_words((int64_t)nn) * 4, 256);
     L.total = off;
     return L;
 }
@@ -919,14 +1011,11 @@ extern "C" int rgx_morton_order(const float *pos, int64_t n, int64_t *codes, int
     uint32_t *v0 = (uint32_t *)(w + L.vals0), *v1 = (uint32_t *)(w + L.vals1);
     hipLaunchKernelGGL(k_init_enc, dim3(1), dim3(64), 0, s, mn, mx);
     hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 256), dim3(256), 0, s, pos, n, mn, mx);
-    hipLaunchKernelGGL(k_decode_enc, dim3(1), dim3(64), 0, s, mn, mx);
-    hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, (const float *)mn, (const float *)mx, k0, v0, codes);
+    hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, mn, mx, k0, v0, codes);
     RGX_LAUNCH_CHECK();
     if (order) {
-        const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + L.hist), s);
+        const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + L.hist), s, order);
         if (r < 0) return r;
-        hipLaunchKernelGGL(k_order64, grid_for(n, 256), dim3(256), 0, s, v0, n, order);
-        RGX_LAUNCH_CHECK();
     }
     return RGX_OK;
 }
@@ -1226,6 +1315,7 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
             put(t0, t1, worst, o1);
             put(t0, t1, worst, o2);
         }
+        for (int k = 0; k < RGX_KNN_SEGS; ++k) reach[k] = wave_max_all(act && seg == k ? worst : -1.f);
     };
     // the points nearby on the curve first: they leave little for the boxes
     const int leaf0 = (int)(first / RGX_KNN_LEAF), leaf1 = (int)((first + P - 1) / RGX_KNN_LEAF) + 1;
@@ -1314,9 +1404,7 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     int32_t *supers = (int32_t *)(w + K.supers);
     hipLaunchKernelGGL(k_knn_begin, dim3(1), dim3(256), 0, s, mn, mx, supers, K.ns);
     hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 256), dim3(256), 0, s, pos, n, mn, mx);
-    hipLaunchKernelGGL(k_decode_enc, dim3(1), dim3(64), 0, s, mn, mx);
-    hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, (const float *)mn, (const float *)mx, k0, v0,
-                       (int64_t *)nullptr);
+    hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, mn, mx, k0, v0, (int64_t *)nullptr);
     RGX_LAUNCH_CHECK();
     const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + K.m.hist), s);
     if (r < 0) return r;
@@ -1334,4 +1422,3 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     RGX_LAUNCH_CHECK();
     return RGX_OK;
 }
-        for (int k = 0; k < RGX_KNN_SEGS; ++k) reach[k] = wave_max_all(act && seg == k ? worst : -1.f);

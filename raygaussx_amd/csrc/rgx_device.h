@@ -149,11 +149,32 @@ struct WsLayout {
 
 static inline size_t rgx_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+// Sorts of more keys than one workgroup takes (RGX_SORT_SMALL) and at most RGX_SORT_SHORT take two launches per pass
+// (k_rs_pass), in tiles of 2^tile_bits keys; tiles = 0: other sizes.
+#define RGX_SORT_SMALL 8192
+#define RGX_SORT_SHORT 196608
+struct RsShort {
+    int tiles = 0, tile_bits = 0;
+};
+static inline RsShort rs_short(int64_t n)
+{
+    RsShort F;
+    if (n <= RGX_SORT_SMALL || n > RGX_SORT_SHORT) return F;
+    F.tile_bits = n <= 65536 ? 9 : 10;
+    F.tiles = (int)((n + (1 << F.tile_bits) - 1) >> F.tile_bits);
+    return F;
+}
+// words of digit counts that a sort of n keys works with
+static inline size_t rs_hist_words(int64_t n)
+{
+    const size_t words = (size_t)256 * rs_short(n).tiles;
+    return words ? words : 256 * (((size_t)n + RGX_RS_TILE - 1) / RGX_RS_TILE + 1);
+}
+
 static inline WsLayout rgx_ws_layout(int64_t n)
 {
     WsLayout L;
     const size_t nn = (size_t)(n > 0 ? n : 1);
-    const size_t nblocks = (nn + RGX_RS_TILE - 1) / RGX_RS_TILE;
     size_t off = 0;
     L.header = off; off = rgx_align_up(off + sizeof(WsHeader), 256);
     L.aabb = off;   off = rgx_align_up(off + nn * 6 * sizeof(float), 256);
@@ -165,7 +186,7 @@ static inline WsLayout rgx_ws_layout(int64_t n)
     L.parent = off; off = rgx_align_up(off + (2 * nn) * sizeof(int32_t), 256);
     L.right = off;  off = rgx_align_up(off + nn * sizeof(int32_t), 256);
     L.flags = off;  off = rgx_align_up(off + nn * sizeof(int32_t), 256);
-    L.hist = off;   off = rgx_align_up(off + 256 * (nblocks + 1) * sizeof(uint32_t), 256);
+    L.hist = off;   off = rgx_align_up(off + rs_hist_words((int64_t)nn) * sizeof(uint32_t), 256);
     L.total = off;
     return L;
 }

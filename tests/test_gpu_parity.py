@@ -730,6 +730,12 @@ def test_orders_of_few_keys(gx, orc, n):
     np.testing.assert_array_equal(order, np.argsort(code, kind="stable"))
 
 
+@pytest.mark.parametrize("n", [8_704, 65_536, 65_537, 196_608, 196_609])
+def test_orders_of_more_keys(gx, orc, n):
+    """Either side of the sizes at which the sort changes its tiles and its launches per pass."""
+    test_orders_of_few_keys(gx, orc, n)
+
+
 def test_reorder_tensors_is_the_per_tensor_gather(gx):
     """PointCloud.reorder_zordercurve's gathers (classes/point_cloud.py:1031-1044) in one launch:
     every tensor equals numpy's `t[index]`, for the parameter shapes of a point cloud with Adam
