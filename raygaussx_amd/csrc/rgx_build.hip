@@ -58,12 +58,23 @@ __global__ void k_refit_begin(WsHeader *h, int64_t n)
 __device__ __forceinline__ bool gate_closed(const int32_t *gate) { return gate != nullptr && *gate == 0; }
 
 // k-sigma AABB of a rotated ellipsoid (optix_utils.py:49-77), canonical arithmetic.
-__global__ __launch_bounds__(256) void k_aabb(const float *__restrict__ pos, const float *__restrict__ scale,
+// The reductions to a bounding box: every block ends with six atomics, on the same six words of all blocks, so blocks are large and
+// few (512 blocks of 256 threads -> these: bounds of 1 M points 16 -> 8 us; tree over 1 M boxes 449 -> 442, 3 M 1 023 -> 1 010).
+#define RGX_REDUCE_THREADS 1024
+__device__ __forceinline__ void fold_bounds(const float (*red)[6], int a, float &mn, float &mx)
+{
+    mn = red[0][a];
+    mx = red[0][a + 3];
+    for (int w = 1; w < RGX_REDUCE_THREADS / 64; ++w) {
+        mn = fminf(mn, red[w][a]);
+        mx = fmaxf(mx, red[w][a + 3]);
+    }
+}
+
+__global__ __launch_bounds__(RGX_REDUCE_THREADS) void k_aabb(const float *__restrict__ pos, const float *__restrict__ scale,
                                               const float *__restrict__ quat, const float *__restrict__ dens,
                                               int64_t n, float thr, float *__restrict__ boxes, int32_t *mn_enc, int32_t *mx_enc)
 {
-    // (a block takes several rounds of 256 Gaussians: every block ends with six atomics on the same six words,
-    // and one per 256 Gaussians made those the kernel's time)
     float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const float t = dens[i] / thr;
@@ -90,7 +101,7 @@ __global__ __launch_bounds__(256) void k_aabb(const float *__restrict__ pos, con
             b[a + 3] = fmaxf(b[a + 3], e[a + 3]);
         }
     }
-    __shared__ float red[4][6];
+    __shared__ float red[RGX_REDUCE_THREADS / 64][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
         const float mn = wave_min_all(b[a]), mx = wave_max_all(b[a + 3]);
@@ -99,8 +110,8 @@ __global__ __launch_bounds__(256) void k_aabb(const float *__restrict__ pos, con
     __syncthreads();
     if (threadIdx.x < 3 && mn_enc) {
         const int a = threadIdx.x;
-        const float mn = fminf(fminf(red[0][a], red[1][a]), fminf(red[2][a], red[3][a]));
-        const float mx = fmaxf(fmaxf(red[0][a + 3], red[1][a + 3]), fmaxf(red[2][a + 3], red[3][a + 3]));
+        float mn, mx;
+        fold_bounds(red, a, mn, mx);
         atomicMin(&mn_enc[a], enc_f(mn));
         atomicMax(&mx_enc[a], enc_f(mx));
     }
@@ -720,8 +731,8 @@ __global__ void k_mark_built(WsHeader *h, const int32_t *gate = nullptr) // of a
 
 // ---------------------------------------------------------------------------
 static inline dim3 grid_for(int64_t n, int block) { return dim3((unsigned)((n + block - 1) / block)); }
-// For the kernels that loop over their input and end with atomics on a few shared words: two blocks per CU.
-static inline dim3 grid_reduce(int64_t n, int block) { return dim3((unsigned)std::min<int64_t>((n + block - 1) / block, 512)); }
+// For the kernels that loop over their input and end with atomics on a few shared words.
+static inline dim3 grid_reduce(int64_t n, int most) { return dim3((unsigned)std::min<int64_t>((n + RGX_REDUCE_THREADS - 1) / RGX_REDUCE_THREADS, most)); }
 
 extern "C" int rgx_aabb(const float *pos, const float *scale, const float *quat, const float *dens, int64_t n,
                         float sigma_threshold, float *bboxes, float *bb_min, float *bb_max, void *stream)
@@ -733,7 +744,7 @@ extern "C" int rgx_aabb(const float *pos, const float *scale, const float *quat,
     int32_t *mn = (int32_t *)bb_min, *mx = (int32_t *)bb_max;
     if (mn) hipLaunchKernelGGL(k_init_enc, dim3(1), dim3(64), 0, s, mn, mx);
     if (n > 0)
-        hipLaunchKernelGGL(k_aabb, grid_reduce(n, 256), dim3(256), 0, s, pos, scale, quat, dens, n, sigma_threshold, bboxes, mn, mx);
+        hipLaunchKernelGGL(k_aabb, grid_reduce(n, 256), dim3(RGX_REDUCE_THREADS), 0, s, pos, scale, quat, dens, n, sigma_threshold, bboxes, mn, mx);
     if (mn) hipLaunchKernelGGL(k_decode_enc, dim3(1), dim3(64), 0, s, mn, mx);
     RGX_LAUNCH_CHECK();
     return RGX_OK;
@@ -747,7 +758,7 @@ extern "C" int rgx_build_workspace_bytes(int64_t n, size_t *bytes)
 }
 
 // Copies caller-supplied boxes into the workspace and reduces the scene bbox.
-__global__ __launch_bounds__(256) void k_take_boxes(const float *__restrict__ in, int64_t n, float *__restrict__ boxes,
+__global__ __launch_bounds__(RGX_REDUCE_THREADS) void k_take_boxes(const float *__restrict__ in, int64_t n, float *__restrict__ boxes,
                                                     int32_t *mn_enc, int32_t *mx_enc, const int32_t *gate = nullptr)
 {
     if (gate_closed(gate)) return; // the whole grid
@@ -757,7 +768,7 @@ __global__ __launch_bounds__(256) void k_take_boxes(const float *__restrict__ in
             const float v = boxes[6 * i + a] = in[6 * i + a];
             b[a] = a < 3 ? fminf(b[a], v) : fmaxf(b[a], v);
         }
-    __shared__ float red[4][6];
+    __shared__ float red[RGX_REDUCE_THREADS / 64][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
         const float mn = wave_min_all(b[a]), mx = wave_max_all(b[a + 3]);
@@ -766,8 +777,10 @@ __global__ __launch_bounds__(256) void k_take_boxes(const float *__restrict__ in
     __syncthreads();
     if (threadIdx.x < 3) {
         const int a = threadIdx.x;
-        atomicMin(&mn_enc[a], enc_f(fminf(fminf(red[0][a], red[1][a]), fminf(red[2][a], red[3][a]))));
-        atomicMax(&mx_enc[a], enc_f(fmaxf(fmaxf(red[0][a + 3], red[1][a + 3]), fmaxf(red[2][a + 3], red[3][a + 3]))));
+        float mn, mx;
+        fold_bounds(red, a, mn, mx);
+        atomicMin(&mn_enc[a], enc_f(mn));
+        atomicMax(&mx_enc[a], enc_f(mx));
     }
 }
 
@@ -808,10 +821,10 @@ static int build_impl(const float *pos, const float *scale, const float *quat, c
     hipLaunchKernelGGL(k_init_header, dim3(1), dim3(64), 0, s, hdr, n);
     if (n > 0) {
         if (in_boxes)
-            hipLaunchKernelGGL(k_take_boxes, grid_reduce(n, 256), dim3(256), 0, s, in_boxes, n, boxes, hdr->bb_min_enc,
+            hipLaunchKernelGGL(k_take_boxes, grid_reduce(n, 256), dim3(RGX_REDUCE_THREADS), 0, s, in_boxes, n, boxes, hdr->bb_min_enc,
                                hdr->bb_max_enc);
         else
-            hipLaunchKernelGGL(k_aabb, grid_reduce(n, 256), dim3(256), 0, s, pos, scale, quat, dens, n, sigma_threshold, boxes,
+            hipLaunchKernelGGL(k_aabb, grid_reduce(n, 256), dim3(RGX_REDUCE_THREADS), 0, s, pos, scale, quat, dens, n, sigma_threshold, boxes,
                                hdr->bb_min_enc, hdr->bb_max_enc);
         hipLaunchKernelGGL(k_morton63, grid_for(n, 256), dim3(256), 0, s, boxes, n, hdr, k0, v0);
         RGX_LAUNCH_CHECK();
@@ -857,7 +870,7 @@ extern "C" int rgx_refit_aabbs(const float *bboxes, int64_t n, void *ws, size_t 
     const int32_t *gate = &hdr->refit_ok;
     hipLaunchKernelGGL(k_refit_begin, dim3(1), dim3(64), 0, s, hdr, n);
     if (n > 0) {
-        hipLaunchKernelGGL(k_take_boxes, grid_reduce(n, 256), dim3(256), 0, s, bboxes, n, boxes, hdr->bb_min_enc, hdr->bb_max_enc, gate);
+        hipLaunchKernelGGL(k_take_boxes, grid_reduce(n, 256), dim3(RGX_REDUCE_THREADS), 0, s, bboxes, n, boxes, hdr->bb_min_enc, hdr->bb_max_enc, gate);
         hipLaunchKernelGGL(k_finish_bbox, dim3(1), dim3(64), 0, s, hdr, (float *)nullptr, (float *)nullptr, gate);
         hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, order, n, nodes, parent, flags, (uint32_t *)(w + L.vals1), gate);
         if (n > 1) hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, flags, gate);
@@ -921,7 +934,7 @@ extern "C" int rgx_build_order(const void *ws, int64_t n, int32_t *order_out, vo
 // ---------------------------------------------------------------------------
 // 30-bit Morton ordering of the point cloud (utils/reordering_utils.py:55-104,
 // classes/point_cloud.py:1017-1024).
-__global__ __launch_bounds__(256) void k_pos_minmax(const float *__restrict__ pos, int64_t n, int32_t *mn_enc, int32_t *mx_enc)
+__global__ __launch_bounds__(RGX_REDUCE_THREADS) void k_pos_minmax(const float *__restrict__ pos, int64_t n, int32_t *mn_enc, int32_t *mx_enc)
 {
     float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
     const int64_t step = (int64_t)gridDim.x * blockDim.x;
@@ -939,7 +952,7 @@ __global__ __launch_bounds__(256) void k_pos_minmax(const float *__restrict__ po
                 b[a + 3] = fmaxf(b[a + 3], v[k][a]);
             }
     }
-    __shared__ float red[4][6];
+    __shared__ float red[RGX_REDUCE_THREADS / 64][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int a = 0; a < 3; ++a) {
         const float mn = wave_min_all(b[a]), mx = wave_max_all(b[a + 3]);
@@ -948,8 +961,10 @@ __global__ __launch_bounds__(256) void k_pos_minmax(const float *__restrict__ po
     __syncthreads();
     if (threadIdx.x < 3) {
         const int a = threadIdx.x;
-        atomicMin(&mn_enc[a], enc_f(fminf(fminf(red[0][a], red[1][a]), fminf(red[2][a], red[3][a]))));
-        atomicMax(&mx_enc[a], enc_f(fmaxf(fmaxf(red[0][a + 3], red[1][a + 3]), fmaxf(red[2][a + 3], red[3][a + 3]))));
+        float mn, mx;
+        fold_bounds(red, a, mn, mx);
+        atomicMin(&mn_enc[a], enc_f(mn));
+        atomicMax(&mx_enc[a], enc_f(mx));
     }
 }
 
@@ -1010,7 +1025,7 @@ extern "C" int rgx_morton_order(const float *pos, int64_t n, int64_t *codes, int
     uint32_t *k0 = (uint32_t *)(w + L.keys0), *k1 = (uint32_t *)(w + L.keys1);
     uint32_t *v0 = (uint32_t *)(w + L.vals0), *v1 = (uint32_t *)(w + L.vals1);
     hipLaunchKernelGGL(k_init_enc, dim3(1), dim3(64), 0, s, mn, mx);
-    hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 256), dim3(256), 0, s, pos, n, mn, mx);
+    hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 128), dim3(RGX_REDUCE_THREADS), 0, s, pos, n, mn, mx);
     hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, mn, mx, k0, v0, codes);
     RGX_LAUNCH_CHECK();
     if (order) {
@@ -1403,7 +1418,7 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     float4 *pts = (float4 *)(w + K.pts), *leaves = (float4 *)(w + K.leaves), *boxes = (float4 *)(w + K.boxes);
     int32_t *supers = (int32_t *)(w + K.supers);
     hipLaunchKernelGGL(k_knn_begin, dim3(1), dim3(256), 0, s, mn, mx, supers, K.ns);
-    hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 256), dim3(256), 0, s, pos, n, mn, mx);
+    hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 128), dim3(RGX_REDUCE_THREADS), 0, s, pos, n, mn, mx);
     hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, mn, mx, k0, v0, (int64_t *)nullptr);
     RGX_LAUNCH_CHECK();
     const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + K.m.hist), s);
