@@ -276,6 +276,13 @@ int rgx_march_viewer(const void *ws, const RgxCamera *cam, const RgxMarch *march
 int rgx_gather_rows(int32_t count, const void *const *src, void *const *dst, const int64_t *row_bytes,
                     const int64_t *order, int64_t n, void *stream);
 
+/* The same with a workspace (256-byte aligned device memory) in which the short rows of many tensors are
+ * put together before they are gathered; rgx_gather_workspace_bytes says how much it takes (0: nothing to
+ * put together).  With less, as rgx_gather_rows. */
+int rgx_gather_workspace_bytes(int32_t count, const int64_t *row_bytes, int64_t n, size_t *bytes);
+int rgx_gather_rows_packed(int32_t count, const void *const *src, void *const *dst, const int64_t *row_bytes,
+                           const int64_t *order, int64_t n, void *ws, size_t ws_bytes, void *stream);
+
 /* Replaces distCUDA2 of the simple-knn extension (submodules/simple-knn/simple_knn.cu:186-222,
  * called at classes/point_cloud.py:252 to initialise the scales): mean_dist2[i] = mean of the
  * squared distances from point i to its three nearest other points (FLT_MAX stands in for a

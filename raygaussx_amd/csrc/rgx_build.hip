@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 
 // ---------------------------------------------------------------------------
 // order-preserving float <-> int encoding for atomicMin/atomicMax
@@ -57,7 +58,6 @@ __global__ void k_refit_begin(WsHeader *h, int64_t n)
 }
 __device__ __forceinline__ bool gate_closed(const int32_t *gate) { return gate != nullptr && *gate == 0; }
 
-// k-sigma AABB of a rotated ellipsoid (optix_utils.py:49-77), canonical arithmetic.
 // The reductions to a bounding box: every block ends with six atomics, on the same six words of all blocks, so blocks are large and
 // few (512 blocks of 256 threads -> these: bounds of 1 M points 16 -> 8 us; tree over 1 M boxes 449 -> 442, 3 M 1 023 -> 1 010).
 #define RGX_REDUCE_THREADS 1024
@@ -71,6 +71,7 @@ __device__ __forceinline__ void fold_bounds(const float (*red)[6], int a, float 
     }
 }
 
+// k-sigma AABB of a rotated ellipsoid (optix_utils.py:49-77), canonical arithmetic.
 __global__ __launch_bounds__(RGX_REDUCE_THREADS) void k_aabb(const float *__restrict__ pos, const float *__restrict__ scale,
                                               const float *__restrict__ quat, const float *__restrict__ dens,
                                               int64_t n, float thr, float *__restrict__ boxes, int32_t *mn_enc, int32_t *mx_enc)
@@ -1044,7 +1045,7 @@ extern "C" int rgx_morton_order(const float *pos, int64_t n, int64_t *codes, int
 // length and the tensors' alignment allow (16, 12, 8 or 4 bytes): writes are coalesced, the reads of a
 // row are contiguous, and every thread has up to four reads in flight.  Bound by memory: one 32-bit word per
 // thread, its row found by a 64-bit division and its number fetched per word, took 0.743 ms for the 15
-// tensors of a 1 M cloud (1.42 GB); this takes 0.438 ms (3.2 TB/s).
+// tensors of a 1 M cloud (1.42 GB); this takes 0.438 ms (3.2 TB/s), and short rows have a way of their own below.
 #define RGX_GATHER_MAX 24
 #define RGX_GATHER_ROWS 128
 #define RGX_GATHER_LONG 4096 // a row of at least this many pieces is moved by the workgroup on its own
@@ -1131,23 +1132,146 @@ __global__ __launch_bounds__(256) void k_gather_rows(const GatherArgs A, const i
     }
 }
 
-extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *const *dst, const int64_t *row_bytes,
-                               const int64_t *order, int64_t n, void *stream)
+// Short rows.  A row of a few words read wherever it lies costs the whole line it lies in: the twelve short tensors of a 1 M
+// cloud (positions, scales, quaternions and densities with both Adam moments, 132 bytes a Gaussian) took 230 us of the
+// reordering's 439, the three tensors of 192-byte rows 249.  So the short rows of a Gaussian are first put together in a record of up to 128
+// bytes, read and written in order, and the records gathered: one line instead of one per tensor.  Both kernels go through a
+// tile of 128 rows in LDS, so that every tensor's rows are read and written as one run of words: 1 M 439 -> 398 us for all tensors
+// (72 to put them together, 67 to gather them, one tensor too many for the record's 32 words; 3.7 and 4.4 TB/s),
+// 3 M 1 454 -> 1 192.
+#define RGX_PACK_WORDS 32    // of a record
+#define RGX_PACK_ROW 8       // words of the longest row that counts as short
+#define RGX_PACK_STRIDE 36   // words from row to row in LDS
+#define RGX_PACK_MIN 2       // tensors that make a record worth while
+#define RGX_PACK_ROWS 262144 // rows from which on it is (300 k 129 -> 125 us, 400 k 174 -> 161; below, the caches hold the short tensors)
+struct PackArgs {
+    const uint32_t *src[RGX_PACK_WORDS];
+    uint32_t *dst[RGX_PACK_WORDS];
+    uint32_t magic[RGX_PACK_WORDS]; // as in GatherArgs, of the row's words
+    uint8_t words[RGX_PACK_WORDS], at[RGX_PACK_WORDS]; // of the row; where it begins in the record
+    uint8_t owner[RGX_PACK_WORDS]; // the tensor that a word of the record belongs to
+    int32_t count, quads, total;   // tensors; 16-byte pieces and words of a record
+    int32_t aligned;               // all tensors begin on a 16-byte boundary
+};
+// Goes through the words that the tensors have in a whole tile, in pieces of 16 bytes: a word of the record stands for
+// RGX_GATHER_ROWS / 4 of them.  each(tensor, piece of the tensor's run of words, where its four words are in the tile)
+template <typename Each>
+__device__ __forceinline__ void pack_pieces(const PackArgs &A, Each each)
 {
-    const DeviceScope on_device(order);
-    if (count < 0 || n < 0 || (count > 0 && (!src || !dst || !row_bytes)) || (n > 0 && count > 0 && !order)) return RGX_EINVAL;
+    constexpr int PER = RGX_GATHER_ROWS / 4;
+    for (int p = threadIdx.x; p < A.total * PER; p += 256) {
+        const int c = p / PER, t = A.owner[c];
+        const uint32_t w = A.words[t], piece = (uint32_t)(c - A.at[t]) * PER + (uint32_t)p % PER;
+        uint32_t r = w == 1 ? 4 * piece : __umulhi(4 * piece, A.magic[t]), k = 4 * piece - r * w;
+        uint32_t at[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            at[i] = r * RGX_PACK_STRIDE + A.at[t] + k;
+            if (++k == w) {
+                k = 0;
+                ++r;
+            }
+        }
+        each(t, piece, at);
+    }
+}
+__global__ __launch_bounds__(256) void k_pack_rows(const PackArgs A, int64_t n, uint4 *__restrict__ rec)
+{
+    __shared__ __align__(16) uint32_t s_tile[RGX_GATHER_ROWS * RGX_PACK_STRIDE];
+    const int64_t row0 = (int64_t)blockIdx.x * RGX_GATHER_ROWS;
+    const int rows = (int)(n - row0 < RGX_GATHER_ROWS ? n - row0 : RGX_GATHER_ROWS);
+    if (rows == RGX_GATHER_ROWS && A.aligned) {
+        pack_pieces(A, [&](int t, uint32_t piece, const uint32_t (&at)[4]) {
+            const uint4 v = ((const uint4 *)(A.src[t] + row0 * A.words[t]))[piece];
+            s_tile[at[0]] = v.x; s_tile[at[1]] = v.y; s_tile[at[2]] = v.z; s_tile[at[3]] = v.w;
+        });
+    } else {
+        for (int t = 0; t < A.count; ++t) {
+            const uint32_t w = A.words[t];
+            const uint32_t *src = A.src[t] + row0 * w;
+            for (uint32_t p = threadIdx.x; p < rows * w; p += 256) {
+                const uint32_t r = w == 1 ? p : __umulhi(p, A.magic[t]);
+                s_tile[r * RGX_PACK_STRIDE + A.at[t] + (p - r * w)] = src[p];
+            }
+        }
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < rows * A.quads; p += 256) {
+        const int r = p / A.quads, q = p - r * A.quads;
+        rec[row0 * A.quads + p] = *(const uint4 *)(s_tile + r * RGX_PACK_STRIDE + 4 * q);
+    }
+}
+__global__ __launch_bounds__(256) void k_unpack_rows(const PackArgs A, const int64_t *__restrict__ order, int64_t n, const uint4 *__restrict__ rec)
+{
+    __shared__ __align__(16) uint32_t s_tile[RGX_GATHER_ROWS * RGX_PACK_STRIDE];
+    const int64_t row0 = (int64_t)blockIdx.x * RGX_GATHER_ROWS;
+    const int rows = (int)(n - row0 < RGX_GATHER_ROWS ? n - row0 : RGX_GATHER_ROWS);
+    for (int p = threadIdx.x; p < rows * A.quads; p += 256) {
+        const int r = p / A.quads, q = p - r * A.quads;
+        *(uint4 *)(s_tile + r * RGX_PACK_STRIDE + 4 * q) = rec[order[row0 + r] * A.quads + q];
+    }
+    __syncthreads();
+    if (rows == RGX_GATHER_ROWS && A.aligned) {
+        pack_pieces(A, [&](int t, uint32_t piece, const uint32_t (&at)[4]) {
+            ((uint4 *)(A.dst[t] + row0 * A.words[t]))[piece] = make_uint4(s_tile[at[0]], s_tile[at[1]], s_tile[at[2]], s_tile[at[3]]);
+        });
+        return;
+    }
+    for (int t = 0; t < A.count; ++t) {
+        const uint32_t w = A.words[t];
+        uint32_t *dst = A.dst[t] + row0 * w;
+        for (uint32_t p = threadIdx.x; p < rows * w; p += 256) {
+            const uint32_t r = w == 1 ? p : __umulhi(p, A.magic[t]);
+            dst[p] = s_tile[r * RGX_PACK_STRIDE + A.at[t] + (p - r * w)];
+        }
+    }
+}
+
+// The tensors not done yet that share the next record (first fit, in order); returns its words.
+static int pack_group(int32_t count, const int64_t *row_bytes, std::vector<bool> &done, std::vector<int32_t> &members)
+{
+    members.clear();
+    int words = 0;
+    for (int32_t i = 0; i < count; ++i) {
+        const int64_t w = row_bytes[i] / 4;
+        if (done[i] || w > RGX_PACK_ROW || words + w > RGX_PACK_WORDS) continue;
+        members.push_back(i);
+        words += (int)w;
+    }
+    return words;
+}
+
+static int gather_check(int32_t count, const int64_t *row_bytes, int64_t n)
+{
+    if (count < 0 || n < 0 || (count > 0 && !row_bytes)) return RGX_EINVAL;
     for (int i = 0; i < count; ++i)
-        if (row_bytes[i] <= 0 || (row_bytes[i] & 3) || row_bytes[i] > 0x7fffffff || ((!src[i] || !dst[i]) && n > 0) || src[i] == dst[i])
-            return RGX_EINVAL;
-    if (n == 0) return RGX_OK;
+        if (row_bytes[i] <= 0 || (row_bytes[i] & 3) || row_bytes[i] > 0x7fffffff) return RGX_EINVAL;
+    return RGX_OK;
+}
+
+extern "C" int rgx_gather_workspace_bytes(int32_t count, const int64_t *row_bytes, int64_t n, size_t *bytes)
+{
+    const int rc = gather_check(count, row_bytes, n);
+    if (rc != RGX_OK || !bytes) return RGX_EINVAL;
+    int shorts = 0;
+    for (int i = 0; i < count; ++i) shorts += row_bytes[i] / 4 <= RGX_PACK_ROW;
+    *bytes = n >= RGX_PACK_ROWS && shorts >= RGX_PACK_MIN ? (size_t)n * RGX_PACK_WORDS * 4 : 0;
+    return RGX_OK;
+}
+
+static int gather_direct(const std::vector<int32_t> &which, const void *const *src, void *const *dst, const int64_t *row_bytes,
+                         const int64_t *order, int64_t n, hipStream_t s)
+{
+    const int32_t count = (int32_t)which.size();
     for (int base = 0; base < count; base += RGX_GATHER_MAX) {
         GatherArgs A;
         const int m = count - base < RGX_GATHER_MAX ? count - base : RGX_GATHER_MAX;
         A.count = m;
         for (int i = 0; i < m; ++i) {
-            A.src[i] = (const uint32_t *)src[base + i];
-            A.dst[i] = (uint32_t *)dst[base + i];
-            const int32_t words = (int32_t)(row_bytes[base + i] / 4);
+            const int32_t t = which[base + i];
+            A.src[i] = (const uint32_t *)src[t];
+            A.dst[i] = (uint32_t *)dst[t];
+            const int32_t words = (int32_t)(row_bytes[t] / 4);
             const uintptr_t at = (uintptr_t)A.src[i] | (uintptr_t)A.dst[i];
             const int w = words % 4 == 0 && (at & 15) == 0 ? 4 : words % 3 == 0 ? 3 : words % 2 == 0 && (at & 7) == 0 ? 2 : 1;
             A.words[i] = (uint8_t)w;
@@ -1157,10 +1281,65 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
         const int64_t blocks = (n + RGX_GATHER_ROWS - 1) / RGX_GATHER_ROWS;
         // a workgroup goes through all tensors where there are enough of them to fill the chip several times over
         const int split = blocks >= 2048 ? 1 : m;
-        hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)blocks, (unsigned)split), dim3(256), 0, (hipStream_t)stream, A, order, n);
+        hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)blocks, (unsigned)split), dim3(256), 0, s, A, order, n);
         RGX_LAUNCH_CHECK();
     }
     return RGX_OK;
+}
+
+// ws, ws_bytes: rgx_gather_workspace_bytes(); with less (or none) every tensor is gathered by itself.
+extern "C" int rgx_gather_rows_packed(int32_t count, const void *const *src, void *const *dst, const int64_t *row_bytes,
+                                      const int64_t *order, int64_t n, void *ws, size_t ws_bytes, void *stream)
+{
+    const DeviceScope on_device(order);
+    const int rc = gather_check(count, row_bytes, n);
+    if (rc != RGX_OK) return rc;
+    if ((count > 0 && (!src || !dst)) || (n > 0 && count > 0 && !order) || ((uintptr_t)ws & 255u)) return RGX_EINVAL;
+    for (int i = 0; i < count; ++i)
+        if (((!src[i] || !dst[i]) && n > 0) || src[i] == dst[i]) return RGX_EINVAL;
+    if (n == 0) return RGX_OK;
+    size_t need = 0;
+    rgx_gather_workspace_bytes(count, row_bytes, n, &need);
+    std::vector<bool> done(count, false);
+    std::vector<int32_t> members;
+    hipStream_t s = (hipStream_t)stream;
+    if (need > 0 && ws && ws_bytes >= need) {
+        const unsigned blocks = (unsigned)((n + RGX_GATHER_ROWS - 1) / RGX_GATHER_ROWS);
+        for (int words = pack_group(count, row_bytes, done, members); (int)members.size() >= RGX_PACK_MIN;
+             words = pack_group(count, row_bytes, done, members)) {
+            PackArgs A;
+            A.count = (int32_t)members.size();
+            A.quads = (words + 3) / 4;
+            A.total = words;
+            A.aligned = 1;
+            int at = 0;
+            for (int i = 0; i < A.count; ++i) {
+                const int32_t t = members[i], w = (int32_t)(row_bytes[t] / 4);
+                A.src[i] = (const uint32_t *)src[t];
+                A.dst[i] = (uint32_t *)dst[t];
+                A.words[i] = (uint8_t)w;
+                A.at[i] = (uint8_t)at;
+                for (int k = 0; k < w; ++k) A.owner[at + k] = (uint8_t)i;
+                A.aligned &= (((uintptr_t)A.src[i] | (uintptr_t)A.dst[i]) & 15) == 0;
+                A.magic[i] = (uint32_t)((1ull << 32) / (uint32_t)w + 1);
+                at += w;
+                done[t] = true;
+            }
+            hipLaunchKernelGGL(k_pack_rows, dim3(blocks), dim3(256), 0, s, A, n, (uint4 *)ws);
+            hipLaunchKernelGGL(k_unpack_rows, dim3(blocks), dim3(256), 0, s, A, order, n, (const uint4 *)ws);
+            RGX_LAUNCH_CHECK();
+        }
+    }
+    members.clear();
+    for (int32_t i = 0; i < count; ++i)
+        if (!done[i]) members.push_back(i);
+    return gather_direct(members, src, dst, row_bytes, order, n, s);
+}
+
+extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *const *dst, const int64_t *row_bytes,
+                               const int64_t *order, int64_t n, void *stream)
+{
+    return rgx_gather_rows_packed(count, src, dst, row_bytes, order, n, nullptr, 0, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -28,7 +28,7 @@ def morton_order(positions, return_codes=False):
 @torch.no_grad()
 def reorder_tensors(order, tensors):
     """Gathers every per-Gaussian tensor (parameters, Adam moments, statistics) with one
-    permutation in one launch: ``[t[order] for t in tensors]`` (``None`` entries pass through).
+    permutation: ``[t[order] for t in tensors]`` (``None`` entries pass through).
     Tensors must have 4- or 8-byte elements (rows that are multiples of 4 bytes)."""
     order = order.to(torch.int64).contiguous()
     n = order.shape[0]
@@ -48,6 +48,9 @@ def reorder_tensors(order, tensors):
         src_p = (C.c_void_p * m)(*[s.data_ptr() for s in srcs])
         dst_p = (C.c_void_p * m)(*[d.data_ptr() for d in dsts])
         rows = (C.c_int64 * m)(*[s[0].numel() * s.element_size() for s in srcs])
-        L.check(L.lib().rgx_gather_rows(C.c_int32(m), src_p, dst_p, rows, L.ptr(order), C.c_int64(n), L.stream(order.device)))
+        size = L.size_query(L.lib().rgx_gather_workspace_bytes, C.c_int32(m), rows, C.c_int64(n))
+        ws = torch.empty(size, dtype=torch.uint8, device=order.device) if size else None
+        L.check(L.lib().rgx_gather_rows_packed(C.c_int32(m), src_p, dst_p, rows, L.ptr(order), C.c_int64(n), L.ptr(ws), C.c_size_t(size),
+                                               L.stream(order.device)))
     it = iter(dsts)
     return [None if t is None else next(it) for t in tensors]

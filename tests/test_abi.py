@@ -77,6 +77,11 @@ def test_bad_arguments_are_rejected_before_any_launch():
     assert lib.rgx_build(null, null, null, null, C.c_int64(10), C.c_float(0.1), null, C.c_size_t(0), null) == -1
     assert lib.rgx_reduce_supersampling(null, 8, 8, 1, 1, 0, null, null, null) == -1
     assert lib.rgx_gather_rows(1, null, null, null, null, C.c_int64(4), null) == -1
+    rows, size = (C.c_int64 * 3)(12, 16, 192), C.c_size_t(7)
+    assert lib.rgx_gather_workspace_bytes(3, rows, C.c_int64(1000), C.byref(size)) == 0 and size.value == 0
+    assert lib.rgx_gather_workspace_bytes(3, rows, C.c_int64(1_000_000), C.byref(size)) == 0 and size.value == 128_000_000
+    assert lib.rgx_gather_workspace_bytes(3, (C.c_int64 * 3)(12, 14, 192), C.c_int64(4), C.byref(size)) == -1
+    assert lib.rgx_gather_rows_packed(3, null, null, rows, null, C.c_int64(4), null, C.c_size_t(0), null) == -1
     assert lib.rgx_dist2_knn3(null, C.c_int64(4), null, null, C.c_size_t(0), null) == -1
     cam = _lib.RgxCamera()
     march = _lib.RgxMarch(0.0025, 0, 2048, 1, 1e-3)

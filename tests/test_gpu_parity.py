@@ -778,6 +778,26 @@ def test_reorder_tensors_of_long_rows_and_off_alignment(gx, n, words, offset):
     assert torch.equal(got, t[order]) and torch.equal(second, plain[order])
 
 
+@pytest.mark.parametrize("n", [262_143, 262_144, 262_145, 300_031])
+@pytest.mark.parametrize("words,odd", [
+    ((3, 4, 3, 1, 3, 4, 3, 1, 3, 4, 3, 1), None),      # the short tensors of a cloud: one word more than a record holds
+    ((8, 8, 8, 8, 2, 9, 7), None),                     # a full record, a second one, and a row too long for either
+    ((1,) * 34, None), ((5, 12), None), ((6, 3, 2), 1)])   # more tensors than a record; one short alone; one off a 16-byte boundary
+def test_reorder_tensors_of_many_short_rows(gx, n, words, odd):
+    """Short rows put together in records: record sizes, what is left over, numbers of rows around the tile of 128 and the
+    line from which on it is done."""
+    from raygaussx_amd.reordering import reorder_tensors
+    gen = torch.Generator(gx.DEV).manual_seed(n)
+    tensors = []
+    for i, w in enumerate(words):
+        off = 1 if i == odd else 0
+        tensors.append(torch.randint(-2 ** 31, 2 ** 31 - 1, (n * w + off,), dtype=torch.int32, device=gx.DEV, generator=gen)[off:].view(n, w))
+    order = torch.randperm(n, device=gx.DEV, generator=gen)
+    _step(f"short rows n={n} words={words}")
+    for got, src in zip(reorder_tensors(order, tensors), tensors):
+        assert torch.equal(got, src[order])
+
+
 def test_reference_style_inference_loop_reuses_the_tree(gx, orc, c0):
     """scripts/test.py:50-126 pattern: boxes -> one acceleration structure -> several cameras."""
     from raygaussx_amd import optix_utils as u_ox
