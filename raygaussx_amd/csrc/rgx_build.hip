@@ -538,10 +538,17 @@ static int radix_sort(K *k0, uint32_t *v0, K *k1, uint32_t *v1, int64_t n, int b
 }
 
 // ---------------------------------------------------------------------------
-// Leaves, radix tree (Karras 2012), refit, skip links.
+// Radix tree (Karras 2012), leaves, refit.
+// Skip links: the node after a subtree is the right child of the one node whose children meet behind the subtree's last leaf;
+// after[j] is that child, for j = the last leaf but the tree's (k_karras knows it: every gap between two leaves is
+// one node's).  (A kernel of its own that climbed from every node to the first ancestor it was left of took 38 us at 1 M boxes and
+// 100 at 3 M.)
+__device__ __forceinline__ int32_t skip_link(const int32_t *after, int64_t n, int64_t last_leaf) { return last_leaf < n - 1 ? after[last_leaf] : -1; }
+
 __global__ __launch_bounds__(256) void k_leaves(const float *__restrict__ boxes, const uint32_t *__restrict__ order, int64_t n,
                                                 Node *__restrict__ nodes, int32_t *__restrict__ parent, int32_t *__restrict__ flags,
-                                                uint32_t *__restrict__ place, const int32_t *gate = nullptr)
+                                                uint32_t *__restrict__ place, const int32_t *__restrict__ after, WsHeader *h,
+                                                const int32_t *gate = nullptr)
 {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n || gate_closed(gate)) return;
@@ -552,10 +559,11 @@ __global__ __launch_bounds__(256) void k_leaves(const float *__restrict__ boxes,
     nd.lo[0] = b[0]; nd.lo[1] = b[1]; nd.lo[2] = b[2];
     nd.hi[0] = b[3]; nd.hi[1] = b[4]; nd.hi[2] = b[5];
     nd.left = ~(int32_t)j;
-    nd.skip = -1;
+    nd.skip = skip_link(after, n, j);
     nodes[n - 1 + j] = nd;
     flags[j] = 0;
     if (j == 0) parent[0] = -1;
+    if (n == 1) h->built = 1; // (no kernel follows)
 }
 
 __device__ __forceinline__ int delta(const uint64_t *keys, int64_t n, int64_t i, int64_t j)
@@ -569,7 +577,7 @@ __device__ __forceinline__ int delta(const uint64_t *keys, int64_t n, int64_t i,
 // other_end[i]: internal node i covers the sorted leaves between i and other_end[i]
 __global__ __launch_bounds__(256) void k_karras(const uint64_t *__restrict__ keys, int64_t n, Node *__restrict__ nodes,
                                                 int32_t *__restrict__ parent, int32_t *__restrict__ right,
-                                                int32_t *__restrict__ other_end)
+                                                int32_t *__restrict__ other_end, int32_t *__restrict__ after)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
@@ -593,6 +601,7 @@ __global__ __launch_bounds__(256) void k_karras(const uint64_t *__restrict__ key
     const int32_t rc = (int32_t)(hi == gamma + 1 ? n - 1 + gamma + 1 : gamma + 1);
     nodes[i].left = lc;
     right[i] = rc;
+    after[gamma] = rc;
     parent[lc] = (int32_t)i;
     parent[rc] = (int32_t)i;
     other_end[i] = (int32_t)j;
@@ -623,7 +632,8 @@ __device__ __forceinline__ float ld_agent(const float *p)
 
 __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int32_t *__restrict__ parent,
                                                const int32_t *__restrict__ right, const int32_t *__restrict__ other_end,
-                                               int32_t *flags, const int32_t *gate = nullptr)
+                                               const int32_t *__restrict__ after, int32_t *flags,
+                                               WsHeader *h, const int32_t *gate = nullptr)
 {
     __shared__ float s_box[2][6][256]; // [which child][lo xyz, hi xyz][node - first leaf of the workgroup]
     __shared__ int s_arrived[256];
@@ -644,7 +654,8 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
     while (node >= 0) {
         const int32_t o = other_end[node];
         if ((node < o ? node : o) < b0 || (node < o ? o : node) > b1) break;
-        const int slot = (int)(node - b0), side = nodes[node].left == child ? 0 : 1;
+        const int32_t left = nodes[node].left;
+        const int slot = (int)(node - b0), side = left == child ? 0 : 1;
         for (int c = 0; c < 3; ++c) {
             s_box[side][c][slot] = lo[c];
             s_box[side][3 + c][slot] = hi[c];
@@ -652,9 +663,14 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
         __threadfence_block();
         if (atomicAdd(&s_arrived[slot], 1) == 0) return; // the sibling subtree is not done yet
         __threadfence_block();
+        float slo[3], shi[3];
         for (int c = 0; c < 3; ++c) {
-            lo[c] = fminf(lo[c], s_box[1 - side][c][slot]);
-            hi[c] = fmaxf(hi[c], s_box[1 - side][3 + c][slot]);
+            slo[c] = s_box[1 - side][c][slot];
+            shi[c] = s_box[1 - side][3 + c][slot];
+        }
+        for (int c = 0; c < 3; ++c) {
+            lo[c] = fminf(lo[c], slo[c]);
+            hi[c] = fmaxf(hi[c], shi[c]);
         }
         child = node;
         node = parent[node];
@@ -662,20 +678,21 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
         // thread arrives there second, maybe on another XCD): only then does it have to go out as agent-scope
         // stores.  Everything below such a subtree root is next read by other kernels: plain stores.
         bool inside = false;
+        const int32_t skip = skip_link(after, n, child < o ? o : child);
         if (node >= 0) {
-            const int32_t o = other_end[node];
-            inside = (node < o ? node : o) >= b0 && (node < o ? o : node) <= b1;
+            const int32_t up = other_end[node];
+            inside = (node < up ? node : up) >= b0 && (node < up ? up : node) <= b1;
         }
         if (inside) {
-            for (int c = 0; c < 3; ++c) {
-                nodes[child].lo[c] = lo[c];
-                nodes[child].hi[c] = hi[c];
-            }
+            float4 *dst = (float4 *)&nodes[child];
+            dst[0] = make_float4(lo[0], lo[1], lo[2], __int_as_float(left));
+            dst[1] = make_float4(hi[0], hi[1], hi[2], __int_as_float(skip));
         } else {
             for (int c = 0; c < 3; ++c) {
                 st_agent(&nodes[child].lo[c], lo[c]);
                 st_agent(&nodes[child].hi[c], hi[c]);
             }
+            nodes[child].skip = skip;
             break;
         }
     }
@@ -684,7 +701,8 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
     // so that each level is three trips to memory one after the other (stores acknowledged, counter, sibling's box)
     // and not five.
     while (node >= 0) {
-        const int32_t left = nodes[node].left, rgt = right[node], up = parent[node];
+        const int32_t left = nodes[node].left, rgt = right[node], up = parent[node], end = other_end[node];
+        const int32_t skip = skip_link(after, n, node < end ? end : node);
 #if defined(__gfx942__) || defined(__gfx950__)
         // (the immediate below is the gfx9 encoding of vmcnt(0) with the other counters left alone, and the
         // argument that the wait suffices rests on how these chips complete agent-scope atomic stores)
@@ -698,31 +716,22 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 #endif
         const Node *sibling = &nodes[left == child ? rgt : left];
+        float slo[3], shi[3];
         for (int c = 0; c < 3; ++c) {
-            lo[c] = fminf(lo[c], ld_agent(&sibling->lo[c]));
-            hi[c] = fmaxf(hi[c], ld_agent(&sibling->hi[c]));
+            slo[c] = ld_agent(&sibling->lo[c]);
+            shi[c] = ld_agent(&sibling->hi[c]);
+        }
+        for (int c = 0; c < 3; ++c) {
+            lo[c] = fminf(lo[c], slo[c]);
+            hi[c] = fmaxf(hi[c], shi[c]);
             st_agent(&nodes[node].lo[c], lo[c]);
             st_agent(&nodes[node].hi[c], hi[c]);
         }
+        nodes[node].skip = skip;
         child = node;
         node = up;
     }
-}
-
-__global__ __launch_bounds__(256) void k_skip_links(int64_t n, Node *__restrict__ nodes, const int32_t *__restrict__ parent,
-                                                    const int32_t *__restrict__ right, WsHeader *h, const int32_t *gate = nullptr)
-{
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= 2 * n - 1 || gate_closed(gate)) return;
-    if (id == 0) h->built = 1; // (the last kernel of a build)
-    int32_t cur = (int32_t)id, skip = -1;
-    for (;;) {
-        const int32_t p = parent[cur];
-        if (p < 0) break;
-        if (nodes[p].left == cur) { skip = right[p]; break; }
-        cur = p;
-    }
-    nodes[id].skip = skip;
+    h->built = 1; // (the thread that has merged the root)
 }
 
 __global__ void k_mark_built(WsHeader *h, const int32_t *gate = nullptr) // of an empty scene
@@ -832,13 +841,11 @@ static int build_impl(const float *pos, const float *scale, const float *quat, c
         const int r = radix_sort<uint64_t>(k0, v0, k1, v1, n, 64, hist, s);
         if (r < 0) return r;
         // 8 passes: the sorted keys / permutation are back in (k0, v0)
-        hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, v0, n, nodes, parent, flags, v1); // (the sort's second value buffer is free again)
-        if (n > 1) {
-            int32_t *other_end = (int32_t *)k1; // the sort's second key buffer is free again
-            hipLaunchKernelGGL(k_karras, grid_for(n - 1, 256), dim3(256), 0, s, k0, n, nodes, parent, right, other_end);
-            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, flags);
-        }
-        hipLaunchKernelGGL(k_skip_links, grid_for(2 * n - 1, 256), dim3(256), 0, s, n, nodes, parent, right, hdr);
+        int32_t *other_end = (int32_t *)k1, *after = other_end + n; // the sort's second key buffer is free again
+        if (n > 1) hipLaunchKernelGGL(k_karras, grid_for(n - 1, 256), dim3(256), 0, s, k0, n, nodes, parent, right, other_end, after);
+        hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, v0, n, nodes, parent, flags, v1, after, hdr); // (the sort's second value buffer is free again)
+        if (n > 1)
+            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, after, flags, hdr);
     } else {
         hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr);
     }
@@ -873,9 +880,10 @@ extern "C" int rgx_refit_aabbs(const float *bboxes, int64_t n, void *ws, size_t 
     if (n > 0) {
         hipLaunchKernelGGL(k_take_boxes, grid_reduce(n, 256), dim3(RGX_REDUCE_THREADS), 0, s, bboxes, n, boxes, hdr->bb_min_enc, hdr->bb_max_enc, gate);
         hipLaunchKernelGGL(k_finish_bbox, dim3(1), dim3(64), 0, s, hdr, (float *)nullptr, (float *)nullptr, gate);
-        hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, order, n, nodes, parent, flags, (uint32_t *)(w + L.vals1), gate);
-        if (n > 1) hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, flags, gate);
-        hipLaunchKernelGGL(k_skip_links, grid_for(2 * n - 1, 256), dim3(256), 0, s, n, nodes, parent, right, hdr, gate);
+        const int32_t *after = other_end + n;
+        hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, order, n, nodes, parent, flags, (uint32_t *)(w + L.vals1), after, hdr, gate);
+        if (n > 1)
+            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, after, flags, hdr, gate);
     } else {
         hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr, gate);
     }
