@@ -630,9 +630,22 @@ __device__ __forceinline__ float ld_agent(const float *p)
     return __int_as_float(__hip_atomic_load((const int *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
+// Node `node` for the sweeps by pairs (NodePair): the thread that merges its children's boxes has both.  own: the child it came from.
+__device__ __forceinline__ void store_pair(NodePair *pairs, int64_t n, int32_t node, int32_t left, int32_t right, int own,
+                                           const float (&lo)[3], const float (&hi)[3], const float (&slo)[3], const float (&shi)[3])
+{
+    float4 *dst = (float4 *)(pairs + node);
+    auto id = [&](int32_t child) { return __int_as_float(child >= n - 1 ? ~(int32_t)(child - (n - 1)) : child); };
+    auto extent = [](float a, float b) { return fmaf(fabsf(a) + fabsf(b), 0x1p-22f, (b - a) * (1.0f + 0x1p-19f)); };
+    dst[2 * own] = make_float4(lo[0] + hi[0], lo[1] + hi[1], lo[2] + hi[2], own ? 0.f : id(left));
+    dst[2 * own + 1] = make_float4(extent(lo[0], hi[0]), extent(lo[1], hi[1]), extent(lo[2], hi[2]), own ? 0.f : id(right));
+    dst[2 - 2 * own] = make_float4(slo[0] + shi[0], slo[1] + shi[1], slo[2] + shi[2], own ? id(left) : 0.f);
+    dst[3 - 2 * own] = make_float4(extent(slo[0], shi[0]), extent(slo[1], shi[1]), extent(slo[2], shi[2]), own ? id(right) : 0.f);
+}
+
 __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int32_t *__restrict__ parent,
                                                const int32_t *__restrict__ right, const int32_t *__restrict__ other_end,
-                                               const int32_t *__restrict__ after, int32_t *flags,
+                                               const int32_t *__restrict__ after, int32_t *flags, NodePair *__restrict__ pairs,
                                                WsHeader *h, const int32_t *gate = nullptr)
 {
     __shared__ float s_box[2][6][256]; // [which child][lo xyz, hi xyz][node - first leaf of the workgroup]
@@ -668,6 +681,9 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
             slo[c] = s_box[1 - side][c][slot];
             shi[c] = s_box[1 - side][3 + c][slot];
         }
+        // (the children of a node meet between two neighbours of the sorted order: the right one starts where the left one ends)
+        const int32_t split = left >= n - 1 ? left - (int32_t)(n - 1) : left;
+        if (pairs) store_pair(pairs, n, node, left, (node < o ? o : node) == split + 1 ? (int32_t)(n - 1) + split + 1 : split + 1, side, lo, hi, slo, shi);
         for (int c = 0; c < 3; ++c) {
             lo[c] = fminf(lo[c], slo[c]);
             hi[c] = fmaxf(hi[c], shi[c]);
@@ -721,6 +737,7 @@ __global__ __launch_bounds__(256) void k_refit(int64_t n, Node *nodes, const int
             slo[c] = ld_agent(&sibling->lo[c]);
             shi[c] = ld_agent(&sibling->hi[c]);
         }
+        if (pairs) store_pair(pairs, n, node, left, rgt, left == child ? 0 : 1, lo, hi, slo, shi);
         for (int c = 0; c < 3; ++c) {
             lo[c] = fminf(lo[c], slo[c]);
             hi[c] = fmaxf(hi[c], shi[c]);
@@ -845,7 +862,7 @@ static int build_impl(const float *pos, const float *scale, const float *quat, c
         if (n > 1) hipLaunchKernelGGL(k_karras, grid_for(n - 1, 256), dim3(256), 0, s, k0, n, nodes, parent, right, other_end, after);
         hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, v0, n, nodes, parent, flags, v1, after, hdr); // (the sort's second value buffer is free again)
         if (n > 1)
-            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, after, flags, hdr);
+            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, after, flags, n <= RGX_PAIR_BOXES ? (NodePair *)(w + L.pairs) : nullptr, hdr);
     } else {
         hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr);
     }
@@ -883,7 +900,8 @@ extern "C" int rgx_refit_aabbs(const float *bboxes, int64_t n, void *ws, size_t 
         const int32_t *after = other_end + n;
         hipLaunchKernelGGL(k_leaves, grid_for(n, 256), dim3(256), 0, s, boxes, order, n, nodes, parent, flags, (uint32_t *)(w + L.vals1), after, hdr, gate);
         if (n > 1)
-            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, after, flags, hdr, gate);
+            hipLaunchKernelGGL(k_refit, grid_for(n, 256), dim3(256), 0, s, n, nodes, parent, right, other_end, after, flags,
+                               n <= RGX_PAIR_BOXES ? (NodePair *)(w + L.pairs) : nullptr, hdr, gate);
     } else {
         hipLaunchKernelGGL(k_mark_built, dim3(1), dim3(1), 0, s, hdr, gate);
     }

@@ -599,6 +599,35 @@ def test_forward_without_a_record_is_the_march_that_its_backward_repeats(gx, dyn
     assert np.array_equal(gx.gpu_render(np_scene, cam, cfg, stats=False)["image"], only.cpu().numpy())
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 129, 6000])
+@pytest.mark.parametrize("w,h", [(225, 224), (1088, 1083), (1096, 1084)])         # 812, 18 496 and 18 632 tiles: six rounds are 18 432
+@pytest.mark.parametrize("dyn", [False, True])
+def test_sweeps_by_pairs_of_nodes_and_by_nodes_find_the_same(gx, n, w, h, dyn):
+    """Trees from a single leaf up, either side of the number of tiles up to which an image that no backward follows
+    sweeps the tree by pairs of nodes: image and counters of the forward that goes by nodes.  Dense scenes fill several
+    tables.  (Sums in another order: 1e-5; adaptive: a ray may be re-phased.)"""
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.render_optix import compute_rgb
+    sc = gx.to_dev(scenes.scene_to_numpy(scenes.make_scene(2 if dyn else 0, n=n, sh_degree=0, seed=33)))
+    cam = scenes.make_camera(0, 1, width=w, height=h)
+    params = sc["positions"], sc["scales"] * 4.0, sc["quaternions"], sc["densities"]
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+    cs = u_ox.camera_struct(cam)
+    rgb = compute_rgb(cam.camera_center, sc["positions"], sc["color_features"], None, None, None, 0, 0)
+    prims = u_ox.pack_prims(gas, cs, *params, rgb)
+    a_st, b_st = u_ox.new_stats(gx.DEV), u_ox.new_stats(gx.DEV)
+    _step(f"pairs n={n} {w}x{h} adaptive {dyn}")
+    a = u_ox.march_forward(gas, cs, prims, 0.01, dyn, 4096, True, stats=a_st)
+    b = u_ox.launch_pipeline_test(None, None, gas, None, None, 0.01, dyn, cam, params[3], rgb, *params[:3], 4096, stats=b_st)
+    plain = u_ox.launch_pipeline_test(None, None, gas, None, None, 0.01, dyn, cam, params[3], rgb, *params[:3], 4096)
+    assert torch.equal(b, plain)
+    assert (a - b).abs().max() <= (5e-3 if dyn else 1e-5)
+    sa, sb = u_ox.read_stats(a_st), u_ox.read_stats(b_st)
+    assert (sa["hit_pairs"] > 0 or n < 64) and sa["rays_hit"] == sb["rays_hit"]
+    if not dyn:
+        assert sa["hit_pairs"] == sb["hit_pairs"] and sa["slabs"] == sb["slabs"]
+
+
 @pytest.mark.parametrize("w,h", [(52, 44), (216, 224)])
 def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     """What the four wavefronts of a tile leave for the backward, in each form: sample sums in floats and in half
