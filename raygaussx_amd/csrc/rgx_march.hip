@@ -89,6 +89,14 @@ struct MarchParams {
     uint32_t *ray_counts;   // counting forward only: per ray, slabs blended and the sum of their hit-list lengths; or null
 };
 
+// The kernel's arguments once more, from the kernel's argument segment: what is read through this is loaded where it is used.
+__device__ __forceinline__ const MarchParams &args_again()
+{
+    auto p = (const __attribute__((address_space(4))) MarchParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const MarchParams *)p;
+}
+
 // Section census (diagnostic builds only: -DRGX_SECTION_CLOCKS, `python -m raygaussx_amd.build --sections`;
 // the product library has none of it).  Every wave of a kernel launched without a statistics block keeps
 // one running time stamp; RGX_SEC(cn, k) adds the cycles since the previous stamp to section k, so the
@@ -576,10 +584,13 @@ __device__ __forceinline__ void frustum_cut_pairs(const MarchParams &P, Frustum 
 
 // Fills the table from the sweep; returns the number of entries.  done: the sweep is finished;
 // plain: every entry passed plain_roots().
+// AGAIN: the descent reads its arguments once more for every table (args_again) and does not hold them, or spill them, across the marches
+// between: images by pairs (300 k Gaussians 800x800 with lobes 2.284 -> 2.245 ms, viewer 1 M 1280x720 6.06 -> 6.00).  Not where it loses: the
+// recording forward (300 k 800x800 2.67 -> 2.71) and images by nodes (3 M 1920x1080 16.2 -> 16.4).
 // PAIRS: the descent opens 64 internal nodes a step and tests both children of each, so it takes half as many steps, each one
 // trip to memory; leaves never enter the stack.  It finds the Gaussians in another order, so only marches whose sums may be taken
 // in any order go this way (launch_forward).
-template <bool PAIRS, typename Cn>
+template <bool PAIRS, bool AGAIN, typename Cn>
 __device__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab,
                           bool &done, bool &plain, Cn &cn)
 {
@@ -588,17 +599,20 @@ __device__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int3
     const float4 *nodes4 = (const float4 *)P.nodes;
     const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
     int C = 0;
+    const MarchParams *again = &P;
     while (C < RGX_CCAP) {
+        if constexpr (AGAIN) again = &args_again();
         while (S.qn > 0 && S.lqn < 64) {
             // A step of the descent: up to 64 nodes, one per lane.  (Lanes beyond them repeat the last one, and their results are
             // masked: straight-line code.  The wavefront's LDS accesses take place in program order.)
             const int m = S.qn > RGX_QCAP - RGX_DFS_MARGIN ? 1 : (S.qn < 64 ? S.qn : 64);
             const int base = S.qn - m;
             if constexpr (PAIRS) {
-                const int32_t top = (int32_t)P.n - 2; // the last internal node (with fewer than two Gaussians the stack stays empty)
+                const MarchParams &A = AGAIN ? *again : P;
+                const int32_t top = (int32_t)A.n - 2; // the last internal node (with fewer than two Gaussians the stack stays empty)
                 const uint32_t popped = (uint32_t)s_queue[base + min(lane, m - 1)], node = min(popped, (uint32_t)top);
                 __builtin_amdgcn_wave_barrier();
-                const float4 *q = (const float4 *)((const char *)P.pairs + ((uint64_t)node << 6));
+                const float4 *q = (const float4 *)((const char *)A.pairs + ((uint64_t)node << 6));
                 const float4 a = q[0], b = q[1], c = q[2], d = q[3];
                 const int32_t left = __float_as_int(a.w), right = __float_as_int(b.w);
                 const uint64_t here = (~0ull >> (64 - m)) & __ballot(popped <= (uint32_t)top);
@@ -1844,7 +1858,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 more = false;
             } else {
                 bool done;
-                C = sweep_next<PAIRS>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
+                C = sweep_next<PAIRS, PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
                 if (split) {
                     seen += C;
                 } else if (phase == 0 && first) {
