@@ -3612,12 +3612,6 @@ __global__ __launch_bounds__(256) void k_tile_order(const MarchParams P)
 // heavy and light blocks and starts with its heaviest.  A block's tiles still run next to each
 // other on one XCD (what its L2 is shared for); only the order of the blocks changes.
 // Layout of the list memory: order[8 * per_xcd], then cost[blocks].
-__global__ __launch_bounds__(256) void k_zero_u32(uint32_t *p, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
-}
-
 // (A workgroup takes a run of consecutive Gaussians and counts in LDS first: the adds of all workgroups to the few
 // blocks in the middle of the image, one after the other in memory, were three quarters of this kernel's time.)
 #define RGX_COST_BINS 2048
@@ -3790,18 +3784,23 @@ __global__ __launch_bounds__(256) void k_unpermute_grads(const float4 *__restric
     dquat[4 * i] = c.z; dquat[4 * i + 1] = c.w; dquat[4 * i + 2] = d.x; dquat[4 * i + 3] = d.y;
 }
 
-__global__ __launch_bounds__(256) void k_zero4(float4 *p, int64_t n4)
+// Clears what a launch starts from, in one kernel: a launch of its own for a few words takes 4.5 us (4 k Gaussians 128x128: two of 24 launches).
+// A backward: the gradient block, and the count of this launch's replays that lost their record (or null).
+__global__ __launch_bounds__(256) void k_clear_backward(float4 *p, int64_t n4, uint32_t *lost)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n4) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i == 0 && lost) *lost = 0u;
 }
 
-// Clears the 16 bytes at a and at b (either may be null): the bump counter of the record's
-// sample-sum pool and the workspace's fault counters, at the start of a forward launch.
-__global__ __launch_bounds__(64) void k_clear2(float4 *a, float4 *b)
+// A forward: the 16 bytes at a and at b (either may be null), the bump counter of the record's sample-sum pool and the
+// workspace's fault counters; and n words at cost.
+__global__ __launch_bounds__(256) void k_clear_forward(float4 *a, float4 *b, uint32_t *cost, int n)
 {
-    if (threadIdx.x == 0 && a) *a = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (threadIdx.x == 1 && b) *b = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0 && a) *a = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i == 1 && b) *b = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < n) cost[i] = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -3943,21 +3942,23 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
     return RGX_OK;
 }
 
-// Launch order of a forward: blocks of tiles by their estimated weight (k_block_cost, k_block_order), when the
-// workspace has room for the lists.
-static void order_blocks(MarchParams &P, hipStream_t s)
+// What precedes a forward's march: counters cleared, and its launch order: blocks of tiles by their estimated weight (k_block_cost,
+// k_block_order), when the workspace has room for the lists.
+static void prepare_forward(MarchParams &P, bool team, hipStream_t s)
 {
     // The order only matters for the end of a launch, where ever fewer tiles still run: with many
     // rounds of tiles per wave slot (3072 slots: 12 per CU) that end is a small part of the launch
     // and the pass over the primitive records takes what it brings (forward without -> with the order: 1 M Gaussians at
     // 800x800, 3.3 rounds: 5.51 -> 5.32 ms; 300 k there 2.84 -> 2.82; 3 M at 1237x822, 5.2 rounds: 9.71 -> 9.67; 3 M at
-    // 1920x1080, 10.5 rounds: 17.12 -> 17.09).
-    if (!P.tile_order || P.n == 0 || (int64_t)P.tiles_x * P.tiles_y > 6 * 3072) return;
+    // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every tile has a CU of its own, and starts at once.
+    const int64_t tiles = (int64_t)P.tiles_x * P.tiles_y;
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);
-    uint32_t *order = P.tile_order, *cost = P.tile_order + 8 * g.per_xcd;
-    hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, cost, nb);
-    if (nb > RGX_COST_BINS) return; // (a very long, thin image: as launched)
+    const bool ordered = P.tile_order && P.n > 0 && tiles <= 6 * 3072 && !(team && tiles <= 256) && nb <= RGX_COST_BINS; // (more blocks: a very long, thin image)
+    uint32_t *order = P.tile_order, *cost = ordered ? P.tile_order + 8 * g.per_xcd : nullptr;
+    if (P.sum_next || P.faults || ordered)
+        hipLaunchKernelGGL(k_clear_forward, dim3(ordered ? (unsigned)((nb + 255) / 256) : 1u), dim3(256), 0, s, (float4 *)P.sum_next, (float4 *)P.faults, cost, ordered ? nb : 0);
+    if (!ordered) return;
     const int per_group = (int)((((P.n + 511) / 512) + 255) / 256 * 256); // 512 workgroups at most, whole waves
     hipLaunchKernelGGL(k_block_cost, dim3((unsigned)((P.n + per_group - 1) / per_group)), dim3(256), 0, s, P, cost, nb, per_group);
     hipLaunchKernelGGL(k_block_order, dim3(1), dim3(1024), 0, s, P, cost, order);
@@ -3999,11 +4000,15 @@ static inline dim3 march_grid(const MarchParams &P)
 // 800x800 2.77 / 2.66 ms, its frame with lobes 2.38 / 2.27, 1 M 800x800 5.28 / 5.19, viewer 1 M 1280x720 6.08 / 6.06; 3 M
 // 1920x1080, 10.5 rounds, 16.88 / 16.96).
 #define RGX_PAIR_TILES (6 * 3072)
-// half: the record's colour sums are in half precision; image_only: no backward follows this launch
+// image_only: no backward follows this launch
+static bool sums_in_any_order(const MarchParams &P, bool image_only) { return image_only || (P.records && !P.m.dynamic_sampling); }
+static bool by_team(const MarchParams &P, bool image_only) { return P.tiles_x * P.tiles_y <= RGX_TEAM_TILES && sums_in_any_order(P, image_only); }
+
+// half: the record's colour sums are in half precision
 static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, bool image_only, hipStream_t s)
 {
-    const bool any_order = image_only || (P.records && !P.m.dynamic_sampling);
-    const bool team = P.tiles_x * P.tiles_y <= RGX_TEAM_TILES && any_order, pairs = any_order && P.n <= RGX_PAIR_BOXES && P.tiles_x * P.tiles_y <= RGX_PAIR_TILES;
+    const bool any_order = sums_in_any_order(P, image_only);
+    const bool team = by_team(P, image_only), pairs = any_order && P.n <= RGX_PAIR_BOXES && P.tiles_x * P.tiles_y <= RGX_PAIR_TILES;
     const dim3 grid = march_grid(P), block(team ? 256 : 64);
 #define RGX_FWD(...)                                                                            \
     do {                                                                                        \
@@ -4069,8 +4074,7 @@ static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxM
     P.ray_counts = ray_counts;
     const bool counting = stats != nullptr || ray_counts != nullptr;
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
-    if (P.sum_pool || P.faults) hipLaunchKernelGGL(k_clear2, dim3(1), dim3(64), 0, (hipStream_t)stream, (float4 *)P.sum_next, (float4 *)P.faults);
-    order_blocks(P, (hipStream_t)stream);
+    prepare_forward(P, by_team(P, image_only), (hipStream_t)stream);
     const bool half = P.sum_pool && P.m.record_format == 1;
     launch_forward(P, false, counting, half, image_only, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
@@ -4089,8 +4093,7 @@ extern "C" int rgx_march_viewer(const void *ws, const RgxCamera *cam, const RgxM
     P.frame = frame;
     P.depth = depth;
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
-    if (P.faults) hipLaunchKernelGGL(k_clear2, dim3(1), dim3(64), 0, (hipStream_t)stream, (float4 *)nullptr, (float4 *)P.faults);
-    order_blocks(P, (hipStream_t)stream);
+    prepare_forward(P, by_team(P, true), (hipStream_t)stream);
     launch_forward(P, true, stats != nullptr, false, true, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
     RGX_LAUNCH_CHECK();
@@ -4177,8 +4180,7 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
     P.fwd_colors = ray_colors;
     P.dloss = dloss;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_zero4, grid_for(4 * n, 256), dim3(256), 0, s, (float4 *)P.gbuf, 4 * n);
-    if (P.faults) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, P.faults, 1); // this launch's replays that lost their record
+    hipLaunchKernelGGL(k_clear_backward, grid_for(4 * n, 256), dim3(256), 0, s, (float4 *)P.gbuf, 4 * n, P.faults);
     void *span = timed ? rgx_span_begin(RGX_T_MARCH_BWD, s) : nullptr;
     if (P.records) {
         // tiles with a complete record replay it; the few whose record overflowed are recomputed
