@@ -400,7 +400,8 @@ __global__ __launch_bounds__(RGX_RS_THREADS) void k_rs_pass(const K *__restrict_
 // above take for them is the latency of their launches, 24 for 64-bit keys (building the tree over 4 096 boxes
 // 181 us, with this 98; over 8 192 185 and 125; with a bitonic network, which moves every key through LDS 78 and 91 times
 // instead of 8, 117 and 177).  Each wavefront has a run
-// of the keys, and ranks 64 at a time as k_rs_scatter does.  The limit is what fits LDS (12 bytes a key, and 16 KB of counters).
+// of the keys, and ranks 64 at a time as k_rs_scatter does; it ranks as it counts, one lane of each digit adding for all of them (an add per key
+// to the counters first: a build of 4 096 boxes 110 -> 107 us, of 8 192 140 -> 135).  The limit is what fits LDS (12 bytes a key, and 16 KB of counters).
 template <typename K>
 __global__ __launch_bounds__(1024) void k_sort_small(K *__restrict__ keys, uint32_t *__restrict__ vals, int n, int bits)
 {
@@ -423,9 +424,27 @@ __global__ __launch_bounds__(1024) void k_sort_small(K *__restrict__ keys, uint3
     for (int shift = 0; shift < bits; shift += 8) {
         for (int d = lane; d < 256; d += 64) cnt[wave][d] = 0;
         __builtin_amdgcn_wave_barrier();
+        // a key's place in its wavefront's run of its digit: keys of the digit in earlier rounds, then in lower lanes
+        uint32_t place[ITEMS];
+        auto *cur = (__attribute__((address_space(3))) uint32_t *)cnt[wave];
 #pragma unroll
-        for (int r = 0; r < ITEMS; ++r)
-            if (r < rounds && base + r * 64 + lane < n) atomicAdd(&cnt[wave][(uint32_t)(key[r] >> shift) & 255u], 1u);
+        for (int r = 0; r < ITEMS; ++r) {
+            if (r >= rounds) break;
+            const bool valid = base + r * 64 + lane < n;
+            const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+            uint64_t same = __ballot(valid);
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t bal = __ballot(bit);
+                same &= bit ? bal : ~bal;
+            }
+            const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
+            const uint32_t before = __hip_atomic_load(cur + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            place[r] = before + rank;
+            __builtin_amdgcn_wave_barrier();
+            if (valid && rank == 0) __hip_atomic_store(cur + d, before + (uint32_t)__popcll(same), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            __builtin_amdgcn_wave_barrier();
+        }
         __syncthreads();
         // where each (digit, wave) run starts: digits before waves
         uint32_t total = 0, upto = 0;
@@ -449,28 +468,13 @@ __global__ __launch_bounds__(1024) void k_sort_small(K *__restrict__ keys, uint3
             }
         }
         __syncthreads();
-        volatile uint32_t *cur = cnt[wave];
 #pragma unroll
-        for (int r = 0; r < ITEMS; ++r) {
-            if (r >= rounds) break;
-            const bool valid = base + r * 64 + lane < n;
-            const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
-            uint64_t same = __ballot(valid);
-            for (int b = 0; b < 8; ++b) {
-                const bool bit = (d >> b) & 1u;
-                const uint64_t bal = __ballot(bit);
-                same &= bit ? bal : ~bal;
-            }
-            const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
-            if (valid) {
-                const uint32_t at = cur[d] + rank;
+        for (int r = 0; r < ITEMS; ++r)
+            if (r < rounds && base + r * 64 + lane < n) {
+                const uint32_t at = cnt[wave][(uint32_t)(key[r] >> shift) & 255u] + place[r];
                 lkey[at] = key[r];
                 lval[at] = val[r];
             }
-            __builtin_amdgcn_wave_barrier();
-            if (valid && rank == 0) cur[d] += __popcll(same);
-            __builtin_amdgcn_wave_barrier();
-        }
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < ITEMS; ++r) {
