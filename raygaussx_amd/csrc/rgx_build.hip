@@ -241,16 +241,32 @@ __device__ __forceinline__ void rs_scatter_tile(const K *__restrict__ kin, const
     // wave w owns the contiguous 64 ITEMS keys from base, 64 per round
     const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)wave * (64 * ITEMS);
     K key[ITEMS];
-    uint32_t val[ITEMS];
+    uint32_t val[ITEMS], place[ITEMS]; // place: in the wave's run of the key's digit
+#pragma unroll
     for (int r = 0; r < ITEMS; ++r) {
         const int64_t i = base + r * 64 + lane;
-        key[r] = 0;
-        val[r] = 0;
-        if (i < n) {
-            key[r] = kin[i];
-            val[r] = vin[i];
-            atomicAdd(&cnt[wave][(uint32_t)(key[r] >> shift) & 255u], 1u);
+        key[r] = i < n ? kin[i] : (K)0;
+        val[r] = i < n ? vin[i] : 0u;
+    }
+    // Ranked as they are counted: the lanes of a digit find each other by ballots, and the first of them adds for all.  (An add per key to
+    // the counters, and the ranking in a second pass over the keys: order of 1 M points 99 -> 90 us; a build of 150 k boxes 212 -> 205, 3 M 920 -> 885.)
+    auto *cur = (__attribute__((address_space(3))) uint32_t *)cnt[wave];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool valid = base + r * 64 + lane < n;
+        const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
+        uint64_t same = __ballot(valid);
+        for (int b = 0; b < 8; ++b) {
+            const bool bit = (d >> b) & 1u;
+            const uint64_t bal = __ballot(bit);
+            same &= bit ? bal : ~bal;
         }
+        const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
+        const uint32_t earlier = __hip_atomic_load(cur + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        place[r] = earlier + rank;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0) __hip_atomic_store(cur + d, earlier + (uint32_t)__popcll(same), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
     // The tile's keys are put in digit order in LDS first and leave from there: keys of one digit are neighbours
@@ -281,27 +297,13 @@ __device__ __forceinline__ void rs_scatter_tile(const K *__restrict__ kin, const
         }
     }
     __syncthreads();
-    volatile uint32_t *cur = cnt[wave];
-    for (int r = 0; r < ITEMS; ++r) {
-        const int64_t i = base + r * 64 + lane;
-        const bool valid = i < n;
-        const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
-        uint64_t same = __ballot(valid);
-        for (int b = 0; b < 8; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t bal = __ballot(bit);
-            same &= bit ? bal : ~bal;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+        if (base + r * 64 + lane < n) {
+            const uint32_t at = cnt[wave][(uint32_t)(key[r] >> shift) & 255u] + place[r];
+            lkey[at] = key[r];
+            lval[at] = val[r];
         }
-        if (valid) {
-            const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
-            const uint32_t off = cur[d];
-            lkey[off + rank] = key[r];
-            lval[off + rank] = val[r];
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (valid && (same & ((1ull << lane) - 1ull)) == 0) cur[d] += __popcll(same);
-        __builtin_amdgcn_wave_barrier();
-    }
     __syncthreads();
     const int64_t tile_base = (int64_t)blockIdx.x * TILE;
     const int tile_n = (int)(n - tile_base < TILE ? n - tile_base : TILE);
