@@ -81,6 +81,7 @@ struct MarchParams {
     uint32_t *tile_order;   // launch order lists (or null: as launched)
     int32_t use_tile_order; // 0: as launched; 1: per XCD, its tiles' list positions from the heaviest to the lightest (k_tile_order);
                             // 2: per XCD, the blocks of tiles it renders, heaviest first (k_block_order)
+    int32_t by_halves;      // forward of an image: two workgroups per tile (launch_forward)
     float4 *sum_pool;       // sample-sum slots of the record (RGX_SUM_SLOT_WORDS each), or null
     uint32_t *sum_next;     // next free slot (bump counter in the record's pool header)
     int32_t sum_slots;      // slots in the pool
@@ -303,11 +304,12 @@ __device__ __forceinline__ f3 plane_normal(f3 a, f3 b, f3 inside)
     return dot3(n, inside) > 0.f ? n * -1.0f : n;
 }
 
-__device__ __forceinline__ void frustum_planes(const RgxCamera &cam, int px0, int py0, Frustum &F)
+// height: of the tile, in pixels (a half tile's is 4)
+__device__ __forceinline__ void frustum_planes(const RgxCamera &cam, int px0, int py0, Frustum &F, int height = 8)
 {
     const f3 d00 = compute_ray(cam, (unsigned)px0, (unsigned)py0), d10 = compute_ray(cam, (unsigned)(px0 + 7), (unsigned)py0);
-    const f3 d01 = compute_ray(cam, (unsigned)px0, (unsigned)(py0 + 7));
-    const f3 d11 = compute_ray(cam, (unsigned)(px0 + 7), (unsigned)(py0 + 7));
+    const f3 d01 = compute_ray(cam, (unsigned)px0, (unsigned)(py0 + height - 1));
+    const f3 d11 = compute_ray(cam, (unsigned)(px0 + 7), (unsigned)(py0 + height - 1));
     const f3 in = (d00 + d10) + (d01 + d11);
     F.o = mk3(cam.eye[0], cam.eye[1], cam.eye[2]);
     F.n[0] = plane_normal(d00, d01, in);
@@ -718,12 +720,16 @@ __host__ __device__ __forceinline__ TileGrid tile_grid(int tiles_x, int tiles_y)
     g.per_xcd = (g.blocks_x * blocks_y + 7) >> 3;
     return g;
 }
-__device__ __forceinline__ bool tile_origin(const MarchParams &P, unsigned id, int &px0, int &py0, int *tile_out = nullptr)
+__device__ __forceinline__ bool tile_origin(const MarchParams &P, unsigned id, int &px0, int &py0, int *tile_out = nullptr, int *half = nullptr)
 {
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int xcd = id & 7;
     const int per_block = g.bw * g.bh;
     int j = id >> 3;
+    if (half && P.by_halves) { // upper 0, lower 1
+        *half = j & 1;
+        j >>= 1;
+    }
     int block;
     if (P.use_tile_order == 2) {
         block = (int)P.tile_order[xcd * g.per_xcd + j / per_block];
@@ -2076,17 +2082,17 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
 {
     static_assert(RECORD || !HALF, "the colour sums' format is a property of the record");
     RGX_TILE_LDS(PAIRS);
-    int px0, py0, tile;
-    if (!tile_origin(P, blockIdx.x, px0, py0, &tile)) return; // whole wave
+    int px0, py0, tile, half = -1;
+    if (!tile_origin(P, blockIdx.x, px0, py0, &tile, RECORD ? nullptr : &half)) return; // whole wave
     typename std::conditional<RECORD, Recorder, NoRecorder>::type rec;
     if constexpr (RECORD) rec = Recorder{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
     int px, py;
     lane_pixel(px0, py0, px, py);
-    const bool valid = px < P.cam.width && py < P.cam.height;
+    const bool valid = px < P.cam.width && py < P.cam.height && (RECORD || half < 0 || (int)(threadIdx.x >> 5) == half); // (lanes 0-31: the upper half)
     CountersFor<STATS> cn;
     RGX_SEC_START(cn, 0);
     Frustum F;
-    frustum_planes(P.cam, px0, py0, F);
+    frustum_planes(P.cam, px0, half == 1 ? py0 + 4 : py0, F, half < 0 ? 8 : 4);
     RayState R;
     ray_begin<false>(P, px, py, valid, R);
     {
@@ -3901,6 +3907,7 @@ static int fill_params(MarchParams &P, const void *ws, const RgxCamera *cam, con
     const size_t order_words = (size_t)8 * g.per_xcd * g.bw * g.bh;
     P.tile_order = M.order + order_words * sizeof(uint32_t) <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.order) : nullptr;
     P.use_tile_order = 0;
+    P.by_halves = 0;
     P.faults = M.order <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.faults) : nullptr;
     P.ray_counts = nullptr;
     P.sum_pool = nullptr;
@@ -3942,9 +3949,55 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
     return RGX_OK;
 }
 
+// Up to this many tiles four wavefronts march a tile (k_march_team), beyond it one.  The team's wavefronts repeat the
+// per-iteration work that one wavefront does once for 64 rays, so it loses where the chip is full anyway; with few tiles
+// the launch is one tile's latency.  Measured, ms of a frame with one wavefront / with four:
+//     tiles                                      256          625          784         1 024        1 600        2 500
+//     fixed step, 4 k Gaussians in a cube    1.04 / 0.55  0.83 / 0.47  0.76 / 0.44  0.71 / 0.43  0.68 / 0.55  0.61 / 0.76
+//     fixed step, 100 k in a ball            4.32 / 2.38  2.54 / 1.58  2.51 / 1.54  2.24 / 1.36  1.68 / 1.20  1.35 / 1.03
+//     adaptive step, 60 k heavy-tailed       1.85 / 1.21  1.14 / 1.02  1.14 / 1.01  1.04 / 1.07  0.97 / 1.58  0.89 / 2.19
+//     adaptive step, 3 M heavy-tailed        9.77 / 4.00  6.73 / 4.53  5.84 / 4.16  5.83 / 4.07  4.57 / 5.59  4.44 / 7.03
+// Images stop at 768 tiles, below the first loss of any of them (the adaptive frames at 1 024): from there half tiles take over (RGX_HALF_TILES).
+// Records of the fixed step have no such losses up to 1 024 tiles (forward at 1 024, one / four: 4 k in a cube 0.76 / 0.50, 100 k in a ball
+// 1.97 / 1.28, 1 M in a ball of radius 2 5.64 / 5.15).
+//
+// Which launches: those whose image is the end of it (rgx_march_test, the viewer), and those that leave a record
+// with the fixed step.  The team adds up a sample's hits in another order, and where max_prim_slice cuts a ray's list it
+// keeps other hits, equally exact both.
+//   No record: the backward searches the tree again, one wavefront per tile, and has to meet the hits and the
+//     transmittance of the forward: that is k_march_fwd then, whatever the step.
+//   A record and the adaptive step: the next step's length depends on the last bit of the transmittance, and a sample that
+//     so crosses a Gaussian's cut-off moves that Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians):
+//     no longer the gradients that larger images give.  k_march_fwd.
+//   A record and the fixed step: what the backward replays is what the team recorded.  (A tile whose region overflowed is
+//     searched again; if max_prim_slice also cut lists in it, they may be cut to other hits there.)
+#ifndef RGX_TEAM_TILES
+#define RGX_TEAM_TILES 768
+#endif
+#define RGX_TEAM_TILES_RECORD 1024
+// Images of so few tiles beyond those are marched by halves of tiles, 8x4 pixels: a wavefront for each, half of whose lanes idle.  A launch in which
+// every wavefront starts at once lasts as long as its longest, and one with half the rays meets fewer Gaussians in a narrower
+// frustum, and walks shorter lists.  Measured, ms of a frame by whole tiles / by halves:
+//     tiles                                      961          1 024          1 296          1 521          2 500
+//     fixed step, 4 k Gaussians in a cube    0.71 / 0.55    0.68 / 0.59    0.65 / 0.53    0.68 / 0.57    0.59 / 0.53
+//     fixed step, 100 k in a ball            2.06 / 1.14    1.78 / 1.47    1.59 / 1.33    1.59 / 1.09
+//     fixed step, 1 M in a ball of radius 2  5.14 / 3.35    5.14 / 3.27    4.43 / 3.00    3.97 / 2.69    3.24 / 3.10
+//     adaptive step, 60 k heavy-tailed       0.96 / 0.76    0.98 / 0.76    0.90 / 0.80    0.86 / 0.88    0.85 / 1.13
+//     adaptive step, 3 M heavy-tailed        4.52 / 3.75    4.42 / 3.62    4.25 / 3.57    3.93 / 4.45    3.55 / 4.97
+// The line lies below the first loss.  (Halves for the heaviest blocks only of an image with more tiles: 300 k 800x800 2.25 -> 2.73 ms for
+// 512 tiles of 10 000.)  Between 400 and 768 tiles four wavefronts per tile and halves win in turn.  A record is tile by tile.
+#define RGX_HALF_TILES 1296
+
+// image_only: no backward follows this launch
+static bool sums_in_any_order(const MarchParams &P, bool image_only) { return image_only || (P.records && !P.m.dynamic_sampling); }
+static bool by_team(const MarchParams &P, bool image_only)
+{
+    return P.tiles_x * P.tiles_y <= (image_only ? RGX_TEAM_TILES : RGX_TEAM_TILES_RECORD) && sums_in_any_order(P, image_only);
+}
+
 // What precedes a forward's march: counters cleared, and its launch order: blocks of tiles by their estimated weight (k_block_cost,
 // k_block_order), when the workspace has room for the lists.
-static void prepare_forward(MarchParams &P, bool team, hipStream_t s)
+static void prepare_forward(MarchParams &P, bool image_only, hipStream_t s)
 {
     // The order only matters for the end of a launch, where ever fewer tiles still run: with many
     // rounds of tiles per wave slot (3072 slots: 12 per CU) that end is a small part of the launch
@@ -3952,6 +4005,8 @@ static void prepare_forward(MarchParams &P, bool team, hipStream_t s)
     // 800x800, 3.3 rounds: 5.51 -> 5.32 ms; 300 k there 2.84 -> 2.82; 3 M at 1237x822, 5.2 rounds: 9.71 -> 9.67; 3 M at
     // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every tile has a CU of its own, and starts at once.
     const int64_t tiles = (int64_t)P.tiles_x * P.tiles_y;
+    const bool team = by_team(P, image_only);
+    P.by_halves = image_only && !team && tiles <= RGX_HALF_TILES;
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);
     const bool ordered = P.tile_order && P.n > 0 && tiles <= 6 * 3072 && !(team && tiles <= 256) && nb <= RGX_COST_BINS; // (more blocks: a very long, thin image)
@@ -3968,42 +4023,14 @@ static void prepare_forward(MarchParams &P, bool team, hipStream_t s)
 static inline dim3 march_grid(const MarchParams &P)
 {
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
-    return dim3((unsigned)(8 * g.per_xcd * g.bw * g.bh));
+    return dim3((unsigned)(8 * g.per_xcd * g.bw * g.bh) << P.by_halves);
 }
 
-// Up to this many tiles four wavefronts march a tile (k_march_team), beyond it one.  The team's wavefronts repeat the
-// per-iteration work that one wavefront does once for 64 rays, so it loses where the chip is full anyway; with few tiles
-// the launch is one tile's latency.  Measured, ms of a frame with one wavefront / with four:
-//     tiles                                      256          625          784         1 024        1 600        2 500
-//     fixed step, 4 k Gaussians in a cube    1.04 / 0.55  0.83 / 0.47  0.76 / 0.44  0.71 / 0.43  0.68 / 0.55  0.61 / 0.76
-//     fixed step, 100 k in a ball            4.32 / 2.38  2.54 / 1.58  2.51 / 1.54  2.24 / 1.36  1.68 / 1.20  1.35 / 1.03
-//     adaptive step, 60 k heavy-tailed       1.85 / 1.21  1.14 / 1.02  1.14 / 1.01  1.04 / 1.07  0.97 / 1.58  0.89 / 2.19
-//     adaptive step, 3 M heavy-tailed        9.77 / 4.00  6.73 / 4.53  5.84 / 4.16  5.83 / 4.07  4.57 / 5.59  4.44 / 7.03
-// One line for all launches, below the first loss of any of them (the adaptive frames at 1 024 tiles).  It is not where
-// the fixed step crosses over: that gains up to some 1 600 tiles.
-//
-// Which launches: those whose image is the end of it (rgx_march_test, the viewer), and those that leave a record
-// with the fixed step.  The team adds up a sample's hits in another order, and where max_prim_slice cuts a ray's list it
-// keeps other hits, equally exact both.
-//   No record: the backward searches the tree again, one wavefront per tile, and has to meet the hits and the
-//     transmittance of the forward: that is k_march_fwd then, whatever the step.
-//   A record and the adaptive step: the next step's length depends on the last bit of the transmittance, and a sample that
-//     so crosses a Gaussian's cut-off moves that Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians):
-//     no longer the gradients that larger images give.  k_march_fwd.
-//   A record and the fixed step: what the backward replays is what the team recorded.  (A tile whose region overflowed is
-//     searched again; if max_prim_slice also cut lists in it, they may be cut to other hits there.)
-#ifndef RGX_TEAM_TILES
-#define RGX_TEAM_TILES 768
-#endif
 // Sweeps by pairs of nodes: the same launches, up to six rounds of tiles, over trees that have them.  A tile's own time gets shorter, which is what a launch with
 // few rounds lasts; with many rounds the wavefronts hide each other's trips to memory (forward by nodes / by pairs: 300 k Gaussians
 // 800x800 2.77 / 2.66 ms, its frame with lobes 2.38 / 2.27, 1 M 800x800 5.28 / 5.19, viewer 1 M 1280x720 6.08 / 6.06; 3 M
 // 1920x1080, 10.5 rounds, 16.88 / 16.96).
 #define RGX_PAIR_TILES (6 * 3072)
-// image_only: no backward follows this launch
-static bool sums_in_any_order(const MarchParams &P, bool image_only) { return image_only || (P.records && !P.m.dynamic_sampling); }
-static bool by_team(const MarchParams &P, bool image_only) { return P.tiles_x * P.tiles_y <= RGX_TEAM_TILES && sums_in_any_order(P, image_only); }
-
 // half: the record's colour sums are in half precision
 static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, bool image_only, hipStream_t s)
 {
@@ -4074,7 +4101,7 @@ static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxM
     P.ray_counts = ray_counts;
     const bool counting = stats != nullptr || ray_counts != nullptr;
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
-    prepare_forward(P, by_team(P, image_only), (hipStream_t)stream);
+    prepare_forward(P, image_only, (hipStream_t)stream);
     const bool half = P.sum_pool && P.m.record_format == 1;
     launch_forward(P, false, counting, half, image_only, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
@@ -4093,7 +4120,7 @@ extern "C" int rgx_march_viewer(const void *ws, const RgxCamera *cam, const RgxM
     P.frame = frame;
     P.depth = depth;
     void *span = rgx_span_begin(RGX_T_MARCH_FWD, (hipStream_t)stream);
-    prepare_forward(P, by_team(P, true), (hipStream_t)stream);
+    prepare_forward(P, true, (hipStream_t)stream);
     launch_forward(P, true, stats != nullptr, false, true, (hipStream_t)stream);
     rgx_span_end(span, (hipStream_t)stream);
     RGX_LAUNCH_CHECK();

@@ -600,7 +600,7 @@ def test_forward_without_a_record_is_the_march_that_its_backward_repeats(gx, dyn
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 129, 6000])
-@pytest.mark.parametrize("w,h", [(225, 224), (1088, 1083), (1096, 1084)])         # 812, 18 496 and 18 632 tiles: six rounds are 18 432
+@pytest.mark.parametrize("w,h", [(225, 224), (285, 281), (289, 288), (1088, 1083), (1096, 1084)])   # 812 and 1 296 tiles, by halves; 1 332; 18 496 and 18 632: six rounds are 18 432
 @pytest.mark.parametrize("dyn", [False, True])
 def test_sweeps_by_pairs_of_nodes_and_by_nodes_find_the_same(gx, n, w, h, dyn):
     """Trees from a single leaf up, either side of the number of tiles up to which an image that no backward follows
@@ -625,10 +625,15 @@ def test_sweeps_by_pairs_of_nodes_and_by_nodes_find_the_same(gx, n, w, h, dyn):
     sa, sb = u_ox.read_stats(a_st), u_ox.read_stats(b_st)
     assert (sa["hit_pairs"] > 0 or n < 64) and sa["rays_hit"] == sb["rays_hit"]
     if not dyn:
-        assert sa["hit_pairs"] == sb["hit_pairs"] and sa["slabs"] == sb["slabs"]
+        # (A ray whose transmittance is within rounding of its end: it ends a slab earlier or later, some hundred hits.  A tile with more
+        # Gaussians in a slab than its table holds does not look for second-half hits of rays that have ended in the first, and
+        # half a tile has fewer: by halves the counts of the 6 000 differ by those.)
+        assert abs(sa["slabs"] - sb["slabs"]) <= 1
+        more = sb["hit_pairs"] - sa["hit_pairs"]
+        assert more == 0 if n < 6000 else abs(more) <= 100 if w > 288 else 0 <= more <= 0.01 * sa["hit_pairs"]
 
 
-@pytest.mark.parametrize("w,h", [(52, 44), (216, 224)])
+@pytest.mark.parametrize("w,h", [(52, 44), (216, 224), (253, 256)])              # 1 024 tiles: the most that four wavefronts march
 def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     """What the four wavefronts of a tile leave for the backward, in each form: sample sums in floats and in half
     precision, and hit lists alone.  The image does not depend on the form.  Float sums and lists give the gradients of
