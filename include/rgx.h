@@ -199,7 +199,7 @@ int rgx_march_forward(const void *ws, const RgxCamera *cam, const RgxMarch *marc
 
 /* Replaces launch_pipeline_test (optix_utils.py:503-601): rgx_march_forward without a record, for an image
  * that no backward follows.  A backward without a record marches the rays once more and has to meet the
- * forward's samples and hits again; this launch need not be met, so small images may go through a kernel that
+ * forward's samples and hits again; this launch need not be met, so it may go through a kernel that
  * adds up a sample's hits, and cuts a list at max_prim_slice, in another order (equally exact). */
 int rgx_march_test(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims,
                    int64_t n, float *ray_colors, void *march_ws, size_t march_ws_bytes, RgxStats *stats, void *stream);
