@@ -216,7 +216,9 @@ int rgx_march_forward_counts(const void *ws, const RgxCamera *cam, const RgxMarc
  * cuda_train/backward/gaussians_aabb.cu: gradients of sum(dloss * ray_colors) with
  * respect to density (N), rgb (N,3), position (N,3), scale (N,3), quaternion (N,4),
  * in INPUT order, overwritten.  ray_colors is the forward's output.  records: the record
- * written by the forward launch with the same ws, cam, march and prims, or NULL. */
+ * written by the forward launch with the same ws, cam, march and prims, or NULL where that forward
+ * wrote none.  (With the fixed step a forward that leaves a record may meet a ray's hits in another order
+ * than one that does not; where max_prim_slice cuts a list, the order decides which hits are kept.) */
 int rgx_march_backward(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims,
                        int64_t n, const float *ray_colors, const float *dloss, float *ddens,
                        float *drgb, float *dpos, float *dscale, float *dquat, void *march_ws,

@@ -587,7 +587,7 @@ __device__ __forceinline__ void frustum_cut_pairs(const MarchParams &P, Frustum 
 // Fills the table from the sweep; returns the number of entries.  done: the sweep is finished;
 // plain: every entry passed plain_roots().
 // AGAIN: the descent reads its arguments once more for every table (args_again) and does not hold them, or spill them, across the marches
-// between: images by pairs (300 k Gaussians 800x800 with lobes 2.284 -> 2.245 ms, viewer 1 M 1280x720 6.06 -> 6.00).  Not where it loses: the
+// between: marches by pairs that record nothing.  Measured for images (300 k Gaussians 800x800 with lobes 2.284 -> 2.245 ms, viewer 1 M 1280x720 6.06 -> 6.00).  Not where it loses: the
 // recording forward (300 k 800x800 2.67 -> 2.71) and images by nodes (3 M 1920x1080 16.2 -> 16.4).
 // PAIRS: the descent opens 64 internal nodes a step and tests both children of each, so it takes half as many steps, each one
 // trip to memory; leaves never enter the stack.  It finds the Gaussians in another order, so only marches whose sums may be taken
@@ -783,14 +783,13 @@ struct RayState {
 // Ray set-up: computeRay and the scene-bbox slab test (fwd: gaussians_aabb.cu:207-231;
 // bwd: backward/gaussians_aabb.cu:211-233, which divides by the direction where the forward
 // multiplies by its reciprocal).  The ray starts out searching from the box entry.
-template <bool DIVIDE>
-__device__ __forceinline__ void ray_begin(const MarchParams &P, int px, int py, bool valid, RayState &R)
+__device__ __forceinline__ void ray_begin(const MarchParams &P, int px, int py, bool valid, bool divide, RayState &R)
 {
     const f3 o = mk3(P.cam.eye[0], P.cam.eye[1], P.cam.eye[2]);
     R.dir = compute_ray(P.cam, (unsigned)px, (unsigned)py);
     const float *bmn = P.hdr->bb_min, *bmx = P.hdr->bb_max;
     float t0x, t1x, t0y, t1y, t0z, t1z;
-    if (DIVIDE) {
+    if (divide) {
         t0x = (bmn[0] - o.x) / R.dir.x; t1x = (bmx[0] - o.x) / R.dir.x;
         t0y = (bmn[1] - o.y) / R.dir.y; t1y = (bmx[1] - o.y) / R.dir.y;
         t0z = (bmn[2] - o.z) / R.dir.z; t1z = (bmx[2] - o.z) / R.dir.z;
@@ -816,9 +815,8 @@ __device__ __forceinline__ void ray_begin(const MarchParams &P, int px, int py, 
 // Top of an iteration: loop condition, adaptive step (gaussians_aabb.cu:266-276) and the interval
 // this ray asks about: its slab when marching (returns true), or one slab length ahead of tbuffer
 // when searching (returns false; the search itself runs to the end of the candidate window).
-// CLIP: the forward clips the slab to [tenter, texit] (275-276), the backward does not (279-280).
-template <bool CLIP>
-__device__ __forceinline__ bool slab_begin(const MarchParams &P, RayState &R, float &tlo, float &thi)
+// clip: the forward clips the slab to [tenter, texit] (275-276), the backward does not (279-280).
+__device__ __forceinline__ bool slab_begin(const MarchParams &P, bool clip, RayState &R, float &tlo, float &thi)
 {
     R.active = R.active && R.tbuffer < R.texit && R.T > P.m.t_eps;
     // a step below one ulp of t cannot advance the ray: stop instead of spinning
@@ -834,8 +832,8 @@ __device__ __forceinline__ bool slab_begin(const MarchParams &P, RayState &R, fl
         thi = fminf(R.texit, R.tbuffer + R.slab_spacing);
         return false;
     }
-    tlo = CLIP ? fmaxf(R.tenter, R.tbuffer) : R.tbuffer;
-    thi = CLIP ? fminf(R.texit, R.tbuffer + R.slab_spacing) : R.tbuffer + R.slab_spacing;
+    tlo = clip ? fmaxf(R.tenter, R.tbuffer) : R.tbuffer;
+    thi = clip ? fminf(R.texit, R.tbuffer + R.slab_spacing) : R.tbuffer + R.slab_spacing;
     return R.active && thi > R.tenter;
 }
 
@@ -2094,7 +2092,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
     Frustum F;
     frustum_planes(P.cam, px0, half == 1 ? py0 + 4 : py0, F, half < 0 ? 8 : 4);
     RayState R;
-    ray_begin<false>(P, px, py, valid, R);
+    ray_begin(P, px, py, valid, false, R);
     {
         const float t_far = wave_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f);
         if constexpr (PAIRS) frustum_cut_pairs(P, F, t_far, L.queue);
@@ -2107,7 +2105,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
 
     while (__any(R.active)) {
         float tlo, thi;
-        const bool need = slab_begin<true>(P, R, tlo, thi);
+        const bool need = slab_begin(P, true, R, tlo, thi);
         int p0 = 0;
         bool ov = false;
         float found = -1.0f, searched_to = 0.f;
@@ -2755,7 +2753,7 @@ __global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const Ma
     Frustum F;
     frustum_planes(P.cam, px0, py0, F);
     RayState R;
-    ray_begin<false>(P, px, py, valid, R);
+    ray_begin(P, px, py, valid, false, R);
     {
         const TeamWord far = team_exchange(T, tp, turn, 0.f, row_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f), 0.f, 0u);
         team_frustum_cut(P, F, far.hi, T, tp);
@@ -2768,7 +2766,7 @@ __global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const Ma
 
     for (;;) {
         float tlo, thi;
-        const bool need = slab_begin<true>(P, R, tlo, thi);
+        const bool need = slab_begin(P, true, R, tlo, thi);
         const bool srch = R.active && R.searching, want = need || srch;
         const float w0 = row_min_all(want ? tlo : INFINITY), w1 = row_max_all(want ? thi : -INFINITY);
         const TeamWord all = team_exchange(T, tp, turn, w0, w1, row_max_all(want ? tlo + (float)Wn.k * R.slab_spacing : -INFINITY),
@@ -3220,10 +3218,12 @@ struct GroupAdd {
 // frame (RGX_NSUM); those are summed over the rays of a group of lanes (a row of 16 in the walk by rows, half a
 // row in a replay) with DPP adds and carried on by one lane per group (all eight in a replay: GroupAdd); the
 // change of variables to the 14 gradient words comes after all sums.
-template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false>
+// PAIRS: how a search of the tree descends (sweep_next).
+template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false, bool PAIRS = false>
 __device__ __forceinline__ void march_bwd(const MarchParams &P)
 {
     static_assert(REPLAY || !SUMS, "sample sums come with a record");
+    static_assert(!REPLAY || !PAIRS, "a replay searches no tree");
     static_assert(SUMS || !HALF, "the colour sums' format is a property of the sample sums");
     int px0, py0, tile;
     // A launch that replays sample sums has a grid for every piece of the tiles' records, the last (longest) pieces first.
@@ -3263,8 +3263,9 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     RGX_SEC_START(cn, 1);
     RayState R;
     // a replay follows the forward's iteration sequence, so it takes the forward's conventions
-    // (reciprocal multiply in the bbox test, clipped slab bounds)
-    ray_begin<!REPLAY>(P, px, py, valid, R);
+    // (reciprocal multiply in the bbox test, clipped slab bounds); so does the search in the place of a replay
+    const bool as_forward = REPLAY || P.only_overflow;
+    ray_begin(P, px, py, valid, !as_forward, R);
     const f3 dir = R.dir;
     f3 g = mk3(0.f, 0.f, 0.f);
     float D = 0.f;
@@ -3278,7 +3279,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     // one slab iteration; `drive(need, tlo, thi, p0, ov, found, searched_to, body_a, mid, body_b)` supplies the hit lists
     auto iteration = [&](auto drive) {
         float tlo, thi;
-        const bool need = slab_begin<REPLAY>(P, R, tlo, thi);
+        const bool need = slab_begin(P, as_forward, R, tlo, thi);
         int p0 = 0;
         bool ov = false;
         float found = -1.0f, searched_to = 0.f;
@@ -3540,15 +3541,19 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             if (P.faults) atomicAdd(&P.faults[0], 1u); // counted with or without a statistics block
         }
     } else {
-        RGX_TILE_LDS(false);
+        RGX_TILE_LDS(PAIRS);
         Frustum F;
         frustum_planes(P.cam, px0, py0, F);
-        frustum_cut(P, F, wave_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f), L.queue);
+        {
+            const float t_far = wave_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f);
+            if constexpr (PAIRS) frustum_cut_pairs(P, F, t_far, L.queue);
+            else frustum_cut(P, F, t_far, L.queue);
+        }
         Window Wn = {0.f, 0, false, 4, false, false};
         NoRecorder rec;
         while (__any(R.active)) {
             iteration([&](bool need, float tlo, float thi, int &p0, bool &ov, float &found, float &searched_to, auto a, auto mid,
-                          auto b) { return slab_tables<WALK_BACKWARD, false>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, a, mid, b); });
+                          auto b) { return slab_tables<WALK_BACKWARD, PAIRS>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, a, mid, b); });
         }
     }
     flush_stats(P.stats, cn);
@@ -3694,8 +3699,8 @@ __global__ __launch_bounds__(1024) void k_block_order(const MarchParams P, const
 // The backward that searches the tree, and those that replay the forward's record: its lists, or its sample sums.
 // (The replay of lists alone keeps the 64 density and colour sums it rebuilds across two walks, and spills 200 bytes a
 // lane; it runs for the first view of a shape, and where memory is short.)
-template <bool STATS>
-__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd(const MarchParams P) { march_bwd<false, false, STATS>(P); }
+template <bool STATS, bool PAIRS>
+__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd(const MarchParams P) { march_bwd<false, false, STATS, false, PAIRS>(P); }
 template <bool STATS>
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd_replay(const MarchParams P) { march_bwd<true, false, STATS>(P); }
 template <bool STATS, bool HALF = false>
@@ -3704,7 +3709,7 @@ template <bool STATS, bool HALF = false>
 #endif
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR_SUMS void k_march_bwd_replay_sums(const MarchParams P) { march_bwd<true, true, STATS, HALF>(P); }
 
-enum { RGX_BWD_TREE, RGX_BWD_LISTS, RGX_BWD_SUMS };
+enum { RGX_BWD_TREE, RGX_BWD_TREE_PAIRS, RGX_BWD_LISTS, RGX_BWD_SUMS };
 static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
 {
     const dim3 wave(64);
@@ -3716,9 +3721,12 @@ static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStr
     } else if (which == RGX_BWD_LISTS) {
         if (stats) hipLaunchKernelGGL(k_march_bwd_replay<true>, grid, wave, 0, s, P);
         else hipLaunchKernelGGL(k_march_bwd_replay<false>, grid, wave, 0, s, P);
+    } else if (which == RGX_BWD_TREE_PAIRS) {
+        if (stats) hipLaunchKernelGGL((k_march_bwd<true, true>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd<false, true>), grid, wave, 0, s, P);
     } else {
-        if (stats) hipLaunchKernelGGL(k_march_bwd<true>, grid, wave, 0, s, P);
-        else hipLaunchKernelGGL(k_march_bwd<false>, grid, wave, 0, s, P);
+        if (stats) hipLaunchKernelGGL((k_march_bwd<true, false>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd<false, false>), grid, wave, 0, s, P);
     }
 }
 
@@ -4030,12 +4038,18 @@ static inline dim3 march_grid(const MarchParams &P)
 // few rounds lasts; with many rounds the wavefronts hide each other's trips to memory (forward by nodes / by pairs: 300 k Gaussians
 // 800x800 2.77 / 2.66 ms, its frame with lobes 2.38 / 2.27, 1 M 800x800 5.28 / 5.19, viewer 1 M 1280x720 6.08 / 6.06; 3 M
 // 1920x1080, 10.5 rounds, 16.88 / 16.96).
+// A backward that searches the tree for a tile whose record overflowed goes as the forward that wrote the record went: the order in which a
+// sweep finds a tile's Gaussians is the order in which max_prim_slice cuts its rays' lists, and of two orders, lists that are cut
+// keep different hits (a gradient that has little to do with the image).
 #define RGX_PAIR_TILES (6 * 3072)
+static bool by_pairs(const MarchParams &P, bool image_only)
+{
+    return sums_in_any_order(P, image_only) && !by_team(P, image_only) && P.n <= RGX_PAIR_BOXES && P.tiles_x * P.tiles_y <= RGX_PAIR_TILES;
+}
 // half: the record's colour sums are in half precision
 static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, bool image_only, hipStream_t s)
 {
-    const bool any_order = sums_in_any_order(P, image_only);
-    const bool team = by_team(P, image_only), pairs = any_order && P.n <= RGX_PAIR_BOXES && P.tiles_x * P.tiles_y <= RGX_PAIR_TILES;
+    const bool team = by_team(P, image_only), pairs = by_pairs(P, image_only);
     const dim3 grid = march_grid(P), block(team ? 256 : 64);
 #define RGX_FWD(...)                                                                            \
     do {                                                                                        \
@@ -4221,7 +4235,7 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
         P.only_overflow = 1;
         P.use_tile_order = 0;
     }
-    launch_march_bwd(RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
+    launch_march_bwd(by_pairs(P, false) ? RGX_BWD_TREE_PAIRS : RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
     rgx_span_end(span, s);
     span = timed ? rgx_span_begin(RGX_T_UNPERMUTE, s) : nullptr;
     hipLaunchKernelGGL(k_unpermute_grads, grid_for(n, 256), dim3(256), 0, s, (const float4 *)P.gbuf, P.place, n, ddens, drgb,

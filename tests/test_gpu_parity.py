@@ -661,6 +661,33 @@ def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     assert np.abs(images[0] - tree["image"]).max() <= 1e-5
 
 
+@pytest.mark.parametrize("w,h", [(257, 256), (312, 304), (1089, 1082)])      # 1 056 and 1 482 tiles: sweeps by pairs with the fixed step; 18 632: by nodes
+@pytest.mark.parametrize("dyn,cap", [(False, 8), (False, 32), (False, 4096), (True, 32)])
+def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx, w, h, dyn, cap):
+    """Where max_prim_slice cuts a ray's list the order of the sweep decides which hits it keeps, so the backward has to
+    search the tiles whose region overflowed as their forward did: the gradients of the same view with room
+    for its record, up to the order of sums and samples at a cut-off (1e-4, as for the forms of a record; measured 4e-5).
+    With lists cut to other hits they were off by as much as the gradient itself, and by 1.1e-4 at 312x304 where only the
+    box test and the clipping of the slabs were not the forward's."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(2 if dyn else 0, n=6000, sh_degree=0, seed=21))
+    sc["scales"] = sc["scales"] * np.float32(6.0)
+    cam = scenes.make_camera(2 if dyn else 0, 1, width=w, height=h)
+    cfg = dict(dt_step=0.01, dynamic_sampling=dyn, max_prim_slice=cap)
+    dloss = np.random.default_rng(3).normal(size=(w * h, 3)).astype(np.float32)
+    _step(f"cut lists, {w}x{h}, adaptive {dyn}, cap {cap}")
+    room = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=16384 * 4)
+    small = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=1024)
+    plain = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=1024, stats=False)
+    assert room["stats_bwd"]["nodes_visited"] == 0 < small["stats_bwd"]["nodes_visited"]
+    assert (room["stats_fwd"]["overflow_rays"] > 1000) == (cap < 4096)
+    assert small["stats_bwd"]["hit_pairs"] == room["stats_bwd"]["hit_pairs"] > 10000
+    for out in (small, plain):
+        assert np.array_equal(out["image"], room["image"])
+        for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+            cos, rel = gx.cos_rel(out["grads"][k], room["grads"][k])
+            assert cos >= 1 - 1e-6 and rel <= 1e-4, (k, cos, rel)
+
+
 def test_long_hit_lists_spill_and_truncation(gx, orc):
     """Fat Gaussians: slabs with far more than 32 hits (LDS part + spill area), then a tiny
     max_prim_slice to exercise the silent truncation path and its counter."""
