@@ -67,15 +67,15 @@ typedef struct RgxMarch {
 
 /* Optional device-side counters, accumulated (not reset) by the march kernels. */
 typedef struct RgxStats {
-    unsigned long long hit_pairs;     /* sum over blended slabs of the hit-list length (a forward without a record
-                                         collects a crowded slab half by half and never collects, or counts, the
-                                         second half for a ray that ends in the first: a few per cent fewer in
-                                         dense scenes; with a record every list is whole, as in the reference) */
+    unsigned long long hit_pairs;     /* sum over blended slabs of the hit-list length, every list whole, as in the reference (a
+                                         forward that collects a crowded slab half by half counts the second half's hits of
+                                         a ray that ends in the first as well) */
     unsigned long long slabs;         /* slabs blended */
     unsigned long long empty_slabs;   /* collect queries that found nothing */
     unsigned long long overflow_rays; /* collect queries truncated at max_prim_slice */
     unsigned long long rays_hit;      /* rays whose first-hit query found a Gaussian */
-    unsigned long long nodes_visited; /* BVH nodes fetched by all queries */
+    unsigned long long nodes_visited; /* BVH nodes tested by all queries (sweeps by pairs test the children of the nodes they
+                                         open, and not the tile's first nodes once more for every sweep) */
     unsigned long long candidates;     /* Gaussians gathered per tile and slab iteration (filter passes) */
     unsigned long long candidates_hit; /* ... of which at least one ray of the tile hit */
     unsigned long long replay_lost;    /* tiles whose backward did not consume its hit-list record exactly (expect 0) */

@@ -1938,6 +1938,27 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
         }
     }
     if (split && seen < RGX_CCAP / 2) Wn.crowded = false; // sparse again: go back to resident windows
+    if constexpr (WALK == WALK_FORWARD && std::is_same<Cn, Counters>::value) {
+        // What is counted are whole lists: the hits of the second half for the rays that have ended in the first, which nothing shades.
+        const bool ask = split && need && !run && tmid < thi;
+        if (__any(ask)) {
+            const Cn work = cn; // (nodes and candidates: those of the march)
+            const float lo = wave_min_all(ask ? fmaxf(tlo, tmid) : INFINITY), hi = wave_max_all(ask ? thi : -INFINITY);
+            frustum_range(F, lo, hi);
+            Sweep S = {0, 0};
+            sweep_begin<PAIRS>(P, S, F, L.queue, L.leafq);
+            for (bool done = false; !done;) {
+                bool plain;
+                const int C = sweep_next<PAIRS, PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
+                const LaneQuery Q = {R.dir, ask, tlo, thi, false, 0.f, 0.f, P.m.max_prim_slice, tmid};
+                float none = -1.0f;
+                filter_table(L, C, lo, hi, Q, 2, plain, p0, ov, none, len, own, cn);
+            }
+            cn.nodes = work.nodes;
+            cn.cands = work.cands;
+            cn.cands_hit = work.cands_hit;
+        }
+    }
     return run;
 }
 
@@ -3021,6 +3042,32 @@ __global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const Ma
             blend(1);
             RGX_SEC(cn, RGX_SEC_BLEND);
             if (split && seen < CAP / 2) Wn.crowded = false;
+            if constexpr (STATS && !RECORD) { // (as in slab_tables)
+                if (split) {
+                    const bool ask = need && !run && tmid < thi;
+                    const TeamWord rest = team_exchange(T, tp, turn, row_min_all(ask ? fmaxf(tlo, tmid) : INFINITY), row_max_all(ask ? thi : -INFINITY), 0.f,
+                                                        __any(ask) ? RUN : 0u);
+                    if (rest.flags & RUN) {
+                        const Counters work = cn;
+                        frustum_range(F, rest.lo, rest.hi);
+                        Sweep S = {0, 0};
+                        team_sweep_begin(P, S, F, T);
+                        for (bool done = false; !done;) {
+                            bool plain;
+                            const int C = team_sweep_next(P, S, F, T, tp, done, plain, cn);
+                            const LaneQuery Q = {R.dir, ask, tlo, thi, false, 0.f, 0.f, P.m.max_prim_slice, tmid};
+                            float none = -1.0f;
+                            const float from = fmaxf(rest.lo, w0), to = fminf(rest.hi, w1);
+                            if (plain) team_filter<false, 2, true>(T, tp, C, from, to, Q, p0, ov, none, len, own, cn);
+                            else team_filter<false, 2, false>(T, tp, C, from, to, Q, p0, ov, none, len, own, cn);
+                            if (!done) __syncthreads(); // every wavefront is done with the table
+                        }
+                        cn.nodes = work.nodes;
+                        cn.cands = work.cands;
+                        cn.cands_hit = work.cands_hit;
+                    }
+                }
+            }
             if (need && p0 > 0 && tp.sub == 0) {
                 cn.slabs++;
                 cn.hit_pairs += p0;

@@ -688,6 +688,26 @@ def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx,
             assert cos >= 1 - 1e-6 and rel <= 1e-4, (k, cos, rel)
 
 
+@pytest.mark.parametrize("w,h", [(19, 13), (221, 216), (225, 224), (289, 288), (1096, 1084)])    # four wavefronts a tile; halves of tiles; pairs; nodes
+@pytest.mark.parametrize("config,scale", [(0, 6.0), (0, 1.0)])
+def test_hits_counted_are_those_of_whole_lists_on_every_way(gx, w, h, config, scale):
+    """``hit_pairs`` says how many hits a view's slabs have, not how a kernel came by them: an image that collects its crowded slabs half by
+    half counts what the recording forward counts.  (A ray whose transmittance is within rounding of its end may end a slab
+    earlier or later, some hundred hits.)"""
+    from raygaussx_amd import optix_utils as u_ox
+    sc = scenes.scene_to_numpy(scenes.make_scene(config, n=6000, sh_degree=0, seed=21))
+    sc["scales"] = sc["scales"] * np.float32(scale)
+    cam = scenes.make_camera(config, 1, width=w, height=h)
+    cfg = dict(dt_step=0.01, dynamic_sampling=False, max_prim_slice=4096)
+    _step(f"hits counted, {w}x{h}, scale {scale}")
+    whole = gx.gpu_render(sc, cam, cfg, want_grad=np.ones((w * h, 3), np.float32))["stats_fwd"]
+    none = gx.gpu_render(sc, cam, cfg, want_grad=np.ones((w * h, 3), np.float32), record_hits=False)
+    test = gx.gpu_render(sc, cam, cfg)
+    assert np.array_equal(test["image"], gx.gpu_render(sc, cam, cfg, stats=False)["image"])
+    for st in (none["stats_fwd"], none["stats_bwd"], test["stats_fwd"]):
+        assert abs(st["slabs"] - whole["slabs"]) <= 1 and abs(st["hit_pairs"] - whole["hit_pairs"]) <= 100 * abs(st["slabs"] - whole["slabs"]), (st, whole)
+
+
 def test_long_hit_lists_spill_and_truncation(gx, orc):
     """Fat Gaussians: slabs with far more than 32 hits (LDS part + spill area), then a tiny
     max_prim_slice to exercise the silent truncation path and its counter."""
