@@ -82,6 +82,7 @@ struct MarchParams {
     int32_t use_tile_order; // 0: as launched; 1: per XCD, its tiles' list positions from the heaviest to the lightest (k_tile_order);
                             // 2: per XCD, the blocks of tiles it renders, heaviest first (k_block_order)
     int32_t by_halves;      // forward of an image: two workgroups per tile (launch_forward)
+    int32_t image_only;     // no backward follows this forward
     float4 *sum_pool;       // sample-sum slots of the record (RGX_SUM_SLOT_WORDS each), or null
     uint32_t *sum_next;     // next free slot (bump counter in the record's pool header)
     int32_t sum_slots;      // slots in the pool
@@ -1796,7 +1797,7 @@ struct Window {
     int n;
     bool resident;
     int k;        // slabs to look ahead when a window is built
-    bool crowded; // the last iteration's Gaussians did not fit one table
+    bool crowded; // the last iteration's Gaussians did not fit one table (image_only launches)
     bool plain;   // the resident table's entries all passed plain_roots()
 };
 
@@ -1828,9 +1829,12 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
     const bool any_search = __any(srch);
     const float tmid = fmaf(R.dt, (float)RGX_CHUNK_SIZE, R.tbuffer);
     // Where slabs hold more Gaussians than a table (the previous iteration found so), a forward
-    // that records nothing sweeps each half of the slab's depth range for its own phase instead
+    // that no backward follows sweeps each half of the slab's depth range for its own phase instead
     // of the whole range twice: phase 0 takes the Gaussians that reach the first 16 samples,
     // phase 1 those that reach the second 16, and a Gaussian of both halves is counted once.
+    // (A backward sweeps the whole range: where max_prim_slice cuts a ray's list, the halves keep other hits.  What a forward without a
+    // record, but with a backward to come, takes for the whole range: 3 M Gaussians 1237x822 7.70 -> 9.05 ms, before a search of 53; 1 M
+    // 800x800 4.75 -> 4.80.)
     const bool split = WALK == WALK_FORWARD && std::is_same<Rec, NoRecorder>::value && Wn.crowded && __any(need);
     int len = 0, q0 = 0, seen = 0;
     uint32_t own[2] = {0u, 0u}; // this ray's hits among the list's first 32 entries, by half of the samples
@@ -1881,7 +1885,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                         continue;
                     } else {
                         Wn.resident = false;
-                        Wn.crowded = true;
+                        Wn.crowded = P.image_only;
                     }
                 }
                 first = false;
@@ -3963,6 +3967,7 @@ static int fill_params(MarchParams &P, const void *ws, const RgxCamera *cam, con
     P.tile_order = M.order + order_words * sizeof(uint32_t) <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.order) : nullptr;
     P.use_tile_order = 0;
     P.by_halves = 0;
+    P.image_only = 0;
     P.faults = M.order <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.faults) : nullptr;
     P.ray_counts = nullptr;
     P.sum_pool = nullptr;
@@ -4020,7 +4025,7 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
 // with the fixed step.  The team adds up a sample's hits in another order, and where max_prim_slice cuts a ray's list it
 // keeps other hits, equally exact both.
 //   No record: the backward searches the tree again, one wavefront per tile, and has to meet the hits and the
-//     transmittance of the forward: that is k_march_fwd then, whatever the step.
+//     transmittance of the forward: that is k_march_fwd then, whatever the step, and every slab's list in one (slab_tables).
 //   A record and the adaptive step: the next step's length depends on the last bit of the transmittance, and a sample that
 //     so crosses a Gaussian's cut-off moves that Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians):
 //     no longer the gradients that larger images give.  k_march_fwd.
@@ -4061,6 +4066,7 @@ static void prepare_forward(MarchParams &P, bool image_only, hipStream_t s)
     // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every tile has a CU of its own, and starts at once.
     const int64_t tiles = (int64_t)P.tiles_x * P.tiles_y;
     const bool team = by_team(P, image_only);
+    P.image_only = image_only;
     P.by_halves = image_only && !team && tiles <= RGX_HALF_TILES;
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);

@@ -694,7 +694,6 @@ def test_hits_counted_are_those_of_whole_lists_on_every_way(gx, w, h, config, sc
     """``hit_pairs`` says how many hits a view's slabs have, not how a kernel came by them: an image that collects its crowded slabs half by
     half counts what the recording forward counts.  (A ray whose transmittance is within rounding of its end may end a slab
     earlier or later, some hundred hits.)"""
-    from raygaussx_amd import optix_utils as u_ox
     sc = scenes.scene_to_numpy(scenes.make_scene(config, n=6000, sh_degree=0, seed=21))
     sc["scales"] = sc["scales"] * np.float32(scale)
     cam = scenes.make_camera(config, 1, width=w, height=h)
@@ -706,6 +705,30 @@ def test_hits_counted_are_those_of_whole_lists_on_every_way(gx, w, h, config, sc
     assert np.array_equal(test["image"], gx.gpu_render(sc, cam, cfg, stats=False)["image"])
     for st in (none["stats_fwd"], none["stats_bwd"], test["stats_fwd"]):
         assert abs(st["slabs"] - whole["slabs"]) <= 1 and abs(st["hit_pairs"] - whole["hit_pairs"]) <= 100 * abs(st["slabs"] - whole["slabs"]), (st, whole)
+
+
+@pytest.mark.parametrize("dyn,w,h,scale", [(True, 100, 80, 6.0), (True, 257, 256, 12.0), (False, 1089, 1082, 6.0)])    # (records by nodes, as without one)
+@pytest.mark.parametrize("cap", [8, 32, 4096])
+def test_forward_without_a_record_keeps_the_hits_that_its_backward_keeps(gx, dyn, w, h, scale, cap):
+    """Crowded slabs (more Gaussians than a table) with lists cut at max_prim_slice: a forward that a backward follows keeps the hits
+    of the slab's one list, with a record or without, so image and counts are the same, and so are the gradients that
+    the replay and the search give (to 1e-4, as above; 2e-2 to 1 where the lists were collected half a slab at a time)."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(2 if dyn else 0, n=6000, sh_degree=0, seed=21))
+    sc["scales"] = sc["scales"] * np.float32(scale)
+    cam = scenes.make_camera(2 if dyn else 0, 1, width=w, height=h)
+    cfg = dict(dt_step=0.01, dynamic_sampling=dyn, max_prim_slice=cap)
+    dloss = np.random.default_rng(3).normal(size=(w * h, 3)).astype(np.float32)
+    _step(f"no record, crowded slabs, {w}x{h}, adaptive {dyn}, cap {cap}")
+    rec = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=16384 * 4)
+    none = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    assert (rec["stats_fwd"]["overflow_rays"] > 1000) == (cap < 4096)
+    assert np.array_equal(none["image"], rec["image"])
+    for k in ("hit_pairs", "slabs", "empty_slabs", "overflow_rays", "rays_hit"):
+        assert none["stats_fwd"][k] == rec["stats_fwd"][k], k
+    for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+        cos, rel = gx.cos_rel(none["grads"][k], rec["grads"][k])
+        print(f"{k}: rel {rel:.2e}", flush=True)
+        assert cos >= 1 - 1e-6 and rel <= 1e-4, (k, cos, rel)
 
 
 def test_long_hit_lists_spill_and_truncation(gx, orc):
