@@ -49,6 +49,9 @@
 // keys with ties broken by a 30-bit index is at most 63 + 30 = 93 deep: with a margin of 160 the
 // stack never holds more than QCAP - 96 + 93 < QCAP entries, whatever the scene.
 #define RGX_DFS_MARGIN 160
+// The same for a sweep of 256 nodes a step, by four wavefronts (k_march_team): a step pops at most as many nodes as leave this margin free.
+#define RGX_TEAM_QCAP 1024
+#define RGX_TEAM_DFS_MARGIN 96
 #define RGX_LDS_HITS 32    // per-lane list of the stand-alone collect hook
 // The march kernels are sized (registers and LDS) for three wavefronts per SIMD.
 #ifndef RGX_WAVES_ATTR
@@ -450,11 +453,21 @@ struct Sweep {
     int lqn; // leaves waiting for their ellipsoid test (wave-uniform)
 };
 
-template <bool PAIRS>
+// The orders in which a sweep can find a tile's Gaussians.  Where max_prim_slice cuts a ray's list the order decides which hits are
+// kept, so a backward that has to search the tree for a tile takes the order of the forward that wrote the tile's record.
+//   BY_NODES  up to 64 nodes a step; where nothing speaks for another
+//   BY_PAIRS  the children of up to 64 nodes a step
+//   BY_TEAM   up to 256 nodes a step: what k_march_team does with four wavefronts, by one
+enum { BY_NODES, BY_PAIRS, BY_TEAM };
+
+template <int ORDER>
 __device__ __forceinline__ void sweep_begin(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq)
 {
     S.lqn = 0;
-    if constexpr (PAIRS) {
+    if constexpr (ORDER == BY_TEAM) {
+        S.qn = F.cut_n;
+        for (int i = threadIdx.x; i < F.cut_n; i += 64) s_queue[i] = s_queue[RGX_TEAM_QCAP + i];
+    } else if constexpr (ORDER == BY_PAIRS) {
         S.qn = F.cut_inner;
         S.lqn = F.cut_n - F.cut_inner;
         const int lane = threadIdx.x;
@@ -585,6 +598,157 @@ __device__ __forceinline__ void frustum_cut_pairs(const MarchParams &P, Frustum 
     F.cut_node = node;
 }
 
+// What a leaf whose box passed turns into: its ellipsoid against the frustum, and its table entry (as in sweep_next,
+// whose kernels have no register for a function that returns one).
+struct LeafEntry {
+    f3 U, V, W, inv, Oe;
+    float dmin, dmax, k, c;
+    bool plain; // passed plain_roots()
+    __device__ __forceinline__ void store(float4 *dst, int32_t left) const
+    {
+        table_store(dst, U, V, W, inv, Oe, ~left, dmin, dmax, k, c);
+    }
+};
+__device__ __forceinline__ bool leaf_entry(const MarchParams &P, const Frustum &F, int32_t left, LeafEntry &e)
+{
+    const Prim p = P.prims[~left];
+    quat_to_cols(p.quat4, e.U, e.V, e.W);
+    const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
+    const bool ok = leaf_meets(F, p, e.U, e.V, e.W, e.dmin, e.dmax);
+    if (ok) {
+        e.k = p.inv_inter4.w;
+        e.inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
+        e.Oe = apply_sinv_rt(O, e.U, e.V, e.W, e.inv);
+        e.c = fmaf(e.Oe.x, e.Oe.x, fmaf(e.Oe.y, e.Oe.y, fmaf(e.Oe.z, e.Oe.z, -1.0f)));
+        e.plain = plain_roots(e.inv, e.c);
+    }
+    return ok;
+}
+
+// What the team's lanes do in one step, a wavefront after the other: each(j, on, value) for the four groups of 64 of the m words at `from`, all of which
+// are read before the first is looked at.
+template <typename Each>
+__device__ __forceinline__ void team_groups(const int32_t *from, int m, Each each)
+{
+    const int lane = threadIdx.x;
+    int32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = 64 * j + lane < m ? from[64 * j + lane] : -1;
+    __syncthreads();
+    for (int j = 0; j < 4 && 64 * j < m; ++j) each(64 * j + lane < m, j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3]);
+    __syncthreads();
+}
+
+// The node's box against the frustum (a lane without a node: nothing met).
+__device__ __forceinline__ void node_meets(const MarchParams &P, const Frustum &F, bool on, int32_t node, bool &leaf, bool &inner, int32_t &left, int32_t &right)
+{
+    leaf = inner = false;
+    left = right = 0;
+    if (on && (uint32_t)node < (uint32_t)(2 * P.n - 1)) {
+        const float4 a = ((const float4 *)P.nodes)[2 * node], b = ((const float4 *)P.nodes)[2 * node + 1];
+        right = P.right[max(0, min(node, (int32_t)P.n - 2))];
+        left = __float_as_int(a.w);
+        const bool meets = !frustum_misses(F, a, b);
+        leaf = meets && left < 0;
+        inner = meets && left >= 0;
+    }
+}
+
+// team_frustum_cut by one wavefront, into the 256 words behind the stack
+__device__ __forceinline__ void frustum_cut_team(const MarchParams &P, Frustum &F, float t_far, int32_t *s_queue)
+{
+    F.range(0.f, INFINITY, 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f)); // no distance shell
+    int32_t *cut = s_queue + RGX_TEAM_QCAP;
+    int count = P.n > 0 ? 1 : 0;
+    if (threadIdx.x == 0) cut[0] = 0;
+    __syncthreads();
+    for (int level = 0; level < 64 && count > 0; ++level) {
+        int kept = 0, opened = 0;
+        team_groups(cut, count, [&](bool on, int32_t node) {
+            bool leaf, inner;
+            int32_t left, right;
+            node_meets(P, F, on, node, leaf, inner, left, right);
+            kept += __popcll(__ballot(leaf));
+            opened += __popcll(__ballot(inner));
+        });
+        const int next = kept + 2 * opened;
+        if (opened == 0 || next > 256) break;
+        int leaves = 0, at = kept;
+        team_groups(cut, count, [&](bool on, int32_t node) {
+            bool leaf, inner;
+            int32_t left, right;
+            node_meets(P, F, on, node, leaf, inner, left, right);
+            const uint64_t bl = __ballot(leaf), bi = __ballot(inner);
+            if (leaf) cut[leaves + rank_in(bl)] = node;
+            if (inner) {
+                cut[at + 2 * rank_in(bi)] = left;
+                cut[at + 2 * rank_in(bi) + 1] = right;
+            }
+            leaves += __popcll(bl);
+            at += 2 * __popcll(bi);
+        });
+        count = next;
+    }
+    F.cut_n = count;
+}
+
+// team_sweep_next by one wavefront
+template <typename Cn>
+__device__ __forceinline__ int sweep_next_team(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab, bool &done,
+                                               bool &plain, Cn &cn)
+{
+    plain = true;
+    int C = 0;
+    while ((S.qn > 0 || S.lqn > 0) && C < RGX_CCAP) {
+        if (S.lqn >= 256 || S.qn == 0) {
+            const int m = S.lqn < 256 ? S.lqn : 256, room = RGX_CCAP - C;
+            int hits = 0;
+            S.lqn -= m;
+            team_groups(s_leafq + S.lqn, m, [&](bool on, int32_t left) {
+                LeafEntry e;
+                const bool hit = on && leaf_entry(P, F, left, e);
+                const uint64_t bl = __ballot(hit);
+                plain = plain && __ballot(hit && !e.plain) == 0;
+                const int rank = hits + rank_in(bl);
+                if (hit) {
+                    if (rank < room) e.store((float4 *)(s_tab + (C + rank) * RGX_TAB), left);
+                    else s_leafq[S.lqn + rank - room] = left; // no room: back to the queue, for the next table
+                }
+                hits += __popcll(bl);
+            });
+            C += hits < room ? hits : room;
+            S.lqn += hits < room ? 0 : hits - room;
+            continue;
+        }
+        const int spare = RGX_TEAM_QCAP - RGX_TEAM_DFS_MARGIN - S.qn;
+        const int m = min(min(S.qn, 256), max(spare, 1));
+        const int base = S.qn - m;
+        int pos = base;
+        if (threadIdx.x == 0) cn.nodes += (unsigned)m;
+        team_groups(s_queue + base, m, [&](bool on, int32_t node) {
+            bool leaf, inner;
+            int32_t left, right;
+            node_meets(P, F, on, node, leaf, inner, left, right);
+            const uint64_t bl = __ballot(leaf), bi = __ballot(inner);
+            if (leaf) s_leafq[S.lqn + rank_in(bl)] = left; // fewer than 256 waiting + at most 256 new
+            S.lqn += __popcll(bl);
+            if (inner) {
+                const int at = pos + 2 * rank_in(bi);
+                if (at + 1 < RGX_TEAM_QCAP) {
+                    s_queue[at] = right;
+                    s_queue[at + 1] = left;
+                } else if (P.faults) { // cannot happen (see RGX_DFS_MARGIN)
+                    atomicAdd(&P.faults[1], 1u);
+                }
+            }
+            pos += 2 * __popcll(bi);
+        });
+        S.qn = min(pos, RGX_TEAM_QCAP);
+    }
+    done = S.qn == 0 && S.lqn == 0;
+    return C;
+}
+
 // Fills the table from the sweep; returns the number of entries.  done: the sweep is finished;
 // plain: every entry passed plain_roots().
 // AGAIN: the descent reads its arguments once more for every table (args_again) and does not hold them, or spill them, across the marches
@@ -593,10 +757,12 @@ __device__ __forceinline__ void frustum_cut_pairs(const MarchParams &P, Frustum 
 // PAIRS: the descent opens 64 internal nodes a step and tests both children of each, so it takes half as many steps, each one
 // trip to memory; leaves never enter the stack.  It finds the Gaussians in another order, so only marches whose sums may be taken
 // in any order go this way (launch_forward).
-template <bool PAIRS, bool AGAIN, typename Cn>
+template <int ORDER, bool AGAIN, typename Cn>
 __device__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab,
                           bool &done, bool &plain, Cn &cn)
 {
+    if constexpr (ORDER == BY_TEAM) return sweep_next_team(P, S, F, s_queue, s_leafq, s_tab, done, plain, cn);
+    constexpr bool PAIRS = ORDER == BY_PAIRS;
     plain = true;
     const int lane = threadIdx.x;
     const float4 *nodes4 = (const float4 *)P.nodes;
@@ -1819,7 +1985,7 @@ __device__ __forceinline__ void frustum_range(Frustum &F, float t0, float t1)
 // row lists in lock step (it sums over the rays of a row).  WALK_ROWS: both bodies over the row lists.
 // Returns the phase-1 participation flag of this lane.
 enum { WALK_FORWARD, WALK_BACKWARD, WALK_ROWS };
-template <int WALK, bool PAIRS, typename Cn, typename Rec, typename BodyA, typename Mid, typename BodyB>
+template <int WALK, int ORDER, typename Cn, typename Rec, typename BodyA, typename Mid, typename BodyB>
 __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds &L, Frustum &F, Window &Wn, const RayState &R,
                                             bool need, float tlo, float thi, int &p0, bool &ov, float &found, float &searched_to,
                                             Cn &cn, Rec &rec, BodyA body_a, Mid mid, BodyB body_b)
@@ -1854,7 +2020,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
             if (!split && phase == 0 && Wn.k > 1)
                 wend = fmaxf(t1, wave_max_all(want ? tlo + (float)Wn.k * R.slab_spacing : -INFINITY));
             frustum_range(F, lo, wend);
-            sweep_begin<PAIRS>(P, S, F, L.queue, L.leafq);
+            sweep_begin<ORDER>(P, S, F, L.queue, L.leafq);
         }
         bool first = true, more = true;
         while (more) {
@@ -1866,7 +2032,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 more = false;
             } else {
                 bool done;
-                C = sweep_next<PAIRS, PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
+                C = sweep_next<ORDER, ORDER == BY_PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
                 if (split) {
                     seen += C;
                 } else if (phase == 0 && first) {
@@ -1881,7 +2047,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                     } else if (Wn.k > 1) {
                         Wn.k = 1; // too many Gaussians ahead: start over with this iteration's range only
                         frustum_range(F, t0, t1);
-                        sweep_begin<PAIRS>(P, S, F, L.queue, L.leafq);
+                        sweep_begin<ORDER>(P, S, F, L.queue, L.leafq);
                         continue;
                     } else {
                         Wn.resident = false;
@@ -1950,10 +2116,10 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
             const float lo = wave_min_all(ask ? fmaxf(tlo, tmid) : INFINITY), hi = wave_max_all(ask ? thi : -INFINITY);
             frustum_range(F, lo, hi);
             Sweep S = {0, 0};
-            sweep_begin<PAIRS>(P, S, F, L.queue, L.leafq);
+            sweep_begin<ORDER>(P, S, F, L.queue, L.leafq);
             for (bool done = false; !done;) {
                 bool plain;
-                const int C = sweep_next<PAIRS, PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
+                const int C = sweep_next<ORDER, ORDER == BY_PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
                 const LaneQuery Q = {R.dir, ask, tlo, thi, false, 0.f, 0.f, P.m.max_prim_slice, tmid};
                 float none = -1.0f;
                 filter_table(L, C, lo, hi, Q, 2, plain, p0, ov, none, len, own, cn);
@@ -2069,9 +2235,9 @@ struct Replayer {
     }
 };
 
-#define RGX_TILE_LDS(PAIRS)                                           \
-    __shared__ int32_t s_queue[RGX_QCAP];                             \
-    __shared__ int32_t s_leafq[PAIRS ? 192 : 128];                    \
+#define RGX_TILE_LDS(ORDER)                                           \
+    __shared__ int32_t s_queue[(ORDER) == BY_TEAM ? RGX_TEAM_QCAP + 256 : RGX_QCAP]; \
+    __shared__ int32_t s_leafq[(ORDER) == BY_TEAM ? 512 : (ORDER) == BY_PAIRS ? 192 : 128]; \
     __shared__ __align__(16) float s_tab[RGX_CCAP * RGX_TAB];         \
     __shared__ __align__(4) uint8_t s_list[RGX_CCAP];                 \
     __shared__ uint32_t s_mask[RGX_MASK_WORDS][64];                   \
@@ -2279,8 +2445,6 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
 // Bound by the latency of the march's chain of slabs: an iteration costs a wavefront some 9 000 clocks, of which the
 // filter 0.27, the lists and the barriers around them 0.21, shading 0.13, the sweep 0.12 and the blend 0.11 (4 k
 // Gaussians, 128x128).  Two wavefronts per SIMD: up to 512 tiles are resident at once, and nothing is spilled.
-#define RGX_TEAM_QCAP 1024
-#define RGX_TEAM_DFS_MARGIN 96 // (see RGX_DFS_MARGIN: a step pops at most as many nodes as leave this margin free)
 template <int CAP>
 struct TeamShared {
     static constexpr int WORDS = (CAP + 31) / 32;
@@ -2363,33 +2527,6 @@ __device__ __forceinline__ void sum_copies(float (&v)[RGX_CHUNK_SIZE], float (&o
         swap16(v[i], v[i + 4]);
         out[i] = v[i] + v[i + 4];
     }
-}
-
-// What a leaf whose box passed turns into: its ellipsoid against the frustum, and its table entry (as in sweep_next,
-// whose kernels have no register for a function that returns one).
-struct LeafEntry {
-    f3 U, V, W, inv, Oe;
-    float dmin, dmax, k, c;
-    bool plain; // passed plain_roots()
-    __device__ __forceinline__ void store(float4 *dst, int32_t left) const
-    {
-        table_store(dst, U, V, W, inv, Oe, ~left, dmin, dmax, k, c);
-    }
-};
-__device__ __forceinline__ bool leaf_entry(const MarchParams &P, const Frustum &F, int32_t left, LeafEntry &e)
-{
-    const Prim p = P.prims[~left];
-    quat_to_cols(p.quat4, e.U, e.V, e.W);
-    const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
-    const bool ok = leaf_meets(F, p, e.U, e.V, e.W, e.dmin, e.dmax);
-    if (ok) {
-        e.k = p.inv_inter4.w;
-        e.inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
-        e.Oe = apply_sinv_rt(O, e.U, e.V, e.W, e.inv);
-        e.c = fmaf(e.Oe.x, e.Oe.x, fmaf(e.Oe.y, e.Oe.y, fmaf(e.Oe.z, e.Oe.z, -1.0f)));
-        e.plain = plain_roots(e.inv, e.c);
-    }
-    return ok;
 }
 
 template <int CAP>
@@ -3269,12 +3406,12 @@ struct GroupAdd {
 // frame (RGX_NSUM); those are summed over the rays of a group of lanes (a row of 16 in the walk by rows, half a
 // row in a replay) with DPP adds and carried on by one lane per group (all eight in a replay: GroupAdd); the
 // change of variables to the 14 gradient words comes after all sums.
-// PAIRS: how a search of the tree descends (sweep_next).
-template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false, bool PAIRS = false>
+// ORDER: how a search of the tree descends.
+template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false, int ORDER = BY_NODES>
 __device__ __forceinline__ void march_bwd(const MarchParams &P)
 {
     static_assert(REPLAY || !SUMS, "sample sums come with a record");
-    static_assert(!REPLAY || !PAIRS, "a replay searches no tree");
+    static_assert(!REPLAY || ORDER == BY_NODES, "a replay searches no tree");
     static_assert(SUMS || !HALF, "the colour sums' format is a property of the sample sums");
     int px0, py0, tile;
     // A launch that replays sample sums has a grid for every piece of the tiles' records, the last (longest) pieces first.
@@ -3592,19 +3729,20 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             if (P.faults) atomicAdd(&P.faults[0], 1u); // counted with or without a statistics block
         }
     } else {
-        RGX_TILE_LDS(PAIRS);
+        RGX_TILE_LDS(ORDER);
         Frustum F;
         frustum_planes(P.cam, px0, py0, F);
         {
             const float t_far = wave_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f);
-            if constexpr (PAIRS) frustum_cut_pairs(P, F, t_far, L.queue);
+            if constexpr (ORDER == BY_TEAM) frustum_cut_team(P, F, t_far, L.queue);
+            else if constexpr (ORDER == BY_PAIRS) frustum_cut_pairs(P, F, t_far, L.queue);
             else frustum_cut(P, F, t_far, L.queue);
         }
         Window Wn = {0.f, 0, false, 4, false, false};
         NoRecorder rec;
         while (__any(R.active)) {
             iteration([&](bool need, float tlo, float thi, int &p0, bool &ov, float &found, float &searched_to, auto a, auto mid,
-                          auto b) { return slab_tables<WALK_BACKWARD, PAIRS>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, a, mid, b); });
+                          auto b) { return slab_tables<WALK_BACKWARD, ORDER>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, a, mid, b); });
         }
     }
     flush_stats(P.stats, cn);
@@ -3750,8 +3888,8 @@ __global__ __launch_bounds__(1024) void k_block_order(const MarchParams P, const
 // The backward that searches the tree, and those that replay the forward's record: its lists, or its sample sums.
 // (The replay of lists alone keeps the 64 density and colour sums it rebuilds across two walks, and spills 200 bytes a
 // lane; it runs for the first view of a shape, and where memory is short.)
-template <bool STATS, bool PAIRS>
-__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd(const MarchParams P) { march_bwd<false, false, STATS, false, PAIRS>(P); }
+template <bool STATS, int ORDER>
+__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd(const MarchParams P) { march_bwd<false, false, STATS, false, ORDER>(P); }
 template <bool STATS>
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd_replay(const MarchParams P) { march_bwd<true, false, STATS>(P); }
 template <bool STATS, bool HALF = false>
@@ -3760,7 +3898,7 @@ template <bool STATS, bool HALF = false>
 #endif
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR_SUMS void k_march_bwd_replay_sums(const MarchParams P) { march_bwd<true, true, STATS, HALF>(P); }
 
-enum { RGX_BWD_TREE, RGX_BWD_TREE_PAIRS, RGX_BWD_LISTS, RGX_BWD_SUMS };
+enum { RGX_BWD_TREE, RGX_BWD_TREE_PAIRS, RGX_BWD_TREE_TEAM, RGX_BWD_LISTS, RGX_BWD_SUMS };
 static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
 {
     const dim3 wave(64);
@@ -3772,12 +3910,15 @@ static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStr
     } else if (which == RGX_BWD_LISTS) {
         if (stats) hipLaunchKernelGGL(k_march_bwd_replay<true>, grid, wave, 0, s, P);
         else hipLaunchKernelGGL(k_march_bwd_replay<false>, grid, wave, 0, s, P);
+    } else if (which == RGX_BWD_TREE_TEAM) {
+        if (stats) hipLaunchKernelGGL((k_march_bwd<true, BY_TEAM>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd<false, BY_TEAM>), grid, wave, 0, s, P);
     } else if (which == RGX_BWD_TREE_PAIRS) {
-        if (stats) hipLaunchKernelGGL((k_march_bwd<true, true>), grid, wave, 0, s, P);
-        else hipLaunchKernelGGL((k_march_bwd<false, true>), grid, wave, 0, s, P);
+        if (stats) hipLaunchKernelGGL((k_march_bwd<true, BY_PAIRS>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd<false, BY_PAIRS>), grid, wave, 0, s, P);
     } else {
-        if (stats) hipLaunchKernelGGL((k_march_bwd<true, false>), grid, wave, 0, s, P);
-        else hipLaunchKernelGGL((k_march_bwd<false, false>), grid, wave, 0, s, P);
+        if (stats) hipLaunchKernelGGL((k_march_bwd<true, BY_NODES>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd<false, BY_NODES>), grid, wave, 0, s, P);
     }
 }
 
@@ -4030,7 +4171,7 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
 //     so crosses a Gaussian's cut-off moves that Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians):
 //     no longer the gradients that larger images give.  k_march_fwd.
 //   A record and the fixed step: what the backward replays is what the team recorded.  (A tile whose region overflowed is
-//     searched again; if max_prim_slice also cut lists in it, they may be cut to other hits there.)
+//     searched again, in the team's order: lists that max_prim_slice cut are cut to the same hits there.)
 #ifndef RGX_TEAM_TILES
 #define RGX_TEAM_TILES 768
 #endif
@@ -4091,9 +4232,8 @@ static inline dim3 march_grid(const MarchParams &P)
 // few rounds lasts; with many rounds the wavefronts hide each other's trips to memory (forward by nodes / by pairs: 300 k Gaussians
 // 800x800 2.77 / 2.66 ms, its frame with lobes 2.38 / 2.27, 1 M 800x800 5.28 / 5.19, viewer 1 M 1280x720 6.08 / 6.06; 3 M
 // 1920x1080, 10.5 rounds, 16.88 / 16.96).
-// A backward that searches the tree for a tile whose record overflowed goes as the forward that wrote the record went: the order in which a
-// sweep finds a tile's Gaussians is the order in which max_prim_slice cuts its rays' lists, and of two orders, lists that are cut
-// keep different hits (a gradient that has little to do with the image).
+// A backward that searches the tree for a tile whose record overflowed goes as the forward that wrote the record went (sweep_begin): with another
+// order, where lists are cut, its gradient has little to do with the image.
 #define RGX_PAIR_TILES (6 * 3072)
 static bool by_pairs(const MarchParams &P, bool image_only)
 {
@@ -4288,7 +4428,7 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
         P.only_overflow = 1;
         P.use_tile_order = 0;
     }
-    launch_march_bwd(by_pairs(P, false) ? RGX_BWD_TREE_PAIRS : RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
+    launch_march_bwd(by_team(P, false) ? RGX_BWD_TREE_TEAM : by_pairs(P, false) ? RGX_BWD_TREE_PAIRS : RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
     rgx_span_end(span, s);
     span = timed ? rgx_span_begin(RGX_T_UNPERMUTE, s) : nullptr;
     hipLaunchKernelGGL(k_unpermute_grads, grid_for(n, 256), dim3(256), 0, s, (const float4 *)P.gbuf, P.place, n, ddens, drgb,

@@ -661,7 +661,8 @@ def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     assert np.abs(images[0] - tree["image"]).max() <= 1e-5
 
 
-@pytest.mark.parametrize("w,h", [(257, 256), (312, 304), (1089, 1082)])      # 1 056 and 1 482 tiles: sweeps by pairs with the fixed step; 18 632: by nodes
+# with the fixed step: up to 1 024 tiles four wavefronts per tile; 1 056 and 1 482 tiles sweeps by pairs; 18 632 by nodes
+@pytest.mark.parametrize("w,h", [(52, 44), (100, 80), (253, 256), (257, 256), (312, 304), (1089, 1082)])
 @pytest.mark.parametrize("dyn,cap", [(False, 8), (False, 32), (False, 4096), (True, 32)])
 def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx, w, h, dyn, cap):
     """Where max_prim_slice cuts a ray's list the order of the sweep decides which hits it keeps, so the backward has to
@@ -679,7 +680,7 @@ def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx,
     small = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=1024)
     plain = gx.gpu_render(sc, cam, cfg, want_grad=dloss, rec_tile_words=1024, stats=False)
     assert room["stats_bwd"]["nodes_visited"] == 0 < small["stats_bwd"]["nodes_visited"]
-    assert (room["stats_fwd"]["overflow_rays"] > 1000) == (cap < 4096)
+    assert (room["stats_fwd"]["overflow_rays"] > 100) == (cap < 4096)
     assert small["stats_bwd"]["hit_pairs"] == room["stats_bwd"]["hit_pairs"] > 10000
     for out in (small, plain):
         assert np.array_equal(out["image"], room["image"])
