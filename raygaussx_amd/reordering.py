@@ -49,7 +49,10 @@ def reorder_tensors(order, tensors):
         dst_p = (C.c_void_p * m)(*[d.data_ptr() for d in dsts])
         rows = (C.c_int64 * m)(*[s[0].numel() * s.element_size() for s in srcs])
         size = L.size_query(L.lib().rgx_gather_workspace_bytes, C.c_int32(m), rows, C.c_int64(n))
-        ws = torch.empty(size, dtype=torch.uint8, device=order.device) if size else None
+        try:
+            ws = torch.empty(size, dtype=torch.uint8, device=order.device) if size else None
+        except torch.cuda.OutOfMemoryError:
+            ws, size = None, 0      # row by row: slower, in no more memory than the results take
         L.check(L.lib().rgx_gather_rows_packed(C.c_int32(m), src_p, dst_p, rows, L.ptr(order), C.c_int64(n), L.ptr(ws), C.c_size_t(size),
                                                L.stream(order.device)))
     it = iter(dsts)

@@ -903,6 +903,29 @@ def test_reorder_tensors_of_many_short_rows(gx, n, words, odd):
         assert torch.equal(got, src[order])
 
 
+def test_reorder_tensors_without_room_for_its_records(gx, monkeypatch):
+    """The records in which short rows are put together are a matter of speed: with no memory left for them the gather goes without."""
+    from raygaussx_amd.reordering import reorder_tensors
+    n = 262_144
+    gen = torch.Generator(gx.DEV).manual_seed(4)
+    tensors = [torch.randint(-2 ** 31, 2 ** 31 - 1, (n, w), dtype=torch.int32, device=gx.DEV, generator=gen) for w in (3, 4, 3, 1, 48)]
+    order = torch.randperm(n, device=gx.DEV, generator=gen)
+    empty, refused = torch.empty, []
+
+    def no_room(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            refused.append(size)
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+    monkeypatch.setattr(torch, "empty", no_room)
+    _step("short rows without room for records")
+    got = reorder_tensors(order, tensors)
+    monkeypatch.undo()
+    assert refused == [(n * 128,)]
+    for a, src in zip(got, tensors):
+        assert torch.equal(a, src[order])
+
+
 def test_reference_style_inference_loop_reuses_the_tree(gx, orc, c0):
     """scripts/test.py:50-126 pattern: boxes -> one acceleration structure -> several cameras."""
     from raygaussx_amd import optix_utils as u_ox
