@@ -8,7 +8,6 @@
 
 #include <algorithm>
 #include <type_traits>
-#include <vector>
 
 // ---------------------------------------------------------------------------
 // order-preserving float <-> int encoding for atomicMin/atomicMax
@@ -1259,18 +1258,21 @@ __global__ __launch_bounds__(256) void k_unpack_rows(const PackArgs A, const int
     }
 }
 
-// The tensors not done yet that share the next record (first fit, in order); returns its words.
-static int pack_group(int32_t count, const int64_t *row_bytes, std::vector<bool> &done, std::vector<int32_t> &members)
+// Tensors are gone through RGX_GATHER_SET at a time, a bit each (no memory of the host's is asked for).
+#define RGX_GATHER_SET 64
+// The tensors of `todo` that share the next record (first fit, in order).
+static uint64_t pack_group(const int64_t *row_bytes, uint64_t todo)
 {
-    members.clear();
+    uint64_t members = 0;
     int words = 0;
-    for (int32_t i = 0; i < count; ++i) {
+    for (; todo; todo &= todo - 1) {
+        const int i = __builtin_ctzll(todo);
         const int64_t w = row_bytes[i] / 4;
-        if (done[i] || w > RGX_PACK_ROW || words + w > RGX_PACK_WORDS) continue;
-        members.push_back(i);
+        if (w > RGX_PACK_ROW || words + w > RGX_PACK_WORDS) continue;
+        members |= 1ull << i;
         words += (int)w;
     }
-    return words;
+    return members;
 }
 
 static int gather_check(int32_t count, const int64_t *row_bytes, int64_t n)
@@ -1291,16 +1293,13 @@ extern "C" int rgx_gather_workspace_bytes(int32_t count, const int64_t *row_byte
     return RGX_OK;
 }
 
-static int gather_direct(const std::vector<int32_t> &which, const void *const *src, void *const *dst, const int64_t *row_bytes,
-                         const int64_t *order, int64_t n, hipStream_t s)
+static int gather_direct(uint64_t todo, const void *const *src, void *const *dst, const int64_t *row_bytes, const int64_t *order, int64_t n, hipStream_t s)
 {
-    const int32_t count = (int32_t)which.size();
-    for (int base = 0; base < count; base += RGX_GATHER_MAX) {
+    while (todo) {
         GatherArgs A;
-        const int m = count - base < RGX_GATHER_MAX ? count - base : RGX_GATHER_MAX;
-        A.count = m;
-        for (int i = 0; i < m; ++i) {
-            const int32_t t = which[base + i];
+        int m = 0;
+        for (; todo && m < RGX_GATHER_MAX; todo &= todo - 1, ++m) {
+            const int t = __builtin_ctzll(todo), i = m;
             A.src[i] = (const uint32_t *)src[t];
             A.dst[i] = (uint32_t *)dst[t];
             const int32_t words = (int32_t)(row_bytes[t] / 4);
@@ -1310,6 +1309,7 @@ static int gather_direct(const std::vector<int32_t> &which, const void *const *s
             A.pieces[i] = words / w;
             A.magic[i] = (uint32_t)((1ull << 32) / (uint32_t)A.pieces[i] + 1);
         }
+        A.count = m;
         const int64_t blocks = (n + RGX_GATHER_ROWS - 1) / RGX_GATHER_ROWS;
         // a workgroup goes through all tensors where there are enough of them to fill the chip several times over
         const int split = blocks >= 2048 ? 1 : m;
@@ -1332,21 +1332,19 @@ extern "C" int rgx_gather_rows_packed(int32_t count, const void *const *src, voi
     if (n == 0) return RGX_OK;
     size_t need = 0;
     rgx_gather_workspace_bytes(count, row_bytes, n, &need);
-    std::vector<bool> done(count, false);
-    std::vector<int32_t> members;
+    const bool pack = need > 0 && ws && ws_bytes >= need;
     hipStream_t s = (hipStream_t)stream;
-    if (need > 0 && ws && ws_bytes >= need) {
-        const unsigned blocks = (unsigned)((n + RGX_GATHER_ROWS - 1) / RGX_GATHER_ROWS);
-        for (int words = pack_group(count, row_bytes, done, members); (int)members.size() >= RGX_PACK_MIN;
-             words = pack_group(count, row_bytes, done, members)) {
+    const unsigned blocks = (unsigned)((n + RGX_GATHER_ROWS - 1) / RGX_GATHER_ROWS);
+    for (; count > 0; count -= RGX_GATHER_SET, src += RGX_GATHER_SET, dst += RGX_GATHER_SET, row_bytes += RGX_GATHER_SET) {
+        uint64_t todo = count < RGX_GATHER_SET ? (1ull << count) - 1 : ~0ull;
+        for (uint64_t members; pack && __builtin_popcountll(members = pack_group(row_bytes, todo)) >= RGX_PACK_MIN; todo &= ~members) {
             PackArgs A;
-            A.count = (int32_t)members.size();
-            A.quads = (words + 3) / 4;
-            A.total = words;
+            A.count = (int32_t)__builtin_popcountll(members);
             A.aligned = 1;
-            int at = 0;
-            for (int i = 0; i < A.count; ++i) {
-                const int32_t t = members[i], w = (int32_t)(row_bytes[t] / 4);
+            int at = 0, i = 0;
+            for (uint64_t left = members; left; left &= left - 1, ++i) {
+                const int t = __builtin_ctzll(left);
+                const int32_t w = (int32_t)(row_bytes[t] / 4);
                 A.src[i] = (const uint32_t *)src[t];
                 A.dst[i] = (uint32_t *)dst[t];
                 A.words[i] = (uint8_t)w;
@@ -1355,17 +1353,17 @@ extern "C" int rgx_gather_rows_packed(int32_t count, const void *const *src, voi
                 A.aligned &= (((uintptr_t)A.src[i] | (uintptr_t)A.dst[i]) & 15) == 0;
                 A.magic[i] = (uint32_t)((1ull << 32) / (uint32_t)w + 1);
                 at += w;
-                done[t] = true;
             }
+            A.quads = (at + 3) / 4;
+            A.total = at;
             hipLaunchKernelGGL(k_pack_rows, dim3(blocks), dim3(256), 0, s, A, n, (uint4 *)ws);
             hipLaunchKernelGGL(k_unpack_rows, dim3(blocks), dim3(256), 0, s, A, order, n, (const uint4 *)ws);
             RGX_LAUNCH_CHECK();
         }
+        const int gathered = gather_direct(todo, src, dst, row_bytes, order, n, s);
+        if (gathered != RGX_OK) return gathered;
     }
-    members.clear();
-    for (int32_t i = 0; i < count; ++i)
-        if (!done[i]) members.push_back(i);
-    return gather_direct(members, src, dst, row_bytes, order, n, s);
+    return RGX_OK;
 }
 
 extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *const *dst, const int64_t *row_bytes,

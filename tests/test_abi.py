@@ -5,6 +5,8 @@ import ctypes as C
 import math
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -12,7 +14,8 @@ import torch
 
 from raygaussx_amd import _lib, scenes, optix_utils as u_ox
 
-HEADER = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "include", "rgx.h")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HEADER = os.path.join(ROOT, "include", "rgx.h")
 
 
 def _declared():
@@ -90,6 +93,29 @@ def test_bad_arguments_are_rejected_before_any_launch():
     assert lib.rgx_march_test(null, C.byref(cam), C.byref(march), null, C.c_int64(0), null, null, C.c_size_t(0), null, null) == -1
     with pytest.raises(_lib.RgxError):
         _lib.check(-2)
+
+
+def test_a_gather_of_many_tensors_asks_for_no_host_memory():
+    """Nothing throws through the C ABI: with the process at its limit of address space, a gather of four million tensors comes back with a code
+    (no device here: RGX_EHIP from the first launch), where a list of them would have ended the process."""
+    if torch.cuda.is_available():
+        pytest.skip("the pointers are not device memory")
+    child = """
+import ctypes as C, resource
+import numpy as np
+from raygaussx_amd import _lib
+lib, n = _lib.lib(), 1 << 22
+words = np.arange(1, n + 2, dtype=np.int64) * 4               # source pointers, destinations (one further) and row sizes
+at = lambda k: C.c_void_p(words.ctypes.data + 8 * k)
+call = lambda count: lib.rgx_gather_rows_packed(count, at(0), at(1), at(0), C.c_void_p(64), C.c_int64(1), C.c_void_p(0), C.c_size_t(0), C.c_void_p(0))
+assert call(3) == -3
+used = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 23), resource.RLIM_INFINITY))
+assert call(n) == -3
+print('came back')
+"""
+    r = subprocess.run([sys.executable, "-c", child], capture_output=True, text=True, timeout=120, cwd=ROOT)
+    assert r.returncode == 0 and "came back" in r.stdout, (r.returncode, r.stderr)
 
 
 def test_refit_of_an_unbuilt_or_mismatched_structure_is_refused_on_the_host():
