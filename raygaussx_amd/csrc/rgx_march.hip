@@ -95,6 +95,8 @@ struct MarchParams {
 };
 
 // The kernel's arguments once more, from the kernel's argument segment: what is read through this is loaded where it is used.
+// Only in a kernel whose first argument is its MarchParams, and in functions that are always inlined into one: in a function that is called, the
+// segment's pointer is none.
 __device__ __forceinline__ const MarchParams &args_again()
 {
     auto p = (const __attribute__((address_space(4))) MarchParams *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -758,7 +760,7 @@ __device__ __forceinline__ int sweep_next_team(const MarchParams &P, Sweep &S, c
 // trip to memory; leaves never enter the stack.  It finds the Gaussians in another order, so only marches whose sums may be taken
 // in any order go this way (launch_forward).
 template <int ORDER, bool AGAIN, typename Cn>
-__device__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab,
+__device__ __forceinline__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab,
                           bool &done, bool &plain, Cn &cn)
 {
     if constexpr (ORDER == BY_TEAM) return sweep_next_team(P, S, F, s_queue, s_leafq, s_tab, done, plain, cn);

@@ -118,6 +118,37 @@ print('came back')
     assert r.returncode == 0 and "came back" in r.stdout, (r.returncode, r.stderr)
 
 
+def _functions(text):
+    """(name, declaration, body) of the functions at the top level of a source in which a body stands between lines "{" and "}", or in one line."""
+    text = re.sub(r"//[^\n]*|^#[^\n]*|__launch_bounds__\(\d+\)", "", text, flags=re.M)
+    for m in re.finditer(r"^(?P<line>\S[^\n]*\)) \{(?P<one>[^\n]*)\}$|^\{\n(?P<body>.*?)^\}$", text, flags=re.S | re.M):
+        declaration = m.group("line") or re.split(r"\n\s*\n|[;}]\n", text[:m.start()], flags=re.M)[-1]
+        name = re.search(r"(\w+)\((?!.*\)\s*__)", declaration, flags=re.S)
+        if name:
+            yield name.group(1), declaration, m.group("body") or m.group("one")
+
+
+def test_the_argument_segment_is_read_in_kernels_only():
+    """The pointer to a kernel's arguments is one in the kernel itself: what takes it (args_again), and whatever calls such a function, is
+    always inlined up to the kernel, and the kernel's first argument is the MarchParams that is read there."""
+    source = open(os.path.join(ROOT, "raygaussx_amd", "csrc", "rgx_march.hip")).read()
+    functions = [f for f in _functions(source) if "__device__" in f[1] or "__global__" in f[1]]
+    assert {"sweep_next", "slab_tables", "march_bwd", "k_march_fwd", "k_collect_tiles"} <= {name for name, _, _ in functions}
+    reads, kernels = {"__builtin_amdgcn_kernarg_segment_ptr"}, set()
+    while True:
+        more = {name for name, _, body in functions if any(re.search(r"\b" + r + r"\s*[<(]", body) for r in reads)} - reads
+        if not more:
+            break
+        reads |= more
+    for name, before, _ in functions:
+        if name in reads and "__global__" in before:
+            kernels.add(name)
+            assert re.search(r"\b" + name + r"\(const MarchParams P\b", before), name
+        elif name in reads:
+            assert "__forceinline__" in before, name
+    assert "args_again" in reads and {"k_march_fwd", "k_march_bwd", "k_collect_tiles"} <= kernels
+
+
 def test_refit_of_an_unbuilt_or_mismatched_structure_is_refused_on_the_host():
     """update_acceleration_structure walks the tree a build left in the workspace, so the mirror refuses it
     for a structure that was never built and for anything but one box per Gaussian of that build -- before
