@@ -85,7 +85,6 @@ struct MarchParams {
     int32_t use_tile_order; // 0: as launched; 1: per XCD, its tiles' list positions from the heaviest to the lightest (k_tile_order);
                             // 2: per XCD, the blocks of tiles it renders, heaviest first (k_block_order)
     int32_t by_halves;      // forward of an image: two workgroups per tile (launch_forward)
-    int32_t image_only;     // no backward follows this forward
     float4 *sum_pool;       // sample-sum slots of the record (RGX_SUM_SLOT_WORDS each), or null
     uint32_t *sum_next;     // next free slot (bump counter in the record's pool header)
     int32_t sum_slots;      // slots in the pool
@@ -1671,7 +1670,7 @@ struct Recorder {
     }
 };
 
-// Stand-in where nothing is recorded.
+// Stand-in where nothing is recorded: an image that no backward follows, or (WholeLists) one whose backward will search the tree.
 struct NoRecorder {
     __device__ __forceinline__ void write_window(const TileLds &, int) {}
     __device__ __forceinline__ void write_lists(const TileLds &, int, bool) {}
@@ -1679,6 +1678,7 @@ struct NoRecorder {
     __device__ __forceinline__ void write_trailer(const MarchParams &, bool, float, float, bool) {}
     __device__ __forceinline__ void finish(const MarchParams &) {}
 };
+struct WholeLists : NoRecorder {};
 
 __device__ __forceinline__ uint32_t uni_u32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
@@ -1965,7 +1965,7 @@ struct Window {
     int n;
     bool resident;
     int k;        // slabs to look ahead when a window is built
-    bool crowded; // the last iteration's Gaussians did not fit one table (image_only launches)
+    bool crowded; // the last iteration's Gaussians did not fit one table
     bool plain;   // the resident table's entries all passed plain_roots()
 };
 
@@ -2001,8 +2001,8 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
     // of the whole range twice: phase 0 takes the Gaussians that reach the first 16 samples,
     // phase 1 those that reach the second 16, and a Gaussian of both halves is counted once.
     // (A backward sweeps the whole range: where max_prim_slice cuts a ray's list, the halves keep other hits.  What a forward without a
-    // record, but with a backward to come, takes for the whole range: 3 M Gaussians 1237x822 7.70 -> 9.05 ms, before a search of 53; 1 M
-    // 800x800 4.75 -> 4.80.)
+    // record, but with a backward to come (WholeLists), takes for the whole range: 3 M Gaussians 1237x822 7.70 -> 9.0 ms, before a search of 53;
+    // 1 M 800x800 4.78 -> 4.74.  A kernel of its own: with the choice at run time, images were 0.3 to 0.7 % slower.)
     const bool split = WALK == WALK_FORWARD && std::is_same<Rec, NoRecorder>::value && Wn.crowded && __any(need);
     int len = 0, q0 = 0, seen = 0;
     uint32_t own[2] = {0u, 0u}; // this ray's hits among the list's first 32 entries, by half of the samples
@@ -2053,7 +2053,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                         continue;
                     } else {
                         Wn.resident = false;
-                        Wn.crowded = P.image_only;
+                        Wn.crowded = true;
                     }
                 }
                 first = false;
@@ -2267,15 +2267,16 @@ __device__ __forceinline__ uint8_t quantize8(float x)
 // colorBlendingT_chunked (182-203).  VIEWER: the interactive viewer's variant of the same march
 // (cuda_gui/gaussians_aabb.cu): black background, uchar4 colours, and the expected depth
 // sum T (1 - w) t over the samples (its colorBlendingT_chunked, 183-205).
-// PAIRS: how the sweeps descend (sweep_next).
-template <bool PAIRS, bool RECORD, bool VIEWER, bool STATS, bool HALF = false>
+// PAIRS: how the sweeps descend (sweep_next).  WHOLE: no record, and a backward that will search the tree (slab_tables).
+template <bool PAIRS, bool RECORD, bool VIEWER, bool STATS, bool HALF = false, bool WHOLE = false>
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchParams P)
 {
     static_assert(RECORD || !HALF, "the colour sums' format is a property of the record");
+    static_assert(!(RECORD || PAIRS) || !WHOLE, "a search without a record goes by nodes");
     RGX_TILE_LDS(PAIRS);
     int px0, py0, tile, half = -1;
     if (!tile_origin(P, blockIdx.x, px0, py0, &tile, RECORD ? nullptr : &half)) return; // whole wave
-    typename std::conditional<RECORD, Recorder, NoRecorder>::type rec;
+    typename std::conditional<RECORD, Recorder, typename std::conditional<WHOLE, WholeLists, NoRecorder>::type>::type rec;
     if constexpr (RECORD) rec = Recorder{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
     int px, py;
     lane_pixel(px0, py0, px, py);
@@ -4110,7 +4111,6 @@ static int fill_params(MarchParams &P, const void *ws, const RgxCamera *cam, con
     P.tile_order = M.order + order_words * sizeof(uint32_t) <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.order) : nullptr;
     P.use_tile_order = 0;
     P.by_halves = 0;
-    P.image_only = 0;
     P.faults = M.order <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.faults) : nullptr;
     P.ray_counts = nullptr;
     P.sum_pool = nullptr;
@@ -4209,7 +4209,6 @@ static void prepare_forward(MarchParams &P, bool image_only, hipStream_t s)
     // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every tile has a CU of its own, and starts at once.
     const int64_t tiles = (int64_t)P.tiles_x * P.tiles_y;
     const bool team = by_team(P, image_only);
-    P.image_only = image_only;
     P.by_halves = image_only && !team && tiles <= RGX_HALF_TILES;
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);
@@ -4261,6 +4260,9 @@ static void launch_forward(const MarchParams &P, bool viewer, bool counting, boo
     } else if (P.records) {
         if (counting) RGX_FWD(true, false, true);
         else RGX_FWD(true, false, false);
+    } else if (!image_only) {
+        if (counting) hipLaunchKernelGGL((k_march_fwd<false, false, false, true, false, true>), grid, block, 0, s, P);
+        else hipLaunchKernelGGL((k_march_fwd<false, false, false, false, false, true>), grid, block, 0, s, P);
     } else {
         if (counting) RGX_FWD(false, false, true);
         else RGX_FWD(false, false, false);
