@@ -4187,8 +4187,9 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
 //     fixed step, 1 M in a ball of radius 2  5.14 / 3.35    5.14 / 3.27    4.43 / 3.00    3.97 / 2.69    3.24 / 3.10
 //     adaptive step, 60 k heavy-tailed       0.96 / 0.76    0.98 / 0.76    0.90 / 0.80    0.86 / 0.88    0.85 / 1.13
 //     adaptive step, 3 M heavy-tailed        4.52 / 3.75    4.42 / 3.62    4.25 / 3.57    3.93 / 4.45    3.55 / 4.97
-// The line lies below the first loss.  (Halves for the heaviest blocks only of an image with more tiles: 300 k 800x800 2.25 -> 2.73 ms for
-// 512 tiles of 10 000.)  Between 400 and 768 tiles four wavefronts per tile and halves win in turn.  A record is tile by tile.
+// One line for both steps, below the adaptive step's first loss (1 521); the fixed step still gains at 2 500 and would bear a line of its own, and between 400 and 768
+// tiles, where four wavefronts per tile and halves win in turn, there is no rule but the team's line.  (Halves for the heaviest blocks only of an image
+// with more tiles: 300 k 800x800 2.25 -> 2.73 ms for 512 tiles of 10 000.)  A record is tile by tile.
 #define RGX_HALF_TILES 1296
 
 // image_only: no backward follows this launch
