@@ -1378,29 +1378,26 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
 // classes/point_cloud.py:252).  As there: points sorted along a Morton curve, boxes of consecutive
 // sorted points, boxes that cannot hold one of the three nearest are left out (the pruning is exact,
 // so the result is the exact 3-NN mean whatever the order and the box size).
-// Here a wavefront searches for the consecutive points of the curve that it owns, together: three
-// levels of boxes (16 points, 64 leaves, 64 boxes), of which each lane tests one child against the
-// bounds of the wavefront's points and the largest distance any of them still has to beat; the leaves that
-// are left are tested by every lane for its own point, and a leaf that some lane needs is read once and met by
-// all lanes in straight-line code.  One lane searching on its own through boxes of
-// 256 points made every lane of a wavefront wait for the scans of all others.  A wavefront owns 64 points, or 32, 16 or 8 whose
-// 2, 4 or 8 lanes each meet their share of a leaf (knn_lanes): a large cloud is bound by the issue of the distance
-// computations (12 instructions per point and leaf point, with 64 points and the leaf's points as scalars), a small one by its
-// longest wavefront, which gets shorter with the stretch of the curve whose bounds it has to search.
-// The whole call, sort and boxes included, us, with 64 points a wavefront / with as many as knn_lanes says:
-//     heavy-tailed cloud of 1 000, 5 000, 20 000, 54 k, 150 k, 300 k, 1 M, 3 M  61/39 122/65 221/107 269/138 319/207 377/340 867/719 1 610
-//     ball or cube of 20 000, 54 k, 300 k, 1 M                                154/104 177/134 269/249 559/560
+// Here the curve is a Hilbert curve (k_knn_keys), and a wavefront searches for the consecutive points of it that it owns, in two steps.
+// Together: three levels of boxes (8 points, 64 leaves, 64 boxes), of which each lane tests one child against the bounds of the
+// wavefront's points, as a few runs, and the largest distance any of them still has to beat; the leaves that are left wait in a list.  Then each
+// lane by itself: it tests its share of the list for its own point, some twenty instructions a leaf, and meets the few leaves that can hold one of
+// its three.  A wavefront owns 32 points, or 16 or 8 whose 4 or 8 lanes share the list (knn_lanes): a large cloud is bound by the issue of the tests
+// and distances, a small one by its longest wavefront, which gets shorter with the stretch of the curve whose bounds it has to search.
+// The whole call, sort and boxes included, us; before (a Morton curve of the box between the outermost points, leaves of 16 met by all lanes of
+// the wavefront for all its points, 30 bits sorted at every size) / now:
+//     heavy-tailed cloud of 1 000, 5 000, 20 000, 54 k, 150 k, 300 k, 1 M, 3 M   36/29 57/48 78/66 119/83 177/109 472/150 681/351 1 612/924
+//     ball of as many                                                          35/26 53/39 77/56 112/70 159/102 230/142 537/309 1 362/795
+// On a Hilbert curve consecutive cells touch: a run of the Morton curve spans jumps, and its bounds meet twice the leaves (counted on the CPU).
 // Distances are (dx*dx + dy*dy) + dz*dz without contraction; rounding is monotone, so the distance to a
 // box that holds a point, computed the same way, is never larger than the distance to the point.
-#define RGX_KNN_LEAF 16
+#define RGX_KNN_LEAF 8
 #define RGX_KNN_FAN 64
 #define RGX_KNN_BOX (RGX_KNN_LEAF * RGX_KNN_FAN)
-#ifndef RGX_KNN_SEGS
-#define RGX_KNN_SEGS 4
-#endif
-#define RGX_KNN_NEAR 4 // leaves before and after a wavefront's own that it looks at first
+#define RGX_KNN_SEGS(C) ((C) == 8 ? 2 : 4) // runs that a wavefront's points are taken as: with two of 32 points 3 M heavy-tailed take 2.96 ms instead of 0.92
+#define RGX_KNN_QUEUE 64 // leaves that wait before the points choose among them
 
-// Gathers the sorted points and bounds them: one workgroup per box of 1024.  A point with a coordinate that is
+// Gathers the sorted points and bounds them: one workgroup per box.  A point with a coordinate that is
 // not a number is at no distance from any other: it becomes a point at infinity, and such points, like the
 // padding behind the last one, are in no box's bounds.
 __global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restrict__ pos, const uint32_t *__restrict__ order,
@@ -1418,22 +1415,27 @@ __global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restr
     const bool fin = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
     float mn[3] = {fin ? p.x : INFINITY, fin ? p.y : INFINITY, fin ? p.z : INFINITY};
     float mx[3] = {fin ? p.x : -INFINITY, fin ? p.y : -INFINITY, fin ? p.z : -INFINITY};
-    auto spread = [&](int o) {
+    auto spread = [&](auto ctrl, auto rows) {
         for (int a = 0; a < 3; ++a) {
-            mn[a] = fminf(mn[a], __shfl_xor(mn[a], o));
-            mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], o));
+            mn[a] = fminf(mn[a], dpp_f<decltype(ctrl)::value, decltype(rows)::value>(INFINITY, mn[a]));
+            mx[a] = fmaxf(mx[a], dpp_f<decltype(ctrl)::value, decltype(rows)::value>(-INFINITY, mx[a]));
         }
     };
-    for (int o = 1; o < RGX_KNN_LEAF; o <<= 1) spread(o);
+    const std::integral_constant<int, 0xf> all{};
+    spread(std::integral_constant<int, 0xB1>{}, all); // over two, four and the eight lanes of a leaf
+    spread(std::integral_constant<int, 0x4E>{}, all);
+    spread(std::integral_constant<int, 0x141>{}, all);
     if ((threadIdx.x & (RGX_KNN_LEAF - 1)) == 0) {
         const int64_t l = i / RGX_KNN_LEAF;
         leaves[2 * l] = make_float4(mn[0], mn[1], mn[2], 0.f);
         leaves[2 * l + 1] = make_float4(mx[0], mx[1], mx[2], 0.f);
     }
-    for (int o = RGX_KNN_LEAF; o < 64; o <<= 1) spread(o);
+    spread(std::integral_constant<int, 0x140>{}, all); // over the row, and over the rows, in the last lane
+    spread(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    spread(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
     __shared__ float red[RGX_KNN_BOX / 64][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0)
+    if (lane == 63)
         for (int a = 0; a < 3; ++a) {
             red[wave][a] = mn[a];
             red[wave][a + 3] = mx[a];
@@ -1450,13 +1452,132 @@ __global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restr
     }
 }
 
-__global__ __launch_bounds__(256) void k_knn_begin(int32_t *mn, int32_t *mx, int32_t *supers_enc, int64_t ns)
+// What the order of the points is made from, and the bounds of the boxes of boxes before any point is in them.
+// The order only decides how many boxes a search has to open, never what it finds, so it may be any curve.  It is a Hilbert
+// curve, whose consecutive cells always touch, through a grid that a sample of the cloud shapes: per axis linear where the bulk of the
+// points lies, logarithmic beyond (knn_warp).  A grid between the outermost points instead, as a few far points stretch it, leaves
+// thousands of the others in one cell, in whose order they say nothing of where they lie.
+#define RGX_KNN_SAMPLE 1024
+// Bits of the grid per axis: 24-bit keys are sorted in three passes, 30-bit keys in four.  Beyond half a million points a cell of the coarser grid
+// holds too many of them where a cloud is dense (us with 8 / 10 bits: 54 k heavy-tailed 83 / 101, 300 k 178 / 184, 1 M 408 / 352, ball 293 / 309).
+static inline int knn_bits(int64_t n) { return n <= 1 << 19 ? 8 : 10; }
+struct KnnGrid {
+    float centre[3], inv_spread[3], inv_reach[3]; // 1 / what knn_warp makes of the sample's outermost points, and a little more
+};
+__device__ __forceinline__ float knn_warp(float x, float centre, float inv_spread)
 {
-    if (threadIdx.x < 3) {
-        mn[threadIdx.x] = enc_f(INFINITY);
-        mx[threadIdx.x] = enc_f(-INFINITY);
+    const float u = (x - centre) * inv_spread, m = fabsf(u);
+    return copysignf(m < 1.f ? m : 1.f + __logf(m), u);
+}
+__global__ __launch_bounds__(256) void k_knn_begin(const float *__restrict__ pos, int64_t n, KnnGrid *grid, int32_t *supers_enc, int64_t ns)
+{
+    if (blockIdx.x > 0) {
+        for (int64_t k = (int64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x; k < 6 * ns; k += (int64_t)(gridDim.x - 1) * blockDim.x)
+            supers_enc[k] = enc_f(k % 6 < 3 ? INFINITY : -INFINITY);
+        return;
     }
-    for (int64_t k = threadIdx.x; k < 6 * ns; k += blockDim.x) supers_enc[k] = enc_f(k % 6 < 3 ? INFINITY : -INFINITY);
+    constexpr int EACH = RGX_KNN_SAMPLE / 256;
+    __shared__ float red[4][4][6];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto sum = [&](int use, float *v, int m, bool most) { // over the workgroup, in every thread; or the largest of the last three
+        for (int a = 0; a < m; ++a) {
+            v[a] = most && a >= m - 3 ? wave_max_all(v[a]) : wave_sum_all(v[a]);
+            if (lane == 0) red[use][wave][a] = v[a];
+        }
+        __syncthreads();
+        for (int a = 0; a < m; ++a) {
+            const float *r = &red[use][0][a];
+            v[a] = most && a >= m - 3 ? fmaxf(fmaxf(r[0], r[6]), fmaxf(r[12], r[18])) : (r[0] + r[6]) + (r[12] + r[18]);
+        }
+    };
+    float x[EACH][3], w[EACH]; // w: 0 for a point that has a coordinate without a finite value
+    for (int k = 0; k < EACH; ++k) {
+        const int64_t t = k * 256 + threadIdx.x;
+        // a few points: all of them; else places without a period that the points' own order could share
+        const int64_t i = n <= RGX_KNN_SAMPLE ? (t < n ? t : n - 1) : (int64_t)(((uint64_t)((uint32_t)t * 2654435761u) * (uint64_t)n) >> 32);
+        for (int a = 0; a < 3; ++a) x[k][a] = pos[3 * i + a];
+    }
+    float v[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < EACH; ++k) {
+        w[k] = fabsf(x[k][0]) < 1e30f && fabsf(x[k][1]) < 1e30f && fabsf(x[k][2]) < 1e30f ? 1.f : 0.f;
+        for (int a = 0; a < 3; ++a) {
+            x[k][a] = w[k] != 0.f ? x[k][a] : 0.f;
+            v[a] += x[k][a];
+        }
+        v[3] += w[k];
+    }
+    sum(0, v, 4, false);
+    const float count = fmaxf(v[3], 1.f);
+    float c[3], off[3]; // the mean, and the mean distance from it
+    for (int a = 0; a < 3; ++a) {
+        c[a] = v[a] / count;
+        v[a] = 0.f;
+        for (int k = 0; k < EACH; ++k) v[a] += w[k] * fabsf(x[k][a] - c[a]);
+    }
+    sum(1, v, 3, false);
+    for (int a = 0; a < 3; ++a) {
+        off[a] = v[a] / count;
+        v[a] = v[a + 3] = 0.f;
+        for (int k = 0; k < EACH; ++k) { // from the mean towards the median: weights fall with the distance
+            const float g = w[k] / (fabsf(x[k][a] - c[a]) + 0.05f * off[a] + 1e-30f);
+            v[a] += g * x[k][a];
+            v[a + 3] += g;
+        }
+    }
+    sum(2, v, 6, false);
+    for (int a = 0; a < 3; ++a) {
+        c[a] = v[a + 3] > 0.f ? v[a] / v[a + 3] : 0.f;
+        v[a] = v[a + 3] = 0.f;
+        for (int k = 0; k < EACH; ++k) {
+            const float d = fabsf(x[k][a] - c[a]);
+            v[a] += w[k] * __logf(fmaxf(d, 1e-3f * off[a]) + 1e-30f);
+            v[a + 3] = fmaxf(v[a + 3], w[k] * d);
+        }
+    }
+    sum(3, v, 6, true);
+    if (threadIdx.x < 3) {
+        const int a = threadIdx.x;
+        // the spread: the geometric mean distance from the centre; e of it is where an even spread ends
+        const float log_mean = a == 0 ? v[0] : a == 1 ? v[1] : v[2], far = a == 0 ? v[3] : a == 1 ? v[4] : v[5], centre = a == 0 ? c[0] : a == 1 ? c[1] : c[2];
+        const float spread = 2.7f * __expf(log_mean / count), inv = spread > 1e-25f ? 1.f / spread : 0.f;
+        grid->centre[a] = centre;
+        grid->inv_spread[a] = inv;
+        grid->inv_reach[a] = 1.f / fmaxf(1.05f * knn_warp(far, 0.f, inv), 1e-3f);
+    }
+}
+
+// The place of every point along a Hilbert curve of 2^30 cells (the transposed form of J. Skilling, "Programming the Hilbert curve", 2004).
+__global__ __launch_bounds__(256) void k_knn_keys(const float *__restrict__ pos, int64_t n, const KnnGrid *__restrict__ grid, int bits,
+                                                  uint32_t *__restrict__ keys, uint32_t *__restrict__ vals)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t top = 1u << (bits - 1);
+    const float half = (float)top;
+    uint32_t q[3];
+    for (int a = 0; a < 3; ++a) {
+        const float u = knn_warp(pos[3 * i + a], grid->centre[a], grid->inv_spread[a]) * grid->inv_reach[a];
+        q[a] = (uint32_t)(half + (half - 1.f) * fminf(fmaxf(u, -1.f), 1.f)); // (not a number: the grid's edge)
+    }
+    for (uint32_t m = top; m > 1; m >>= 1)
+        for (int a = 0; a < 3; ++a) {
+            const uint32_t t = (q[0] ^ q[a]) & (m - 1);
+            if (q[a] & m) {
+                q[0] ^= m - 1;
+            } else {
+                q[0] ^= t;
+                q[a] ^= t;
+            }
+        }
+    q[1] ^= q[0];
+    q[2] ^= q[1];
+    uint32_t t = 0;
+    for (uint32_t m = top; m > 1; m >>= 1) t ^= q[2] & m ? m - 1 : 0u;
+    uint32_t code = 0;
+    for (int b = bits - 1; b >= 0; --b)
+        for (int a = 0; a < 3; ++a) code = code << 1 | ((q[a] ^ t) >> b & 1u);
+    keys[i] = code;
+    vals[i] = (uint32_t)i;
 }
 
 // Squared distance between two boxes (a point is a box of no size): simple_knn.cu:124-135 distBoxPoint.
@@ -1468,10 +1589,22 @@ __device__ __forceinline__ float knn_box_dist(f3 lo, f3 hi, f3 qlo, f3 qhi)
     return (dx * dx + dy * dy) + dz * dz;
 }
 
-// Lanes per point.  The lines lie where the larger number stops gaining for either kind of cloud (us with 8 / 4 / 2 / 1 lanes a
-// point: 54 k heavy-tailed 138 / 151 / 168 / 269, ball 134 / 132 / 139 / 177; 150 k heavy-tailed 225 / 207 / 253 / 319; 300 k 341 / 350 /
-// 340 / 377, ball 300 / 249 / 248 / 269; 1 M 925 / 693 / 719 / 867, ball 782 / 602 / 560 / 559; 3 M 2 739 / 1 965 / 1 705 / 1 610).
-static inline int knn_lanes(int64_t n) { return n <= 1 << 16 ? 8 : n <= 1 << 18 ? 4 : n <= 1 << 20 ? 2 : 1; }
+// Lanes per point (us with 8 / 4 / 2 lanes, keys of 30 bits: heavy-tailed 5 000 52 / 59 / 80, 54 k 101 / 101 / 244, 150 k 120 / 126 / 230, 300 k
+// 184 / 167 / 215, 1 M 474 / 375 / 352, 3 M 1 133 / 976 / 924; ball 54 k 85 / 85 / 95, 300 k 161 / 160 / 154, 1 M 360 / 345 / 309, 3 M 991 / 920 / 795).
+static inline int knn_lanes(int64_t n) { return n <= 1 << 18 ? 8 : n <= 1 << 19 ? 4 : 2; }
+
+// the smallest of the first P lanes' values (all lanes must be active)
+template <int P> __device__ __forceinline__ float first_min(float v)
+{
+    v = fminf(v, dpp_f<0xB1, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x4E, 0xf>(INFINITY, v));
+    v = fminf(v, dpp_f<0x141, 0xf>(INFINITY, v));
+    if constexpr (P > 8) v = fminf(v, dpp_f<0x140, 0xf>(INFINITY, v));
+    if constexpr (P > 16) v = fminf(v, dpp_f<0x142, 0xa>(INFINITY, v));
+    if constexpr (P > 32) v = fminf(v, dpp_f<0x143, 0xc>(INFINITY, v));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), P - 1));
+}
+template <int P> __device__ __forceinline__ float first_max(float v) { return -first_min<P>(-v); }
 
 // simple_knn.cu:137-184 updateKBest<3>, boxMeanDist.  C: lanes per point.
 template <int C>
@@ -1479,24 +1612,28 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
                                               const float4 *__restrict__ leaves, const float4 *__restrict__ boxes, int64_t nb,
                                               const int32_t *__restrict__ supers_enc, int64_t ns, float *__restrict__ out)
 {
-    constexpr int P = 64 / C, EACH = RGX_KNN_LEAF / C; // points of a wavefront; points of a leaf that a lane meets
+    static_assert(RGX_KNN_LEAF == 8, "eight lanes hold a leaf");
+    constexpr int P = 64 / C, SHARE = 2 * RGX_KNN_QUEUE / C; // points of a wavefront; waiting leaves that a lane looks at, at most
+    constexpr int WORDS = (SHARE + 31) / 32;
+    constexpr int SEGS = RGX_KNN_SEGS(C);
+    __shared__ int queue[4][2 * RGX_KNN_QUEUE];
     const int lane = threadIdx.x & 63, copy = lane / P;
+    int *const list = queue[threadIdx.x >> 6];
     const int64_t first = __builtin_amdgcn_readfirstlane((int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6)) * (int64_t)P;
     if (first >= n) return; // whole wave
     const int64_t i = first + (lane & (P - 1));
     const float4 p4 = pts[i]; // (the array is padded to whole boxes)
     const f3 p = mk3(p4.x, p4.y, p4.z);
     const bool act = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
-    // The wavefront's points as RGX_KNN_SEGS runs of the curve, cut where it jumps farthest: the bounds of a run that
-    // spans such a jump would meet most of the cloud (one such wavefront was the whole launch's time).
+    // The wavefront's points as SEGS runs of the curve, cut where it jumps farthest: the bounds of a run that
+    // spans such a jump would meet most of the cloud.
     uint64_t cuts = 0; // over the first P lanes
     {
-        const f3 prev = mk3(__shfl_up(p.x, 1), __shfl_up(p.y, 1), __shfl_up(p.z, 1));
-        const f3 step = p - prev;
+        const f3 step = p - mk3(__shfl_up(p.x, 1), __shfl_up(p.y, 1), __shfl_up(p.z, 1));
         float gap = lane > 0 && lane < P ? dot3(step, step) : -1.f;
         if (!(gap < INFINITY)) gap = -1.f;
-        for (int k = 1; k < RGX_KNN_SEGS; ++k) {
-            const float g = wave_max_all(gap);
+        for (int k = 1; k < SEGS; ++k) {
+            const float g = first_max<P>(gap);
             const uint64_t at = __ballot(gap == g && g > 0.f);
             if (at == 0) break;
             cuts |= at & -at;
@@ -1504,12 +1641,12 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
         }
     }
     const int seg = __popcll(cuts & (~0ull >> (63 - (lane & (P - 1)))));
-    f3 slo[RGX_KNN_SEGS], shi[RGX_KNN_SEGS];
-    float reach[RGX_KNN_SEGS]; // the largest distance a point of the run still has to beat
-    for (int k = 0; k < RGX_KNN_SEGS; ++k) {
+    f3 slo[SEGS], shi[SEGS];
+    float reach[SEGS]; // the largest distance a point of the run still has to beat
+    for (int k = 0; k < SEGS; ++k) {
         const bool in = act && seg == k;
-        slo[k] = mk3(wave_min_all(in ? p.x : INFINITY), wave_min_all(in ? p.y : INFINITY), wave_min_all(in ? p.z : INFINITY));
-        shi[k] = mk3(wave_max_all(in ? p.x : -INFINITY), wave_max_all(in ? p.y : -INFINITY), wave_max_all(in ? p.z : -INFINITY));
+        slo[k] = mk3(first_min<P>(in ? p.x : INFINITY), first_min<P>(in ? p.y : INFINITY), first_min<P>(in ? p.z : INFINITY));
+        shi[k] = mk3(first_max<P>(in ? p.x : -INFINITY), first_max<P>(in ? p.y : -INFINITY), first_max<P>(in ? p.z : -INFINITY));
     }
     float b0 = FLT_MAX, b1 = FLT_MAX, b2 = FLT_MAX; // the three smallest that this lane has met, ascending
     auto put = [](float &c0, float &c1, float &c2, float d) {
@@ -1517,16 +1654,10 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
         c1 = __builtin_amdgcn_fmed3f(c0, c1, d);
         c0 = fminf(c0, d);
     };
-    auto meet = [&](int l, auto own) { // all points of leaf l (the same in every lane)
-        l = __builtin_amdgcn_readfirstlane(l);
-        const float4 *q = pts + (int64_t)l * RGX_KNN_LEAF + (C > 1 ? copy * EACH : 0);
-#pragma unroll
-        for (int k = 0; k < EACH; ++k) {
-            const float dx = q[k].x - p.x, dy = q[k].y - p.y, dz = q[k].z - p.z;
-            float d = (dx * dx + dy * dy) + dz * dz;
-            if constexpr (decltype(own)::value) d = (int64_t)l * RGX_KNN_LEAF + copy * EACH + k == i ? FLT_MAX : d;
-            put(b0, b1, b2, d);
-        }
+    auto meet = [&](f3 q, bool not_itself = true) {
+        const float dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
+        const float d = (dx * dx + dy * dy) + dz * dz;
+        put(b0, b1, b2, not_itself ? d : FLT_MAX);
     };
     float t0, t1, worst; // the three smallest that the point's lanes have met
     auto measure = [&]() {
@@ -1539,54 +1670,125 @@ __global__ __launch_bounds__(256) void k_knn3(const float4 *__restrict__ pts, co
             put(t0, t1, worst, o1);
             put(t0, t1, worst, o2);
         }
-        for (int k = 0; k < RGX_KNN_SEGS; ++k) reach[k] = wave_max_all(act && seg == k ? worst : -1.f);
+        for (int k = 0; k < SEGS; ++k) reach[k] = first_max<P>(act && seg == k ? worst : -1.f);
     };
-    // the points nearby on the curve first: they leave little for the boxes
-    const int leaf0 = (int)(first / RGX_KNN_LEAF), leaf1 = (int)((first + P - 1) / RGX_KNN_LEAF) + 1;
-    for (int l = leaf0; l < leaf1; ++l) meet(l, std::true_type{});
-    const int n_leaves = (int)(nb * RGX_KNN_FAN);
-    const int done0 = std::max(leaf0 - RGX_KNN_NEAR, 0), done1 = std::min(leaf1 + RGX_KNN_NEAR, n_leaves);
-    for (int l = done0; l < leaf0; ++l) meet(l, std::false_type{});
-    for (int l = leaf1; l < done1; ++l) meet(l, std::false_type{});
+    // The points nearby on the curve first, those of the point's own leaf and of the two beside it: they leave little for the boxes.
+    // Eight lanes hold a leaf and hand its points around among themselves.
+    const int own = (int)(i / RGX_KNN_LEAF), n_leaves = (int)(nb * RGX_KNN_FAN);
+    for (int turn = copy; turn < (C > 3 ? C : 3); turn += C) { // (a leaf's eight lanes take the same turns)
+        const int l = turn == 0 ? own : turn == 1 ? own - 1 : own + 1;
+        const bool there = turn < 3 && l >= 0 && l < n_leaves;
+        const float4 q4 = pts[(int64_t)(there ? l : own) * RGX_KNN_LEAF + (lane & (RGX_KNN_LEAF - 1))];
+        const f3 q = mk3(there ? q4.x : INFINITY, q4.y, q4.z);
+        auto across = [](f3 v, auto ctrl) {
+            constexpr int X = decltype(ctrl)::value;
+            return mk3(dpp_f<X, 0xf>(v.x, v.x), dpp_f<X, 0xf>(v.y, v.y), dpp_f<X, 0xf>(v.z, v.z));
+        };
+        const std::integral_constant<int, 0xB1> by1{}; // lanes of a quad exchanged: with the neighbour,
+        const std::integral_constant<int, 0x4E> by2{}; // with the one after it,
+        const std::integral_constant<int, 0x1B> by3{}; // mirrored
+        const f3 r = across(q, std::integral_constant<int, 0x141>{}); // the eight lanes mirrored
+        meet(q, l != own);
+        meet(across(q, by1));
+        meet(across(q, by2));
+        meet(across(q, by3));
+        meet(r);
+        meet(across(r, by1));
+        meet(across(r, by2));
+        meet(across(r, by3));
+    }
     measure();
     auto open = [&](f3 lo, f3 hi) { // is the box within some run's reach?
         bool o = false;
-        for (int k = 0; k < RGX_KNN_SEGS; ++k) o |= knn_box_dist(lo, hi, slo[k], shi[k]) < reach[k];
+        for (int k = 0; k < SEGS; ++k) o |= knn_box_dist(lo, hi, slo[k], shi[k]) < reach[k];
         return o;
     };
-    auto open_at = [&](const float4 *b) {
-        const float4 lo = b[0], hi = b[1];
-        return open(mk3(lo.x, lo.y, lo.z), mk3(hi.x, hi.y, hi.z));
-    };
-    for (int64_t s0 = 0; s0 < ns; s0 += 64) {
-        bool super = false;
-        if (s0 + lane < ns) {
-            const int32_t *e = supers_enc + 6 * (s0 + lane);
-            super = open(mk3(dec_f(e[0]), dec_f(e[1]), dec_f(e[2])), mk3(dec_f(e[3]), dec_f(e[4]), dec_f(e[5])));
-        }
-        for (uint64_t ms = __ballot(super); ms; ms &= ms - 1) {
-            const int64_t box0 = (s0 + __builtin_ctzll(ms)) * RGX_KNN_FAN;
-            for (uint64_t mb = __ballot(box0 + lane < nb && open_at(boxes + 2 * (box0 + lane))); mb; mb &= mb - 1) {
-                const int l0 = (int)(box0 + __builtin_ctzll(mb)) * RGX_KNN_FAN;
-                const float4 lo = leaves[2 * (int64_t)(l0 + lane)], hi = leaves[2 * (int64_t)(l0 + lane) + 1];
-                const bool near = (l0 + lane < done0 || l0 + lane >= done1) && open(mk3(lo.x, lo.y, lo.z), mk3(hi.x, hi.y, hi.z));
-                const uint64_t some = __ballot(near);
-                for (uint64_t ml = some; ml; ml &= ml - 1) {
-                    const int t = __builtin_ctzll(ml);
-                    auto at = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), t)); };
-                    const float d = knn_box_dist(mk3(at(lo.x), at(lo.y), at(lo.z)), mk3(at(hi.x), at(hi.y), at(hi.z)), p, p);
-                    if (__any(act && d < worst)) meet(l0 + t, std::false_type{});
+    int waiting = 0; // leaves in the list
+    // Of its share of the leaves in the list every lane chooses those that can hold one of its point's three, and meets them by itself.
+    auto choose = [&]() {
+        __builtin_amdgcn_wave_barrier();
+        uint32_t mine[WORDS] = {};
+        const int rounds = (waiting + C - 1) / C;
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w)
+            for (int c0 = 32 * w; c0 < rounds && c0 < 32 * w + 32; c0 += 4) {
+                int l[4];
+                float4 lo[4], hi[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    l[k] = list[std::min((c0 + k) * C + copy, waiting - 1)];
+                    lo[k] = leaves[2 * (int64_t)l[k]];
+                    hi[k] = leaves[2 * (int64_t)l[k] + 1];
                 }
-                if (some) measure();
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const bool near = knn_box_dist(mk3(lo[k].x, lo[k].y, lo[k].z), mk3(hi[k].x, hi[k].y, hi[k].z), p, p) < worst &&
+                                      (uint32_t)(l[k] - own + 1) > 2u && (c0 + k) * C + copy < waiting;
+                    mine[w] |= near ? 1u << (c0 + k - 32 * w) : 0u;
+                }
+            }
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w) {
+            if (!act) mine[w] = 0;
+            while (mine[w]) {
+                const int l = list[(32 * w + __builtin_ctz(mine[w])) * C + copy];
+                mine[w] &= mine[w] - 1;
+                const float4 *q = pts + (int64_t)l * RGX_KNN_LEAF;
+#pragma unroll
+                for (int k = 0; k < RGX_KNN_LEAF; ++k) meet(mk3(q[k].x, q[k].y, q[k].z));
             }
         }
+        __builtin_amdgcn_wave_barrier();
+        waiting = 0;
+        measure();
+    };
+    // The children that lie within reach, one in each lane, one after the other.  More than MANY of them are open to a run that has not met
+    // its neighbours yet (points between a dense part and a sparse one): then the nearest first, and the others only if they
+    // are still within reach.
+    auto each_open = [&](bool there, f3 lo, f3 hi, int many, auto visit) {
+        uint64_t todo = __ballot(there && open(lo, hi));
+        while (todo) {
+            int t = __builtin_ctzll(todo);
+            const bool nearest = __popcll(todo) > many;
+            if (nearest) {
+                float d = INFINITY;
+                for (int k = 0; k < SEGS; ++k) d = fminf(d, knn_box_dist(lo, hi, slo[k], shi[k]));
+                if (!(todo >> lane & 1)) d = INFINITY;
+                const uint64_t at = __ballot(d == wave_min_all(d)) & todo;
+                if (at) t = __builtin_ctzll(at);
+            }
+            todo &= ~(1ull << t);
+            visit(t);
+            if (nearest) {
+                if (waiting) choose();
+                todo &= __ballot(open(lo, hi));
+            }
+        }
+    };
+    for (int64_t s0 = 0; s0 < ns; s0 += 64) {
+        const int32_t *e = supers_enc + 6 * std::min(s0 + lane, ns - 1);
+        each_open(s0 + lane < ns, mk3(dec_f(e[0]), dec_f(e[1]), dec_f(e[2])), mk3(dec_f(e[3]), dec_f(e[4]), dec_f(e[5])), 4, [&](int ts) {
+            const int64_t box0 = (s0 + ts) * RGX_KNN_FAN;
+            const float4 *b = boxes + 2 * std::min(box0 + lane, nb - 1);
+            const float4 blo = b[0], bhi = b[1];
+            each_open(box0 + lane < nb, mk3(blo.x, blo.y, blo.z), mk3(bhi.x, bhi.y, bhi.z), 8, [&](int tb) {
+                const int l = (int)(box0 + tb) * RGX_KNN_FAN + lane;
+                const float4 lo = leaves[2 * (int64_t)l], hi = leaves[2 * (int64_t)l + 1];
+                const bool wanted = open(mk3(lo.x, lo.y, lo.z), mk3(hi.x, hi.y, hi.z));
+                const uint64_t some = __ballot(wanted);
+                if (wanted) list[waiting + __popcll(some & ((1ull << lane) - 1ull))] = l;
+                waiting += __popcll(some);
+                if (waiting >= RGX_KNN_QUEUE) choose();
+            });
+        });
     }
+    if (waiting) choose();
     if (i < n && copy == 0) out[order[i]] = act ? ((t0 + t1) + worst) / 3.0f : INFINITY;
 }
 
 struct KnnLayout {
     MortonLayout m;
-    size_t pts, leaves, boxes, supers, total;
+    size_t pts, leaves, boxes, supers, grid, total;
     int64_t nb, ns;
 };
 static inline KnnLayout knn_layout(int64_t n)
@@ -1601,6 +1803,7 @@ static inline KnnLayout knn_layout(int64_t n)
     K.leaves = off; off = rgx_align_up(off + (size_t)K.nb * RGX_KNN_FAN * 32, 256);
     K.boxes = off;  off = rgx_align_up(off + (size_t)K.nb * 32, 256);
     K.supers = off; off = rgx_align_up(off + (size_t)K.ns * 24, 256);
+    K.grid = off;   off = rgx_align_up(off + sizeof(KnnGrid), 256);
     K.total = off;
     return K;
 }
@@ -1621,27 +1824,27 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     if (n == 0) return RGX_OK;
     hipStream_t s = (hipStream_t)stream;
     char *w = (char *)ws;
-    int32_t *mn = (int32_t *)(w + K.m.enc), *mx = mn + 4;
     uint32_t *k0 = (uint32_t *)(w + K.m.keys0), *k1 = (uint32_t *)(w + K.m.keys1);
     uint32_t *v0 = (uint32_t *)(w + K.m.vals0), *v1 = (uint32_t *)(w + K.m.vals1);
     float4 *pts = (float4 *)(w + K.pts), *leaves = (float4 *)(w + K.leaves), *boxes = (float4 *)(w + K.boxes);
     int32_t *supers = (int32_t *)(w + K.supers);
-    hipLaunchKernelGGL(k_knn_begin, dim3(1), dim3(256), 0, s, mn, mx, supers, K.ns);
-    hipLaunchKernelGGL(k_pos_minmax, grid_reduce(n, 128), dim3(RGX_REDUCE_THREADS), 0, s, pos, n, mn, mx);
-    hipLaunchKernelGGL(k_morton30, grid_for(n, 256), dim3(256), 0, s, pos, n, mn, mx, k0, v0, (int64_t *)nullptr);
+    KnnGrid *grid = (KnnGrid *)(w + K.grid);
+    const int bits = knn_bits(n);
+    hipLaunchKernelGGL(k_knn_begin, dim3(1 + (unsigned)std::min<int64_t>((6 * K.ns + 255) / 256, 256)), dim3(256), 0, s, pos, n, grid, supers, K.ns);
+    hipLaunchKernelGGL(k_knn_keys, grid_for(n, 256), dim3(256), 0, s, pos, n, grid, bits, k0, v0);
     RGX_LAUNCH_CHECK();
-    const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 32, (uint32_t *)(w + K.m.hist), s);
+    const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 3 * bits, (uint32_t *)(w + K.m.hist), s);
     if (r < 0) return r;
-    hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)K.nb), dim3(RGX_KNN_BOX), 0, s, pos, v0, n, pts, leaves, boxes, supers);
+    const uint32_t *order = r ? v1 : v0;
+    hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)K.nb), dim3(RGX_KNN_BOX), 0, s, pos, order, n, pts, leaves, boxes, supers);
     const auto search = [&](auto lanes) {
         constexpr int C = decltype(lanes)::value;
-        hipLaunchKernelGGL(k_knn3<C>, grid_for(n * C, 256), dim3(256), 0, s, pts, v0, n, leaves, boxes, K.nb, supers, K.ns, mean_dist2);
+        hipLaunchKernelGGL(k_knn3<C>, grid_for(n * C, 256), dim3(256), 0, s, pts, order, n, leaves, boxes, K.nb, supers, K.ns, mean_dist2);
     };
     switch (knn_lanes(n)) {
     case 8: search(std::integral_constant<int, 8>{}); break;
     case 4: search(std::integral_constant<int, 4>{}); break;
-    case 2: search(std::integral_constant<int, 2>{}); break;
-    default: search(std::integral_constant<int, 1>{});
+    default: search(std::integral_constant<int, 2>{});
     }
     RGX_LAUNCH_CHECK();
     return RGX_OK;

@@ -66,6 +66,16 @@ __device__ __forceinline__ float wave_min_all(float v)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 __device__ __forceinline__ float wave_max_all(float v) { return -wave_min_all(-v); }
+__device__ __forceinline__ float wave_sum_all(float v)
+{
+    v += dpp_f<0xB1, 0xf>(0.f, v);
+    v += dpp_f<0x4E, 0xf>(0.f, v);
+    v += dpp_f<0x141, 0xf>(0.f, v);
+    v += dpp_f<0x140, 0xf>(0.f, v);
+    v += dpp_f<0x142, 0xa>(0.f, v);
+    v += dpp_f<0x143, 0xc>(0.f, v);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
 
 // 64-byte primitive record (cuda_train/forward/gaussians_aabb.h:7-12).
 struct __align__(16) Prim {

@@ -1098,6 +1098,36 @@ def test_dist2_knn3_with_any_number_of_lanes_per_point(gx, n):
     assert np.isfinite(got[9001:]).all()
 
 
+@pytest.mark.parametrize("n", [7, 8, 9, 511, 512, 513, 8192, 8193, 32_767, 32_768, 32_769])
+def test_dist2_knn3_at_the_sizes_of_leaves_and_boxes(gx, orc, n):
+    """Either side of a leaf of eight, a box of 64 leaves, a box of 64 boxes and the sort in one workgroup; half of the points far out and
+    sparse, so that the runs between the two halves have many boxes open at first."""
+    from raygaussx_amd.simple_knn import distCUDA2
+    rng = np.random.default_rng(n)
+    p = rng.normal(size=(n, 3)).astype(np.float32)
+    p[n // 2:] *= (rng.uniform(10.0, 50.0, size=(n - n // 2, 1)) / np.linalg.norm(p[n // 2:], axis=1, keepdims=True)).astype(np.float32)
+    _step(f"distCUDA2 n={n}")
+    got = distCUDA2(torch.from_numpy(p).to(gx.DEV)).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), orc.dist2_knn3(p).view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [524_287, 524_288, 524_289])
+def test_dist2_knn3_where_its_grid_changes(gx, n):
+    """Either side of the size from which the curve's grid has ten bits per axis and a point two lanes, against a k-d tree: squared distances are
+    rounded five times, 3e-7 of themselves, and their mean three times."""
+    from scipy.spatial import cKDTree
+    from raygaussx_amd.simple_knn import distCUDA2
+    rng = np.random.default_rng(n)
+    p = rng.normal(size=(n, 3)).astype(np.float32)
+    p[: n // 3] *= 20.0
+    p[5] = p[6] = p[7] = p[8]
+    _step(f"distCUDA2 n={n}")
+    got = distCUDA2(torch.from_numpy(p).to(gx.DEV)).cpu().numpy()
+    ids = np.concatenate([[5, n - 1], rng.choice(n, 3000, replace=False)])
+    d, _ = cKDTree(p.astype(np.float64)).query(p[ids].astype(np.float64), k=4)
+    np.testing.assert_allclose(got[ids], (d[:, 1:] ** 2).mean(1), rtol=1e-6)
+
+
 @pytest.mark.parametrize("kind", ["outliers", "two clumps", "nan", "inf", "nan and inf", "all nan", "huge"])
 def test_dist2_knn3_of_clouds_that_the_curve_does_not_sort(gx, orc, kind):
     """A few far points leave nearly all the others in one or two cells of the Morton grid, in whose order they say nothing of
