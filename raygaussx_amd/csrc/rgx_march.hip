@@ -84,7 +84,7 @@ struct MarchParams {
     uint32_t *tile_order;   // launch order lists (or null: as launched)
     int32_t use_tile_order; // 0: as launched; 1: per XCD, its tiles' list positions from the heaviest to the lightest (k_tile_order);
                             // 2: per XCD, the blocks of tiles it renders, heaviest first (k_block_order)
-    int32_t by_halves;      // forward of an image: two workgroups per tile (launch_forward)
+    int32_t part_bits;      // forward of an image: each tile by 2^part_bits workgroups (launch_forward)
     float4 *sum_pool;       // sample-sum slots of the record (RGX_SUM_SLOT_WORDS each), or null
     uint32_t *sum_next;     // next free slot (bump counter in the record's pool header)
     int32_t sum_slots;      // slots in the pool
@@ -309,12 +309,12 @@ __device__ __forceinline__ f3 plane_normal(f3 a, f3 b, f3 inside)
     return dot3(n, inside) > 0.f ? n * -1.0f : n;
 }
 
-// height: of the tile, in pixels (a half tile's is 4)
-__device__ __forceinline__ void frustum_planes(const RgxCamera &cam, int px0, int py0, Frustum &F, int height = 8)
+// width, height: in pixels (of a tile, or of the part of one that a wavefront marches)
+__device__ __forceinline__ void frustum_planes(const RgxCamera &cam, int px0, int py0, Frustum &F, int width = 8, int height = 8)
 {
-    const f3 d00 = compute_ray(cam, (unsigned)px0, (unsigned)py0), d10 = compute_ray(cam, (unsigned)(px0 + 7), (unsigned)py0);
+    const f3 d00 = compute_ray(cam, (unsigned)px0, (unsigned)py0), d10 = compute_ray(cam, (unsigned)(px0 + width - 1), (unsigned)py0);
     const f3 d01 = compute_ray(cam, (unsigned)px0, (unsigned)(py0 + height - 1));
-    const f3 d11 = compute_ray(cam, (unsigned)(px0 + 7), (unsigned)(py0 + height - 1));
+    const f3 d11 = compute_ray(cam, (unsigned)(px0 + width - 1), (unsigned)(py0 + height - 1));
     const f3 in = (d00 + d10) + (d01 + d11);
     F.o = mk3(cam.eye[0], cam.eye[1], cam.eye[2]);
     F.n[0] = plane_normal(d00, d01, in);
@@ -888,15 +888,15 @@ __host__ __device__ __forceinline__ TileGrid tile_grid(int tiles_x, int tiles_y)
     g.per_xcd = (g.blocks_x * blocks_y + 7) >> 3;
     return g;
 }
-__device__ __forceinline__ bool tile_origin(const MarchParams &P, unsigned id, int &px0, int &py0, int *tile_out = nullptr, int *half = nullptr)
+__device__ __forceinline__ bool tile_origin(const MarchParams &P, unsigned id, int &px0, int &py0, int *tile_out = nullptr, int part_bits = 0, int *part = nullptr)
 {
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int xcd = id & 7;
     const int per_block = g.bw * g.bh;
     int j = id >> 3;
-    if (half && P.by_halves) { // upper 0, lower 1
-        *half = j & 1;
-        j >>= 1;
+    if (part) {
+        *part = j & ((1 << part_bits) - 1);
+        j >>= part_bits;
     }
     int block;
     if (P.use_tile_order == 2) {
@@ -1234,6 +1234,129 @@ struct SampleBlock {
     }
 };
 
+// a's upper 32 lanes and b's lower 32 lanes change places; the same with the rows of 16 of each half
+__device__ __forceinline__ void swap32(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+// the value of each of the four copies of a ray, in every copy
+__device__ __forceinline__ void copies(float v, float (&out)[4])
+{
+    float a = v, b = v; // -> a: copies 0 and 1 (in the lower and upper rows of both halves), b: copies 2 and 3
+    swap32(a, b);
+    float a1 = a, b1 = b;
+    swap16(a, a1);
+    swap16(b, b1);
+    out[0] = a; out[1] = a1; out[2] = b; out[3] = b1;
+}
+// 16 values per lane -> four: copy `sub` gets the sums over the copies of v[4 sub .. 4 sub + 3]
+__device__ __forceinline__ void sum_copies(float (&v)[RGX_CHUNK_SIZE], float (&out)[4])
+{
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        swap32(v[i], v[i + 8]);
+        v[i] += v[i + 8];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        swap16(v[i], v[i + 4]);
+        out[i] = v[i] + v[i + 4];
+    }
+}
+
+// Parts of tiles.  A wavefront that marches only RAYS of a tile's 64 rays has each of them 64 / RAYS times over (lane = RAYS * copy + ray).  The
+// copies test as many table entries at a time, and each shades every 64 / RAYS-th hit.
+template <int RAYS>
+struct Part {
+    static_assert(RAYS == 64 || RAYS == 32 || RAYS == 16 || RAYS == 8, "a tile; its upper or lower half; a 4x4 block; 4x2 pixels");
+    static constexpr int COPIES = 64 / RAYS, BITS = RAYS == 64 ? 0 : RAYS == 32 ? 1 : RAYS == 16 ? 2 : 3;
+    static constexpr int WIDTH = RAYS < 32 ? 4 : 8, HEIGHT = RAYS / WIDTH; // in pixels
+    static constexpr int EACH = RGX_CHUNK_SIZE / COPIES;                   // samples of a chunk that a copy blends
+    // what the lanes of copy s say, said by all copies
+    static __device__ __forceinline__ uint64_t spread(uint64_t lanes, int s)
+    {
+        const uint32_t own = (uint32_t)(lanes >> (RAYS * s));
+        const uint32_t word = RAYS == 32 ? own : RAYS == 16 ? (own & 0xffffu) * 0x10001u : (own & 0xffu) * 0x1010101u;
+        return (uint64_t)word << 32 | word;
+    }
+    // hits without the first n of them, n < COPIES
+    static __device__ __forceinline__ uint32_t skip(uint32_t bits, int n)
+    {
+        for (int k = 0; k < COPIES - 1; ++k) bits = n > k ? bits & (bits - 1u) : bits;
+        return bits;
+    }
+    static __device__ __forceinline__ float other_half_row(float v) // (row_ror:8)
+    {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
+    }
+    // the value of each copy of a ray, in every copy
+    static __device__ __forceinline__ void of_all(float v, float (&out)[COPIES])
+    {
+        if constexpr (RAYS == 32) {
+            float a = v, b = v;
+            swap32(a, b);
+            out[0] = a;
+            out[1] = b;
+        } else if constexpr (RAYS == 16) {
+            copies(v, out);
+        } else {
+            const float o = other_half_row(v);
+            const bool odd = threadIdx.x & 8;
+            float even_ones[4], odd_ones[4];
+            copies(odd ? o : v, even_ones);
+            copies(odd ? v : o, odd_ones);
+#pragma unroll
+            for (int k = 0; k < COPIES; ++k) out[k] = k & 1 ? odd_ones[k >> 1] : even_ones[k >> 1];
+        }
+    }
+    static __device__ __forceinline__ float sum_of_all(float v)
+    {
+        float c[COPIES];
+        of_all(v, c);
+        float sum = c[0];
+        for (int k = 1; k < COPIES; ++k) sum += c[k];
+        return sum;
+    }
+    static __device__ __forceinline__ float least_of_all(float v)
+    {
+        float c[COPIES];
+        of_all(v, c);
+        float least = c[0];
+        for (int k = 1; k < COPIES; ++k) least = fminf(least, c[k]);
+        return least;
+    }
+    // a chunk's values per lane -> copy c gets the sums over the copies of the c-th run of EACH of them
+    static __device__ __forceinline__ void sums(float (&v)[RGX_CHUNK_SIZE], float (&out)[EACH])
+    {
+        if constexpr (RAYS == 32) {
+#pragma unroll
+            for (int i = 0; i < EACH; ++i) {
+                swap32(v[i], v[i + EACH]);
+                out[i] = v[i] + v[i + EACH];
+            }
+        } else if constexpr (RAYS == 16) {
+            sum_copies(v, out);
+        } else {
+            float four[4];
+            sum_copies(v, four); // over the copies of the lane's half of the row: samples 4 row .. 4 row + 3
+            const bool odd = threadIdx.x & 8;
+#pragma unroll
+            for (int i = 0; i < EACH; ++i) { // two of the four, from both halves
+                const float mine = odd ? four[i + EACH] : four[i], theirs = odd ? four[i] : four[i + EACH];
+                out[i] = mine + other_half_row(theirs);
+            }
+        }
+    }
+};
+
 // What one lane asks of the candidate table in this iteration.
 struct LaneQuery {
     f3 dir;
@@ -1366,6 +1489,126 @@ __device__ __forceinline__ void filter_table(const TileLds &L, int C, float t0, 
     __syncthreads();
 }
 
+// filter_table for a part of a tile: as many entries at a time as a ray has copies.
+template <int RAYS, typename Cn>
+__device__ __forceinline__ void filter_part(const TileLds &L, int C, float t0, float t1, const LaneQuery &Q, int part, bool plain,
+                                            int &p0, bool &ov, float &found, int &len_out, uint32_t (&own)[2], Cn &cn)
+{
+    constexpr int COPIES = 64 / RAYS;
+    const int lane = threadIdx.x, copy = lane / RAYS;
+    int len = 0;
+    uint32_t first = 0, second = 0; // the ray's hits with samples in the first / second half (the same in all copies)
+    int slots = 0;                  // lane i: slot of entry i of the list's current 64
+    own[0] = own[1] = 0u;
+    const bool asks = Q.need && !Q.search;
+    const uint64_t searching = __ballot(Q.search);
+    const float none = 1e15f;
+    const float lo = Q.search ? Q.slo : asks ? Q.tlo : none, hi = Q.search ? Q.shi : asks ? Q.thi : none;
+    const float mid = Q.search ? hi : asks ? fminf(Q.tmid, hi) : none;
+    const bool slow = !plain || __any(asks && (ov || p0 + C > Q.cap)); // (then one entry at a time, which the first copy decides)
+    const uint64_t take_first = part != 2 ? ~0ull : 0ull, take_second = part != 1 ? ~0ull : 0ull;
+    auto flush = [&](int w) {
+        const uint32_t bits = (part != 2 ? first : 0u) | (part != 1 ? second : 0u);
+        L.mask[w][lane] = bits;
+        if (!slow) p0 += __popc(part == 2 ? second & ~first : bits);
+        if (w == 0) {
+            own[0] = first;
+            own[1] = second;
+        }
+        const uint32_t f = row_or(first), g = row_or(second);
+        if ((lane & 15) == 0) {
+            L.half[0][lane >> 4][w] = f;
+            L.half[1][lane >> 4][w] = g;
+        }
+        first = second = 0;
+        if (lane < len - (w & ~1) * 32) L.list[(w & ~1) * 32 + lane] = (uint8_t)slots;
+    };
+    for (int h = 0; h < RGX_CCAP; h += 64) {
+        const int cl = h + lane;
+        bool rel = false;
+        float margins = INFINITY;
+        if (cl < C) {
+            const float dmin = L.tab[cl * RGX_TAB + RGX_TAB_DMIN], dmax = L.tab[cl * RGX_TAB + RGX_TAB_DMAX];
+            rel = dmax >= t0 && dmin <= t1;
+            margins = slow ? INFINITY : filter_margin(L.tab[cl * RGX_TAB + RGX_TAB_C]);
+        }
+        uint64_t m = __ballot(rel);
+        if (lane == 0) cn.cands += (unsigned)__popcll(m);
+        while (m) {
+            int at[COPIES], c = 0;
+            float margin = 0.f;
+            int there = 0; // copies with an entry (the others go through the first one's again, to no effect)
+#pragma unroll
+            for (int s = 0; s < COPIES; ++s) {
+                at[s] = s == 0 || (m && !slow) ? __builtin_ctzll(m) : at[0];
+                const bool is = s == 0 || (m && !slow);
+                const float ms = is ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(margins), at[s])) : -INFINITY;
+                if (is) {
+                    m &= m - 1;
+                    ++there;
+                }
+                c = copy == s ? at[s] : c;
+                margin = copy == s ? ms : margin;
+            }
+            const float4 *e = (const float4 *)(L.tab + (h + c) * RGX_TAB);
+            f3 U, V, W, inv;
+            table_frame(e, U, V, W, inv);
+            const float4 e4 = e[3];
+            const f3 De = apply_sinv_rt(Q.dir, U, V, W, inv);
+            const float a = fmaf(De.x, De.x, fmaf(De.y, De.y, De.z * De.z));
+            const float b = -fmaf(e4.x, De.x, fmaf(e4.y, De.y, e4.z * De.z));
+            const float tc = b * __builtin_amdgcn_rcpf(a);
+            const f3 Pc = mk3(fmaf(tc, De.x, e4.x), fmaf(tc, De.y, e4.y), fmaf(tc, De.z, e4.z));
+            const float out = fmaf(Pc.x, Pc.x, fmaf(Pc.y, Pc.y, Pc.z * Pc.z)) - 1.0f;
+            const float x1 = __builtin_amdgcn_fmed3f(tc, lo, mid) - tc, x2 = __builtin_amdgcn_fmed3f(tc, mid, hi) - tc;
+            const float u1 = fmaf(x1 * x1, a, out), u2 = fmaf(x2 * x2, a, out);
+            uint64_t f = __ballot(!(u1 > margin)), g = __ballot(!(u2 > margin));
+            const uint64_t sure = __ballot(fminf(fabsf(u1), fabsf(u2)) > margin);
+            const uint64_t valid = there * RAYS < 64 ? (1ull << (there * RAYS)) - 1ull : ~0ull;
+            f &= valid;
+            g &= valid;
+            if ((f | g) == 0) continue;
+            if (__builtin_expect(((~sure & valid) | ((f | g) & searching)) != 0, 0)) {
+                float r1, r2;
+                const bool ok = lane_roots<false, false>(e, Q.dir, r1, r2) && copy < there;
+                const float ts = fmaxf(Q.slo, r1);
+                const bool sfound = Q.search && ok && ts <= fminf(Q.shi, r2);
+                found = sfound ? (found < 0.0f ? ts : fminf(found, ts)) : found;
+                bool seg = asks && !ov && ok && fmaxf(Q.tlo, r1) <= fminf(Q.thi, r2);
+                const bool to_second = r2 > Q.tmid, to_first = r1 < Q.tmid || !to_second;
+                if (slow) {
+                    const bool counts = part != 2 || !to_first, over = seg && counts && p0 >= Q.cap;
+                    seg = seg && !over;
+                    ov = ov || __builtin_amdgcn_inverse_ballot_w64(Part<RAYS>::spread(__ballot(over), 0));
+                    p0 += __builtin_amdgcn_inverse_ballot_w64(Part<RAYS>::spread(__ballot(seg && counts && (part != 1 || to_first)), 0)) ? 1 : 0;
+                }
+                f = __ballot(seg && to_first);
+                g = __ballot(seg && to_second);
+            }
+            if (((f & take_first) | (g & take_second)) == 0) continue;
+#pragma unroll
+            for (int s = 0; s < COPIES; ++s) {
+                const uint64_t fs = Part<RAYS>::spread(f, s), gs = Part<RAYS>::spread(g, s);
+                if (((fs & take_first) | (gs & take_second)) == 0) continue;
+                if (lane == 0) cn.cands_hit++;
+                const uint32_t bit = 1u << (len & 31);
+                first |= __builtin_amdgcn_inverse_ballot_w64(fs) ? bit : 0u;
+                second |= __builtin_amdgcn_inverse_ballot_w64(gs) ? bit : 0u;
+                slots = lane == (len & 63) ? h + at[s] : slots;
+                ++len;
+                if ((len & 31) == 0) flush((len >> 5) - 1);
+            }
+        }
+    }
+    if (len & 31) flush(len >> 5);
+    len_out = len;
+    if (searching) {
+        const float best = Part<RAYS>::least_of_all(found < 0.0f ? INFINITY : found);
+        found = best < INFINITY ? best : -1.0f;
+    }
+    __syncthreads();
+}
+
 // Tag telling a shading body which 16 of the slab's 32 samples its walk is for.
 template <int H>
 struct Half {
@@ -1421,18 +1664,20 @@ __device__ __forceinline__ void shade_rows(const MarchParams &P, const TileLds &
 // body gets Half<TAG>.  For the list's first 32 entries the ray goes by its own chords (own[half]: its
 // hits with samples in that half, as the filter left them), for the rest by its row's notes, which
 // also hold for rays whose own chord stays in the other half.
-template <int TAG, typename Body>
+// RAYS < 64: each copy of a ray takes every 64 / RAYS-th of the ray's hits.
+template <int TAG, int RAYS = 64, typename Body>
 __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds &L, int len, bool run, int half,
                                             const uint32_t (&own)[2], Body body)
 {
     const int lane = threadIdx.x, row = lane >> 4;
     const int nw = (len + 31) >> 5;
     int w = 0;
-    uint32_t bits = (run && nw > 0) ? (half ? own[1] : own[0]) : 0u;
+    const int copy = lane / RAYS;
+    uint32_t bits = (run && nw > 0) ? Part<RAYS>::skip(half ? own[1] : own[0], copy) : 0u;
     for (;;) {
         while (bits == 0u && run && w + 1 < nw) {
             ++w;
-            bits = L.mask[w][lane] & L.half[half][row][w];
+            bits = Part<RAYS>::skip(L.mask[w][lane] & L.half[half][row][w], copy);
         }
         const bool has = bits != 0u;
         if (!__any(has)) break;
@@ -1440,6 +1685,7 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
         if (has) {
             c = L.list[w * 32 + __builtin_ctz(bits)];
             bits &= bits - 1u;
+            for (int k = 1; k < 64 / RAYS; ++k) bits &= bits - 1u;
         }
         const float4 *tab = (const float4 *)(L.tab + c * RGX_TAB);
         const int32_t pid = __float_as_int(L.tab[c * RGX_TAB + RGX_TAB_PID]);
@@ -1987,7 +2233,7 @@ __device__ __forceinline__ void frustum_range(Frustum &F, float t0, float t1)
 // row lists in lock step (it sums over the rays of a row).  WALK_ROWS: both bodies over the row lists.
 // Returns the phase-1 participation flag of this lane.
 enum { WALK_FORWARD, WALK_BACKWARD, WALK_ROWS };
-template <int WALK, int ORDER, typename Cn, typename Rec, typename BodyA, typename Mid, typename BodyB>
+template <int WALK, int ORDER, int RAYS = 64, typename Cn, typename Rec, typename BodyA, typename Mid, typename BodyB>
 __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds &L, Frustum &F, Window &Wn, const RayState &R,
                                             bool need, float tlo, float thi, int &p0, bool &ov, float &found, float &searched_to,
                                             Cn &cn, Rec &rec, BodyA body_a, Mid mid, BodyB body_b)
@@ -2070,7 +2316,9 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 int cnt = real ? p0 : q0;
                 bool cut = real ? ov : qov;
                 float best = phase == 0 ? found : -1.0f;
-                filter_table(L, C, lo, phase == 0 && any_search ? cover : hi, Q, split ? 1 + phase : 0, plain, cnt, cut, best, len, own, cn);
+                const float to = phase == 0 && any_search ? cover : hi;
+                if constexpr (RAYS == 64) filter_table(L, C, lo, to, Q, split ? 1 + phase : 0, plain, cnt, cut, best, len, own, cn);
+                else filter_part<RAYS>(L, C, lo, to, Q, split ? 1 + phase : 0, plain, cnt, cut, best, len, own, cn);
                 if (real) {
                     p0 = cnt;
                     ov = cut;
@@ -2088,7 +2336,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
             }
             if constexpr (WALK == WALK_FORWARD) {
                 static_assert(std::is_same<BodyA, BodyB>::value, "the forward shades both halves with one body");
-                shade_lanes<0>(P, L, len, run, phase, own, body_a);
+                shade_lanes<0, RAYS>(P, L, len, run, phase, own, body_a);
             } else if constexpr (WALK == WALK_BACKWARD) {
                 if (phase == 0) {
                     shade_lanes<0>(P, L, len, run, 0, own, body_a);
@@ -2124,7 +2372,8 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 const int C = sweep_next<ORDER, ORDER == BY_PAIRS && std::is_same<Rec, NoRecorder>::value>(P, S, F, L.queue, L.leafq, L.tab, done, plain, cn);
                 const LaneQuery Q = {R.dir, ask, tlo, thi, false, 0.f, 0.f, P.m.max_prim_slice, tmid};
                 float none = -1.0f;
-                filter_table(L, C, lo, hi, Q, 2, plain, p0, ov, none, len, own, cn);
+                if constexpr (RAYS == 64) filter_table(L, C, lo, hi, Q, 2, plain, p0, ov, none, len, own, cn);
+                else filter_part<RAYS>(L, C, lo, hi, Q, 2, plain, p0, ov, none, len, own, cn);
             }
             cn.nodes = work.nodes;
             cn.cands = work.cands;
@@ -2247,9 +2496,9 @@ struct Replayer {
     const TileLds L = {s_queue, s_leafq, s_tab, s_list, s_mask, s_half}
 
 // lane -> pixel: row r = lane / 16 is the 4x4 block (r & 1, r >> 1) of the 8x8 tile
-__device__ __forceinline__ void lane_pixel(int px0, int py0, int &px, int &py)
+__device__ __forceinline__ void lane_pixel(int px0, int py0, int lane, int &px, int &py)
 {
-    const int lane = threadIdx.x, row = lane >> 4, j = lane & 15;
+    const int row = lane >> 4, j = lane & 15;
     px = px0 + (row & 1) * 4 + (j & 3);
     py = py0 + (row >> 1) * 4 + (j >> 2);
 }
@@ -2268,23 +2517,29 @@ __device__ __forceinline__ uint8_t quantize8(float x)
 // (cuda_gui/gaussians_aabb.cu): black background, uchar4 colours, and the expected depth
 // sum T (1 - w) t over the samples (its colorBlendingT_chunked, 183-205).
 // PAIRS: how the sweeps descend (sweep_next).  WHOLE: no record, and a backward that will search the tree (slab_tables).
-template <bool PAIRS, bool RECORD, bool VIEWER, bool STATS, bool HALF = false, bool WHOLE = false>
+// RAYS: of a tile that one wavefront marches; fewer than 64 for images only (launch_forward).
+template <bool PAIRS, bool RECORD, bool VIEWER, bool STATS, bool HALF = false, bool WHOLE = false, int RAYS = 64>
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchParams P)
 {
     static_assert(RECORD || !HALF, "the colour sums' format is a property of the record");
+    static_assert(RAYS == 64 || !(RECORD || WHOLE), "a record is tile by tile, and what searches the tree for a backward has 64 rays");
+    using Pt = Part<RAYS>;
     static_assert(!(RECORD || PAIRS) || !WHOLE, "a search without a record goes by nodes");
     RGX_TILE_LDS(PAIRS);
-    int px0, py0, tile, half = -1;
-    if (!tile_origin(P, blockIdx.x, px0, py0, &tile, RECORD ? nullptr : &half)) return; // whole wave
+    int px0, py0, tile, part = 0;
+    if (!tile_origin(P, blockIdx.x, px0, py0, &tile, Pt::BITS, &part)) return; // whole wave
+    const int copy = (int)threadIdx.x / RAYS;
+    px0 += Pt::WIDTH == 4 ? 4 * (part & 1) : 0;
+    py0 += Pt::HEIGHT * (Pt::WIDTH == 4 ? part >> 1 : part);
     typename std::conditional<RECORD, Recorder, typename std::conditional<WHOLE, WholeLists, NoRecorder>::type>::type rec;
     if constexpr (RECORD) rec = Recorder{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
     int px, py;
-    lane_pixel(px0, py0, px, py);
-    const bool valid = px < P.cam.width && py < P.cam.height && (RECORD || half < 0 || (int)(threadIdx.x >> 5) == half); // (lanes 0-31: the upper half)
+    lane_pixel(px0, py0, threadIdx.x % RAYS, px, py);
+    const bool valid = px < P.cam.width && py < P.cam.height;
     CountersFor<STATS> cn;
     RGX_SEC_START(cn, 0);
     Frustum F;
-    frustum_planes(P.cam, px0, half == 1 ? py0 + 4 : py0, F, half < 0 ? 8 : 4);
+    frustum_planes(P.cam, px0, py0, F, Pt::WIDTH, Pt::HEIGHT);
     RayState R;
     ray_begin(P, px, py, valid, false, R);
     {
@@ -2330,6 +2585,40 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
             };
             auto blend = [&](bool second_chunk) { // gaussians_aabb.cu:195-201
                 const float first_sample = second_chunk ? 16.5f : 0.5f; // (viewer: cuda_gui/gaussians_aabb.cu:189)
+                if constexpr (RAYS < 64) { // each copy has its run of the samples: all lanes, also of rays whose sums are zero
+                    constexpr int N = Pt::EACH;
+                    float sum[4][N];
+                    Pt::sums(sg, sum[0]);
+                    Pt::sums(cr, sum[1]);
+                    Pt::sums(cg, sum[2]);
+                    Pt::sums(cb, sum[3]);
+                    float w[N], s[N], all = 1.f;
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        const float x = sum[0][i] * dt;
+                        w[i] = __expf(-x);
+                        s[i] = dt * ((1.0f - w[i]) * __builtin_amdgcn_rcpf(fmaxf(x, 1e-6f)));
+                        all *= w[i];
+                    }
+                    float through[Pt::COPIES];
+                    Pt::of_all(all, through);
+                    float T = R.T;
+#pragma unroll
+                    for (int k = 0; k < Pt::COPIES; ++k) {
+                        T = copy == k ? R.T : T;
+                        R.T *= through[k];
+                    }
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        const float ts = T * s[i];
+                        Cr = fmaf(ts, sum[1][i], Cr);
+                        Cg = fmaf(ts, sum[2][i], Cg);
+                        Cb = fmaf(ts, sum[3][i], Cb);
+                        if constexpr (VIEWER) depth += T * (1.0f - w[i]) * fmaf(dt, first_sample + (float)(N * copy + i), R.tbuffer);
+                        T *= w[i];
+                    }
+                    return;
+                }
 #pragma unroll
                 for (int i = 0; i < RGX_CHUNK_SIZE; ++i) {
                     const float x = sg[i] * dt;
@@ -2386,7 +2675,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
             };
             auto second_half = [&](bool split) { // split: the hits of the second half are not known yet
                 const bool has = need && (p0 > 0 || split);
-                if (has) blend(false);
+                if (RAYS < 64 ? __any(has) : has) blend(false);
                 RGX_SEC(cn, RGX_SEC_BLEND);
                 keep_sums(0);
                 RGX_SEC(cn, RGX_SEC_SUMS);
@@ -2396,23 +2685,38 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                 rdt = dir * fmaf(dt, 16.5f, R.tbuffer);
                 return has && R.T > P.m.t_eps;
             };
-            const bool run2 = slab_tables<WALK_FORWARD, PAIRS>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, accumulate,
+            const bool run2 = slab_tables<WALK_FORWARD, PAIRS, RAYS>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, accumulate,
                                           second_half, accumulate);
             RGX_SEC(cn, RGX_SEC_TOP); // (what slab_tables did after its last section: nothing to speak of)
-            if (run2) blend(true);
+            if (RAYS < 64 ? __any(run2) : run2) blend(true);
             RGX_SEC(cn, RGX_SEC_BLEND);
             keep_sums(RGX_CHUNK_SIZE);
             RGX_SEC(cn, RGX_SEC_SUMS);
-            if (need && p0 > 0) {
+            if (need && p0 > 0 && copy == 0) {
                 cn.slabs++;
                 cn.hit_pairs += p0;
             }
-            if (ov) cn.overflow++;
+            if (ov && copy == 0) cn.overflow++;
         }
-        slab_end(R, need, p0, found, searched_to, cn);
+        if constexpr (STATS && RAYS < 64) {
+            Counters mine = {};
+            slab_end(R, need, p0, found, searched_to, mine);
+            if (copy == 0) {
+                cn.rays_hit += mine.rays_hit;
+                cn.empty += mine.empty;
+            }
+        } else {
+            slab_end(R, need, p0, found, searched_to, cn);
+        }
         RGX_SEC(cn, RGX_SEC_END);
     }
-    if (valid) {
+    if constexpr (RAYS < 64) {
+        Cr = Pt::sum_of_all(Cr);
+        Cg = Pt::sum_of_all(Cg);
+        Cb = Pt::sum_of_all(Cb);
+        if constexpr (VIEWER) depth = Pt::sum_of_all(depth);
+    }
+    if (valid && copy == 0) {
         const int64_t ray = (int64_t)py * P.cam.width + px;
         if constexpr (VIEWER) {
             *(uchar4 *)(P.frame + 4 * ray) = make_uchar4(quantize8(Cr), quantize8(Cg), quantize8(Cb), 255);
@@ -2425,7 +2729,7 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
         }
     }
     if constexpr (STATS) {
-        if (valid && P.ray_counts) {
+        if (valid && copy == 0 && P.ray_counts) {
             const int64_t ray = (int64_t)py * P.cam.width + px;
             P.ray_counts[2 * ray] = cn.slabs;
             P.ray_counts[2 * ray + 1] = cn.hit_pairs;
@@ -2493,44 +2797,6 @@ __device__ __forceinline__ float row_min_all(float v)
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 __device__ __forceinline__ float row_max_all(float v) { return -row_min_all(-v); }
-
-// a's upper 32 lanes and b's lower 32 lanes change places; the same with the rows of 16 of each half
-__device__ __forceinline__ void swap32(float &a, float &b)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]);
-    b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void swap16(float &a, float &b)
-{
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]);
-    b = __uint_as_float(r[1]);
-}
-// the value of each of the four copies of a ray, in every copy
-__device__ __forceinline__ void copies(float v, float (&out)[4])
-{
-    float a = v, b = v; // -> a: copies 0 and 1 (in the lower and upper rows of both halves), b: copies 2 and 3
-    swap32(a, b);
-    float a1 = a, b1 = b;
-    swap16(a, a1);
-    swap16(b, b1);
-    out[0] = a; out[1] = a1; out[2] = b; out[3] = b1;
-}
-// 16 values per lane -> four: copy `sub` gets the sums over the copies of v[4 sub .. 4 sub + 3]
-__device__ __forceinline__ void sum_copies(float (&v)[RGX_CHUNK_SIZE], float (&out)[4])
-{
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        swap32(v[i], v[i + 8]);
-        v[i] += v[i + 8];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        swap16(v[i], v[i + 4]);
-        out[i] = v[i] + v[i + 4];
-    }
-}
 
 template <int CAP>
 __device__ __forceinline__ void team_sweep_begin(const MarchParams &P, Sweep &S, const Frustum &F, TeamShared<CAP> &T)
@@ -3448,7 +3714,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
         __syncthreads();
     }
     int px, py;
-    lane_pixel(px0, py0, px, py);
+    lane_pixel(px0, py0, threadIdx.x, px, py);
     const bool valid = px < P.cam.width && py < P.cam.height;
     CountersFor<STATS> cn;
     RGX_SEC_START(cn, 1);
@@ -3938,7 +4204,7 @@ __global__ __launch_bounds__(64) void k_collect_tiles(const MarchParams P, const
     if (!tile_origin(P, blockIdx.x, px0, py0)) return;
     const int lane = threadIdx.x;
     int px, py;
-    lane_pixel(px0, py0, px, py);
+    lane_pixel(px0, py0, threadIdx.x, px, py);
     const bool valid = px < P.cam.width && py < P.cam.height;
     const int64_t ray = (int64_t)py * P.cam.width + px;
     CountersFor<STATS> cn; // with counters or without, as the march kernels
@@ -4110,7 +4376,7 @@ static int fill_params(MarchParams &P, const void *ws, const RgxCamera *cam, con
     const size_t order_words = (size_t)8 * g.per_xcd * g.bw * g.bh;
     P.tile_order = M.order + order_words * sizeof(uint32_t) <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.order) : nullptr;
     P.use_tile_order = 0;
-    P.by_halves = 0;
+    P.part_bits = 0;
     P.faults = M.order <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.faults) : nullptr;
     P.ray_counts = nullptr;
     P.sum_pool = nullptr;
@@ -4152,21 +4418,35 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
     return RGX_OK;
 }
 
-// Up to this many tiles four wavefronts march a tile (k_march_team), beyond it one.  The team's wavefronts repeat the
-// per-iteration work that one wavefront does once for 64 rays, so it loses where the chip is full anyway; with few tiles
-// the launch is one tile's latency.  Measured, ms of a frame with one wavefront / with four:
-//     tiles                                      256          625          784         1 024        1 600        2 500
-//     fixed step, 4 k Gaussians in a cube    1.04 / 0.55  0.83 / 0.47  0.76 / 0.44  0.71 / 0.43  0.68 / 0.55  0.61 / 0.76
-//     fixed step, 100 k in a ball            4.32 / 2.38  2.54 / 1.58  2.51 / 1.54  2.24 / 1.36  1.68 / 1.20  1.35 / 1.03
-//     adaptive step, 60 k heavy-tailed       1.85 / 1.21  1.14 / 1.02  1.14 / 1.01  1.04 / 1.07  0.97 / 1.58  0.89 / 2.19
-//     adaptive step, 3 M heavy-tailed        9.77 / 4.00  6.73 / 4.53  5.84 / 4.16  5.83 / 4.07  4.57 / 5.59  4.44 / 7.03
-// Images stop at 768 tiles, below the first loss of any of them (the adaptive frames at 1 024): from there half tiles take over (RGX_HALF_TILES).
-// Records of the fixed step have no such losses up to 1 024 tiles (forward at 1 024, one / four: 4 k in a cube 0.76 / 0.50, 100 k in a ball
-// 1.97 / 1.28, 1 M in a ball of radius 2 5.64 / 5.15).
-//
-// Which launches: those whose image is the end of it (rgx_march_test, the viewer), and those that leave a record
-// with the fixed step.  The team adds up a sample's hits in another order, and where max_prim_slice cuts a ray's list it
-// keeps other hits, equally exact both.
+// A launch in which every wavefront starts at once lasts as long as its longest, and one with few tiles leaves most of the chip idle.  So an image of few
+// tiles is marched by parts of tiles: halves (8x4 pixels), 4x4 blocks or 4x2 pixels, a wavefront for each, whose lanes hold each ray twice, four
+// or eight times over (Part).  A part has a narrower frustum, whose tables hold fewer Gaussians, as many entries tested at a time as its rays have
+// copies, and walks that are shorter by as much; what is done more often is the sweep.  Measured, ms of a frame by whole tiles / halves / 4x4 / 4x2,
+// where not taken before by four wavefronts a tile that swept together, met at barriers and had the tile's 64 rays four times over (up to 768 tiles: in brackets) or
+// by halves whose idle lanes did nothing (769 to 1 296: likewise):
+//     tiles                                     64                  256                 625                 900
+//     fixed step, 4 k Gaussians in a cube   [1.32] 0.58 0.45    [0.56] 0.49 0.41    [0.49] 0.42 0.41    [0.61] 0.41 0.44
+//     fixed step, 30 k in a ball            [2.65] 1.19 0.57    [1.43] 0.60 0.41    [0.94] 0.47 0.41    [1.18] 0.46 0.40
+//     fixed step, 100 k in a ball           [5.36] 2.23 1.22    [2.30] 1.11 0.54    [1.59] 0.88 0.55    [1.75] 0.76 0.49
+//     fixed step, 1 M in a ball of radius 2 [13.3] 5.35 3.41    [5.47] 2.94 1.65    [4.77] 1.92 1.86    [3.38] 2.00 2.30
+//     adaptive step, 60 k heavy-tailed      [2.28] 0.95 0.64    [1.18] 0.65 0.56    [0.97] 0.66 0.94    [0.80] 0.80 1.17
+//     adaptive step, 3 M heavy-tailed       [8.46] 5.29 3.26    [3.68] 3.01 2.12    [4.07] 2.31 3.01    [3.67] 2.90 3.61
+//     tiles                                    1 225                 1 600               2 025               3 025               4 056
+//     fixed step, 4 k in a cube          [0.55] 0.47 0.40 0.53   0.67 0.49 0.42      0.67 0.46 0.44      0.62 0.48 0.61      0.55 0.61 0.93
+//     fixed step, 100 k in a ball        [1.45] 1.24 0.63 0.62   2.17 1.04 0.60      1.88 0.89 0.62      1.24 0.71 0.70      1.06 0.83 1.01
+//     fixed step, 1 M, radius 2          [3.03] 2.68 2.18 2.68   4.34 2.32 2.36      3.99 2.59 2.61      2.99 2.82 3.41      2.92 2.99 4.15
+//     adaptive step, 60 k heavy-tailed   [0.81] 0.74 0.94 1.52   0.88 0.85 1.09      0.83 1.01 1.28      0.87 1.14 1.69      1.07 1.39 2.11
+//     adaptive step, 3 M heavy-tailed    [3.59] 3.00 3.19 4.30   4.00 3.68 3.86      3.85 3.86 4.20      4.61 4.70 5.42      4.56 4.92 6.25
+// The lines lie where a finer part stops gaining over the scenes of each step; the step stands for what else those scenes differ in: around an object half the tiles are
+// empty, from within a scene all are heavy.  (Halves for the heaviest blocks only of an image with more tiles: 300 k 800x800 2.25 -> 2.73 ms
+// for 512 tiles of 10 000.)  The sums of a ray's hits are added up in another order, and where max_prim_slice cuts a ray's list other hits are kept, equally exact both.
+struct PartLines {
+    int eighths, quarters, halves; // up to so many tiles
+};
+static inline PartLines image_part_lines(bool adaptive) { return adaptive ? PartLines{256, 800, 1600} : PartLines{768, 2048, 3200}; }
+
+// Records of the fixed step, up to this many tiles: four wavefronts march a tile (k_march_team), beyond it one (forward at 1 024, one / four: 4 k in a cube 0.76 / 0.50, 100 k in a ball
+// 1.97 / 1.28, 1 M in a ball of radius 2 5.64 / 5.15).  The team, too, adds up a sample's hits in another order, and keeps other hits of a list that is cut.
 //   No record: the backward searches the tree again, one wavefront per tile, and has to meet the hits and the
 //     transmittance of the forward: that is k_march_fwd then, whatever the step, and every slab's list in one (slab_tables).
 //   A record and the adaptive step: the next step's length depends on the last bit of the transmittance, and a sample that
@@ -4174,29 +4454,20 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
 //     no longer the gradients that larger images give.  k_march_fwd.
 //   A record and the fixed step: what the backward replays is what the team recorded.  (A tile whose region overflowed is
 //     searched again, in the team's order: lists that max_prim_slice cut are cut to the same hits there.)
-#ifndef RGX_TEAM_TILES
-#define RGX_TEAM_TILES 768
-#endif
 #define RGX_TEAM_TILES_RECORD 1024
-// Images of so few tiles beyond those are marched by halves of tiles, 8x4 pixels: a wavefront for each, half of whose lanes idle.  A launch in which
-// every wavefront starts at once lasts as long as its longest, and one with half the rays meets fewer Gaussians in a narrower
-// frustum, and walks shorter lists.  Measured, ms of a frame by whole tiles / by halves:
-//     tiles                                      961          1 024          1 296          1 521          2 500
-//     fixed step, 4 k Gaussians in a cube    0.71 / 0.55    0.68 / 0.59    0.65 / 0.53    0.68 / 0.57    0.59 / 0.53
-//     fixed step, 100 k in a ball            2.06 / 1.14    1.78 / 1.47    1.59 / 1.33    1.59 / 1.09
-//     fixed step, 1 M in a ball of radius 2  5.14 / 3.35    5.14 / 3.27    4.43 / 3.00    3.97 / 2.69    3.24 / 3.10
-//     adaptive step, 60 k heavy-tailed       0.96 / 0.76    0.98 / 0.76    0.90 / 0.80    0.86 / 0.88    0.85 / 1.13
-//     adaptive step, 3 M heavy-tailed        4.52 / 3.75    4.42 / 3.62    4.25 / 3.57    3.93 / 4.45    3.55 / 4.97
-// One line for both steps, below the adaptive step's first loss (1 521); the fixed step still gains at 2 500 and would bear a line of its own, and between 400 and 768
-// tiles, where four wavefronts per tile and halves win in turn, there is no rule but the team's line.  (Halves for the heaviest blocks only of an image
-// with more tiles: 300 k 800x800 2.25 -> 2.73 ms for 512 tiles of 10 000.)  A record is tile by tile.
-#define RGX_HALF_TILES 1296
 
 // image_only: no backward follows this launch
 static bool sums_in_any_order(const MarchParams &P, bool image_only) { return image_only || (P.records && !P.m.dynamic_sampling); }
 static bool by_team(const MarchParams &P, bool image_only)
 {
-    return P.tiles_x * P.tiles_y <= (image_only ? RGX_TEAM_TILES : RGX_TEAM_TILES_RECORD) && sums_in_any_order(P, image_only);
+    return !image_only && P.tiles_x * P.tiles_y <= RGX_TEAM_TILES_RECORD && sums_in_any_order(P, image_only);
+}
+static int part_bits(const MarchParams &P, bool image_only)
+{
+    if (!image_only) return 0;
+    const PartLines L = image_part_lines(P.m.dynamic_sampling);
+    const int tiles = P.tiles_x * P.tiles_y;
+    return tiles <= L.eighths ? 3 : tiles <= L.quarters ? 2 : tiles <= L.halves ? 1 : 0;
 }
 
 // What precedes a forward's march: counters cleared, and its launch order: blocks of tiles by their estimated weight (k_block_cost,
@@ -4207,13 +4478,14 @@ static void prepare_forward(MarchParams &P, bool image_only, hipStream_t s)
     // rounds of tiles per wave slot (3072 slots: 12 per CU) that end is a small part of the launch
     // and the pass over the primitive records takes what it brings (forward without -> with the order: 1 M Gaussians at
     // 800x800, 3.3 rounds: 5.51 -> 5.32 ms; 300 k there 2.84 -> 2.82; 3 M at 1237x822, 5.2 rounds: 9.71 -> 9.67; 3 M at
-    // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every tile has a CU of its own, and starts at once.
+    // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every wavefront starts at once.
     const int64_t tiles = (int64_t)P.tiles_x * P.tiles_y;
     const bool team = by_team(P, image_only);
-    P.by_halves = image_only && !team && tiles <= RGX_HALF_TILES;
+    P.part_bits = part_bits(P, image_only);
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);
-    const bool ordered = P.tile_order && P.n > 0 && tiles <= 6 * 3072 && !(team && tiles <= 256) && nb <= RGX_COST_BINS; // (more blocks: a very long, thin image)
+    const bool at_once = team ? tiles <= 256 : P.part_bits > 0 && tiles << P.part_bits <= 3072;
+    const bool ordered = P.tile_order && P.n > 0 && tiles <= 6 * 3072 && !at_once && nb <= RGX_COST_BINS; // (more blocks: a very long, thin image)
     uint32_t *order = P.tile_order, *cost = ordered ? P.tile_order + 8 * g.per_xcd : nullptr;
     if (P.sum_next || P.faults || ordered)
         hipLaunchKernelGGL(k_clear_forward, dim3(ordered ? (unsigned)((nb + 255) / 256) : 1u), dim3(256), 0, s, (float4 *)P.sum_next, (float4 *)P.faults, cost, ordered ? nb : 0);
@@ -4227,7 +4499,7 @@ static void prepare_forward(MarchParams &P, bool image_only, hipStream_t s)
 static inline dim3 march_grid(const MarchParams &P)
 {
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
-    return dim3((unsigned)(8 * g.per_xcd * g.bw * g.bh) << P.by_halves);
+    return dim3((unsigned)(8 * g.per_xcd * g.bw * g.bh) << P.part_bits);
 }
 
 // Sweeps by pairs of nodes: the same launches, up to six rounds of tiles, over trees that have them.  A tile's own time gets shorter, which is what a launch with
@@ -4252,9 +4524,21 @@ static void launch_forward(const MarchParams &P, bool viewer, bool counting, boo
         else if (pairs) hipLaunchKernelGGL((k_march_fwd<true, __VA_ARGS__>), grid, block, 0, s, P); \
         else hipLaunchKernelGGL((k_march_fwd<false, __VA_ARGS__>), grid, block, 0, s, P);       \
     } while (0)
+#define RGX_FWD_PART(RAYS, ...)                                                                 \
+    do {                                                                                        \
+        if (pairs) hipLaunchKernelGGL((k_march_fwd<true, false, __VA_ARGS__, false, false, RAYS>), grid, block, 0, s, P); \
+        else hipLaunchKernelGGL((k_march_fwd<false, false, __VA_ARGS__, false, false, RAYS>), grid, block, 0, s, P); \
+    } while (0)
+#define RGX_FWD_IMAGE(...)                                                                      \
+    do {                                                                                        \
+        if (P.part_bits == 0) RGX_FWD_PART(64, __VA_ARGS__);                                    \
+        else if (P.part_bits == 1) RGX_FWD_PART(32, __VA_ARGS__);                               \
+        else if (P.part_bits == 2) RGX_FWD_PART(16, __VA_ARGS__);                               \
+        else RGX_FWD_PART(8, __VA_ARGS__);                                                      \
+    } while (0)
     if (viewer) {
-        if (counting) RGX_FWD(false, true, true);
-        else RGX_FWD(false, true, false);
+        if (counting) RGX_FWD_IMAGE(true, true);
+        else RGX_FWD_IMAGE(true, false);
     } else if (P.records && half) {
         if (counting) RGX_FWD(true, false, true, true);
         else RGX_FWD(true, false, false, true);
@@ -4265,9 +4549,11 @@ static void launch_forward(const MarchParams &P, bool viewer, bool counting, boo
         if (counting) hipLaunchKernelGGL((k_march_fwd<false, false, false, true, false, true>), grid, block, 0, s, P);
         else hipLaunchKernelGGL((k_march_fwd<false, false, false, false, false, true>), grid, block, 0, s, P);
     } else {
-        if (counting) RGX_FWD(false, false, true);
-        else RGX_FWD(false, false, false);
+        if (counting) RGX_FWD_IMAGE(false, true);
+        else RGX_FWD_IMAGE(false, false);
     }
+#undef RGX_FWD_IMAGE
+#undef RGX_FWD_PART
 #undef RGX_FWD
 }
 

@@ -628,6 +628,46 @@ def test_sweeps_by_pairs_of_nodes_and_by_nodes_find_the_same(gx, n, w, h, dyn):
         assert abs(sb["hit_pairs"] - sa["hit_pairs"]) <= (0 if n < 6000 else 100)
 
 
+# fixed step: 768 and 784 tiles, 2 048 and 2 064, 3 200 and 3 240; adaptive: 256 and 272, 800 and 825, 1 600 and 1 640.  Odd sizes: parts without a ray
+@pytest.mark.parametrize("dyn,w,h", [(False, 5, 3), (False, 256, 190), (False, 219, 219), (False, 507, 256), (False, 509, 257), (False, 512, 395),
+                                     (False, 479, 427), (True, 5, 3), (True, 125, 126), (True, 131, 126), (True, 200, 251), (True, 195, 259),
+                                     (True, 313, 318), (True, 328, 313)])
+@pytest.mark.parametrize("scale,n", [(1.0, 6000), (5.0, 6000), (1.0, 3)])
+def test_images_by_parts_of_tiles(gx, dyn, w, h, scale, n):
+    """Either side of the numbers of tiles at which an image goes over from 4x2 pixels a wavefront to 4x4, to half a tile and to a tile: the image and
+    the counters of the forward that leaves a record.  Sparse slabs, and slabs whose candidates fill several tables; with lists that
+    max_prim_slice could cut but does not (the filter then goes entry by entry).  (Sums in another order: 1e-5; adaptive: a ray may be re-phased.)"""
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.render_optix import compute_rgb
+    sc = gx.to_dev(scenes.scene_to_numpy(scenes.make_scene(2 if dyn else 0, n=n, sh_degree=0, seed=33)))
+    cam = scenes.make_camera(2 if dyn else 0, 1, width=w, height=h)
+    params = sc["positions"], sc["scales"] * scale, sc["quaternions"], sc["densities"]
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+    cs = u_ox.camera_struct(cam)
+    rgb = compute_rgb(cam.camera_center, sc["positions"], sc["color_features"], None, None, None, 0, 0)
+    prims = u_ox.pack_prims(gas, cs, *params, rgb)
+    tol = 5e-3 if dyn else 1e-5
+    _step(f"parts {w}x{h} n={n} scale {scale} adaptive {dyn}")
+    st = [u_ox.new_stats(gx.DEV) for _ in range(3)]
+    rec = torch.empty(u_ox.records_bytes(cs, 16384 * 4), dtype=torch.uint8, device=gx.DEV)
+    whole = u_ox.march_forward(gas, cs, prims, 0.01, dyn, 4096, True, records=rec, stats=st[0])
+    test = lambda cap, **kw: u_ox.launch_pipeline_test(None, None, gas, None, None, 0.01, dyn, cam, params[3], rgb, *params[:3], cap, **kw)
+    image = test(4096, stats=st[1])
+    assert torch.equal(image, test(4096)) and (image - whole).abs().max() <= tol
+    a, b = u_ox.read_stats(st[0]), u_ox.read_stats(st[1])
+    assert a["rays_hit"] == b["rays_hit"] and a["overflow_rays"] == b["overflow_rays"] == 0
+    if not dyn:
+        assert abs(a["slabs"] - b["slabs"]) <= 1 and abs(a["hit_pairs"] - b["hit_pairs"]) <= 100 * abs(a["slabs"] - b["slabs"]), (a, b)
+    cut = test(60, stats=st[2])
+    if u_ox.read_stats(st[2])["overflow_rays"] == 0:
+        assert (cut - whole).abs().max() <= tol
+    frame, depth = u_ox.march_viewer(gas, cs, prims, 0.01, dyn, 4096)
+    black = u_ox.march_forward(gas, cs, prims, 0.01, dyn, 4096, False, records=rec)
+    assert (frame.reshape(-1, 4)[:, :3].float() - (black.clamp(0, 1) * 256).floor().clamp(max=255)).abs().max() <= (1 if not dyn else 2)
+    hit = (whole - black).amax(1) < 1 - 1e-6                                   # (some of the background is gone: something was met)
+    assert torch.equal(depth.reshape(-1)[hit] > 0, torch.ones_like(hit[hit]))
+
+
 @pytest.mark.parametrize("w,h", [(52, 44), (216, 224), (253, 256)])              # 1 024 tiles: the most that four wavefronts march
 def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     """What the four wavefronts of a tile leave for the backward, in each form: sample sums in floats and in half
