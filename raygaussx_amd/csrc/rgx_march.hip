@@ -18,7 +18,7 @@
 //      walk the entries that one of their rays hits, in lock step, and sum each entry's 13 whitened-frame
 //      sums over their rays with DPP adds (the backward's gradient pass: half rows of 8 lanes in a replay, rows
 //      of 16 in the backward that searches the tree).
-// An image of few tiles is marched by four wavefronts per tile (k_march_team, launch_forward).
+// An image of few tiles is marched by parts of tiles (Part, launch_forward).
 // The forward can record what 1 and 2 produced, and the per-sample density and colour sums of 3;
 // the replaying backward then needs no tree, no table, no predicate and no density pass, sums a window's
 // gradients in LDS before adding them to memory, and replays a tile in several pieces side by side.
@@ -49,14 +49,14 @@
 // keys with ties broken by a 30-bit index is at most 63 + 30 = 93 deep: with a margin of 160 the
 // stack never holds more than QCAP - 96 + 93 < QCAP entries, whatever the scene.
 #define RGX_DFS_MARGIN 160
-// The same for a sweep of 256 nodes a step, by four wavefronts (k_march_team): a step pops at most as many nodes as leave this margin free.
-#define RGX_TEAM_QCAP 1024
-#define RGX_TEAM_DFS_MARGIN 96
 #define RGX_LDS_HITS 32    // per-lane list of the stand-alone collect hook
 // The march kernels are sized (registers and LDS) for three wavefronts per SIMD.
 #ifndef RGX_WAVES_ATTR
 #define RGX_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(3, 3)))
 #endif
+// The forward that leaves a record by parts of tiles, for two: what it keeps of a part's record does not fit 168 registers beside the rest (112 bytes of
+// spills a lane), and a launch by parts seldom fills more (4 k Gaussians 128x128 0.82 -> 0.74 ms a step, 100 k in a ball 256x240 1.22 -> 1.16).
+#define RGX_WAVES_ATTR_FWD(two) __attribute__((amdgpu_waves_per_eu((two) ? 2 : 3, (two) ? 2 : 3)))
 
 struct MarchParams {
     RgxCamera cam;
@@ -77,20 +77,23 @@ struct MarchParams {
     float *gbuf;             // bwd: (n,16) gradient block in Morton order
     RgxStats *stats;
     int32_t tiles_x, tiles_y;
-    uint32_t *records;      // hit-list record stream, rec_tile_words per tile, or null
+    uint32_t *records;      // hit-list record stream, rec_tile_words per tile or part of one, or null
     int32_t rec_tile_words;
-    int32_t only_overflow;  // backward: handle only the tiles whose record overflowed
+    int32_t only_overflow;  // backward: handle only the tiles (parts) whose record overflowed
     int32_t rec_pieces, rec_first, rec_equal, rec_turn; // the pieces of a tile's record (record_pieces)
     uint32_t *tile_order;   // launch order lists (or null: as launched)
     int32_t use_tile_order; // 0: as launched; 1: per XCD, its tiles' list positions from the heaviest to the lightest (k_tile_order);
                             // 2: per XCD, the blocks of tiles it renders, heaviest first (k_block_order)
-    int32_t part_bits;      // forward of an image: each tile by 2^part_bits workgroups (launch_forward)
+    int32_t part_bits;      // each tile by 2^part_bits workgroups (launch_forward)
     float4 *sum_pool;       // sample-sum slots of the record (RGX_SUM_SLOT_WORDS each), or null
     uint32_t *sum_next;     // next free slot (bump counter in the record's pool header)
-    int32_t sum_slots;      // slots in the pool
-    int32_t sum_slot_words; // words per slot: RGX_SUM_SLOT_WORDS, or RGX_SUM_SLOT_WORDS_HALF with half-precision colour sums
+    int32_t sum_slots;      // slots in the pool (a part's: 2^part_bits to one of the bump counter's)
+    int32_t sum_slot_words; // words per slot: RGX_SUM_SLOT_WORDS, or RGX_SUM_SLOT_WORDS_HALF with half-precision colour sums, >> part_bits
     uint32_t *faults;       // march workspace: [0] replays that lost their record, [1] sweeps that dropped nodes; or null
     uint32_t *ray_counts;   // counting forward only: per ray, slabs blended and the sum of their hit-list lengths; or null
+    // (at the end: where the others lie decides which of them one load fetches)
+    int32_t rec_bits;       // each tile has 2^rec_bits regions of the record
+    uint32_t sum_first;     // the first slot of the pool that is not kept for a part's lists
 };
 
 // The kernel's arguments once more, from the kernel's argument segment: what is read through this is loaded where it is used.
@@ -458,17 +461,13 @@ struct Sweep {
 // kept, so a backward that has to search the tree for a tile takes the order of the forward that wrote the tile's record.
 //   BY_NODES  up to 64 nodes a step; where nothing speaks for another
 //   BY_PAIRS  the children of up to 64 nodes a step
-//   BY_TEAM   up to 256 nodes a step: what k_march_team does with four wavefronts, by one
-enum { BY_NODES, BY_PAIRS, BY_TEAM };
+enum { BY_NODES, BY_PAIRS };
 
 template <int ORDER>
 __device__ __forceinline__ void sweep_begin(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq)
 {
     S.lqn = 0;
-    if constexpr (ORDER == BY_TEAM) {
-        S.qn = F.cut_n;
-        for (int i = threadIdx.x; i < F.cut_n; i += 64) s_queue[i] = s_queue[RGX_TEAM_QCAP + i];
-    } else if constexpr (ORDER == BY_PAIRS) {
+    if constexpr (ORDER == BY_PAIRS) {
         S.qn = F.cut_inner;
         S.lqn = F.cut_n - F.cut_inner;
         const int lane = threadIdx.x;
@@ -599,170 +598,10 @@ __device__ __forceinline__ void frustum_cut_pairs(const MarchParams &P, Frustum 
     F.cut_node = node;
 }
 
-// What a leaf whose box passed turns into: its ellipsoid against the frustum, and its table entry (as in sweep_next,
-// whose kernels have no register for a function that returns one).
-struct LeafEntry {
-    f3 U, V, W, inv, Oe;
-    float dmin, dmax, k, c;
-    bool plain; // passed plain_roots()
-    __device__ __forceinline__ void store(float4 *dst, int32_t left) const
-    {
-        table_store(dst, U, V, W, inv, Oe, ~left, dmin, dmax, k, c);
-    }
-};
-__device__ __forceinline__ bool leaf_entry(const MarchParams &P, const Frustum &F, int32_t left, LeafEntry &e)
-{
-    const Prim p = P.prims[~left];
-    quat_to_cols(p.quat4, e.U, e.V, e.W);
-    const f3 O = mk3(p.pos4.x, p.pos4.y, p.pos4.z);
-    const bool ok = leaf_meets(F, p, e.U, e.V, e.W, e.dmin, e.dmax);
-    if (ok) {
-        e.k = p.inv_inter4.w;
-        e.inv = mk3(p.inv_inter4.x, p.inv_inter4.y, p.inv_inter4.z);
-        e.Oe = apply_sinv_rt(O, e.U, e.V, e.W, e.inv);
-        e.c = fmaf(e.Oe.x, e.Oe.x, fmaf(e.Oe.y, e.Oe.y, fmaf(e.Oe.z, e.Oe.z, -1.0f)));
-        e.plain = plain_roots(e.inv, e.c);
-    }
-    return ok;
-}
-
-// What the team's lanes do in one step, a wavefront after the other: each(j, on, value) for the four groups of 64 of the m words at `from`, all of which
-// are read before the first is looked at.
-template <typename Each>
-__device__ __forceinline__ void team_groups(const int32_t *from, int m, Each each)
-{
-    const int lane = threadIdx.x;
-    int32_t v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = 64 * j + lane < m ? from[64 * j + lane] : -1;
-    __syncthreads();
-    for (int j = 0; j < 4 && 64 * j < m; ++j) each(64 * j + lane < m, j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3]);
-    __syncthreads();
-}
-
-// The node's box against the frustum (a lane without a node: nothing met).
-__device__ __forceinline__ void node_meets(const MarchParams &P, const Frustum &F, bool on, int32_t node, bool &leaf, bool &inner, int32_t &left, int32_t &right)
-{
-    leaf = inner = false;
-    left = right = 0;
-    if (on && (uint32_t)node < (uint32_t)(2 * P.n - 1)) {
-        const float4 a = ((const float4 *)P.nodes)[2 * node], b = ((const float4 *)P.nodes)[2 * node + 1];
-        right = P.right[max(0, min(node, (int32_t)P.n - 2))];
-        left = __float_as_int(a.w);
-        const bool meets = !frustum_misses(F, a, b);
-        leaf = meets && left < 0;
-        inner = meets && left >= 0;
-    }
-}
-
-// team_frustum_cut by one wavefront, into the 256 words behind the stack
-__device__ __forceinline__ void frustum_cut_team(const MarchParams &P, Frustum &F, float t_far, int32_t *s_queue)
-{
-    F.range(0.f, INFINITY, 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f)); // no distance shell
-    int32_t *cut = s_queue + RGX_TEAM_QCAP;
-    int count = P.n > 0 ? 1 : 0;
-    if (threadIdx.x == 0) cut[0] = 0;
-    __syncthreads();
-    for (int level = 0; level < 64 && count > 0; ++level) {
-        int kept = 0, opened = 0;
-        team_groups(cut, count, [&](bool on, int32_t node) {
-            bool leaf, inner;
-            int32_t left, right;
-            node_meets(P, F, on, node, leaf, inner, left, right);
-            kept += __popcll(__ballot(leaf));
-            opened += __popcll(__ballot(inner));
-        });
-        const int next = kept + 2 * opened;
-        if (opened == 0 || next > 256) break;
-        int leaves = 0, at = kept;
-        team_groups(cut, count, [&](bool on, int32_t node) {
-            bool leaf, inner;
-            int32_t left, right;
-            node_meets(P, F, on, node, leaf, inner, left, right);
-            const uint64_t bl = __ballot(leaf), bi = __ballot(inner);
-            if (leaf) cut[leaves + rank_in(bl)] = node;
-            if (inner) {
-                cut[at + 2 * rank_in(bi)] = left;
-                cut[at + 2 * rank_in(bi) + 1] = right;
-            }
-            leaves += __popcll(bl);
-            at += 2 * __popcll(bi);
-        });
-        count = next;
-    }
-    F.cut_n = count;
-}
-
-// team_sweep_next by one wavefront
-template <typename Cn>
-__device__ __forceinline__ int sweep_next_team(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab, bool &done,
-                                               bool &plain, Cn &cn)
-{
-    plain = true;
-    int C = 0;
-    while ((S.qn > 0 || S.lqn > 0) && C < RGX_CCAP) {
-        if (S.lqn >= 256 || S.qn == 0) {
-            const int m = S.lqn < 256 ? S.lqn : 256, room = RGX_CCAP - C;
-            int hits = 0;
-            S.lqn -= m;
-            team_groups(s_leafq + S.lqn, m, [&](bool on, int32_t left) {
-                LeafEntry e;
-                const bool hit = on && leaf_entry(P, F, left, e);
-                const uint64_t bl = __ballot(hit);
-                plain = plain && __ballot(hit && !e.plain) == 0;
-                const int rank = hits + rank_in(bl);
-                if (hit) {
-                    if (rank < room) e.store((float4 *)(s_tab + (C + rank) * RGX_TAB), left);
-                    else s_leafq[S.lqn + rank - room] = left; // no room: back to the queue, for the next table
-                }
-                hits += __popcll(bl);
-            });
-            C += hits < room ? hits : room;
-            S.lqn += hits < room ? 0 : hits - room;
-            continue;
-        }
-        const int spare = RGX_TEAM_QCAP - RGX_TEAM_DFS_MARGIN - S.qn;
-        const int m = min(min(S.qn, 256), max(spare, 1));
-        const int base = S.qn - m;
-        int pos = base;
-        if (threadIdx.x == 0) cn.nodes += (unsigned)m;
-        team_groups(s_queue + base, m, [&](bool on, int32_t node) {
-            bool leaf, inner;
-            int32_t left, right;
-            node_meets(P, F, on, node, leaf, inner, left, right);
-            const uint64_t bl = __ballot(leaf), bi = __ballot(inner);
-            if (leaf) s_leafq[S.lqn + rank_in(bl)] = left; // fewer than 256 waiting + at most 256 new
-            S.lqn += __popcll(bl);
-            if (inner) {
-                const int at = pos + 2 * rank_in(bi);
-                if (at + 1 < RGX_TEAM_QCAP) {
-                    s_queue[at] = right;
-                    s_queue[at + 1] = left;
-                } else if (P.faults) { // cannot happen (see RGX_DFS_MARGIN)
-                    atomicAdd(&P.faults[1], 1u);
-                }
-            }
-            pos += 2 * __popcll(bi);
-        });
-        S.qn = min(pos, RGX_TEAM_QCAP);
-    }
-    done = S.qn == 0 && S.lqn == 0;
-    return C;
-}
-
-// Fills the table from the sweep; returns the number of entries.  done: the sweep is finished;
-// plain: every entry passed plain_roots().
-// AGAIN: the descent reads its arguments once more for every table (args_again) and does not hold them, or spill them, across the marches
-// between: marches by pairs that record nothing.  Measured for images (300 k Gaussians 800x800 with lobes 2.284 -> 2.245 ms, viewer 1 M 1280x720 6.06 -> 6.00).  Not where it loses: the
-// recording forward (300 k 800x800 2.67 -> 2.71) and images by nodes (3 M 1920x1080 16.2 -> 16.4).
-// PAIRS: the descent opens 64 internal nodes a step and tests both children of each, so it takes half as many steps, each one
-// trip to memory; leaves never enter the stack.  It finds the Gaussians in another order, so only marches whose sums may be taken
-// in any order go this way (launch_forward).
 template <int ORDER, bool AGAIN, typename Cn>
 __device__ __forceinline__ int sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, int32_t *s_queue, int32_t *s_leafq, float *s_tab,
                           bool &done, bool &plain, Cn &cn)
 {
-    if constexpr (ORDER == BY_TEAM) return sweep_next_team(P, S, F, s_queue, s_leafq, s_tab, done, plain, cn);
     constexpr bool PAIRS = ORDER == BY_PAIRS;
     plain = true;
     const int lane = threadIdx.x;
@@ -1280,6 +1119,11 @@ struct Part {
     static constexpr int COPIES = 64 / RAYS, BITS = RAYS == 64 ? 0 : RAYS == 32 ? 1 : RAYS == 16 ? 2 : 3;
     static constexpr int WIDTH = RAYS < 32 ? 4 : 8, HEIGHT = RAYS / WIDTH; // in pixels
     static constexpr int EACH = RGX_CHUNK_SIZE / COPIES;                   // samples of a chunk that a copy blends
+    static constexpr int LISTS_HEAD = RAYS == 64 ? 8 : 2;                  // words of a LISTS item before its slots
+    static constexpr int ROWS = RAYS > 16 ? RAYS / 16 : 1;                 // rows of lanes that hold all rays
+    // a lane's ray and copy (with one copy: what the compiler need not find out)
+    static __device__ __forceinline__ int ray(int lane) { return RAYS == 64 ? lane : lane % RAYS; }
+    static __device__ __forceinline__ int copy(int lane) { return RAYS == 64 ? 0 : lane / RAYS; }
     // what the lanes of copy s say, said by all copies
     static __device__ __forceinline__ uint64_t spread(uint64_t lanes, int s)
     {
@@ -1495,7 +1339,7 @@ __device__ __forceinline__ void filter_part(const TileLds &L, int C, float t0, f
                                             int &p0, bool &ov, float &found, int &len_out, uint32_t (&own)[2], Cn &cn)
 {
     constexpr int COPIES = 64 / RAYS;
-    const int lane = threadIdx.x, copy = lane / RAYS;
+    const int lane = threadIdx.x, copy = Part<RAYS>::copy(lane);
     int len = 0;
     uint32_t first = 0, second = 0; // the ray's hits with samples in the first / second half (the same in all copies)
     int slots = 0;                  // lane i: slot of entry i of the list's current 64
@@ -1672,7 +1516,7 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
     const int lane = threadIdx.x, row = lane >> 4;
     const int nw = (len + 31) >> 5;
     int w = 0;
-    const int copy = lane / RAYS;
+    const int copy = Part<RAYS>::copy(lane);
     uint32_t bits = (run && nw > 0) ? Part<RAYS>::skip(half ? own[1] : own[0], copy) : 0u;
     for (;;) {
         while (bits == 0u && run && w + 1 < nw) {
@@ -1704,10 +1548,14 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 //   words 4 .. 4 + RGX_REC_PIECES_MAX: where a backward can start in the middle of a tile (below);
 //   from word RGX_REC_HEAD, per iteration: WINDOW when a table was built, one LISTS per table, then TRAIL
 //   WINDOW: {tag | C, -, -, -}, pid[pad4(C)]            the table's Gaussians, by slot
-//   LISTS:  {tag | one << 9 | last << 8 | nw, len[4], -, -, -}, slot bytes of row r in pad4(len[r]) / 4 words
-//           for r = 0..3, mask[nw][64], half[2][4][nw]   (the TileLds arrays of the same names;
-//           bytes and words past a row's length are junk).  one: the rows share one list, written once.
+//   LISTS:  {tag | last << 8 | nw, len[4] (four times the same), -, -, -}, slot bytes in pad4(len) / 4 words,
+//           mask[nw][64], half[2][4][nw]   (the TileLds arrays of the same names; bytes past the list's length are junk)
 //   TRAIL:  {tag | any_search, cover (float), sample-sum slot + 1, -}, found[64] when any_search
+// Where a tile is marched by parts (record_part_lines) each of them has that share of the region and of a slot, laid out the same with as many rays as
+// the part has in the place of 64, as many rows in the place of 4, and two words before a list's slots.  Their lists together need more than the tile's, so a
+// part whose share is used up goes on in a slot of the pool (the pool's first slots are kept for that, one for each part, where they are not most of it):
+// word RGX_REC_MORE + 1 of its region is that slot + 1 (0: none), word RGX_REC_MORE the offset of the first item there; the slot's words count from the
+// end of the share.
 //
 // Sample sums.  A record with room beyond RGX_REC_LIST_WORDS per tile also has a pool of slots
 // shared by all tiles: per slab iteration that blends something, the per-sample density and colour
@@ -1734,10 +1582,10 @@ typedef uint32_t quad_bits __attribute__((ext_vector_type(4)));
 #define RGX_REC_COMPLETE 0u        // word 0 of a tile: hit lists complete
 #define RGX_REC_OVERFLOWED 1u      //   the region overflowed (record unusable)
 #define RGX_REC_COMPLETE_SUMS 2u   //   hit lists and sample sums complete
+#define RGX_REC_OVERFLOWED_UNCUT 3u //  (parts) as 1, and no list was cut at max_prim_slice: a search in any order finds the same hits
 #define RGX_REC_WINDOW 0x57000000u
 #define RGX_REC_LISTS 0x4C000000u
 #define RGX_REC_TRAIL 0x54000000u
-#define RGX_REC_ONE_LIST 0x200u    // LISTS: see above
 // Pieces of a tile's record.  A tile is a serial march for the forward, but with the rays' state at a few of its
 // iterations (transmittance, colour so far, position, step) the backward can replay the stretches between
 // them side by side, each with a wavefront of its own: a launch no longer lasts as long as its longest tile.
@@ -1754,6 +1602,7 @@ typedef uint32_t quad_bits __attribute__((ext_vector_type(4)));
 //     with pieces from 8, but 0.2 more in the forward).
 #define RGX_REC_PIECES_MAX 16
 #define RGX_REC_HEAD (4 + RGX_REC_PIECES_MAX)
+#define RGX_REC_MORE (RGX_REC_HEAD - 2)
 #define RGX_REC_STATE_WORDS (8 * 64)
 static_assert((RGX_REC_PIECES_MAX - 1) * RGX_REC_STATE_WORDS <= RGX_SUM_SLOT_WORDS, "a slot holds the states of a tile");
 struct RecordPieces {
@@ -1789,13 +1638,19 @@ __device__ __forceinline__ uint32_t record_status(const MarchParams &P, const ui
                       (uint32_t)__builtin_amdgcn_readfirstlane((int)reg[3]) == record_mark(P, 1);
     return mine && (st == RGX_REC_COMPLETE || (st == RGX_REC_COMPLETE_SUMS && P.sum_pool)) ? st : RGX_REC_OVERFLOWED;
 }
+// Of a part: overflowed, without a list that was cut (each lane may ask of another region).
+__device__ __forceinline__ bool record_uncut(const MarchParams &P, const uint32_t *reg)
+{
+    return reg[0] == RGX_REC_OVERFLOWED_UNCUT && reg[2] == record_mark(P, 0) && reg[3] == record_mark(P, 1);
+}
 __device__ __forceinline__ bool record_usable(const MarchParams &P, const uint32_t *reg)
 {
     return record_status(P, reg) != RGX_REC_OVERFLOWED;
 }
 
+template <int RAYS>
 struct Recorder {
-    uint32_t *reg;  // this tile's region, or null
+    uint32_t *reg;  // the region of this tile, or part of one, or null
     int off;        // next free word (wave-uniform)
     int cap;        // words in the region
     bool ovf;       // the region is exhausted
@@ -1807,11 +1662,32 @@ struct Recorder {
     int since = 0;       // blending iterations of the current piece
     uint32_t batch_next = 0; // the next slot of the batch this tile last took from the pool
     int batch_left = 0;      // slots left in that batch
+    uint32_t *more = nullptr; // (parts) where the region goes on, less the share's size
+    int more_from = 0, more_slot = -1;
+    bool cut = false;         // (parts) max_prim_slice has cut a ray's list
     __device__ __forceinline__ bool on() const { return reg != nullptr && !ovf; }
+    __device__ __forceinline__ uint32_t *item() const { return (RAYS < 64 && more ? more : reg) + off; }
     // room for an item and the iteration's trailer?
-    __device__ __forceinline__ bool fits(int size)
+    __device__ __forceinline__ bool fits(const MarchParams &P, int size)
     {
-        if (off + size + 72 > cap) ovf = true;
+        if (off + size + 72 > cap) {
+            if (RAYS < 64 && !more && P.sum_next) {
+                constexpr int COPIES = Part<RAYS>::COPIES;
+                uint32_t s = 0;
+                if (P.sum_first) s = (uint32_t)((reg - P.records) / P.rec_tile_words); // its own
+                else if (threadIdx.x == 0) s = atomicAdd(P.sum_next, 1u);
+                s = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
+                if (s < (uint32_t)P.sum_slots / COPIES && size + 72 <= P.sum_slot_words * COPIES) {
+                    more_slot = (int)s * COPIES;
+                    more_from = off;
+                    more = (uint32_t *)(P.sum_pool + (int64_t)more_slot * (P.sum_slot_words / 4)) - cap;
+                    off = cap;
+                    cap += P.sum_slot_words * COPIES;
+                    return true;
+                }
+            }
+            ovf = true;
+        }
         return !ovf;
     }
 
@@ -1822,9 +1698,10 @@ struct Recorder {
     {
         if (batch_left == 0) {
             uint32_t s = 0;
-            if (threadIdx.x == 0) s = atomicAdd(P.sum_next, (uint32_t)RGX_SUM_SLOT_BATCH);
-            batch_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
-            batch_left = RGX_SUM_SLOT_BATCH;
+            constexpr int COPIES = Part<RAYS>::COPIES; // (a part's slots are that share of a tile's: the counter's unit holds as many)
+            if (threadIdx.x == 0) s = atomicAdd(P.sum_next, COPIES > 1 ? 1u : (uint32_t)RGX_SUM_SLOT_BATCH);
+            batch_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)s) * (uint32_t)COPIES;
+            batch_left = COPIES > 1 ? COPIES : RGX_SUM_SLOT_BATCH;
         }
         const uint32_t s = batch_next++;
         --batch_left;
@@ -1846,38 +1723,43 @@ struct Recorder {
             }
         }
         if (threadIdx.x == 0) reg[5 + states] = (uint32_t)off;
-        float *st = (float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + states * RGX_REC_STATE_WORDS + threadIdx.x;
-        st[0] = R.T; st[64] = R.tbuffer; st[2 * 64] = R.tenter; st[3 * 64] = R.dt;
-        st[4 * 64] = Cr; st[5 * 64] = Cg; st[6 * 64] = Cb;
-        ((uint32_t *)st)[7 * 64] = (R.active ? 1u : 0u) | (R.searching ? 2u : 0u) | (R.first ? 4u : 0u);
+        float *st = (float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + states * (8 * RAYS) + threadIdx.x;
+        if (RAYS == 64 || threadIdx.x < RAYS) {
+            st[0] = R.T; st[RAYS] = R.tbuffer; st[2 * RAYS] = R.tenter; st[3 * RAYS] = R.dt;
+            st[4 * RAYS] = Cr; st[5 * RAYS] = Cg; st[6 * RAYS] = Cb;
+            ((uint32_t *)st)[7 * RAYS] = (R.active ? 1u : 0u) | (R.searching ? 2u : 0u) | (R.first ? 4u : 0u);
+        }
         ++states;
         since = 0;
         if (states >= P.rec_equal) length += (length + 1) >> 1;
     }
 
-    __device__ __forceinline__ void write_window(const TileLds &L, int C)
+    __device__ __forceinline__ void write_window(const MarchParams &P, const TileLds &L, int C)
     {
-        if (!on() || !fits(4 + ((C + 3) & ~3))) return;
-        uint32_t *it = reg + off;
+        if (!on() || !fits(P, 4 + ((C + 3) & ~3))) return;
+        uint32_t *it = item();
         if (threadIdx.x == 0) it[0] = RGX_REC_WINDOW | (uint32_t)C;
         for (int i = threadIdx.x; i < C; i += 64) it[4 + i] = __float_as_uint(L.tab[i * RGX_TAB + RGX_TAB_PID]);
         off += 4 + ((C + 3) & ~3);
     }
 
-    __device__ __forceinline__ void write_lists(const TileLds &L, int len, bool last)
+    __device__ __forceinline__ void write_lists(const MarchParams &P, const TileLds &L, int len, bool last)
     {
         if (!on()) return;
         const int lane = threadIdx.x, row = lane >> 4;
         const int nw = (len + 31) >> 5, q = (len + 3) >> 2;
-        const int size = 8 + q + nw * 72;
-        if (!fits(size)) return;
-        uint32_t *it = reg + off;
-        if (lane < 5) it[lane] = lane == 0 ? RGX_REC_LISTS | RGX_REC_ONE_LIST | (last ? 0x100u : 0u) | (uint32_t)nw : (uint32_t)len;
-        if (lane < q) it[8 + lane] = ((const uint32_t *)L.list)[lane];
+        constexpr int ROWS = Part<RAYS>::ROWS;
+        constexpr int HEAD = Part<RAYS>::LISTS_HEAD;
+        const int size = HEAD + q + nw * (RAYS + 2 * ROWS);
+        if (!fits(P, size)) return;
+        uint32_t *it = item();
+        if (lane < (RAYS == 64 ? 5 : 2)) it[lane] = lane == 0 ? RGX_REC_LISTS | (last ? 0x100u : 0u) | (uint32_t)nw : (uint32_t)len;
+        if (lane < q) it[HEAD + lane] = ((const uint32_t *)L.list)[lane];
         static_assert(RGX_CCAP <= 4 * 64, "a word of the list per lane");
-        for (int w = 0; w < nw; ++w) it[8 + q + w * 64 + lane] = L.mask[w][lane];
-        if ((lane & 15) < 2) // two lanes per row: one per half
-            for (int w = 0; w < nw; ++w) it[8 + q + nw * 64 + ((lane & 15) * 4 + row) * nw + w] = L.half[lane & 15][row][w];
+        if (RAYS == 64 || lane < RAYS)
+            for (int w = 0; w < nw; ++w) it[HEAD + q + w * RAYS + lane] = L.mask[w][lane];
+        if ((lane & 15) < 2 && (ROWS == 4 || row < ROWS)) // two lanes per row: one per half
+            for (int w = 0; w < nw; ++w) it[HEAD + q + nw * RAYS + ((lane & 15) * ROWS + row) * nw + w] = L.half[lane & 15][row][w];
         off += size;
     }
 
@@ -1894,22 +1776,26 @@ struct Recorder {
             if (sums && s >= 0) slot = s;
             else sums = false;
         }
-        uint32_t *it = reg + off;
+        uint32_t *it = item();
         if (threadIdx.x == 0) {
             it[0] = RGX_REC_TRAIL | (any_search ? 1u : 0u);
             it[1] = __float_as_uint(cover);
             it[2] = (uint32_t)(slot + 1);
         }
-        if (any_search) it[4 + threadIdx.x] = __float_as_uint(found);
-        off += 4 + (any_search ? 64 : 0);
+        if (any_search && (RAYS == 64 || threadIdx.x < RAYS)) it[4 + threadIdx.x] = __float_as_uint(found);
+        off += 4 + (any_search ? RAYS : 0);
     }
 
     __device__ __forceinline__ void finish(const MarchParams &P)
     {
         if (reg && threadIdx.x == 0) {
-            reg[0] = ovf ? RGX_REC_OVERFLOWED : (sums ? RGX_REC_COMPLETE_SUMS : RGX_REC_COMPLETE);
+            reg[0] = ovf ? (RAYS < 64 && !cut ? RGX_REC_OVERFLOWED_UNCUT : RGX_REC_OVERFLOWED) : (sums ? RGX_REC_COMPLETE_SUMS : RGX_REC_COMPLETE);
             reg[1] = (uint32_t)off;
             reg[4] = (uint32_t)states | (uint32_t)max(state_slot, 0) << 8;
+            if (RAYS < 64) {
+                reg[RGX_REC_MORE] = (uint32_t)more_from;
+                reg[RGX_REC_MORE + 1] = (uint32_t)(more_slot + 1);
+            }
             reg[2] = record_mark(P, 0);
             reg[3] = record_mark(P, 1);
         }
@@ -1918,8 +1804,8 @@ struct Recorder {
 
 // Stand-in where nothing is recorded: an image that no backward follows, or (WholeLists) one whose backward will search the tree.
 struct NoRecorder {
-    __device__ __forceinline__ void write_window(const TileLds &, int) {}
-    __device__ __forceinline__ void write_lists(const TileLds &, int, bool) {}
+    __device__ __forceinline__ void write_window(const MarchParams &, const TileLds &, int) {}
+    __device__ __forceinline__ void write_lists(const MarchParams &, const TileLds &, int, bool) {}
     static constexpr int slot = -1;
     __device__ __forceinline__ void write_trailer(const MarchParams &, bool, float, float, bool) {}
     __device__ __forceinline__ void finish(const MarchParams &) {}
@@ -1981,19 +1867,28 @@ __device__ __forceinline__ void sums_to_gradients(const Prim *pr, const float *s
 // memory every link of that chain is a round trip; staged, the chain costs one.  Words outside the staged
 // range are read from memory as before.
 #define RGX_STAGE_WORDS 448 // (as many as fit beside the rest: twelve tiles per CU)
-template <bool STAGED>
+template <bool STAGED, bool PARTS>
 struct RecordView {
     const uint32_t *reg; // the tile's region
     uint32_t *lds;       // [RGX_STAGE_WORDS] (STAGED)
     int at;              // first staged word (wave-uniform)
     int used;            // words the forward wrote
+    const uint32_t *more; // (PARTS) where words from `share` on are, less as many
+    int share, more_from; // more_from: the item after which the stream goes on at `share`, or -1
+    __device__ __forceinline__ uint32_t from_memory(int i) const
+    {
+        if constexpr (PARTS) return (i < share ? reg : more)[i];
+        else return reg[i];
+    }
+    // where the next item after the one that ends at i begins
+    __device__ __forceinline__ int next(int i) const { return PARTS && i == more_from ? share : i; }
     __device__ __forceinline__ uint32_t word(int i) const
     {
         if constexpr (STAGED) {
             const unsigned o = (unsigned)(i - at);
-            return o < (unsigned)RGX_STAGE_WORDS ? lds[o] : reg[i];
+            return o < (unsigned)RGX_STAGE_WORDS ? lds[o] : from_memory(i);
         } else {
-            return reg[i];
+            return from_memory(i);
         }
     }
     __device__ __forceinline__ uint32_t uni(int i) const { return (uint32_t)__builtin_amdgcn_readfirstlane((int)word(i)); }
@@ -2005,7 +1900,7 @@ struct RecordView {
 #pragma unroll
             for (int k = 0; k < RGX_STAGE_WORDS / 64; ++k) {
                 const int i = from + k * 64 + (int)threadIdx.x;
-                v[k] = i < used ? reg[i] : 0u;
+                v[k] = i < used ? from_memory(i) : 0u;
             }
             __syncthreads();
 #pragma unroll
@@ -2093,28 +1988,24 @@ __device__ __forceinline__ void replay_window(const MarchParams &P, const Replay
 // step); WALK 0 / 1: as shade_lanes over one half's entries; WALK_LANES_ALL: every ray walks all
 // its hits; WALK_NONE: no walk.  COUNT adds the lane's hits to p0.  Returns the item's size.
 enum { WALK_LANES_ALL = 2, WALK_ROWS_ALL = 3, WALK_NONE = 4 };
-template <bool COUNT, int WALK, typename Body, typename Cn, typename Rv>
+template <bool COUNT, int WALK, int RAYS, typename Body, typename Cn, typename Rv>
 __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLds &RL, const Rv &rv, int it, bool run, int &p0, Body body, Cn &cn)
 {
     const int lane = threadIdx.x, row = lane >> 4;
-    const uint32_t item = rv.uni(it);
-    const int nw = (int)(item & 0xffu);
-    const bool one = item & RGX_REC_ONE_LIST;
-    const int l0 = (int)rv.uni(it + 1), l1 = (int)rv.uni(it + 2), l2 = (int)rv.uni(it + 3), l3 = (int)rv.uni(it + 4);
-    const int q0 = (l0 + 3) >> 2, q1 = one ? 0 : (l1 + 3) >> 2, q2 = one ? 0 : (l2 + 3) >> 2, q3 = one ? 0 : (l3 + 3) >> 2;
-    const int len = row == 0 ? l0 : row == 1 ? l1 : row == 2 ? l2 : l3;
-    const int slots_at = it + 8 + (row > 0 && !one ? q0 : 0) + (row > 1 ? q1 : 0) + (row > 2 ? q2 : 0); // the row's slot bytes start at this word
-    const int masks_at = it + 8 + q0 + q1 + q2 + q3 + lane;                                      // word w of this lane: masks_at + w * 64
+    const int nw = (int)(rv.uni(it) & 0xffu), len = (int)rv.uni(it + 1), q = (len + 3) >> 2;
+    constexpr int HEAD = Part<RAYS>::LISTS_HEAD;
+    const int slots_at = it + HEAD;                      // the slot bytes start at this word
+    const int masks_at = slots_at + q + Part<RAYS>::ray(lane);    // word w of this lane: masks_at + w * RAYS
     if constexpr (WALK == WALK_NONE) {
         const int nwr = run ? min((len + 31) >> 5, nw) : 0;
         if (COUNT)
-            for (int w = 0; w < nwr; ++w) p0 += __popc(rv.word(masks_at + w * 64));
+            for (int w = 0; w < nwr; ++w) p0 += __popc(rv.word(masks_at + w * RAYS));
     } else if constexpr (WALK != WALK_ROWS_ALL) {
-        const int nwr = run ? min((len + 31) >> 5, nw) : 0; // words of this lane's row; later words are not its own
-        const int half_at = it + 8 + q0 + q1 + q2 + q3 + nw * 64 + ((WALK & 1) * 4 + row) * nw;
-        auto word = [&](int w) { return WALK == WALK_LANES_ALL ? rv.word(masks_at + w * 64) : rv.word(masks_at + w * 64) & rv.word(half_at + w); };
+        const int nwr = run ? min((len + 31) >> 5, nw) : 0;
+        const int half_at = slots_at + q + nw * RAYS + ((WALK & 1) * Part<RAYS>::ROWS + (RAYS == 64 ? row : row % Part<RAYS>::ROWS)) * nw;
+        auto word = [&](int w) { return WALK == WALK_LANES_ALL ? rv.word(masks_at + w * RAYS) : rv.word(masks_at + w * RAYS) & rv.word(half_at + w); };
         if (COUNT)
-            for (int w = 0; w < nwr; ++w) p0 += __popc(rv.word(masks_at + w * 64));
+            for (int w = 0; w < nwr; ++w) p0 += __popc(rv.word(masks_at + w * RAYS));
         int w = 0;
         uint32_t bits = nwr > 0 ? word(0) : 0u;
         for (;;) {
@@ -2142,11 +2033,14 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
         static_assert(!COUNT, "the rows' walk counts nothing");
         // Each half of a row (8 lanes, 2 x 4 pixels) walks the entries that one of its own rays hits: the set bits
         // of the OR of its lanes' masks.  Fewer trips than with whole rows in lock step (a trip lasts until the
-        // longest list of the wave is done, and half a row's list is shorter than the row's).
+        // longest list of the wave is done, and half a row's list is shorter than the row's).  Where a ray has copies the groups of the
+        // same rays share their entries among themselves.
+        using Pt = Part<RAYS>;
+        const int copy = Pt::copy(lane);
         const int nwr = min((len + 31) >> 5, nw);
         auto lane_word = [&](int w) {
             const int left = len - w * 32;
-            return (run ? rv.word(masks_at + w * 64) : 0u) & (left >= 32 ? ~0u : ((1u << left) - 1u));
+            return (run ? rv.word(masks_at + w * RAYS) : 0u) & (left >= 32 ? ~0u : ((1u << left) - 1u));
         };
         auto group_or = [](uint32_t m) {
             m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, true);  // quad_perm [1,0,3,2]
@@ -2156,7 +2050,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
         };
         int w = 0;
         uint32_t mword = nwr > 0 ? lane_word(0) : 0u;
-        uint32_t bits = group_or(mword);
+        uint32_t bits = Pt::skip(group_or(mword), copy);
 #ifdef RGX_SECTION_CLOCKS
         asm volatile("" :: "v"(bits)); // the first words have arrived: their wait belongs to the set-up, not to the first trip
 #endif
@@ -2174,7 +2068,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
             while (nw > 1 && __any(bits == 0u && w + 1 < nwr)) {
                 const bool next = bits == 0u && w + 1 < nwr;
                 const uint32_t m = next ? lane_word(w + 1) : 0u;
-                const uint32_t o = group_or(m);
+                const uint32_t o = Pt::skip(group_or(m), copy);
                 if (next) {
                     ++w;
                     mword = m;
@@ -2184,7 +2078,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
             Ahead a;
             a.live = bits != 0u;
             const int pos = __builtin_ctz(bits | 0x80000000u);
-            bits &= bits - 1u;
+            for (int k = 0; k < Pt::COPIES; ++k) bits &= bits - 1u;
             a.hit = a.live && ((mword >> pos) & 1u);
             a.slot = min((int)slots[min(w * 32 + pos, RGX_CCAP - 1)], RGX_CCAP - 1);
             a.pid = (int32_t)RL.pid[a.slot];
@@ -2201,7 +2095,7 @@ __device__ __forceinline__ int replay_lists(const MarchParams &P, const ReplayLd
             body(EntryAhead{(const float4 *)(RL.frame + a.slot), P.prims + (uint32_t)a.pid, a.pid, a.slot, a.pos4, a.inv4, a.rgba4}, a.hit, a.live, HalfRows{});
         }
     }
-    return 8 + q0 + q1 + q2 + q3 + nw * 72;
+    return HEAD + q + nw * (RAYS + 2 * Part<RAYS>::ROWS);
 }
 
 // Resident candidate window: the table holds every Gaussian of the tile frustum between the
@@ -2306,7 +2200,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 more = !done;
             }
             RGX_SEC(cn, RGX_SEC_SWEEP);
-            if (phase == 0 && !reuse) rec.write_window(L, C);
+            if (phase == 0 && !reuse) rec.write_window(P, L, C);
             RGX_SEC(cn, RGX_SEC_LISTS);
             if (phase == 0 || !Wn.resident || split) {
                 // phase 0 asks the lane's real question; a phase-1 re-filter only recounts the slab hits
@@ -2330,7 +2224,7 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
                 if (phase == 0) {
                     found = best;
                     searched_to = fmaxf(Q.slo, Q.shi); // a split phase may end before a searching ray's start
-                    rec.write_lists(L, len, !more);
+                    rec.write_lists(P, L, len, !more);
                 }
                 RGX_SEC(cn, RGX_SEC_LISTS);
             }
@@ -2384,21 +2278,16 @@ __device__ __forceinline__ bool slab_tables(const MarchParams &P, const TileLds 
 }
 
 // Size in words of the LISTS item at `it`.
-template <typename Rv>
+template <int RAYS, typename Rv>
 __device__ __forceinline__ int lists_size(const Rv &rv, int it)
 {
-    const uint32_t item = rv.uni(it);
-    const int nw = (int)(item & 0xffu);
-    const int l0 = (int)rv.uni(it + 1);
-    if (item & RGX_REC_ONE_LIST) return 8 + ((l0 + 3) >> 2) + nw * 72;
-    const int l1 = (int)rv.uni(it + 2), l2 = (int)rv.uni(it + 3), l3 = (int)rv.uni(it + 4);
-    return 8 + ((l0 + 3) >> 2) + ((l1 + 3) >> 2) + ((l2 + 3) >> 2) + ((l3 + 3) >> 2) + nw * 72;
+    return Part<RAYS>::LISTS_HEAD + (((int)rv.uni(it + 1) + 3) >> 2) + (int)(rv.uni(it) & 0xffu) * (RAYS + 2 * Part<RAYS>::ROWS);
 }
 
-// Walks the record stream of one tile for the backward.
-template <bool STAGED>
+// Walks the record stream of one tile, or part of one, for the backward.
+template <bool STAGED, int RAYS>
 struct Replayer {
-    RecordView<STAGED> rv; // the tile's region
+    RecordView<STAGED, (RAYS < 64)> rv; // the tile's region
     int at;              // next item
     int win_at;          // the WINDOW item whose Gaussians sit in RL.pid (-1: none yet)
     bool lost;           // the stream did not hold the items an iteration expects (the caller stops)
@@ -2411,22 +2300,23 @@ struct Replayer {
     __device__ __forceinline__ bool slab(const MarchParams &P, const RayState &R, bool need, int &p0, float &found,
                                          float &searched_to, Cn &cn, BodyA body_a, Mid mid, BodyB body_b)
     {
-        const int start = at, used = rv.used;
+        const int start = rv.next(at), used = rv.used;
         rv.stage(start);
-        int end = at; // the iteration's TRAIL item
+        int end = start; // the iteration's TRAIL item
         for (;;) {
+            end = rv.next(end);
             if (end + 4 > used) break;
             const uint32_t head = rv.uni(end);
             int size;
             if ((head & 0xff000000u) == RGX_REC_WINDOW) size = 4 + (((int)(head & 0xffffu) + 3) & ~3);
-            else if ((head & 0xff000000u) == RGX_REC_LISTS && end + 8 <= used) size = lists_size(rv, end);
+            else if ((head & 0xff000000u) == RGX_REC_LISTS && end + 2 <= used) size = lists_size<RAYS>(rv, end);
             else break;
             if (end + size > used) break;
             end += size;
         }
         const uint32_t tr = end + 4 <= used ? rv.uni(end) : 0u;
         const bool any_search = tr & 1u;
-        if ((tr & 0xff000000u) != RGX_REC_TRAIL || end + 4 + (any_search ? 64 : 0) > used) {
+        if ((tr & 0xff000000u) != RGX_REC_TRAIL || end + 4 + (any_search ? RAYS : 0) > used) {
             lost = true;
             mid(false);
             return false;
@@ -2435,13 +2325,13 @@ struct Replayer {
         RGX_SEC(cn, RGX_SEC_PARSE);
         if constexpr (SUMS) {
             auto none = [](const auto &, bool, bool, auto) {};
-            for (int a = start; a < end;) {
+            for (int a = start; a < end; a = rv.next(a)) {
                 const uint32_t head = rv.uni(a);
                 if ((head & 0xff000000u) == RGX_REC_WINDOW) {
                     replay_window(P, RL, rv, a, win_at, cn); // later iterations of the window carry no WINDOW item
                     a += 4 + (((int)(head & 0xffffu) + 3) & ~3);
                 } else {
-                    a += replay_lists<true, WALK_NONE>(P, RL, rv, a, need, p0, none, cn);
+                    a += replay_lists<true, WALK_NONE, RAYS>(P, RL, rv, a, need, p0, none, cn);
                 }
             }
             RGX_SEC(cn, RGX_SEC_COUNT);
@@ -2455,30 +2345,30 @@ struct Replayer {
                 body_a(P.sum_pool + (int64_t)(slot1 - 1u) * (P.sum_slot_words / 4));
             }
         } else {
-            for (int a = start; a < end;) {
+            for (int a = start; a < end; a = rv.next(a)) {
                 const uint32_t head = rv.uni(a);
                 if ((head & 0xff000000u) == RGX_REC_WINDOW) {
                     replay_window(P, RL, rv, a, win_at, cn);
                     a += 4 + (((int)(head & 0xffffu) + 3) & ~3);
                 } else {
-                    replay_lists<true, 0>(P, RL, rv, a, need, p0, body_a, cn);
-                    a += replay_lists<false, 1>(P, RL, rv, a, need, dummy, body_a, cn);
+                    replay_lists<true, 0, RAYS>(P, RL, rv, a, need, p0, body_a, cn);
+                    a += replay_lists<false, 1, RAYS>(P, RL, rv, a, need, dummy, body_a, cn);
                 }
             }
         }
         const float cover = __uint_as_float(rv.uni(end + 1));
-        found = any_search ? __uint_as_float(rv.word(end + 4 + (int)threadIdx.x)) : -1.0f;
+        found = any_search ? __uint_as_float(rv.word(end + 4 + Part<RAYS>::ray(threadIdx.x))) : -1.0f;
         searched_to = fminf(R.texit, cover);
-        at = end + 4 + (any_search ? 64 : 0);
+        at = end + 4 + (any_search ? RAYS : 0);
         const bool run = mid(false);
         if (__any(run)) {
-            for (int b = start; b < end;) {
+            for (int b = start; b < end; b = rv.next(b)) {
                 const uint32_t head = rv.uni(b);
                 if ((head & 0xff000000u) == RGX_REC_WINDOW) {
                     replay_window(P, RL, rv, b, win_at, cn);
                     b += 4 + (((int)(head & 0xffffu) + 3) & ~3);
                 } else {
-                    b += replay_lists<false, WALK_ROWS_ALL>(P, RL, rv, b, run, dummy, body_b, cn);
+                    b += replay_lists<false, WALK_ROWS_ALL, RAYS>(P, RL, rv, b, run, dummy, body_b, cn);
                 }
             }
         }
@@ -2487,8 +2377,8 @@ struct Replayer {
 };
 
 #define RGX_TILE_LDS(ORDER)                                           \
-    __shared__ int32_t s_queue[(ORDER) == BY_TEAM ? RGX_TEAM_QCAP + 256 : RGX_QCAP]; \
-    __shared__ int32_t s_leafq[(ORDER) == BY_TEAM ? 512 : (ORDER) == BY_PAIRS ? 192 : 128]; \
+    __shared__ int32_t s_queue[RGX_QCAP];                             \
+    __shared__ int32_t s_leafq[(ORDER) == BY_PAIRS ? 192 : 128];      \
     __shared__ __align__(16) float s_tab[RGX_CCAP * RGX_TAB];         \
     __shared__ __align__(4) uint8_t s_list[RGX_CCAP];                 \
     __shared__ uint32_t s_mask[RGX_MASK_WORDS][64];                   \
@@ -2517,24 +2407,24 @@ __device__ __forceinline__ uint8_t quantize8(float x)
 // (cuda_gui/gaussians_aabb.cu): black background, uchar4 colours, and the expected depth
 // sum T (1 - w) t over the samples (its colorBlendingT_chunked, 183-205).
 // PAIRS: how the sweeps descend (sweep_next).  WHOLE: no record, and a backward that will search the tree (slab_tables).
-// RAYS: of a tile that one wavefront marches; fewer than 64 for images only (launch_forward).
+// RAYS: of a tile that one wavefront marches (launch_forward).
 template <bool PAIRS, bool RECORD, bool VIEWER, bool STATS, bool HALF = false, bool WHOLE = false, int RAYS = 64>
-__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchParams P)
+__global__ __launch_bounds__(64) RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) void k_march_fwd(const MarchParams P)
 {
     static_assert(RECORD || !HALF, "the colour sums' format is a property of the record");
-    static_assert(RAYS == 64 || !(RECORD || WHOLE), "a record is tile by tile, and what searches the tree for a backward has 64 rays");
+    static_assert(RAYS == 64 || !WHOLE, "a backward that searches the tree without a record goes tile by tile");
     using Pt = Part<RAYS>;
     static_assert(!(RECORD || PAIRS) || !WHOLE, "a search without a record goes by nodes");
     RGX_TILE_LDS(PAIRS);
     int px0, py0, tile, part = 0;
     if (!tile_origin(P, blockIdx.x, px0, py0, &tile, Pt::BITS, &part)) return; // whole wave
-    const int copy = (int)threadIdx.x / RAYS;
+    const int copy = Pt::copy(threadIdx.x);
     px0 += Pt::WIDTH == 4 ? 4 * (part & 1) : 0;
     py0 += Pt::HEIGHT * (Pt::WIDTH == 4 ? part >> 1 : part);
-    typename std::conditional<RECORD, Recorder, typename std::conditional<WHOLE, WholeLists, NoRecorder>::type>::type rec;
-    if constexpr (RECORD) rec = Recorder{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
+    typename std::conditional<RECORD, Recorder<RAYS>, typename std::conditional<WHOLE, WholeLists, NoRecorder>::type>::type rec;
+    if constexpr (RECORD) rec = Recorder<RAYS>{P.records + (((int64_t)tile << Pt::BITS) + part) * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
     int px, py;
-    lane_pixel(px0, py0, threadIdx.x % RAYS, px, py);
+    lane_pixel(px0, py0, Pt::ray(threadIdx.x), px, py);
     const bool valid = px < P.cam.width && py < P.cam.height;
     CountersFor<STATS> cn;
     RGX_SEC_START(cn, 0);
@@ -2564,8 +2454,9 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                 if (rec.piece_due(P, false)) {
                     const bool reuse = Wn.resident && wave_max_all(need || (R.active && R.searching) ? thi : -INFINITY) <= Wn.hi;
                     if (rec.piece_due(P, reuse)) {
-                        rec.begin_piece(P, R, Cr, Cg, Cb);
-                        if (reuse) rec.write_window(L, Wn.n);
+                        if constexpr (RAYS == 64) rec.begin_piece(P, R, Cr, Cg, Cb);
+                        else rec.begin_piece(P, R, Pt::sum_of_all(Cr), Pt::sum_of_all(Cg), Pt::sum_of_all(Cb));
+                        if (reuse) rec.write_window(P, L, Wn.n);
                     }
                 }
             }
@@ -2583,30 +2474,43 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                     accumulate_samples(hs, col, sg, cr, cg, cb);
                 }
             };
+            [[maybe_unused]] float sum[4][Pt::EACH]; // (parts) a copy's run of the chunk's sums
             auto blend = [&](bool second_chunk) { // gaussians_aabb.cu:195-201
                 const float first_sample = second_chunk ? 16.5f : 0.5f; // (viewer: cuda_gui/gaussians_aabb.cu:189)
                 if constexpr (RAYS < 64) { // each copy has its run of the samples: all lanes, also of rays whose sums are zero
                     constexpr int N = Pt::EACH;
-                    float sum[4][N];
                     Pt::sums(sg, sum[0]);
                     Pt::sums(cr, sum[1]);
                     Pt::sums(cg, sum[2]);
                     Pt::sums(cb, sum[3]);
-                    float w[N], s[N], all = 1.f;
+                    float w[N], s[N], T = R.T;
 #pragma unroll
                     for (int i = 0; i < N; ++i) {
                         const float x = sum[0][i] * dt;
                         w[i] = __expf(-x);
                         s[i] = dt * ((1.0f - w[i]) * __builtin_amdgcn_rcpf(fmaxf(x, 1e-6f)));
-                        all *= w[i];
                     }
-                    float through[Pt::COPIES];
-                    Pt::of_all(all, through);
-                    float T = R.T;
+                    if constexpr (RECORD) {
+                        // one sample after the other, in every copy: a replay of the record rounds the transmittance the same way
+                        float ws[N][Pt::COPIES];
 #pragma unroll
-                    for (int k = 0; k < Pt::COPIES; ++k) {
-                        T = copy == k ? R.T : T;
-                        R.T *= through[k];
+                        for (int i = 0; i < N; ++i) Pt::of_all(w[i], ws[i]);
+#pragma unroll
+                        for (int k = 0; k < Pt::COPIES; ++k) {
+                            T = copy == k ? R.T : T;
+#pragma unroll
+                            for (int i = 0; i < N; ++i) R.T *= ws[i][k];
+                        }
+                    } else {
+                        float through[Pt::COPIES], all = w[0];
+#pragma unroll
+                        for (int i = 1; i < N; ++i) all *= w[i];
+                        Pt::of_all(all, through);
+#pragma unroll
+                        for (int k = 0; k < Pt::COPIES; ++k) {
+                            T = copy == k ? R.T : T;
+                            R.T *= through[k];
+                        }
                     }
 #pragma unroll
                     for (int i = 0; i < N; ++i) {
@@ -2635,17 +2539,67 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
                 }
             };
             // the chunk's sums go to the iteration's sample-sum slot, if it has one
-            auto keep_sums = [&](int first_sample) {
-                if constexpr (RECORD) {
+            auto keep_sums = [&](int first_sample, [[maybe_unused]] bool blended) {
+                if constexpr (RECORD && RAYS < 64) {
+                    if (rec.slot >= 0) {
+                        if (!blended) {
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                                for (int i = 0; i < Pt::EACH; ++i) sum[c][i] = 0.f;
+                        }
+                        float *slot = (float *)(P.sum_pool + (int64_t)rec.slot * (P.sum_slot_words / 4));
+                        const int sample = first_sample + Pt::EACH * copy, ray = Pt::ray(threadIdx.x);
+                        auto keep = [&](int c) { // [component][8][RAYS][4 samples]: 8 or 16 bytes at a time
+                            constexpr int RUN = Pt::EACH < 4 ? Pt::EACH : 4;
+                            typedef float run __attribute__((ext_vector_type(RUN)));
+#pragma unroll
+                            for (int i = 0; i < Pt::EACH; i += RUN) {
+                                run v;
+#pragma unroll
+                                for (int k = 0; k < RUN; ++k) v[k] = sum[c][i + k];
+                                __builtin_nontemporal_store(v, (run *)(slot + ((c * RGX_BUFFER_SIZE + sample + i) / 4 * RAYS + ray) * 4 + (sample + i) % 4));
+                            }
+                        };
+                        keep(0);
+                        if constexpr (!HALF) {
+                            keep(1);
+                            keep(2);
+                            keep(3);
+                        } else {
+                            float big = 0.f;
+#pragma unroll
+                            for (int i = 0; i < Pt::EACH; ++i) big = fmaxf(big, fmaxf(fabsf(sum[1][i]), fmaxf(fabsf(sum[2][i]), fabsf(sum[3][i]))));
+                            big = -Pt::least_of_all(-big);
+                            const int e = big > 0.f ? __builtin_amdgcn_frexp_expf(big) : 0;
+                            const float down = __builtin_amdgcn_ldexpf(1.0f, -e);
+                            const int chunk = first_sample / RGX_CHUNK_SIZE;
+                            uint32_t *col = (uint32_t *)slot + RGX_BUFFER_SIZE * RAYS + chunk * (24 * RAYS) + 3 * Pt::EACH / 2 * copy * RAYS + ray;
+                            auto value = [&](int k) { return sum[1 + k % 3][k / 3] * down; };
+#pragma unroll
+                            for (int j = 0; j < 3 * Pt::EACH / 2; ++j) {
+                                const __half2 two = __floats2half2_rn(value(2 * j), value(2 * j + 1));
+                                __builtin_nontemporal_store(*(const uint32_t *)&two, col + j * RAYS);
+                            }
+                            if (copy == 0)
+                                __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(1.0f, e), slot + RGX_BUFFER_SIZE * RAYS + 2 * 24 * RAYS + chunk * RAYS + ray);
+                        }
+                    }
+                } else if constexpr (RECORD) {
                     if (rec.slot >= 0) {
                         float *slot = (float *)(P.sum_pool + (int64_t)rec.slot * (P.sum_slot_words / 4));
                         // written once, read once by the backward: keep them out of the caches' way
                         const auto desc = __builtin_amdgcn_make_buffer_rsrc(slot, 0, P.sum_slot_words * 4, 0x00020000);
                         auto keep = [&](const float (&v)[RGX_CHUNK_SIZE], int component) {
 #pragma unroll
-                            for (int i = 0; i < RGX_CHUNK_SIZE; i += 4)
-                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(quad_bits, (quad){v[i], v[i + 1], v[i + 2], v[i + 3]}), desc, threadIdx.x * 16,
+                            for (int i = 0; i < RGX_CHUNK_SIZE; i += 4) {
+                                const quad four = {v[i], v[i + 1], v[i + 2], v[i + 3]};
+                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(quad_bits, four), desc, threadIdx.x * 16,
                                                                        (component * RGX_BUFFER_SIZE + first_sample + i) * 256, 2);
+                                // A store of 16 bytes reads its registers until one instruction later.  The compiler knows that of every form but this
+                                // one, with an offset in a scalar register: a row's last four lanes have stored what the next instruction wrote there.
+                                asm volatile("s_nop 0" ::"v"(four));
+                            }
                         };
                         keep(sg, 0);
                         if constexpr (!HALF) {
@@ -2675,9 +2629,10 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
             };
             auto second_half = [&](bool split) { // split: the hits of the second half are not known yet
                 const bool has = need && (p0 > 0 || split);
-                if (RAYS < 64 ? __any(has) : has) blend(false);
+                const bool blends = RAYS < 64 ? __any(has) : has;
+                if (blends) blend(false);
                 RGX_SEC(cn, RGX_SEC_BLEND);
-                keep_sums(0);
+                keep_sums(0, blends);
                 RGX_SEC(cn, RGX_SEC_SUMS);
                 // samples 16..31, only for rays still above the transmittance floor (gaussians_aabb.cu:190)
 #pragma unroll
@@ -2688,14 +2643,16 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
             const bool run2 = slab_tables<WALK_FORWARD, PAIRS, RAYS>(P, L, F, Wn, R, need, tlo, thi, p0, ov, found, searched_to, cn, rec, accumulate,
                                           second_half, accumulate);
             RGX_SEC(cn, RGX_SEC_TOP); // (what slab_tables did after its last section: nothing to speak of)
-            if (RAYS < 64 ? __any(run2) : run2) blend(true);
+            const bool blends2 = RAYS < 64 ? __any(run2) : run2;
+            if (blends2) blend(true);
             RGX_SEC(cn, RGX_SEC_BLEND);
-            keep_sums(RGX_CHUNK_SIZE);
+            keep_sums(RGX_CHUNK_SIZE, blends2);
             RGX_SEC(cn, RGX_SEC_SUMS);
             if (need && p0 > 0 && copy == 0) {
                 cn.slabs++;
                 cn.hit_pairs += p0;
             }
+            if constexpr (RECORD && RAYS < 64) rec.cut = rec.cut || __any(ov);
             if (ov && copy == 0) cn.overflow++;
         }
         if constexpr (STATS && RAYS < 64) {
@@ -2742,797 +2699,6 @@ __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_fwd(const MarchPara
 }
 
 // ---------------------------------------------------------------------------
-// The forward with four wavefronts per tile.  One wavefront per tile leaves most of the chip idle where an image has
-// few tiles, and ends every launch in a tail as long as one tile's serial march.  Here a workgroup of four marches the
-// tile: wavefront w has the 16 rays of the tile's 4x4 block w, each ray four times over (lane = 16 * sub + ray), and
-// the four copies share the ray's work -- in the filter they test four table entries at a time, in the shading
-// every fourth hit each; the copies' sample sums are then added up across the wavefront's rows (permlane swaps) so that
-// copy `sub` ends up with samples 4 sub .. 4 sub + 3 of the half, and blends those.  The tree is swept by all four wavefronts, 256 nodes or leaves at a time, into one table for the tile.
-// A record is written in the same format, 4x4 block by block.
-// Bound by the latency of the march's chain of slabs: an iteration costs a wavefront some 9 000 clocks, of which the
-// filter 0.27, the lists and the barriers around them 0.21, shading 0.13, the sweep 0.12 and the blend 0.11 (4 k
-// Gaussians, 128x128).  Two wavefronts per SIMD: up to 512 tiles are resident at once, and nothing is spilled.
-template <int CAP>
-struct TeamShared {
-    static constexpr int WORDS = (CAP + 31) / 32;
-    float tab[CAP * RGX_TAB];
-    int32_t queue[RGX_TEAM_QCAP];
-    int32_t leafq[512];
-    uint32_t mask[WORDS][3][4][16]; // hits over the block's list: all, with samples in the first / second half
-    uint32_t cnt[4];                // a sweep step's counts
-    float4 red[2][4];               // team_exchange
-    int32_t msg[8];                 // list lengths; [4]: the batch of sample-sum slots taken
-    uint8_t rowlist[4][(CAP + 3) & ~3];
-    uint8_t rel[4][(CAP + 3) & ~3];
-};
-struct TeamPos {
-    int wave, lane, sub, ray;
-};
-
-// What the four wavefronts have to agree on: minimum, two maxima, OR.  The barrier in here also ends every
-// wavefront's use of what was in the shared memory before it.
-struct TeamWord {
-    float lo, hi, ahead;
-    uint32_t flags;
-};
-template <int CAP>
-__device__ __forceinline__ TeamWord team_exchange(TeamShared<CAP> &S, const TeamPos &tp, int &turn, float lo, float hi, float ahead, uint32_t flags)
-{
-    if (tp.lane == 0) S.red[turn][tp.wave] = make_float4(lo, hi, ahead, __uint_as_float(flags));
-    __syncthreads();
-    const float4 a = S.red[turn][0], b = S.red[turn][1], c = S.red[turn][2], d = S.red[turn][3];
-    turn ^= 1;
-    auto uni = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
-    return {uni(fminf(fminf(a.x, b.x), fminf(c.x, d.x))), uni(fmaxf(fmaxf(a.y, b.y), fmaxf(c.y, d.y))),
-            uni(fmaxf(fmaxf(a.z, b.z), fmaxf(c.z, d.z))),
-            uni_u32(__float_as_uint(a.w) | __float_as_uint(b.w) | __float_as_uint(c.w) | __float_as_uint(d.w))};
-}
-// minimum / maximum over a row of 16 lanes, all rows holding the same values
-__device__ __forceinline__ float row_min_all(float v)
-{
-    v = fminf(v, dpp_f<0xB1, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x4E, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x141, 0xf>(INFINITY, v));
-    v = fminf(v, dpp_f<0x140, 0xf>(INFINITY, v));
-    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ float row_max_all(float v) { return -row_min_all(-v); }
-
-template <int CAP>
-__device__ __forceinline__ void team_sweep_begin(const MarchParams &P, Sweep &S, const Frustum &F, TeamShared<CAP> &T)
-{
-    S.lqn = 0;
-    if (F.cut_n > 0) {
-        S.qn = F.cut_n;
-        if ((int)threadIdx.x < F.cut_n) T.queue[threadIdx.x] = F.cut_node;
-    } else {
-        S.qn = P.n > 0 ? 1 : 0;
-        if (threadIdx.x == 0) T.queue[0] = 0;
-    }
-    __syncthreads();
-}
-
-// exclusive sum over the team's wavefronts of a 16-bit count in each half of a word, and the totals; two barriers have to
-// separate one call's word from the next one's (the caller's own barrier is the second)
-template <int CAP>
-__device__ __forceinline__ void team_counts(TeamShared<CAP> &T, const TeamPos &tp, uint32_t mine, uint32_t &before, uint32_t &total)
-{
-    if (tp.lane == 0) T.cnt[tp.wave] = mine;
-    __syncthreads();
-    const uint32_t c0 = T.cnt[0], c1 = T.cnt[1], c2 = T.cnt[2], c3 = T.cnt[3];
-    before = uni_u32((tp.wave > 0 ? c0 : 0u) + (tp.wave > 1 ? c1 : 0u) + (tp.wave > 2 ? c2 : 0u));
-    total = uni_u32(c0 + c1 + c2 + c3);
-}
-
-// frustum_cut by the team: at most 256 nodes, one per lane
-template <int CAP>
-__device__ __forceinline__ void team_frustum_cut(const MarchParams &P, Frustum &F, float t_far, TeamShared<CAP> &T, const TeamPos &tp)
-{
-    const uint64_t lt = (1ull << tp.lane) - 1ull;
-    const float4 *nodes4 = (const float4 *)P.nodes;
-    const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
-    F.range(0.f, INFINITY, 2.0f * RGX_PAD_REL * fmaxf(t_far, 1.0f));
-    int32_t node = threadIdx.x == 0 && P.n > 0 ? 0 : -1;
-    int count = P.n > 0 ? 1 : 0;
-    for (int level = 0; level < 64 && count > 0; ++level) {
-        bool keep = false, inner = false;
-        int32_t left = 0, right = 0;
-        if ((uint32_t)node < n_nodes) {
-            const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
-            right = P.right[max(0, min(node, (int32_t)P.n - 2))];
-            if (!frustum_misses(F, a, b)) {
-                left = __float_as_int(a.w);
-                inner = left >= 0;
-                keep = !inner;
-            }
-        }
-        const uint64_t bk = __ballot(keep), bi = __ballot(inner);
-        uint32_t before, total;
-        team_counts(T, tp, (uint32_t)__popcll(bk) | (uint32_t)__popcll(bi) << 16, before, total);
-        const int kept = total & 0xffff, opened = total >> 16, next = kept + 2 * opened;
-        if (opened == 0 || next > 256) break;
-        if (keep) T.queue[(before & 0xffff) + __popcll(bk & lt)] = node;
-        if (inner) {
-            const int at = kept + 2 * ((int)(before >> 16) + __popcll(bi & lt));
-            T.queue[at] = left;
-            T.queue[at + 1] = right;
-        }
-        __syncthreads();
-        node = (int)threadIdx.x < next ? T.queue[threadIdx.x] : -1;
-        count = next;
-    }
-    F.cut_n = count;
-    F.cut_node = node;
-    __syncthreads();
-}
-
-// sweep_next by the team
-template <int CAP, typename Cn>
-__device__ int team_sweep_next(const MarchParams &P, Sweep &S, const Frustum &F, TeamShared<CAP> &T, const TeamPos &tp, bool &done, bool &plain,
-                               Cn &cn)
-{
-    plain = true;
-    const uint64_t lt = (1ull << tp.lane) - 1ull;
-    const float4 *nodes4 = (const float4 *)P.nodes;
-    const uint32_t n_nodes = (uint32_t)(2 * P.n - 1);
-    int C = 0;
-    while ((S.qn > 0 || S.lqn > 0) && C < CAP) {
-        if (S.lqn >= 256 || S.qn == 0) {
-            const int m = S.lqn < 256 ? S.lqn : 256;
-            const bool mine = (int)threadIdx.x < m;
-            const int32_t left = mine ? T.leafq[S.lqn - m + threadIdx.x] : 0;
-            S.lqn -= m;
-            LeafEntry e;
-            const bool hit = mine && leaf_entry(P, F, left, e);
-            const uint64_t bl = __ballot(hit), rough = __ballot(hit && !e.plain);
-            uint32_t before, total;
-            team_counts(T, tp, (uint32_t)__popcll(bl) | (rough ? 0x10000u : 0u), before, total);
-            const int hits = total & 0xffff, room = CAP - C, rank = (int)(before & 0xffff) + __popcll(bl & lt);
-            plain = plain && (total >> 16) == 0;
-            if (hit) {
-                if (rank < room) e.store((float4 *)(T.tab + (C + rank) * RGX_TAB), left);
-                else T.leafq[S.lqn + rank - room] = left; // no room: back to the queue, for the next table
-            }
-            C += hits < room ? hits : room;
-            S.lqn += hits < room ? 0 : hits - room;
-            __syncthreads();
-            continue;
-        }
-        const int spare = RGX_TEAM_QCAP - RGX_TEAM_DFS_MARGIN - S.qn;
-        const int m = min(min(S.qn, 256), max(spare, 1));
-        const int base = S.qn - m;
-        int32_t node = -1;
-        if ((int)threadIdx.x < m) node = T.queue[base + threadIdx.x];
-        bool leaf_hit = false, inner_hit = false;
-        int32_t left = 0, right = 0;
-        if ((uint32_t)node < n_nodes) {
-            const float4 a = nodes4[2 * node], b = nodes4[2 * node + 1];
-            right = P.right[max(0, min(node, (int32_t)P.n - 2))];
-            if (!frustum_misses(F, a, b)) {
-                left = __float_as_int(a.w);
-                leaf_hit = left < 0;
-                inner_hit = !leaf_hit;
-            }
-        }
-        if (threadIdx.x == 0) cn.nodes += (unsigned)m;
-        const uint64_t bl = __ballot(leaf_hit), bi = __ballot(inner_hit);
-        uint32_t before, total;
-        team_counts(T, tp, (uint32_t)__popcll(bl) | (uint32_t)__popcll(bi) << 16, before, total); // (every node has been read)
-        if (leaf_hit) T.leafq[S.lqn + (before & 0xffff) + __popcll(bl & lt)] = left; // fewer than 256 waiting + at most 256 new
-        S.lqn += (int)(total & 0xffff);
-        if (inner_hit) {
-            const int pos = base + 2 * ((int)(before >> 16) + __popcll(bi & lt));
-            if (pos + 1 < RGX_TEAM_QCAP) {
-                T.queue[pos] = right;
-                T.queue[pos + 1] = left;
-            } else if (P.faults) {
-                atomicAdd(&P.faults[1], 1u);
-            }
-        }
-        S.qn = min(base + 2 * (int)(total >> 16), RGX_TEAM_QCAP);
-        __syncthreads();
-    }
-    done = S.qn == 0 && S.lqn == 0;
-    return C;
-}
-
-// filter_table for a block's 16 rays, four entries at a time.  len: the block's list length (wave-uniform); first, second:
-// this ray's masks over the list's first 32 entries.
-template <bool SEARCH, int PART, bool PLAIN, int CAP, typename Cn>
-__device__ __forceinline__ void team_filter(TeamShared<CAP> &T, const TeamPos &tp, int C, float t0, float t1, const LaneQuery &Q, int &p0, bool &ov,
-                                            float &found, int &len, uint32_t (&own)[2], Cn &cn)
-{
-    len = 0;
-    own[0] = own[1] = 0u;
-    // the entries whose shell meets the block's range
-    int nrel = 0;
-    for (int h = 0; h < CAP; h += 64) {
-        const int c = h + tp.lane;
-        bool rel = false;
-        if (c < C) rel = T.tab[c * RGX_TAB + RGX_TAB_DMAX] >= t0 && T.tab[c * RGX_TAB + RGX_TAB_DMIN] <= t1;
-        const uint64_t b = __ballot(rel);
-        if (rel) T.rel[tp.wave][nrel + __popcll(b & ((1ull << tp.lane) - 1ull))] = (uint8_t)c;
-        nrel += __popcll(b);
-    }
-    if (tp.lane == 0) cn.cands += (unsigned)nrel;
-    __builtin_amdgcn_wave_barrier();
-    uint32_t bits = 0, first = 0, second = 0;
-    auto flush = [&](int w) {
-        if (tp.sub == 0) {
-            T.mask[w][0][tp.wave][tp.ray] = bits;
-            T.mask[w][1][tp.wave][tp.ray] = first;
-            T.mask[w][2][tp.wave][tp.ray] = second;
-        }
-        if (w == 0) {
-            own[0] = first;
-            own[1] = second;
-        }
-        bits = first = second = 0;
-    };
-    // max_prim_slice cuts a ray's list in the order of the entries: where it could, one entry at a time
-    const int step = __any(p0 + nrel > Q.cap) ? 1 : 4;
-    for (int i = 0; i < nrel; i += step) {
-        const bool there = tp.sub < step && i + tp.sub < nrel;
-        const int c = there ? T.rel[tp.wave][i + tp.sub] : 0;
-        float r1, r2;
-        constexpr bool EXIT = std::is_same<Cn, NoCounters>::value;
-        const bool ok = lane_roots<PLAIN, EXIT>((const float4 *)(T.tab + c * RGX_TAB), Q.dir, r1, r2) && there;
-        if constexpr (EXIT) {
-            if (!__any(ok)) continue;
-        }
-        if constexpr (SEARCH) {
-            const float ts = fmaxf(Q.slo, r1);
-            const bool sfound = Q.search && ok && ts <= fminf(Q.shi, r2);
-            found = sfound ? (found < 0.0f ? ts : fminf(found, ts)) : found;
-        }
-        const bool seg = Q.need && !(SEARCH && Q.search) && !ov && ok && fmaxf(Q.tlo, r1) <= fminf(Q.thi, r2);
-        const bool f = r1 < Q.tmid, g = r2 > Q.tmid;
-        bool hit = seg && (PART == 0 || (PART == 1 ? f : g));
-        const bool counts = PART != 2 || !f;
-        if (step == 1) { // (copy 0 decides for all)
-            const bool over = seg && counts && p0 >= Q.cap;
-            hit = hit && !over;
-            const uint64_t bo = __ballot(over);
-            ov = ov || ((uint32_t)bo >> tp.ray & 1u);
-        }
-        const uint64_t bh = __ballot(hit);
-        if (bh == 0) continue;
-        if (tp.lane == 0) cn.cands_hit++;
-        const uint64_t bf = __ballot(hit && f), bg = __ballot(hit && g), bc = __ballot(hit && counts);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const uint32_t h = (uint32_t)(bh >> (16 * s)) & 0xffffu;
-            if (h == 0) continue;
-            const int at = len & 31;
-            bits |= (h >> tp.ray & 1u) << at;
-            first |= ((uint32_t)(bf >> (16 * s)) >> tp.ray & 1u) << at;
-            second |= ((uint32_t)(bg >> (16 * s)) >> tp.ray & 1u) << at;
-            p0 += (uint32_t)(bc >> (16 * s)) >> tp.ray & 1u;
-            if (tp.lane == 16 * s) T.rowlist[tp.wave][len] = (uint8_t)c;
-            ++len;
-            if ((len & 31) == 0) flush((len >> 5) - 1);
-        }
-    }
-    if (len & 31) flush(len >> 5);
-    if constexpr (SEARCH) {
-        float v[4];
-        copies(found < 0.0f ? INFINITY : found, v);
-        const float best = fminf(fminf(v[0], v[1]), fminf(v[2], v[3]));
-        found = best < INFINITY ? best : -1.0f;
-    }
-    __builtin_amdgcn_wave_barrier();
-}
-
-// shade_lanes for a block: each copy of a ray takes every fourth of the ray's hits
-template <int CAP, typename Body>
-__device__ __forceinline__ void team_shade(const MarchParams &P, TeamShared<CAP> &T, const TeamPos &tp, int len, bool run, int half,
-                                           const uint32_t (&own)[2], Body body)
-{
-    const int nw = (len + 31) >> 5;
-    auto mine = [&](uint32_t bits) { // without the first `sub` hits
-        bits = tp.sub > 0 ? bits & (bits - 1u) : bits;
-        bits = tp.sub > 1 ? bits & (bits - 1u) : bits;
-        return tp.sub > 2 ? bits & (bits - 1u) : bits;
-    };
-    int w = 0;
-    uint32_t bits = run && nw > 0 ? mine(half ? own[1] : own[0]) : 0u;
-    for (;;) {
-        while (bits == 0u && run && w + 1 < nw) {
-            ++w;
-            bits = mine(T.mask[w][1 + half][tp.wave][tp.ray]);
-        }
-        const bool has = bits != 0u;
-        if (!__any(has)) break;
-        int c = 0;
-        if (has) {
-            c = T.rowlist[tp.wave][w * 32 + __builtin_ctz(bits)];
-            bits &= bits - 1u;
-            bits &= bits - 1u;
-            bits &= bits - 1u;
-            bits &= bits - 1u;
-        }
-        const float4 *tab = (const float4 *)(T.tab + c * RGX_TAB);
-        const int32_t pid = __float_as_int(T.tab[c * RGX_TAB + RGX_TAB_PID]);
-        body(Entry<true>{tab, P.prims + pid, pid, c}, has);
-    }
-}
-
-// Recorder for a team: all its lanes carry the same offsets and flags.
-struct TeamRecorder : Recorder {
-    template <int CAP>
-    __device__ __forceinline__ void window(const TeamShared<CAP> &T, int C)
-    {
-        if (!on() || !fits(4 + ((C + 3) & ~3))) return;
-        uint32_t *it = reg + off;
-        if (threadIdx.x == 0) it[0] = RGX_REC_WINDOW | (uint32_t)C;
-        for (int i = threadIdx.x; i < C; i += 256) it[4 + i] = __float_as_uint(T.tab[i * RGX_TAB + RGX_TAB_PID]);
-        off += 4 + ((C + 3) & ~3);
-    }
-    // the blocks' list lengths are in T.msg
-    template <int CAP>
-    __device__ __forceinline__ void lists(const TeamShared<CAP> &T, const TeamPos &tp, bool last)
-    {
-        if (!on()) return;
-        const int l0 = (int)uni_u32((uint32_t)T.msg[0] & 0xffffu), l1 = (int)uni_u32((uint32_t)T.msg[1] & 0xffffu);
-        const int l2 = (int)uni_u32((uint32_t)T.msg[2] & 0xffffu), l3 = (int)uni_u32((uint32_t)T.msg[3] & 0xffffu);
-        const int nw = (max(max(l0, l1), max(l2, l3)) + 31) >> 5;
-        const int q0 = (l0 + 3) >> 2, q1 = (l1 + 3) >> 2, q2 = (l2 + 3) >> 2, q3 = (l3 + 3) >> 2;
-        const int size = 8 + q0 + q1 + q2 + q3 + nw * 72;
-        if (!fits(size)) return;
-        uint32_t *it = reg + off;
-        if (threadIdx.x == 0) {
-            it[0] = RGX_REC_LISTS | (last ? 0x100u : 0u) | (uint32_t)nw;
-            it[1] = (uint32_t)l0; it[2] = (uint32_t)l1; it[3] = (uint32_t)l2; it[4] = (uint32_t)l3;
-        }
-        const int len = tp.wave == 0 ? l0 : tp.wave == 1 ? l1 : tp.wave == 2 ? l2 : l3;
-        const int base = 8 + (tp.wave > 0 ? q0 : 0) + (tp.wave > 1 ? q1 : 0) + (tp.wave > 2 ? q2 : 0);
-        const uint32_t *slots = (const uint32_t *)T.rowlist[tp.wave];
-        if (tp.lane < ((len + 3) >> 2)) it[base + tp.lane] = slots[tp.lane];
-        const int mbase = 8 + q0 + q1 + q2 + q3, words = (len + 31) >> 5;
-        // copy s of a ray writes word s, s + 4, ...; words past the block's own list are zero
-        for (int w = tp.sub; w < nw; w += 4) it[mbase + w * 64 + tp.wave * 16 + tp.ray] = w < words ? T.mask[w][0][tp.wave][tp.ray] : 0u;
-        // which entries reach each half for some ray of the block
-        for (int w = 0; w < nw; ++w)
-            for (int half = 0; half < 2; ++half) {
-                const uint32_t v = row_or(w < words ? T.mask[w][1 + half][tp.wave][tp.ray] : 0u);
-                if (tp.lane == 0) it[mbase + nw * 64 + (half * 4 + tp.wave) * nw + w] = v;
-            }
-        off += size;
-    }
-    // A slot from the pool: thread 0 asks, where the last batch is used up (a barrier in there, for all or for none).
-    template <int CAP>
-    __device__ __forceinline__ int team_slot(const MarchParams &P, TeamShared<CAP> &T)
-    {
-        if (batch_left == 0) {
-            if (threadIdx.x == 0) T.msg[4] = (int32_t)atomicAdd(P.sum_next, (uint32_t)RGX_SUM_SLOT_BATCH);
-            __syncthreads();
-            batch_next = uni_u32((uint32_t)T.msg[4]);
-            batch_left = RGX_SUM_SLOT_BATCH;
-        }
-        const uint32_t s = batch_next++;
-        --batch_left;
-        return s < (uint32_t)P.sum_slots ? (int)s : -1;
-    }
-    template <int CAP>
-    __device__ __forceinline__ void trailer(const MarchParams &P, TeamShared<CAP> &T, const TeamPos &tp, bool any_search, float cover, float found, bool blends)
-    {
-        slot = -1;
-        if (!on()) return;
-        since += blends ? 1 : 0;
-        if (blends && P.sum_next) {
-            const int s = team_slot(P, T);
-            if (sums && s >= 0) slot = s;
-            else sums = false;
-        }
-        uint32_t *it = reg + off;
-        if (threadIdx.x == 0) {
-            it[0] = RGX_REC_TRAIL | (any_search ? 1u : 0u);
-            it[1] = __float_as_uint(cover);
-            it[2] = (uint32_t)(slot + 1);
-        }
-        if (any_search && tp.sub == 0) it[4 + tp.wave * 16 + tp.ray] = __float_as_uint(found);
-        off += 4 + (any_search ? 64 : 0);
-    }
-    // Cr, Cg, Cb: the copies' shares of the ray's colour
-    template <int CAP>
-    __device__ __forceinline__ void piece(const MarchParams &P, TeamShared<CAP> &T, const TeamPos &tp, const RayState &R, float Cr, float Cg, float Cb)
-    {
-        if (state_slot < 0) {
-            state_slot = team_slot(P, T);
-            if (state_slot < 0) {
-                sums = false;
-                return;
-            }
-        }
-        if (threadIdx.x == 0) reg[5 + states] = (uint32_t)off;
-        float r[4], g[4], b[4];
-        copies(Cr, r);
-        copies(Cg, g);
-        copies(Cb, b);
-        if (tp.sub == 0) {
-            float *st = (float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + states * RGX_REC_STATE_WORDS + tp.wave * 16 + tp.ray;
-            st[0] = R.T; st[64] = R.tbuffer; st[2 * 64] = R.tenter; st[3 * 64] = R.dt;
-            st[4 * 64] = (r[0] + r[1]) + (r[2] + r[3]);
-            st[5 * 64] = (g[0] + g[1]) + (g[2] + g[3]);
-            st[6 * 64] = (b[0] + b[1]) + (b[2] + b[3]);
-            ((uint32_t *)st)[7 * 64] = (R.active ? 1u : 0u) | (R.searching ? 2u : 0u) | (R.first ? 4u : 0u);
-        }
-        ++states;
-        since = 0;
-        if (states >= P.rec_equal) length += (length + 1) >> 1;
-    }
-};
-
-#define RGX_TEAM_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(2, 2)))
-template <bool RECORD, bool VIEWER, bool STATS, bool HALF = false>
-__global__ __launch_bounds__(256) RGX_TEAM_WAVES_ATTR void k_march_team(const MarchParams P)
-{
-    constexpr int CAP = RGX_CCAP;
-    static_assert(CAP <= 256, "a slot of the table is a byte");
-    __shared__ __align__(16) TeamShared<CAP> T;
-    int px0, py0, tile;
-    if (!tile_origin(P, blockIdx.x, px0, py0, &tile)) return; // whole workgroup
-    const int lane = threadIdx.x & 63;
-    const TeamPos tp = {__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane, lane >> 4, lane & 15};
-    typename std::conditional<RECORD, TeamRecorder, NoRecorder>::type rec;
-    if constexpr (RECORD) rec = TeamRecorder{{P.records + (int64_t)tile * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first}};
-    const int px = px0 + (tp.wave & 1) * 4 + (tp.ray & 3), py = py0 + (tp.wave >> 1) * 4 + (tp.ray >> 2);
-    const bool valid = px < P.cam.width && py < P.cam.height;
-    CountersFor<STATS> cn;
-    RGX_SEC_START(cn, 0);
-    int turn = 0;
-    Frustum F;
-    frustum_planes(P.cam, px0, py0, F);
-    RayState R;
-    ray_begin(P, px, py, valid, false, R);
-    {
-        const TeamWord far = team_exchange(T, tp, turn, 0.f, row_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f), 0.f, 0u);
-        team_frustum_cut(P, F, far.hi, T, tp);
-    }
-    const f3 dir = R.dir;
-    float Cr = 0.f, Cg = 0.f, Cb = 0.f, depth = 0.f; // this copy's shares
-    Window Wn = {0.f, 0, false, 4, false, false};
-    RGX_SEC(cn, RGX_SEC_SETUP);
-    constexpr uint32_t ACTIVE = 1u, WANT = 2u, SEARCH = 4u, NEED = 8u, RUN = 16u;
-
-    for (;;) {
-        float tlo, thi;
-        const bool need = slab_begin(P, true, R, tlo, thi);
-        const bool srch = R.active && R.searching, want = need || srch;
-        const float w0 = row_min_all(want ? tlo : INFINITY), w1 = row_max_all(want ? thi : -INFINITY);
-        const TeamWord all = team_exchange(T, tp, turn, w0, w1, row_max_all(want ? tlo + (float)Wn.k * R.slab_spacing : -INFINITY),
-                                           (__any(R.active) ? ACTIVE : 0u) | (__any(want) ? WANT : 0u) | (__any(srch) ? SEARCH : 0u) | (__any(need) ? NEED : 0u));
-        if (!(all.flags & ACTIVE)) break;
-        RGX_SEC(cn, RGX_SEC_TOP);
-        int p0 = 0;
-        bool ov = false;
-        float found = -1.0f, searched_to = 0.f;
-        if (all.flags & WANT) {
-            const float t0 = all.lo, t1 = all.hi, dt = R.dt;
-            const bool any_search = all.flags & SEARCH;
-            if constexpr (RECORD) {
-                if (rec.piece_due(P, Wn.resident && t1 <= Wn.hi)) {
-                    rec.piece(P, T, tp, R, Cr, Cg, Cb);
-                    if (Wn.resident && t1 <= Wn.hi) rec.window(T, Wn.n);
-                }
-            }
-            const float tmid = fmaf(dt, (float)RGX_CHUNK_SIZE, R.tbuffer);
-            const bool split = !RECORD && Wn.crowded && (all.flags & NEED);
-            int len = 0, q0 = 0, seen = 0;
-            uint32_t own[2] = {0u, 0u};
-            bool run = need, qov = false;
-            float sg[RGX_CHUNK_SIZE], cr[RGX_CHUNK_SIZE], cg[RGX_CHUNK_SIZE], cb[RGX_CHUNK_SIZE];
-            bool live = false; // the block has hits in this half, and sums
-            f3 rdt = dir * fmaf(dt, 0.5f, R.tbuffer);
-            auto accumulate = [&](const auto &e, bool hit) {
-                if (hit) {
-                    const float4 col = e.prim->rgba4;
-                    f3 U, V, W, inv;
-                    float k;
-                    e.frame(U, V, W, inv, k);
-                    HitSetup hs = hit_setup(U, V, W, inv, k, e.prim->pos4, dir, rdt, dt);
-                    accumulate_samples(hs, col, sg, cr, cg, cb);
-                }
-            };
-            // The half's sums over the copies, four samples per copy; they are blended (a ray without hits has none, and
-            // stays as it is) and kept in the iteration's sample-sum slot, if it has one.
-            auto blend = [&](int half) {
-                float d4[4], r4[4], g4[4], b4[4];
-                if (live) {
-                    sum_copies(sg, d4);
-                    sum_copies(cr, r4);
-                    sum_copies(cg, g4);
-                    sum_copies(cb, b4);
-                } else {
-                    if constexpr (!RECORD) return;
-                    else if (rec.slot < 0) return;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) d4[i] = r4[i] = g4[i] = b4[i] = 0.f;
-                }
-                live = false;
-                // The transmittance goes through the 16 samples one after the other, in every copy, as it does where one
-                // lane has them all: a replay of the record rounds it the same way.
-                float w4[4], s4[4], Tb = R.T, T_all = R.T;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = d4[i] * dt;
-                    w4[i] = __expf(-x);
-                    s4[i] = dt * ((1.0f - w4[i]) * __builtin_amdgcn_rcpf(fmaxf(x, 1e-6f)));
-                }
-                {
-                    float w0[4], w1[4], w2[4], w3[4];
-                    copies(w4[0], w0);
-                    copies(w4[1], w1);
-                    copies(w4[2], w2);
-                    copies(w4[3], w3);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        Tb = tp.sub == c ? T_all : Tb;
-                        T_all = (((T_all * w0[c]) * w1[c]) * w2[c]) * w3[c];
-                    }
-                }
-                float t_sample = fmaf(dt, (float)(half * RGX_CHUNK_SIZE + 4 * tp.sub) + 0.5f, R.tbuffer); // (viewer)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float ts = Tb * s4[i];
-                    Cr = fmaf(ts, r4[i], Cr);
-                    Cg = fmaf(ts, g4[i], Cg);
-                    Cb = fmaf(ts, b4[i], Cb);
-                    if constexpr (VIEWER) {
-                        depth += Tb * (1.0f - w4[i]) * t_sample;
-                        t_sample += dt;
-                    }
-                    Tb *= w4[i];
-                }
-                R.T = T_all;
-                if constexpr (RECORD) {
-                    if (rec.slot >= 0) {
-                        float *slot = (float *)(P.sum_pool + (int64_t)rec.slot * (P.sum_slot_words / 4));
-                        const int first = half * RGX_CHUNK_SIZE + 4 * tp.sub, at = tp.wave * 16 + tp.ray;
-                        quad *q = (quad *)slot + first / 4 * 64 + at;
-                        __builtin_nontemporal_store((quad){d4[0], d4[1], d4[2], d4[3]}, q);
-                        if constexpr (!HALF) {
-                            __builtin_nontemporal_store((quad){r4[0], r4[1], r4[2], r4[3]}, q + RGX_BUFFER_SIZE / 4 * 64);
-                            __builtin_nontemporal_store((quad){g4[0], g4[1], g4[2], g4[3]}, q + 2 * (RGX_BUFFER_SIZE / 4 * 64));
-                            __builtin_nontemporal_store((quad){b4[0], b4[1], b4[2], b4[3]}, q + 3 * (RGX_BUFFER_SIZE / 4 * 64));
-                        } else {
-                            float big = 0.f;
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) big = fmaxf(big, fmaxf(fabsf(r4[i]), fmaxf(fabsf(g4[i]), fabsf(b4[i]))));
-                            float v[4];
-                            copies(big, v);
-                            big = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-                            const int e = big > 0.f ? __builtin_amdgcn_frexp_expf(big) : 0;
-                            const float down = __builtin_amdgcn_ldexpf(1.0f, -e);
-                            uint32_t *col = (uint32_t *)slot + RGX_BUFFER_SIZE * 64 + half * (24 * 64) + 6 * tp.sub * 64 + at;
-                            auto value = [&](int k) { return (k % 3 == 0 ? r4[k / 3] : k % 3 == 1 ? g4[k / 3] : b4[k / 3]) * down; };
-#pragma unroll
-                            for (int k = 0; k < 6; ++k) {
-                                const __half2 two = __floats2half2_rn(value(2 * k), value(2 * k + 1));
-                                __builtin_nontemporal_store(*(const uint32_t *)&two, col + k * 64);
-                            }
-                            if (tp.sub == 0)
-                                __builtin_nontemporal_store(__builtin_amdgcn_ldexpf(1.0f, e), slot + RGX_BUFFER_SIZE * 64 + 2 * 24 * 64 + half * 64 + at);
-                        }
-                    }
-                }
-            };
-            for (int phase = 0; phase < 2; ++phase) {
-                const bool reuse = !split && Wn.resident && t1 <= Wn.hi;
-                float lo = t0, hi = t1;
-                if (split) {
-                    if (phase == 0) {
-                        hi = team_exchange(T, tp, turn, 0.f, row_max_all(need ? fminf(thi, tmid) : -INFINITY), 0.f, 0u).hi;
-                    } else {
-                        const TeamWord second = team_exchange(T, tp, turn, row_min_all(run && tmid < thi ? fmaxf(tlo, tmid) : INFINITY),
-                                                              row_max_all(run ? thi : -INFINITY), 0.f, 0u);
-                        lo = second.lo;
-                        hi = second.hi;
-                    }
-                    if (!(lo <= hi)) break;
-                }
-                Sweep S = {0, 0};
-                if (!reuse) {
-                    float wend = hi;
-                    if (!split && phase == 0 && Wn.k > 1) wend = fmaxf(t1, all.ahead);
-                    frustum_range(F, lo, wend);
-                    team_sweep_begin(P, S, F, T);
-                }
-                bool first = true, more = true;
-                while (more) {
-                    int C;
-                    bool plain;
-                    if (reuse) {
-                        C = Wn.n;
-                        plain = Wn.plain;
-                        more = false;
-                    } else {
-                        bool done;
-                        C = team_sweep_next(P, S, F, T, tp, done, plain, cn);
-                        if (split) {
-                            seen += C;
-                        } else if (phase == 0 && first) {
-                            if (done) {
-                                Wn.hi = F.t1;
-                                Wn.n = C;
-                                Wn.resident = true;
-                                Wn.plain = plain;
-                                Wn.crowded = false;
-                                if (C > RGX_KHI) Wn.k = Wn.k > 1 ? Wn.k / 2 : 1;
-                                else if (C < RGX_KLO && Wn.k < 32) Wn.k *= 2;
-                            } else if (Wn.k > 1) {
-                                Wn.k = 1;
-                                frustum_range(F, t0, t1);
-                                team_sweep_begin(P, S, F, T);
-                                continue;
-                            } else {
-                                Wn.resident = false;
-                                Wn.crowded = true;
-                            }
-                        }
-                        first = false;
-                        more = !done;
-                    }
-                    RGX_SEC(cn, RGX_SEC_SWEEP);
-                    if constexpr (RECORD) {
-                        if (phase == 0 && !reuse) rec.window(T, C);
-                    }
-                    RGX_SEC(cn, RGX_SEC_LISTS);
-                    if (phase == 0 || !Wn.resident || split) {
-                        const float cover = split ? hi : (Wn.resident ? Wn.hi : t1);
-                        const LaneQuery Q = {R.dir, run, tlo, thi, phase == 0 && srch, R.tbuffer, fminf(R.texit, cover), P.m.max_prim_slice, tmid};
-                        const bool real = phase == 0 || split;
-                        int cnt = real ? p0 : q0;
-                        bool cut = real ? ov : qov;
-                        float best = phase == 0 ? found : -1.0f;
-                        // the block's own range (its searching rays look through the whole table)
-                        const float from = fmaxf(lo, w0);
-                        auto filter = [&](auto search, auto part) {
-                            const float to = decltype(search)::value ? cover : fminf(hi, w1);
-                            if (__builtin_expect(plain, 1)) team_filter<decltype(search)::value, decltype(part)::value, true>(T, tp, C, from, to, Q, cnt, cut, best, len, own, cn);
-                            else team_filter<decltype(search)::value, decltype(part)::value, false>(T, tp, C, from, to, Q, cnt, cut, best, len, own, cn);
-                        };
-                        using std::integral_constant;
-                        if (!split) {
-                            if (phase == 0 && __any(srch)) filter(std::true_type{}, integral_constant<int, 0>{});
-                            else filter(std::false_type{}, integral_constant<int, 0>{});
-                        } else if (phase == 0) {
-                            if (__any(srch)) filter(std::true_type{}, integral_constant<int, 1>{});
-                            else filter(std::false_type{}, integral_constant<int, 1>{});
-                        } else {
-                            filter(std::false_type{}, integral_constant<int, 2>{});
-                        }
-                        if (real) {
-                            p0 = cnt;
-                            ov = cut;
-                        } else {
-                            q0 = cnt;
-                            qov = cut;
-                        }
-                        RGX_SEC(cn, RGX_SEC_FILTER);
-                        if (phase == 0) {
-                            found = best;
-                            searched_to = fmaxf(Q.slo, Q.shi);
-                            if constexpr (RECORD) {
-                                if (tp.lane == 0) T.msg[tp.wave] = len;
-                                const bool blends = __any(need && p0 > 0);
-                                if (tp.lane == 0 && blends) T.msg[tp.wave] = len | 0x10000;
-                                __syncthreads();
-                                rec.lists(T, tp, !more);
-                            }
-                        }
-                    }
-                    RGX_SEC(cn, RGX_SEC_LISTS);
-                    if (len > 0 && __any(run)) {
-                        if (!live) {
-#pragma unroll
-                            for (int i = 0; i < RGX_CHUNK_SIZE; ++i) sg[i] = cr[i] = cg[i] = cb[i] = 0.f;
-                            live = true;
-                        }
-                        team_shade(P, T, tp, len, run, phase, own, accumulate);
-                    }
-                    RGX_SEC(cn, RGX_SEC_SHADE);
-                    if (more) __syncthreads(); // every wavefront is done with the table
-                }
-                if (phase == 0) {
-                    if constexpr (RECORD) {
-                        const bool blends = uni_u32((uint32_t)(T.msg[0] | T.msg[1] | T.msg[2] | T.msg[3]) & 0x10000u) != 0;
-                        rec.trailer(P, T, tp, any_search, Wn.resident ? Wn.hi : t1, found, blends);
-                    }
-                    RGX_SEC(cn, RGX_SEC_LISTS);
-                    const bool has = need && (p0 > 0 || split);
-                    blend(0);
-                    RGX_SEC(cn, RGX_SEC_BLEND);
-                    rdt = dir * fmaf(dt, 16.5f, R.tbuffer);
-                    run = has && R.T > P.m.t_eps;
-                    if (Wn.resident && !split) continue; // the lists are still there
-                    if (!(team_exchange(T, tp, turn, 0.f, 0.f, 0.f, __any(run) ? RUN : 0u).flags & RUN)) break;
-                }
-            }
-            blend(1);
-            RGX_SEC(cn, RGX_SEC_BLEND);
-            if (split && seen < CAP / 2) Wn.crowded = false;
-            if constexpr (STATS && !RECORD) { // (as in slab_tables)
-                if (split) {
-                    const bool ask = need && !run && tmid < thi;
-                    const TeamWord rest = team_exchange(T, tp, turn, row_min_all(ask ? fmaxf(tlo, tmid) : INFINITY), row_max_all(ask ? thi : -INFINITY), 0.f,
-                                                        __any(ask) ? RUN : 0u);
-                    if (rest.flags & RUN) {
-                        const Counters work = cn;
-                        frustum_range(F, rest.lo, rest.hi);
-                        Sweep S = {0, 0};
-                        team_sweep_begin(P, S, F, T);
-                        for (bool done = false; !done;) {
-                            bool plain;
-                            const int C = team_sweep_next(P, S, F, T, tp, done, plain, cn);
-                            const LaneQuery Q = {R.dir, ask, tlo, thi, false, 0.f, 0.f, P.m.max_prim_slice, tmid};
-                            float none = -1.0f;
-                            const float from = fmaxf(rest.lo, w0), to = fminf(rest.hi, w1);
-                            if (plain) team_filter<false, 2, true>(T, tp, C, from, to, Q, p0, ov, none, len, own, cn);
-                            else team_filter<false, 2, false>(T, tp, C, from, to, Q, p0, ov, none, len, own, cn);
-                            if (!done) __syncthreads(); // every wavefront is done with the table
-                        }
-                        cn.nodes = work.nodes;
-                        cn.cands = work.cands;
-                        cn.cands_hit = work.cands_hit;
-                    }
-                }
-            }
-            if (need && p0 > 0 && tp.sub == 0) {
-                cn.slabs++;
-                cn.hit_pairs += p0;
-            }
-            if (ov && tp.sub == 0) cn.overflow++;
-        }
-        if constexpr (STATS) {
-            Counters mine = {};
-            slab_end(R, need, p0, found, searched_to, mine);
-            if (tp.sub == 0) {
-                cn.rays_hit += mine.rays_hit;
-                cn.empty += mine.empty;
-            }
-        } else {
-            slab_end(R, need, p0, found, searched_to, cn);
-        }
-        RGX_SEC(cn, RGX_SEC_END);
-    }
-    {
-        float r[4], g[4], b[4];
-        copies(Cr, r);
-        copies(Cg, g);
-        copies(Cb, b);
-        Cr = (r[0] + r[1]) + (r[2] + r[3]);
-        Cg = (g[0] + g[1]) + (g[2] + g[3]);
-        Cb = (b[0] + b[1]) + (b[2] + b[3]);
-        if constexpr (VIEWER) {
-            copies(depth, r);
-            depth = (r[0] + r[1]) + (r[2] + r[3]);
-        }
-    }
-    if (valid && tp.sub == 0) {
-        const int64_t ray = (int64_t)py * P.cam.width + px;
-        if constexpr (VIEWER) {
-            *(uchar4 *)(P.frame + 4 * ray) = make_uchar4(quantize8(Cr), quantize8(Cg), quantize8(Cb), 255);
-            P.depth[ray] = depth;
-        } else {
-            const float bg = P.m.white_background ? 1.0f : 0.0f;
-            P.ray_colors[3 * ray] = Cr + R.T * bg;
-            P.ray_colors[3 * ray + 1] = Cg + R.T * bg;
-            P.ray_colors[3 * ray + 2] = Cb + R.T * bg;
-        }
-        if constexpr (STATS) {
-            if (P.ray_counts) {
-                P.ray_counts[2 * ray] = cn.slabs;
-                P.ray_counts[2 * ray + 1] = cn.hit_pairs;
-            }
-        }
-    }
-    rec.finish(P);
-    flush_stats(P.stats, cn);
-    RGX_SEC(cn, RGX_SEC_EPILOGUE);
-    RGX_SEC_FLUSH(cn, RECORD ? RGX_SECK_FWD_RECORD : RGX_SECK_FWD_PLAIN);
-}
-
 // sum over the 16 lanes of each row, left in every lane of the row.  (Every lane of these four
 // patterns reads a lane of its own row, so bound_ctrl changes nothing but the instruction: without
 // it the last stage, whose add the compiler sinks into the one-lane-per-row branch that uses it,
@@ -3675,27 +2841,39 @@ struct GroupAdd {
 // frame (RGX_NSUM); those are summed over the rays of a group of lanes (a row of 16 in the walk by rows, half a
 // row in a replay) with DPP adds and carried on by one lane per group (all eight in a replay: GroupAdd); the
 // change of variables to the 14 gradient words comes after all sums.
-// ORDER: how a search of the tree descends.
-template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false, int ORDER = BY_NODES>
+// ORDER: how a search of the tree descends.  RAYS: of a tile, in a replay, as the forward had them; their copies share the gradient trips.  (A search of parts
+// goes by the launch's part_bits, and has lanes to spare.)
+template <bool REPLAY, bool SUMS, bool STATS, bool HALF = false, int ORDER = BY_NODES, int RAYS = 64>
 __device__ __forceinline__ void march_bwd(const MarchParams &P)
 {
     static_assert(REPLAY || !SUMS, "sample sums come with a record");
     static_assert(!REPLAY || ORDER == BY_NODES, "a replay searches no tree");
     static_assert(SUMS || !HALF, "the colour sums' format is a property of the sample sums");
-    int px0, py0, tile;
+    static_assert(REPLAY || RAYS == 64, "a search goes by part_bits");
+    using Pt = Part<RAYS>;
+    const int bits = REPLAY ? Pt::BITS : P.part_bits;
+    int px0, py0, tile, part = 0;
     // A launch that replays sample sums has a grid for every piece of the tiles' records, the last (longest) pieces first.
     const unsigned grid = SUMS ? gridDim.x / (unsigned)P.rec_pieces : gridDim.x;
     const int turn = P.rec_turn ? (int)(blockIdx.x & 7) : 0; // (the workgroup's XCD)
     const int piece = SUMS ? (2 * P.rec_pieces - 1 - (int)(blockIdx.x / grid) - turn) % P.rec_pieces : 0;
-    if (!tile_origin(P, SUMS ? blockIdx.x % grid : blockIdx.x, px0, py0, &tile)) return; // whole wave
-    const uint32_t *reg = P.records ? P.records + (int64_t)tile * P.rec_tile_words : nullptr;
+    if (!tile_origin(P, SUMS ? blockIdx.x % grid : blockIdx.x, px0, py0, &tile, bits, &part)) return; // whole wave
+    const uint32_t *reg = P.records ? P.records + (((int64_t)tile << (REPLAY ? bits : P.rec_bits)) + part) * P.rec_tile_words : nullptr;
+    [[maybe_unused]] bool mine = true; // (a search)
+    const int rays = REPLAY ? RAYS : 64 >> bits, width = bits > 1 ? 4 : 8, height = bits == 0 ? 8 : bits == 3 ? 2 : 4;
+    px0 += bits > 1 ? 4 * (part & 1) : 0;
+    py0 += height * (bits > 1 ? part >> 1 : part);
     if (REPLAY) {
         // overflowed, not this launch's, or with / without sample sums: another kernel handles the tile
         if (record_status(P, reg) != (SUMS ? RGX_REC_COMPLETE_SUMS : RGX_REC_COMPLETE)) return;
         if (SUMS && HALF != (P.m.record_format == 1)) return; // (the launcher picks the variant of the record's format)
         if (SUMS && piece > (int)(uni_u32(reg[4]) & 0xffu)) return; // the record has fewer pieces
+    } else if (P.only_overflow && bits == P.rec_bits) {
+        if (record_usable(P, reg) || (bits > 0 && record_uncut(P, reg))) return; // replayed, or the tile's
     } else if (P.only_overflow) {
-        if (record_usable(P, reg)) return; // replayed
+        // The tile, for those of its parts whose lists a search in any order finds again: one for all of them costs less than one for each.
+        mine = record_uncut(P, reg + ((int)threadIdx.x >> (6 - P.rec_bits)) * P.rec_tile_words);
+        if (!__any(mine)) return;
     }
     const int lane = threadIdx.x;
     __shared__ float s_acc[REPLAY ? RGX_NSUM * RGX_CCAP : 1];
@@ -3714,8 +2892,9 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
         __syncthreads();
     }
     int px, py;
-    lane_pixel(px0, py0, threadIdx.x, px, py);
-    const bool valid = px < P.cam.width && py < P.cam.height;
+    lane_pixel(px0, py0, Pt::ray(threadIdx.x), px, py);
+    const int copy = REPLAY ? Pt::copy(threadIdx.x) : 0;
+    const bool valid = px < P.cam.width && py < P.cam.height && (REPLAY || ((int)threadIdx.x < rays && mine));
     CountersFor<STATS> cn;
     RGX_SEC_START(cn, 1);
     RayState R;
@@ -3781,8 +2960,45 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 // A ray without a hit in the iteration asks past the end of the slot: the descriptor's check returns zeros, which is what the forward
                 // stored, and reads nothing (150 k Gaussians 619x411, rays that leave the scene early beside rays that do not: 1.48 -> 1.37 ms).
                 // (The stores of the zeros stay: lines written in part cost the forward more, 2.01 -> 2.30 there.)
-                const int mine = need && p0 > 0 ? lane * 16 : P.sum_slot_words * 4;
-                auto load = [&](int i) { return __builtin_bit_cast(quad, __builtin_amdgcn_raw_buffer_load_b128(desc, mine, i * 1024, 2)); };
+                const int mine = need && p0 > 0 ? (RAYS == 64 ? lane : copy * (QUADS / Pt::COPIES) * RAYS + Pt::ray(lane)) * 16 : P.sum_slot_words * 4;
+                auto load = [&](int i) { return __builtin_bit_cast(quad, __builtin_amdgcn_raw_buffer_load_b128(desc, mine, i * (RAYS * 16), 2)); };
+                if constexpr (RAYS < 64) { // each copy its run of the samples, in the first places (prefix)
+                    constexpr int OWN = RGX_BUFFER_SIZE / Pt::COPIES, OWN_QUADS = OWN / 4;
+                    quad d[OWN_QUADS], r[OWN_QUADS], gr[OWN_QUADS], b[OWN_QUADS];
+#pragma unroll
+                    for (int i = 0; i < OWN_QUADS; ++i) {
+                        d[i] = load(i);
+                        if constexpr (!HALF) {
+                            r[i] = load(QUADS + i);
+                            gr[i] = load(2 * QUADS + i);
+                            b[i] = load(3 * QUADS + i);
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < OWN_QUADS; ++i)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            PA[4 * i + k] = d[i][k];
+                            if constexpr (!HALF) PB[4 * i + k] = fmaf(g.x, r[i][k], fmaf(g.y, gr[i][k], g.z * b[i][k]));
+                        }
+                    if constexpr (HALF) {
+                        const int chunk = copy * OWN / RGX_CHUNK_SIZE, first = copy * OWN % RGX_CHUNK_SIZE;
+                        const uint32_t *col = (const uint32_t *)slot + RGX_BUFFER_SIZE * RAYS + (chunk * 24 + 3 * first / 2) * RAYS + Pt::ray(lane);
+                        const f3 gs = g * __builtin_nontemporal_load((const float *)slot + RGX_BUFFER_SIZE * RAYS + 2 * 24 * RAYS + chunk * RAYS + Pt::ray(lane));
+                        float v[3 * OWN];
+#pragma unroll
+                        for (int j = 0; j < 3 * OWN / 2; ++j) {
+                            const uint32_t w = __builtin_nontemporal_load(col + j * RAYS);
+                            const float2 two = __half22float2(*(const __half2 *)&w);
+                            v[2 * j] = two.x;
+                            v[2 * j + 1] = two.y;
+                        }
+#pragma unroll
+                        for (int i = 0; i < OWN; ++i) PB[i] = fmaf(gs.x, v[3 * i], fmaf(gs.y, v[3 * i + 1], gs.z * v[3 * i + 2]));
+                    }
+                    RGX_SEC(cn, RGX_SEC_SUMS);
+                    return;
+                }
 #pragma unroll
                 for (int i = 0; i < QUADS; ++i) {
                     const quad d = load(i);
@@ -3809,13 +3025,13 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 } else {
 #pragma unroll
                     for (int chunk = 0; chunk < 2; ++chunk) {
-                        const uint32_t *col = (const uint32_t *)slot + RGX_BUFFER_SIZE * 64 + chunk * (24 * 64) + lane;
-                        const float up = __builtin_nontemporal_load((const float *)slot + RGX_BUFFER_SIZE * 64 + 2 * 24 * 64 + chunk * 64 + lane);
+                        const uint32_t *col = (const uint32_t *)slot + RGX_BUFFER_SIZE * RAYS + chunk * (24 * RAYS) + Pt::ray(lane);
+                        const float up = __builtin_nontemporal_load((const float *)slot + RGX_BUFFER_SIZE * RAYS + 2 * 24 * RAYS + chunk * RAYS + Pt::ray(lane));
                         const f3 gs = g * up; // the chunk's power of two goes into dL/dC once instead of into 48 sums
                         float v[48];
 #pragma unroll
                         for (int j = 0; j < 24; ++j) {
-                            const uint32_t w = __builtin_nontemporal_load(col + j * 64);
+                            const uint32_t w = __builtin_nontemporal_load(col + j * RAYS);
                             const float2 two = __half22float2(*(const __half2 *)&w);
                             v[2 * j] = two.x;
                             v[2 * j + 1] = two.y;
@@ -3834,6 +3050,72 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             auto prefix = [&](bool) {
                 RGX_SEC(cn, RGX_SEC_WALK);
                 const bool has = need && p0 > 0;
+                if constexpr (SUMS && RAYS < 64) {
+                    // Each copy goes through its run of the samples, and has the others' results handed over (a ray without a hit goes through zeros).
+                    // (All samples in every copy: a step of 4 k Gaussians 256x256 0.83 instead of 0.79 ms, 100 k in a ball 1.17 instead of 1.14.)
+                    constexpr int OWN = RGX_BUFFER_SIZE / Pt::COPIES;
+                    float w[OWN], e[OWN], inv_d[OWN], all[Pt::COPIES], T = R.T, T_mid = R.T, sum = 0.f, before[OWN];
+                    T_after = R.T;
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) {
+                        const float sd = PA[i];
+                        inv_d[i] = sd > 0.0f ? __builtin_amdgcn_rcpf(sd) : 0.0f;
+                        e[i] = PB[i] * inv_d[i];
+                        w[i] = __expf(-sd * dt);
+                    }
+                    // the transmittance one sample after the other, as the forward rounded it
+                    float ws[OWN][Pt::COPIES];
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) Pt::of_all(w[i], ws[i]);
+#pragma unroll
+                    for (int k = 0; k < Pt::COPIES; ++k) {
+                        T = copy == k ? T_after : T;
+                        if (k * OWN == RGX_CHUNK_SIZE) T_mid = T_after;
+#pragma unroll
+                        for (int i = 0; i < OWN; ++i) T_after *= ws[i][k];
+                    }
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) {
+                        const float a = T * (1.0f - w[i]) * inv_d[i];
+                        before[i] = sum;
+                        sum += T * (1.0f - w[i]) * e[i];
+                        PA[i] = a;
+                        PB[i] = T * e[i];
+                        T *= w[i];
+                    }
+                    Pt::of_all(sum, all);
+                    float D_own = D;
+#pragma unroll
+                    for (int k = 0; k < Pt::COPIES; ++k) {
+                        D_own = copy == k ? D_after : D_own;
+                        D_after -= all[k];
+                    }
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) PB[i] = (PB[i] - (D_own - before[i])) * dt - PA[i] * e[i];
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) {
+                        float a[Pt::COPIES], b[Pt::COPIES];
+                        Pt::of_all(PA[i], a);
+                        Pt::of_all(PB[i], b);
+#pragma unroll
+                        for (int k = 0; k < Pt::COPIES; ++k) { // (the run itself last: it lies in the first places)
+                            w[i] = a[0];
+                            e[i] = b[0];
+                            if (k > 0) {
+                                PA[k * OWN + i] = a[k];
+                                PB[k * OWN + i] = b[k];
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) {
+                        PA[i] = w[i];
+                        PB[i] = e[i];
+                    }
+                    use_second = T_mid > P.m.t_eps;
+                    RGX_SEC(cn, RGX_SEC_BLEND);
+                    return has;
+                }
                 if (has) {
                     float T_mid = R.T;
 #pragma unroll
@@ -3952,19 +3234,32 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             if (has) {
                 D = D_after;
                 R.T = T_after;
-                cn.slabs++;
-                cn.hit_pairs += p0;
+                if (copy == 0) {
+                    cn.slabs++;
+                    cn.hit_pairs += p0;
+                }
             }
             if (ov) cn.overflow++;
         }
         RGX_SEC(cn, RGX_SEC_WALK);
-        slab_end(R, need, p0, found, searched_to, cn);
+        if constexpr (STATS && RAYS < 64) {
+            Counters mine = {};
+            slab_end(R, need, p0, found, searched_to, mine);
+            if (copy == 0) {
+                cn.rays_hit += mine.rays_hit;
+                cn.empty += mine.empty;
+            }
+        } else {
+            slab_end(R, need, p0, found, searched_to, cn);
+        }
         RGX_SEC(cn, RGX_SEC_END);
     };
 
     RGX_SEC(cn, RGX_SEC_SETUP);
     if constexpr (REPLAY) {
-        int used = min((int)uni_u32(reg[1]), P.rec_tile_words), start = RGX_REC_HEAD;
+        // (a part's stream may go on in a slot of the pool)
+        const int most = P.rec_tile_words + (RAYS < 64 && uni_u32(reg[RGX_REC_MORE + 1]) != 0u ? P.sum_slot_words * Pt::COPIES : 0);
+        int used = min((int)uni_u32(reg[1]), most), start = RGX_REC_HEAD;
         if constexpr (SUMS) {
             const int states = (int)(uni_u32(reg[4]) & 0xffu);
             if (piece < states && piece + 1 < P.rec_pieces) used = min((int)uni_u32(reg[5 + piece]), used);
@@ -3973,20 +3268,30 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
                 // the piece starts with the state the forward had there; what the loss's gradient still sees of the ray's
                 // colour is what the forward had not yet added to it
                 start = min((int)uni_u32(reg[5 + piece - 1]), used);
-                const float *st = (const float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + (piece - 1) * RGX_REC_STATE_WORDS + lane;
+                const float *st = (const float *)(P.sum_pool + (int64_t)state_slot * (P.sum_slot_words / 4)) + (piece - 1) * (8 * RAYS) + Pt::ray(lane);
                 R.T = st[0];
-                R.tbuffer = st[64];
-                R.tenter = st[2 * 64];
-                R.dt = st[3 * 64];
+                R.tbuffer = st[RAYS];
+                R.tenter = st[2 * RAYS];
+                R.dt = st[3 * RAYS];
                 R.slab_spacing = R.dt * RGX_BUFFER_SIZE;
-                D -= dot3(g, mk3(st[4 * 64], st[5 * 64], st[6 * 64]));
-                const uint32_t flags = ((const uint32_t *)st)[7 * 64];
+                D -= dot3(g, mk3(st[4 * RAYS], st[5 * RAYS], st[6 * RAYS]));
+                const uint32_t flags = ((const uint32_t *)st)[7 * RAYS];
                 R.active = flags & 1u;
                 R.searching = flags & 2u;
                 R.first = flags & 4u;
             }
         }
-        Replayer<SUMS> rp = {RecordView<SUMS>{reg, s_stage, -(1 << 30), used}, start, -1, false, RL};
+        const uint32_t *more = reg;
+        int share = 0, more_from = -1;
+        if constexpr (RAYS < 64) {
+            share = P.rec_tile_words;
+            const uint32_t slot1 = uni_u32(reg[RGX_REC_MORE + 1]);
+            if (slot1 != 0u && slot1 - 1u + (uint32_t)Pt::COPIES <= (uint32_t)P.sum_slots) {
+                more_from = (int)uni_u32(reg[RGX_REC_MORE]);
+                more = (const uint32_t *)(P.sum_pool + (int64_t)(slot1 - 1u) * (P.sum_slot_words / 4)) - share;
+            }
+        }
+        Replayer<SUMS, RAYS> rp = {RecordView<SUMS, (RAYS < 64)>{reg, s_stage, -(1 << 30), used, more, share, more_from}, start, -1, false, RL};
         while (__any(R.active) && !rp.lost && (!SUMS || rp.at < used)) {
             iteration([&](bool need, float, float, int &p0, bool &, float &found, float &searched_to, auto a, auto mid, auto b) {
                 return rp.template slab<SUMS>(P, R, need, p0, found, searched_to, cn, a, mid, b);
@@ -4000,11 +3305,10 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     } else {
         RGX_TILE_LDS(ORDER);
         Frustum F;
-        frustum_planes(P.cam, px0, py0, F);
+        frustum_planes(P.cam, px0, py0, F, width, height);
         {
             const float t_far = wave_max_all(R.active && R.texit < 1e30f ? R.texit : 0.f);
-            if constexpr (ORDER == BY_TEAM) frustum_cut_team(P, F, t_far, L.queue);
-            else if constexpr (ORDER == BY_PAIRS) frustum_cut_pairs(P, F, t_far, L.queue);
+            if constexpr (ORDER == BY_PAIRS) frustum_cut_pairs(P, F, t_far, L.queue);
             else frustum_cut(P, F, t_far, L.queue);
         }
         Window Wn = {0.f, 0, false, 4, false, false};
@@ -4159,29 +3463,36 @@ __global__ __launch_bounds__(1024) void k_block_order(const MarchParams P, const
 // lane; it runs for the first view of a shape, and where memory is short.)
 template <bool STATS, int ORDER>
 __global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd(const MarchParams P) { march_bwd<false, false, STATS, false, ORDER>(P); }
-template <bool STATS>
-__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd_replay(const MarchParams P) { march_bwd<true, false, STATS>(P); }
-template <bool STATS, bool HALF = false>
+template <bool STATS, int RAYS = 64>
+__global__ __launch_bounds__(64) RGX_WAVES_ATTR void k_march_bwd_replay(const MarchParams P) { march_bwd<true, false, STATS, false, BY_NODES, RAYS>(P); }
+template <bool STATS, bool HALF = false, int RAYS = 64>
 #ifndef RGX_WAVES_ATTR_SUMS
 #define RGX_WAVES_ATTR_SUMS RGX_WAVES_ATTR
 #endif
-__global__ __launch_bounds__(64) RGX_WAVES_ATTR_SUMS void k_march_bwd_replay_sums(const MarchParams P) { march_bwd<true, true, STATS, HALF>(P); }
+__global__ __launch_bounds__(64) RGX_WAVES_ATTR_SUMS void k_march_bwd_replay_sums(const MarchParams P) { march_bwd<true, true, STATS, HALF, BY_NODES, RAYS>(P); }
 
-enum { RGX_BWD_TREE, RGX_BWD_TREE_PAIRS, RGX_BWD_TREE_TEAM, RGX_BWD_LISTS, RGX_BWD_SUMS };
-static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
+enum { RGX_BWD_TREE, RGX_BWD_TREE_PAIRS, RGX_BWD_LISTS, RGX_BWD_SUMS };
+template <int RAYS>
+static void launch_replay(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
 {
     const dim3 wave(64);
     if (which == RGX_BWD_SUMS) {
-        if (stats && half) hipLaunchKernelGGL((k_march_bwd_replay_sums<true, true>), grid, wave, 0, s, P);
-        else if (stats) hipLaunchKernelGGL((k_march_bwd_replay_sums<true, false>), grid, wave, 0, s, P);
-        else if (half) hipLaunchKernelGGL((k_march_bwd_replay_sums<false, true>), grid, wave, 0, s, P);
-        else hipLaunchKernelGGL((k_march_bwd_replay_sums<false, false>), grid, wave, 0, s, P);
-    } else if (which == RGX_BWD_LISTS) {
-        if (stats) hipLaunchKernelGGL(k_march_bwd_replay<true>, grid, wave, 0, s, P);
-        else hipLaunchKernelGGL(k_march_bwd_replay<false>, grid, wave, 0, s, P);
-    } else if (which == RGX_BWD_TREE_TEAM) {
-        if (stats) hipLaunchKernelGGL((k_march_bwd<true, BY_TEAM>), grid, wave, 0, s, P);
-        else hipLaunchKernelGGL((k_march_bwd<false, BY_TEAM>), grid, wave, 0, s, P);
+        if (stats && half) hipLaunchKernelGGL((k_march_bwd_replay_sums<true, true, RAYS>), grid, wave, 0, s, P);
+        else if (stats) hipLaunchKernelGGL((k_march_bwd_replay_sums<true, false, RAYS>), grid, wave, 0, s, P);
+        else if (half) hipLaunchKernelGGL((k_march_bwd_replay_sums<false, true, RAYS>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd_replay_sums<false, false, RAYS>), grid, wave, 0, s, P);
+    } else {
+        if (stats) hipLaunchKernelGGL((k_march_bwd_replay<true, RAYS>), grid, wave, 0, s, P);
+        else hipLaunchKernelGGL((k_march_bwd_replay<false, RAYS>), grid, wave, 0, s, P);
+    }
+}
+static void launch_march_bwd(int which, bool stats, bool half, dim3 grid, hipStream_t s, const MarchParams &P)
+{
+    const dim3 wave(64);
+    if (which == RGX_BWD_SUMS || which == RGX_BWD_LISTS) {
+        if (P.part_bits == 0) launch_replay<64>(which, stats, half, grid, s, P);
+        else if (P.part_bits == 1) launch_replay<32>(which, stats, half, grid, s, P);
+        else launch_replay<16>(which, stats, half, grid, s, P);
     } else if (which == RGX_BWD_TREE_PAIRS) {
         if (stats) hipLaunchKernelGGL((k_march_bwd<true, BY_PAIRS>), grid, wave, 0, s, P);
         else hipLaunchKernelGGL((k_march_bwd<false, BY_PAIRS>), grid, wave, 0, s, P);
@@ -4270,10 +3581,10 @@ __global__ __launch_bounds__(256) void k_clear_backward(float4 *p, int64_t n4, u
 
 // A forward: the 16 bytes at a and at b (either may be null), the bump counter of the record's sample-sum pool and the
 // workspace's fault counters; and n words at cost.
-__global__ __launch_bounds__(256) void k_clear_forward(float4 *a, float4 *b, uint32_t *cost, int n)
+__global__ __launch_bounds__(256) void k_clear_forward(float4 *a, uint32_t first, float4 *b, uint32_t *cost, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0 && a) *a = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i == 0 && a) *a = make_float4(__uint_as_float(first), 0.f, 0.f, 0.f);
     if (i == 1 && b) *b = make_float4(0.f, 0.f, 0.f, 0.f);
     if (i < n) cost[i] = 0u;
 }
@@ -4366,21 +3677,19 @@ static int fill_params(MarchParams &P, const void *ws, const RgxCamera *cam, con
     P.records = nullptr;
     P.rec_tile_words = 0;
     P.only_overflow = 0;
-    const RecordPieces rp = record_pieces(P.tiles_x * P.tiles_y);
-    P.rec_pieces = march->record_format == 1 ? min(rp.most, RGX_SUM_SLOT_WORDS_HALF / RGX_REC_STATE_WORDS + 1) : rp.most;
-    P.rec_first = rp.first;
-    P.rec_equal = rp.equal;
-    P.rec_turn = rp.turn;
+    P.rec_pieces = 1;
+    P.rec_first = P.rec_equal = P.rec_turn = 0;
     // room for the tile order?  (a workspace sized for fewer rays, or an image of extreme proportions, goes without)
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const size_t order_words = (size_t)8 * g.per_xcd * g.bw * g.bh;
     P.tile_order = M.order + order_words * sizeof(uint32_t) <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.order) : nullptr;
     P.use_tile_order = 0;
-    P.part_bits = 0;
+    P.part_bits = P.rec_bits = 0;
     P.faults = M.order <= march_ws_bytes ? (uint32_t *)((char *)march_ws + M.faults) : nullptr;
     P.ray_counts = nullptr;
     P.sum_pool = nullptr;
     P.sum_next = nullptr;
+    P.sum_first = 0;
     P.sum_slots = 0;
     P.sum_slot_words = RGX_SUM_SLOT_WORDS;
     if (march->record_format != 0 && march->record_format != 1) return RGX_EINVAL;
@@ -4396,6 +3705,7 @@ extern "C" int rgx_march_records_bytes(int32_t width, int32_t height, int32_t ti
     return RGX_OK;
 }
 
+static int part_bits(const MarchParams &P, bool image_only);
 static int attach_records(MarchParams &P, void *records, size_t records_bytes)
 {
     if (!records) return RGX_OK;
@@ -4415,6 +3725,19 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
     } else {
         P.rec_tile_words = (int32_t)words & ~3;
     }
+    // By parts of tiles: each has its share of the region, and slots of its share of the size.
+    const int bits = part_bits(P, false);
+    P.part_bits = P.rec_bits = bits;
+    P.rec_tile_words = P.rec_tile_words >> bits & ~3;
+    if (bits > 0 && P.sum_slots >= (int64_t)(ntiles << bits) + (int64_t)ntiles) P.sum_first = (uint32_t)(ntiles << bits); // (a slot for each, before the sums have taken all)
+    P.sum_slot_words >>= bits;
+    P.sum_slots = (int32_t)std::min<int64_t>((int64_t)P.sum_slots << bits, 0x7fffffff);
+    RecordPieces rp = record_pieces((int)std::min<int64_t>((int64_t)ntiles << bits, 0x7fffffff));
+    if (bits > 0) rp.most = std::min(rp.most, RGX_REC_MORE - 4); // (what would be the last pieces' words say where a region goes on)
+    P.rec_pieces = P.m.record_format == 1 ? min(rp.most, RGX_SUM_SLOT_WORDS_HALF / RGX_REC_STATE_WORDS + 1) : rp.most;
+    P.rec_first = rp.first;
+    P.rec_equal = rp.equal;
+    P.rec_turn = rp.turn;
     return RGX_OK;
 }
 
@@ -4445,27 +3768,38 @@ struct PartLines {
 };
 static inline PartLines image_part_lines(bool adaptive) { return adaptive ? PartLines{256, 800, 1600} : PartLines{768, 2048, 3200}; }
 
-// Records of the fixed step, up to this many tiles: four wavefronts march a tile (k_march_team), beyond it one (forward at 1 024, one / four: 4 k in a cube 0.76 / 0.50, 100 k in a ball
-// 1.97 / 1.28, 1 M in a ball of radius 2 5.64 / 5.15).  The team, too, adds up a sample's hits in another order, and keeps other hits of a list that is cut.
+// Records by parts.  Which: those of the fixed step.
 //   No record: the backward searches the tree again, one wavefront per tile, and has to meet the hits and the
-//     transmittance of the forward: that is k_march_fwd then, whatever the step, and every slab's list in one (slab_tables).
+//     transmittance of the forward: that is a march of whole tiles then, whatever the step, and every slab's list in one (slab_tables).
 //   A record and the adaptive step: the next step's length depends on the last bit of the transmittance, and a sample that
 //     so crosses a Gaussian's cut-off moves that Gaussian's gradient by a visible part (1e-3 of the norm at 150 k Gaussians):
-//     no longer the gradients that larger images give.  k_march_fwd.
-//   A record and the fixed step: what the backward replays is what the team recorded.  (A tile whose region overflowed is
-//     searched again, in the team's order: lists that max_prim_slice cut are cut to the same hits there.)
-#define RGX_TEAM_TILES_RECORD 1024
+//     no longer the gradients that larger images give.  Whole tiles.
+//   A record and the fixed step: what the backward replays is what the parts recorded, and against 64 bits its gradients are as good (3 k Gaussians,
+//     512 rays 240x320: 2.2e-6 to 3.0e-6 of their norm, whole tiles 4.8e-6 to 5.4e-6; where a sample lies at a cut-off both the same).  (A part whose region overflowed is
+//     searched again, as it was marched: lists that max_prim_slice cut are cut to the same hits there.)
+// Measured, ms of a training step by whole tiles / halves / 4x4, where not taken before by four wavefronts a tile (up to 1 024 tiles: in brackets):
+//     tiles                               400                    784                  1 024                 1 156
+//     4 k Gaussians in a cube     [0.87] 0.86 0.75       [0.83] 0.88 0.79      [0.80] 0.89 0.79
+//     16 k in a cube              [1.43] 1.25 0.93       [1.24] 1.26 1.02      [1.15] 1.28 1.04       1.61 1.30 1.09
+//     300 k in a ball             [16.2] 4.31 3.06 (625)
+//     20 k in a ball of radius 2  [0.70] 0.75 0.66       [0.81] 0.79 0.76      [0.89] 0.80 0.84       0.93 0.80 0.90
+//     100 k, radius 2             [7.99] 2.53 1.47       [2.35] 1.88 1.85      [2.30] 1.83 1.97       2.73 2.06 2.29
+//     300 k, radius 2             [13.4] 3.79 2.14       [11.5] 3.13 2.69      [10.7] 3.13 2.96       10.1 3.32 3.29
+//     tiles                             1 296                1 600                1 936                2 304           2 500
+//     16 k in a cube                1.60 1.30 1.17       1.54 1.23 1.29       1.62 1.31            1.69 1.45
+//     20 k, radius 2                0.92 0.81 0.96       1.00 0.89 1.07       0.95 0.94            1.00 1.02
+//     100 k, radius 2               2.73 2.28 2.37       2.86 2.38 2.68       2.69 2.48            2.47 2.80      2.61 3.00
+//     300 k, radius 2               9.51 3.58 3.52       10.1 3.50 3.88       4.20 3.72            4.58 4.43      4.05 4.50
+// The lines lie where one of these scenes stops gaining (1 k Gaussians alone take 0.52 -> 0.54 at 900 to 1 024 tiles).  The large gains are
+// those of scenes whose tiles' lists overflowed their regions: by parts these go on in slots.  (Eighths: a record's overhead per part outgrows them.)
+static inline PartLines record_part_lines() { return {0, 1200, 2000}; }
 
 // image_only: no backward follows this launch
 static bool sums_in_any_order(const MarchParams &P, bool image_only) { return image_only || (P.records && !P.m.dynamic_sampling); }
-static bool by_team(const MarchParams &P, bool image_only)
-{
-    return !image_only && P.tiles_x * P.tiles_y <= RGX_TEAM_TILES_RECORD && sums_in_any_order(P, image_only);
-}
 static int part_bits(const MarchParams &P, bool image_only)
 {
-    if (!image_only) return 0;
-    const PartLines L = image_part_lines(P.m.dynamic_sampling);
+    if (!sums_in_any_order(P, image_only)) return 0;
+    const PartLines L = image_only ? image_part_lines(P.m.dynamic_sampling) : record_part_lines();
     const int tiles = P.tiles_x * P.tiles_y;
     return tiles <= L.eighths ? 3 : tiles <= L.quarters ? 2 : tiles <= L.halves ? 1 : 0;
 }
@@ -4480,15 +3814,14 @@ static void prepare_forward(MarchParams &P, bool image_only, hipStream_t s)
     // 800x800, 3.3 rounds: 5.51 -> 5.32 ms; 300 k there 2.84 -> 2.82; 3 M at 1237x822, 5.2 rounds: 9.71 -> 9.67; 3 M at
     // 1920x1080, 10.5 rounds: 17.12 -> 17.09).  Nor does it where every wavefront starts at once.
     const int64_t tiles = (int64_t)P.tiles_x * P.tiles_y;
-    const bool team = by_team(P, image_only);
-    P.part_bits = part_bits(P, image_only);
+    if (!P.records) P.part_bits = part_bits(P, image_only); // (else it is the record's)
     const TileGrid g = tile_grid(P.tiles_x, P.tiles_y);
     const int nb = g.blocks_x * ((P.tiles_y + g.bh - 1) / g.bh);
-    const bool at_once = team ? tiles <= 256 : P.part_bits > 0 && tiles << P.part_bits <= 3072;
+    const bool at_once = P.part_bits > 0 && tiles << P.part_bits <= 3072;
     const bool ordered = P.tile_order && P.n > 0 && tiles <= 6 * 3072 && !at_once && nb <= RGX_COST_BINS; // (more blocks: a very long, thin image)
     uint32_t *order = P.tile_order, *cost = ordered ? P.tile_order + 8 * g.per_xcd : nullptr;
     if (P.sum_next || P.faults || ordered)
-        hipLaunchKernelGGL(k_clear_forward, dim3(ordered ? (unsigned)((nb + 255) / 256) : 1u), dim3(256), 0, s, (float4 *)P.sum_next, (float4 *)P.faults, cost, ordered ? nb : 0);
+        hipLaunchKernelGGL(k_clear_forward, dim3(ordered ? (unsigned)((nb + 255) / 256) : 1u), dim3(256), 0, s, (float4 *)P.sum_next, P.sum_first, (float4 *)P.faults, cost, ordered ? nb : 0);
     if (!ordered) return;
     const int per_group = (int)((((P.n + 511) / 512) + 255) / 256 * 256); // 512 workgroups at most, whole waves
     hipLaunchKernelGGL(k_block_cost, dim3((unsigned)((P.n + per_group - 1) / per_group)), dim3(256), 0, s, P, cost, nb, per_group);
@@ -4511,50 +3844,50 @@ static inline dim3 march_grid(const MarchParams &P)
 #define RGX_PAIR_TILES (6 * 3072)
 static bool by_pairs(const MarchParams &P, bool image_only)
 {
-    return sums_in_any_order(P, image_only) && !by_team(P, image_only) && P.n <= RGX_PAIR_BOXES && P.tiles_x * P.tiles_y <= RGX_PAIR_TILES;
+    return sums_in_any_order(P, image_only) && P.n <= RGX_PAIR_BOXES && P.tiles_x * P.tiles_y <= RGX_PAIR_TILES;
 }
 // half: the record's colour sums are in half precision
 static void launch_forward(const MarchParams &P, bool viewer, bool counting, bool half, bool image_only, hipStream_t s)
 {
-    const bool team = by_team(P, image_only), pairs = by_pairs(P, image_only);
-    const dim3 grid = march_grid(P), block(team ? 256 : 64);
+    const bool pairs = by_pairs(P, image_only);
+    const dim3 grid = march_grid(P), block(64);
+    // what: RECORD, VIEWER, STATS, HALF
+#define RGX_FWD_OF(RAYS, RECORD, VIEWER, STATS, HALF)                                           \
+    do {                                                                                        \
+        if (pairs) hipLaunchKernelGGL((k_march_fwd<true, RECORD, VIEWER, STATS, HALF, false, RAYS>), grid, block, 0, s, P); \
+        else hipLaunchKernelGGL((k_march_fwd<false, RECORD, VIEWER, STATS, HALF, false, RAYS>), grid, block, 0, s, P); \
+    } while (0)
 #define RGX_FWD(...)                                                                            \
     do {                                                                                        \
-        if (team) hipLaunchKernelGGL((k_march_team<__VA_ARGS__>), grid, block, 0, s, P);        \
-        else if (pairs) hipLaunchKernelGGL((k_march_fwd<true, __VA_ARGS__>), grid, block, 0, s, P); \
-        else hipLaunchKernelGGL((k_march_fwd<false, __VA_ARGS__>), grid, block, 0, s, P);       \
+        if (P.part_bits == 0) RGX_FWD_OF(64, __VA_ARGS__);                                      \
+        else if (P.part_bits == 1) RGX_FWD_OF(32, __VA_ARGS__);                                 \
+        else if (P.part_bits == 2) RGX_FWD_OF(16, __VA_ARGS__);                                 \
+        else RGX_FWD_EIGHTH(__VA_ARGS__);                                                       \
     } while (0)
-#define RGX_FWD_PART(RAYS, ...)                                                                 \
-    do {                                                                                        \
-        if (pairs) hipLaunchKernelGGL((k_march_fwd<true, false, __VA_ARGS__, false, false, RAYS>), grid, block, 0, s, P); \
-        else hipLaunchKernelGGL((k_march_fwd<false, false, __VA_ARGS__, false, false, RAYS>), grid, block, 0, s, P); \
-    } while (0)
-#define RGX_FWD_IMAGE(...)                                                                      \
-    do {                                                                                        \
-        if (P.part_bits == 0) RGX_FWD_PART(64, __VA_ARGS__);                                    \
-        else if (P.part_bits == 1) RGX_FWD_PART(32, __VA_ARGS__);                               \
-        else if (P.part_bits == 2) RGX_FWD_PART(16, __VA_ARGS__);                               \
-        else RGX_FWD_PART(8, __VA_ARGS__);                                                      \
-    } while (0)
+#define RGX_FWD_EIGHTH(...) RGX_FWD_OF(8, __VA_ARGS__) // (a record is of quarters at the finest)
     if (viewer) {
-        if (counting) RGX_FWD_IMAGE(true, true);
-        else RGX_FWD_IMAGE(true, false);
+        if (counting) RGX_FWD(false, true, true, false);
+        else RGX_FWD(false, true, false, false);
+#undef RGX_FWD_EIGHTH
+#define RGX_FWD_EIGHTH(...) RGX_FWD_OF(16, __VA_ARGS__)
     } else if (P.records && half) {
         if (counting) RGX_FWD(true, false, true, true);
         else RGX_FWD(true, false, false, true);
     } else if (P.records) {
-        if (counting) RGX_FWD(true, false, true);
-        else RGX_FWD(true, false, false);
+        if (counting) RGX_FWD(true, false, true, false);
+        else RGX_FWD(true, false, false, false);
     } else if (!image_only) {
         if (counting) hipLaunchKernelGGL((k_march_fwd<false, false, false, true, false, true>), grid, block, 0, s, P);
         else hipLaunchKernelGGL((k_march_fwd<false, false, false, false, false, true>), grid, block, 0, s, P);
     } else {
-        if (counting) RGX_FWD_IMAGE(false, true);
-        else RGX_FWD_IMAGE(false, false);
+#undef RGX_FWD_EIGHTH
+#define RGX_FWD_EIGHTH(...) RGX_FWD_OF(8, __VA_ARGS__)
+        if (counting) RGX_FWD(false, false, true, false);
+        else RGX_FWD(false, false, false, false);
     }
-#undef RGX_FWD_IMAGE
-#undef RGX_FWD_PART
+#undef RGX_FWD_EIGHTH
 #undef RGX_FWD
+#undef RGX_FWD_OF
 }
 
 static int march_forward_launch(const void *ws, const RgxCamera *cam, const RgxMarch *march, const float *prims, int64_t n,
@@ -4709,7 +4042,7 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
     void *span = timed ? rgx_span_begin(RGX_T_MARCH_BWD, s) : nullptr;
     if (P.records) {
         // tiles with a complete record replay it; the few whose record overflowed are recomputed
-        if (P.tile_order) {
+        if (P.tile_order && P.part_bits == 0) {
             hipLaunchKernelGGL(k_tile_order, dim3(8), dim3(256), 0, s, P);
             P.use_tile_order = 1;
         }
@@ -4719,7 +4052,12 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
         P.only_overflow = 1;
         P.use_tile_order = 0;
     }
-    launch_march_bwd(by_team(P, false) ? RGX_BWD_TREE_TEAM : by_pairs(P, false) ? RGX_BWD_TREE_PAIRS : RGX_BWD_TREE, stats != nullptr, false, march_grid(P), s, P);
+    const int tree = by_pairs(P, false) ? RGX_BWD_TREE_PAIRS : RGX_BWD_TREE;
+    launch_march_bwd(tree, stats != nullptr, false, march_grid(P), s, P);
+    if (P.part_bits > 0) {
+        P.part_bits = 0;
+        launch_march_bwd(tree, stats != nullptr, false, march_grid(P), s, P);
+    }
     rgx_span_end(span, s);
     span = timed ? rgx_span_begin(RGX_T_UNPERMUTE, s) : nullptr;
     hipLaunchKernelGGL(k_unpermute_grads, grid_for(n, 256), dim3(256), 0, s, (const float4 *)P.gbuf, P.place, n, ddens, drgb,

@@ -218,6 +218,7 @@ REC_TILE_WORDS = 16384 + 64 * 8192
 # this many slots per tile: its forward counts the slots it would have used, tiles that find the pool empty
 # are replayed from their hit lists (slower, same gradients), and the second view's pool is sized from the count.
 REC_FIRST_SLOTS = 12
+REC_PART_TILES = 2000         # images of more tiles are not recorded by parts of tiles (record_part_lines, rgx_march.hip)
 
 
 REC_LIST_WORDS = 16384        # the hit lists' share of a tile's record
@@ -299,7 +300,8 @@ def new_records(cam, device, tile_words=REC_TILE_WORDS, budget_bytes=None, n=0, 
                 have = (want + REC_POOL_STEP - 1) // REC_POOL_STEP * REC_POOL_STEP
         elif not have:
             have = REC_FIRST_SLOTS * ntiles
-        have = max(min(have, 64 * ntiles), ntiles)     # (the library wants at least one slot per tile to keep sums at all)
+        # (the library wants at least one slot per tile to keep sums at all; of an image by parts, parts' lists go on in slots as well)
+        have = max(min(have, (64 if ntiles > REC_PART_TILES else 96) * ntiles), ntiles)
         nbytes = max(head + 256 + have * _slot_words(record_format) * 4, ntiles * (REC_LIST_WORDS + REC_SLOT_WORDS) * 4)
         if nbytes <= budget_bytes:
             try:

@@ -668,9 +668,9 @@ def test_images_by_parts_of_tiles(gx, dyn, w, h, scale, n):
     assert torch.equal(depth.reshape(-1)[hit] > 0, torch.ones_like(hit[hit]))
 
 
-@pytest.mark.parametrize("w,h", [(52, 44), (216, 224), (253, 256)])              # 1 024 tiles: the most that four wavefronts march
+@pytest.mark.parametrize("w,h", [(52, 44), (216, 224), (253, 256)])              # by 4x4 blocks
 def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
-    """What the four wavefronts of a tile leave for the backward, in each form: sample sums in floats and in half
+    """What the parts of a tile leave for the backward, in each form: sample sums in floats and in half
     precision, and hit lists alone.  The image does not depend on the form.  Float sums and lists give the gradients of
     a backward that searches the tree; half precision rounds a colour sum by at most 2^-12 of the chunk's
     largest, and a gradient's norm is that of many of them: 2^-12 of it."""
@@ -696,7 +696,34 @@ def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     assert np.abs(images[0] - tree["image"]).max() <= 1e-5
 
 
-# with the fixed step: up to 1 024 tiles four wavefronts per tile; 1 056 and 1 482 tiles sweeps by pairs; 18 632 by nodes
+# either side of 1 200 and of 2 000 tiles: 4x4 blocks, halves, whole tiles.  Odd sizes: parts without a ray
+@pytest.mark.parametrize("w,h", [(5, 3), (237, 315), (240, 320), (243, 319), (317, 399), (319, 408)])
+def test_records_by_parts_of_tiles(gx, w, h):
+    """The gradients of a record by parts, in each form, with hardly room for a part's share (its lists go on in a slot of the pool) and with none in the
+    pool either (some parts are searched again): those of a backward that searches whole tiles, up to the order of sums (1e-4, as above).
+    Half precision rounds a colour sum by at most 2^-12 times the power of two above its chunk's largest: by 2^-11 of the largest, and a gradient's norm with it."""
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=5000, sh_degree=1, seed=21))
+    sc["scales"] = sc["scales"] * 3.0
+    cam = scenes.make_camera(0, 0, width=w, height=h)
+    cfg = dict(dt_step=0.01, dynamic_sampling=False, max_prim_slice=4096)
+    dloss = np.random.default_rng(3).normal(size=(w * h, 3)).astype(np.float32)
+    _step(f"records by parts {w}x{h}")
+    tree = gx.gpu_render(sc, cam, cfg, want_grad=dloss, record_hits=False)
+    images = []
+    for name, kw, tol in [("sums", dict(), 1e-4), ("half sums", dict(half_sums=True), 2.0 ** -11), ("lists", dict(rec_tile_words=16384), 1e-4),
+                          ("few slots", dict(rec_tile_words=16384 + 2 * 8192), 1e-4), ("short lists", dict(rec_tile_words=2048), 1e-4)]:
+        out = gx.gpu_render(sc, cam, cfg, want_grad=dloss, **kw)
+        assert out["stats_bwd"]["hit_pairs"] == tree["stats_bwd"]["hit_pairs"], name
+        assert w == 5 or (out["stats_bwd"]["nodes_visited"] > 0) == (name == "short lists"), name
+        images.append(out["image"])
+        for k in ("positions", "scales", "quaternions", "densities", "color_features"):
+            cos, rel = gx.cos_rel(out["grads"][k], tree["grads"][k])
+            assert cos >= 1 - 1e-6 and rel <= tol, (name, k, cos, rel)
+    assert all(np.array_equal(images[0], i) for i in images[1:])
+    assert np.abs(images[0] - tree["image"]).max() <= 1e-5
+
+
+# with the fixed step: up to 1 200 tiles by 4x4 blocks; 1 482 by halves; 18 632 whole tiles, by nodes
 @pytest.mark.parametrize("w,h", [(52, 44), (100, 80), (253, 256), (257, 256), (312, 304), (1089, 1082)])
 @pytest.mark.parametrize("dyn,cap", [(False, 8), (False, 32), (False, 4096), (True, 32)])
 def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx, w, h, dyn, cap):
@@ -725,7 +752,7 @@ def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx,
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 129, 257, 1025, -3000])      # (negative: at one place, a tree of chains)
-@pytest.mark.parametrize("w,h", [(52, 44), (264, 264)])                          # in the order of four wavefronts; by pairs
+@pytest.mark.parametrize("w,h", [(52, 44), (264, 264)])                          # by 4x4 blocks
 @pytest.mark.parametrize("cap", [4, 4096])
 def test_searches_in_the_place_of_a_replay_find_what_the_forward_found(gx, n, w, h, cap):
     """Trees from a single leaf up, with the backward handed an empty record: every tile is searched, in the forward's order, and the gradients are
@@ -760,7 +787,7 @@ def test_searches_in_the_place_of_a_replay_find_what_the_forward_found(gx, n, w,
             assert not x.any() and not got.any() or (cos >= 1 - 1e-6 and rel <= 1e-4), (cos, rel)
 
 
-@pytest.mark.parametrize("w,h", [(19, 13), (221, 216), (225, 224), (289, 288), (1096, 1084)])    # four wavefronts a tile; halves of tiles; pairs; nodes
+@pytest.mark.parametrize("w,h", [(19, 13), (221, 216), (225, 224), (289, 288), (1096, 1084)])    # parts of tiles; pairs; nodes
 @pytest.mark.parametrize("config,scale", [(0, 6.0), (0, 1.0)])
 def test_hits_counted_are_those_of_whole_lists_on_every_way(gx, w, h, config, scale):
     """``hit_pairs`` says how many hits a view's slabs have, not how a kernel came by them: an image that collects its crowded slabs half by
