@@ -2851,13 +2851,15 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     static_assert(SUMS || !HALF, "the colour sums' format is a property of the sample sums");
     static_assert(REPLAY || RAYS == 64, "a search goes by part_bits");
     using Pt = Part<RAYS>;
-    const int bits = REPLAY ? Pt::BITS : P.part_bits;
+    // A search in the place of a replay by parts has a grid for the parts, then one for the whole tiles.
+    const unsigned of_parts = REPLAY || P.part_bits == 0 ? 0u : (gridDim.x / ((1u << P.part_bits) + 1u)) << P.part_bits;
+    const int bits = REPLAY ? Pt::BITS : blockIdx.x < of_parts ? P.part_bits : 0;
     int px0, py0, tile, part = 0;
     // A launch that replays sample sums has a grid for every piece of the tiles' records, the last (longest) pieces first.
     const unsigned grid = SUMS ? gridDim.x / (unsigned)P.rec_pieces : gridDim.x;
     const int turn = P.rec_turn ? (int)(blockIdx.x & 7) : 0; // (the workgroup's XCD)
     const int piece = SUMS ? (2 * P.rec_pieces - 1 - (int)(blockIdx.x / grid) - turn) % P.rec_pieces : 0;
-    if (!tile_origin(P, SUMS ? blockIdx.x % grid : blockIdx.x, px0, py0, &tile, bits, &part)) return; // whole wave
+    if (!tile_origin(P, SUMS ? blockIdx.x % grid : REPLAY || bits > 0 ? blockIdx.x : blockIdx.x - of_parts, px0, py0, &tile, bits, &part)) return; // whole wave
     const uint32_t *reg = P.records ? P.records + (((int64_t)tile << (REPLAY ? bits : P.rec_bits)) + part) * P.rec_tile_words : nullptr;
     [[maybe_unused]] bool mine = true; // (a search)
     const int rays = REPLAY ? RAYS : 64 >> bits, width = bits > 1 ? 4 : 8, height = bits == 0 ? 8 : bits == 3 ? 2 : 4;
@@ -4053,11 +4055,8 @@ static int march_backward_launch(const void *ws, const RgxCamera *cam, const Rgx
         P.use_tile_order = 0;
     }
     const int tree = by_pairs(P, false) ? RGX_BWD_TREE_PAIRS : RGX_BWD_TREE;
-    launch_march_bwd(tree, stats != nullptr, false, march_grid(P), s, P);
-    if (P.part_bits > 0) {
-        P.part_bits = 0;
-        launch_march_bwd(tree, stats != nullptr, false, march_grid(P), s, P);
-    }
+    const unsigned parts = march_grid(P).x;
+    launch_march_bwd(tree, stats != nullptr, false, dim3(P.part_bits > 0 ? parts + (parts >> P.part_bits) : parts), s, P);
     rgx_span_end(span, s);
     span = timed ? rgx_span_begin(RGX_T_UNPERMUTE, s) : nullptr;
     hipLaunchKernelGGL(k_unpermute_grads, grid_for(n, 256), dim3(256), 0, s, (const float4 *)P.gbuf, P.place, n, ddens, drgb,
