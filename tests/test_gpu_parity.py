@@ -1680,6 +1680,25 @@ def test_update_acceleration_structure_refits_the_tree(gx, orc):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 511, 512, 513, 1024, 1025, 5000])      # a workgroup of the refit has 512 leaves
+@pytest.mark.parametrize("kind", ["spread", "line", "one place"])
+def test_tree_at_the_edges_of_the_refits_workgroups(gx, n, kind):
+    """Boxes, children, parents and skip links of a build and of a refit, checked node by node on the host."""
+    from raygaussx_amd import optix_utils as u_ox
+    from test_gpu_fullsize import _check_tree, _read_tree
+    rng = np.random.default_rng(n)
+    centre = {"spread": rng.normal(size=(n, 3)), "line": np.linspace(0, 1, n)[:, None] * np.float32([1, 0, 0]), "one place": np.zeros((n, 3))}[kind]
+    half = rng.uniform(0.01, 0.1, size=(n, 3))
+    boxes = torch.tensor(np.concatenate([centre - half, centre + half], 1).astype(np.float32), device=gx.DEV)
+    _step(f"tree of {n}, {kind}")
+    gas = u_ox.create_acceleration_structure(None, boxes)
+    _check_tree(_read_tree(gx, gas), n, boxes.cpu().numpy())
+    boxes = boxes + 0.25
+    u_ox.update_acceleration_structure(gas, boxes)
+    _check_tree(_read_tree(gx, gas), n, boxes.cpu().numpy())
+
+
+@pytest.mark.gpu
 def test_settings_update_refits_inside_the_render_function(gx):
     """render_optix.py:114-117: with ``settings.update`` the forward hands the new boxes to the
     existing acceleration structure instead of creating one.  A loop that moves the Gaussians between
