@@ -418,7 +418,8 @@ __device__ __forceinline__ void table_frame(const float4 *e, f3 &U, f3 &V, f3 &W
 // compiler emits for `/` and sqrtf(), without their range handling (v_div_scale / v_div_fixup,
 // the 2^32 pre-scaling of small sqrt arguments, the special-value checks).  Where that handling
 // would do nothing -- b and a / b far from the ends of the exponent range, |a| >= 2^-104,
-// 2^-96 <= x < infinity -- the results are bit-identical to `/` and sqrtf().
+// 2^-96 <= x < infinity -- the results are bit-identical to `/` and sqrtf().  (Kept for rgx_check_plain_arith: no kernel takes roots where
+// their cost shows.)
 __device__ __forceinline__ float div_rn_plain(float a, float b)
 {
     float r = __builtin_amdgcn_rcpf(b);
@@ -436,8 +437,7 @@ __device__ __forceinline__ float sqrt_rn_plain(float x)
     return r_up > 0.0f ? up : z;
 }
 
-// Whether the divisions and the square root of lane_roots() may take the plain forms for every
-// ray through a Gaussian: inv = (1 / scale) / k per axis, c = |S^-1 R^T (eye - centre)|^2 - 1.
+// Whether every ray through a Gaussian has a quadratic of ordinary size, which the filter's margin is derived for, and the plain forms' range: inv = (1 / scale) / k per axis, c = |S^-1 R^T (eye - centre)|^2 - 1.
 // For a unit direction a = |De|^2 lies in [min inv^2, max inv^2]; where the line hits
 // (disc > 1e-7) disc * a >= 1e-7 min inv^2 and |q| lies in [sqrt(1e-7) min inv, (sqrt(c + 1) + 1) max inv].
 __device__ __forceinline__ bool plain_roots(f3 inv, float c)
@@ -895,10 +895,7 @@ struct TileLds {
 };
 
 // Ray-interval-independent half of __intersection__gaussian (gaussians_aabb.cu:43-82) on a table
-// entry: same arithmetic as line_roots(), with the precomputed ray-independent parts.  PLAIN: the
-// entry passed plain_roots().  EXIT: return early (false for every lane, roots zero) when no
-// lane's line meets the ellipsoid.
-template <bool PLAIN, bool EXIT>
+// entry: same arithmetic as line_roots(), with the precomputed ray-independent parts.
 __device__ __forceinline__ bool lane_roots(const float4 *e, f3 dir, float &r1, float &r2)
 {
     f3 U, V, W, inv;
@@ -909,22 +906,15 @@ __device__ __forceinline__ bool lane_roots(const float4 *e, f3 dir, float &r1, f
     const float a = fmaf(De.x, De.x, fmaf(De.y, De.y, De.z * De.z));
     const float b = -fmaf(Oe.x, De.x, fmaf(Oe.y, De.y, Oe.z * De.z));
     const float c = ((const float *)e)[RGX_TAB_C];
-    const float inv_a = PLAIN ? div_rn_plain(1.0f, a) : 1.0f / a;
+    const float inv_a = 1.0f / a;
     const float b_inv_a = b * inv_a;
     const f3 Pc = mk3(fmaf(b_inv_a, De.x, Oe.x), fmaf(b_inv_a, De.y, Oe.y), fmaf(b_inv_a, De.z, Oe.z));
     const float d2 = fmaf(Pc.x, Pc.x, fmaf(Pc.y, Pc.y, Pc.z * Pc.z));
     const float disc = 1.0f - d2;
-    // EXIT: an entry whose ellipsoid the lines of all 64 rays miss needs no roots
-    if constexpr (EXIT) {
-        if (!__any(disc > 1e-7f)) {
-            r1 = r2 = 0.f;
-            return false;
-        }
-    }
     // no branch per lane: where the line misses (disc <= 1e-7) the roots are garbage and the result false
-    const float sdisc = PLAIN ? sqrt_rn_plain(disc * a) : sqrtf(disc * a);
+    const float sdisc = sqrtf(disc * a);
     const float q = b + copysignf(sdisc, b);
-    r1 = PLAIN ? div_rn_plain(c, q) : c / q;
+    r1 = c / q;
     r2 = q * inv_a;
     return disc > 1e-7f;
 }
@@ -1301,7 +1291,7 @@ __device__ __forceinline__ void filter_table(const TileLds &L, int C, float t0, 
             if ((f | g) == 0) continue;
             if (__builtin_expect((~sure | ((f | g) & searching)) != 0, 0)) {
                 float r1, r2;
-                const bool ok = lane_roots<false, false>(e, Q.dir, r1, r2);
+                const bool ok = lane_roots(e, Q.dir, r1, r2);
                 // first-hit query (searching lanes): smallest max(slo, r1) over the entries hit in [slo, shi]
                 const float ts = fmaxf(Q.slo, r1);
                 const bool sfound = Q.search && ok && ts <= fminf(Q.shi, r2);
@@ -1414,7 +1404,7 @@ __device__ __forceinline__ void filter_part(const TileLds &L, int C, float t0, f
             if ((f | g) == 0) continue;
             if (__builtin_expect(((~sure & valid) | ((f | g) & searching)) != 0, 0)) {
                 float r1, r2;
-                const bool ok = lane_roots<false, false>(e, Q.dir, r1, r2) && copy < there;
+                const bool ok = lane_roots(e, Q.dir, r1, r2) && copy < there;
                 const float ts = fmaxf(Q.slo, r1);
                 const bool sfound = Q.search && ok && ts <= fminf(Q.shi, r2);
                 found = sfound ? (found < 0.0f ? ts : fminf(found, ts)) : found;
