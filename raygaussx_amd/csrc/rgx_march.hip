@@ -2399,7 +2399,7 @@ __device__ __forceinline__ uint8_t quantize8(float x)
 // PAIRS: how the sweeps descend (sweep_next).  WHOLE: no record, and a backward that will search the tree (slab_tables).
 // RAYS: of a tile that one wavefront marches (launch_forward).
 template <bool PAIRS, bool RECORD, bool VIEWER, bool STATS, bool HALF = false, bool WHOLE = false, int RAYS = 64>
-__global__ __launch_bounds__(64) RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) void k_march_fwd(const MarchParams P)
+RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) __global__ __launch_bounds__(64) void k_march_fwd(const MarchParams P)
 {
     static_assert(RECORD || !HALF, "the colour sums' format is a property of the record");
     static_assert(RAYS == 64 || !WHOLE, "a backward that searches the tree without a record goes tile by tile");
