@@ -3783,7 +3783,9 @@ static inline PartLines image_part_lines(bool adaptive) { return adaptive ? Part
 //     100 k, radius 2               2.73 2.28 2.37       2.86 2.38 2.68       2.69 2.48            2.47 2.80      2.61 3.00
 //     300 k, radius 2               9.51 3.58 3.52       10.1 3.50 3.88       4.20 3.72            4.58 4.43      4.05 4.50
 // The lines lie where one of these scenes stops gaining (1 k Gaussians alone take 0.52 -> 0.54 at 900 to 1 024 tiles).  The large gains are
-// those of scenes whose tiles' lists overflowed their regions: by parts these go on in slots.  (Eighths of a tile have not been built for a record.)
+// those of scenes whose tiles' lists overflowed their regions: by parts these go on in slots.
+// (Eighths gain with up to 144 tiles -- 64 tiles: 4 k 0.80 -> 0.67, 16 k 1.27 -> 0.92, 300 k in a ball 52.8 -> 3.78 -- and lose from 256 on: 20 k of radius 2
+// 0.64 -> 0.70.  But their windows, eight times as many, add a Gaussian's sums to memory more often than a search for the whole tile would.)
 static inline PartLines record_part_lines() { return {0, 1200, 2000}; }
 
 // image_only: no backward follows this launch
