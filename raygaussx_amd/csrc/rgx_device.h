@@ -269,12 +269,20 @@ __device__ __forceinline__ bool box_overlaps(const RayBox &rb, float4 a, float4 
 }
 
 // Pixel -> ray (cuda_train/forward/gaussians_aabb.cu:95-110 computeRay).
-__device__ __forceinline__ f3 compute_ray(const RgxCamera &c, unsigned ix, unsigned iy)
+// What a pixel column's rays have of u, and a pixel row's of v, before they are normalised.
+__device__ __forceinline__ float column_x(const RgxCamera &c, unsigned ix)
 {
     const float idx_x = ((float)ix + 0.5f) / (float)(unsigned)c.width;
+    return 2.0f * (idx_x - c.principal_x) * c.tan_half_fov_x;
+}
+__device__ __forceinline__ float row_y(const RgxCamera &c, unsigned iy)
+{
     const float idx_y = ((float)iy + 0.5f) / (float)(unsigned)c.height;
-    const float px = 2.0f * (idx_x - c.principal_x), py = 2.0f * (idx_y - c.principal_y);
-    const float dx = px * c.tan_half_fov_x, dy = py * c.tan_half_fov_y;
+    return 2.0f * (idx_y - c.principal_y) * c.tan_half_fov_y;
+}
+__device__ __forceinline__ f3 compute_ray(const RgxCamera &c, unsigned ix, unsigned iy)
+{
+    const float dx = column_x(c, ix), dy = row_y(c, iy);
     const f3 d = mk3((dx * c.u[0] + dy * c.v[0]) + c.w[0], (dx * c.u[1] + dy * c.v[1]) + c.w[1],
                      (dx * c.u[2] + dy * c.v[2]) + c.w[2]);
     const float inv = 1.0f / sqrtf(dot3(d, d)); // vec_math.h:554-558 normalize

@@ -668,6 +668,39 @@ def test_images_by_parts_of_tiles(gx, dyn, w, h, scale, n):
     assert torch.equal(depth.reshape(-1)[hit] > 0, torch.ones_like(hit[hit]))
 
 
+# an image by 4x2 pixels (756 tiles; a strip of 760), 4x4 blocks (1 225), halves (2 500) and whole tiles (3 249); its record by 4x4 blocks, halves, whole tiles
+@pytest.mark.parametrize("fov,w,h", [(5.0, 216, 224), (40.0, 760, 64), (5.0, 276, 276), (5.0, 312, 304), (5.0, 400, 400), (5.0, 456, 456), (1.0, 216, 224), (1.0, 456, 456)])
+def test_narrow_pixels_lose_no_hit(gx, orc, fov, w, h):
+    """Where neighbouring rays are a ten-thousandth apart a part's frustum still holds all that its rays meet: as many slabs and hits as the oracle counts
+    ray by ray (small spheres, of which many are only grazed, and too thin for any ray to end), in the image, in the forward that leaves a record, in the forward by
+    whole tiles, and in a search of the tree in the place of a replay."""
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.render_optix import compute_rgb
+    n = 6000
+    sc = scenes.scene_to_numpy(scenes.make_scene(0, n=n, sh_degree=0, seed=5))
+    sc["scales"] = np.repeat(np.exp(np.random.default_rng(1).normal(size=(n, 1)) * 0.4 - 3.5).astype(np.float32), 3, 1)
+    sc["densities"][:] = 0.2
+    at = np.float32([13.0, 14.0, 12.0]) * (5.0 / fov if fov < 40.0 else 0.18)
+    cam = scenes.look_at_camera(tuple(float(x) for x in at), fov_x_deg=fov, width=w, height=h)
+    _, want, ctx = orc.render_forward(sc, cam, 0.01, False, 4096, cull=True)
+    orc.cull_free()
+    d = gx.to_dev(sc)
+    params = d["positions"], d["scales"], d["quaternions"], d["densities"]
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+    cs = u_ox.camera_struct(cam)
+    rgb = compute_rgb(cam.camera_center, d["positions"], d["color_features"], None, None, None, 0, 0)
+    prims = u_ox.pack_prims(gas, cs, *params, rgb)
+    _step(f"narrow pixels, {w}x{h} over {fov} degrees")
+    st = [u_ox.new_stats(gx.DEV) for _ in range(4)]
+    u_ox.launch_pipeline_test(None, None, gas, None, None, 0.01, False, cam, params[3], rgb, *params[:3], 4096, stats=st[0])
+    rec = torch.empty(u_ox.records_bytes(cs, 16384 * 4), dtype=torch.uint8, device=gx.DEV)
+    image = u_ox.march_forward(gas, cs, prims, 0.01, False, 4096, True, records=rec, stats=st[1])
+    u_ox.march_forward(gas, cs, prims, 0.01, False, 4096, True, stats=st[2])
+    u_ox.march_backward(gas, cs, prims, image, torch.ones_like(image), 0.01, False, 4096, True, records=torch.zeros_like(rec), stats=st[3])
+    got = [u_ox.read_stats(s) for s in st]
+    assert [(g["slabs"], g["hit_pairs"]) for g in got] == [(want["slabs"], want["hit_pairs"])] * 4
+
+
 @pytest.mark.parametrize("w,h", [(52, 44), (216, 224), (253, 256)])              # by 4x4 blocks
 def test_record_forms_of_a_small_image_with_the_fixed_step(gx, w, h):
     """What the parts of a tile leave for the backward, in each form: sample sums in floats and in half
