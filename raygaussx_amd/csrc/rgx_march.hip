@@ -2481,6 +2481,7 @@ RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) __global__ __launch_bounds__(64) void k_
                     Pt::sums(cg, sum[2]);
                     Pt::sums(cb, sum[3]);
                     float w[N], s[N], T = R.T;
+                    [[maybe_unused]] const float tbuffer = need ? R.tbuffer : 0.0f; // (a ray that is not marching may be at no finite place)
 #pragma unroll
                     for (int i = 0; i < N; ++i) {
                         const float x = sum[0][i] * dt;
@@ -2515,7 +2516,7 @@ RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) __global__ __launch_bounds__(64) void k_
                         Cr = fmaf(ts, sum[1][i], Cr);
                         Cg = fmaf(ts, sum[2][i], Cg);
                         Cb = fmaf(ts, sum[3][i], Cb);
-                        if constexpr (VIEWER) depth += T * (1.0f - w[i]) * fmaf(dt, first_sample + (float)(N * copy + i), R.tbuffer);
+                        if constexpr (VIEWER) depth += T * (1.0f - w[i]) * fmaf(dt, first_sample + (float)(N * copy + i), tbuffer);
                         T *= w[i];
                     }
                     return;

@@ -668,6 +668,37 @@ def test_images_by_parts_of_tiles(gx, dyn, w, h, scale, n):
     assert torch.equal(depth.reshape(-1)[hit] > 0, torch.ones_like(hit[hit]))
 
 
+@pytest.mark.parametrize("w,h", [(45, 64), (225, 224), (393, 400), (457, 456)])    # 4x2 pixels, 4x4 blocks, halves, whole tiles
+@pytest.mark.parametrize("axis", [0, 1])
+def test_viewer_depth_of_rays_that_are_nowhere(gx, axis, w, h):
+    """A ray whose direction has a component of exactly zero, with the eye beside the box on that axis, enters the box at no finite distance: its depth is
+    zero, whatever the rays marched together with it meet."""
+    from raygaussx_amd import _lib as L
+    from raygaussx_amd import optix_utils as u_ox
+    w, h = (w, h) if axis == 0 else (h, w)
+    n = 4000
+    rng = np.random.default_rng(2)
+    pos = rng.uniform(0.0, 0.5, size=(n, 3)).astype(np.float32)
+    pos[:, 1 - axis] -= 0.25
+    pos[:, 2] += 4.0
+    d = gx.to_dev(dict(positions=pos, scales=np.full((n, 3), 0.02, np.float32), quaternions=np.float32([[1, 0, 0, 0]]).repeat(n, 0),
+                       densities=np.full(n, 2.0, np.float32), rgb=np.full((n, 3), 0.5, np.float32)))
+    params = d["positions"], d["scales"], d["quaternions"], d["densities"]
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+    cs = L.RgxCamera()
+    cs.u[0] = cs.v[1] = cs.w[2] = 1.0
+    cs.tan_half_fov_x = cs.tan_half_fov_y = 0.1
+    cs.principal_x = cs.principal_y = 0.5
+    cs.width, cs.height = w, h
+    cs.eye[axis] = float(u_ox.ellipsoids_bbox_from_quat(params[2], params[0], params[1], params[3])[1][axis]) - 1e-3
+    prims = u_ox.pack_prims(gas, cs, *params, d["rgb"])
+    _step(f"viewer depth, {w}x{h}")
+    _, depth = u_ox.march_viewer(gas, cs, prims, 0.01, False, 4096)
+    depth = depth if axis == 0 else depth.T
+    mid = depth.shape[1] // 2
+    assert torch.isfinite(depth).all() and (depth[:, : mid + 1] == 0).all() and (depth[:, mid + 1:] > 3.0).sum() > 100
+
+
 # an image by 4x2 pixels (756 tiles; a strip of 760), 4x4 blocks (1 225), halves (2 500) and whole tiles (3 249); its record by 4x4 blocks, halves, whole tiles
 @pytest.mark.parametrize("fov,w,h", [(5.0, 216, 224), (40.0, 760, 64), (5.0, 276, 276), (5.0, 312, 304), (5.0, 400, 400), (5.0, 456, 456), (1.0, 216, 224), (1.0, 456, 456)])
 def test_narrow_pixels_lose_no_hit(gx, orc, fov, w, h):
