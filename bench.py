@@ -528,7 +528,7 @@ def training_leg(dev, workload, steps, warmup, opts, in_flight=1):
     out["views_in_flight"] = flight
     if sections is not None:
         out["sections"] = sections
-    rec_use = None if forward_only else u_ox.record_use(cam_structs[0], dev, n, 1 if opts.half_sums else 0)
+    rec_use = None if forward_only else u_ox.record_use(cam_structs[0], dev, n, 1 if opts.half_sums else 0, cfg["dynamic_sampling"])
     out["memory"] = dict(first_view_peak_GB=round(first_peak / 1e9, 3), steady_peak_GB=round(steady_peak / 1e9, 3),
                          first_over_steady=round(first_peak / max(steady_peak, 1), 3),
                          resident_before_GB=round(base_mem / 1e9, 3),

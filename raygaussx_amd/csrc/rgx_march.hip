@@ -1620,12 +1620,13 @@ static inline RecordPieces record_pieces(int tiles)
 }
 
 // Words 2 and 3 of a tile's region name the launch the record belongs to (number of Gaussians,
-// image size, step), so that a backward handed a record of another scene or view recomputes the
-// tile instead of following indices that mean nothing in its own tables.
+// image size, step, fixed or adaptive), so that a backward handed a record of another scene or view recomputes the
+// tile instead of following indices that mean nothing in its own tables.  (Size and kind of step also say by which parts of tiles a region
+// is laid out: record_part_lines.)
 __device__ __forceinline__ uint32_t record_mark(const MarchParams &P, int which)
 {
     return which == 0 ? (uint32_t)P.n ^ ((uint32_t)P.m.record_format << 31)
-                      : ((uint32_t)P.cam.width << 16 ^ (uint32_t)P.cam.height ^ __float_as_uint(P.m.dt_step));
+                      : ((uint32_t)P.cam.width << 16 ^ (uint32_t)P.cam.height ^ __float_as_uint(P.m.dt_step) ^ (P.m.dynamic_sampling ? 0x55555555u : 0u));
 }
 // Status of a tile's record if it is this launch's and complete, else RGX_REC_OVERFLOWED.
 __device__ __forceinline__ uint32_t record_status(const MarchParams &P, const uint32_t *reg)

@@ -248,7 +248,7 @@ def fit_tile_words(cam, tile_words, budget_bytes):
 # What the forward launches of one scene size and image shape on one stream asked of the sample-sum pool
 # (the launch's whole demand: every blending slab iteration asks, served or not), so that the next record
 # is allocated for the need:
-# (device, stream, Gaussians, width, height) -> {"pinned": host int32[1], "event", "pending", "need": slots the
+# (device, stream, Gaussians, width, height, record format, adaptive step) -> {"pinned": host int32[1], "event", "pending", "need": slots the
 #                             last views asked for, "slots": the pool size in use, "allocated": bytes of the last record}
 _rec_usage = {}
 REC_POOL_MARGIN = 1.05        # pool = this times the largest need of the last views ...
@@ -256,8 +256,9 @@ REC_POOL_STEP = 1 << 12       # ... rounded up to a multiple of this many slots 
 REC_POOL_HISTORY = 8
 
 
-def _usage_key(cam, device, n, record_format=0):
-    return (str(device), torch.cuda.current_stream(device).cuda_stream, int(n), cam.width, cam.height, int(record_format))
+def _usage_key(cam, device, n, record_format=0, dynamic_sampling=False):
+    return (str(device), torch.cuda.current_stream(device).cuda_stream, int(n), cam.width, cam.height, int(record_format),
+            bool(dynamic_sampling))
 
 
 def _slot_words(record_format):
@@ -269,7 +270,7 @@ def _pool_geometry(cam):
     return ntiles, ntiles * REC_LIST_WORDS * 4        # tiles, bytes of the hit-list regions (the pool header follows)
 
 
-def new_records(cam, device, tile_words=REC_TILE_WORDS, budget_bytes=None, n=0, record_format=0):
+def new_records(cam, device, tile_words=REC_TILE_WORDS, budget_bytes=None, n=0, record_format=0, dynamic_sampling=False):
     """Buffer for the record of one forward launch (see rgx_march_records_bytes), or None when no
     record fits the budget or the allocator.  The budget defaults to REC_MEMORY_SHARE of the device's
     memory and at most 80 % of what is free now.  With the default ``tile_words`` the pool of sample
@@ -282,7 +283,7 @@ def new_records(cam, device, tile_words=REC_TILE_WORDS, budget_bytes=None, n=0, 
         free, total = torch.cuda.mem_get_info(device)
         budget_bytes = int(min(REC_MEMORY_SHARE * total, 0.8 * free))
     if tile_words == REC_TILE_WORDS:
-        key = _usage_key(cam, device, n, record_format)
+        key = _usage_key(cam, device, n, record_format, dynamic_sampling)
         use = _rec_usage.get(key)
         if use is None:
             if len(_rec_usage) >= 64:
@@ -325,12 +326,12 @@ def _read_record_use(use):
         use["need"] = (use["need"] + [int(use["pinned"][0])])[-REC_POOL_HISTORY:]
 
 
-def note_record_use(records, cam, device, n=0, record_format=0):
+def note_record_use(records, cam, device, n=0, record_format=0, dynamic_sampling=False):
     """After a forward launch that wrote ``records``: queue a 4-byte copy of the pool's bump counter
     (the slots the launch asked for, also beyond the pool's end) to pinned host memory.  Nothing waits
     for it; the next ``new_records`` of this scene size and image shape on this stream reads it."""
     ntiles, head = _pool_geometry(cam)
-    use = _rec_usage.get(_usage_key(cam, device, n, record_format))
+    use = _rec_usage.get(_usage_key(cam, device, n, record_format, dynamic_sampling))
     # (the library keeps sample sums only in a record with room for the hit lists and at least one slot per tile)
     if use is None or records is None or records.numel() // 4 // ntiles < REC_LIST_WORDS + REC_SLOT_WORDS:
         return
@@ -343,10 +344,10 @@ def note_record_use(records, cam, device, n=0, record_format=0):
     use["pending"] = True
 
 
-def record_use(cam, device, n=0, record_format=0):
+def record_use(cam, device, n=0, record_format=0, dynamic_sampling=False):
     """(bytes allocated for the last record of this scene size and image shape on this stream, bytes the last
     launch read back asked for: hit-list regions + sample-sum slots), or None before the first launch has reported."""
-    use = _rec_usage.get(_usage_key(cam, device, n, record_format))
+    use = _rec_usage.get(_usage_key(cam, device, n, record_format, dynamic_sampling))
     if use is None:
         return None
     _read_record_use(use)

@@ -133,12 +133,13 @@ class RenderOptixFunction(torch.autograd.Function):
         # when a backward will follow, the forward leaves a record of its hit lists for it to replay
         fmt = 1 if settings.rec_half_sums else 0
         backward_follows = any(ctx.needs_input_grad[:8])
-        records = (u_ox.new_records(cam, dev, settings.rec_tile_words, n=n, record_format=fmt)
+        records = (u_ox.new_records(cam, dev, settings.rec_tile_words, n=n, record_format=fmt,
+                                    dynamic_sampling=settings.dynamic_sampling)
                    if (backward_follows and settings.record_hits) else None)
         ray_colors = u_ox.march_forward(gas, cam, prims, settings.dt_step, settings.dynamic_sampling,
                                         settings.max_prim_slice, settings.white_background, settings.t_eps,
                                         settings.stats, records, record_format=fmt, backward_follows=backward_follows)
-        u_ox.note_record_use(records, cam, dev, n, fmt)
+        u_ox.note_record_use(records, cam, dev, n, fmt, settings.dynamic_sampling)
         ctx.record_format = fmt
         ctx.records = records
         ctx.settings = settings

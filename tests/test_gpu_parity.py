@@ -851,6 +851,36 @@ def test_searches_in_the_place_of_a_replay_find_what_the_forward_found(gx, n, w,
             assert not x.any() and not got.any() or (cos >= 1 - 1e-6 and rel <= 1e-4), (cos, rel)
 
 
+@pytest.mark.parametrize("w,h", [(52, 44), (312, 304), (400, 400)])              # fixed step: 4x4 blocks, halves, whole tiles; adaptive: whole tiles
+@pytest.mark.parametrize("dyn", [False, True])
+def test_a_record_of_the_other_kind_of_step_is_searched_again(gx, dyn, w, h):
+    """A record is laid out as its forward's kind of step says.  A backward of the other kind takes no tile from it: the gradients of an empty record (1e-4, as above)."""
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.render_optix import compute_rgb
+    n = 3000
+    sc = gx.to_dev(scenes.scene_to_numpy(scenes.make_scene(0, n=n, sh_degree=0, seed=33)))
+    cam = scenes.make_camera(0, 1, width=w, height=h)
+    params = sc["positions"], sc["scales"] * 3.0, sc["quaternions"], sc["densities"]
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+    cs = u_ox.camera_struct(cam)
+    rgb = compute_rgb(cam.camera_center, sc["positions"], sc["color_features"], None, None, None, 0, 0)
+    prims = u_ox.pack_prims(gas, cs, *params, rgb)
+    dloss = torch.from_numpy(np.random.default_rng(3).normal(size=(w * h, 3)).astype(np.float32)).to(gx.DEV)
+    _step(f"record of the other step, {w}x{h}, backward adaptive {dyn}")
+    rec = torch.zeros(u_ox.records_bytes(cs, 16384 * 4), dtype=torch.uint8, device=gx.DEV)
+    empty = torch.zeros_like(rec)
+    image = u_ox.march_forward(gas, cs, prims, 0.01, not dyn, 4096, True, records=rec)
+    st = [u_ox.new_stats(gx.DEV) for _ in range(2)]
+    a = u_ox.march_backward(gas, cs, prims, image, dloss, 0.01, dyn, 4096, True, records=rec, stats=st[0])
+    b = u_ox.march_backward(gas, cs, prims, image, dloss, 0.01, dyn, 4096, True, records=empty, stats=st[1])
+    sa, sb = (u_ox.read_stats(s) for s in st)
+    assert all(sa[k] == sb[k] for k in ("slabs", "hit_pairs", "candidates", "nodes_visited")) and sa["candidates"] > 0 == sa["replay_lost"]
+    assert u_ox.march_faults(n, gx.DEV) == (0, 0)
+    for x, y in zip(a, b):
+        cos, rel = gx.cos_rel(y.cpu().numpy(), x.cpu().numpy())
+        assert cos >= 1 - 1e-6 and rel <= 1e-4, (cos, rel)
+
+
 @pytest.mark.parametrize("w,h", [(19, 13), (221, 216), (225, 224), (289, 288), (1096, 1084)])    # parts of tiles; pairs; nodes
 @pytest.mark.parametrize("config,scale", [(0, 6.0), (0, 1.0)])
 def test_hits_counted_are_those_of_whole_lists_on_every_way(gx, w, h, config, scale):
