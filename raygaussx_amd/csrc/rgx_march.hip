@@ -93,7 +93,7 @@ struct MarchParams {
     uint32_t *ray_counts;   // counting forward only: per ray, slabs blended and the sum of their hit-list lengths; or null
     // (at the end: where the others lie decides which of them one load fetches)
     int32_t rec_bits;       // each tile has 2^rec_bits regions of the record
-    uint32_t sum_first;     // the first slot of the pool that is not kept for a part's lists
+    uint32_t sum_first;     // the first slot of the pool that is not a part's own to begin with
 };
 
 // The kernel's arguments once more, from the kernel's argument segment: what is read through this is loaded where it is used.
@@ -1550,8 +1550,10 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 //   TRAIL:  {tag | any_search, cover (float), sample-sum slot + 1, -}, found[64] when any_search
 // Where a tile is marched by parts (record_part_lines) each of them has that share of the region and of a slot, laid out the same with as many rays as
 // the part has in the place of 64, as many rows in the place of 4, and two words before a list's slots.  Their lists together need more than the tile's, so a
-// part whose share is used up goes on in a slot of the pool (the pool's first slots are kept for that, one for each part, where they are not most of it):
-// word RGX_REC_MORE + 1 of its region is that slot + 1 (0: none), word RGX_REC_MORE the offset of the first item there; the slot's words count from the
+// part whose share is used up goes on in a slot of the pool, or, where the pool is empty, in the first that it took for its sums, and leaves lists alone.  (The pool's first
+// slots, where it has more than those, are one for each part to begin with, so that no part is without.  Kept for the lists alone they left the sums without: 4 k Gaussians in a cube
+// 240x240, sums for 5.3 slots a tile in a pool of six and no list that goes on: two parts in three, now one in sixty.)  The
+// word RGX_REC_MORE + 1 of a region is that slot + 1 (0: none), word RGX_REC_MORE the offset of the first item there; the slot's words count from the
 // end of the share.
 //
 // Sample sums.  A record with room beyond RGX_REC_LIST_WORDS per tile also has a pool of slots
@@ -1662,6 +1664,7 @@ struct Recorder {
     int batch_left = 0;      // slots left in that batch
     uint32_t *more = nullptr; // (parts) where the region goes on, less the share's size
     int more_from = 0, more_slot = -1;
+    uint32_t own = ~0u;       // (parts) the first of the pool's slots that it took for sums
     bool cut = false;         // (parts) max_prim_slice has cut a ray's list
     __device__ __forceinline__ bool on() const { return reg != nullptr && !ovf; }
     __device__ __forceinline__ uint32_t *item() const { return (RAYS < 64 && more ? more : reg) + off; }
@@ -1671,11 +1674,16 @@ struct Recorder {
         if (off + size + 72 > cap) {
             if (RAYS < 64 && !more && P.sum_next) {
                 constexpr int COPIES = Part<RAYS>::COPIES;
+                const uint32_t units = (uint32_t)P.sum_slots / COPIES;
                 uint32_t s = 0;
-                if (P.sum_first) s = (uint32_t)((reg - P.records) / P.rec_tile_words); // its own
-                else if (threadIdx.x == 0) s = atomicAdd(P.sum_next, 1u);
+                if (threadIdx.x == 0) s = atomicAdd(P.sum_next, 1u);
                 s = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
-                if (s < (uint32_t)P.sum_slots / COPIES && size + 72 <= P.sum_slot_words * COPIES) {
+                if (s >= units && own < units) {
+                    s = own;
+                    sums = false;
+                    __threadfence(); // (what lanes stored there before is behind what others store now)
+                }
+                if (s < units && size + 72 <= P.sum_slot_words * COPIES) {
                     more_slot = (int)s * COPIES;
                     more_from = off;
                     more = (uint32_t *)(P.sum_pool + (int64_t)more_slot * (P.sum_slot_words / 4)) - cap;
@@ -1700,6 +1708,7 @@ struct Recorder {
             if (threadIdx.x == 0) s = atomicAdd(P.sum_next, COPIES > 1 ? 1u : (uint32_t)RGX_SUM_SLOT_BATCH);
             batch_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)s) * (uint32_t)COPIES;
             batch_left = COPIES > 1 ? COPIES : RGX_SUM_SLOT_BATCH;
+            if (COPIES > 1 && own == ~0u) own = batch_next / COPIES;
         }
         const uint32_t s = batch_next++;
         --batch_left;
@@ -2420,7 +2429,15 @@ RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) __global__ __launch_bounds__(64) void k_
     px0 += Pt::WIDTH == 4 ? 4 * (part & 1) : 0;
     py0 += Pt::HEIGHT * (Pt::WIDTH == 4 ? part >> 1 : part);
     typename std::conditional<RECORD, Recorder<RAYS>, typename std::conditional<WHOLE, WholeLists, NoRecorder>::type>::type rec;
-    if constexpr (RECORD) rec = Recorder<RAYS>{P.records + (((int64_t)tile << Pt::BITS) + part) * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
+    if constexpr (RECORD) {
+        const int64_t region = ((int64_t)tile << Pt::BITS) + part;
+        rec = Recorder<RAYS>{P.records + region * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
+        if (RAYS < 64 && P.sum_first) { // (the slot that it has to begin with)
+            rec.own = (uint32_t)region;
+            rec.batch_next = rec.own * (uint32_t)Pt::COPIES;
+            rec.batch_left = Pt::COPIES;
+        }
+    }
     int px, py;
     lane_pixel(px0, py0, Pt::ray(threadIdx.x), px, py);
     const bool valid = px < P.cam.width && py < P.cam.height;
@@ -3730,7 +3747,7 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
     const int bits = part_bits(P, false);
     P.part_bits = P.rec_bits = bits;
     P.rec_tile_words = P.rec_tile_words >> bits & ~3;
-    if (bits > 0 && P.sum_slots >= (int64_t)(ntiles << bits) + (int64_t)ntiles) P.sum_first = (uint32_t)(ntiles << bits); // (a slot for each, before the sums have taken all)
+    if (bits > 0 && P.sum_slots >= (int64_t)(ntiles << bits) + (int64_t)ntiles) P.sum_first = (uint32_t)(ntiles << bits); // (one for each part)
     P.sum_slot_words >>= bits;
     P.sum_slots = (int32_t)std::min<int64_t>((int64_t)P.sum_slots << bits, 0x7fffffff);
     RecordPieces rp = record_pieces((int)std::min<int64_t>((int64_t)ntiles << bits, 0x7fffffff));

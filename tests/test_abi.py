@@ -95,6 +95,13 @@ def test_bad_arguments_are_rejected_before_any_launch():
         _lib.check(-2)
 
 
+def test_the_line_of_records_by_parts_is_the_librarys():
+    """The number of tiles up to which a record's pool may be larger is that up to which the march records by parts."""
+    text = open(os.path.join(ROOT, "raygaussx_amd", "csrc", "rgx_march.hip")).read()
+    lines = [int(x) for x in re.search(r"record_part_lines\(\) \{ return \{(\d+), (\d+), (\d+)\}; \}", text).groups()]
+    assert lines[0] == 0 and lines[1] < lines[2] == u_ox.REC_PART_TILES
+
+
 def test_a_gather_of_many_tensors_asks_for_no_host_memory():
     """Nothing throws through the C ABI: with the process at its limit of address space, a gather of four million tensors comes back with a code
     (no device here: RGX_EHIP from the first launch), where a list of them would have ended the process."""

@@ -787,6 +787,31 @@ def test_records_by_parts_of_tiles(gx, w, h):
     assert np.abs(images[0] - tree["image"]).max() <= 1e-5
 
 
+@pytest.mark.parametrize("config,n,w,h,slots", [(0, 4096, 240, 240, 7), (1, 30_011, 256, 256, None), (1, 30_011, 304, 304, None)])
+def test_sums_find_room_in_a_pool_that_has_it(gx, config, n, w, h, slots):
+    """The slots that parts have to begin with hold sums: a pool of seven slots a tile where the sums ask for 5.3 and no list goes on in a slot, and the
+    first view's of a scene whose sums ask for 8.7 (fewer by halves).  Every part then has its sums (status 2, first word of its region)."""
+    from raygaussx_amd import optix_utils as u_ox
+    from raygaussx_amd.render_optix import compute_rgb
+    sc = gx.to_dev(scenes.scene_to_numpy(scenes.make_scene(config, n=n, sh_degree=0, seed=33)))
+    cam = scenes.make_camera(config, 1, width=w, height=h)
+    params = sc["positions"], sc["scales"], sc["quaternions"], sc["densities"]
+    gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+    cs = u_ox.camera_struct(cam)
+    rgb = compute_rgb(cam.camera_center, sc["positions"], sc["color_features"], None, None, None, 0, 0)
+    prims = u_ox.pack_prims(gas, cs, *params, rgb)
+    ntiles = ((w + 7) // 8) * ((h + 7) // 8)
+    parts = 4 if ntiles <= 1200 else 2
+    if slots is None:
+        rec = u_ox.new_records(cs, gx.DEV, n=n)
+    else:
+        rec = torch.empty(u_ox.records_bytes(cs, 16384 + slots * 8192), dtype=torch.uint8, device=gx.DEV)
+    _step(f"room for sums, {w}x{h}")
+    u_ox.march_forward(gas, cs, prims, 0.01 if config == 0 else 0.0025, False, 4096, True, records=rec)
+    regions = rec[:ntiles * 16384 * 4].view(torch.int32).view(ntiles * parts, -1)
+    assert torch.equal(regions[:, 0], torch.full_like(regions[:, 0], 2))
+
+
 # with the fixed step: up to 1 200 tiles by 4x4 blocks; 1 482 by halves; 18 632 whole tiles, by nodes
 @pytest.mark.parametrize("w,h", [(52, 44), (100, 80), (253, 256), (257, 256), (312, 304), (1089, 1082)])
 @pytest.mark.parametrize("dyn,cap", [(False, 8), (False, 32), (False, 4096), (True, 32)])
