@@ -1550,8 +1550,8 @@ __device__ __forceinline__ void shade_lanes(const MarchParams &P, const TileLds 
 //   TRAIL:  {tag | any_search, cover (float), sample-sum slot + 1, -}, found[64] when any_search
 // Where a tile is marched by parts (record_part_lines) each of them has that share of the region and of a slot, laid out the same with as many rays as
 // the part has in the place of 64, as many rows in the place of 4, and two words before a list's slots.  Their lists together need more than the tile's, so a
-// part whose share is used up goes on in a slot of the pool, or, where the pool is empty, in the first that it took for its sums, and leaves lists alone.  (The pool's first
-// slots, where it has more than those, are one for each part to begin with, so that no part is without.  Kept for the lists alone they left the sums without: 4 k Gaussians in a cube
+// part whose share is used up goes on in a slot of the pool, or, where the pool is empty, in its own, and leaves lists alone.  (The pool's first
+// slots, where it has more than those, are one for each part, which holds its first sums.  Kept for the lists alone they left the sums without: 4 k Gaussians in a cube
 // 240x240, sums for 5.3 slots a tile in a pool of six and no list that goes on: two parts in three, now one in sixty.)  The
 // word RGX_REC_MORE + 1 of a region is that slot + 1 (0: none), word RGX_REC_MORE the offset of the first item there; the slot's words count from the
 // end of the share.
@@ -1664,22 +1664,21 @@ struct Recorder {
     int batch_left = 0;      // slots left in that batch
     uint32_t *more = nullptr; // (parts) where the region goes on, less the share's size
     int more_from = 0, more_slot = -1;
-    uint32_t own = ~0u;       // (parts) the first of the pool's slots that it took for sums
     bool cut = false;         // (parts) max_prim_slice has cut a ray's list
     __device__ __forceinline__ bool on() const { return reg != nullptr && !ovf; }
     __device__ __forceinline__ uint32_t *item() const { return (RAYS < 64 && more ? more : reg) + off; }
     // room for an item and the iteration's trailer?
     __device__ __forceinline__ bool fits(const MarchParams &P, int size)
     {
-        if (off + size + 72 > cap) {
+        if (__builtin_expect(off + size + 72 > cap, 0)) {
             if (RAYS < 64 && !more && P.sum_next) {
                 constexpr int COPIES = Part<RAYS>::COPIES;
                 const uint32_t units = (uint32_t)P.sum_slots / COPIES;
                 uint32_t s = 0;
                 if (threadIdx.x == 0) s = atomicAdd(P.sum_next, 1u);
                 s = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
-                if (s >= units && own < units) {
-                    s = own;
+                if (s >= units && P.sum_first) {
+                    s = (uint32_t)((reg - P.records) / P.rec_tile_words); // its own
                     sums = false;
                     __threadfence(); // (what lanes stored there before is behind what others store now)
                 }
@@ -1708,7 +1707,6 @@ struct Recorder {
             if (threadIdx.x == 0) s = atomicAdd(P.sum_next, COPIES > 1 ? 1u : (uint32_t)RGX_SUM_SLOT_BATCH);
             batch_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)s) * (uint32_t)COPIES;
             batch_left = COPIES > 1 ? COPIES : RGX_SUM_SLOT_BATCH;
-            if (COPIES > 1 && own == ~0u) own = batch_next / COPIES;
         }
         const uint32_t s = batch_next++;
         --batch_left;
@@ -2433,8 +2431,7 @@ RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) __global__ __launch_bounds__(64) void k_
         const int64_t region = ((int64_t)tile << Pt::BITS) + part;
         rec = Recorder<RAYS>{P.records + region * P.rec_tile_words, RGX_REC_HEAD, P.rec_tile_words, false, P.sum_pool != nullptr, -1, P.rec_first};
         if (RAYS < 64 && P.sum_first) { // (the slot that it has to begin with)
-            rec.own = (uint32_t)region;
-            rec.batch_next = rec.own * (uint32_t)Pt::COPIES;
+            rec.batch_next = (uint32_t)region * (uint32_t)Pt::COPIES;
             rec.batch_left = Pt::COPIES;
         }
     }
