@@ -829,10 +829,10 @@ __device__ __forceinline__ void ray_begin(const MarchParams &P, int px, int py, 
 // Top of an iteration: loop condition, adaptive step (gaussians_aabb.cu:266-276) and the interval
 // this ray asks about: its slab when marching (returns true), or one slab length ahead of tbuffer
 // when searching (returns false; the search itself runs to the end of the candidate window).
-// clip: the forward clips the slab to [tenter, texit] (275-276), the backward does not (279-280).
-__device__ __forceinline__ bool slab_begin(const MarchParams &P, bool clip, RayState &R, float &tlo, float &thi)
+// clip: the forward clips the slab to [tenter, texit] (275-276), the backward does not (279-280).  t_floor: t_eps.
+__device__ __forceinline__ bool slab_begin(const MarchParams &P, bool clip, float t_floor, RayState &R, float &tlo, float &thi)
 {
-    R.active = R.active && R.tbuffer < R.texit && R.T > P.m.t_eps;
+    R.active = R.active && R.tbuffer < R.texit && R.T > t_floor;
     // a step below one ulp of t cannot advance the ray: stop instead of spinning
     R.active = R.active && (R.tbuffer + R.slab_spacing > R.tbuffer);
     if (R.active && !R.searching && P.m.dynamic_sampling) {
@@ -2456,7 +2456,7 @@ RGX_WAVES_ATTR_FWD(RECORD && RAYS < 64) __global__ __launch_bounds__(64) void k_
 
     while (__any(R.active)) {
         float tlo, thi;
-        const bool need = slab_begin(P, true, R, tlo, thi);
+        const bool need = slab_begin(P, true, P.m.t_eps, R, tlo, thi);
         int p0 = 0;
         bool ov = false;
         float found = -1.0f, searched_to = 0.f;
@@ -2927,10 +2927,16 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
     }
     const bool any_odd = REPLAY && __any(!(fabsf(g.x) < INFINITY && fabsf(g.y) < INFINITY && fabsf(g.z) < INFINITY));
 
+    // A replay of lists alone, by parts, adds a ray's hits up one after the other where its forward's copies each had some: its transmittance is the forward's up to
+    // rounding, some 1e-6 of it.  So that no ray ends before the forward's did its floor lies below that; one that goes on for it finds no hit, and the
+    // record's end is its own.
+    constexpr bool LOOSE = REPLAY && !SUMS && RAYS < 64;
+    const float t_floor = LOOSE ? P.m.t_eps * (1.0f - 0x1p-16f) : P.m.t_eps;
+
     // one slab iteration; `drive(need, tlo, thi, p0, ov, found, searched_to, body_a, mid, body_b)` supplies the hit lists
     auto iteration = [&](auto drive) {
         float tlo, thi;
-        const bool need = slab_begin(P, as_forward, R, tlo, thi);
+        const bool need = slab_begin(P, as_forward, t_floor, R, tlo, thi);
         int p0 = 0;
         bool ov = false;
         float found = -1.0f, searched_to = 0.f;
@@ -3307,7 +3313,7 @@ __device__ __forceinline__ void march_bwd(const MarchParams &P)
             }
         }
         Replayer<SUMS, RAYS> rp = {RecordView<SUMS, (RAYS < 64)>{reg, s_stage, -(1 << 30), used, more, share, more_from}, start, -1, false, RL};
-        while (__any(R.active) && !rp.lost && (!SUMS || rp.at < used)) {
+        while (__any(R.active) && !rp.lost && (!(SUMS || LOOSE) || rp.at < used)) {
             iteration([&](bool need, float, float, int &p0, bool &, float &found, float &searched_to, auto a, auto mid, auto b) {
                 return rp.template slab<SUMS>(P, R, need, p0, found, searched_to, cn, a, mid, b);
             });

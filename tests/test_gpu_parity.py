@@ -812,6 +812,42 @@ def test_sums_find_room_in_a_pool_that_has_it(gx, config, n, w, h, slots):
     assert torch.equal(regions[:, 0], torch.full_like(regions[:, 0], 2))
 
 
+@pytest.mark.parametrize("w,h", [(1, 1), (256, 304)])                            # 4x4 blocks; halves
+def test_replay_of_lists_where_a_ray_ends_on_the_floor(gx, orc, w, h):
+    """A replay of lists alone, by parts, may round a ray's transmittance otherwise than its forward, whose ray ended with just t_eps left: no record is lost for it, in
+    views of one ray (of an otherwise empty image) through sixty Gaussians, at every floor that the ray itself reaches."""
+    from raygaussx_amd import optix_utils as u_ox
+    n = 70
+    cam = scenes.look_at_camera((4.0, 0.5, 0.2), fov_x_deg=1.0 if w == 1 else 170.0, width=w, height=h)
+    cs = u_ox.camera_struct(cam)
+    px = 0 if w == 1 else (h // 2) * w + w // 2
+    along = orc.ray_dirs(orc.camera_struct(cam), np.int32([px]))[0]
+    ones = torch.ones(w * h, 3, device=gx.DEV)
+    rec = torch.empty(u_ox.records_bytes(cs, 16384), dtype=torch.uint8, device=gx.DEV)
+    _step(f"floors, {w}x{h}")
+    floors = set()
+    for seed in range(12):
+        rng = np.random.default_rng(seed)
+        t = rng.uniform(3.7, 4.3, size=(n, 1)) + (np.arange(n)[:, None] >= 60) * 4.0
+        pos = (np.float32([4.0, 0.5, 0.2]) + t * along + rng.normal(size=(n, 3)) * 0.01).astype(np.float32)
+        d = gx.to_dev(dict(pos=pos, scales=rng.uniform(0.02, 0.06, size=(n, 3)).astype(np.float32),
+                           quat=rng.normal(size=(n, 4)).astype(np.float32), dens=rng.uniform(0.2, 2.0, size=n).astype(np.float32), rgb=np.zeros((n, 3), np.float32)))
+        params = d["pos"], d["scales"], torch.nn.functional.normalize(d["quat"]), d["dens"]
+        gas = u_ox.AccelerationStructure(n, gx.DEV).build_from_gaussians(*params)
+        prims = u_ox.pack_prims(gas, cs, *params, d["rgb"])
+        for guess in np.linspace(0.99, 0.3, 24):
+            left = lambda eps: float(u_ox.march_forward(gas, cs, prims, 0.004, False, 4096, True, t_eps=eps, records=rec)[px, 0])  # (black on white: what is left of the ray)
+            eps = left(float(guess))
+            image = u_ox.march_forward(gas, cs, prims, 0.004, False, 4096, True, t_eps=eps, records=rec)
+            if float(image[px, 0]) != eps or eps in floors:
+                continue
+            floors.add(eps)
+            st = u_ox.new_stats(gx.DEV)
+            u_ox.march_backward(gas, cs, prims, image, ones, 0.004, False, 4096, True, t_eps=eps, records=rec, stats=st)
+            assert u_ox.read_stats(st)["replay_lost"] == 0 == u_ox.march_faults(n, gx.DEV)[0], (seed, eps)
+    assert len(floors) > 30
+
+
 # with the fixed step: up to 1 200 tiles by 4x4 blocks; 1 482 by halves; 18 632 whole tiles, by nodes
 @pytest.mark.parametrize("w,h", [(52, 44), (100, 80), (253, 256), (257, 256), (312, 304), (1089, 1082)])
 @pytest.mark.parametrize("dyn,cap", [(False, 8), (False, 32), (False, 4096), (True, 32)])
