@@ -1410,19 +1410,105 @@ extern "C" int rgx_gather_rows(int32_t count, const void *const *src, void *cons
 #define RGX_KNN_SEGS(C) ((C) == 8 ? 2 : 4) // runs that a wavefront's points are taken as: with two of 32 points 3 M heavy-tailed take 2.96 ms instead of 0.92
 #define RGX_KNN_QUEUE 64 // leaves that wait before the points choose among them
 
+// What the order of the points is made from (k_knn_begin).
+#define RGX_KNN_SAMPLE 1024
+struct KnnGrid {
+    float centre[3], inv_spread[3], inv_reach[3]; // 1 / what knn_warp makes of the sample's outermost points, and a little more
+    int32_t crowded;                              // so many points share a cell of that grid that it is not taken
+    float line[3][RGX_KNN_SAMPLE];                // the sample's coordinates, ascending: the lines of the other grid
+};
+
+// How far along a Hilbert curve of 2^(3 bits) cells a cell lies (the transposed form of J. Skilling, "Programming the Hilbert curve", 2004).
+__device__ __forceinline__ uint32_t hilbert_place(uint32_t (&q)[3], int bits)
+{
+    const uint32_t top = 1u << (bits - 1);
+    for (uint32_t m = top; m > 1; m >>= 1)
+        for (int a = 0; a < 3; ++a) {
+            const uint32_t t = (q[0] ^ q[a]) & (m - 1);
+            if (q[a] & m) {
+                q[0] ^= m - 1;
+            } else {
+                q[0] ^= t;
+                q[a] ^= t;
+            }
+        }
+    q[1] ^= q[0];
+    q[2] ^= q[1];
+    uint32_t t = 0;
+    for (uint32_t m = top; m > 1; m >>= 1) t ^= q[2] & m ? m - 1 : 0u;
+    uint32_t code = 0;
+    for (int b = bits - 1; b >= 0; --b)
+        for (int a = 0; a < 3; ++a) code = code << 1 | ((q[a] ^ t) >> b & 1u);
+    return code;
+}
+
+// The points of a crowded box, in the order of a curve through the box alone (there the cells of the whole cloud's say too little): thread t has the t-th of them
+// then.  p, id: a point and its index, what comes behind the last one with valid = false.
+__device__ __forceinline__ void knn_sort_box(float4 &p, uint32_t &id, bool valid)
+{
+    __shared__ float x[3][RGX_KNN_BOX], bound[RGX_KNN_BOX / 64][6];
+    __shared__ uint32_t ids[RGX_KNN_BOX];
+    __shared__ __align__(16) uint32_t key[RGX_KNN_BOX];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const bool fin = fabsf(p.x) < 1e30f && fabsf(p.y) < 1e30f && fabsf(p.z) < 1e30f;
+    const float v[3] = {p.x, p.y, p.z};
+    for (int a = 0; a < 3; ++a) {
+        const float lo = wave_min_all(fin ? v[a] : INFINITY), hi = wave_max_all(fin ? v[a] : -INFINITY);
+        if (lane == 0) {
+            bound[wave][a] = lo;
+            bound[wave][a + 3] = hi;
+        }
+        x[a][t] = v[a];
+    }
+    ids[t] = id;
+    __syncthreads();
+    uint32_t q[3];
+    for (int a = 0; a < 3; ++a) {
+        float lo = bound[0][a], hi = bound[0][a + 3];
+        for (int w = 1; w < RGX_KNN_BOX / 64; ++w) {
+            lo = fminf(lo, bound[w][a]);
+            hi = fmaxf(hi, bound[w][a + 3]);
+        }
+        const float scale = hi - lo > 1e-30f ? 128.f / (hi - lo) : 0.f;
+        q[a] = fin ? (uint32_t)fminf((v[a] - lo) * scale, 127.f) : 127u;
+    }
+    static_assert(RGX_KNN_BOX == 512, "a key is 21 bits of the curve and nine of the place");
+    const uint32_t k = (valid ? hilbert_place(q, 7) : 1u << 21) << 9 | (uint32_t)t;
+    key[t] = k;
+    __syncthreads();
+    int rank = 0;
+#pragma unroll 8
+    for (int o = 0; o < RGX_KNN_BOX; o += 4) {
+        const uint4 other = *(const uint4 *)&key[o];
+        rank += (other.x < k) + (other.y < k) + (other.z < k) + (other.w < k);
+    }
+    __syncthreads();
+    key[rank] = (uint32_t)t;
+    __syncthreads();
+    const uint32_t from = key[t];
+    p = make_float4(x[0][from], x[1][from], x[2][from], 0.f);
+    id = ids[from];
+}
+
 // Gathers the sorted points and bounds them: one workgroup per box.  A point with a coordinate that is
 // not a number is at no distance from any other: it becomes a point at infinity, and such points, like the
 // padding behind the last one, are in no box's bounds.
-__global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restrict__ pos, const uint32_t *__restrict__ order,
+__global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restrict__ pos, uint32_t *__restrict__ order, const KnnGrid *__restrict__ grid,
                                                             int64_t n, float4 *__restrict__ pts, float4 *__restrict__ leaves,
                                                             float4 *__restrict__ boxes, int32_t *supers_enc)
 {
     const int64_t i = (int64_t)blockIdx.x * RGX_KNN_BOX + threadIdx.x;
     float4 p = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+    uint32_t id = 0;
     if (i < n) {
-        const int64_t j = order[i];
+        id = order[i];
+        const int64_t j = id;
         const float x = pos[3 * j], y = pos[3 * j + 1], z = pos[3 * j + 2];
         if (x == x && y == y && z == z) p = make_float4(x, y, z, 0.f);
+    }
+    if (grid->crowded) { // (the whole launch)
+        knn_sort_box(p, id, i < n);
+        if (i < n) order[i] = id;
     }
     pts[i] = p;
     const bool fin = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
@@ -1470,26 +1556,83 @@ __global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restr
 // curve, whose consecutive cells always touch, through a grid that a sample of the cloud shapes: per axis linear where the bulk of the
 // points lies, logarithmic beyond (knn_warp).  A grid between the outermost points instead, as a few far points stretch it, leaves
 // thousands of the others in one cell, in whose order they say nothing of where they lie.
-#define RGX_KNN_SAMPLE 1024
+// Where there is no one bulk -- clumps far apart, points along a line -- a cell of that grid holds hundreds.  So a cloud of which the sample says that RGX_KNN_CROWD
+// others or more share a point's cell is sorted along the grid of the sample's quantiles, as many points between any two lines of an axis, and box by box once more along
+// a curve through the box (knn_sort_box).  Not the other clouds: the cells of sparse points far out become long and thin (54 k heavy-tailed 81 us, by quantiles 179).
+// Clouds like those of the table above come out below 10, up to a million points, clumps above 30.  The whole call, us: by a Morton curve of 30 bits through the
+// box between the outermost points and leaves of 16 / by the first grid always / now:
+//     points                             54 k              150 k                500 k                   1 M
+//     10 clumps of 0.005 in a cube    124/130/89       196/432/133       440/3 183/251        850/1 180/498
+//     3 clumps of 0.002               120/242/87       252/1 090/129     635/11 640/270     1 550/3 830/534
+//     100 clumps of 0.002             104/83/78        157/236/120       430/1 580/252      1 030/1 380/457
+//     20 clumps of 0.001 to 0.3       146/142/101      270/395/164     1 260/3 250/345      1 800/1 900/1 050
+//     along a line                     77/142/87       106/310/123       246/1 024/285        620/1 190/547
+// (A line is what a Morton curve sorts best.  A ball or a heavy-tailed cloud pays 1 to 2 us for being asked.)
+#define RGX_KNN_RANKED 64 // of the sample: a workgroup ranks so many, along one axis
+#define RGX_KNN_CROWD 16
 // Bits of the grid per axis: 24-bit keys are sorted in three passes, 30-bit keys in four.  Beyond half a million points a cell of the coarser grid
 // holds too many of them where a cloud is dense (us with 8 / 10 bits: 54 k heavy-tailed 83 / 101, 300 k 178 / 184, 1 M 408 / 352, ball 293 / 309).
 static inline int knn_bits(int64_t n) { return n <= 1 << 19 ? 8 : 10; }
-struct KnnGrid {
-    float centre[3], inv_spread[3], inv_reach[3]; // 1 / what knn_warp makes of the sample's outermost points, and a little more
-};
 __device__ __forceinline__ float knn_warp(float x, float centre, float inv_spread)
 {
     const float u = (x - centre) * inv_spread, m = fabsf(u);
     return copysignf(m < 1.f ? m : 1.f + __logf(m), u);
 }
-__global__ __launch_bounds__(256) void k_knn_begin(const float *__restrict__ pos, int64_t n, KnnGrid *grid, int32_t *supers_enc, int64_t ns)
+// the t-th point of the sample.  A few points: all of them; else places without a period that the points' own order could share
+__device__ __forceinline__ int64_t knn_sample(int t, int64_t n)
 {
-    if (blockIdx.x > 0) {
-        for (int64_t k = (int64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x; k < 6 * ns; k += (int64_t)(gridDim.x - 1) * blockDim.x)
+    return n <= RGX_KNN_SAMPLE ? (t < n ? t : n - 1) : (int64_t)(((uint64_t)((uint32_t)t * 2654435761u) * (uint64_t)n) >> 32);
+}
+// Which cell of the warped grid a point lies in, per axis.
+__device__ __forceinline__ void knn_cell(const float (&x)[3], const float (&centre)[3], const float (&inv_spread)[3], const float (&inv_reach)[3], int bits, uint32_t (&q)[3])
+{
+    const float half = (float)(1u << (bits - 1));
+    for (int a = 0; a < 3; ++a) {
+        const float u = knn_warp(x[a], centre[a], inv_spread[a]) * inv_reach[a];
+        q[a] = (uint32_t)(half + (half - 1.f) * fminf(fmaxf(u, -1.f), 1.f)); // (not a number: the grid's edge)
+    }
+}
+// One workgroup for the warped grid, RANKING for the lines of the other, the others for the bounds.
+__global__ __launch_bounds__(RGX_KNN_SAMPLE) void k_knn_begin(const float *__restrict__ pos, int64_t n, int bits, KnnGrid *grid, int32_t *supers_enc, int64_t ns)
+{
+    constexpr int RANKING = 3 * RGX_KNN_SAMPLE / RGX_KNN_RANKED;
+    __shared__ __align__(16) uint32_t s_words[4 * RGX_KNN_SAMPLE];
+    if (blockIdx.x > RANKING) {
+        for (int64_t k = (int64_t)(blockIdx.x - 1 - RANKING) * blockDim.x + threadIdx.x; k < 6 * ns; k += (int64_t)(gridDim.x - 1 - RANKING) * blockDim.x)
             supers_enc[k] = enc_f(k % 6 < 3 ? INFINITY : -INFINITY);
         return;
     }
+    if (blockIdx.x > 0) {
+        if (n <= RGX_KNN_SAMPLE) return; // (never crowded)
+        const int axis = (blockIdx.x - 1) % 3, first = (blockIdx.x - 1) / 3 * RGX_KNN_RANKED;
+        float *const x = (float *)s_words;
+        int *const count = (int *)(s_words + RGX_KNN_SAMPLE);
+        const float mine = pos[3 * knn_sample(threadIdx.x, n) + axis];
+        x[threadIdx.x] = mine == mine ? mine : INFINITY;
+        __syncthreads();
+        // how many of a sixteenth of the sample come before each (the sixteenth is a wavefront's); of equal ones the earlier of the sample
+        const int s = first + (threadIdx.x & 63), from = threadIdx.x & ~63;
+        const float v = x[s];
+        int before = 0;
+#pragma unroll 4
+        for (int t = from; t < from + 64; t += 4) {
+            const float4 o = *(const float4 *)&x[t];
+            if (from < first) before += (o.x <= v) + (o.y <= v) + (o.z <= v) + (o.w <= v);
+            else if (from > first) before += (o.x < v) + (o.y < v) + (o.z < v) + (o.w < v);
+            else before += (t < s ? o.x <= v : o.x < v) + (t + 1 < s ? o.y <= v : o.y < v) + (t + 2 < s ? o.z <= v : o.z < v) + (t + 3 < s ? o.w <= v : o.w < v);
+        }
+        count[threadIdx.x] = before;
+        __syncthreads();
+        if (threadIdx.x < RGX_KNN_RANKED) {
+            int rank = 0;
+            for (int k = 0; k < RGX_KNN_SAMPLE; k += 64) rank += count[threadIdx.x + k];
+            grid->line[axis][rank] = v;
+        }
+        return;
+    }
     constexpr int EACH = RGX_KNN_SAMPLE / 256;
+    if (threadIdx.x >= 256) return; // (four wavefronts meet sooner than sixteen)
+    for (int k = threadIdx.x; k < 4 * RGX_KNN_SAMPLE; k += 256) s_words[k] = ~0u;
     __shared__ float red[4][4][6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     auto sum = [&](int use, float *v, int m, bool most) { // over the workgroup, in every thread; or the largest of the last three
@@ -1505,9 +1648,7 @@ __global__ __launch_bounds__(256) void k_knn_begin(const float *__restrict__ pos
     };
     float x[EACH][3], w[EACH]; // w: 0 for a point that has a coordinate without a finite value
     for (int k = 0; k < EACH; ++k) {
-        const int64_t t = k * 256 + threadIdx.x;
-        // a few points: all of them; else places without a period that the points' own order could share
-        const int64_t i = n <= RGX_KNN_SAMPLE ? (t < n ? t : n - 1) : (int64_t)(((uint64_t)((uint32_t)t * 2654435761u) * (uint64_t)n) >> 32);
+        const int64_t i = knn_sample(k * 256 + threadIdx.x, n);
         for (int a = 0; a < 3; ++a) x[k][a] = pos[3 * i + a];
     }
     float v[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -1548,48 +1689,58 @@ __global__ __launch_bounds__(256) void k_knn_begin(const float *__restrict__ pos
         }
     }
     sum(3, v, 6, true);
+    float inv_spread[3], inv_reach[3];
+    for (int a = 0; a < 3; ++a) {
+        // the spread: the geometric mean distance from the centre; e of it is where an even spread ends
+        const float spread = 2.7f * __expf(v[a] / count);
+        inv_spread[a] = spread > 1e-25f ? 1.f / spread : 0.f;
+        inv_reach[a] = 1.f / fmaxf(1.05f * knn_warp(v[a + 3], 0.f, inv_spread[a]), 1e-3f);
+    }
+    // How many of the sample lie in a cell that others of it lie in: a place for each cell, maybe others' too, holds who was there last.
+    uint32_t before[EACH], cell[EACH];
+    for (int k = 0; k < EACH; ++k) {
+        uint32_t q[3];
+        knn_cell(x[k], c, inv_spread, inv_reach, bits, q);
+        cell[k] = w[k] != 0.f ? (q[0] << bits | q[1]) << bits | q[2] : ~0u - 1u;
+        before[k] = atomicExch(&s_words[cell[k] * 2654435761u >> 20], cell[k]);
+    }
+    v[0] = 0.f;
+    for (int k = 0; k < EACH; ++k) v[0] += w[k] != 0.f && before[k] == cell[k] ? 1.f : 0.f;
+    sum(0, v, 1, false);
     if (threadIdx.x < 3) {
         const int a = threadIdx.x;
-        // the spread: the geometric mean distance from the centre; e of it is where an even spread ends
-        const float log_mean = a == 0 ? v[0] : a == 1 ? v[1] : v[2], far = a == 0 ? v[3] : a == 1 ? v[4] : v[5], centre = a == 0 ? c[0] : a == 1 ? c[1] : c[2];
-        const float spread = 2.7f * __expf(log_mean / count), inv = spread > 1e-25f ? 1.f / spread : 0.f;
-        grid->centre[a] = centre;
-        grid->inv_spread[a] = inv;
-        grid->inv_reach[a] = 1.f / fmaxf(1.05f * knn_warp(far, 0.f, inv), 1e-3f);
+        grid->centre[a] = a == 0 ? c[0] : a == 1 ? c[1] : c[2];
+        grid->inv_spread[a] = a == 0 ? inv_spread[0] : a == 1 ? inv_spread[1] : inv_spread[2];
+        grid->inv_reach[a] = a == 0 ? inv_reach[0] : a == 1 ? inv_reach[1] : inv_reach[2];
+        // as many as of points spread over so few cells that RGX_KNN_CROWD share one
+        const float cells = (float)n / RGX_KNN_CROWD;
+        if (a == 0) grid->crowded = n > RGX_KNN_SAMPLE && v[0] >= RGX_KNN_SAMPLE - cells * (1.f - __expf(-RGX_KNN_SAMPLE / cells));
     }
 }
 
-// The place of every point along a Hilbert curve of 2^30 cells (the transposed form of J. Skilling, "Programming the Hilbert curve", 2004).
+// The place of every point along the curve.
 __global__ __launch_bounds__(256) void k_knn_keys(const float *__restrict__ pos, int64_t n, const KnnGrid *__restrict__ grid, int bits,
                                                   uint32_t *__restrict__ keys, uint32_t *__restrict__ vals)
 {
+    __shared__ float line[3][RGX_KNN_SAMPLE];
+    const bool crowded = grid->crowded; // (the whole launch)
+    if (crowded) {
+        const int each = RGX_KNN_SAMPLE >> bits; // of the sample's coordinates to a cell
+        for (int k = threadIdx.x; k < 3 << bits; k += 256) line[k >> bits][k & ((1 << bits) - 1)] = grid->line[k >> bits][(k & ((1 << bits) - 1)) * each + each - 1];
+        __syncthreads();
+    }
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const uint32_t top = 1u << (bits - 1);
-    const float half = (float)top;
-    uint32_t q[3];
-    for (int a = 0; a < 3; ++a) {
-        const float u = knn_warp(pos[3 * i + a], grid->centre[a], grid->inv_spread[a]) * grid->inv_reach[a];
-        q[a] = (uint32_t)(half + (half - 1.f) * fminf(fmaxf(u, -1.f), 1.f)); // (not a number: the grid's edge)
+    float x[3];
+    uint32_t q[3] = {0u, 0u, 0u};
+    for (int a = 0; a < 3; ++a) x[a] = pos[3 * i + a];
+    if (crowded) {
+        for (uint32_t m = 1u << (bits - 1); m > 0; m >>= 1) // how many lines are below it (not a number: none)
+            for (int a = 0; a < 3; ++a) q[a] += line[a][q[a] + m - 1] < x[a] ? m : 0u;
+    } else {
+        knn_cell(x, grid->centre, grid->inv_spread, grid->inv_reach, bits, q);
     }
-    for (uint32_t m = top; m > 1; m >>= 1)
-        for (int a = 0; a < 3; ++a) {
-            const uint32_t t = (q[0] ^ q[a]) & (m - 1);
-            if (q[a] & m) {
-                q[0] ^= m - 1;
-            } else {
-                q[0] ^= t;
-                q[a] ^= t;
-            }
-        }
-    q[1] ^= q[0];
-    q[2] ^= q[1];
-    uint32_t t = 0;
-    for (uint32_t m = top; m > 1; m >>= 1) t ^= q[2] & m ? m - 1 : 0u;
-    uint32_t code = 0;
-    for (int b = bits - 1; b >= 0; --b)
-        for (int a = 0; a < 3; ++a) code = code << 1 | ((q[a] ^ t) >> b & 1u);
-    keys[i] = code;
+    keys[i] = hilbert_place(q, bits);
     vals[i] = (uint32_t)i;
 }
 
@@ -1843,13 +1994,14 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     int32_t *supers = (int32_t *)(w + K.supers);
     KnnGrid *grid = (KnnGrid *)(w + K.grid);
     const int bits = knn_bits(n);
-    hipLaunchKernelGGL(k_knn_begin, dim3(1 + (unsigned)std::min<int64_t>((6 * K.ns + 255) / 256, 256)), dim3(256), 0, s, pos, n, grid, supers, K.ns);
+    hipLaunchKernelGGL(k_knn_begin, dim3(1 + 3 * RGX_KNN_SAMPLE / RGX_KNN_RANKED + (unsigned)std::min<int64_t>((6 * K.ns + RGX_KNN_SAMPLE - 1) / RGX_KNN_SAMPLE, 256)), dim3(RGX_KNN_SAMPLE), 0, s, pos, n, bits, grid, supers,
+                       K.ns);
     hipLaunchKernelGGL(k_knn_keys, grid_for(n, 256), dim3(256), 0, s, pos, n, grid, bits, k0, v0);
     RGX_LAUNCH_CHECK();
     const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 3 * bits, (uint32_t *)(w + K.m.hist), s);
     if (r < 0) return r;
-    const uint32_t *order = r ? v1 : v0;
-    hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)K.nb), dim3(RGX_KNN_BOX), 0, s, pos, order, n, pts, leaves, boxes, supers);
+    uint32_t *order = r ? v1 : v0;
+    hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)K.nb), dim3(RGX_KNN_BOX), 0, s, pos, order, grid, n, pts, leaves, boxes, supers);
     const auto search = [&](auto lanes) {
         constexpr int C = decltype(lanes)::value;
         hipLaunchKernelGGL(k_knn3<C>, grid_for(n * C, 256), dim3(256), 0, s, pts, order, n, leaves, boxes, K.nb, supers, K.ns, mean_dist2);

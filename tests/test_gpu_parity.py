@@ -1350,6 +1350,72 @@ def test_dist2_knn3_where_its_grid_changes(gx, n):
     np.testing.assert_allclose(got[ids], (d[:, 1:] ** 2).mean(1), rtol=1e-6)
 
 
+def _crowded_cloud(kind, n, rng):
+    if kind == "line":
+        return (rng.uniform(-1.0, 1.0, size=(n, 1)) * [1.0, 0.7, 0.4] + rng.normal(size=(n, 3)) * 1e-4).astype(np.float32)
+    if kind == "one place":
+        return np.full((n, 3), 0.3, np.float32)
+    if kind == "lattice":
+        return (rng.integers(0, 12, size=(n, 3)) * 0.25).astype(np.float32)
+    count, width = {"3 clumps": (3, 0.002), "10 clumps": (10, 0.005), "clumps and nan": (3, 0.002)}[kind]
+    p = (rng.uniform(-1.0, 1.0, size=(count, 3))[rng.integers(0, count, n)] + rng.normal(size=(n, 3)) * width).astype(np.float32)
+    if kind == "clumps and nan":
+        p[3::50, 1] = np.nan
+        p[5::60, 0] = np.inf
+        p[n // 2: n // 2 + 700] = np.nan
+    return p
+
+
+@pytest.mark.parametrize("n", [1024, 1025, 8193, 32_769])                        # from 1 025 on a cloud can be crowded; boxes of 512
+@pytest.mark.parametrize("kind", ["3 clumps", "10 clumps", "clumps and nan", "line", "one place", "lattice"])
+def test_dist2_knn3_of_crowded_clouds(gx, orc, kind, n):
+    """Clouds of which a cell of the first grid holds hundreds: sorted by quantiles, and box by box."""
+    from raygaussx_amd.simple_knn import distCUDA2
+    p = _crowded_cloud(kind, n, np.random.default_rng(n))
+    _step(f"distCUDA2, {kind} n={n}")
+    got = distCUDA2(torch.from_numpy(p).to(gx.DEV)).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), orc.dist2_knn3(p).view(np.uint32))
+
+
+def test_dist2_knn3_of_a_large_crowded_cloud(gx):
+    """Ten bits per axis; against a k-d tree, with the tolerance of test_dist2_knn3_where_its_grid_changes."""
+    from scipy.spatial import cKDTree
+    from raygaussx_amd.simple_knn import distCUDA2
+    n = 524_289
+    p = _crowded_cloud("10 clumps", n, np.random.default_rng(3))
+    _step("distCUDA2, ten clumps")
+    got = distCUDA2(torch.from_numpy(p).to(gx.DEV)).cpu().numpy()
+    ids = np.random.default_rng(4).choice(n, 3000, replace=False)
+    d, _ = cKDTree(p.astype(np.float64)).query(p[ids].astype(np.float64), k=4)
+    np.testing.assert_allclose(got[ids], (d[:, 1:] ** 2).mean(1), rtol=1e-6)
+
+
+@pytest.mark.parametrize("n", [54_000, 300_000])
+def test_dist2_knn3_is_not_slow_where_points_are_crowded(gx, n):
+    """Three tight clumps cost at most three times what a ball of as many points costs (measured 1.3; by one grid for all clouds 7 and 89 times), the best
+    of eight calls of each."""
+    from raygaussx_amd.simple_knn import distCUDA2
+    rng = np.random.default_rng(1)
+    v = rng.normal(size=(n, 3))
+    ball = torch.from_numpy((v / np.linalg.norm(v, axis=1, keepdims=True) * np.cbrt(rng.uniform(size=(n, 1)))).astype(np.float32)).to(gx.DEV)
+    clumps = torch.from_numpy(_crowded_cloud("3 clumps", n, rng)).to(gx.DEV)
+    _step(f"distCUDA2, times n={n}")
+
+    def best(p):
+        distCUDA2(p)
+        times = []
+        for _ in range(8):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            distCUDA2(p)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    assert best(clumps) <= 3.0 * best(ball)
+
+
 @pytest.mark.parametrize("kind", ["outliers", "two clumps", "nan", "inf", "nan and inf", "all nan", "huge"])
 def test_dist2_knn3_of_clouds_that_the_curve_does_not_sort(gx, orc, kind):
     """A few far points leave nearly all the others in one or two cells of the Morton grid, in whose order they say nothing of
