@@ -3781,6 +3781,8 @@ static int attach_records(MarchParams &P, void *records, size_t records_bytes)
 //     fixed step, 1 M, radius 2          [3.03] 2.68 2.18 2.68   4.34 2.32 2.36      3.99 2.59 2.61      2.99 2.82 3.41      2.92 2.99 4.15
 //     adaptive step, 60 k heavy-tailed   [0.81] 0.74 0.94 1.52   0.88 0.85 1.09      0.83 1.01 1.28      0.87 1.14 1.69      1.07 1.39 2.11
 //     adaptive step, 3 M heavy-tailed    [3.59] 3.00 3.19 4.30   4.00 3.68 3.86      3.85 3.86 4.20      4.61 4.70 5.42      4.56 4.92 6.25
+// Halves / 4x4 with the adaptive step, which the first columns leave out: 60 k heavy-tailed 625 tiles 0.76 / 0.68, 784 0.74 / 0.77, 900 0.73 / 0.81; 3 M heavy-tailed 2.90 / 2.19,
+// 2.50 / 2.22, 2.63 / 2.35.
 // The lines lie where a finer part stops gaining over the scenes of each step; the step stands for what else those scenes differ in: around an object half the tiles are
 // empty, from within a scene all are heavy.  (Halves for the heaviest blocks only of an image with more tiles: 300 k 800x800 2.25 -> 2.73 ms
 // for 512 tiles of 10 000.)  The sums of a ray's hits are added up in another order, and where max_prim_slice cuts a ray's list other hits are kept, equally exact both.
@@ -3811,11 +3813,12 @@ static inline PartLines image_part_lines(bool adaptive) { return adaptive ? Part
 //     20 k, radius 2                0.92 0.81 0.96       1.00 0.89 1.07       0.95 0.94            1.00 1.02
 //     100 k, radius 2               2.73 2.28 2.37       2.86 2.38 2.68       2.69 2.48            2.47 2.80      2.61 3.00
 //     300 k, radius 2               9.51 3.58 3.52       10.1 3.50 3.88       4.20 3.72            4.58 4.43      4.05 4.50
-// The lines lie where one of these scenes stops gaining (1 k Gaussians alone take 0.52 -> 0.54 at 900 to 1 024 tiles).  The large gains are
+// The line of halves lies where one of these scenes stops gaining.  That of 4x4 lies between what they gain and what they lose: from 784 to 1 156 tiles 4x4 are 10 to 20 % ahead of halves in the
+// cubes, even in the ball with 300 k, 5 to 12 % behind with 20 k and 100 k.  (1 k Gaussians alone take 0.52 -> 0.54 at 900 to 1 024 tiles by parts.)  The large gains are
 // those of scenes whose tiles' lists overflowed their regions: by parts these go on in slots.
 // (Eighths gain with up to 144 tiles -- 64 tiles: 4 k 0.80 -> 0.67, 16 k 1.27 -> 0.92, 300 k in a ball 52.8 -> 3.78 -- and lose from 256 on: 20 k of radius 2
 // 0.64 -> 0.70.  But their windows, eight times as many, add a Gaussian's sums to memory more often than a search for the whole tile would.)
-static inline PartLines record_part_lines() { return {0, 1200, 2000}; }
+static constexpr PartLines record_part_lines() { return {0, 1200, 2000}; }
 
 // image_only: no backward follows this launch
 static bool sums_in_any_order(const MarchParams &P, bool image_only) { return image_only || (P.records && !P.m.dynamic_sampling); }
@@ -3884,15 +3887,17 @@ static void launch_forward(const MarchParams &P, bool viewer, bool counting, boo
     do {                                                                                        \
         if (P.part_bits == 0) RGX_FWD_OF(64, __VA_ARGS__);                                      \
         else if (P.part_bits == 1) RGX_FWD_OF(32, __VA_ARGS__);                                 \
-        else if (P.part_bits == 2) RGX_FWD_OF(16, __VA_ARGS__);                                 \
-        else RGX_FWD_EIGHTH(__VA_ARGS__);                                                       \
+        else RGX_FWD_OF(16, __VA_ARGS__);                                                       \
     } while (0)
-#define RGX_FWD_EIGHTH(...) RGX_FWD_OF(8, __VA_ARGS__) // (a record is of quarters at the finest)
+#define RGX_FWD_IMAGE(...)                                                                      \
+    do {                                                                                        \
+        if (P.part_bits == 3) RGX_FWD_OF(8, __VA_ARGS__);                                       \
+        else RGX_FWD(__VA_ARGS__);                                                              \
+    } while (0)
+    static_assert(record_part_lines().eighths == 0, "a record is of quarters at the finest");
     if (viewer) {
-        if (counting) RGX_FWD(false, true, true, false);
-        else RGX_FWD(false, true, false, false);
-#undef RGX_FWD_EIGHTH
-#define RGX_FWD_EIGHTH(...) RGX_FWD_OF(16, __VA_ARGS__)
+        if (counting) RGX_FWD_IMAGE(false, true, true, false);
+        else RGX_FWD_IMAGE(false, true, false, false);
     } else if (P.records && half) {
         if (counting) RGX_FWD(true, false, true, true);
         else RGX_FWD(true, false, false, true);
@@ -3903,12 +3908,10 @@ static void launch_forward(const MarchParams &P, bool viewer, bool counting, boo
         if (counting) hipLaunchKernelGGL((k_march_fwd<false, false, false, true, false, true>), grid, block, 0, s, P);
         else hipLaunchKernelGGL((k_march_fwd<false, false, false, false, false, true>), grid, block, 0, s, P);
     } else {
-#undef RGX_FWD_EIGHTH
-#define RGX_FWD_EIGHTH(...) RGX_FWD_OF(8, __VA_ARGS__)
-        if (counting) RGX_FWD(false, false, true, false);
-        else RGX_FWD(false, false, false, false);
+        if (counting) RGX_FWD_IMAGE(false, false, true, false);
+        else RGX_FWD_IMAGE(false, false, false, false);
     }
-#undef RGX_FWD_EIGHTH
+#undef RGX_FWD_IMAGE
 #undef RGX_FWD
 #undef RGX_FWD_OF
 }
