@@ -598,7 +598,8 @@ def test_forward_without_a_record_is_the_march_that_its_backward_repeats(gx, dyn
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 129, 6000])
-@pytest.mark.parametrize("w,h", [(225, 224), (285, 281), (289, 288), (1088, 1083), (1096, 1084)])   # 812 and 1 296 tiles, by halves; 1 332; 18 496 and 18 632: six rounds are 18 432
+# 812, 1 296 and 1 332 tiles, by 4x4 blocks (adaptive: halves); 3 249 whole tiles, by pairs; 18 496 and 18 632, by nodes: six rounds are 18 432
+@pytest.mark.parametrize("w,h", [(225, 224), (285, 281), (289, 288), (456, 456), (1088, 1083), (1096, 1084)])
 @pytest.mark.parametrize("dyn", [False, True])
 def test_sweeps_by_pairs_of_nodes_and_by_nodes_find_the_same(gx, n, w, h, dyn):
     """Trees from a single leaf up, either side of the number of tiles up to which an image that no backward follows
@@ -848,8 +849,8 @@ def test_replay_of_lists_where_a_ray_ends_on_the_floor(gx, orc, w, h):
     assert len(floors) > 30
 
 
-# with the fixed step: up to 1 200 tiles by 4x4 blocks; 1 482 by halves; 18 632 whole tiles, by nodes
-@pytest.mark.parametrize("w,h", [(52, 44), (100, 80), (253, 256), (257, 256), (312, 304), (1089, 1082)])
+# with the fixed step: up to 1 200 tiles by 4x4 blocks; 1 482 by halves; 2 500 whole tiles by pairs of nodes, 18 632 by nodes
+@pytest.mark.parametrize("w,h", [(52, 44), (100, 80), (253, 256), (257, 256), (312, 304), (400, 400), (1089, 1082)])
 @pytest.mark.parametrize("dyn,cap", [(False, 8), (False, 32), (False, 4096), (True, 32)])
 def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx, w, h, dyn, cap):
     """Where max_prim_slice cuts a ray's list the order of the sweep decides which hits it keeps, so the backward has to
@@ -877,7 +878,7 @@ def test_a_tile_whose_record_overflowed_keeps_the_hits_that_its_forward_kept(gx,
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 129, 257, 1025, -3000])      # (negative: at one place, a tree of chains)
-@pytest.mark.parametrize("w,h", [(52, 44), (264, 264)])                          # by 4x4 blocks
+@pytest.mark.parametrize("w,h", [(52, 44), (264, 264), (312, 304), (400, 400)])  # by 4x4 blocks; halves; whole tiles, by pairs of nodes
 @pytest.mark.parametrize("cap", [4, 4096])
 def test_searches_in_the_place_of_a_replay_find_what_the_forward_found(gx, n, w, h, cap):
     """Trees from a single leaf up, with the backward handed an empty record: every tile is searched, in the forward's order, and the gradients are
@@ -942,7 +943,8 @@ def test_a_record_of_the_other_kind_of_step_is_searched_again(gx, dyn, w, h):
         assert cos >= 1 - 1e-6 and rel <= 1e-4, (cos, rel)
 
 
-@pytest.mark.parametrize("w,h", [(19, 13), (221, 216), (225, 224), (289, 288), (1096, 1084)])    # parts of tiles; pairs; nodes
+# the image by 4x2 pixels (two sizes), 4x4 blocks (two), halves, whole tiles by pairs of nodes, by nodes; the record by 4x4 blocks (three), halves, whole tiles
+@pytest.mark.parametrize("w,h", [(19, 13), (221, 216), (225, 224), (289, 288), (400, 408), (456, 456), (1096, 1084)])
 @pytest.mark.parametrize("config,scale", [(0, 6.0), (0, 1.0)])
 def test_hits_counted_are_those_of_whole_lists_on_every_way(gx, w, h, config, scale):
     """``hit_pairs`` says how many hits a view's slabs have, not how a kernel came by them: an image that collects its crowded slabs half by
