@@ -177,7 +177,7 @@ int rgx_march_workspace_bytes(int64_t n, int64_t n_rays, int32_t max_prim_slice,
  * which Gaussians each 4x4 pixel row hits and each ray's hit bits (16384 is ample for the benchmark
  * scenes).  A backward given the record of its forward replays those lists instead of searching the
  * tree again; tiles whose region overflowed, or whose region was not written by a forward launch
- * with the same number of Gaussians, image size and step, are recomputed.  The role the
+ * with the same number of Gaussians, image size, step and kind of step, are recomputed.  The role the
  * reference's hit_prim_idx buffer plays between its collect and blend steps (optix_utils.py:306),
  * at a few hundred bytes per tile and slab instead of max_prim_slice ints per ray.
  * What tile_words gives beyond 16384 (at least 8192 more) becomes one pool of 32 KiB slots shared
