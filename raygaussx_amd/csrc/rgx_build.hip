@@ -1556,20 +1556,23 @@ __global__ __launch_bounds__(RGX_KNN_BOX) void k_knn_gather(const float *__restr
 // curve, whose consecutive cells always touch, through a grid that a sample of the cloud shapes: per axis linear where the bulk of the
 // points lies, logarithmic beyond (knn_warp).  A grid between the outermost points instead, as a few far points stretch it, leaves
 // thousands of the others in one cell, in whose order they say nothing of where they lie.
-// Where there is no one bulk -- clumps far apart, points along a line -- a cell of that grid holds hundreds.  So a cloud of which the sample says that RGX_KNN_CROWD
+// Where there is no one bulk -- clumps far apart, points along a line -- a cell of that grid holds hundreds.  So a cloud of which the sample says that knn_crowd
 // others or more share a point's cell is sorted along the grid of the sample's quantiles, as many points between any two lines of an axis, and box by box once more along
 // a curve through the box (knn_sort_box).  Not the other clouds: the cells of sparse points far out become long and thin (54 k heavy-tailed 81 us, by quantiles 179).
 // Clouds like those of the table above come out below 10, up to a million points, clumps above 30.  The whole call, us: by a Morton curve of 30 bits through the
 // box between the outermost points and leaves of 16 / by the first grid always / now:
 //     points                             54 k              150 k                500 k                   1 M
-//     10 clumps of 0.005 in a cube    124/130/89       196/432/133       440/3 183/251        850/1 180/498
-//     3 clumps of 0.002               120/242/87       252/1 090/129     635/11 640/270     1 550/3 830/534
-//     100 clumps of 0.002             104/83/78        157/236/120       430/1 580/252      1 030/1 380/457
-//     20 clumps of 0.001 to 0.3       146/142/101      270/395/164     1 260/3 250/345      1 800/1 900/1 050
-//     along a line                     77/142/87       106/310/123       246/1 024/285        620/1 190/547
+//     10 clumps of 0.005 in a cube    124/130/91       196/432/133       440/3 183/255        850/1 180/501
+//     3 clumps of 0.002               120/242/87       252/1 090/129     635/11 640/267     1 550/3 830/538
+//     100 clumps of 0.002             104/83/79        157/236/120       430/1 580/254      1 030/1 380/462
+//     20 clumps of 0.001 to 0.3       146/142/102      270/395/166     1 260/3 250/355      1 800/1 900/1 050
+//     along a line                     77/142/88       106/310/124       246/1 024/287        620/1 190/548
 // (A line is what a Morton curve sorts best.  A ball or a heavy-tailed cloud pays 1 to 2 us for being asked.)
 #define RGX_KNN_RANKED 64 // of the sample: a workgroup ranks so many, along one axis
-#define RGX_KNN_CROWD 16
+// Up to so many points nothing is asked: what it and the other grid take is more than crowded cells do (5 000 points in 10 clumps 41 us, asked 52; in a ball 40 and 41).
+#define RGX_KNN_ASKED 8192
+// From so many others in a point's cell on a cloud is crowded: the fewer points, the more (16 384 in 10 clumps, some 90 others: 54 us, by quantiles 73; 32 768, some 180: 87 and 68).
+__device__ __forceinline__ float knn_crowd(int64_t n) { return fminf(fmaxf(0x1p21f / (float)n, 16.f), 128.f); }
 // Bits of the grid per axis: 24-bit keys are sorted in three passes, 30-bit keys in four.  Beyond half a million points a cell of the coarser grid
 // holds too many of them where a cloud is dense (us with 8 / 10 bits: 54 k heavy-tailed 83 / 101, 300 k 178 / 184, 1 M 408 / 352, ball 293 / 309).
 static inline int knn_bits(int64_t n) { return n <= 1 << 19 ? 8 : 10; }
@@ -1592,18 +1595,16 @@ __device__ __forceinline__ void knn_cell(const float (&x)[3], const float (&cent
         q[a] = (uint32_t)(half + (half - 1.f) * fminf(fmaxf(u, -1.f), 1.f)); // (not a number: the grid's edge)
     }
 }
-// One workgroup for the warped grid, RANKING for the lines of the other, the others for the bounds.
-__global__ __launch_bounds__(RGX_KNN_SAMPLE) void k_knn_begin(const float *__restrict__ pos, int64_t n, int bits, KnnGrid *grid, int32_t *supers_enc, int64_t ns)
+// One workgroup for the warped grid, `ranking` of them for the lines of the other (none: it is not asked for), the others for the bounds.
+__global__ __launch_bounds__(RGX_KNN_SAMPLE) void k_knn_begin(const float *__restrict__ pos, int64_t n, int bits, int ranking, KnnGrid *grid, int32_t *supers_enc, int64_t ns)
 {
-    constexpr int RANKING = 3 * RGX_KNN_SAMPLE / RGX_KNN_RANKED;
     __shared__ __align__(16) uint32_t s_words[4 * RGX_KNN_SAMPLE];
-    if (blockIdx.x > RANKING) {
-        for (int64_t k = (int64_t)(blockIdx.x - 1 - RANKING) * blockDim.x + threadIdx.x; k < 6 * ns; k += (int64_t)(gridDim.x - 1 - RANKING) * blockDim.x)
+    if ((int)blockIdx.x > ranking) {
+        for (int64_t k = (int64_t)((int)blockIdx.x - 1 - ranking) * blockDim.x + threadIdx.x; k < 6 * ns; k += (int64_t)((int)gridDim.x - 1 - ranking) * blockDim.x)
             supers_enc[k] = enc_f(k % 6 < 3 ? INFINITY : -INFINITY);
         return;
     }
     if (blockIdx.x > 0) {
-        if (n <= RGX_KNN_SAMPLE) return; // (never crowded)
         const int axis = (blockIdx.x - 1) % 3, first = (blockIdx.x - 1) / 3 * RGX_KNN_RANKED;
         float *const x = (float *)s_words;
         int *const count = (int *)(s_words + RGX_KNN_SAMPLE);
@@ -1696,25 +1697,27 @@ __global__ __launch_bounds__(RGX_KNN_SAMPLE) void k_knn_begin(const float *__res
         inv_spread[a] = spread > 1e-25f ? 1.f / spread : 0.f;
         inv_reach[a] = 1.f / fmaxf(1.05f * knn_warp(v[a + 3], 0.f, inv_spread[a]), 1e-3f);
     }
-    // How many of the sample lie in a cell that others of it lie in: a place for each cell, maybe others' too, holds who was there last.
-    uint32_t before[EACH], cell[EACH];
-    for (int k = 0; k < EACH; ++k) {
-        uint32_t q[3];
-        knn_cell(x[k], c, inv_spread, inv_reach, bits, q);
-        cell[k] = w[k] != 0.f ? (q[0] << bits | q[1]) << bits | q[2] : ~0u - 1u;
-        before[k] = atomicExch(&s_words[cell[k] * 2654435761u >> 20], cell[k]);
-    }
     v[0] = 0.f;
-    for (int k = 0; k < EACH; ++k) v[0] += w[k] != 0.f && before[k] == cell[k] ? 1.f : 0.f;
-    sum(0, v, 1, false);
+    if (ranking) {
+        // How many of the sample lie in a cell that others of it lie in: a place for each cell, maybe others' too, holds who was there last.
+        uint32_t before[EACH], cell[EACH];
+        for (int k = 0; k < EACH; ++k) {
+            uint32_t q[3];
+            knn_cell(x[k], c, inv_spread, inv_reach, bits, q);
+            cell[k] = w[k] != 0.f ? (q[0] << bits | q[1]) << bits | q[2] : ~0u - 1u;
+            before[k] = atomicExch(&s_words[cell[k] * 2654435761u >> 20], cell[k]);
+        }
+        for (int k = 0; k < EACH; ++k) v[0] += w[k] != 0.f && before[k] == cell[k] ? 1.f : 0.f;
+        sum(0, v, 1, false);
+    }
     if (threadIdx.x < 3) {
         const int a = threadIdx.x;
         grid->centre[a] = a == 0 ? c[0] : a == 1 ? c[1] : c[2];
         grid->inv_spread[a] = a == 0 ? inv_spread[0] : a == 1 ? inv_spread[1] : inv_spread[2];
         grid->inv_reach[a] = a == 0 ? inv_reach[0] : a == 1 ? inv_reach[1] : inv_reach[2];
-        // as many as of points spread over so few cells that RGX_KNN_CROWD share one
-        const float cells = (float)n / RGX_KNN_CROWD;
-        if (a == 0) grid->crowded = n > RGX_KNN_SAMPLE && v[0] >= RGX_KNN_SAMPLE - cells * (1.f - __expf(-RGX_KNN_SAMPLE / cells));
+        // as many as of points spread over so few cells that as many share one
+        const float cells = (float)n / knn_crowd(n);
+        if (a == 0) grid->crowded = ranking && v[0] >= RGX_KNN_SAMPLE - cells * (1.f - __expf(-RGX_KNN_SAMPLE / cells));
     }
 }
 
@@ -1994,8 +1997,9 @@ extern "C" int rgx_dist2_knn3(const float *pos, int64_t n, float *mean_dist2, vo
     int32_t *supers = (int32_t *)(w + K.supers);
     KnnGrid *grid = (KnnGrid *)(w + K.grid);
     const int bits = knn_bits(n);
-    hipLaunchKernelGGL(k_knn_begin, dim3(1 + 3 * RGX_KNN_SAMPLE / RGX_KNN_RANKED + (unsigned)std::min<int64_t>((6 * K.ns + RGX_KNN_SAMPLE - 1) / RGX_KNN_SAMPLE, 256)), dim3(RGX_KNN_SAMPLE), 0, s, pos, n, bits, grid, supers,
-                       K.ns);
+    const int ranking = n > RGX_KNN_ASKED ? 3 * RGX_KNN_SAMPLE / RGX_KNN_RANKED : 0;
+    hipLaunchKernelGGL(k_knn_begin, dim3(1 + ranking + (unsigned)std::min<int64_t>((6 * K.ns + RGX_KNN_SAMPLE - 1) / RGX_KNN_SAMPLE, 256)), dim3(RGX_KNN_SAMPLE), 0, s, pos, n, bits, ranking,
+                       grid, supers, K.ns);
     hipLaunchKernelGGL(k_knn_keys, grid_for(n, 256), dim3(256), 0, s, pos, n, grid, bits, k0, v0);
     RGX_LAUNCH_CHECK();
     const int r = radix_sort<uint32_t>(k0, v0, k1, v1, n, 3 * bits, (uint32_t *)(w + K.m.hist), s);

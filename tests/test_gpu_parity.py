@@ -1368,7 +1368,7 @@ def _crowded_cloud(kind, n, rng):
     return p
 
 
-@pytest.mark.parametrize("n", [1024, 1025, 8193, 32_769])                        # from 1 025 on a cloud can be crowded; boxes of 512
+@pytest.mark.parametrize("n", [1025, 8192, 8193, 16_385, 32_769])                # from 8 193 on a cloud can be crowded; boxes of 512
 @pytest.mark.parametrize("kind", ["3 clumps", "10 clumps", "clumps and nan", "line", "one place", "lattice"])
 def test_dist2_knn3_of_crowded_clouds(gx, orc, kind, n):
     """Clouds of which a cell of the first grid holds hundreds: sorted by quantiles, and box by box."""
